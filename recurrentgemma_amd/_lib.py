@@ -12,6 +12,7 @@ import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "librg_lru.so")
+HOST_PATH = os.path.join(_HERE, "_host_ops.so")
 CSRC = os.path.join(_HERE, "csrc")
 
 RG_OK = 0
@@ -111,6 +112,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
 
 
 class KernelError(RuntimeError):
@@ -118,7 +120,8 @@ class KernelError(RuntimeError):
 
 
 def build(force: bool = True) -> str:
-  """Compiles the HIP sources for gfx950 into librg_lru.so (in-tree)."""
+  """Compiles the HIP sources for gfx950 into librg_lru.so and the native host
+  path into _host_ops.so (in-tree)."""
   cmd = ["make", "-C", CSRC, "-j4"]
   if force:
     cmd.append("-B")
@@ -147,6 +150,22 @@ def lib() -> ctypes.CDLL:
       raise RuntimeError(f"librg_lru.so has ABI {got}, expected {ABI_VERSION}")
     _lib = handle
   return _lib
+
+
+def host():
+  """The native host path (csrc/host_ops.cpp): the calls that run once per
+  token or small prompt, from argument checks to launch in one native call."""
+  global _host
+  if _host is None:
+    lib()
+    if not os.path.exists(HOST_PATH):
+      raise RuntimeError(
+          f"{HOST_PATH} is missing: build it with `make -C {CSRC}` "
+          "(or __graft_entry__.build()).")
+    from recurrentgemma_amd import _host_ops
+    _host_ops.set_kernel_error(KernelError)
+    _host = _host_ops
+  return _host
 
 
 def check(status: int) -> None:

@@ -1,0 +1,513 @@
+// The short host path of the calls that are launched once per token or per
+// small prompt: a decode step, a prefill, the linear layers of a few rows.
+//
+// From Python through ctypes such a call costs 13-23 us of host time (argument
+// checks on ~15 tensors, attribute lookups, three allocations, ~20 converted
+// arguments) around a kernel of 5-10 us, so the GPU waits for the host.  Here
+// the same checks, allocations and the one C-ABI call are native code behind a
+// METH_FASTCALL entry.
+//
+// Each function serves the ordinary case only -- plain dense, 16-byte aligned
+// torch tensors of one dtype on the current GPU, shapes as documented -- and
+// answers None for anything else; its caller in ops.py then takes the general
+// path, which makes copies, converts, or raises the error that belongs to the
+// argument.  So there is one place that words the errors, and nothing here
+// has to.
+//
+// Plain C++ on torch's and this library's public interfaces; no device code.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <memory>
+#include <unordered_map>
+#include <vector>
+
+#include "../../include/rg_lru.h"
+
+namespace {
+
+PyObject* g_kernel_error = nullptr;  // _lib.KernelError
+
+struct Fallback {};  // take the general path
+struct Raised {};    // a Python exception is set
+
+using at::Tensor;
+
+// ------------------------------------------------------------- arguments --
+
+// The tensor behind a Python object: exactly torch.Tensor or Parameter (a
+// subclass may stand for something else).
+const Tensor& tensor_of(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) throw Fallback{};
+  return THPVariable_Unpack(o);
+}
+
+int dtype_code(const Tensor& t) {
+  const auto d = t.scalar_type();
+  if (d == at::kBFloat16) return RG_DTYPE_BF16;
+  if (d == at::kFloat) return RG_DTYPE_F32;
+  throw Fallback{};
+}
+
+// What a kernel can take as it lies: dense, aligned, on GPU `device`.
+void* dense(const Tensor& t, at::ScalarType dtype, c10::DeviceIndex device) {
+  if (t.scalar_type() != dtype || !t.is_cuda() ||
+      t.device().index() != device || !t.is_contiguous())
+    throw Fallback{};
+  void* p = const_cast<void*>(t.const_data_ptr());
+  if (reinterpret_cast<uintptr_t>(p) & 15u) throw Fallback{};
+  return p;
+}
+
+void need(bool ok) {
+  if (!ok) throw Fallback{};
+}
+
+bool shape_is(const Tensor& t, std::initializer_list<int64_t> want) {
+  if (t.dim() != (int64_t)want.size()) return false;
+  int i = 0;
+  for (int64_t n : want)
+    if (t.size(i++) != n) return false;
+  return true;
+}
+
+// The first tensor of a call: on the current GPU (no guard is entered here).
+struct Call {
+  const Tensor& x;
+  at::ScalarType dtype;
+  int code;
+  c10::DeviceIndex device;
+  explicit Call(PyObject* o)
+      : x(tensor_of(o)),
+        dtype(x.scalar_type()),
+        code(dtype_code(x)),
+        device(x.device().index()) {
+    need(x.is_cuda() && device == c10::hip::current_device());
+  }
+  void* operator()(PyObject* o) const {  // dense tensor of the call's dtype
+    return dense(tensor_of(o), dtype, device);
+  }
+  void* shaped(PyObject* o, std::initializer_list<int64_t> want) const {
+    const Tensor& t = tensor_of(o);
+    need(shape_is(t, want));
+    return dense(t, dtype, device);
+  }
+  void* f32(PyObject* o, std::initializer_list<int64_t> want) const {
+    const Tensor& t = tensor_of(o);
+    need(shape_is(t, want));
+    return dense(t, at::kFloat, device);
+  }
+  void* positions(PyObject* o, int64_t B, int64_t T, int* is64) const {
+    const Tensor& t = tensor_of(o);
+    need(shape_is(t, {B, T}));
+    *is64 = t.scalar_type() == at::kLong;
+    return dense(t, *is64 ? at::kLong : at::kInt, device);
+  }
+  Tensor empty(at::IntArrayRef shape, at::ScalarType t) const {
+    return at::detail::empty_cuda(
+        shape, t, at::Device(at::kCUDA, device), std::nullopt);
+  }
+  Tensor empty(at::IntArrayRef shape) const { return empty(shape, dtype); }
+  void* stream() const {
+    return c10::hip::getCurrentHIPStream(device).stream();
+  }
+};
+
+// Runs a C-ABI call without the GIL (a full queue blocks the launch).
+template <class F>
+void launch(F&& f) {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS;
+  rc = f();
+  Py_END_ALLOW_THREADS;
+  if (rc == RG_OK) return;
+  PyErr_Format(g_kernel_error ? g_kernel_error : PyExc_RuntimeError,
+               "librg_lru status %d: %s", rc, rg_last_error());
+  throw Raised{};
+}
+
+PyObject* wrap(const Tensor& t) {
+  if (!t.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(t);
+}
+
+PyObject* triple(const Tensor& a, const Tensor& b, const Tensor& c) {
+  PyObject* t = PyTuple_New(3);
+  if (!t) throw Raised{};
+  PyTuple_SET_ITEM(t, 0, wrap(a));
+  PyTuple_SET_ITEM(t, 1, wrap(b));
+  PyTuple_SET_ITEM(t, 2, wrap(c));
+  return t;
+}
+
+// Entry points share this: Fallback becomes None, torch's exceptions become
+// Python's.
+template <class F>
+PyObject* guarded(F&& f) {
+  try {
+    return f();
+  } catch (const Fallback&) {
+    Py_RETURN_NONE;
+  } catch (const Raised&) {
+    return nullptr;
+  } catch (const c10::OutOfMemoryError&) {
+    // (the general path asks again and raises torch's own exception)
+    Py_RETURN_NONE;
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+// --------------------------------------------------------------- stamps --
+
+// The state of a tensor that something was derived from: same object, same
+// storage, not written to since.  Holds a weak reference, so that the
+// object's address is not given to another tensor meanwhile.
+struct Stamp {
+  c10::weak_intrusive_ptr<c10::TensorImpl> ref;
+  c10::TensorImpl* impl;
+  const void* data;
+  int64_t version;
+  explicit Stamp(const Tensor& t)
+      : ref(t.getIntrusivePtr()),
+        impl(t.unsafeGetTensorImpl()),
+        data(t.const_data_ptr()),
+        version(t.is_inference() ? -1 : t._version()) {}
+  bool matches(const Tensor& t) const {
+    // (inference tensors keep no version counter: never known to be unchanged)
+    return t.unsafeGetTensorImpl() == impl && version >= 0 &&
+           !t.is_inference() && t._version() == version &&
+           t.const_data_ptr() == data;
+  }
+};
+
+// Gate weights in operand order, by the pair of tensors they came from.
+// ops.packed_gate_weights fills and sweeps it (remember_packed); at most
+// kMaxPacked entries are looked up here, the rest take the general path.
+struct PackedEntry {
+  Stamp x, a;
+  Tensor packed;
+};
+constexpr size_t kMaxPacked = 1024;
+std::unordered_map<c10::TensorImpl*, PackedEntry>* g_packed;
+
+// (by value: the caller keeps it alive while it launches without the GIL)
+Tensor packed_for(const Tensor& w_x, const Tensor& w_a) {
+  auto it = g_packed->find(w_x.unsafeGetTensorImpl());
+  need(it != g_packed->end() && it->second.x.matches(w_x) &&
+       it->second.a.matches(w_a));
+  return it->second.packed;
+}
+
+PyObject* remember_packed(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 3);
+    const Tensor &w_x = tensor_of(v[0]), &w_a = tensor_of(v[1]);
+    const Tensor& packed = tensor_of(v[2]);
+    for (auto it = g_packed->begin(); it != g_packed->end();)
+      it = it->second.x.ref.expired() || it->second.a.ref.expired()
+               ? g_packed->erase(it)
+               : std::next(it);
+    g_packed->erase(w_x.unsafeGetTensorImpl());
+    if (g_packed->size() < kMaxPacked && !w_x.is_inference() &&
+        !w_a.is_inference())
+      g_packed->emplace(w_x.unsafeGetTensorImpl(),
+                        PackedEntry{Stamp(w_x), Stamp(w_a), packed});
+    Py_RETURN_NONE;
+  });
+}
+
+// --------------------------------------------------------- recurrent core --
+
+// (x, segment_pos, conv_state, h, conv_w, conv_b, w_x, b_x, w_a, b_a, a_param,
+//  in_place, gate_branch | None) -> (y, h, conv_state) | None
+PyObject* recurrent_step(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 13);
+    Call c(v[0]);
+    need(c.x.dim() == 3 && c.x.size(1) == 1);
+    const int64_t B = c.x.size(0), W = c.x.size(2);
+    const Tensor &w_x = tensor_of(v[6]), &w_a = tensor_of(v[8]);
+    need(B > 0 && w_x.dim() == 3);
+    const int64_t H = w_x.size(0);
+    need(H > 0 && W % H == 0 && B <= INT32_MAX && W <= INT32_MAX);
+    const int64_t bw = W / H;
+    void* wx = c.shaped(v[6], {H, bw, bw});
+    void* wa = c.shaped(v[8], {H, bw, bw});
+    void* x = c(v[0]);
+    int is64;
+    void* pos = c.positions(v[1], B, 1, &is64);
+    void* conv_in = c.shaped(v[2], {B, 3, W});
+    void* h_in = c.f32(v[3], {B, W});
+    void* conv_w = c.shaped(v[4], {4, W});
+    void* conv_b = c.shaped(v[5], {W});
+    void* b_x = c.shaped(v[7], {H, bw});
+    void* b_a = c.shaped(v[9], {H, bw});
+    void* a_param = c.shaped(v[10], {W});
+    // one launch on re-laid-out weights, or conv step + gate GEMM + scan step
+    // (+ the join) through a workspace
+    Tensor packed, ws;
+    if (c.code == RG_DTYPE_BF16 && bw == 256) {
+      packed = packed_for(w_x, w_a);
+      need(packed.device() == c.x.device());
+    }
+    const bool in_place = v[11] == Py_True;
+    void* gate = v[12] == Py_None ? nullptr : c.shaped(v[12], {B, 1, W});
+    Tensor y = c.empty(c.x.sizes());
+    Tensor h, conv;
+    if (in_place) {
+      h = THPVariable_Unpack(v[3]);
+      conv = THPVariable_Unpack(v[2]);
+    } else {
+      h = c.empty({B, W}, at::kFloat);
+      conv = c.empty({B, 3, W});
+    }
+    void *yp = y.mutable_data_ptr(), *hp = h.mutable_data_ptr(),
+         *cp = conv.mutable_data_ptr();
+    void* s = c.stream();
+    if (!packed.defined()) {
+      const size_t bytes =
+          rg_recurrent_step_workspace_bytes((int)B, (int)W, c.code);
+      ws = c.empty({(int64_t)bytes}, at::kByte);
+      void* wp = ws.mutable_data_ptr();
+      launch([&] {
+        const int rc = rg_recurrent_step(
+            x, pos, is64, conv_in, cp, (const float*)h_in, (float*)hp, conv_w,
+            conv_b, wx, b_x, wa, b_a, a_param, yp, wp, bytes, (int)B, (int)W,
+            (int)H, c.code, s);
+        if (rc != RG_OK || !gate) return rc;
+        return rg_gelu_mul(yp, gate, yp, B * W, c.code, s);
+      });
+      return triple(y, h, conv);
+    }
+    const void* pk = packed.const_data_ptr();
+    launch([&] {
+      if (gate)
+        return rg_recurrent_step_gelu_mul(
+            x, gate, pos, is64, conv_in, cp, (const float*)h_in, (float*)hp,
+            conv_w, conv_b, pk, b_x, b_a, a_param, yp, (int)B, (int)W, (int)H,
+            c.code, s);
+      return rg_recurrent_step_packed(
+          x, pos, is64, conv_in, cp, (const float*)h_in, (float*)hp, conv_w,
+          conv_b, pk, b_x, b_a, a_param, yp, (int)B, (int)W, (int)H, c.code, s);
+    });
+    return triple(y, h, conv);
+  });
+}
+
+// (x, segment_pos, conv_w | None, conv_b | None, w_x, b_x, w_a, b_a, a_param,
+//  h0 | None, return_h, return_conv_cache, gate_branch | None)
+//   -> (y, h | None, conv_cache | None) | None
+PyObject* recurrent_core(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 13);
+    Call c(v[0]);
+    need(c.x.dim() == 3 && c.x.numel() > 0);
+    const int64_t B = c.x.size(0), T = c.x.size(1), W = c.x.size(2);
+    const Tensor &w_x = tensor_of(v[4]), &w_a = tensor_of(v[6]);
+    need(w_x.dim() == 3 && B <= INT32_MAX && T <= INT32_MAX && W <= INT32_MAX);
+    const int64_t H = w_x.size(0);
+    need(H > 0 && W % H == 0);
+    const int64_t bw = W / H;
+    void* x = c(v[0]);
+    int is64;
+    void* pos = c.positions(v[1], B, T, &is64);
+    const bool conv = v[2] != Py_None;
+    need(conv == (v[3] != Py_None));
+    void* conv_w = conv ? c.shaped(v[2], {4, W}) : nullptr;
+    void* conv_b = conv ? c.shaped(v[3], {W}) : nullptr;
+    void* wx = c.shaped(v[4], {H, bw, bw});
+    void* b_x = c.shaped(v[5], {H, bw});
+    void* wa = c.shaped(v[6], {H, bw, bw});
+    void* b_a = c.shaped(v[7], {H, bw});
+    void* a_param = c.shaped(v[8], {W});
+    void* h0 = v[9] == Py_None ? nullptr : c.f32(v[9], {B, W});
+    void* gate = v[12] == Py_None ? nullptr : c.shaped(v[12], {B, T, W});
+    const void* pk = nullptr;
+    Tensor packed;
+    if (c.code == RG_DTYPE_BF16 && bw == 256 && T * W * 2 < INT32_MAX) {
+      packed = packed_for(w_x, w_a);
+      need(packed.device() == c.x.device());
+      pk = packed.const_data_ptr();
+    }
+    Tensor y = c.empty(c.x.sizes()), h, cache, ws;
+    if (v[10] == Py_True) h = c.empty({B, W}, at::kFloat);
+    if (v[11] == Py_True && conv) cache = c.empty({B, 3, W});
+    const size_t bytes = rg_recurrent_core_workspace_bytes(
+        (int)B, (int)T, (int)W, (int)H, c.code);
+    if (bytes) ws = c.empty({(int64_t)bytes}, at::kByte);
+    void* yp = y.mutable_data_ptr();
+    void* hp = h.defined() ? h.mutable_data_ptr() : nullptr;
+    void* cp = cache.defined() ? cache.mutable_data_ptr() : nullptr;
+    void* wp = bytes ? ws.mutable_data_ptr() : nullptr;
+    void* s = c.stream();
+    launch([&] {
+      return rg_recurrent_core(x, gate, pos, is64, conv_w, conv_b, wx, b_x, wa,
+                               b_a, pk, a_param, h0, yp, hp, cp, wp, bytes,
+                               (int)B, (int)T, (int)W, (int)H, c.code, s);
+    });
+    return triple(y, h, cache);
+  });
+}
+
+// ------------------------------------------------- linear layers, few rows --
+
+// What ops.PackedLinear prepared from its weights and biases.
+struct RowsPlan {
+  std::vector<Stamp> sources;
+  Tensor packed, bias;
+  int N, K, groups;
+  bool gelu_pair;
+};
+const char kPlanName[] = "recurrentgemma_amd.rows_plan";
+
+void free_plan(PyObject* capsule) {
+  delete static_cast<RowsPlan*>(PyCapsule_GetPointer(capsule, kPlanName));
+}
+
+// (sources tuple, packed, bias | None, N, K, groups, gelu_pair) -> plan
+PyObject* rows_plan(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 7 && PyTuple_Check(v[0]));
+    auto plan = std::make_unique<RowsPlan>();
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(v[0]); ++i)
+      plan->sources.emplace_back(tensor_of(PyTuple_GET_ITEM(v[0], i)));
+    plan->packed = tensor_of(v[1]);
+    if (v[2] != Py_None) plan->bias = tensor_of(v[2]);
+    plan->N = (int)PyLong_AsLong(v[3]);
+    plan->K = (int)PyLong_AsLong(v[4]);
+    plan->groups = (int)PyLong_AsLong(v[5]);
+    plan->gelu_pair = v[6] == Py_True;
+    if (PyErr_Occurred()) throw Raised{};
+    return PyCapsule_New(plan.release(), kPlanName, free_plan);
+  });
+}
+
+// The plan of a call, if its weights and biases are what it was made from.
+const RowsPlan& plan_of(PyObject* capsule, PyObject* weights, PyObject* biases) {
+  need(PyCapsule_IsValid(capsule, kPlanName));
+  const auto& p =
+      *static_cast<RowsPlan*>(PyCapsule_GetPointer(capsule, kPlanName));
+  size_t at = 0;
+  for (PyObject* list : {weights, biases}) {
+    if (list == Py_None) continue;
+    need(PyTuple_Check(list));
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(list); ++i) {
+      PyObject* o = PyTuple_GET_ITEM(list, i);
+      if (o == Py_None) continue;
+      need(at < p.sources.size() && p.sources[at].matches(tensor_of(o)));
+      ++at;
+    }
+  }
+  need(at == p.sources.size());
+  return p;
+}
+
+// leading dimensions of x, and how many rows they make
+std::vector<int64_t> lead_of(const Call& c, int K, int64_t* M) {
+  need(c.code == RG_DTYPE_BF16 && c.x.dim() >= 1 && c.x.size(-1) == K);
+  std::vector<int64_t> lead(c.x.sizes().begin(), c.x.sizes().end() - 1);
+  *M = c.x.numel() / K;
+  need(*M > 0 && *M <= 64);
+  return lead;
+}
+
+// (plan, x, weights, biases | None, residual | None) -> out | tuple | None
+PyObject* rows_linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 5);
+    const RowsPlan& p = plan_of(v[0], v[2], v[3]);
+    Call c(v[1]);
+    int64_t M;
+    std::vector<int64_t> shape = lead_of(c, p.K, &M);
+    need(p.packed.device() == c.x.device());
+    void* x = c(v[1]);
+    const bool grouped = p.groups > 1 && !p.gelu_pair;
+    shape.push_back(p.gelu_pair ? p.N / 2 : p.N / p.groups);
+    void* residual = nullptr;
+    if (v[4] != Py_None) {
+      const Tensor& r = tensor_of(v[4]);
+      need(!grouped && !p.gelu_pair && r.sizes() == at::IntArrayRef(shape));
+      residual = dense(r, c.dtype, c.device);
+    }
+    // (one allocation per group: the kernel wants [G, M, N / G] in one piece)
+    if (grouped) shape.insert(shape.begin(), p.groups);
+    Tensor out = c.empty(shape), ws;
+    const size_t bytes =
+        p.gelu_pair ? 0 : rg_linear_rows_workspace_bytes((int)M, p.K, p.N);
+    if (bytes) ws = c.empty({(int64_t)bytes}, at::kByte);
+    void* op = out.mutable_data_ptr();
+    void* wp = bytes ? ws.mutable_data_ptr() : nullptr;
+    const void* pk = p.packed.const_data_ptr();
+    const void* bias = p.bias.defined() ? p.bias.const_data_ptr() : nullptr;
+    void* s = c.stream();
+    launch([&] {
+      return rg_linear_rows(x, pk, bias, residual, op, wp, bytes, (int)M, p.K,
+                            p.N, grouped ? p.groups : 1, p.gelu_pair, s);
+    });
+    if (!grouped) return wrap(out);
+    PyObject* t = PyTuple_New(p.groups);
+    if (!t) throw Raised{};
+    for (int i = 0; i < p.groups; ++i)
+      PyTuple_SET_ITEM(t, i, wrap(out.select(0, i)));
+    return t;
+  });
+}
+
+// (plan, x, weights, biases | None, slices) -> sums [slices, M, N] | None
+PyObject* rows_partial(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 5);
+    const RowsPlan& p = plan_of(v[0], v[2], v[3]);
+    Call c(v[1]);
+    int64_t M;
+    lead_of(c, p.K, &M);
+    need(p.packed.device() == c.x.device() && p.groups == 1 && !p.gelu_pair);
+    void* x = c(v[1]);
+    const long slices = PyLong_AsLong(v[4]);
+    need(slices > 0);
+    Tensor sums = c.empty({slices, M, (int64_t)p.N}, at::kFloat);
+    void* op = sums.mutable_data_ptr();
+    const void* pk = p.packed.const_data_ptr();
+    void* s = c.stream();
+    launch([&] {
+      return rg_linear_rows_partial(x, pk, (float*)op, (int)M, p.K, p.N,
+                                    (int)slices, s);
+    });
+    return wrap(sums);
+  });
+}
+
+PyObject* set_kernel_error(PyObject*, PyObject* type) {
+  Py_INCREF(type);
+  Py_XDECREF(g_kernel_error);
+  g_kernel_error = type;
+  Py_RETURN_NONE;
+}
+
+PyMethodDef kMethods[] = {
+    {"recurrent_step", (PyCFunction)(void*)recurrent_step, METH_FASTCALL, ""},
+    {"recurrent_core", (PyCFunction)(void*)recurrent_core, METH_FASTCALL, ""},
+    {"rows_plan", (PyCFunction)(void*)rows_plan, METH_FASTCALL, ""},
+    {"rows_linear", (PyCFunction)(void*)rows_linear, METH_FASTCALL, ""},
+    {"rows_partial", (PyCFunction)(void*)rows_partial, METH_FASTCALL, ""},
+    {"remember_packed", (PyCFunction)(void*)remember_packed, METH_FASTCALL, ""},
+    {"set_kernel_error", set_kernel_error, METH_O, ""},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host_ops", nullptr, -1,
+                       kMethods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host_ops(void) {
+  g_packed = new std::unordered_map<c10::TensorImpl*, PackedEntry>();
+  return PyModule_Create(&kModule);
+}

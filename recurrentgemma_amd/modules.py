@@ -33,7 +33,27 @@ def gelu(x: torch.Tensor) -> torch.Tensor:
   return nn.functional.gelu(x, approximate="tanh")
 
 
-@torch.no_grad()
+def _parameters(module, *names):
+  """Parameters of a module by name.  nn.Module's attribute lookup costs about
+  half a microsecond each, which a decode step with its twenty tensors does
+  not have; the dictionary behind it is read instead, and the attribute where
+  the name is not in it (a parametrised weight)."""
+  own = module._parameters
+  return [own[n] if n in own else getattr(module, n) for n in names]
+
+
+def _core_weights(conv_1d, rg_lru):
+  """conv_w, conv_b, w_x, b_x, w_a, b_a, a_param."""
+  if compiled.tracing():
+    gx, ga = rg_lru.input_gate, rg_lru.a_gate
+    return conv_1d.w, conv_1d.b, gx.w, gx.b, ga.w, ga.b, rg_lru.a_param
+  gates = rg_lru._modules
+  return (*_parameters(conv_1d, "w", "b"),
+          *_parameters(gates["input_gate"], "w", "b"),
+          *_parameters(gates["a_gate"], "w", "b"),
+          *_parameters(rg_lru, "a_param"))
+
+
 def recurrent_core(conv_1d: layers.Conv1D, rg_lru: layers.RGLRU, x,
                    segment_pos, cache: RecurrentBlockCache | None = None,
                    return_cache: bool = True, in_place: bool = False,
@@ -46,9 +66,21 @@ def recurrent_core(conv_1d: layers.Conv1D, rg_lru: layers.RGLRU, x,
   gate_branch: the block's linear_y output; the result is then the join
   y * gelu(gate_branch) of modules.py:627-628, 644 -- inside the prefill
   kernel where that runs, as a pass of its own (ops.gelu_mul) elsewhere."""
+  if not torch.is_grad_enabled():
+    return _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
+                           in_place, gate_branch)
+  with torch.no_grad():
+    return _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
+                           in_place, gate_branch)
+
+
+def _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
+                    in_place, gate_branch):
   bs, l, _ = x.shape
   assert segment_pos.shape == (bs, l)
   fused = conv_1d.temporal_width == 4
+  if fused:
+    weights = _core_weights(conv_1d, rg_lru)
   if cache is not None:
     b, num_tokens, d = x.shape
     assert cache.conv1d_state.shape == (b, conv_1d.temporal_width - 1, d)
@@ -57,14 +89,11 @@ def recurrent_core(conv_1d: layers.Conv1D, rg_lru: layers.RGLRU, x,
       if compiled.tracing() and not in_place:
         # (a traced program holds the step as one operator node)
         y, h, conv_state = torch.ops.recurrentgemma_amd.recurrent_step(
-            x, segment_pos, cache.conv1d_state, cache.rg_lru_state, conv_1d.w,
-            conv_1d.b, rg_lru.input_gate.w, rg_lru.input_gate.b,
-            rg_lru.a_gate.w, rg_lru.a_gate.b, rg_lru.a_param, gate_branch)
+            x, segment_pos, cache.conv1d_state, cache.rg_lru_state, *weights,
+            gate_branch)
       else:
         y, h, conv_state = ops.recurrent_step(
-            x, segment_pos, cache.conv1d_state, cache.rg_lru_state, conv_1d.w,
-            conv_1d.b, rg_lru.input_gate.w, rg_lru.input_gate.b,
-            rg_lru.a_gate.w, rg_lru.a_gate.b, rg_lru.a_param,
+            x, segment_pos, cache.conv1d_state, cache.rg_lru_state, *weights,
             in_place=in_place, gate_branch=gate_branch)
       if not return_cache:
         return y, None
@@ -87,14 +116,10 @@ def recurrent_core(conv_1d: layers.Conv1D, rg_lru: layers.RGLRU, x,
     # form it is a pass of its own).
     if compiled.tracing():
       y, h, conv_state = torch.ops.recurrentgemma_amd.recurrent_core(
-          x, segment_pos, conv_1d.w, conv_1d.b, rg_lru.input_gate.w,
-          rg_lru.input_gate.b, rg_lru.a_gate.w, rg_lru.a_gate.b,
-          rg_lru.a_param, None, gate_branch)
+          x, segment_pos, *weights, None, gate_branch)
     else:
       y, h, conv_state = ops.recurrent_core(
-          x, segment_pos, conv_1d.w, conv_1d.b, rg_lru.input_gate.w,
-          rg_lru.input_gate.b, rg_lru.a_gate.w, rg_lru.a_gate.b,
-          rg_lru.a_param, h0=None, return_h=return_cache,
+          x, segment_pos, *weights, h0=None, return_h=return_cache,
           return_conv_cache=return_cache, gate_branch=gate_branch)
     gate_branch = None
   if gate_branch is not None:
@@ -168,8 +193,11 @@ class RecurrentBlock(nn.Module):
           ops.PackedLinear.usable(x, self.width, self.lru_width) and
           ops.PackedLinear.usable(x, self.lru_width, self.width))
       if few_rows:
-        y, x = self._rows_yx(x, (self.linear_y.weight, self.linear_x.weight),
-                             (self.linear_y.bias, self.linear_x.bias))
+        linear = self._modules
+        w_y, b_y = _parameters(linear["linear_y"], "weight", "bias")
+        w_x, b_x = _parameters(linear["linear_x"], "weight", "bias")
+        w_out, b_out = _parameters(linear["linear_out"], "weight", "bias")
+        y, x = self._rows_yx(x, (w_y, w_x), (b_y, b_x))
       else:
         y = self.linear_y(x)
         x = self.linear_x(x)
@@ -181,11 +209,9 @@ class RecurrentBlock(nn.Module):
           gate_branch=y)
       if few_rows and defer_out and ops.PackedLinear.partial_slices(
           x, self.lru_width, self.width):
-        x = self._rows_out.partial(x, (self.linear_out.weight,),
-                                   (self.linear_out.bias,))
+        x = self._rows_out.partial(x, (w_out,), (b_out,))
       elif few_rows:
-        x = self._rows_out(x, (self.linear_out.weight,),
-                           (self.linear_out.bias,))
+        x = self._rows_out(x, (w_out,), (b_out,))
       else:
         x = self.linear_out(x)
     if not return_cache:

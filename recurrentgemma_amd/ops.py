@@ -7,6 +7,8 @@ HIP stream.  Nothing here computes on the CPU.
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from recurrentgemma_amd import _lib
@@ -397,6 +399,11 @@ def recurrent_core(x, segment_pos, conv_w, conv_b, w_x, b_x, w_a, b_a, a_param,
   conv_w = conv_b = None: x is the conv output already (RGLRU.forward on its
   own, layers.py:313-365); there is then no conv cache to return.
   Returns (y, h_last | None, conv_cache | None)."""
+  done = _lib.host().recurrent_core(x, segment_pos, conv_w, conv_b, w_x, b_x,
+                                    w_a, b_a, a_param, h0, return_h,
+                                    return_conv_cache, gate_branch)
+  if done is not None:  # (None: not the ordinary case, see host_ops.cpp)
+    return done
   B, T, W = x.shape
   H = w_x.shape[0]
   if conv_w is None:
@@ -866,6 +873,7 @@ def packed_gate_weights(w_x, w_a):
             if v[0]() is None or v[1]() is None]:
     del _packed_weights[k]  # entries whose tensors are gone
   _packed_weights[key] = (weakref.ref(w_x), weakref.ref(w_a), stamp, packed)
+  _lib.host().remember_packed(w_x, w_a, packed)
   return packed
 
 
@@ -899,6 +907,11 @@ class PendingSum:
     return self.a + self.b
 
 
+@functools.lru_cache(maxsize=256)
+def _packable(N, K, gelu_pair) -> bool:
+  return _lib.lib().rg_linear_packed_bytes(N, K, gelu_pair) > 0
+
+
 class PackedLinear:
   """Linear layers that read the same few rows (a decode step), on the
   weight-streaming kernel (rg_linear_rows).  Holds the weights in the kernel's
@@ -921,17 +934,20 @@ class PackedLinear:
     self._packed = None
     self._bias = None
     self._shape = None  # (N, K, groups)
+    self._plan = None   # the same for the native call (host_ops.cpp)
 
   def __deepcopy__(self, memo):
     return PackedLinear(self.layout, self.gelu_pair)
+
+  def __reduce__(self):  # (packed again where it is unpickled)
+    return PackedLinear, (self.layout, self.gelu_pair)
 
   @staticmethod
   def usable(x, K, N, gelu_pair=False) -> bool:
     """Whether x [..., K] qualifies: bf16 on the GPU, at most 64 rows, and a
     weight shape the packed layout covers."""
     return (x.is_cuda and x.dtype == torch.bfloat16 and
-            x.numel() // K <= 64 and
-            _lib.lib().rg_linear_packed_bytes(N, K, int(gelu_pair)) > 0)
+            x.numel() // K <= 64 and _packable(N, K, int(gelu_pair)))
 
   def _prepare(self, weights, biases):
     tensors = tuple(weights) + tuple(b for b in (biases or ()) if b is not None)
@@ -985,6 +1001,8 @@ class PackedLinear:
     self._packed, self._bias = packed, bias
     self._shape = (N, K, groups)
     self._stamp = stamp
+    self._plan = _lib.host().rows_plan(tensors, packed, bias, N, K, groups,
+                                       self.gelu_pair)
 
   @staticmethod
   def partial_slices(x, K, N) -> int:
@@ -1001,6 +1019,13 @@ class PackedLinear:
     """One layer, left as partial sums for the norm that follows it
     (add_rms_norm): K is split over the grid, so three times as many
     workgroups stream the weights, and no separate pass adds the slices."""
+    if self._plan is not None:
+      N, K, _ = self._shape
+      sums = _lib.host().rows_partial(self._plan, x, weights, biases,
+                                      self.partial_slices(x, K, N))
+      if sums is not None:
+        return PartialSums(sums, self._bias, (*x.shape[:-1], N), x.dtype,
+                           addend)
     x = _dev(x, "x")
     self._prepare(weights, biases)
     N, K, groups = self._shape
@@ -1019,6 +1044,10 @@ class PackedLinear:
     """x [..., K].  Returns out [..., N] (one layer), a tuple of outputs
     (several layers / a stacked weight), or the gelu pair product [..., N/2].
     residual (one layer only): added after the output is rounded."""
+    if self._plan is not None:
+      out = _lib.host().rows_linear(self._plan, x, weights, biases, residual)
+      if out is not None:
+        return out
     x = _dev(x, "x")
     _dtype_code(x)
     self._prepare(weights, biases)
@@ -1065,6 +1094,11 @@ def recurrent_step(x, segment_pos, conv_cache, h, conv_w, conv_b, w_x, b_x, w_a,
   (packed once per weight version); other shapes as conv step + gate GEMM +
   scan step.  gate_branch: the block's linear_y output [B,1,W]; y is then
   y * gelu(gate_branch) (inside the one launch where that runs)."""
+  done = _lib.host().recurrent_step(x, segment_pos, conv_cache, h, conv_w,
+                                    conv_b, w_x, b_x, w_a, b_a, a_param,
+                                    in_place, gate_branch)
+  if done is not None:  # (None: not the ordinary case, see host_ops.cpp)
+    return done
   B, n_tok, W = x.shape
   assert n_tok == 1
   assert conv_cache.shape == (B, 3, W)
