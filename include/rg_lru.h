@@ -300,10 +300,9 @@ int rg_recurrent_prefill_gelu_mul(
 
 /* conv_1d -> rg_lru of a prefill as RecurrentBlock.forward chains them
  * (recurrentgemma/torch/modules.py:632-643), for every shape and both dtypes,
- * with the choice of kernels made here: the single prefill kernel
- * (rg_recurrent_prefill_split; bf16, 256-wide heads, enough (row, head) pairs
- * or rows long enough to be cut into chunks, but not more than 256 pairs of
- * fewer than 64 tokens); for float32 with 256-wide heads and at most 32
+ * with the choice of kernels made here: a single prefill kernel (bf16, heads
+ * of 256 channels: rg_recurrent_prefill_split, but for very many rows of a few
+ * tokens; heads of 136 .. 248 channels where that is ahead); for float32 with 256-wide heads and at most 32
  * (row, head) pairs one launch that does the same in float32 (needs no
  * workspace; no entry point of its own); else rg_gates_gemm with the conv
  * applied on load followed by rg_lru_scan_fused_split, the pre-activations of
@@ -509,16 +508,17 @@ int rg_attention_decode_fused(const void* q, int64_t ldq, const void* k_new,
 /* The same decode step in ONE launch, for bf16 with 256-wide heads (no
  * counterpart call in the reference: it is RecurrentBlock.forward with a
  * cache, modules.py:632-643, after a one-time re-layout of the two gate
- * matrices).  rg_pack_gate_weights writes w_x and w_a ([H,256,256] each, the
+ * matrices).  rg_pack_gate_weights writes w_x and w_a ([H,bw,bw] each, the
  * reference's BlockDiagonalLinear layout, layers.py:105-112) into `packed`
- * (rg_packed_gate_weights_bytes(W, H, dtype) bytes, 16-byte aligned) in the
- * order the MFMA operand registers are filled: head, group of 32 output
- * channels, 16-row k-step, gate, lane, 8 values.  Pack again whenever the
- * weights change.  rg_recurrent_step_packed then takes `packed` in place of
+ * (rg_packed_gate_weights_bytes(W, H, dtype) bytes, 16-byte aligned; bf16 and
+ * heads of 136 .. 256 channels, a multiple of 8 -- the count is 0 otherwise) in
+ * the order the MFMA operand registers are filled: head, group of 32 output
+ * channels, 16-row k-step, gate, lane, 8 values, zeros beyond the head.  Pack
+ * again whenever the weights change.  rg_recurrent_step_packed then takes `packed` in place of
  * w_x / w_a and needs no workspace; all other arguments are as for
- * rg_recurrent_step (outputs may alias inputs).  Both return
- * RG_ERR_UNSUPPORTED for other dtypes or head widths (the byte count is 0
- * then): use rg_recurrent_step. */
+ * rg_recurrent_step (outputs may alias inputs).  It returns
+ * RG_ERR_UNSUPPORTED for other dtypes or head widths than bf16 and 256: use
+ * rg_recurrent_step. */
 size_t rg_packed_gate_weights_bytes(int W, int H, int dtype);
 int rg_pack_gate_weights(const void* w_x, const void* w_a, void* packed, int W,
                          int H, int dtype, void* stream);

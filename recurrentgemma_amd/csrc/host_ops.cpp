@@ -332,7 +332,7 @@ PyObject* recurrent_core(PyObject*, PyObject* const* v, Py_ssize_t n) {
     void* gate = v[12] == Py_None ? nullptr : c.shaped(v[12], {B, T, W});
     const void* pk = nullptr;
     Tensor packed;
-    if (c.code == RG_DTYPE_BF16 && bw == 256 && T * W * 2 < INT32_MAX) {
+    if (rg_packed_gate_weights_bytes((int)W, (int)H, c.code) > 0) {
       packed = packed_for(w_x, w_a);
       need(packed.device() == c.x.device());
       pk = packed.const_data_ptr();

@@ -188,6 +188,13 @@ static bool mfma_bf16_takes(int bw) {
   return bw >= 128 && bw <= 256 && bw % 8 == 0;
 }
 
+// Head widths the single-launch kernels take: 256, and narrower ones (the
+// paper presets' 176) in slices.  128-wide heads stay with the gate GEMM and
+// the scan, whose outputs they are held to bit for bit.
+static bool single_takes(int bw) {
+  return bw > 128 && bw <= 256 && bw % 8 == 0;
+}
+
 int rg_block_diag_linear(const void* x, const void* w, const void* b, void* y,
                          int64_t M, int H, int bw, int dtype, void* stream) {
   RG_CHECK_DTYPE(dtype);
@@ -439,7 +446,7 @@ size_t rg_recurrent_prefill_split_workspace_bytes(int B, int T, int W, int H) {
 
 #undef RG_WHO
 #define RG_WHO who
-static int recurrent_prefill_impl(const char* who, const void* x,
+static int recurrent_prefill_impl(const char* who, bool narrow, const void* x,
                                   const void* segpos, int segpos_is_i64,
                                   const void* conv_w, const void* conv_b,
                                   const void* w_x, const void* b_x,
@@ -476,10 +483,11 @@ static int recurrent_prefill_impl(const char* who, const void* x,
   RG_CHECK_OPT_PTR(conv_cache_out);
   RG_CHECK_OPT_PTR(gate_branch);
   RG_REQUIRE(y != x, "%s: y must not alias x", who);
-  // The single-launch kernel exists for bf16 with 256-wide heads and
+  // The single-launch kernels exist for bf16 with 256-wide heads (`narrow`, as
+  // rg_recurrent_core calls it: also for narrower ones) and
   // sequences whose byte offsets fit 31 bits; everything else is served by
   // rg_gates_gemm + rg_lru_scan_fused.
-  if (dtype != RG_DTYPE_BF16 || W / H != 256 ||
+  if (dtype != RG_DTYPE_BF16 || !(narrow ? single_takes(W / H) : W / H == 256) ||
       (int64_t)T * W * 2 >= (int64_t)0x7fffffff) {
     return fail(RG_ERR_UNSUPPORTED,
                 "%s: unsupported shape or dtype (needs bf16, W/H == 256, "
@@ -537,7 +545,7 @@ int rg_recurrent_prefill(const void* x, const void* segpos, int segpos_is_i64,
                          const void* a_param, const void* h0, void* y,
                          void* h_last, void* conv_cache_out, int B, int T,
                          int W, int H, int dtype, void* stream) {
-  return recurrent_prefill_impl(__func__, x, segpos, segpos_is_i64, conv_w,
+  return recurrent_prefill_impl(__func__, false, x, segpos, segpos_is_i64, conv_w,
                                 conv_b, w_x, b_x, w_a, b_a, w_packed, a_param,
                                 h0, nullptr, y, h_last, conv_cache_out,
                                 nullptr, 0, false, B, T, W, H, dtype, stream);
@@ -552,7 +560,7 @@ int rg_recurrent_prefill_split(const void* x, const void* segpos,
                                void* h_last, void* conv_cache_out,
                                void* workspace, size_t workspace_bytes, int B,
                                int T, int W, int H, int dtype, void* stream) {
-  return recurrent_prefill_impl(__func__, x, segpos, segpos_is_i64, conv_w,
+  return recurrent_prefill_impl(__func__, false, x, segpos, segpos_is_i64, conv_w,
                                 conv_b, w_x, b_x, w_a, b_a, w_packed, a_param,
                                 h0, nullptr, y, h_last, conv_cache_out,
                                 workspace, workspace_bytes, true, B, T, W, H,
@@ -568,7 +576,7 @@ int rg_recurrent_prefill_gelu_mul(
     int W, int H, int dtype, void* stream) {
   RG_CHECK_PTR(gate_branch);
   RG_REQUIRE(gate_branch != x, "%s: gate_branch must not alias x", __func__);
-  return recurrent_prefill_impl(__func__, x, segpos, segpos_is_i64, conv_w,
+  return recurrent_prefill_impl(__func__, false, x, segpos, segpos_is_i64, conv_w,
                                 conv_b, w_x, b_x, w_a, b_a, w_packed, a_param,
                                 h0, gate_branch, out, h_last, conv_cache_out,
                                 workspace, workspace_bytes, true, B, T, W, H,
@@ -590,7 +598,7 @@ static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
   // three launches' worth of latency otherwise)
   p.small_f32 = dtype == RG_DTYPE_F32 && rg::core_f32_small_serves(B, T, W, H);
   if (p.small_f32) return p;
-  const bool fits = dtype == RG_DTYPE_BF16 && W / H == 256 &&
+  const bool fits = dtype == RG_DTYPE_BF16 && single_takes(W / H) &&
                     (int64_t)T * W * 2 < (int64_t)0x7fffffff;
   const size_t chunk_bytes =
       fits ? rg_recurrent_prefill_split_workspace_bytes(B, T, W, H) : 0;
@@ -605,7 +613,9 @@ static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
   const int64_t pairs = (int64_t)B * H;
   const bool many_short_rows =
       (pairs > 512 && T <= 16) || (pairs > 1024 && T <= 32);
-  p.single = fits && !many_short_rows;
+  // (narrower heads: where the form in slices is ahead of gate GEMM + scan)
+  p.single = fits && !many_short_rows &&
+             (W / H == 256 || rg::prefill_narrow_pays(B, H, T, W));
   if (p.single) {
     p.split_bytes = chunk_bytes;
   } else {
@@ -696,7 +706,7 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
     // the join is part of the kernel's output stage, for rows in chunks too
     // (the launches that write y apply it)
     return recurrent_prefill_impl(
-        __func__, x, segpos, segpos_is_i64, conv_w, conv_b, w_x, b_x, w_a, b_a,
+        __func__, true, x, segpos, segpos_is_i64, conv_w, conv_b, w_x, b_x, w_a, b_a,
         w_packed, a_param, h0, gate_branch, out, h_last, conv_cache_out,
         workspace, workspace_bytes, true, B, T, W, H, dtype, stream);
   } else {
@@ -1242,26 +1252,28 @@ int rg_attention_decode_fused(const void* q, int64_t ldq, const void* k_new,
 }
 
 size_t rg_packed_gate_weights_bytes(int W, int H, int dtype) {
-  if (W <= 0 || H <= 0 || W % H != 0 || dtype != RG_DTYPE_BF16 || W / H != 256)
+  if (W <= 0 || H <= 0 || W % H != 0 || !single_takes(W / H) ||
+      dtype != RG_DTYPE_BF16)
     return 0;
-  return (size_t)2 * H * 256 * 256 * 2;
+  return rg::packed_gate_weights_bytes(W, H);
 }
 
 int rg_pack_gate_weights(const void* w_x, const void* w_a, void* packed, int W,
                          int H, int dtype, void* stream) {
   RG_CHECK_DTYPE(dtype);
   RG_REQUIRE(W > 0 && H > 0 && W % H == 0, "%s: W=%d H=%d", __func__, W, H);
-  if (dtype != RG_DTYPE_BF16 || W / H != 256)
+  if (rg_packed_gate_weights_bytes(W, H, dtype) == 0)
     return fail(RG_ERR_UNSUPPORTED,
-                "%s: needs bf16 and W/H == 256 (dtype=%d W=%d H=%d)", __func__,
-                dtype, W, H);
+                "%s: needs bf16 and heads of 136 .. 256 channels, a multiple "
+                "of 8 (dtype=%d W=%d H=%d)", __func__, dtype, W, H);
   RG_CHECK_PTR(w_x);
   RG_CHECK_PTR(w_a);
   RG_CHECK_PTR(packed);
   RG_REQUIRE(packed != w_x && packed != w_a, "%s: packed must not alias",
              __func__);
-  return launch_status(__func__, rg::launch_pack_gate_weights(
-                                     w_x, w_a, packed, H, (hipStream_t)stream));
+  return launch_status(__func__,
+                       rg::launch_pack_gate_weights(w_x, w_a, packed, W, H,
+                                                    (hipStream_t)stream));
 }
 
 size_t rg_linear_packed_bytes(int N, int K, int gelu_pair) {

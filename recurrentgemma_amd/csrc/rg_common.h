@@ -213,6 +213,28 @@ __device__ __forceinline__ void conv4_dot_x2(
         "v"(w10[0]), "v"(w10[1]), "v"(w32[0]), "v"(w32[1]), "v"(bias[0]),
         "v"(bias[1]));
 }
+// ... of two channels at two rows in a row (o_*: the time pairs that end at the
+// even row, e_*: at the odd one)
+__device__ __forceinline__ void conv4_dot_row_pair(
+    const uint32_t (&o_old)[2], const uint32_t (&o_new)[2],
+    const uint32_t (&e_old)[2], const uint32_t (&e_new)[2],
+    const uint32_t (&w10)[2], const uint32_t (&w32)[2], const float (&bias)[2],
+    float (&even)[2], float (&odd)[2]) {
+  asm("v_dot2_f32_bf16 %0, %4, %12, %16\n\t"
+      "v_dot2_f32_bf16 %1, %5, %13, %17\n\t"
+      "v_dot2_f32_bf16 %2, %8, %12, %16\n\t"
+      "v_dot2_f32_bf16 %3, %9, %13, %17\n\t"
+      "v_dot2_f32_bf16 %0, %6, %14, %0\n\t"
+      "v_dot2_f32_bf16 %1, %7, %15, %1\n\t"
+      "v_dot2_f32_bf16 %2, %10, %14, %2\n\t"
+      "v_dot2_f32_bf16 %3, %11, %15, %3\n\t"
+      "s_nop 2"
+      : "=&v"(even[0]), "=&v"(even[1]), "=&v"(odd[0]), "=&v"(odd[1])
+      : "v"(o_old[0]), "v"(o_old[1]), "v"(o_new[0]), "v"(o_new[1]),
+        "v"(e_old[0]), "v"(e_old[1]), "v"(e_new[0]), "v"(e_new[1]),
+        "v"(w10[0]), "v"(w10[1]), "v"(w32[0]), "v"(w32[1]), "v"(bias[0]),
+        "v"(bias[1]));
+}
 __device__ __forceinline__ void conv4_dot_x4(
     const uint32_t (&p_old)[4], const uint32_t (&p_new)[4],
     const uint32_t (&w10)[4], const uint32_t (&w32)[4], const float (&bias)[4],

@@ -17,28 +17,33 @@ union Frag {
 };
 
 // ---------------------------------------------------------------- decode --
-// Gate weights in the order the MFMA B operand is consumed: for head h, wave
-// w (32 output channels), k-step ks, gate g and lane l the 8 bf16 values
+// Gate weights in the order the MFMA B operand is consumed: for head h, group
+// w of 32 output channels, k-step ks, gate g and lane l the 8 bf16 values
 // w_g[h][16 ks + 8 (l/32) + 0..7][32 w + l%32], 16 bytes per lane, so that a
-// kernel fills its 128 weight registers with 32 coalesced 16-byte loads.
-// One thread per 16-byte group; run once per set of weights.
+// kernel fills its weight registers with coalesced 16-byte loads.  Heads
+// narrower than 256 are padded with zeros to whole groups and to the k-steps
+// their kernel takes.  One thread per 16-byte group; run once per set of
+// weights.
 __global__ void __launch_bounds__(256)
 pack_gate_weights_kernel(const uint16_t* __restrict__ w_x,
                          const uint16_t* __restrict__ w_a,
-                         uint16_t* __restrict__ packed, int H) {
+                         uint16_t* __restrict__ packed, int H, int bw,
+                         int groups, int ksteps) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t total = (int64_t)H * 8 * 16 * 2 * 64;
+  const int64_t total = (int64_t)H * groups * ksteps * 2 * 64;
   if (idx >= total) return;
   const int l = (int)(idx & 63);
   const int g = (int)((idx >> 6) & 1);
-  const int ks = (int)((idx >> 7) & 15);
-  const int w = (int)((idx >> 11) & 7);
-  const int h = (int)(idx >> 14);
-  const uint16_t* src = (g ? w_a : w_x) + (int64_t)h * kBW * kBW +
-                        (int64_t)(16 * ks + 8 * (l >> 5)) * kBW + 32 * w + (l & 31);
+  const int64_t rest = idx >> 7;
+  const int ks = (int)(rest % ksteps);
+  const int w = (int)(rest / ksteps % groups);
+  const int h = (int)(rest / ksteps / groups);
+  const int k0 = 16 * ks + 8 * (l >> 5), n = 32 * w + (l & 31);
+  const uint16_t* src = (g ? w_a : w_x) + (int64_t)h * bw * bw + n;
   Frag f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) f.u[e] = src[(int64_t)e * kBW];
+  for (int e = 0; e < 8; ++e)
+    f.u[e] = n < bw && k0 + e < bw ? src[(int64_t)(k0 + e) * bw] : (uint16_t)0;
   *reinterpret_cast<f32x4*>(packed + idx * 8) = f.q;
 }
 
@@ -315,11 +320,18 @@ __global__ void __launch_bounds__(512) block_step_bf16_kernel(StepArgs p) {
 
 }  // namespace
 
+size_t packed_gate_weights_bytes(int W, int H) {
+  const int bw = W / H;
+  return (size_t)H * ((bw + 31) / 32) * gate_k_steps(bw) * 2 * 1024;
+}
+
 hipError_t launch_pack_gate_weights(const void* w_x, const void* w_a,
-                                    void* packed, int H, hipStream_t s) {
-  const int64_t total = (int64_t)H * 8 * 16 * 2 * 64;
+                                    void* packed, int W, int H, hipStream_t s) {
+  const int64_t total = (int64_t)(packed_gate_weights_bytes(W, H) / 16);
+  const int bw = W / H;
   pack_gate_weights_kernel<<<dim3((unsigned)((total + 255) / 256)), 256, 0, s>>>(
-      (const uint16_t*)w_x, (const uint16_t*)w_a, (uint16_t*)packed, H);
+      (const uint16_t*)w_x, (const uint16_t*)w_a, (uint16_t*)packed, H, bw,
+      (bw + 31) / 32, gate_k_steps(bw));
   return hipGetLastError();
 }
 

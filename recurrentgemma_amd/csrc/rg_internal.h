@@ -249,14 +249,17 @@ void scan_split_plan(int B, int T, int W, int granule, int* chunks,
 int scan_split_granule(int dtype, int W);
 hipError_t launch_block_prefill_bf16(const FusedArgs& a, hipStream_t s);
 hipError_t launch_block_prefill_teams_bf16(const FusedArgs& a, hipStream_t s);
+// the same for heads of 128 .. 256 channels, cut into slices of 64: few (row,
+// head) pairs, short rows, narrower heads (rg_prefill_slices.hip)
+bool prefill_slices_serve(int B, int H, int T, bool joined);  // 256-wide heads
+bool prefill_narrow_pays(int B, int H, int T, int W);         // narrower ones
+hipError_t launch_block_prefill_slices_bf16(const FusedArgs& a, hipStream_t s);
 // float32, 256-wide heads, few rows: conv, gate projections, gates and
 // recurrence in one launch (rg_core_f32.hip)
 bool core_f32_small_serves(int B, int T, int W, int H);
 hipError_t launch_core_f32_small(const FusedArgs& a, hipStream_t s);
 void prefill_chunk_plan(int B, int H, int T, int* chunks, int* tiles_per_chunk);
 hipError_t launch_block_step_bf16(const StepArgs& a, hipStream_t s);
-// bf16 [H,256,256] x 2 -> one buffer of the same total size in MFMA operand
-// order (head, wave, k-step, gate, lane, 8 values).
 // out[i] = a[i] * gelu_tanh(g[i]) over n elements (out may alias a or g).
 hipError_t launch_gelu_mul(const void* a, const void* g, void* out, int64_t n,
                            int dtype, hipStream_t s);
@@ -315,8 +318,12 @@ hipError_t launch_gates_wgrad(const void* x, const void* dgx, const void* dga,
                               void* dwx, void* dwa, void* dbx, void* dba,
                               void* workspace, int64_t M, int W, int H,
                               hipStream_t s);
+// bf16 [H,bw,bw] x 2 -> one buffer in MFMA operand order (head, group of 32
+// channels, k-step, gate, lane, 8 values), zeros beyond bw.
+int gate_k_steps(int bw);
+size_t packed_gate_weights_bytes(int W, int H);
 hipError_t launch_pack_gate_weights(const void* w_x, const void* w_a,
-                                    void* packed, int H, hipStream_t s);
+                                    void* packed, int W, int H, hipStream_t s);
 
 }  // namespace rg
 #endif  // RG_INTERNAL_H_

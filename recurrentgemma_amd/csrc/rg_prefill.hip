@@ -997,10 +997,15 @@ void prefill_chunk_plan(int B, int H, int T, int* chunks, int* tiles_per_chunk) 
 }
 
 hipError_t launch_block_prefill_bf16(const FusedArgs& a, hipStream_t s) {
-  // needs head width 256 and a sequence whose rows fit 31-bit byte offsets
-  // (checked by the caller)
+  // needs a head width that one of the forms takes and a sequence whose rows
+  // fit 31-bit byte offsets (checked by the caller)
   const int64_t blocks = (int64_t)a.B * a.H;
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
+  // narrow heads, few pairs, short rows: heads in slices
+  if (a.W / a.H != 256 ||
+      (a.chunks <= 1 &&
+       prefill_slices_serve(a.B, a.H, a.T, a.gate_branch != nullptr)))
+    return launch_block_prefill_slices_bf16(a, s);
   // with re-laid-out weights: the form with two waves per SIMD
   // (rg_prefill_teams.hip), a tenth to a fifth faster
   if (a.w_packed) return launch_block_prefill_teams_bf16(a, s);

@@ -33,6 +33,7 @@
 
 #include "rg_common.h"
 #include "rg_internal.h"
+#include "rg_weight_frags.h"
 
 namespace rg {
 namespace {
@@ -93,90 +94,6 @@ typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-// out[c] = bias[c] + p_old[c] . w10[c] + p_new[c] . w32[c] for two channels
-// (v_dot2_f32_bf16; its result may be read by an instruction of another kind
-// only three issue slots later).
-__device__ __forceinline__ void conv_dot_row(const uint32_t (&p_old)[2],
-                                             const uint32_t (&p_new)[2],
-                                             const uint32_t (&w10)[2],
-                                             const uint32_t (&w32)[2],
-                                             const float (&bias)[2],
-                                             float (&out)[2]) {
-  asm("v_dot2_f32_bf16 %0, %2, %6, %10\n\t"
-      "v_dot2_f32_bf16 %1, %3, %7, %11\n\t"
-      "v_dot2_f32_bf16 %0, %4, %8, %0\n\t"
-      "v_dot2_f32_bf16 %1, %5, %9, %1\n\t"
-      "s_nop 2"
-      : "=&v"(out[0]), "=&v"(out[1])
-      : "v"(p_old[0]), "v"(p_old[1]), "v"(p_new[0]), "v"(p_new[1]),
-        "v"(w10[0]), "v"(w10[1]), "v"(w32[0]), "v"(w32[1]), "v"(bias[0]),
-        "v"(bias[1]));
-}
-__device__ __forceinline__ void conv_dot_row_pair(
-    const uint32_t (&o_old)[2], const uint32_t (&o_new)[2],
-    const uint32_t (&e_old)[2], const uint32_t (&e_new)[2],
-    const uint32_t (&w10)[2], const uint32_t (&w32)[2], const float (&bias)[2],
-    float (&even)[2], float (&odd)[2]) {
-  asm("v_dot2_f32_bf16 %0, %4, %12, %16\n\t"
-      "v_dot2_f32_bf16 %1, %5, %13, %17\n\t"
-      "v_dot2_f32_bf16 %2, %8, %12, %16\n\t"
-      "v_dot2_f32_bf16 %3, %9, %13, %17\n\t"
-      "v_dot2_f32_bf16 %0, %6, %14, %0\n\t"
-      "v_dot2_f32_bf16 %1, %7, %15, %1\n\t"
-      "v_dot2_f32_bf16 %2, %10, %14, %2\n\t"
-      "v_dot2_f32_bf16 %3, %11, %15, %3\n\t"
-      "s_nop 2"
-      : "=&v"(even[0]), "=&v"(even[1]), "=&v"(odd[0]), "=&v"(odd[1])
-      : "v"(o_old[0]), "v"(o_old[1]), "v"(o_new[0]), "v"(o_new[1]),
-        "v"(e_old[0]), "v"(e_old[1]), "v"(e_new[0]), "v"(e_new[1]),
-        "v"(w10[0]), "v"(w10[1]), "v"(w32[0]), "v"(w32[1]), "v"(bias[0]),
-        "v"(bias[1]));
-}
-
-// The wave's 32 weight fragments (fragment F = 2 k-step + gate, four registers
-// each) live in the accumulation registers a[4F : 4F+3], written and read by
-// inline assembly with the register numbers spelled out.
-#define RG_TFRAG_CASES(X)                                                     \
-  X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13)   \
-  X(14) X(15) X(16) X(17) X(18) X(19) X(20) X(21) X(22) X(23) X(24) X(25)     \
-  X(26) X(27) X(28) X(29) X(30) X(31)
-
-__device__ __forceinline__ void set_weight_frag(int F, f32x4 v) {
-  switch (F) {
-#define RG_SET_CASE(F)                                                   \
-  case F:                                                                \
-    asm volatile("v_accvgpr_write_b32 a[" #F "*4], %0\n\t"               \
-                 "v_accvgpr_write_b32 a[" #F "*4+1], %1\n\t"             \
-                 "v_accvgpr_write_b32 a[" #F "*4+2], %2\n\t"             \
-                 "v_accvgpr_write_b32 a[" #F "*4+3], %3"                  \
-                 :                                                       \
-                 : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3])            \
-                 : "a127");                                              \
-    break;
-    RG_TFRAG_CASES(RG_SET_CASE)
-#undef RG_SET_CASE
-  }
-}
-__device__ __forceinline__ void mfma_weight_frag(int F, bool first,
-                                                 const f32x4& a, f32x16& acc) {
-  switch (F) {
-#define RG_MFMA_CASE(F)                                                        \
-  case F:                                                                      \
-    if (first)                                                                 \
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, a[" #F "*4:" #F "*4+3], 0" \
-                   : "=&v"(acc)                                                \
-                   : "v"(a));                                                  \
-    else                                                                       \
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, a[" #F "*4:" #F            \
-                   "*4+3], %0"                                                 \
-                   : "+v"(acc)                                                 \
-                   : "v"(a));                                                  \
-    break;
-    RG_TFRAG_CASES(RG_MFMA_CASE)
-#undef RG_MFMA_CASE
-  }
 }
 
 __device__ __forceinline__ void phase_barrier() {
@@ -348,7 +265,7 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
 #pragma unroll
     for (int c = 0; c < 2; ++c)
       o[c] = __builtin_amdgcn_alignbit(e[c], cr.e_prev[c], 16);
-    conv_dot_row_pair(cr.o_prev, o, cr.e_prev, e, cw10, cw32, cbias, even, odd);
+    conv4_dot_row_pair(cr.o_prev, o, cr.e_prev, e, cw10, cw32, cbias, even, odd);
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       cr.e_prev[c] = e[c];
@@ -372,7 +289,7 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
       pair_rows(r_prev, r, pt);
       if (i >= 3) {
         float o[2];
-        conv_dot_row(p2, pt, cw10, cw32, cbias, o);
+        conv4_dot_x2(p2, pt, cw10, cw32, cbias, o);
         *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at + (i - 3) * kXcRowBytes) =
             pack_bf16x2(o[0], o[1]);
       }

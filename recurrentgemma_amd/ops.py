@@ -440,7 +440,7 @@ def recurrent_core(x, segment_pos, conv_w, conv_b, w_x, b_x, w_a, b_a, a_param,
             if return_h else None)
   cache = x.new_empty((B, 3, W)) if return_conv_cache else None
   packed = (packed_gate_weights(w_x, w_a)  # cached per weight version
-            if recurrent_prefill_supported(x, H) else None)
+            if x.dtype == torch.bfloat16 else None)
   lib = _lib.lib()
   code = _dtype_code(x)
   need = lib.rg_recurrent_core_workspace_bytes(B, T, W, H, code)

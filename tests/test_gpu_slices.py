@@ -1,0 +1,88 @@
+"""Prefill with a head's channels in slices (csrc/rg_prefill_slices.hip): narrow
+heads, few (row, head) pairs, rows of a few tokens."""
+
+import pytest
+import torch
+
+from oracle import torch_ref as R
+from recurrentgemma_amd import _lib
+from recurrentgemma_amd import ops
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+NAMES = ("conv_w", "conv_b", "w_x", "b_x", "w_a", "b_a", "a_param")
+
+
+@pytest.mark.parametrize("B,T,bw,H,mean_doc", [
+    # edges of the 32-token tiles, of a pass (64 or 128 tokens), one row
+    (1, 1, 176, 2, 5), (1, 31, 256, 1, 5), (1, 32, 176, 1, 40),
+    (1, 33, 256, 2, 7), (1, 64, 176, 2, 9), (1, 65, 176, 2, 30),
+    (1, 128, 256, 1, 60), (1, 129, 256, 2, 3), (2, 97, 176, 3, 1000),
+    # rows of a few tokens, several of them per workgroup and pass
+    (7, 1, 256, 2, 2), (40, 5, 176, 32, 3), (33, 32, 256, 10, 12),
+    (50, 33, 176, 32, 20), (48, 16, 256, 10, -5),
+    # head widths between the presets': padding in k, in channels, in both
+    (2, 70, 136, 2, 20), (2, 70, 168, 3, 20), (3, 150, 184, 2, 50),
+    (3, 150, 200, 1, 50), (2, 70, 248, 3, 20),
+    # long rows, left padding
+    (2, 700, 176, 4, -200), (3, 333, 256, 10, 80)])
+@pytest.mark.parametrize("joined", [False, True])
+def test_prefill_in_slices(B, T, bw, H, mean_doc, joined):
+  W = bw * H
+  p = R.make_params(W, H, torch.bfloat16, seed=21, gate_bias_std=0.4)
+  ws = [p[n].to(DEV) for n in NAMES]
+  g = torch.Generator().manual_seed(22)
+  x = torch.randn(B, T, W, generator=g).bfloat16()
+  gate = torch.randn(B, T, W, generator=g).bfloat16().to(DEV)
+  if mean_doc < 0:
+    pads = torch.randint(0, min(T, -mean_doc) + 1, (B, 1), generator=g)
+    seg = (torch.arange(T)[None] - pads).clamp(min=-1)
+  else:
+    seg = helpers.document_positions(B, T, mean_doc, seed=23)
+  xd, sd = x.to(DEV), seg.to(DEV).to(torch.int32 if B % 2 else torch.int64)
+  y, h, c = ops.recurrent_core(xd, sd, *ws)
+  yo, co = R.widened_recurrent_core(x, seg, p, None)
+  assert helpers.max_rel(y, yo) < 1e-2
+  assert helpers.max_rel(h, co.rg_lru_state) < 2e-3
+  assert torch.equal(c.cpu(), co.conv1d_state)
+  if joined:  # the join inside the kernel: the separate pass, bit for bit
+    yj, hj, cj = ops.recurrent_core(xd, sd, *ws, gate_branch=gate)
+    assert torch.equal(yj, ops.gelu_mul(y, gate))
+    assert torch.equal(hj, h) and torch.equal(cj, c)
+  # a carried-in state: the row in two calls
+  if T > 1 and mean_doc > 0:
+    cut = T // 2
+    tail = sd[:, cut:].contiguous()
+    gates = ops.recurrent_core(xd[:, :cut].contiguous(),
+                               sd[:, :cut].contiguous(), *ws)
+    xc, _ = ops.conv1d_prefill(xd, sd, ws[0], ws[1])
+    whole = ops.recurrent_core(xc, sd, None, None, *ws[2:])
+    part = ops.recurrent_core(xc[:, cut:].contiguous(), tail, None, None,
+                              *ws[2:], h0=gates[1])
+    assert helpers.max_rel(whole[0], yo) < 1e-2
+    assert helpers.max_rel(part[1], h) < 2e-3
+    assert helpers.max_rel(part[0], y[:, cut:]) < 1e-2
+
+
+@pytest.mark.parametrize("B,T,bw,H", [(3, 100, 176, 2), (2, 300, 256, 2),
+                                      (5, 40, 200, 3)])
+def test_slices_without_packed_weights(B, T, bw, H):
+  """w_packed == NULL: the weights fetched from the reference layout, same bits."""
+  W = bw * H
+  p = R.make_params(W, H, torch.bfloat16, seed=31, gate_bias_std=0.4)
+  ws = [p[n].to(DEV) for n in NAMES]
+  g = torch.Generator().manual_seed(32)
+  x = torch.randn(B, T, W, generator=g).bfloat16().to(DEV)
+  seg = helpers.document_positions(B, T, 30, seed=33).to(DEV)
+  y1, h1, c1 = ops.recurrent_core(x, seg, *ws)
+  lib = _lib.lib()
+  assert lib.rg_recurrent_core_workspace_bytes(B, T, W, H, 1) == 0
+  y2, c2 = torch.empty_like(x), x.new_empty(B, 3, W)
+  h2 = torch.empty(B, W, dtype=torch.float32, device=DEV)
+  ptr = lambda t: t.data_ptr()
+  _lib.check(lib.rg_recurrent_core(
+      ptr(x), None, ptr(seg), 1, *[ptr(t) for t in ws[:6]], None, ptr(ws[6]),
+      None, ptr(y2), ptr(h2), ptr(c2), None, 0, B, T, W, H, 1,
+      torch.cuda.current_stream().cuda_stream))
+  assert torch.equal(y1, y2) and torch.equal(h1, h2) and torch.equal(c1, c2)
