@@ -243,6 +243,27 @@ struct RglruBwdArgs {
 };
 hipError_t launch_rglru_backward(const RglruBwdArgs& a, int dtype,
                                  hipStream_t s);
+// One pass over every element, 16 bytes of channels per lane
+// (rg_scan_tiles.hip).
+struct ScanTileArgs {
+  // forward: x, a | gated: x, input gate, recurrence gate (pre-activations)
+  // backward: dy, a, y | gated: dy, x, input gate, recurrence gate, y
+  const void* in[5];
+  const void* flags;     // [B, T] document starts
+  int flag_kind;         // SegKind
+  const void* a_param;   // [W], gated
+  const float* init;     // [B, W] or null: h0 | backward: dh_last
+  const float* h0;       // backward: [B, W] or null
+  void* out[3];          // y | dx, da | dx, d input gate, d recurrence gate
+  float* last;           // [B, W] or null: h_last | dh0
+  float* dlam;           // [B, W], gated backward: each row's share
+  int B, T, W;
+};
+enum ScanTileMode { kTilesFwdPlain, kTilesBwdPlain, kTilesFwdGated, kTilesBwdGated };
+// whether it takes the shape and is the faster form for it
+bool scan_tiles_serve(int B, int T, int W, int dtype, int mode);
+hipError_t launch_scan_tiles(const ScanTileArgs& a, int mode, int dtype,
+                             hipStream_t s);
 void scan_split_plan(int B, int T, int W, int granule, int* chunks,
                      int* t_chunk);
 // Chunk lengths are multiples of this for the kernel that handles (dtype, W).

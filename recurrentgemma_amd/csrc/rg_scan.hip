@@ -900,6 +900,20 @@ int scan_split_granule(int dtype, int W) {
 }
 
 hipError_t launch_lru_scan(const ScanArgs& a, int dtype, hipStream_t s) {
+  if (a.plain && scan_tiles_serve(a.B, a.T, a.W, dtype, kTilesFwdPlain)) {
+    ScanTileArgs t{};
+    t.in[0] = a.x;
+    t.in[1] = a.ga;
+    t.flags = a.segpos;
+    t.flag_kind = a.seg_kind;
+    t.init = a.h0;
+    t.out[0] = a.y;
+    t.last = a.h_last;
+    t.B = a.B;
+    t.T = a.T;
+    t.W = a.W;
+    return launch_scan_tiles(t, kTilesFwdPlain, dtype, s);
+  }
   // Channels per lane: 8 bytes per lane where the width allows it (every row
   // then starts on a vector boundary; base pointers are checked by the
   // caller), with short steps; narrower vectors take longer steps.

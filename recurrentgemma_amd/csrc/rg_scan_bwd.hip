@@ -19,6 +19,8 @@
 // recurrentgemma/jax/scan.py:161-187, from the end); pass 2: the chunk again
 // from its true incoming value, writing dx and da (dy and a are read a second
 // time, mostly from cache).
+// Rows of whole 16-byte vectors take rg_scan_tiles.hip instead; these kernels
+// are left for the other widths.
 #include "rg_common.h"
 #include "rg_internal.h"
 
@@ -417,6 +419,28 @@ static bool two_channels_per_lane(int B, int W) {
 
 hipError_t launch_rglru_backward(const RglruBwdArgs& a, int dtype,
                                  hipStream_t s) {
+  if (scan_tiles_serve(a.B, a.T, a.W, dtype, kTilesBwdGated)) {
+    ScanTileArgs t{};
+    t.in[0] = a.dy;
+    t.in[1] = a.x;
+    t.in[2] = a.gx;
+    t.in[3] = a.ga;
+    t.in[4] = a.y;
+    t.flags = a.reset;
+    t.flag_kind = kSegMaskU8;
+    t.a_param = a.a_param;
+    t.init = a.dh_last;
+    t.h0 = a.h0;
+    t.out[0] = a.dx;
+    t.out[1] = a.dgx;
+    t.out[2] = a.dga;
+    t.last = a.dh0;
+    t.dlam = a.dlam;
+    t.B = a.B;
+    t.T = a.T;
+    t.W = a.W;
+    return launch_scan_tiles(t, kTilesBwdGated, dtype, s);
+  }
   const bool two = two_channels_per_lane(a.B, a.W);
   if (dtype == 0)
     return two ? launch_gates_as<float, 2, false>(a, s)
@@ -427,6 +451,23 @@ hipError_t launch_rglru_backward(const RglruBwdArgs& a, int dtype,
 
 hipError_t launch_linear_scan_backward(const ScanBwdArgs& a, int dtype,
                                        hipStream_t s) {
+  if (scan_tiles_serve(a.B, a.T, a.W, dtype, kTilesBwdPlain)) {
+    ScanTileArgs t{};
+    t.in[0] = a.dy;
+    t.in[1] = a.a;
+    t.in[2] = a.y;
+    t.flags = a.reset;
+    t.flag_kind = kSegMaskU8;
+    t.init = a.dh_last;
+    t.h0 = a.h0;
+    t.out[0] = a.dx;
+    t.out[1] = a.da;
+    t.last = a.dh0;
+    t.B = a.B;
+    t.T = a.T;
+    t.W = a.W;
+    return launch_scan_tiles(t, kTilesBwdPlain, dtype, s);
+  }
   const bool two = two_channels_per_lane(a.B, a.W);
   if (dtype == 0) return two ? launch_as<float, 2>(a, s) : launch_as<float, 1>(a, s);
   return two ? launch_as<uint16_t, 2>(a, s) : launch_as<uint16_t, 1>(a, s);

@@ -1,0 +1,575 @@
+// The linear recurrence and the RG-LRU's gating around it, forward and
+// backward, reading every element once: rnn_scan and RGLRU.forward of a
+// training step (recurrentgemma/torch/layers.py:140-191, 335-360) and what
+// autograd makes of them.
+//
+//   forward   h_t = a'_t h_{t-1} + x_t                      y_t = h_t
+//   backward  g_t = dy_t + u_{t+1},  u_t = a'_t g_t         (from the end, the
+//             dx_t = g_t,  da_t = g_t h_{t-1},  dh0 = u_0    incoming u is dh_last)
+// with a' = a, zeroed at document starts.  Both are first-order recurrences
+// on pairs (coefficient, input): (a', x) forwards, (a', a' dy) backwards.
+//
+// A lane owns 16 bytes of adjacent channels and KL consecutive tokens, a wave
+// eight lanes of channels (128 bytes of a row) by eight groups of tokens, a
+// workgroup of eight waves 64 groups: one step of 64 KL tokens.  Per step
+//   1  every lane reduces its tokens, which stay in registers, to (P, H) per
+//      channel;
+//   2  the 64 pairs of a channel meet in LDS and are scanned by 512 / channels
+//      threads, 64 channels / 8 pairs each, their totals by lane shifts (the
+//      scan operator of recurrentgemma/jax/scan.py:161-187); the state that
+//      comes into every group goes back through LDS;
+//   3  every lane replays its tokens from that state and stores.
+// Rows are asked for as early as the registers allow (see below), so that the
+// memory pipe works while a step computes.
+// The kernels this replaces where it runs (rg_scan.hip, rg_scan_bwd.hip) keep
+// one or two channels per lane: 80 .. 160 workgroups with 2- and 4-byte
+// accesses at B4 W2560, and the backward ones read their inputs twice and
+// evaluated the gates twice.
+#include <type_traits>
+
+#include "rg_common.h"
+#include "rg_internal.h"
+
+namespace rg {
+namespace {
+
+constexpr int kWaves = 8;
+constexpr int kThreads = kWaves * 64;
+constexpr int kLanes = 8;             // lanes side by side along the channels
+constexpr int kGroups = kThreads / kLanes;  // token groups of a step
+
+constexpr int kFwdPlain = kTilesFwdPlain, kBwdPlain = kTilesBwdPlain,
+              kFwdGated = kTilesFwdGated, kBwdGated = kTilesBwdGated;
+// cond ? a : b with both sides computed (the compiler would put the expensive
+// one behind a branch per token, and split the replay into pieces that no load
+// crosses).
+__device__ __forceinline__ float choose(bool cond, float a, float b) {
+  asm("" : "+v"(b));
+  return cond ? a : b;
+}
+
+constexpr int streams_of(int mode) {
+  return mode == kFwdPlain ? 2 : mode == kBwdGated ? 5 : 3;
+}
+
+template <typename T>
+struct Vec;  // 16 bytes of channels
+template <>
+struct Vec<uint16_t> {
+  static constexpr int n = 8;
+  __device__ static void unpack(u32x4 r, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(r[i] << 16);
+      v[2 * i + 1] = __uint_as_float(r[i] & 0xffff0000u);
+    }
+  }
+  // rounded to the stored type (and v replaced by the rounded values)
+  __device__ static u32x4 pack(float (&v)[8]) {
+    u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+    unpack(r, v);
+    return r;
+  }
+};
+template <>
+struct Vec<float> {
+  static constexpr int n = 4;
+  __device__ static void unpack(u32x4 r, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(r[i]);
+  }
+  __device__ static u32x4 pack(float (&v)[4]) {
+    return u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]),
+                 __float_as_uint(v[2]), __float_as_uint(v[3])};
+  }
+};
+
+template <typename T>
+struct TileLds {
+  static constexpr int channels = kLanes * Vec<T>::n;
+  // (two floats of padding: the scanning threads of a wave, whose first groups
+  // lie channels / 8 rows apart, then start on different banks)
+  float pair[kGroups][2 * channels + 2];  // P, H per channel
+  float in[kGroups][channels + 4];        // state before the group
+  float sp[channels];                     // softplus of a_param
+};
+
+template <typename T, int MODE, int KL>
+__global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
+  using V = Vec<T>;
+  using Lds = TileLds<T>;
+  constexpr int N = V::n;
+  constexpr int CH = Lds::channels;
+  constexpr int NS = streams_of(MODE);
+  constexpr bool kBwd = MODE == kBwdPlain || MODE == kBwdGated;
+  constexpr bool kGated = MODE == kFwdGated || MODE == kBwdGated;
+  constexpr bool kFast = sizeof(T) == 2;  // hardware exp2 / rcp, as in the
+                                          // other bf16 kernels
+  constexpr int kSegs = kThreads / CH;    // scanning threads of a channel
+  constexpr int kPer = kGroups / kSegs;   // pairs each of them takes
+  constexpr int kSegLane = 64 / kSegs;    // lanes between neighbours
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  Lds& lds = *reinterpret_cast<Lds*>(lds_raw);
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Workgroups go to the eight XCDs in turn: neighbouring slabs of channels,
+  // which share cache lines where W is no multiple of a slab, to one of them.
+  int block = blockIdx.x;
+  {
+    const int per_xcd = (int)gridDim.x / 8;
+    if (block < 8 * per_xcd) block = (block & 7) * per_xcd + (block >> 3);
+  }
+  const int slabs = (p.W + CH - 1) / CH;
+  const int b = block / slabs;
+  const int c0 = (block - b * slabs) * CH;
+  const int T_len = p.T;
+  const int oct = lane % kLanes, q = lane / kLanes;
+  const int group = wave * (64 / kLanes) + q;
+  const int c = c0 + oct * N;
+  const bool c_ok = c < p.W;  // W % N == 0: all of the vector or nothing
+
+  const uint32_t row_bytes = (uint32_t)p.W * sizeof(T);
+  const uint32_t seq_bytes = (uint32_t)T_len * row_bytes;  // < 2^31 (launcher)
+  __amdgpu_buffer_rsrc_t rs[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    rs[s] = make_rsrc((const char*)p.in[s] + (int64_t)b * seq_bytes, seq_bytes);
+  // which of them is y (read one row before the token): backward only
+  constexpr int kY = MODE == kBwdPlain ? 2 : 4;
+  const uint32_t c_off = (uint32_t)c * sizeof(T);
+
+  // Blocks of KL tokens in the order of the recurrence.
+  const int blocks = (T_len + KL - 1) / KL;
+  const int steps = (blocks + kGroups - 1) / kGroups;
+  auto first_token = [&](int step, int g) {
+    const int o = step * kGroups + g;
+    return (kBwd ? blocks - 1 - o : o) * KL;  // (may lie before or past the row)
+  };
+  // Rows in registers.  What step 1 wants of the backward forms (dy and the
+  // coefficient's stream) and both streams of the plain forward are asked for
+  // a step ahead (`next`), the rest at the top of their own step: they are
+  // used behind the scan.  The gated forward's rows are consumed in step 1 and
+  // reloaded there.
+  u32x4 raw[NS][KL];
+  constexpr bool kReload = MODE == kFwdGated;
+  constexpr int kCoef = MODE == kBwdGated ? 3 : 1;
+  auto is_early = [](int s) {
+    return MODE == kFwdPlain || s == 0 || (kBwd && s == kCoef);
+  };
+  u32x4 next[kReload ? 1 : 2][KL];
+  auto fetch = [&](int s, int t0, int i) {
+    const int t = kBwd && s == kY ? t0 + i - 1 : t0 + i;
+    // (a row before or past the sequence falls outside the descriptor)
+    return __builtin_amdgcn_raw_buffer_load_b128(
+        rs[s], c_ok ? c_off + (uint32_t)t * row_bytes : kBufferOutOfRange, 0, 0);
+  };
+  // Document starts of the wave's 8 KL tokens, one token per lane.
+  uint32_t flag_lo = 1, flag_hi = 0;
+  bool flag_in = false;
+  auto load_flags = [&](int step) {
+    const int lo = first_token(step, kBwd ? wave * 8 + 7 : wave * 8);
+    const int t = lo + lane;
+    flag_in = lane < 8 * KL && t >= 0 && t < T_len;
+    const int64_t at = (int64_t)b * T_len + (flag_in ? t : 0);
+    if (p.flag_kind == kSegMaskU8) {
+      flag_lo = reinterpret_cast<const uint8_t*>(p.flags)[at] == 0;
+      flag_hi = 0;
+    } else if (p.flag_kind == kSegI32) {
+      flag_lo = reinterpret_cast<const uint32_t*>(p.flags)[at];
+      flag_hi = 0;
+    } else {
+      const u32x2 v = reinterpret_cast<const u32x2*>(p.flags)[at];
+      flag_lo = v[0];
+      flag_hi = v[1];
+    }
+  };
+
+  // softplus of a_param, log2 a = -8 log2(e) sp sigmoid(.): read from LDS
+  // twice a step (no registers to keep it in)
+  auto lambda_of = [&](int ch) {  // a_param of the workgroup's channel ch
+    return c0 + ch < p.W ? load_scalar((const T*)p.a_param + c0 + ch) : 0.0f;
+  };
+  if (kGated) {
+    if (tid < CH) lds.sp[tid] = softplus_precise(lambda_of(tid));
+    __syncthreads();
+  }
+  auto read_sp = [&](float (&sp)[N]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < N; e += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(&lds.sp[oct * N + e]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) sp[e + k] = v[k];
+    }
+  };
+  auto sigmoid_of = [](float v) {
+    return kFast ? sigmoid_fast(v) : sigmoid_precise(v);
+  };
+
+  // The scanning thread's channel and its state before the step.
+  const int seg = lane / kSegLane;
+  const int scan_ch = wave * kSegLane + lane % kSegLane;
+  float carry = 0.0f;
+  if (p.init && c0 + scan_ch < p.W)
+    carry = p.init[(int64_t)b * p.W + c0 + scan_ch];
+
+  float lam_acc[MODE == kBwdGated ? N : 1];
+  if (MODE == kBwdGated) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) lam_acc[e] = 0.0f;
+  }
+
+  load_flags(0);
+  {
+    const int t0 = first_token(0, group);
+#pragma unroll
+    for (int i = 0; i < KL; ++i)
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        if (kReload || is_early(s)) raw[s][i] = fetch(s, t0, i);
+  }
+  // (the last step apart: only it can hold the row's end)
+  auto one_step = [&](int step, auto LAST) __attribute__((always_inline)) {
+    constexpr bool more = !decltype(LAST)::value;
+    const int t0 = first_token(step, group);
+    const int next_t0 = first_token(step + 1, group);
+    if (!kReload) {
+#pragma unroll
+      for (int j = 0; j < KL; ++j) {
+        const int i = kBwd ? KL - 1 - j : j;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          if (!is_early(s)) raw[s][i] = fetch(s, t0, i);
+      }
+    }
+    uint32_t starts;
+    {
+      const uint64_t mask = __ballot(flag_in && (flag_lo | flag_hi) == 0u);
+      starts = (uint32_t)(mask >> ((kBwd ? 7 - q : q) * KL)) & ((1u << KL) - 1u);
+    }
+    if (more) {
+      load_flags(step + 1);
+      if (!kReload) {
+#pragma unroll
+        for (int j = 0; j < KL; ++j) {
+          const int i = kBwd ? KL - 1 - j : j;
+          next[0][i] = fetch(0, next_t0, i);
+          next[kReload ? 0 : 1][i] = fetch(kCoef, next_t0, i);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- 1: this lane's tokens as (P, H) ------------------------------------
+    // Kept for the replay: the gated forms' coefficients (the plain ones' are
+    // the rows themselves), the forward's scaled inputs, and the float32
+    // backward's recurrence gates (bf16 has no registers for them, and its
+    // sigmoid is six instructions).
+    constexpr bool kKeepGate = MODE == kBwdGated && !kFast;
+    float coef[kGated ? KL : 1][N];
+    float kept[MODE == kFwdGated || kKeepGate ? KL : 1][N];
+    float P[N], H[N], sp[N];
+    if (kGated) read_sp(sp);
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      P[e] = 1.0f;
+      H[e] = 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < KL; ++j) {
+      const int i = kBwd ? KL - 1 - j : j;
+      const bool start = (starts >> i) & 1u;
+      const bool behind = kBwd && t0 + i >= T_len;  // identity
+      float first[N];
+      V::unpack(raw[0][i], first);
+      float cf[N];  // a'
+      if constexpr (!kGated) {
+        V::unpack(raw[1][i], cf);
+      } else {
+        float ga[N];
+        V::unpack(raw[MODE == kFwdGated ? 2 : 3][i], ga);
+        float gx[N];
+        if (MODE == kFwdGated) V::unpack(raw[1][i], gx);
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+          const float gate_a = sigmoid_of(ga[e]);
+          coef[i][e] = kFast ? __builtin_amdgcn_exp2f(gate_a * ((-8.0f * kLog2e) * sp[e]))
+                             : expf((-8.0f * gate_a) * sp[e]);
+          cf[e] = coef[i][e];
+          if constexpr (kKeepGate) kept[i][e] = gate_a;
+          if constexpr (MODE == kFwdGated) {
+            const float gate_x = sigmoid_of(gx[e]);
+            float m = kFast
+                          ? __builtin_amdgcn_sqrtf(
+                                __builtin_fmaf(-coef[i][e], coef[i][e], 1.0f))
+                          : sqrtf(1.0f - expf(2.0f * ((-8.0f * gate_a) * sp[e])));
+            m = choose(start, 1.0f, m);
+            first[e] = (first[e] * gate_x) * m;
+            kept[i][e] = first[e];
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        cf[e] = choose(start, 0.0f, kBwd ? choose(behind, 1.0f, cf[e]) : cf[e]);
+        if (MODE == kFwdGated) coef[i][e] = cf[e];
+        H[e] = kBwd ? cf[e] * (H[e] + first[e])
+                    : __builtin_fmaf(cf[e], H[e], first[e]);
+        P[e] *= cf[e];
+      }
+      if (kReload && more) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) raw[s][i] = fetch(s, next_t0, i);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < N; e += 2) {
+      // (rows are padded by 8 bytes: 8-byte stores)
+      *reinterpret_cast<f32x2*>(&lds.pair[group][2 * (oct * N + e)]) =
+          f32x2{P[e], H[e]};
+      *reinterpret_cast<f32x2*>(&lds.pair[group][2 * (oct * N + e) + 2]) =
+          f32x2{P[e + 1], H[e + 1]};
+    }
+    lds_barrier();
+
+    // ---- 2: scan over the groups ---------------------------------------------
+    {
+      f32x2 v[kPer];
+#pragma unroll
+      for (int k = 0; k < kPer; ++k)
+        v[k] = *reinterpret_cast<const f32x2*>(
+            &lds.pair[seg * kPer + k][2 * scan_ch]);
+      float sp_ = 1.0f, sh = 0.0f;
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        sh = __builtin_fmaf(v[k][0], sh, v[k][1]);
+        sp_ *= v[k][0];
+      }
+#pragma unroll
+      for (int d = 1; d < kSegs; d *= 2) {
+        const float pp = __shfl_up(sp_, d * kSegLane);
+        const float ph = __shfl_up(sh, d * kSegLane);
+        if (seg >= d) {
+          sh = __builtin_fmaf(sp_, ph, sh);
+          sp_ *= pp;
+        }
+      }
+      float ep = __shfl_up(sp_, kSegLane), eh = __shfl_up(sh, kSegLane);
+      if (seg == 0) {
+        ep = 1.0f;
+        eh = 0.0f;
+      }
+      float s = __builtin_fmaf(ep, carry, eh);
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        lds.in[seg * kPer + k][scan_ch] = s;
+        s = __builtin_fmaf(v[k][0], s, v[k][1]);
+      }
+      carry = __shfl(s, (kSegs - 1) * kSegLane + lane % kSegLane);
+    }
+    lds_barrier();
+
+    // ---- 3: replay ------------------------------------------------------------
+    if (MODE == kBwdGated) {
+      asm volatile("" ::: "memory");
+      read_sp(sp);
+    }
+    float st[N];  // h, or the u that comes in from behind
+#pragma unroll
+    for (int e = 0; e < N; e += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(&lds.in[group][oct * N + e]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) st[e + k] = v[k];
+    }
+#pragma unroll
+    for (int j = 0; j < KL; ++j) {
+      const int i = kBwd ? KL - 1 - j : j;
+      const int t = t0 + i;
+      const bool start = (starts >> i) & 1u;
+      const bool inside = t >= 0 && t < T_len;
+      const uint32_t at = c_ok && inside
+                              ? c_off + (uint32_t)t * row_bytes
+                              : kBufferOutOfRange;
+      auto store = [&](int o, u32x4 v) {
+        buffer_store_16(v, make_rsrc((char*)p.out[o] + (int64_t)b * seq_bytes,
+                                     seq_bytes), at, 0);
+      };
+      // (out of the compiler's sight: it would keep what it unpacked in step 1
+      // in registers instead of the packed rows)
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        if (!kReload) asm volatile("" : "+v"(raw[s][i]));
+      float in0[N], cf[N];
+      if (!kReload) V::unpack(raw[0][i], in0);
+      if constexpr (!kGated) {
+        V::unpack(raw[1][i], cf);
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+          cf[e] = choose(start, 0.0f,
+                         kBwd ? choose(t >= T_len, 1.0f, cf[e]) : cf[e]);
+      }
+      if constexpr (!kBwd) {
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+          st[e] = kGated ? __builtin_fmaf(coef[kGated ? i : 0][e], st[e], kept[kGated ? i : 0][e])
+                         : __builtin_fmaf(cf[e], st[e], in0[e]);
+        float y[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) y[e] = st[e];
+        store(0, V::pack(y));
+        if (!more && p.last && t == T_len - 1 && c_ok) {
+#pragma unroll
+          for (int e = 0; e < N; ++e) p.last[(int64_t)b * p.W + c + e] = st[e];
+        }
+      } else {
+        float hp[N];
+        V::unpack(raw[kY][i], hp);
+        if (i == 0 && t == 0) {  // (t0 is a multiple of KL)
+#pragma unroll
+          for (int e = 0; e < N; ++e)  // h_{-1} in the activation dtype
+            hp[e] = p.h0 && c_ok ? round_act<T>(p.h0[(int64_t)b * p.W + c + e])
+                                 : 0.0f;
+        }
+        float g[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) g[e] = in0[e] + st[e];
+        if constexpr (MODE == kBwdPlain) {
+#pragma unroll
+          for (int e = 0; e < N; ++e) st[e] = cf[e] * g[e];
+          store(0, V::pack(g));
+          float da[N];
+#pragma unroll
+          for (int e = 0; e < N; ++e) da[e] = choose(start, 0.0f, g[e] * hp[e]);
+          store(1, V::pack(da));
+        } else {
+          float x[N], px[N], pa[N], dx[N], dgx[N], dga[N];
+          if (!kKeepGate) V::unpack(raw[3][i], pa);
+          V::unpack(raw[1][i], x);
+          V::unpack(raw[2][i], px);
+#pragma unroll
+          for (int e = 0; e < N; ++e) {
+            const float a = coef[i][e];
+            const float gate_a = kKeepGate ? kept[kKeepGate ? i : 0][e] : sigmoid_of(pa[e]);
+            const float c_t =
+                choose(start, 0.0f, choose(t >= T_len, 1.0f, a));
+            st[e] = c_t * g[e];
+            const float gr = round_act<T>(g[e]);  // the gradient of xn as a tensor
+            const float gate_x = sigmoid_of(px[e]);
+            const float a2 =
+                kFast ? a * a : expf(2.0f * ((-8.0f * gate_a) * sp[e]));
+            const float om = 1.0f - a2;
+            const float m = choose(
+                start, 1.0f, kFast ? __builtin_amdgcn_sqrtf(om) : sqrtf(om));
+            const float d_gated = gr * m;
+            const float d_m = gr * (x[e] * gate_x);
+            const float clipped = fmaxf(4.0f * om, 1e-6f);
+            const float d_om = kFast ? d_m * __builtin_amdgcn_rsqf(clipped)
+                                     : d_m / sqrtf(clipped);
+            const float d_log_a = choose(start || !inside, 0.0f,
+                                         (gr * hp[e]) * a - 2.0f * a2 * d_om);
+            dx[e] = d_gated * gate_x;
+            dgx[e] = (d_gated * x[e]) * (gate_x * (1.0f - gate_x));
+            dga[e] = (-8.0f * sp[e]) * d_log_a * (gate_a * (1.0f - gate_a));
+            lam_acc[e] = __builtin_fmaf(-8.0f * gate_a, d_log_a, lam_acc[e]);
+          }
+          store(0, V::pack(dx));
+          store(1, V::pack(dgx));
+          store(2, V::pack(dga));
+        }
+        if (i == 0 && p.last && t == 0 && c_ok) {  // dh0
+#pragma unroll
+          for (int e = 0; e < N; ++e) p.last[(int64_t)b * p.W + c + e] = st[e];
+        }
+      }
+    }
+    if (more && !kReload) {
+#pragma unroll
+      for (int i = 0; i < KL; ++i) {
+        raw[0][i] = next[0][i];
+        raw[kCoef][i] = next[kReload ? 0 : 1][i];
+      }
+    }
+  };
+  for (int step = 0; step + 1 < steps; ++step) one_step(step, std::false_type{});
+  one_step(steps - 1, std::true_type{});
+
+  if constexpr (MODE == kBwdGated) {
+    // gradient of a_param: this row's share, summed over the groups in order
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < N; e += 4)
+      *reinterpret_cast<f32x4*>(&lds.in[group][oct * N + e]) =
+          f32x4{lam_acc[e], lam_acc[e + 1], lam_acc[e + 2], lam_acc[e + 3]};
+    __syncthreads();
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) sum += lds.in[seg * kPer + k][scan_ch];
+#pragma unroll
+    for (int d = 1; d < kSegs; d *= 2) sum += __shfl_xor(sum, d * kSegLane);
+    if (seg == 0 && c0 + scan_ch < p.W)
+      p.dlam[(int64_t)b * p.W + c0 + scan_ch] =
+          sum * sigmoid_precise(lambda_of(scan_ch));
+  }
+}
+
+template <typename T, int MODE, int KL>
+hipError_t launch_as(const ScanTileArgs& a, hipStream_t s) {
+  constexpr int lds = sizeof(TileLds<T>);
+  static OncePerDevice once;
+  hipError_t e =
+      set_max_dynamic_lds(once, (const void*)scan_tiles_kernel<T, MODE, KL>, lds);
+  if (e != hipSuccess) return e;
+  const int64_t blocks =
+      (int64_t)a.B * ((a.W + TileLds<T>::channels - 1) / TileLds<T>::channels);
+  if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
+  scan_tiles_kernel<T, MODE, KL><<<dim3((unsigned)blocks), kThreads, lds, s>>>(a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool scan_tiles_serve(int B, int T, int W, int dtype, int mode) {
+  const int64_t es = dtype == 0 ? 4 : 2;
+  if ((int64_t)W * es % 16 != 0 ||
+      ((int64_t)T + 1024) * W * es >= (int64_t)0x7fffffff)
+    return false;
+  // The backward forms: everywhere (us, B4 T2048 W2560 bf16: plain 77 -> 40,
+  // gated 140 -> 118; B16 T8192 W4096: 1555 -> 1104, 2067 -> 1710).
+  if (mode == kBwdPlain || mode == kBwdGated) return true;
+  // The forward ones (B4 T2048 W2560 bf16: plain 52 -> 28, gated 83 -> 44), but
+  // for two ranges where rg_scan.hip's kernel is ahead: one or two long rows,
+  // which it cuts into chunks (B1 T16384 W1000: plain 139, here 148; gated from
+  // 4096 tokens on: T8192 105, here 146), and many workgroups on more data than
+  // the last-level cache holds, which it streams with more waves per CU (B16
+  // T1024 W4096: plain 73, here 102, gated 101, here 162).
+  int chunks, t_chunk;
+  scan_split_plan(B, T, W, 64, &chunks, &t_chunk);
+  if (chunks > 1 && T > (mode == kFwdPlain ? 8192 : 4096)) return false;
+  const int64_t slab = dtype == 0 ? TileLds<float>::channels : TileLds<uint16_t>::channels;
+  const int64_t blocks = (int64_t)B * ((W + slab - 1) / slab);
+  return blocks < (dtype == 0 ? 2048 : 1024) ||
+         3 * es * (int64_t)B * T * W < ((int64_t)256 << 20);
+}
+
+hipError_t launch_scan_tiles(const ScanTileArgs& a, int mode, int dtype,
+                             hipStream_t s) {
+  if (dtype == 0) {
+    switch (mode) {
+      case kFwdPlain: return launch_as<float, kFwdPlain, 8>(a, s);
+      case kBwdPlain: return launch_as<float, kBwdPlain, 4>(a, s);
+      case kFwdGated: return launch_as<float, kFwdGated, 4>(a, s);
+      default: return launch_as<float, kBwdGated, 4>(a, s);
+    }
+  }
+  switch (mode) {
+    case kFwdPlain: return launch_as<uint16_t, kFwdPlain, 8>(a, s);
+    case kBwdPlain: return launch_as<uint16_t, kBwdPlain, 4>(a, s);
+    case kFwdGated: return launch_as<uint16_t, kFwdGated, 4>(a, s);
+    default: return launch_as<uint16_t, kBwdGated, 4>(a, s);
+  }
+}
+
+}  // namespace rg
