@@ -15,155 +15,11 @@
 // has to.
 //
 // Plain C++ on torch's and this library's public interfaces; no device code.
-#define PY_SSIZE_T_CLEAN
-#include <Python.h>
-
-#include <ATen/ATen.h>
-#include <ATen/hip/EmptyTensor.h>
-#include <c10/hip/HIPFunctions.h>
-#include <c10/hip/HIPStream.h>
-#include <torch/csrc/autograd/python_variable.h>
-
-#include <memory>
-#include <unordered_map>
-#include <vector>
-
-#include "../../include/rg_lru.h"
+#include "host_call.h"
 
 namespace {
 
-PyObject* g_kernel_error = nullptr;  // _lib.KernelError
-
-struct Fallback {};  // take the general path
-struct Raised {};    // a Python exception is set
-
-using at::Tensor;
-
-// ------------------------------------------------------------- arguments --
-
-// The tensor behind a Python object: exactly torch.Tensor or Parameter (a
-// subclass may stand for something else).
-const Tensor& tensor_of(PyObject* o) {
-  if (!THPVariable_CheckExact(o)) throw Fallback{};
-  return THPVariable_Unpack(o);
-}
-
-int dtype_code(const Tensor& t) {
-  const auto d = t.scalar_type();
-  if (d == at::kBFloat16) return RG_DTYPE_BF16;
-  if (d == at::kFloat) return RG_DTYPE_F32;
-  throw Fallback{};
-}
-
-// What a kernel can take as it lies: dense, aligned, on GPU `device`.
-void* dense(const Tensor& t, at::ScalarType dtype, c10::DeviceIndex device) {
-  if (t.scalar_type() != dtype || !t.is_cuda() ||
-      t.device().index() != device || !t.is_contiguous())
-    throw Fallback{};
-  void* p = const_cast<void*>(t.const_data_ptr());
-  if (reinterpret_cast<uintptr_t>(p) & 15u) throw Fallback{};
-  return p;
-}
-
-void need(bool ok) {
-  if (!ok) throw Fallback{};
-}
-
-bool shape_is(const Tensor& t, std::initializer_list<int64_t> want) {
-  if (t.dim() != (int64_t)want.size()) return false;
-  int i = 0;
-  for (int64_t n : want)
-    if (t.size(i++) != n) return false;
-  return true;
-}
-
-// The first tensor of a call: on the current GPU (no guard is entered here).
-struct Call {
-  const Tensor& x;
-  at::ScalarType dtype;
-  int code;
-  c10::DeviceIndex device;
-  explicit Call(PyObject* o)
-      : x(tensor_of(o)),
-        dtype(x.scalar_type()),
-        code(dtype_code(x)),
-        device(x.device().index()) {
-    need(x.is_cuda() && device == c10::hip::current_device());
-  }
-  void* operator()(PyObject* o) const {  // dense tensor of the call's dtype
-    return dense(tensor_of(o), dtype, device);
-  }
-  void* shaped(PyObject* o, std::initializer_list<int64_t> want) const {
-    const Tensor& t = tensor_of(o);
-    need(shape_is(t, want));
-    return dense(t, dtype, device);
-  }
-  void* f32(PyObject* o, std::initializer_list<int64_t> want) const {
-    const Tensor& t = tensor_of(o);
-    need(shape_is(t, want));
-    return dense(t, at::kFloat, device);
-  }
-  void* positions(PyObject* o, int64_t B, int64_t T, int* is64) const {
-    const Tensor& t = tensor_of(o);
-    need(shape_is(t, {B, T}));
-    *is64 = t.scalar_type() == at::kLong;
-    return dense(t, *is64 ? at::kLong : at::kInt, device);
-  }
-  Tensor empty(at::IntArrayRef shape, at::ScalarType t) const {
-    return at::detail::empty_cuda(
-        shape, t, at::Device(at::kCUDA, device), std::nullopt);
-  }
-  Tensor empty(at::IntArrayRef shape) const { return empty(shape, dtype); }
-  void* stream() const {
-    return c10::hip::getCurrentHIPStream(device).stream();
-  }
-};
-
-// Runs a C-ABI call without the GIL (a full queue blocks the launch).
-template <class F>
-void launch(F&& f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = f();
-  Py_END_ALLOW_THREADS;
-  if (rc == RG_OK) return;
-  PyErr_Format(g_kernel_error ? g_kernel_error : PyExc_RuntimeError,
-               "librg_lru status %d: %s", rc, rg_last_error());
-  throw Raised{};
-}
-
-PyObject* wrap(const Tensor& t) {
-  if (!t.defined()) Py_RETURN_NONE;
-  return THPVariable_Wrap(t);
-}
-
-PyObject* triple(const Tensor& a, const Tensor& b, const Tensor& c) {
-  PyObject* t = PyTuple_New(3);
-  if (!t) throw Raised{};
-  PyTuple_SET_ITEM(t, 0, wrap(a));
-  PyTuple_SET_ITEM(t, 1, wrap(b));
-  PyTuple_SET_ITEM(t, 2, wrap(c));
-  return t;
-}
-
-// Entry points share this: Fallback becomes None, torch's exceptions become
-// Python's.
-template <class F>
-PyObject* guarded(F&& f) {
-  try {
-    return f();
-  } catch (const Fallback&) {
-    Py_RETURN_NONE;
-  } catch (const Raised&) {
-    return nullptr;
-  } catch (const c10::OutOfMemoryError&) {
-    // (the general path asks again and raises torch's own exception)
-    Py_RETURN_NONE;
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
-  }
-}
+using namespace rg_host;
 
 // --------------------------------------------------------------- stamps --
 
@@ -499,6 +355,10 @@ PyMethodDef kMethods[] = {
     {"rows_linear", (PyCFunction)(void*)rows_linear, METH_FASTCALL, ""},
     {"rows_partial", (PyCFunction)(void*)rows_partial, METH_FASTCALL, ""},
     {"remember_packed", (PyCFunction)(void*)remember_packed, METH_FASTCALL, ""},
+    {"linear_scan", (PyCFunction)(void*)linear_scan, METH_FASTCALL, ""},
+    {"train_scan", (PyCFunction)(void*)train_scan, METH_FASTCALL, ""},
+    {"train_rglru", (PyCFunction)(void*)train_rglru, METH_FASTCALL, ""},
+    {"train_block", (PyCFunction)(void*)train_block, METH_FASTCALL, ""},
     {"set_kernel_error", set_kernel_error, METH_O, ""},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -382,5 +382,33 @@ __device__ __forceinline__ float gelu_mul_f32(float av, float gv) {
   return __fmul_rn(av, gelu);
 }
 
+// The backward pass of the join, out = a * gelu_tanh(g) (modules.py:289-291,
+// :627-628, :644), one pass over the three operands:
+//   d_a = dout * gelu(g)
+//   d_g = (dout * a) * gelu'(g),
+//   gelu'(g) = 0.5 (1 + t) + 0.5 g (1 - t^2) sqrt(2/pi) (1 + 3 c1 g^2),
+//   t = tanh(sqrt(2/pi) (g + c1 g^3)).
+// bf16: gelu(g) and dout * a are rounded to bf16 first, as the tensors they
+// are when autograd walks the reference's two ops; each output is rounded
+// once.
+template <bool BF16>
+__device__ __forceinline__ void gelu_mul_backward_one(float dv, float av,
+                                                      float gv, float& da,
+                                                      float& dg) {
+  constexpr float c0 = 0.7978845608028654f;  // sqrt(2/pi)
+  constexpr float c1 = 0.044715f;
+  const float g2 = gv * gv;
+  const float u = c0 * __builtin_fmaf(c1 * g2, gv, gv);
+  const float t = BF16 ? __builtin_fmaf(2.0f, sigmoid_fast(2.0f * u), -1.0f)
+                       : tanhf(u);
+  const float half_g = 0.5f * gv;
+  const float gelu = half_g * (1.0f + t);
+  const float slope = __builtin_fmaf(
+      half_g * __builtin_fmaf(-t, t, 1.0f),
+      c0 * __builtin_fmaf(3.0f * c1, g2, 1.0f), 0.5f * (1.0f + t));
+  da = dv * (BF16 ? round_to_bf16(gelu) : gelu);
+  dg = (BF16 ? round_to_bf16(dv * av) : dv * av) * slope;
+}
+
 }  // namespace rg
 #endif  // RG_COMMON_H_

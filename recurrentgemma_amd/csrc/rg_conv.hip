@@ -349,7 +349,8 @@ __global__ void __launch_bounds__(64)
 conv1d_backward_k4_kernel(const T* __restrict__ dout, const T* __restrict__ x,
                           const void* __restrict__ segpos, int seg_kind,
                           const T* __restrict__ w, T* __restrict__ dx,
-                          float* __restrict__ partial, int T_len, int W,
+                          float* __restrict__ partial,
+                          float* __restrict__ dx_sums, int T_len, int W,
                           int64_t M, int rows) {
   using V = Vec16<T>;
   constexpr int N = V::N;
@@ -370,10 +371,10 @@ conv1d_backward_k4_kernel(const T* __restrict__ dout, const T* __restrict__ x,
   V::unpack(row(w, 1), w1);
   V::unpack(row(w, 2), w2);
   V::unpack(row(w, 3), w3);
-  float h1[N], h2[N], h3[N], d0[N], d1[N], d2[N], d3[N], db[N];
+  float h1[N], h2[N], h3[N], d0[N], d1[N], d2[N], d3[N], db[N], dxs[N];
 #pragma unroll
   for (int e = 0; e < N; ++e)
-    h1[e] = h2[e] = h3[e] = d0[e] = d1[e] = d2[e] = d3[e] = db[e] = 0.0f;
+    h1[e] = h2[e] = h3[e] = d0[e] = d1[e] = d2[e] = d3[e] = db[e] = dxs[e] = 0.0f;
   for (int64_t j = m0 - 3; j < m0; ++j) {
     if (j < 0) continue;
     if (conv_row_starts(segpos, seg_kind, seq, j)) {
@@ -453,9 +454,18 @@ conv1d_backward_k4_kernel(const T* __restrict__ dout, const T* __restrict__ x,
         }
         f1 = f2;
         f2 = f3;
-        *reinterpret_cast<u32x4*>(dx + m * W + c) = V::pack(o);
+        const u32x4 packed = V::pack(o);
+        *reinterpret_cast<u32x4*>(dx + m * W + c) = packed;
+        // (of what is stored: the bias gradient of the layer in front)
+        V::unpack(packed, o);
+#pragma unroll
+        for (int e = 0; e < N; ++e) dxs[e] += o[e];
       }
     }
+  }
+  if (dx_sums != nullptr) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) dx_sums[(int64_t)blockIdx.x * W + c + e] = dxs[e];
   }
   float* outp = partial + (int64_t)blockIdx.x * 5 * W + c;
 #pragma unroll
@@ -599,6 +609,11 @@ int conv1d_backward_chunks(int B, int T) {
   return (int)((M + rows - 1) / rows);
 }
 
+bool conv1d_backward_sums_dx(int B, int T, int W, int K, int dtype) {
+  const int64_t M = (int64_t)B * T;
+  return dtype == 0 ? conv_k4_fits<float>(K, W, M) : conv_k4_fits<uint16_t>(K, W, M);
+}
+
 hipError_t launch_conv1d_backward(const ConvBwdArgs& a, int dtype,
                                   hipStream_t s) {
   const int64_t M = (int64_t)a.B * a.T;
@@ -614,15 +629,17 @@ hipError_t launch_conv1d_backward(const ConvBwdArgs& a, int dtype,
       conv1d_backward_k4_kernel<float>
           <<<dim3((unsigned)chunks, (unsigned)((a.W / 4 + 63) / 64)), 64, 0, s>>>(
               (const float*)a.dout, (const float*)a.x, a.segpos, a.seg_kind,
-              (const float*)a.w, (float*)a.dx, a.partial, a.T, a.W, M, rows);
+              (const float*)a.w, (float*)a.dx, a.partial, a.dx_sums, a.T, a.W, M,
+              rows);
     else
       conv1d_backward_k4_kernel<uint16_t>
           <<<dim3((unsigned)chunks, (unsigned)((a.W / 8 + 63) / 64)), 64, 0, s>>>(
               (const uint16_t*)a.dout, (const uint16_t*)a.x, a.segpos,
-              a.seg_kind, (const uint16_t*)a.w, (uint16_t*)a.dx, a.partial, a.T,
-              a.W, M, rows);
+              a.seg_kind, (const uint16_t*)a.w, (uint16_t*)a.dx, a.partial,
+              a.dx_sums, a.T, a.W, M, rows);
     return hipGetLastError();
   }
+  if (a.dx_sums != nullptr) return hipErrorInvalidValue;
   const dim3 grid((unsigned)chunks, (unsigned)cblocks);
   if (dtype == 0)
     conv1d_backward_kernel<float><<<grid, 256, 0, s>>>(

@@ -199,9 +199,12 @@ struct ConvBwdArgs {
   const void* w;     // [K, W]
   void* dx;          // [B, T, W]
   float* partial;    // [conv1d_backward_chunks(B, T)][K + 1][W]
+  float* dx_sums;    // or null: [chunks][W], each chunk's column sums of dx (only
+                     // where conv1d_backward_sums_dx)
   int B, T, W, K;
 };
 int conv1d_backward_chunks(int B, int T);
+bool conv1d_backward_sums_dx(int B, int T, int W, int K, int dtype);
 hipError_t launch_conv1d_backward(const ConvBwdArgs& a, int dtype,
                                   hipStream_t s);
 hipError_t launch_gemm_generic(const GemmArgs& a, int dtype, hipStream_t s);
@@ -252,11 +255,15 @@ struct ScanTileArgs {
   const void* flags;     // [B, T] document starts
   int flag_kind;         // SegKind
   const void* a_param;   // [W], gated
+  const void* bias[2];   // gated float32: [W] or null, added to the input and
+                         // recurrence gates' pre-activations
   const float* init;     // [B, W] or null: h0 | backward: dh_last
   const float* h0;       // backward: [B, W] or null
   void* out[3];          // y | dx, da | dx, d input gate, d recurrence gate
   float* last;           // [B, W] or null: h_last | dh0
   float* dlam;           // [B, W], gated backward: each row's share
+  float* dbias;          // gated float32 backward, or null: [2][B, W], each
+                         // row's sums of the gates' gradients
   int B, T, W;
 };
 enum ScanTileMode { kTilesFwdPlain, kTilesBwdPlain, kTilesFwdGated, kTilesBwdGated };
@@ -332,6 +339,30 @@ hipError_t launch_rms_norm_partial(const float* sums, int slices,
 // out[0] = shader cycles, out[1] = 10 ns ticks that `iters` rounds of a short
 // dependent instruction chain took (rg_elementwise.hip)
 hipError_t launch_clock_probe(uint64_t* out, int iters, hipStream_t s);
+// rg_train.hip: the rest of a training step's backward pass.
+// dx += dgx W_x^T + dga W_a^T per head (bf16, 256-wide heads)
+hipError_t launch_gates_dgrad(const void* dgx, const void* dga, const void* w_x,
+                              const void* w_a, void* dx, int64_t M, int W, int H,
+                              hipStream_t s);
+// rows per partial sum of the column sums below
+constexpr int kColSumRows = 64;
+// partial[ceil(M / kColSumRows)][W] of in [M, W] (W a multiple of 16 bytes)
+hipError_t launch_col_sums(const void* in, float* partial, int64_t M, int W,
+                           int dtype, hipStream_t s);
+// launch_gelu_mul_backward and the column sums of d_g in one pass
+hipError_t launch_gelu_mul_backward_sums(const void* dout, const void* a,
+                                         const void* g, void* d_a, void* d_g,
+                                         float* partial, int64_t M, int W,
+                                         int dtype, hipStream_t s);
+// out[n] = sum over rows of in[row * ld + n], rounded once; several at a time
+struct SumTask {
+  const float* in;
+  int rows, n, ld;
+  void* out;
+};
+constexpr int kMaxSumTasks = 8;
+hipError_t launch_sum_rows(const SumTask* tasks, int count, int dtype,
+                           hipStream_t s);
 // rg_gates_wgrad.hip: weight and bias gradients of both gate projections
 bool gates_wgrad_serves(int64_t M, int W, int H);
 size_t gates_wgrad_workspace_bytes(int64_t M, int W, int H);

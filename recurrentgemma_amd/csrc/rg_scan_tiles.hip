@@ -94,6 +94,7 @@ struct TileLds {
   float pair[kGroups][2 * channels + 2];  // P, H per channel
   float in[kGroups][channels + 4];        // state before the group
   float sp[channels];                     // softplus of a_param
+  float bias[2][channels];                // float32: of the gate projections
 };
 
 template <typename T, int MODE, int KL>
@@ -107,6 +108,7 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
   constexpr bool kGated = MODE == kFwdGated || MODE == kBwdGated;
   constexpr bool kFast = sizeof(T) == 2;  // hardware exp2 / rcp, as in the
                                           // other bf16 kernels
+  constexpr bool kBias = kGated && !kFast;
   constexpr int kSegs = kThreads / CH;    // scanning threads of a channel
   constexpr int kPer = kGroups / kSegs;   // pairs each of them takes
   constexpr int kSegLane = 64 / kSegs;    // lanes between neighbours
@@ -194,15 +196,36 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
     return c0 + ch < p.W ? load_scalar((const T*)p.a_param + c0 + ch) : 0.0f;
   };
   if (kGated) {
-    if (tid < CH) lds.sp[tid] = softplus_precise(lambda_of(tid));
+    if (tid < CH) {
+      lds.sp[tid] = softplus_precise(lambda_of(tid));
+      if (kBias) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          lds.bias[g][tid] = p.bias[g] && c0 + tid < p.W
+                                 ? load_scalar((const T*)p.bias[g] + c0 + tid)
+                                 : 0.0f;
+      }
+    }
     __syncthreads();
   }
-  auto read_sp = [&](float (&sp)[N]) __attribute__((always_inline)) {
+  auto read_row = [&](const float* row, float (&v)[N]) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < N; e += 4) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(&lds.sp[oct * N + e]);
+      const f32x4 r = *reinterpret_cast<const f32x4*>(row + oct * N + e);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) sp[e + k] = v[k];
+      for (int k = 0; k < 4; ++k) v[e + k] = r[k];
+    }
+  };
+  auto read_sp = [&](float (&sp)[N]) __attribute__((always_inline)) {
+    read_row(lds.sp, sp);
+  };
+  // a gate's pre-activations (0: input, 1: recurrence), the bias included
+  auto add_bias = [&](int g, float (&v)[N]) __attribute__((always_inline)) {
+    if constexpr (kBias) {
+      float b_[N];
+      read_row(lds.bias[g], b_);
+#pragma unroll
+      for (int e = 0; e < N; ++e) v[e] += b_[e];
     }
   };
   auto sigmoid_of = [](float v) {
@@ -217,9 +240,17 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
     carry = p.init[(int64_t)b * p.W + c0 + scan_ch];
 
   float lam_acc[MODE == kBwdGated ? N : 1];
+  // float32: also the sums of the gates' gradients (bf16 has no registers for
+  // them, and its weight gradients' kernel forms them)
+  constexpr bool kBiasGrads = MODE == kBwdGated && kBias;
+  float bias_acc[2][kBiasGrads ? N : 1];
   if (MODE == kBwdGated) {
 #pragma unroll
     for (int e = 0; e < N; ++e) lam_acc[e] = 0.0f;
+  }
+  if (kBiasGrads) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) bias_acc[0][e] = bias_acc[1][e] = 0.0f;
   }
 
   load_flags(0);
@@ -291,8 +322,12 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
       } else {
         float ga[N];
         V::unpack(raw[MODE == kFwdGated ? 2 : 3][i], ga);
+        add_bias(1, ga);
         float gx[N];
-        if (MODE == kFwdGated) V::unpack(raw[1][i], gx);
+        if (MODE == kFwdGated) {
+          V::unpack(raw[1][i], gx);
+          add_bias(0, gx);
+        }
 #pragma unroll
         for (int e = 0; e < N; ++e) {
           const float gate_a = sigmoid_of(ga[e]);
@@ -449,6 +484,7 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
           if (!kKeepGate) V::unpack(raw[3][i], pa);
           V::unpack(raw[1][i], x);
           V::unpack(raw[2][i], px);
+          add_bias(0, px);
 #pragma unroll
           for (int e = 0; e < N; ++e) {
             const float a = coef[i][e];
@@ -474,6 +510,10 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
             dgx[e] = (d_gated * x[e]) * (gate_x * (1.0f - gate_x));
             dga[e] = (-8.0f * sp[e]) * d_log_a * (gate_a * (1.0f - gate_a));
             lam_acc[e] = __builtin_fmaf(-8.0f * gate_a, d_log_a, lam_acc[e]);
+            if constexpr (kBiasGrads) {  // (zeros behind the row's end)
+              bias_acc[0][e] += dgx[e];
+              bias_acc[1][e] += dga[e];
+            }
           }
           store(0, V::pack(dx));
           store(1, V::pack(dgx));
@@ -497,21 +537,34 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
   one_step(steps - 1, std::true_type{});
 
   if constexpr (MODE == kBwdGated) {
-    // gradient of a_param: this row's share, summed over the groups in order
-    __syncthreads();
+    // sums over the row: over the groups in order
+    auto total = [&](const float (&v)[N]) __attribute__((always_inline)) {
+      __syncthreads();
 #pragma unroll
-    for (int e = 0; e < N; e += 4)
-      *reinterpret_cast<f32x4*>(&lds.in[group][oct * N + e]) =
-          f32x4{lam_acc[e], lam_acc[e + 1], lam_acc[e + 2], lam_acc[e + 3]};
-    __syncthreads();
-    float sum = 0.0f;
+      for (int e = 0; e < N; e += 4)
+        *reinterpret_cast<f32x4*>(&lds.in[group][oct * N + e]) =
+            f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
+      __syncthreads();
+      float sum = 0.0f;
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) sum += lds.in[seg * kPer + k][scan_ch];
+      for (int k = 0; k < kPer; ++k) sum += lds.in[seg * kPer + k][scan_ch];
 #pragma unroll
-    for (int d = 1; d < kSegs; d *= 2) sum += __shfl_xor(sum, d * kSegLane);
-    if (seg == 0 && c0 + scan_ch < p.W)
-      p.dlam[(int64_t)b * p.W + c0 + scan_ch] =
-          sum * sigmoid_precise(lambda_of(scan_ch));
+      for (int d = 1; d < kSegs; d *= 2) sum += __shfl_xor(sum, d * kSegLane);
+      return sum;
+    };
+    const bool writes = seg == 0 && c0 + scan_ch < p.W;
+    const int64_t at = (int64_t)b * p.W + c0 + scan_ch;
+    const float lam = total(lam_acc);
+    if (writes) p.dlam[at] = lam * sigmoid_precise(lambda_of(scan_ch));
+    if constexpr (kBiasGrads) {
+      if (p.dbias != nullptr) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          const float sum = total(bias_acc[g]);
+          if (writes) p.dbias[(int64_t)g * p.B * p.W + at] = sum;
+        }
+      }
+    }
   }
 }
 

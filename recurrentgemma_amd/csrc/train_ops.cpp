@@ -1,0 +1,617 @@
+// The differentiable calls (training.differentiable()) as native autograd
+// functions: the bare recurrence, the RG-LRU, and the whole recurrent block.
+//
+// One training step of the block through one Python autograd function per
+// operator is 26 to 60 launches and about as many allocations and interpreter
+// rounds; float32 RG-LRU at B3 T1001 W2560 spent 640 us of host time on 560 us
+// of kernels.  As one function per direction the passes in between can also be
+// joined: bias gradients come out of the kernels that write or read the tensor
+// anyway, input gradients accumulate where they are, and the reductions left
+// share one launch.
+//
+// As in host_ops.cpp each entry serves the ordinary case and answers None
+// otherwise; training.py then takes the general path.
+#include "host_call.h"
+
+#include <ATen/autocast_mode.h>
+#include <torch/csrc/autograd/custom_function.h>
+
+#include "rg_internal.h"
+
+namespace rg_host {
+namespace {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+// (an absent last argument is no input edge: the indices before it stay)
+using OptTensor = std::optional<Tensor>;
+
+// Raised without the GIL, also on autograd's threads; `guarded` makes it the
+// package's exception.
+void check(int rc) {
+  if (rc != RG_OK)
+    throw KernelFailure("librg_lru status " + std::to_string(rc) + ": " +
+                        rg_last_error());
+}
+void check_hip(hipError_t e) {
+  if (e != hipSuccess)
+    throw KernelFailure(std::string("librg_lru launch: ") + hipGetErrorString(e));
+}
+
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+Tensor empty(at::IntArrayRef shape, at::ScalarType t, const Tensor& like) {
+  return at::detail::empty_cuda(shape, t, like.device(), std::nullopt);
+}
+Tensor empty(at::IntArrayRef shape, const Tensor& like) {
+  return empty(shape, like.scalar_type(), like);
+}
+const void* in(const Tensor& t) {
+  return t.defined() ? t.const_data_ptr() : nullptr;
+}
+void* out(const Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
+
+// A gradient from elsewhere in the graph as the kernels take it.
+Tensor dense_grad(const Tensor& t, at::ScalarType dtype) {
+  if (t.scalar_type() == dtype && t.is_contiguous() &&
+      !(reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u))
+    return t;
+  return t.to(dtype).clone(at::MemoryFormat::Contiguous);
+}
+
+struct Dims {
+  int64_t B, T, W;
+  int code;
+  hipStream_t stream;
+  explicit Dims(const Tensor& x)
+      : B(x.size(0)),
+        T(x.size(1)),
+        W(x.size(2)),
+        code(dtype_code(x)),
+        stream(c10::hip::getCurrentHIPStream(x.device().index()).stream()) {}
+  int64_t M() const { return B * T; }
+};
+int seg_kind(const Tensor& pos) { return pos.scalar_type() == at::kLong ? 1 : 0; }
+
+// ---------------------------------------------------------- bare recurrence --
+
+void scan_forward(const Tensor& x, const Tensor& a, const Tensor& reset,
+                  const Tensor& h0, const Tensor& y, const Tensor& h) {
+  const Dims d(x);
+  const size_t bytes =
+      rg_scan_split_workspace_bytes((int)d.B, (int)d.T, (int)d.W);
+  Tensor ws;
+  if (bytes) ws = empty({(int64_t)bytes}, at::kByte, x);
+  check(bytes ? rg_linear_scan_split(in(x), in(a), in(reset), in(h0), out(y),
+                                     out(h), out(ws), bytes, (int)d.B, (int)d.T,
+                                     (int)d.W, d.code, d.stream)
+              : rg_linear_scan(in(x), in(a), in(reset), in(h0), out(y), out(h),
+                               (int)d.B, (int)d.T, (int)d.W, d.code, d.stream));
+}
+
+struct Scan : Function<Scan> {
+  static variable_list forward(AutogradContext* ctx, Tensor x, Tensor a,
+                               Tensor reset, OptTensor h0_) {
+    const Tensor h0 = h0_.value_or(Tensor());
+    ctx->set_materialize_grads(false);
+    Tensor y = empty(x.sizes(), x);
+    Tensor h = empty({x.size(0), x.size(2)}, at::kFloat, x);
+    scan_forward(x, a, reset, h0, y, h);
+    ctx->save_for_backward({a, reset, y, h0});
+    return {y, h};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    at::AutoGradMode off(false);
+    auto saved = ctx->get_saved_variables();
+    const Tensor &a = saved[0], &reset = saved[1], &y = saved[2], &h0 = saved[3];
+    const Dims d(y);
+    Tensor dy = grads[0].defined() ? dense_grad(grads[0], y.scalar_type())
+                                   : at::zeros_like(y);
+    Tensor dh;
+    if (grads[1].defined()) dh = dense_grad(grads[1], at::kFloat);
+    Tensor dx = empty(y.sizes(), y), da = empty(y.sizes(), y), dh0;
+    if (h0.defined()) dh0 = empty(h0.sizes(), h0);
+    check(rg_linear_scan_backward(in(dy), in(a), in(reset), in(y), in(h0), in(dh),
+                                  out(dx), out(da), out(dh0), (int)d.B, (int)d.T,
+                                  (int)d.W, d.code, d.stream));
+    return {dx, da, Tensor(), dh0};
+  }
+};
+
+// ------------------------------------------------------------------ RG-LRU --
+
+struct GateWeights {
+  Tensor a_param, w_x, b_x, w_a, b_a;
+};
+
+// Where both directions of the recurrence run on the one-pass kernels, they
+// take the document starts from the positions themselves and (float32) add
+// the gates' biases.
+bool on_tiles(const Dims& d) {
+  return rg::scan_tiles_serve((int)d.B, (int)d.T, (int)d.W, d.code,
+                              rg::kTilesFwdGated) &&
+         rg::scan_tiles_serve((int)d.B, (int)d.T, (int)d.W, d.code,
+                              rg::kTilesBwdGated);
+}
+
+// [M, W] as a batch of heads [H, M, bw], no copy
+Tensor by_head(const Tensor& t, int64_t H) {
+  const int64_t bw = t.size(-1) / H;
+  return t.view({-1, H, bw}).transpose(0, 1);
+}
+
+void gated_forward(const Tensor& x, const Tensor& pos, const GateWeights& g,
+                   const Tensor& h0, const Tensor& gx, const Tensor& ga,
+                   const Tensor& y, const Tensor& h) {
+  const Dims d(x);
+  const int64_t H = g.w_x.size(0);
+  const bool tiles = on_tiles(d);
+  const bool f32 = d.code == RG_DTYPE_F32;
+  if (f32) {
+    // the library's batched products, on strided views: no permuted copies
+    Tensor xs = by_head(x, H), gxs = by_head(gx, H), gas = by_head(ga, H);
+    at::bmm_out(gxs, xs, g.w_x);
+    at::bmm_out(gas, xs, g.w_a);
+    if (!tiles) {
+      gx.view({-1, d.W}).add_(g.b_x.view({1, d.W}));
+      ga.view({-1, d.W}).add_(g.b_a.view({1, d.W}));
+    }
+  } else {
+    check(rg_gates_gemm(in(x), 0, nullptr, 0, nullptr, nullptr, in(g.w_x),
+                        in(g.b_x), in(g.w_a), in(g.b_a), out(gx), out(ga),
+                        (int)d.B, (int)d.T, (int)d.W, (int)H, d.code, d.stream));
+  }
+  if (tiles) {
+    rg::ScanTileArgs t{};
+    t.in[0] = in(x);
+    t.in[1] = in(gx);
+    t.in[2] = in(ga);
+    t.flags = in(pos);
+    t.flag_kind = seg_kind(pos);
+    t.a_param = in(g.a_param);
+    if (f32) {
+      t.bias[0] = in(g.b_x);
+      t.bias[1] = in(g.b_a);
+    }
+    t.init = (const float*)in(h0);
+    t.out[0] = out(y);
+    t.last = (float*)out(h);
+    t.B = (int)d.B;
+    t.T = (int)d.T;
+    t.W = (int)d.W;
+    check_hip(rg::launch_scan_tiles(t, rg::kTilesFwdGated, d.code, d.stream));
+    return;
+  }
+  const size_t bytes =
+      rg_scan_split_workspace_bytes((int)d.B, (int)d.T, (int)d.W);
+  Tensor ws;
+  if (bytes) ws = empty({(int64_t)bytes}, at::kByte, x);
+  check(bytes
+            ? rg_lru_scan_fused_split(
+                  in(x), 0, nullptr, nullptr, in(gx), in(ga), in(g.a_param),
+                  in(pos), seg_kind(pos), in(h0), out(y), out(h), nullptr, out(ws),
+                  bytes, (int)d.B, (int)d.T, (int)d.W, d.code, d.stream)
+            : rg_lru_scan_fused(in(x), 0, nullptr, nullptr, in(gx), in(ga),
+                                in(g.a_param), in(pos), seg_kind(pos), in(h0),
+                                out(y), out(h), nullptr, (int)d.B, (int)d.T,
+                                (int)d.W, d.code, d.stream));
+}
+
+struct GateNeeds {
+  bool w_x, b_x, w_a, b_a;
+};
+
+// The reductions over rows that a backward pass ends with, in one launch.
+struct Sums {
+  rg::SumTask tasks[rg::kMaxSumTasks];
+  int count = 0;
+  std::vector<Tensor> keep;
+  Tensor add(const Tensor& partial, int64_t offset, int64_t rows, int64_t n,
+             int64_t ld, at::IntArrayRef shape, const Tensor& like) {
+    if (count == rg::kMaxSumTasks) throw KernelFailure("too many row sums");
+    Tensor sum = empty(shape, like);
+    tasks[count++] = {(const float*)in(partial) + offset, (int)rows, (int)n,
+                      (int)ld, out(sum)};
+    keep.push_back(partial);
+    return sum;
+  }
+  void launch(const Dims& d) {
+    if (count) check_hip(rg::launch_sum_rows(tasks, count, d.code, d.stream));
+  }
+};
+
+struct GatedGrads {
+  Tensor dx, dlam, dw_x, db_x, dw_a, db_a, dh0;
+};
+
+GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
+                          const Tensor& pos, const GateWeights& g,
+                          const Tensor& gx, const Tensor& ga, const Tensor& y,
+                          const Tensor& h0, const GateNeeds& need_, Sums& sums) {
+  const Dims d(x);
+  const int64_t H = g.w_x.size(0), bw = d.W / H;
+  const bool f32 = d.code == RG_DTYPE_F32;
+  GatedGrads r;
+  r.dx = empty(x.sizes(), x);
+  Tensor dgx = empty(x.sizes(), x), dga = empty(x.sizes(), x);
+  Tensor lam_rows = empty({d.B, d.W}, at::kFloat, x), bias_rows;
+  if (h0.defined()) r.dh0 = empty(h0.sizes(), h0);
+  const bool tiles = on_tiles(d);
+  if (tiles) {
+    rg::ScanTileArgs t{};
+    t.in[0] = in(dy);
+    t.in[1] = in(x);
+    t.in[2] = in(gx);
+    t.in[3] = in(ga);
+    t.in[4] = in(y);
+    t.flags = in(pos);
+    t.flag_kind = seg_kind(pos);
+    t.a_param = in(g.a_param);
+    if (f32) {
+      t.bias[0] = in(g.b_x);
+      t.bias[1] = in(g.b_a);
+      bias_rows = empty({2, d.B, d.W}, at::kFloat, x);
+      t.dbias = (float*)out(bias_rows);
+    }
+    t.init = (const float*)in(dh);
+    t.h0 = (const float*)in(h0);
+    t.out[0] = out(r.dx);
+    t.out[1] = out(dgx);
+    t.out[2] = out(dga);
+    t.last = (float*)out(r.dh0);
+    t.dlam = (float*)out(lam_rows);
+    t.B = (int)d.B;
+    t.T = (int)d.T;
+    t.W = (int)d.W;
+    check_hip(rg::launch_scan_tiles(t, rg::kTilesBwdGated, d.code, d.stream));
+  } else {
+    Tensor reset = at::eq(pos, 0);
+    check(rg_rglru_backward(in(dy), in(x), in(gx), in(ga), in(g.a_param),
+                            in(reset), in(y), in(h0), in(dh), out(r.dx), out(dgx),
+                            out(dga), (float*)out(lam_rows), out(r.dh0), (int)d.B,
+                            (int)d.T, (int)d.W, d.code, d.stream));
+  }
+  r.dlam = sums.add(lam_rows, 0, d.B, d.W, d.W, {d.W}, x);
+  if (f32) {
+    Tensor xs = by_head(x, H), dxs = by_head(r.dx, H);
+    Tensor dgs[2] = {by_head(dgx, H), by_head(dga, H)};
+    const Tensor* w[2] = {&g.w_x, &g.w_a};
+    Tensor* dw[2] = {&r.dw_x, &r.dw_a};
+    Tensor* db[2] = {&r.db_x, &r.db_a};
+    const bool needs_w[2] = {need_.w_x, need_.w_a};
+    const bool needs_b[2] = {need_.b_x, need_.b_a};
+    for (int i = 0; i < 2; ++i) {
+      // added to the recurrence's share where it lies
+      at::baddbmm_out(dxs, dxs, dgs[i], w[i]->transpose(1, 2), 1, 1);
+      if (needs_w[i]) *dw[i] = at::bmm(xs.transpose(1, 2), dgs[i]);
+      if (!needs_b[i]) continue;
+      if (tiles)
+        *db[i] = sums.add(bias_rows, i * d.B * d.W, d.B, d.W, d.W, {H, bw}, x);
+      else
+        *db[i] = (i ? dga : dgx).view({-1, H, bw}).sum(0);
+    }
+    return r;
+  }
+  if (need_.w_x || need_.w_a || need_.b_x || need_.b_a) {
+    r.dw_x = empty({H, bw, bw}, x);
+    r.dw_a = empty({H, bw, bw}, x);
+    if (need_.b_x || need_.b_a) {
+      r.db_x = empty({H, bw}, x);
+      r.db_a = empty({H, bw}, x);
+    }
+    const size_t bytes =
+        rg_gates_weight_grads_workspace_bytes(d.M(), (int)d.W, (int)H);
+    Tensor ws = empty({(int64_t)bytes}, at::kByte, x);
+    check(rg_gates_weight_grads(in(x), in(dgx), in(dga), out(r.dw_x), out(r.dw_a),
+                                out(r.db_x), out(r.db_a), out(ws), bytes, d.M(),
+                                (int)d.W, (int)H, d.code, d.stream));
+  }
+  check_hip(rg::launch_gates_dgrad(in(dgx), in(dga), in(g.w_x), in(g.w_a),
+                                   out(r.dx), d.M(), (int)d.W, (int)H, d.stream));
+  return r;
+}
+
+struct Rglru : Function<Rglru> {
+  static variable_list forward(AutogradContext* ctx, Tensor x, Tensor pos,
+                               Tensor a_param, Tensor w_x, Tensor b_x, Tensor w_a,
+                               Tensor b_a, OptTensor h0_) {
+    const Tensor h0 = h0_.value_or(Tensor());
+    ctx->set_materialize_grads(false);
+    Tensor gx = empty(x.sizes(), x), ga = empty(x.sizes(), x);
+    Tensor y = empty(x.sizes(), x);
+    Tensor h = empty({x.size(0), x.size(2)}, at::kFloat, x);
+    gated_forward(x, pos, {a_param, w_x, b_x, w_a, b_a}, h0, gx, ga, y, h);
+    ctx->save_for_backward({x, pos, a_param, w_x, b_x, w_a, b_a, h0, gx, ga, y});
+    return {y, h};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    at::AutoGradMode off(false);
+    auto s = ctx->get_saved_variables();
+    const Tensor &x = s[0], &y = s[10];
+    Tensor dy = grads[0].defined() ? dense_grad(grads[0], y.scalar_type())
+                                   : at::zeros_like(y);
+    Tensor dh;
+    if (grads[1].defined()) dh = dense_grad(grads[1], at::kFloat);
+    Sums sums;
+    GatedGrads r = gated_backward(
+        dy, dh, x, s[1], {s[2], s[3], s[4], s[5], s[6]}, s[8], s[9], y, s[7],
+        {ctx->needs_input_grad(3), ctx->needs_input_grad(4),
+         ctx->needs_input_grad(5), ctx->needs_input_grad(6)},
+        sums);
+    sums.launch(Dims(x));
+    return {r.dx, Tensor(), r.dlam, r.dw_x, r.db_x, r.dw_a, r.db_a, r.dh0};
+  }
+};
+
+// --------------------------------------------------------- recurrent block --
+
+// (modules.py:605-655 of the reference, without a cache)
+struct Block : Function<Block> {
+  static variable_list forward(AutogradContext* ctx, Tensor x, Tensor pos,
+                               Tensor w_y, Tensor b_y, Tensor w_lx, Tensor b_lx,
+                               Tensor conv_w, Tensor conv_b, Tensor a_param,
+                               Tensor w_x, Tensor b_x, Tensor w_a, Tensor b_a,
+                               Tensor w_out, Tensor b_out, bool want_cache) {
+    ctx->set_materialize_grads(false);
+    const int64_t B = x.size(0), T = x.size(1), W = w_y.size(0);
+    Tensor x2 = x.view({B * T, x.size(2)});
+    Tensor gate = at::linear(x2, w_y, b_y).view({B, T, W});
+    Tensor lx = at::linear(x2, w_lx, b_lx).view({B, T, W});
+    const Dims d(lx);
+    Tensor xc = empty(lx.sizes(), x), conv_state, h;
+    if (want_cache) {
+      conv_state = empty({B, 3, W}, x);
+      h = empty({B, W}, at::kFloat, x);
+    }
+    check(rg_conv1d_prefill(in(lx), in(pos), seg_kind(pos), in(conv_w), in(conv_b),
+                            out(xc), out(conv_state), (int)B, (int)T, (int)W, 4,
+                            d.code, d.stream));
+    Tensor gx = empty(lx.sizes(), x), ga = empty(lx.sizes(), x);
+    Tensor y = empty(lx.sizes(), x);
+    gated_forward(xc, pos, {a_param, w_x, b_x, w_a, b_a}, Tensor(), gx, ga, y, h);
+    Tensor join = empty(lx.sizes(), x);
+    check(rg_gelu_mul(in(y), in(gate), out(join), d.M() * W, d.code, d.stream));
+    Tensor result = at::linear(join.view({B * T, W}), w_out, b_out)
+                        .view({B, T, w_out.size(0)});
+    ctx->save_for_backward({x, pos, w_y, w_lx, conv_w, a_param, w_x, b_x, w_a, b_a,
+                            w_out, gate, lx, xc, gx, ga, y, join});
+    if (!want_cache) return {result};
+    ctx->mark_non_differentiable({conv_state});
+    return {result, h, conv_state};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    at::AutoGradMode off(false);
+    auto s = ctx->get_saved_variables();
+    const Tensor &x = s[0], &pos = s[1], &w_y = s[2], &w_lx = s[3], &conv_w = s[4],
+                 &w_out = s[10], &gate = s[11], &lx = s[12], &xc = s[13],
+                 &y = s[16], &join = s[17];
+    const Dims d(lx);
+    const int64_t M = d.M(), W = d.W;
+    const Tensor x2 = x.view({M, x.size(2)});
+    auto needs = [&](int i) { return ctx->needs_input_grad(i); };
+    Sums sums;
+    variable_list r(16);  // (the flag takes no gradient)
+    Tensor dy, dgate2;
+    if (grads[0].defined()) {
+      const Tensor dout =
+          dense_grad(grads[0], x.scalar_type()).view({M, w_out.size(0)});
+      const int64_t parts = (M + rg::kColSumRows - 1) / rg::kColSumRows;
+      if (needs(14)) {
+        Tensor part = empty({parts, dout.size(1)}, at::kFloat, x);
+        check_hip(rg::launch_col_sums(in(dout), (float*)out(part), M,
+                                      (int)dout.size(1), d.code, d.stream));
+        r[14] = sums.add(part, 0, parts, dout.size(1), dout.size(1),
+                         {dout.size(1)}, x);
+      }
+      if (needs(13)) r[13] = at::mm(dout.t(), join.view({M, W}));
+      Tensor djoin = at::mm(dout, w_out);
+      dy = empty(lx.sizes(), x);
+      dgate2 = empty({M, W}, x);
+      Tensor part = empty({parts, W}, at::kFloat, x);
+      check_hip(rg::launch_gelu_mul_backward_sums(
+          in(djoin), in(y), in(gate), out(dy), out(dgate2), (float*)out(part), M,
+          (int)W, d.code, d.stream));
+      if (needs(3)) r[3] = sums.add(part, 0, parts, W, W, {W}, x);
+      if (needs(2)) r[2] = at::mm(dgate2.t(), x2);
+      if (needs(0)) r[0] = at::mm(dgate2, w_y);
+    } else {
+      dy = at::zeros_like(y);  // only the final state is differentiated
+    }
+    Tensor dh;
+    if (grads.size() > 1 && grads[1].defined())
+      dh = dense_grad(grads[1], at::kFloat);
+    GatedGrads g = gated_backward(
+        dy, dh, xc, pos, {s[5], s[6], s[7], s[8], s[9]}, s[14], s[15], y, Tensor(),
+        {needs(9), needs(10), needs(11), needs(12)}, sums);
+    r[8] = g.dlam;
+    r[9] = g.dw_x;
+    r[10] = g.db_x;
+    r[11] = g.dw_a;
+    r[12] = g.db_a;
+    rg::ConvBwdArgs c{};
+    const int64_t chunks = rg::conv1d_backward_chunks((int)d.B, (int)d.T);
+    Tensor part = empty({chunks, 5, W}, at::kFloat, x);
+    Tensor dlx_part = empty({chunks, W}, at::kFloat, x);
+    Tensor dlx2 = dy.view({M, W});  // (dy has been read)
+    c.dout = in(g.dx);
+    c.x = in(lx);
+    c.segpos = in(pos);
+    c.seg_kind = seg_kind(pos);
+    c.w = in(conv_w);
+    c.dx = out(dlx2);
+    c.partial = (float*)out(part);
+    c.dx_sums = (float*)out(dlx_part);
+    c.B = (int)d.B;
+    c.T = (int)d.T;
+    c.W = (int)W;
+    c.K = 4;
+    check_hip(rg::launch_conv1d_backward(c, d.code, d.stream));
+    if (needs(6)) r[6] = sums.add(part, 0, chunks, 4 * W, 5 * W, {4, W}, x);
+    if (needs(7)) r[7] = sums.add(part, 4 * W, chunks, W, 5 * W, {W}, x);
+    if (needs(5)) r[5] = sums.add(dlx_part, 0, chunks, W, W, {W}, x);
+    sums.launch(d);
+    if (needs(4)) r[4] = at::mm(dlx2.t(), x2);
+    if (needs(0)) {
+      if (r[0].defined())
+        r[0].addmm_(dlx2, w_lx);
+      else
+        r[0] = at::mm(dlx2, w_lx);
+      r[0] = r[0].view(x.sizes());
+    }
+    return r;
+  }
+};
+
+// Shared by the two entries below: the RG-LRU's tensors at v[0..4].
+GateWeights gate_weights(const Call& c, PyObject* const* v, int64_t W) {
+  GateWeights g{tensor_of(v[0]), tensor_of(v[1]), tensor_of(v[2]), tensor_of(v[3]),
+                tensor_of(v[4])};
+  need(g.w_x.dim() == 3);
+  const int64_t H = g.w_x.size(0);
+  need(H > 0 && W % H == 0);
+  const int64_t bw = W / H;
+  c.shaped(v[0], {W});
+  c.shaped(v[1], {H, bw, bw});
+  c.shaped(v[2], {H, bw});
+  c.shaped(v[3], {H, bw, bw});
+  c.shaped(v[4], {H, bw});
+  need(c.code == RG_DTYPE_F32 || bw == 256);
+  return g;
+}
+
+// The calls below: under autograd or not, never under autocast (which would
+// have other dtypes in between).
+Call plain_call(PyObject* o) {
+  need(!at::autocast::is_autocast_enabled(at::kCUDA));
+  Call c(o);
+  need(c.x.dim() == 3 && c.x.numel() > 0);
+  for (int i = 0; i < 3; ++i) need(c.x.size(i) <= INT32_MAX);
+  c(o);
+  return c;
+}
+
+struct ScanCall {
+  Call c;
+  Tensor a, reset;
+  OptTensor h0;
+  explicit ScanCall(PyObject* const* v) : c(plain_call(v[0])) {
+    const int64_t B = c.x.size(0), T = c.x.size(1), W = c.x.size(2);
+    c.shaped(v[1], {B, T, W});
+    a = tensor_of(v[1]);
+    reset = tensor_of(v[2]);
+    need(shape_is(reset, {B, T}));
+    dense(reset, at::kBool, c.device);
+    if (v[3] != Py_None) {
+      c.f32(v[3], {B, W});
+      h0 = tensor_of(v[3]);
+    }
+  }
+};
+
+PyObject* pair(const Tensor& a, const Tensor& b) {
+  PyObject* t = PyTuple_New(2);
+  if (!t) throw Raised{};
+  PyTuple_SET_ITEM(t, 0, wrap(a));
+  PyTuple_SET_ITEM(t, 1, wrap(b));
+  return t;
+}
+
+}  // namespace
+
+// (x, a, reset, h0 | None) -> (y, h_last) | None
+PyObject* linear_scan(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 4);
+    ScanCall s(v);
+    Tensor y = empty(s.c.x.sizes(), s.c.x);
+    Tensor h = empty({s.c.x.size(0), s.c.x.size(2)}, at::kFloat, s.c.x);
+    {
+      NoGil nogil;
+      scan_forward(s.c.x, s.a, s.reset, s.h0.value_or(Tensor()), y, h);
+    }
+    return pair(y, h);
+  });
+}
+
+// (x, a, reset, h0 | None) -> (y, h_last) | None, differentiable
+PyObject* train_scan(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 4);
+    ScanCall s(v);
+    variable_list r;
+    {
+      NoGil nogil;
+      r = Scan::apply(s.c.x, s.a, s.reset, s.h0);
+    }
+    return pair(r[0], r[1]);
+  });
+}
+
+// (x, segment_pos, a_param, w_x, b_x, w_a, b_a, h0 | None)
+//   -> (y, h_last) | None, differentiable
+PyObject* train_rglru(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 8);
+    Call c = plain_call(v[0]);
+    const int64_t B = c.x.size(0), T = c.x.size(1), W = c.x.size(2);
+    int is64;
+    c.positions(v[1], B, T, &is64);
+    const Tensor pos = tensor_of(v[1]);
+    const GateWeights g = gate_weights(c, v + 2, W);
+    OptTensor h0;
+    if (v[7] != Py_None) {
+      c.f32(v[7], {B, W});
+      h0 = tensor_of(v[7]);
+    }
+    variable_list r;
+    {
+      NoGil nogil;
+      r = Rglru::apply(c.x, pos, g.a_param, g.w_x, g.b_x, g.w_a, g.b_a, h0);
+    }
+    return pair(r[0], r[1]);
+  });
+}
+
+// (x, segment_pos, w_y, b_y, w_x, b_x, conv_w, conv_b, a_param, gate w_x, b_x,
+//  w_a, b_a, w_out, b_out, want_cache)
+//   -> (out, h_last | None, conv_state | None) | None, differentiable
+PyObject* train_block(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 16);
+    Call c = plain_call(v[0]);
+    const int64_t B = c.x.size(0), T = c.x.size(1), D = c.x.size(2);
+    int is64;
+    c.positions(v[1], B, T, &is64);
+    Tensor t[14];
+    for (int i = 1; i < 15; ++i) t[i - 1] = tensor_of(v[i]);
+    need(t[1].dim() == 2);
+    const int64_t W = t[1].size(0);
+    c.shaped(v[2], {W, D});
+    c.shaped(v[3], {W});
+    c.shaped(v[4], {W, D});
+    c.shaped(v[5], {W});
+    c.shaped(v[6], {4, W});
+    c.shaped(v[7], {W});
+    gate_weights(c, v + 8, W);
+    c.shaped(v[13], {D, W});
+    c.shaped(v[14], {D});
+    const int per = c.code == RG_DTYPE_F32 ? 4 : 8;
+    need(W % per == 0 && D % per == 0 &&
+         (B * T + rg::kColSumRows - 1) / rg::kColSumRows <= 65535 &&
+         rg::conv1d_backward_sums_dx((int)B, (int)T, (int)W, 4, c.code));
+    const bool want_cache = v[15] == Py_True;
+    variable_list r;
+    {
+      NoGil nogil;
+      r = Block::apply(c.x, t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8],
+                       t[9], t[10], t[11], t[12], t[13], want_cache);
+    }
+    return want_cache ? triple(r[0], r[1], r[2]) : triple(r[0], Tensor(), Tensor());
+  });
+}
+
+}  // namespace rg_host

@@ -18,6 +18,7 @@ from typing import NamedTuple
 import torch
 from torch import nn
 
+from recurrentgemma_amd import _lib
 from recurrentgemma_amd import compiled
 from recurrentgemma_amd import layers
 from recurrentgemma_amd import ops
@@ -40,6 +41,20 @@ def _parameters(module, *names):
   the name is not in it (a parametrised weight)."""
   own = module._parameters
   return [own[n] if n in own else getattr(module, n) for n in names]
+
+
+def _as_written(module, kind) -> bool:
+  """Whether calling the module is nothing but kind.forward on its own
+  parameters: no subclass, hook, parametrisation or replaced method."""
+  return (type(module) is kind and "forward" not in module.__dict__ and
+          not (module._forward_hooks or module._forward_pre_hooks or
+               module._backward_hooks or module._backward_pre_hooks))
+
+
+def _global_hooks() -> bool:
+  m = nn.modules.module
+  return bool(m._global_forward_hooks or m._global_forward_pre_hooks or
+              m._global_backward_hooks or m._global_backward_pre_hooks)
 
 
 def _core_weights(conv_1d, rg_lru):
@@ -222,6 +237,12 @@ class RecurrentBlock(nn.Module):
     """The reference's op sequence (modules.py:605-655) under autograd."""
     if cache is not None:
       raise NotImplementedError("the differentiable path is prefill only")
+    done = self._differentiable_natively(x, segment_pos, return_cache)
+    if done is not None:
+      x, h, conv_state = done
+      if not return_cache:
+        return x, None
+      return x, RecurrentBlockCache(rg_lru_state=h, conv1d_state=conv_state)
     y = self.linear_y(x)
     x = self.linear_x(x)
     x, conv_state = self.conv_1d(x, segment_pos, None, return_cache)
@@ -230,6 +251,24 @@ class RecurrentBlock(nn.Module):
     if not return_cache:
       return x, None
     return x, RecurrentBlockCache(rg_lru_state=h, conv1d_state=conv_state)
+
+  def _differentiable_natively(self, x, segment_pos, return_cache):
+    """The whole block as one native autograd function (csrc/train_ops.cpp), or
+    None: where a layer has been wrapped, hooked or replaced, or the arguments
+    are not as that function takes them."""
+    own = self._modules
+    y, lx, out = own["linear_y"], own["linear_x"], own["linear_out"]
+    conv, lru = own["conv_1d"], own["rg_lru"]
+    if (compiled.tracing() or _global_hooks() or
+        not (_as_written(y, nn.Linear) and _as_written(lx, nn.Linear) and
+             _as_written(out, nn.Linear) and _as_written(conv, layers.Conv1D) and
+             _as_written(lru, layers.RGLRU))):
+      return None
+    conv_w, conv_b, w_x, b_x, w_a, b_a, a_param = _core_weights(conv, lru)
+    return _lib.host().train_block(
+        x, segment_pos, *_parameters(y, "weight", "bias"),
+        *_parameters(lx, "weight", "bias"), conv_w, conv_b, a_param, w_x, b_x,
+        w_a, b_a, *_parameters(out, "weight", "bias"), bool(return_cache))
 
   @classmethod
   def init_cache(cls, batch_size, lru_width, dtype, conv1d_temporal_width=4,

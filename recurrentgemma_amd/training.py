@@ -27,6 +27,7 @@ import contextlib
 
 import torch
 
+from recurrentgemma_amd import _lib
 from recurrentgemma_amd import ops
 
 _MAX_SQRT_GRADIENT = 1000.0
@@ -86,6 +87,11 @@ class _BoundedSqrt(torch.autograd.Function):
 def rnn_scan(x, a, reset, h0=None):
   if a.shape != x.shape:
     a = a.expand_as(x)
+  got = None
+  if not torch.compiler.is_compiling():
+    got = _lib.host().train_scan(x, a, reset, h0)
+  if got is not None:
+    return got
   return _LinearScan.apply(x.contiguous(), a.contiguous(), reset, h0)
 
 
@@ -277,7 +283,14 @@ class _GatedScan(torch.autograd.Function):
 def rg_lru(x, segment_pos, a_param, w_x, b_x, w_a, b_a, h0=None):
   """RGLRU.forward (layers.py:313-365) on kernels in both directions: the two
   gate projections (bf16; float32: batched products of the library), then
-  everything after them.  Returns (y, h_last)."""
+  everything after them.  One native autograd function (csrc/train_ops.cpp),
+  which joins the passes between them, where it takes the arguments as they
+  lie; one function per operator otherwise.  Returns (y, h_last)."""
+  got = None
+  if not torch.compiler.is_compiling():
+    got = _lib.host().train_rglru(x, segment_pos, a_param, w_x, b_x, w_a, b_a, h0)
+  if got is not None:
+    return got
   if x.dim() == 3 and _projections_on_kernels(x):
     gx_pre, ga_pre = _GateProjections.apply(x, w_x, b_x, w_a, b_a)
   else:

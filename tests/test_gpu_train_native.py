@@ -1,0 +1,140 @@
+"""The native differentiable path (csrc/train_ops.cpp and the kernels of
+csrc/rg_train.hip behind it) against the same block written in float32 tensor
+ops under autograd, at the edges of its tiles: rows around multiples of 64 and
+32, one token, one head, odd widths (float32), both position types."""
+
+import pytest
+import torch
+from torch.nn import functional as F
+
+import recurrentgemma_amd as rg
+from recurrentgemma_amd import _lib
+from recurrentgemma_amd import training
+
+pytestmark = pytest.mark.gpu
+BF16, F32 = torch.bfloat16, torch.float32
+
+
+def close(got, want, dtype, what):
+  got, want = got.detach().float(), want.detach().float()
+  assert got.shape == want.shape, what
+  err = (got - want).norm().item() / max(want.norm().item(), 1e-6)
+  assert err < (2e-2 if dtype == BF16 else 2e-5), (what, err)
+
+
+def reference(block, x, pos, p):
+  """modules.py:605-655 of the reference in float32; p: name -> tensor."""
+  gate = F.linear(x, p["linear_y.weight"], p["linear_y.bias"])
+  h = F.linear(x, p["linear_x.weight"], p["linear_x.bias"])
+  h = training.conv1d_tensor_ops(h, pos, p["conv_1d.w"], p["conv_1d.b"])
+  h, last = training.rg_lru_tensor_ops(
+      h, pos, *(p["rg_lru." + n] for n in (
+          "a_param", "input_gate.w", "input_gate.b", "a_gate.w", "a_gate.b")))
+  h = h * F.gelu(gate, approximate="tanh")
+  return F.linear(h, p["linear_out.weight"], p["linear_out.bias"]), last
+
+
+def make(B, T, width, heads, dtype, seed=0):
+  torch.manual_seed(seed)
+  block = rg.RecurrentBlock(width=width, num_heads=heads, device="cuda",
+                            dtype=dtype)
+  with torch.no_grad():
+    for name, q in block.named_parameters():
+      if name.endswith("bias") or name.endswith(".b"):
+        q.normal_(std=0.1)
+      if name.startswith("conv_1d.w"):
+        q.normal_(std=0.5)
+  x = torch.randn(B, T, width, device="cuda").to(dtype).requires_grad_()
+  pos = torch.arange(T, device="cuda").expand(B, T).clone()
+  pos[0, T // 2:] -= T // 2  # a second document
+  return block, x, pos
+
+
+SHAPES = [(1, 1, 256, 1, BF16), (1, 63, 256, 1, BF16), (3, 64, 512, 2, BF16),
+          (1, 65, 256, 1, BF16), (2, 97, 768, 3, BF16), (5, 333, 512, 2, BF16),
+          (1, 1, 48, 2, F32), (2, 130, 48, 2, F32), (3, 65, 512, 2, F32)]
+
+
+@pytest.mark.parametrize("B,T,width,heads,dtype", SHAPES)
+@pytest.mark.parametrize("pos_dtype", [torch.int32, torch.int64])
+def test_block_gradients(B, T, width, heads, dtype, pos_dtype, monkeypatch):
+  block, x, pos = make(B, T, width, heads, dtype)
+  pos = pos.to(pos_dtype)
+  # the native function takes the call: the general path is out of reach
+  monkeypatch.setattr(training, "gelu_mul", None)
+  with training.differentiable():
+    y, cache = block(x, pos)
+    dy = torch.randn_like(y)
+    dh = torch.randn_like(cache.rg_lru_state)
+    names = [n for n, _ in block.named_parameters()]
+    wanted = [x] + [q for _, q in block.named_parameters()]
+    got = torch.autograd.grad((y, cache.rg_lru_state), wanted, (dy, dh))
+    p = {n: q.detach().float().requires_grad_() for n, q in
+         block.named_parameters()}
+    xf = x.detach().float().requires_grad_()
+    yr, hr = reference(block, xf, pos, p)
+    want = torch.autograd.grad((yr, hr), [xf] + [p[n] for n in names],
+                               (dy.float(), dh))
+  close(y, yr, dtype, "y")
+  close(cache.rg_lru_state, hr, dtype, "h")
+  assert cache.conv1d_state.shape == (B, 3, width)
+  for name, g, w in zip(["x"] + names, got, want):
+    assert g.dtype == dtype
+    close(g, w, dtype, name)
+
+
+@pytest.mark.parametrize("B,T,width,heads,dtype", SHAPES)
+def test_rglru_gradients(B, T, width, heads, dtype):
+  block, x, pos = make(B, T, width, heads, dtype)
+  lru = block.rg_lru
+  h0 = torch.randn(B, width, device="cuda").requires_grad_()
+  with training.differentiable():
+    y, h = lru(x, pos, h0)
+    dy = torch.randn_like(y)
+    params = list(lru.parameters())
+    got = torch.autograd.grad((y,), [x, h0] + params, dy)
+    copies = [q.detach().float().requires_grad_() for q in params]
+    xf = x.detach().float().requires_grad_()
+    hf = h0.detach().clone().requires_grad_()
+    by = {n: c for (n, _), c in zip(lru.named_parameters(), copies)}
+    yr, hr = training.rg_lru_tensor_ops(
+        xf, pos, by["a_param"], by["input_gate.w"], by["input_gate.b"],
+        by["a_gate.w"], by["a_gate.b"], hf)
+    want = torch.autograd.grad((yr,), [xf, hf] + copies, dy.float())
+  close(y, yr, dtype, "y")
+  close(h, hr, dtype, "h")
+  for i, (g, w) in enumerate(zip(got, want)):
+    close(g, w, dtype, i)
+
+
+def test_frozen_parts_and_wrapped_layers():
+  """Only what needs a gradient gets one, and a hooked layer is called."""
+  block, x, pos = make(2, 70, 512, 2, BF16)
+  for q in block.parameters():
+    q.requires_grad_(False)
+  block.linear_y.bias.requires_grad_()
+  with training.differentiable():
+    y, _ = block(x.detach(), pos, return_cache=False)
+    (alone,) = torch.autograd.grad(y.float().square().sum(),
+                                   [block.linear_y.bias])
+  called = []
+  handle = block.linear_x.register_forward_hook(
+      lambda *a: called.append(1))
+  with training.differentiable():
+    y2, _ = block(x.detach(), pos, return_cache=False)
+    (hooked,) = torch.autograd.grad(y2.float().square().sum(),
+                                    [block.linear_y.bias])
+  handle.remove()
+  assert called
+  close(y, y2, BF16, "y")
+  close(alone, hooked, BF16, "bias")
+  # a tensor that does not start at 16 bytes takes the general path
+  flat = torch.empty(x.numel() + 1, dtype=BF16, device="cuda")
+  odd = flat[1:].view(x.shape).copy_(x.detach())
+  assert _lib.host().train_block(
+      odd, pos, *(getattr(block.linear_y, n) for n in ("weight", "bias")),
+      *(getattr(block.linear_x, n) for n in ("weight", "bias")),
+      block.conv_1d.w, block.conv_1d.b, block.rg_lru.a_param,
+      block.rg_lru.input_gate.w, block.rg_lru.input_gate.b,
+      block.rg_lru.a_gate.w, block.rg_lru.a_gate.b, block.linear_out.weight,
+      block.linear_out.bias, False) is None
