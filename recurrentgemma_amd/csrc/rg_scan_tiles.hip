@@ -589,22 +589,37 @@ bool scan_tiles_serve(int B, int T, int W, int dtype, int mode) {
   if ((int64_t)W * es % 16 != 0 ||
       ((int64_t)T + 1024) * W * es >= (int64_t)0x7fffffff)
     return false;
-  // The backward forms: everywhere (us, B4 T2048 W2560 bf16: plain 77 -> 40,
-  // gated 140 -> 118; B16 T8192 W4096: 1555 -> 1104, 2067 -> 1710).
-  if (mode == kBwdPlain || mode == kBwdGated) return true;
-  // The forward ones (B4 T2048 W2560 bf16: plain 52 -> 28, gated 83 -> 44), but
-  // for two ranges where rg_scan.hip's kernel is ahead: one or two long rows,
-  // which it cuts into chunks (B1 T16384 W1000: plain 139, here 148; gated from
-  // 4096 tokens on: T8192 105, here 146), and many workgroups on more data than
-  // the last-level cache holds, which it streams with more waves per CU (B16
-  // T1024 W4096: plain 73, here 102, gated 101, here 162).
-  int chunks, t_chunk;
-  scan_split_plan(B, T, W, 64, &chunks, &t_chunk);
-  if (chunks > 1 && T > (mode == kFwdPlain ? 8192 : 4096)) return false;
+  // The eight waves of a workgroup walk a slab of channels in steps of 256
+  // or 512 tokens, one workgroup per CU: a launch costs a round of the chip per
+  // 256 slabs and at least one step, where rg_scan.hip's and rg_scan_bwd.hip's
+  // kernels cost by the token.  The lines below are where they meet.
   const int64_t slab = dtype == 0 ? TileLds<float>::channels : TileLds<uint16_t>::channels;
   const int64_t blocks = (int64_t)B * ((W + slab - 1) / slab);
-  return blocks < (dtype == 0 ? 2048 : 1024) ||
-         3 * es * (int64_t)B * T * W < ((int64_t)256 << 20);
+  // The backward forms but for several rounds of short rows (us, B4 T2048 W2560
+  // bf16: plain 77 -> 40, gated 140 -> 118; B16 T8192 W4096: 1555 -> 1104, 2067
+  // -> 1710; but B16 T64 W4096 plain 13, here 19; float32 22, here 28).
+  if (mode == kBwdGated) return true;
+  if (mode == kBwdPlain)
+    return dtype == 0 ? blocks < 800 || T >= 128 : blocks < 512 || T >= 400;
+  // The forward ones (B4 T2048 W2560 bf16: plain 52 -> 28, gated 83 -> 44).
+  // One or two long rows rg_scan.hip cuts into chunks (bf16 plain: B1 T4096
+  // W512 26, here 32, W4096 60, here 41; gated from 4096 tokens on: T8192 105,
+  // here 146; float32 plain B1 T8192 W512 60, here 49).
+  int chunks, t_chunk;
+  scan_split_plan(B, T, W, 64, &chunks, &t_chunk);
+  if (chunks > 1) {
+    const int64_t few = blocks * 64 > 2048 ? blocks * 64 : 2048;
+    const int64_t most = mode == kFwdGated ? 4096 : dtype == 0 ? 8192 : few;
+    if (T > most) return false;
+  }
+  const bool cached = 3 * es * (int64_t)B * T * W < ((int64_t)256 << 20);
+  if (mode == kFwdGated) return blocks < (dtype == 0 ? 2048 : 1024) || cached;
+  // Plain: while every slab has a CU of its own; beyond, what the last-level
+  // cache holds of a few rounds (bf16 B16 T1024 W2560: 62 -> 47, but T300 21,
+  // here 22, and B8 T1600 W4096 61, here 71; float32 B8 T500 W2560 30 -> 24, but
+  // T180 13, here 14, and B16 T500 W2048 35, here 35).
+  if (blocks <= (dtype == 0 ? 512 : 256)) return true;
+  return cached && (dtype == 0 ? blocks < 800 && T >= 400 : blocks > 512 && T >= 500);
 }
 
 hipError_t launch_scan_tiles(const ScanTileArgs& a, int mode, int dtype,
