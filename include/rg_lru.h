@@ -452,6 +452,30 @@ int rg_attention_prefill(const void* q, const void* k, const void* v_t,
                          int T_pad, int H, int head_dim, float scale, int dtype,
                          void* stream);
 
+/* first_key of rg_attention_prefill for a prompt's positions [B,T]
+ * (int32/int64): max(last position 0 at or before the query, else 0;
+ * t - window) -- the mask of recurrentgemma/torch/modules.py:86-127. */
+int rg_attention_first_key(const void* positions, int positions_is_i64,
+                           int32_t* first_key, int B, int T, int window,
+                           void* stream);
+
+/* A prompt pass of the local-attention block between its projections
+ * (modules.py:431-476, ring cache :253-283) in two launches: rg_rope_pair on q
+ * and k, rg_attention_prefill, and the cache it leaves.  q, out [B,T,H,256],
+ * k, v [B,T,256] as the projections leave them, inv_freq [64], first_key
+ * [B,T]; ring_keys, ring_values [B,window,256] and num_tokens [B] are written
+ * whole (all three NULL: no cache); workspace of
+ * rg_attention_prompt_workspace_bytes(B, T).  RG_ERR_UNSUPPORTED as for
+ * rg_attention_prefill. */
+size_t rg_attention_prompt_workspace_bytes(int B, int T);
+int rg_attention_prompt(const void* q, const void* k, const void* v,
+                        const void* positions, int positions_is_i64,
+                        const float* inv_freq, const int32_t* first_key,
+                        void* out, void* ring_keys, void* ring_values,
+                        int32_t* num_tokens, void* workspace, int B, int T,
+                        int H, int head_dim, int window, float scale, int dtype,
+                        void* stream);
+
 /* Masked softmax of one decoded token against the ring cache and itself
  * (modules.py:152-183 `_compute_cache_mask`, :462-470): scores
  * [B, heads, window] = q . k of the ring slots, unscaled, in `dtype`; q

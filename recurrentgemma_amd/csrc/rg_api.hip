@@ -1127,6 +1127,96 @@ int rg_attention_prefill(const void* q, const void* k, const void* v_t,
       __func__, rg::launch_attn_prefill_bf16(a, (hipStream_t)stream));
 }
 
+int rg_attention_first_key(const void* positions, int positions_is_i64,
+                           int32_t* first_key, int B, int T, int window,
+                           void* stream) {
+  RG_REQUIRE(B > 0 && T > 0 && window > 0,
+             "%s: B=%d T=%d window=%d must be positive", __func__, B, T,
+             window);
+  RG_CHECK_PTR(positions);
+  RG_CHECK_PTR(first_key);
+  return launch_status(
+      __func__,
+      rg::launch_first_key(positions,
+                           positions_is_i64 ? 1 : 0,
+                           first_key, B, T, window, (hipStream_t)stream));
+}
+
+size_t rg_attention_prompt_workspace_bytes(int B, int T) {
+  if (B <= 0 || T <= 0) return 0;
+  const size_t t_pad = ((size_t)T + 63) / 64 * 64;
+  // rotated keys, transposed values, sines and cosines
+  return (size_t)B * ((size_t)T * 512 + t_pad * 512 + (size_t)T * 256);
+}
+
+int rg_attention_prompt(const void* q, const void* k, const void* v,
+                        const void* positions, int positions_is_i64,
+                        const float* inv_freq, const int32_t* first_key,
+                        void* out, void* ring_keys, void* ring_values,
+                        int32_t* num_tokens, void* workspace, int B, int T,
+                        int H, int head_dim, int window, float scale, int dtype,
+                        void* stream) {
+  RG_CHECK_DTYPE(dtype);
+  RG_REQUIRE(B > 0 && T > 0 && H > 0 && window > 0,
+             "%s: B=%d T=%d H=%d window=%d must be positive", __func__, B, T, H,
+             window);
+  if (dtype != RG_DTYPE_BF16 || head_dim != 256)
+    return fail(RG_ERR_UNSUPPORTED,
+                "%s: needs bf16 and head_dim == 256 (dtype=%d head_dim=%d)",
+                __func__, dtype, head_dim);
+  const int64_t t_pad = ((int64_t)T + 63) / 64 * 64;
+  RG_REQUIRE((int64_t)T * H * 512 < ((int64_t)1 << 31) &&
+                 t_pad * 512 < ((int64_t)1 << 31),
+             "%s: T=%d H=%d: a row's queries exceed 2 GiB", __func__, T, H);
+  RG_CHECK_PTR(q);
+  RG_CHECK_PTR(k);
+  RG_CHECK_PTR(v);
+  RG_CHECK_PTR(positions);
+  RG_CHECK_PTR(inv_freq);
+  RG_CHECK_PTR(first_key);
+  RG_CHECK_PTR(out);
+  RG_CHECK_PTR(workspace);
+  if (ring_keys || ring_values || num_tokens) {
+    RG_CHECK_PTR(ring_keys);
+    RG_CHECK_PTR(ring_values);
+    RG_CHECK_PTR(num_tokens);
+  }
+  RG_REQUIRE(out != q && out != k && out != v,
+             "%s: out must not alias an input", __func__);
+  rg::AttnPromptArgs p{};
+  p.k = (const uint16_t*)k;
+  p.v = (const uint16_t*)v;
+  p.pos = positions;
+  p.pos_kind = positions_is_i64 ? 1 : 0;
+  p.inv_freq = inv_freq;
+  p.k_rot = (uint16_t*)workspace;
+  p.v_t = p.k_rot + (int64_t)B * T * 256;
+  p.rope_table = (uint32_t*)(p.v_t + (int64_t)B * t_pad * 256);
+  p.ring_k = (uint16_t*)ring_keys;
+  p.ring_v = (uint16_t*)ring_values;
+  p.num_tokens = num_tokens;
+  p.B = B;
+  p.T = T;
+  p.T_pad = (int)t_pad;
+  p.window = window;
+  hipError_t e = rg::launch_attn_prompt_prepare(p, (hipStream_t)stream);
+  if (e != hipSuccess) return launch_status(__func__, e);
+  rg::AttnPrefillArgs a{};
+  a.q = q;
+  a.k = p.k_rot;
+  a.v_t = p.v_t;
+  a.lo = first_key;
+  a.out = out;
+  a.B = B;
+  a.T = T;
+  a.T_pad = (int)t_pad;
+  a.H = H;
+  a.scale = scale;
+  a.rope_table = p.rope_table;
+  return launch_status(
+      __func__, rg::launch_attn_prefill_bf16(a, (hipStream_t)stream));
+}
+
 int rg_attention_decode_probs(const void* scores, const void* q,
                               const void* k_new, const int32_t* num_tokens,
                               void* probs, int B, int heads, int head_dim,

@@ -24,6 +24,11 @@
 // out in LDS in that order.  The values arrive transposed ([row, 256, T]: the
 // caller's one extra pass over them), which makes the contraction index the
 // contiguous one of both operands of both products.
+//
+// What a block does around that for a prompt -- rotary embedding, the values'
+// transposition, the ring cache it leaves -- is attn_prompt_prepare_kernel at
+// the end of this file; the queries take their rotary embedding inside the
+// attention kernel.
 #include <utility>
 
 #include "rg_common.h"
@@ -96,6 +101,41 @@ __device__ __forceinline__ void wait_for_matrix_results() {
   asm volatile("s_nop 15\n\ts_nop 7");
 }
 
+// Rotary embedding of the first half of a query's dimensions (elements i and
+// i + 64, i < 64) where the query lies as operand fragments: k-steps 0..3 hold
+// this lane's elements 16 ks + 8 half + 0..7, k-steps 4..7 their partners.
+// `table` is the query's row of sines and cosines (see
+// attn_prompt_prepare_kernel).  The arithmetic of rg_rope_pair, element for
+// element: products and sums rounded one by one.
+__device__ __forceinline__ void rotate_query(AFrag (&qf)[16],
+                                             const u32x4 (&table)[8]) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      float vlo[2], vhi[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint32_t sc = table[2 * ks + (w >> 1)][2 * (w & 1) + e];
+        const float sn = __uint_as_float(sc << 16);
+        const float cs = __uint_as_float(sc & 0xffff0000u);
+        const uint32_t l = qf[ks].u[w], h = qf[ks + 4].u[w];
+        const float lo = __uint_as_float(e == 0 ? l << 16 : l & 0xffff0000u);
+        const float hi = __uint_as_float(e == 0 ? h << 16 : h & 0xffff0000u);
+        vlo[e] = round_to_bf16(lo * cs) - round_to_bf16(hi * sn);
+        vhi[e] = round_to_bf16(hi * cs) + round_to_bf16(lo * sn);
+      }
+      qf[ks].u[w] = pack_bf16x2(vlo[0], vlo[1]);
+      qf[ks + 4].u[w] = pack_bf16x2(vhi[0], vhi[1]);
+    }
+  }
+}
+
+// ROPE: the queries come before their rotary embedding and take it here, in
+// the registers they are loaded to (p.rope_table); a pass of its own over them
+// reads and writes every query once more (8 x 2047 tokens, 10 heads: 43 us).
+template <bool ROPE>
 __global__ void __launch_bounds__(256)
 attn_prefill_bf16_kernel(AttnPrefillArgs p) {
   extern __shared__ __align__(16) unsigned char attn_lds[];
@@ -142,18 +182,6 @@ attn_prefill_bf16_kernel(AttnPrefillArgs p) {
   const __amdgpu_buffer_rsrc_t rlo = make_rsrc(
       (const char*)p.lo + (int64_t)b * T * 4, (uint32_t)T * 4u);
 
-  // this lane's query as the B operand of the first product: 16 k-steps of
-  // 8 dimensions (16 bytes); queries past the end read as zero
-  AFrag qf[16];
-  {
-    const uint32_t off = (uint32_t)q * q_row_bytes + (uint32_t)head * 512u +
-                         16u * (uint32_t)half;
-#pragma unroll
-    for (int ks = 0; ks < 16; ++ks)
-      qf[ks].q = __builtin_bit_cast(
-          f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     rq, q < T ? off + 32u * ks : kBufferOutOfRange, 0, 0));
-  }
   // first visible key of this lane's query, and of the tile's / wave's first
   // query (lo is non-decreasing: they bound the keys the tile / wave needs)
   auto lo_at = [&](int t) {
@@ -168,6 +196,33 @@ attn_prefill_bf16_kernel(AttnPrefillArgs p) {
   const int q_last_wave = qw0 + 31 < T - 1 ? qw0 + 31 : T - 1;
   const int kt_begin = lo_tile / kAttnK;
   const int kt_end = q_last_tile / kAttnK;  // inclusive
+
+  // (after the bounds, which the first tile's addresses wait for: loads return
+  // in order, and the tile is requested with the queries on their way)
+  // this lane's query as the B operand of the first product: 16 k-steps of
+  // 8 dimensions (16 bytes); queries past the end read as zero
+  AFrag qf[16];
+  {
+    const uint32_t off = (uint32_t)q * q_row_bytes + (uint32_t)head * 512u +
+                         16u * (uint32_t)half;
+#pragma unroll
+    for (int ks = 0; ks < 16; ++ks)
+      qf[ks].q = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     rq, q < T ? off + 32u * ks : kBufferOutOfRange, 0, 0));
+  }
+  u32x4 table[ROPE ? 8 : 1];  // this lane's share of the query's sines, cosines
+  if (ROPE) {
+    const __amdgpu_buffer_rsrc_t rt =
+        make_rsrc((const char*)p.rope_table + (int64_t)b * T * 256,
+                  (uint32_t)T * 256u);
+    const uint32_t off = (uint32_t)q * 256u + 32u * (uint32_t)half;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      table[i] = __builtin_amdgcn_raw_buffer_load_b128(
+          rt, q < T ? off + 64u * (i >> 1) + 16u * (i & 1) : kBufferOutOfRange,
+          0, 0);
+  }
 
   acc_fill(0.0f, std::make_integer_sequence<int, 128>{});
   float m_run = -__builtin_inff();  // running maximum, in units of log2
@@ -215,6 +270,7 @@ attn_prefill_bf16_kernel(AttnPrefillArgs p) {
   // arrives in registers and is written to the other afterwards; one barrier
   // per tile.
   request_tile(kt_begin);
+  if constexpr (ROPE) rotate_query(qf, table);
   stage_tile(0);
   __syncthreads();
   if (kt_begin < kt_end) request_tile(kt_begin + 1);
@@ -391,7 +447,218 @@ attn_prefill_bf16_kernel(AttnPrefillArgs p) {
 #undef RG_ATTN_STORE
 }
 
+// ---------------------------------------------------------------- prepare --
+// Everything of the block between its projections and the attention kernel,
+// in one pass over the keys and values (recurrentgemma/torch/modules.py:431-440
+// and the ring cache of a prompt, :253-283): rotary embedding of the keys, the
+// sines and cosines the queries are rotated with (one word per token and pair:
+// sine in the low half, cosine in the high half, bf16), the values transposed
+// for the second product (zeros behind the last token), the last min(window, T)
+// keys and values in their ring slots, zeros in the slots never written, and
+// the token count.
+//
+// One workgroup per (row, 32 tokens and 32 ring slots), which leaves the chip
+// full from 8 x 1024 tokens on.  Bound by memory (8 x 2047 tokens: 17 MB in,
+// 38 MB out); the tensor operations it replaces were ten launches, 146 us
+// there.  32 tokens make runs of 64 bytes of a transposed row; with 64 a single
+// prompt fills half as many CUs.
+constexpr int kPrepTokens = 32;
+constexpr int kPrepStride = kAttnHd + 8;  // of a token's values in LDS
+
+__device__ __forceinline__ int64_t position_at(const AttnPromptArgs& p,
+                                               int64_t i) {
+  return p.pos_kind == kSegI64
+             ? reinterpret_cast<const int64_t*>(p.pos)[i]
+             : (int64_t)reinterpret_cast<const int32_t*>(p.pos)[i];
+}
+
+__global__ void __launch_bounds__(256)
+attn_prompt_prepare_kernel(AttnPromptArgs p) {
+#pragma clang fp contract(off)
+  __shared__ __align__(16) uint16_t values[kPrepTokens * kPrepStride];
+  const int tid = threadIdx.x;
+  const int T = p.T, b = (int)(blockIdx.x / p.groups);
+  const int t0 = (int)(blockIdx.x % p.groups) * kPrepTokens;
+  const int64_t row0 = (int64_t)b * T;
+  const uint16_t* const k = p.k + row0 * kAttnHd;
+  const uint16_t* const v = p.v + row0 * kAttnHd;
+  uint16_t* const k_out = p.k_rot + row0 * kAttnHd;
+  const bool cache = p.ring_k != nullptr;
+  uint16_t* const ring_k = p.ring_k + (int64_t)b * p.window * kAttnHd;
+  uint16_t* const ring_v = p.ring_v + (int64_t)b * p.window * kAttnHd;
+
+  // token t of the last `kept` lies in slot (t - (T - kept) + shift) % kept
+  const int kept = p.window < T ? p.window : T;
+  int shift = 0;
+  if (cache) {
+    const int count = (int)position_at(p, row0 + T - 1) + 1;
+    shift = count % p.window;
+    if (shift < 0) shift += p.window;
+    if (t0 == 0 && tid == 0) p.num_tokens[b] = count;
+  }
+  auto slot_of = [&](int t) {  // -1: not kept
+    const int i = t - (T - kept);
+    return cache && i >= 0 ? (int)(((int64_t)i + shift) % kept) : -1;
+  };
+
+  // keys, rotated half: thread = 8 pairs of one token
+  const int t_of = t0 + tid / 8;
+  if (t_of < T) {
+    const int i0 = 8 * (tid % 8);
+    const u32x4 lo4 =
+        *reinterpret_cast<const u32x4*>(k + (int64_t)t_of * kAttnHd + i0);
+    const u32x4 hi4 =
+        *reinterpret_cast<const u32x4*>(k + (int64_t)t_of * kAttnHd + 64 + i0);
+    const float at = p.pos_kind == kSegI64
+                         ? (float)position_at(p, row0 + t_of)
+                         : (float)(int32_t)position_at(p, row0 + t_of);
+    u32x4 olo, ohi, table[2];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      float vlo[2], vhi[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float angle = at * p.inv_freq[i0 + 2 * w + e];
+        const float sn = round_to_bf16(sinf(angle));
+        const float cs = round_to_bf16(cosf(angle));
+        table[w >> 1][2 * (w & 1) + e] =
+            (__float_as_uint(sn) >> 16) | (__float_as_uint(cs) & 0xffff0000u);
+        const float lo =
+            __uint_as_float(e == 0 ? lo4[w] << 16 : lo4[w] & 0xffff0000u);
+        const float hi =
+            __uint_as_float(e == 0 ? hi4[w] << 16 : hi4[w] & 0xffff0000u);
+        vlo[e] = round_to_bf16(lo * cs) - round_to_bf16(hi * sn);
+        vhi[e] = round_to_bf16(hi * cs) + round_to_bf16(lo * sn);
+      }
+      olo[w] = pack_bf16x2(vlo[0], vlo[1]);
+      ohi[w] = pack_bf16x2(vhi[0], vhi[1]);
+    }
+    u32x4* const tab =
+        reinterpret_cast<u32x4*>(p.rope_table + (row0 + t_of) * 64 + i0);
+    tab[0] = table[0];
+    tab[1] = table[1];
+    uint16_t* const dst = k_out + (int64_t)t_of * kAttnHd + i0;
+    *reinterpret_cast<u32x4*>(dst) = olo;
+    *reinterpret_cast<u32x4*>(dst + 64) = ohi;
+    const int slot = slot_of(t_of);
+    if (slot >= 0) {
+      uint16_t* const r = ring_k + (int64_t)slot * kAttnHd + i0;
+      *reinterpret_cast<u32x4*>(r) = olo;
+      *reinterpret_cast<u32x4*>(r + 64) = ohi;
+    }
+  }
+  // keys, the half that is not rotated
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int t = t0 + 16 * j + tid / 16;
+    const int d = 128 + 8 * (tid % 16);
+    if (t < T) {
+      const u32x4 w = *reinterpret_cast<const u32x4*>(k + (int64_t)t * kAttnHd + d);
+      *reinterpret_cast<u32x4*>(k_out + (int64_t)t * kAttnHd + d) = w;
+      const int slot = slot_of(t);
+      if (slot >= 0)
+        *reinterpret_cast<u32x4*>(ring_k + (int64_t)slot * kAttnHd + d) = w;
+    }
+  }
+  // values: to their ring slots, and through LDS into transposed rows
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = 8 * j + tid / 32, t = t0 + i;
+    const int d = 8 * (tid % 32);
+    u32x4 w = {0, 0, 0, 0};
+    if (t < T) {
+      w = *reinterpret_cast<const u32x4*>(v + (int64_t)t * kAttnHd + d);
+      const int slot = slot_of(t);
+      if (slot >= 0)
+        *reinterpret_cast<u32x4*>(ring_v + (int64_t)slot * kAttnHd + d) = w;
+    }
+    *reinterpret_cast<u32x4*>(values + i * kPrepStride + d) = w;
+  }
+  // ring slots that no token of the prompt fills
+  if (cache) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int slot = t0 + 8 * j + tid / 32;
+      if (slot >= kept && slot < p.window) {
+        const int64_t at = (int64_t)slot * kAttnHd + 8 * (tid % 32);
+        *reinterpret_cast<u32x4*>(ring_k + at) = u32x4{0, 0, 0, 0};
+        *reinterpret_cast<u32x4*>(ring_v + at) = u32x4{0, 0, 0, 0};
+      }
+    }
+  }
+  __syncthreads();
+  if (t0 < p.T_pad) {  // (T_pad is a multiple of 64: all 32 columns exist)
+    uint16_t* const vt = p.v_t + (int64_t)b * kAttnHd * p.T_pad + t0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int d = 64 * j + tid / 4, part = tid % 4;
+      u32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint16_t* const c =
+            values + (8 * part + 2 * e) * kPrepStride + d;
+        w[e] = (uint32_t)c[0] | ((uint32_t)c[kPrepStride] << 16);
+      }
+      *reinterpret_cast<u32x4*>(vt + (int64_t)d * p.T_pad + 8 * part) = w;
+    }
+  }
+}
+
+// First key that each query of a prompt sees: the later of the start of its
+// document (the last position 0 at or before it, else the row's first token)
+// and the token `window` before it.  One workgroup per row, 1024 tokens at a
+// time; within a wave the last start is the highest set bit of a ballot.
+__global__ void __launch_bounds__(1024)
+first_key_kernel(const void* pos, int pos_kind, int32_t* __restrict__ first,
+                 int T, int window) {
+  __shared__ int last[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t row0 = (int64_t)blockIdx.x * T;
+  int carry = 0;  // start of the document that reaches into this round
+  for (int t0 = 0, round = 0; t0 < T; t0 += 1024, ++round) {
+    const int t = t0 + tid;
+    bool starts = false;
+    if (t < T)
+      starts = pos_kind == kSegI64
+                   ? reinterpret_cast<const int64_t*>(pos)[row0 + t] == 0
+                   : reinterpret_cast<const int32_t*>(pos)[row0 + t] == 0;
+    const uint64_t mask = __ballot(starts);
+    int* const found = last[round & 1];
+    if (lane == 0)
+      found[wave] = mask ? t0 + 64 * wave + 63 - __builtin_clzll(mask) : -1;
+    __syncthreads();
+    const uint64_t upto = mask & (~(uint64_t)0 >> (63 - lane));
+    int start = upto ? t0 + 64 * wave + 63 - __builtin_clzll(upto) : -1;
+    int before = carry;
+    for (int w = 0; w < 16; ++w) {
+      if (w < wave) before = max(before, found[w]);
+      carry = max(carry, found[w]);
+    }
+    start = max(start, before);
+    if (t < T) first[row0 + t] = max(start, t - window);
+  }
+}
+
 }  // namespace
+
+hipError_t launch_attn_prompt_prepare(const AttnPromptArgs& args,
+                                      hipStream_t s) {
+  AttnPromptArgs a = args;
+  const int64_t tokens = a.ring_k && a.window > a.T_pad ? a.window : a.T_pad;
+  const int64_t groups = (tokens + kPrepTokens - 1) / kPrepTokens;
+  if (groups <= 0 || a.B <= 0 || groups * a.B > 0x7fffffff)
+    return hipErrorInvalidValue;
+  a.groups = (unsigned)groups;
+  attn_prompt_prepare_kernel<<<dim3((unsigned)(groups * a.B)), 256, 0, s>>>(a);
+  return hipGetLastError();
+}
+
+hipError_t launch_first_key(const void* pos, int pos_kind, int32_t* first,
+                            int B, int T, int window, hipStream_t s) {
+  first_key_kernel<<<dim3((unsigned)B), 1024, 0, s>>>(pos, pos_kind, first, T,
+                                                      window);
+  return hipGetLastError();
+}
 
 hipError_t launch_attn_prefill_bf16(const AttnPrefillArgs& a, hipStream_t s) {
   // needs head dimension 256, T_pad a multiple of 64 >= T, and rows whose byte
@@ -401,11 +668,16 @@ hipError_t launch_attn_prefill_bf16(const AttnPrefillArgs& a, hipStream_t s) {
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
   constexpr size_t lds = 2 * (size_t)(kKTileBytes + kVTileBytes);
   static_assert(lds <= 160 * 1024, "LDS of one CU");
-  static OncePerDevice once;
-  hipError_t e =
-      set_max_dynamic_lds(once, (const void*)attn_prefill_bf16_kernel, lds);
+  static OncePerDevice once[2];
+  const bool rope = a.rope_table != nullptr;
+  hipError_t e = set_max_dynamic_lds(
+      once[rope], rope ? (const void*)attn_prefill_bf16_kernel<true>
+                       : (const void*)attn_prefill_bf16_kernel<false>, lds);
   if (e != hipSuccess) return e;
-  attn_prefill_bf16_kernel<<<dim3((unsigned)blocks), 256, lds, s>>>(a);
+  if (rope)
+    attn_prefill_bf16_kernel<true><<<dim3((unsigned)blocks), 256, lds, s>>>(a);
+  else
+    attn_prefill_bf16_kernel<false><<<dim3((unsigned)blocks), 256, lds, s>>>(a);
   return hipGetLastError();
 }
 

@@ -144,6 +144,7 @@ struct StepArgs {
 // Prompt-pass attention (rg_attention_prefill.hip).
 struct AttnPrefillArgs {
   const void* q;    // [B, T, H, 256] bf16, after the rotary embedding
+                    // (before it where rope_table is given)
   const void* k;    // [B, T, 256] bf16, after the rotary embedding
   const void* v_t;  // [B, 256, T_pad] bf16: the values transposed, zeros
                     // behind token T - 1 (T_pad a multiple of 64)
@@ -151,8 +152,28 @@ struct AttnPrefillArgs {
   void* out;        // [B, T, H, 256] bf16
   int B, T, T_pad, H;
   float scale;      // of the scores (head_dim ** -0.5)
+  const uint32_t* rope_table;  // [B, T, 64] (sine, cosine) pairs, or null
 };
 hipError_t launch_attn_prefill_bf16(const AttnPrefillArgs& a, hipStream_t s);
+// What precedes it in a block (same file).
+struct AttnPromptArgs {
+  const uint16_t* k;      // [B, T, 256] before the rotary embedding
+  const uint16_t* v;      // [B, T, 256]
+  const void* pos;        // [B, T]
+  int pos_kind;
+  const float* inv_freq;  // [64]
+  uint16_t* k_rot;        // [B, T, 256]
+  uint16_t* v_t;          // [B, 256, T_pad]
+  uint32_t* rope_table;   // [B, T, 64]
+  uint16_t* ring_k;       // [B, window, 256], null: no cache wanted
+  uint16_t* ring_v;
+  int32_t* num_tokens;    // [B]
+  int B, T, T_pad, window;
+  unsigned groups;        // workgroups per row (set by the launch)
+};
+hipError_t launch_attn_prompt_prepare(const AttnPromptArgs& a, hipStream_t s);
+hipError_t launch_first_key(const void* pos, int pos_kind, int32_t* first,
+                            int B, int T, int window, hipStream_t s);
 
 // One decoded token against the ring cache (rg_attention_decode.hip).
 constexpr int kAttnDecodeChunk = 256;     // ring slots per workgroup

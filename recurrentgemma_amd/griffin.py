@@ -279,11 +279,7 @@ def _first_visible_key(segment_pos, window):
   if (ref is not None and ref() is segment_pos and now is not None and
       version == now and w == window):
     return answer
-  b, t = segment_pos.shape
-  pos = torch.arange(t, device=segment_pos.device)[None].expand(b, t)
-  start = torch.cummax(
-      torch.where(segment_pos == 0, pos, torch.zeros_like(pos)), dim=-1).values
-  answer = torch.maximum(start, pos - window).to(torch.int32).contiguous()
+  answer = ops.attention_first_key(segment_pos, window)
   _first_key[:] = [weakref.ref(segment_pos), now, window, answer]
   return answer
 
@@ -391,6 +387,18 @@ class LocalAttentionBlock(nn.Module):
     q = q.reshape(b, t, self.num_heads, self.head_dim)
     k = k.reshape(b, t, 1, self.head_dim)
     v = v.reshape(b, t, 1, self.head_dim)
+    if cache is None and ops.attention_prefill_supported(q):
+      # bf16, head_dim 256: rotary embedding, scores, mask, softmax, values
+      # and the ring cache in two launches (the mask of modules.py:86-127 for
+      # a prompt is a band: a query sees from the start of its document, or
+      # the window's width back, up to itself)
+      out, ring_k, ring_v, count = ops.attention_prompt(
+          q, k, v, segment_pos, self._inv_freq,
+          _first_visible_key(segment_pos, self.window_size), self.window_size,
+          self.head_dim ** -0.5, return_cache)
+      return (self._project_out(out.reshape(b, t, self.width), defer_out),
+              AttentionBlockCache(keys=ring_k, values=ring_v, num_tokens=count)
+              if return_cache else None)
     # rotary embedding of queries and keys (modules.py:431-432), one kernel
     q, k = ops.rope_pair(q, k, segment_pos, self._inv_freq)
 
@@ -415,16 +423,6 @@ class LocalAttentionBlock(nn.Module):
       if return_cache:
         new_cache = self._cache_from_prompt(k, v, segment_pos,
                                             self.window_size)
-      if ops.attention_prefill_supported(q):
-        # bf16, head_dim 256: scores, mask, softmax and values in one kernel
-        # (the mask of modules.py:86-127 for a prompt is a band: a query sees
-        # from the start of its document, or the window's width back, up to
-        # itself)
-        out = ops.attention_prefill(
-            q, k, v, _first_visible_key(segment_pos, self.window_size),
-            self.head_dim ** -0.5)
-        return self._project_out(out.reshape(b, t, self.width),
-                                 defer_out), new_cache
       if (x.is_cuda and 1 < t <= self.window_size + 1 and
           _rows_are_one_document(segment_pos)):
         # one document per row, all of it inside the window: the mask of

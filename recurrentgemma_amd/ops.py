@@ -684,6 +684,53 @@ def attention_prefill(q, k, v, first_key, scale):
   return out
 
 
+def attention_first_key(positions, window):
+  """[B, T] int32: the first key each query of a prompt sees -- the later of
+  the first token of its document (the latest position 0, else the start of
+  the row) and `window` tokens back."""
+  B, T = positions.shape
+  pos, is64 = _segpos(positions, B, T)
+  first = torch.empty((B, T), dtype=torch.int32, device=pos.device)
+  with _on(pos.device):
+    _lib.check(_lib.lib().rg_attention_first_key(
+        _p(pos), is64, _p(first), B, T, window, _stream(pos)))
+  return first
+
+
+def attention_prompt(q, k, v, positions, inv_freq, first_key, window, scale,
+                     return_cache=True):
+  """A prompt's attention from the projections' outputs (before the rotary
+  embedding): q [B,T,H,256], k and v [B,T,1,256] or [B,T,256], first_key
+  [B,T] int32.  Returns (out [B,T,H,256], ring keys and values
+  [B,window,1,256], num_tokens [B] int32) -- the last three None without
+  return_cache.  Shapes as attention_prefill_supported says."""
+  B, T, H, hd = q.shape
+  q = _dev(q, "q")
+  k = _dev(k.reshape(B, T, hd), "k")
+  v = _dev(v.reshape(B, T, hd), "v")
+  _same(q.dtype, q.device, k=k, v=v)
+  pos, is64 = _segpos(positions, B, T)
+  inv = _dev(inv_freq, "inv_freq")
+  assert inv.dtype == torch.float32 and inv.shape == (hd // 4,)
+  assert first_key.shape == (B, T) and first_key.dtype == torch.int32
+  first_key = _dev(first_key, "first_key")
+  out = torch.empty_like(q)
+  ring_k = ring_v = count = None
+  if return_cache:
+    ring_k = torch.empty((B, window, 1, hd), dtype=q.dtype, device=q.device)
+    ring_v = torch.empty_like(ring_k)
+    count = torch.empty((B,), dtype=torch.int32, device=q.device)
+  lib = _lib.lib()
+  work = torch.empty(lib.rg_attention_prompt_workspace_bytes(B, T),
+                     dtype=torch.uint8, device=q.device)
+  with _on(q.device):
+    _lib.check(lib.rg_attention_prompt(
+        _p(q), _p(k), _p(v), _p(pos), is64, _p(inv), _p(first_key), _p(out),
+        _p(ring_k), _p(ring_v), _p(count), _p(work), B, T, H, hd, window,
+        float(scale), _dtype_code(q), _stream(q)))
+  return out, ring_k, ring_v, count
+
+
 def attention_decode_probs(scores, q, k_new, num_tokens, scale):
   """softmax over the written ring slots and the new token: scores
   [B, heads, window] (unscaled), q [B, heads, hd], k_new [B, hd], num_tokens

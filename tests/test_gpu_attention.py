@@ -8,7 +8,7 @@ the library's attention routine where the mask is one it can take."""
 import pytest
 import torch
 
-from recurrentgemma_amd import ops
+from recurrentgemma_amd import griffin, ops
 from tests import helpers
 
 pytestmark = pytest.mark.gpu
@@ -119,6 +119,47 @@ def test_attention_prefill_against_library_attention(B, T, H, window):
   want = want.transpose(1, 2)
   helpers.assert_close_elementwise(got, want, rtol=2e-2, atol_of_max=2e-2,
                                    what="attention vs library")
+
+
+@pytest.mark.parametrize("B,T,H,window,layout", [
+    (1, 1, 2, 16, "one"), (2, 31, 1, 16, "padded"), (3, 33, 10, 2048, "padded"),
+    (2, 64, 3, 64, "documents"), (2, 65, 2, 64, "padded"),
+    (1, 1025, 2, 48, "documents"), (5, 300, 4, 100, "documents"),
+    (2, 2100, 1, 2048, "padded"), (1, 3000, 2, 700, "int64")])
+@pytest.mark.parametrize("return_cache", [True, False])
+def test_attention_prompt_equals_its_parts(B, T, H, window, layout,
+                                           return_cache):
+  """One call from the projections' outputs against the rotary embedding, the
+  attention kernel and the ring cache as separate steps: the same arithmetic,
+  so the same bits."""
+  hd = 256
+  g = torch.Generator().manual_seed(B * 1000 + T)
+  q, k, v = (torch.randn(B, T, n, hd, generator=g).bfloat16().cuda()
+             for n in (H, 1, 1))
+  at = torch.arange(T).expand(B, T)
+  if layout == "padded":
+    seg = (at - torch.randint(0, T // 2 + 1, (B, 1), generator=g)).clamp(min=-1)
+  elif layout == "documents":
+    starts = torch.rand(B, T, generator=g) < 0.02
+    seg = at - torch.cummax(torch.where(starts, at, 0), dim=1).values
+    seg[0] += 5  # a row that continues a document
+  else:
+    seg = at.clone()
+  seg = seg.to("cuda", torch.int64 if layout == "int64" else torch.int32)
+  inv = griffin._inv_frequencies(hd, "cuda")
+  first = ops.attention_first_key(seg, window)
+  assert torch.equal(first, band(seg, window))
+  got, ring_k, ring_v, count = ops.attention_prompt(
+      q, k, v, seg, inv, first, window, hd ** -0.5, return_cache)
+  qr, kr = ops.rope_pair(q, k, seg, inv)
+  assert torch.equal(got, ops.attention_prefill(qr, kr, v, first, hd ** -0.5))
+  if not return_cache:
+    assert ring_k is None and ring_v is None and count is None
+    return
+  want = griffin.LocalAttentionBlock._cache_from_prompt(kr, v, seg, window)
+  assert torch.equal(ring_k, want.keys)
+  assert torch.equal(ring_v, want.values)
+  assert count.dtype == torch.int32 and torch.equal(count, want.num_tokens)
 
 
 def test_attention_prefill_refuses_other_shapes():
