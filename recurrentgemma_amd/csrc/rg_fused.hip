@@ -55,17 +55,23 @@ pack_gate_weights_kernel(const uint16_t* __restrict__ w_x,
 //
 // Replaces Conv1D.forward's decode branch (layers.py:469-474, 491-529) and
 // RGLRU.forward / rnn_scan with T == 1 (layers.py:313-365, 170-177).
-// ROWS = 32 rows of a tile, or 16 where 32 would leave CUs without a
-// workgroup (the matrix instructions then run half empty, which costs
+// ROWS = 32 rows of a tile, or 16 or 8 where that would leave CUs without a
+// workgroup (the matrix instructions then run partly empty, which costs
 // nothing here: a step is loads and stores).
 
 // GELU: y leaves as y * gelu(gate_branch), the join of the recurrent block's
 // two branches (recurrentgemma/torch/modules.py:627-628, 644) with the
 // arithmetic and roundings of the stand-alone gelu_mul pass.
-template <bool GELU, int ROWS>
-__global__ void __launch_bounds__(512) block_step_bf16_kernel(StepArgs p) {
+// WAVES = 8: a workgroup has a whole head; 2: a quarter of its channels (see
+// launch_block_step_bf16), each of a head's four workgroups repeating the
+// conv step of all 256 channels and storing the conv state of its own.
+template <bool GELU, int ROWS, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+block_step_bf16_kernel(StepArgs p) {
   constexpr int kStepRows = ROWS;
-  constexpr int kStepRowsPerThread = ROWS / 8;  // rows x 64 channel quads / 512
+  constexpr int kSlices = 8 / WAVES;  // workgroups per head
+  // rows x 64 channel quads / threads
+  constexpr int kStepRowsPerThread = ROWS / WAVES;
   constexpr int kRuns = ROWS / 2;  // of a lane's 16 accumulator rows: in use
   // (32 rows staged whatever ROWS is: the matrix instructions read 32)
   __shared__ __align__(16) uint16_t stage[32 * kLdsStride];
@@ -85,12 +91,14 @@ __global__ void __launch_bounds__(512) block_step_bf16_kernel(StepArgs p) {
     const int per_xcd = (int)gridDim.x / 8;
     if (pair < 8 * per_xcd) pair = (pair & 7) * per_xcd + (pair >> 3);
   }
-  const int h = pair / tiles;
-  const int b0 = (pair - h * tiles) * kStepRows;
+  const int slice = pair / tiles % kSlices;
+  const int h = pair / (tiles * kSlices);
+  const int b0 = pair % tiles * kStepRows;
   const int B = p.B;
   const int64_t W = p.W;
   const bool upper = lane >= 32;
-  const int n0 = wave * 32;
+  const int group = slice * WAVES + wave;  // of 32 channels
+  const int n0 = group * 32;
   const int ch = h * kBW + n0 + (lane & 31);
 
   // Everything per row goes through descriptors over this tile's rows only:
@@ -190,7 +198,7 @@ __global__ void __launch_bounds__(512) block_step_bf16_kernel(StepArgs p) {
   Frag bfrag[16][2];
   {
     const f32x4* src = reinterpret_cast<const f32x4*>(p.w_packed) +
-                       ((int64_t)(h * 8 + wave) * 16 * 2) * 64 + lane;
+                       ((int64_t)(h * 8 + group) * 16 * 2) * 64 + lane;
 #pragma unroll
     for (int ks = 0; ks < 16; ++ks)
 #pragma unroll
@@ -203,6 +211,9 @@ __global__ void __launch_bounds__(512) block_step_bf16_kernel(StepArgs p) {
 
   // ---- conv step of this tile's rows -> LDS (bf16), new conv state ---------
   {
+    // (channels of the head's other workgroups: out of range, dropped)
+    const uint32_t c_out = kSlices == 1 || cq / (8 * WAVES) == slice
+                               ? 2u * c : kBufferOutOfRange;
 #pragma unroll
     for (int j = 0; j < kStepRowsPerThread; ++j) {
       const uint32_t row = rg * kStepRowsPerThread + j;
@@ -224,11 +235,11 @@ __global__ void __launch_bounds__(512) block_step_bf16_kernel(StepArgs p) {
       }
       *reinterpret_cast<u32x2*>(stage + (size_t)row * kLdsStride + cq * 4) =
           packed;
-      __builtin_amdgcn_raw_buffer_store_b64(s1[j], rcout, 2u * c,
+      __builtin_amdgcn_raw_buffer_store_b64(s1[j], rcout, c_out,
                                             (row * 3u + 0u) * row_bytes, 0);
-      __builtin_amdgcn_raw_buffer_store_b64(s2[j], rcout, 2u * c,
+      __builtin_amdgcn_raw_buffer_store_b64(s2[j], rcout, c_out,
                                             (row * 3u + 1u) * row_bytes, 0);
-      __builtin_amdgcn_raw_buffer_store_b64(xr[j], rcout, 2u * c,
+      __builtin_amdgcn_raw_buffer_store_b64(xr[j], rcout, c_out,
                                             (row * 3u + 2u) * row_bytes, 0);
     }
   }
@@ -335,24 +346,59 @@ hipError_t launch_pack_gate_weights(const void* w_x, const void* w_a,
   return hipGetLastError();
 }
 
+namespace {
+
+template <int ROWS, int WAVES>
+void step(const StepArgs& a, hipStream_t s) {
+  const int64_t tiles = (a.B + ROWS - 1) / ROWS;
+  const dim3 grid((unsigned)(tiles * a.H * (8 / WAVES)));
+  if (a.gate_branch)
+    block_step_bf16_kernel<true, ROWS, WAVES><<<grid, 64 * WAVES, 0, s>>>(a);
+  else
+    block_step_bf16_kernel<false, ROWS, WAVES><<<grid, 64 * WAVES, 0, s>>>(a);
+}
+
+bool overlap(const void* a, const void* b, int64_t bytes) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return x < y + (uintptr_t)bytes && y < x + (uintptr_t)bytes;
+}
+
+}  // namespace
+
+// How a step is dealt out.  What bounds a workgroup is what its CU draws: a
+// head's 256 KB of weights at some 60 bytes a ns (4 us) and the rows, whose
+// loads are issued whether the rows exist or not.  So: the fewest rows and the
+// smallest share of a head per workgroup that one round of the 256 CUs holds
+// (a second round costs more than either saves).  us a step, replayed from a
+// graph over 24 sets of weights, rows x share of a head:
+//   width 2560, 10 heads   32 x 1  16 x 1   8 x 1  16 x 1/2  16 x 1/4  8 x 1/4
+//     1 row                  9.0     7.3     6.5       5.5       4.9      4.3
+//     48                       -     7.7     7.1       5.9       5.3      4.7
+//     64 (1/4 of 8: 320)     7.8     7.8     7.1       5.9       5.3      6.2
+//     128 (1/4 of 16: 320)   8.7     8.8     8.1       6.8       7.1      8.2
+//     192 (1/4 of 16: 480)     -    10.2     9.5       8.1       8.7     10.7
+//     256 (8 x 1: 320)      11.0    10.9    15.2      11.4      13.7     13.0
+//   width 4096, 16 heads
+//     32                       -     7.7     6.9       5.9       5.5      4.8
+//     128 (16 x 1/2: 256)   10.7    10.6     9.7       8.2       9.2     11.1
+//     256 (16 x 1: 256)        -    12.0    17.1      12.5      15.4     18.0
+// A head is shared among workgroups only where what all of them read -- x and
+// the conv state -- is not written in the same launch; a step that updates its
+// caches in place keeps whole heads.
 hipError_t launch_block_step_bf16(const StepArgs& a, hipStream_t s) {
   // needs head width 256 (checked by the caller)
-  const int tiles32 = (a.B + 31) / 32;
-  if (tiles32 <= 0 || (int64_t)tiles32 * 2 * a.H > 0x7fffffff)
-    return hipErrorInvalidValue;
-  // tiles of 16 rows while 32 would give fewer workgroups than CUs (256 rows
-  // x 16 heads: 128 workgroups 10.2 us, 256 workgroups 9.0 us, 512 of 8 rows
-  // 13.6 us a step)
-  const bool half = (int64_t)tiles32 * a.H < 256 && a.B > 16;
-  const int tiles = half ? (a.B + 15) / 16 : tiles32;
-  const dim3 grid((unsigned)(tiles * a.H));
-  if (a.gate_branch) {
-    if (half) block_step_bf16_kernel<true, 16><<<grid, 512, 0, s>>>(a);
-    else block_step_bf16_kernel<true, 32><<<grid, 512, 0, s>>>(a);
-  } else {
-    if (half) block_step_bf16_kernel<false, 16><<<grid, 512, 0, s>>>(a);
-    else block_step_bf16_kernel<false, 32><<<grid, 512, 0, s>>>(a);
-  }
+  const int64_t tiles8 = ((int64_t)a.B + 7) / 8, tiles16 = (tiles8 + 1) / 2;
+  if (tiles8 <= 0 || tiles8 * 4 * a.H > 0x7fffffff) return hipErrorInvalidValue;
+  constexpr int64_t kCUs = 256;
+  const int64_t row = (int64_t)a.W * 2;
+  const bool shared = !overlap(a.cache_in, a.cache_out, a.B * 3 * row) &&
+                      !overlap(a.x, a.y, a.B * row);
+  if (shared && tiles8 * a.H * 4 <= kCUs) step<8, 2>(a, s);
+  else if (shared && tiles16 * a.H * 4 <= kCUs) step<16, 2>(a, s);
+  else if (shared && tiles16 * a.H * 2 <= kCUs) step<16, 4>(a, s);
+  else if (tiles8 * a.H <= kCUs) step<8, 8>(a, s);
+  else if ((tiles16 + 1) / 2 * a.H < kCUs) step<16, 8>(a, s);
+  else step<32, 8>(a, s);
   return hipGetLastError();
 }
 
