@@ -384,6 +384,15 @@ struct SumTask {
 constexpr int kMaxSumTasks = 8;
 hipError_t launch_sum_rows(const SumTask* tasks, int count, int dtype,
                            hipStream_t s);
+// rg_gates_wgrad_f32.hip: weight gradients of both gate projections in float32
+// (256-wide heads); workspace may be null where it needs no bytes.
+bool gates_wgrad_f32_serves(int64_t M, int W, int H);
+size_t gates_wgrad_f32_workspace_bytes(int64_t M, int W, int H);
+hipError_t launch_gates_wgrad_f32(const void* x, const void* dgx,
+                                  const void* dga, void* dwx, void* dwa,
+                                  void* workspace, int64_t M, int W, int H,
+                                  hipStream_t s);
+
 // rg_gates_wgrad.hip: weight and bias gradients of both gate projections
 bool gates_wgrad_serves(int64_t M, int W, int H);
 size_t gates_wgrad_workspace_bytes(int64_t M, int W, int H);

@@ -284,10 +284,23 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
     Tensor* db[2] = {&r.db_x, &r.db_a};
     const bool needs_w[2] = {need_.w_x, need_.w_a};
     const bool needs_b[2] = {need_.b_x, need_.b_a};
+    const bool pair = need_.w_x && need_.w_a &&
+                      rg::gates_wgrad_f32_serves(d.M(), (int)d.W, (int)H);
+    if (pair) {
+      r.dw_x = empty({H, bw, bw}, x);
+      r.dw_a = empty({H, bw, bw}, x);
+      const size_t bytes =
+          rg::gates_wgrad_f32_workspace_bytes(d.M(), (int)d.W, (int)H);
+      Tensor ws;
+      if (bytes) ws = empty({(int64_t)bytes}, at::kByte, x);
+      check_hip(rg::launch_gates_wgrad_f32(in(x), in(dgx), in(dga), out(r.dw_x),
+                                           out(r.dw_a), out(ws), d.M(), (int)d.W,
+                                           (int)H, d.stream));
+    }
     for (int i = 0; i < 2; ++i) {
       // added to the recurrence's share where it lies
       at::baddbmm_out(dxs, dxs, dgs[i], w[i]->transpose(1, 2), 1, 1);
-      if (needs_w[i]) *dw[i] = at::bmm(xs.transpose(1, 2), dgs[i]);
+      if (needs_w[i] && !pair) *dw[i] = at::bmm(xs.transpose(1, 2), dgs[i]);
       if (!needs_b[i]) continue;
       if (tiles)
         *db[i] = sums.add(bias_rows, i * d.B * d.W, d.B, d.W, d.W, {H, bw}, x);

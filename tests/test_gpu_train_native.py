@@ -107,6 +107,16 @@ def test_rglru_gradients(B, T, width, heads, dtype):
     close(g, w, dtype, i)
 
 
+# rows around one wave's batch (8), one step of a workgroup (32) and the edges
+# of row ranges (128, 512 rows), one to sixteen ranges, the last one short or
+# empty
+@pytest.mark.parametrize("B,T,heads", [(1, 7, 1), (1, 31, 1), (1, 33, 2),
+                                       (1, 129, 1), (3, 171, 1), (1, 2049, 1),
+                                       (2, 350, 10), (1, 300, 16), (1, 161, 33)])
+def test_float32_gate_weight_gradients(B, T, heads):
+  test_rglru_gradients(B, T, 256 * heads, heads, F32)
+
+
 def test_frozen_parts_and_wrapped_layers():
   """Only what needs a gradient gets one, and a hooked layer is called."""
   block, x, pos = make(2, 70, 512, 2, BF16)
