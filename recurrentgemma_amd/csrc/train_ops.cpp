@@ -152,10 +152,15 @@ void gated_forward(const Tensor& x, const Tensor& pos, const GateWeights& g,
   const bool tiles = on_tiles(d);
   const bool f32 = d.code == RG_DTYPE_F32;
   if (f32) {
-    // the library's batched products, on strided views: no permuted copies
-    Tensor xs = by_head(x, H), gxs = by_head(gx, H), gas = by_head(ga, H);
-    at::bmm_out(gxs, xs, g.w_x);
-    at::bmm_out(gas, xs, g.w_a);
+    if (rg::gates_f32_serves(d.M(), (int)d.W, (int)H)) {
+      check_hip(rg::launch_gates_f32(in(x), in(g.w_x), in(g.w_a), out(gx), out(ga),
+                                     d.M(), (int)d.W, (int)H, d.stream));
+    } else {
+      // the library's batched products, on strided views: no permuted copies
+      Tensor xs = by_head(x, H), gxs = by_head(gx, H), gas = by_head(ga, H);
+      at::bmm_out(gxs, xs, g.w_x);
+      at::bmm_out(gas, xs, g.w_a);
+    }
     if (!tiles) {
       gx.view({-1, d.W}).add_(g.b_x.view({1, d.W}));
       ga.view({-1, d.W}).add_(g.b_a.view({1, d.W}));
