@@ -359,10 +359,14 @@ attn_prefill_bf16_kernel(AttnPrefillArgs p) {
         // (no visible key so far: keep every exponent finite)
         const float alpha = __builtin_amdgcn_exp2f(
             m_run - (m_new == -__builtin_inff() ? 0.0f : m_new));
+        // (before a query's first visible key its accumulators are zeros)
+        const bool started = __ballot(m_run != -__builtin_inff()) != 0;
         m_run = m_new;
         l_run *= alpha;
-        wait_for_matrix_results();
-        acc_scale(alpha, std::make_integer_sequence<int, 128>{});
+        if (started) {
+          wait_for_matrix_results();
+          acc_scale(alpha, std::make_integer_sequence<int, 128>{});
+        }
       }
       const float m_sub = m_run == -__builtin_inff() ? 0.0f : m_run;
       AFrag pf[2 * kAttnKB];
