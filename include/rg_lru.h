@@ -577,11 +577,17 @@ int rg_recurrent_step_gelu_mul(const void* x, const void* gate_branch,
  *   tanh, product); out may alias x.
  * rg_argmax_rows: out[r] = index of the largest of x[r, 0..n), the first among
  *   equals, NaN above everything (torch.argmax, greedy sampling,
- *   sampler.py:126-128); x [rows, n] contiguous, out int64. */
+ *   sampler.py:126-128); x [rows, n] contiguous, out int64.
+ * rg_argmax_rows_split: the same with several workgroups to a row, which need
+ *   a workspace of rg_argmax_workspace_bytes (0: one workgroup is enough, and
+ *   workspace may be NULL). */
 int rg_soft_cap(const void* x, void* out, int64_t n, float cap, int dtype,
                 void* stream);
 int rg_argmax_rows(const void* x, int64_t* out, int rows, int n, int dtype,
                    void* stream);
+size_t rg_argmax_workspace_bytes(int rows, int n);
+int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
+                         int n, int dtype, void* stream);
 
 /* Measurement aid, no counterpart in the reference: one wave per compute unit
  * runs `iters` (1 .. 2^20) rounds of 64 dependent multiply-adds (about 260

@@ -89,6 +89,8 @@ SIGNATURES = {
                           _i, _i, _i, _vp]),
     "rg_soft_cap": (_i, [_vp, _vp, ctypes.c_int64, ctypes.c_float, _i, _vp]),
     "rg_argmax_rows": (_i, [_vp, _vp, _i, _i, _i, _vp]),
+    "rg_argmax_workspace_bytes": (_sz, [_i, _i]),
+    "rg_argmax_rows_split": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
     "rg_linear_rows_partial": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "rg_add_rms_norm_partial": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i,
                                      ctypes.c_float, _i, _vp]),

@@ -1001,17 +1001,27 @@ int rg_clock_probe(uint64_t* out, int iters, void* stream) {
       __func__, rg::launch_clock_probe(out, iters, (hipStream_t)stream));
 }
 
-int rg_argmax_rows(const void* x, int64_t* out, int rows, int n, int dtype,
-                   void* stream) {
+size_t rg_argmax_workspace_bytes(int rows, int n) {
+  return rows > 0 && n > 0 ? rg::argmax_workspace_bytes(rows, n) : 0;
+}
+
+int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
+                         int n, int dtype, void* stream) {
   RG_CHECK_DTYPE(dtype);
   RG_REQUIRE(rows > 0 && n > 0, "%s: rows=%d n=%d must be positive", __func__,
              rows, n);
   RG_CHECK_PTR(x);
+  RG_CHECK_OPT_PTR(workspace);
   RG_REQUIRE(out != nullptr && ((uintptr_t)out & 7) == 0,
              "%s: out is null or not 8-byte aligned", __func__);
   return launch_status(__func__,
-                       rg::launch_argmax_rows(x, out, rows, n, dtype,
+                       rg::launch_argmax_rows(x, out, workspace, rows, n, dtype,
                                               (hipStream_t)stream));
+}
+
+int rg_argmax_rows(const void* x, int64_t* out, int rows, int n, int dtype,
+                   void* stream) {
+  return rg_argmax_rows_split(x, out, nullptr, rows, n, dtype, stream);
 }
 
 int rg_rms_norm(const void* x, const void* scale, void* out, int64_t rows,

@@ -303,22 +303,49 @@ soft_cap_kernel(const T* __restrict__ x, T* __restrict__ out, int64_t n,
 
 // Index of the largest element of every row (the first one among equals, a NaN
 // counts as larger than everything: torch.argmax's rule; greedy sampling,
-// recurrentgemma/torch/sampler.py:126-128).  One workgroup per row.
+// recurrentgemma/torch/sampler.py:126-128).  `parts` workgroups per row, each
+// with `len` elements (a multiple of 16 bytes); with more than one each leaves
+// its best element in `best`, which argmax_parts_kernel compares.  A workgroup
+// alone with a row of 256 000 is bound by its own comparisons (13 us) and by
+// one load in flight per thread.
+struct Best {
+  float v;
+  int i;  // kNone: no element
+};
+constexpr int kNone = 0x7fffffff;
+
+// a beats b: larger, or NaN where b is not; equal values keep the lower index
+__device__ __forceinline__ bool better(float v, int i, float w, int j) {
+  if (j == kNone) return true;
+  const bool vn = v != v, wn = w != w;
+  if (vn || wn) return vn && (!wn || i < j);
+  return v > w || (v == w && i < j);
+}
+
+__device__ __forceinline__ void best_of_wave(float& bv, int& bi) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float ov = __shfl_xor(bv, off, 64);
+    const int oi = __shfl_xor(bi, off, 64);
+    if (oi != kNone && better(ov, oi, bv, bi)) {
+      bv = ov;
+      bi = oi;
+    }
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(1024)
-argmax_rows_kernel(const T* __restrict__ x, int64_t* __restrict__ out, int n) {
+argmax_rows_kernel(const T* __restrict__ x, int64_t* __restrict__ out,
+                   Best* __restrict__ best, int row_n, int parts, int len) {
   __shared__ float best_v[16];
   __shared__ int best_i[16];
-  const T* row = x + (int64_t)blockIdx.x * n;
+  const int64_t at = blockIdx.x / parts;
+  const int begin = (int)(blockIdx.x % parts) * len;
+  const int n = row_n - begin < len ? row_n - begin : len;
+  const T* row = x + at * row_n + begin;
   float bv = 0.0f;
-  int bi = 0x7fffffff;
-  // a beats b: larger, or NaN where b is not; equal values keep the lower index
-  auto better = [](float v, int i, float w, int j) {
-    if (j == 0x7fffffff) return true;
-    const bool vn = v != v, wn = w != w;
-    if (vn || wn) return vn && (!wn || i < j);
-    return v > w || (v == w && i < j);
-  };
+  int bi = kNone;
   constexpr int kPer = 16 / sizeof(T);
   const int vec_n = ((reinterpret_cast<uintptr_t>(row) & 15) == 0) ? n / kPer : 0;
   for (int c = threadIdx.x; c < vec_n; c += 1024) {
@@ -341,15 +368,7 @@ argmax_rows_kernel(const T* __restrict__ x, int64_t* __restrict__ out, int n) {
       bi = i;
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const float ov = __shfl_xor(bv, off, 64);
-    const int oi = __shfl_xor(bi, off, 64);
-    if (oi != 0x7fffffff && better(ov, oi, bv, bi)) {
-      bv = ov;
-      bi = oi;
-    }
-  }
+  best_of_wave(bv, bi);
   if ((threadIdx.x & 63) == 0) {
     best_v[threadIdx.x >> 6] = bv;
     best_i[threadIdx.x >> 6] = bi;
@@ -357,13 +376,37 @@ argmax_rows_kernel(const T* __restrict__ x, int64_t* __restrict__ out, int n) {
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 16; ++w)
-      if (best_i[w] != 0x7fffffff && better(best_v[w], best_i[w], bv, bi)) {
+      if (best_i[w] != kNone && better(best_v[w], best_i[w], bv, bi)) {
         bv = best_v[w];
         bi = best_i[w];
       }
-    out[blockIdx.x] = bi;
+    if (parts == 1) out[at] = bi;
+    else best[blockIdx.x] = Best{bv, bi == kNone ? kNone : begin + bi};
   }
 }
+
+// One wave per row, one lane per part (at most 64).
+__global__ void __launch_bounds__(64)
+argmax_parts_kernel(const Best* __restrict__ best, int64_t* __restrict__ out,
+                    int parts) {
+  Best b{0.0f, kNone};
+  if ((int)threadIdx.x < parts) b = best[(int64_t)blockIdx.x * parts + threadIdx.x];
+  best_of_wave(b.v, b.i);
+  if (threadIdx.x == 0) out[blockIdx.x] = b.i;
+}
+
+// Workgroups per row: two to a CU over all rows, each with a load of 16 bytes
+// of bf16 per thread at least.  us with one to a row / with this, rows of
+// 256 000 bf16 logits: 1 row 38 / 9, 16 rows 40 / 13, 64 rows 42 / 19, 128 rows
+// 46 / 27, 256 rows 48 / 42.
+int argmax_parts(int rows, int n) {
+  int64_t parts = 512 / (rows > 512 ? 512 : rows);
+  const int64_t most = n / 8192;
+  if (parts > most) parts = most;
+  if (parts > 64) parts = 64;
+  return parts < 1 ? 1 : (int)parts;
+}
+
 
 }  // namespace
 
@@ -382,14 +425,27 @@ hipError_t launch_soft_cap(const void* x, void* out, int64_t n, float cap,
   return hipGetLastError();
 }
 
-hipError_t launch_argmax_rows(const void* x, int64_t* out, int rows, int n,
-                              int dtype, hipStream_t s) {
+size_t argmax_workspace_bytes(int rows, int n) {
+  const int parts = argmax_parts(rows, n);
+  return parts == 1 ? 0 : (size_t)rows * parts * sizeof(Best);
+}
+
+hipError_t launch_argmax_rows(const void* x, int64_t* out, void* workspace,
+                              int rows, int n, int dtype, hipStream_t s) {
+  const int parts = workspace ? argmax_parts(rows, n) : 1;
+  // (whole 16-byte items per part)
+  const int len = parts == 1 ? n : ((n + parts - 1) / parts + 7) / 8 * 8;
+  if ((int64_t)rows * parts > 0x7fffffff) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(rows * parts));
   if (dtype == 0)
-    argmax_rows_kernel<float><<<dim3((unsigned)rows), 1024, 0, s>>>(
-        (const float*)x, out, n);
+    argmax_rows_kernel<float><<<grid, 1024, 0, s>>>(
+        (const float*)x, out, (Best*)workspace, n, parts, len);
   else
-    argmax_rows_kernel<uint16_t><<<dim3((unsigned)rows), 1024, 0, s>>>(
-        (const uint16_t*)x, out, n);
+    argmax_rows_kernel<uint16_t><<<grid, 1024, 0, s>>>(
+        (const uint16_t*)x, out, (Best*)workspace, n, parts, len);
+  if (parts > 1)
+    argmax_parts_kernel<<<dim3((unsigned)rows), 64, 0, s>>>(
+        (const Best*)workspace, out, parts);
   return hipGetLastError();
 }
 

@@ -318,8 +318,10 @@ hipError_t launch_gelu_mul_backward(const void* dout, const void* a,
 // out = tanh(x / cap) * cap, n elements; out[r] = argmax(x[r, :n])
 hipError_t launch_soft_cap(const void* x, void* out, int64_t n, float cap,
                            int dtype, hipStream_t s);
-hipError_t launch_argmax_rows(const void* x, int64_t* out, int rows, int n,
-                              int dtype, hipStream_t s);
+size_t argmax_workspace_bytes(int rows, int n);
+// workspace: null, or of argmax_workspace_bytes (a row by several workgroups)
+hipError_t launch_argmax_rows(const void* x, int64_t* out, void* workspace,
+                              int rows, int n, int dtype, hipStream_t s);
 // out[r, :] = v * rsqrt(mean(v^2) + eps) * (scale + 1) with v = x[r, :], or,
 // with an addend, v = x[r, :] + addend[r, :] (also written to sum_out)
 hipError_t launch_rms_norm(const void* x, const void* addend, const void* scale,

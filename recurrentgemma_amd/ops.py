@@ -594,10 +594,15 @@ def argmax_last(x):
   """torch.argmax(x, dim=-1) (first index among equals), one pass."""
   x = _dev(x, "x")
   n = x.shape[-1]
+  rows = x.numel() // n
   out = torch.empty(x.shape[:-1], dtype=torch.int64, device=x.device)
+  lib = _lib.lib()
+  need = lib.rg_argmax_workspace_bytes(rows, n)
+  work = (torch.empty(need, dtype=torch.uint8, device=x.device) if need
+          else None)
   with _on(x.device):
-    _lib.check(_lib.lib().rg_argmax_rows(_p(x), _p(out), x.numel() // n, n,
-                                         _dtype_code(x), _stream(x)))
+    _lib.check(lib.rg_argmax_rows_split(_p(x), _p(out), _p(work), rows, n,
+                                        _dtype_code(x), _stream(x)))
   return out
 
 

@@ -381,6 +381,26 @@ def test_argmax_kernel(dtype):
   assert torch.equal(ops.argmax_last(odd), torch.argmax(odd, dim=-1))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,n", [(1, 8191), (1, 16384), (3, 16385),
+                                    (2, 70001), (255, 16400), (257, 16400),
+                                    (1, 1000003)])
+def test_argmax_kernel_rows_in_parts(dtype, rows, n):
+  """Rows that several workgroups share, on both sides of every line: equal
+  maxima in different parts, a NaN in the last one, infinities only."""
+  from recurrentgemma_amd import ops
+  gen = torch.Generator().manual_seed(n)
+  x = torch.randn(rows, n, generator=gen).to(dtype).to(DEV)
+  for variant in range(4):
+    if variant == 1:
+      x[0, n // 3] = x[0, n - 2] = 90.0
+    if variant == 2:
+      x[rows - 1] = float("-inf")
+    if variant == 3:
+      x[0, n - 1] = x[0, n - 9] = float("nan")
+    assert torch.equal(ops.argmax_last(x), torch.argmax(x, dim=-1)), variant
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-4),
                                        (torch.bfloat16, 3e-2)])
 def test_prompt_attention_causal_shortcut(monkeypatch, dtype, tol):
