@@ -37,8 +37,10 @@ union Frag {
 constexpr int kXStride = 72;  // elements per staged x row: 64 + 8 of padding
 constexpr int kWaves = 8;
 
-__host__ __device__ constexpr int wave_lds_bytes(int nt) {
-  return nt * 8192 > 64 * kXStride * 2 ? nt * 8192 : 64 * kXStride * 2;
+// LDS of a wave: its x tile (whole blocks of 32 rows) or its sums.
+__host__ __device__ constexpr int wave_lds_bytes(int nt, int blocks) {
+  const int sums = nt * blocks * 4096, x = 32 * blocks * kXStride * 2;
+  return sums > x ? sums : x;
 }
 
 enum LinearMode { kStore = 0, kGeluPair = 1, kPartial = 2 };
@@ -57,11 +59,16 @@ __device__ __forceinline__ size_t out_index(int m, int n, int M, int gw) {
   return ((size_t)grp * M + m) * gw + (n - grp * gw);
 }
 
-template <int NT, int MODE>
+// XR: rows of x that are loaded and staged (M rounded up to 16, 32 or 64).
+// Every workgroup draws all of x beside its weights: 64 rows are twice the
+// bytes of one tile's weights, whether the rows exist or not.
+template <int NT, int MODE, int XR>
 __global__ void __launch_bounds__(kWaves * 64)
 linear_rows_kernel(LinearArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  constexpr int kWaveLds = wave_lds_bytes(NT);
+  constexpr int kLoads = XR / 8;          // of x per chunk
+  constexpr int kMB = XR > 32 ? 2 : 1;    // blocks of 32 result rows
+  constexpr int kWaveLds = wave_lds_bytes(NT, kMB);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 31, g = lane >> 5;
   const int M = p.M, K = p.K;
@@ -74,13 +81,14 @@ linear_rows_kernel(LinearArgs p) {
   const int c1 = min(wg1, c0 + per);
   uint16_t* xs = reinterpret_cast<uint16_t*>(smem + (size_t)wave * kWaveLds);
 
-  // x chunk = 64 rows x 128 B; load j covers rows 8 j + lane / 8 (rows >= M
-  // repeat row M - 1; their results are never stored)
+  // x chunk = XR rows x 128 B; load j covers rows 8 j + lane / 8 (rows >= M
+  // repeat row M - 1, rows >= XR of the tile hold what LDS held: their results
+  // are never stored)
   const int xrow = lane >> 3, xseg = lane & 7;
   const uint16_t* x = reinterpret_cast<const uint16_t*>(p.x);
-  const uint16_t* xg[8];
+  const uint16_t* xg[kLoads];
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
+  for (int j = 0; j < kLoads; ++j)
     xg[j] = x + (size_t)min(8 * j + xrow, M - 1) * K + 8 * xseg;
   const u32x4* wg[NT];
 #pragma unroll
@@ -88,21 +96,21 @@ linear_rows_kernel(LinearArgs p) {
     wg[t] = reinterpret_cast<const u32x4*>(p.w_packed) +
             ((size_t)(blockIdx.x * NT + t) * (K / 16)) * 64 + lane;
 
-  f32x16 acc[NT][2];
+  f32x16 acc[NT][kMB];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+    for (int m = 0; m < kMB; ++m)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[t][m][i] = 0.0f;
 
-  u32x4 xr[8];
+  u32x4 xr[kLoads];
   Frag wq[2][NT][4];
   // loads of the chunk after the last one read the last one again
   auto load_chunk = [&](int c, int slot) {
     const int cc = min(c, chunks - 1);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < kLoads; ++j)
       xr[j] = *reinterpret_cast<const u32x4*>(xg[j] + (size_t)cc * 64);
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -113,23 +121,25 @@ linear_rows_kernel(LinearArgs p) {
   };
   auto body = [&](int slot, int c) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < kLoads; ++j)
       *reinterpret_cast<u32x4*>(xs + (8 * j + xrow) * kXStride + 8 * xseg) =
           xr[j];
-    Frag xf[4][2];
+    Frag xf[4][kMB];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int m = 0; m < 2; ++m)
+      for (int m = 0; m < kMB; ++m)
         xf[k][m].u = *reinterpret_cast<const u32x4*>(
             xs + (32 * m + r) * kXStride + 16 * k + 8 * g);
     load_chunk(c + 1, slot ^ 1);
+    // (the next chunk's loads stay in front of this one's products)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
+        for (int m = 0; m < kMB; ++m)
           acc[t][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               wq[slot][t][k].v, xf[k][m].v, acc[t][m], 0, 0, 0);
   };
@@ -148,10 +158,10 @@ linear_rows_kernel(LinearArgs p) {
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+    for (int m = 0; m < kMB; ++m)
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        mine[((t * 2 + m) * 16 + i) * 64 + lane] = acc[t][m][i];
+        mine[((t * kMB + m) * 16 + i) * 64 + lane] = acc[t][m][i];
   lds_barrier();
   const float* red = reinterpret_cast<const float*>(smem);
   // sum of accumulator registers 4 q .. 4 q + 3 of (tile t, half m, lane l):
@@ -161,7 +171,7 @@ linear_rows_kernel(LinearArgs p) {
     for (int i = 0; i < 4; ++i) v[i] = 0.0f;
     for (int wv = 0; wv < kWaves; ++wv) {
       const float* src = red + (size_t)wv * (kWaveLds / 4) +
-                         ((t * 2 + m) * 16 + q * 4) * 64 + l;
+                         ((t * kMB + m) * 16 + q * 4) * 64 + l;
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] += src[i * 64];
     }
@@ -172,7 +182,7 @@ linear_rows_kernel(LinearArgs p) {
     // tile 0 = 32 rows of the gate half, tile 1 = the same rows of the up half
     static_assert(MODE != kGeluPair || NT == 2, "pairs need two tiles");
     const int half = p.N / 2;
-    for (int qd = threadIdx.x; qd < 2 * 4 * 64; qd += kWaves * 64) {
+    for (int qd = threadIdx.x; qd < kMB * 4 * 64; qd += kWaves * 64) {
       const int l = qd & 63, q = (qd >> 6) & 3, m = qd >> 8;
       const int row = 32 * m + (l & 31);
       const int col = blockIdx.x * 32 + 8 * q + 4 * (l >> 5);
@@ -199,8 +209,9 @@ linear_rows_kernel(LinearArgs p) {
     }
     return;
   }
-  for (int qd = threadIdx.x; qd < NT * 2 * 4 * 64; qd += kWaves * 64) {
-    const int l = qd & 63, q = (qd >> 6) & 3, m = (qd >> 8) & 1, t = qd >> 9;
+  for (int qd = threadIdx.x; qd < NT * kMB * 4 * 64; qd += kWaves * 64) {
+    const int l = qd & 63, q = (qd >> 6) & 3, m = (qd >> 8) % kMB;
+    const int t = (qd >> 8) / kMB;
     const int row = 32 * m + (l & 31);
     const int col = (blockIdx.x * NT + t) * 32 + 8 * q + 4 * (l >> 5);
     if (row >= M) continue;
@@ -299,15 +310,33 @@ linear_pack_kernel(const uint16_t* __restrict__ w, u32x4* __restrict__ packed,
   packed[idx] = v;
 }
 
-template <int NT, int MODE>
-hipError_t launch_rows(const LinearArgs& a, dim3 grid, hipStream_t s) {
-  constexpr int lds = kWaves * wave_lds_bytes(NT);
+template <int NT, int MODE, int XR>
+hipError_t launch_rows_of(const LinearArgs& a, dim3 grid, hipStream_t s) {
+  constexpr int lds = kWaves * wave_lds_bytes(NT, XR > 32 ? 2 : 1);
   static OncePerDevice once;  // one per instantiation of this launcher
   hipError_t e = set_max_dynamic_lds(
-      once, (const void*)linear_rows_kernel<NT, MODE>, lds);
+      once, (const void*)linear_rows_kernel<NT, MODE, XR>, lds);
   if (e != hipSuccess) return e;
-  linear_rows_kernel<NT, MODE><<<grid, kWaves * 64, lds, s>>>(a);
+  linear_rows_kernel<NT, MODE, XR><<<grid, kWaves * 64, lds, s>>>(a);
   return hipGetLastError();
+}
+
+// How many rows of x a launch loads and stages.  us a layer, replayed from a
+// graph over 16 sets of weights, always 64 rows and without the barrier that
+// keeps the next chunk's loads in front of the products / as it is:
+//   rows                     1           16           32           64
+//   K 2560, N 2560     8.7 /  6.5   8.7 /  7.6   9.9 /  9.1  11.8 / 11.3
+//   K 2560, N 5120    10.6 /  7.6  10.8 /  9.3  10.3 / 10.1  12.6 / 12.1
+//   K 7680, N 2560    12.7 / 11.2  13.1 / 12.0  14.6 / 13.6  17.1 / 16.2
+//   K 4096, N 8192    17.8 / 15.1  17.9 / 15.4  17.9 / 16.7  20.7 / 20.0
+// (8 staged rows are within 2 % of 16.  Fewer rows without the barrier are
+// slower than 64, 10.0 us for one row at 2560 x 2560: the compiler moves the
+// loads behind the products.)
+template <int NT, int MODE>
+hipError_t launch_rows(const LinearArgs& a, dim3 grid, hipStream_t s) {
+  if (a.M <= 16) return launch_rows_of<NT, MODE, 16>(a, grid, s);
+  if (a.M <= 32) return launch_rows_of<NT, MODE, 32>(a, grid, s);
+  return launch_rows_of<NT, MODE, 64>(a, grid, s);
 }
 
 }  // namespace

@@ -40,6 +40,14 @@ def _check(got, x, w_rows, bias):
   assert worst <= 0, worst
 
 
+# either side of every number of rows that is staged, in each way the sums
+# leave the kernel
+@pytest.mark.parametrize("M", [15, 16, 17, 32, 33])
+@pytest.mark.parametrize("K,N", [(192, 96), (5120, 64), (64, 12800)])
+def test_linear_rows_by_rows_staged(M, K, N):
+  test_linear_rows(M, K, N, True)
+
+
 @pytest.mark.parametrize("M,K,N,with_bias", [
     (64, 2560, 2560, True),    # one tile of 32 weight rows per workgroup
     (5, 128, 64, False),       # fewer rows than a tile, two chunks of K
