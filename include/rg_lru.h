@@ -452,30 +452,6 @@ int rg_attention_prefill(const void* q, const void* k, const void* v_t,
                          int T_pad, int H, int head_dim, float scale, int dtype,
                          void* stream);
 
-/* first_key of rg_attention_prefill for a prompt's positions [B,T]
- * (int32/int64): max(last position 0 at or before the query, else 0;
- * t - window) -- the mask of recurrentgemma/torch/modules.py:86-127. */
-int rg_attention_first_key(const void* positions, int positions_is_i64,
-                           int32_t* first_key, int B, int T, int window,
-                           void* stream);
-
-/* A prompt pass of the local-attention block between its projections
- * (modules.py:431-476, ring cache :253-283) in two launches: rg_rope_pair on q
- * and k, rg_attention_prefill, and the cache it leaves.  q, out [B,T,H,256],
- * k, v [B,T,256] as the projections leave them, inv_freq [64], first_key
- * [B,T]; ring_keys, ring_values [B,window,256] and num_tokens [B] are written
- * whole (all three NULL: no cache); workspace of
- * rg_attention_prompt_workspace_bytes(B, T).  RG_ERR_UNSUPPORTED as for
- * rg_attention_prefill. */
-size_t rg_attention_prompt_workspace_bytes(int B, int T);
-int rg_attention_prompt(const void* q, const void* k, const void* v,
-                        const void* positions, int positions_is_i64,
-                        const float* inv_freq, const int32_t* first_key,
-                        void* out, void* ring_keys, void* ring_values,
-                        int32_t* num_tokens, void* workspace, int B, int T,
-                        int H, int head_dim, int window, float scale, int dtype,
-                        void* stream);
-
 /* Masked softmax of one decoded token against the ring cache and itself
  * (modules.py:152-183 `_compute_cache_mask`, :462-470): scores
  * [B, heads, window] = q . k of the ring slots, unscaled, in `dtype`; q
@@ -577,17 +553,11 @@ int rg_recurrent_step_gelu_mul(const void* x, const void* gate_branch,
  *   tanh, product); out may alias x.
  * rg_argmax_rows: out[r] = index of the largest of x[r, 0..n), the first among
  *   equals, NaN above everything (torch.argmax, greedy sampling,
- *   sampler.py:126-128); x [rows, n] contiguous, out int64.
- * rg_argmax_rows_split: the same with several workgroups to a row, which need
- *   a workspace of rg_argmax_workspace_bytes (0: one workgroup is enough, and
- *   workspace may be NULL). */
+ *   sampler.py:126-128); x [rows, n] contiguous, out int64. */
 int rg_soft_cap(const void* x, void* out, int64_t n, float cap, int dtype,
                 void* stream);
 int rg_argmax_rows(const void* x, int64_t* out, int rows, int n, int dtype,
                    void* stream);
-size_t rg_argmax_workspace_bytes(int rows, int n);
-int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
-                         int n, int dtype, void* stream);
 
 /* Measurement aid, no counterpart in the reference: one wave per compute unit
  * runs `iters` (1 .. 2^20) rounds of 64 dependent multiply-adds (about 260

@@ -61,10 +61,6 @@ SIGNATURES = {
                                 _i, _i, _i, _vp]),
     "rg_attention_prefill": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i,
                                   ctypes.c_float, _i, _vp]),
-    "rg_attention_first_key": (_i, [_vp, _i, _vp, _i, _i, _i, _vp]),
-    "rg_attention_prompt_workspace_bytes": (_sz, [_i, _i]),
-    "rg_attention_prompt": (_i, [_vp, _vp, _vp, _vp, _i] + [_vp] * 7 +
-                            [_i] * 5 + [ctypes.c_float, _i, _vp]),
     "rg_rglru_backward": (_i, [_vp] * 14 + [_i, _i, _i, _i, _vp]),
     "rg_scan_split_workspace_bytes": (_sz, [_i, _i, _i]),
     "rg_lru_scan_fused_split": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i,
@@ -89,8 +85,6 @@ SIGNATURES = {
                           _i, _i, _i, _vp]),
     "rg_soft_cap": (_i, [_vp, _vp, ctypes.c_int64, ctypes.c_float, _i, _vp]),
     "rg_argmax_rows": (_i, [_vp, _vp, _i, _i, _i, _vp]),
-    "rg_argmax_workspace_bytes": (_sz, [_i, _i]),
-    "rg_argmax_rows_split": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
     "rg_linear_rows_partial": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "rg_add_rms_norm_partial": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i,
                                      ctypes.c_float, _i, _vp]),
@@ -115,6 +109,16 @@ SIGNATURES = {
     "rg_recurrent_step": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i,
                                _vp]),
+}
+
+# csrc/rg_package_calls.h: for this package's modules only
+PACKAGE_SIGNATURES = {
+    "rg_attention_first_key": (_i, [_vp, _i, _vp, _i, _i, _i, _vp]),
+    "rg_attention_prompt_workspace_bytes": (_sz, [_i, _i]),
+    "rg_attention_prompt": (_i, [_vp, _vp, _vp, _vp, _i] + [_vp] * 7 +
+                            [_i] * 5 + [ctypes.c_float, _i, _vp]),
+    "rg_argmax_workspace_bytes": (_sz, [_i, _i]),
+    "rg_argmax_rows_split": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
 }
 
 _lib = None
@@ -147,7 +151,7 @@ def lib() -> ctypes.CDLL:
           "(or __graft_entry__.build()). recurrentgemma_amd has no fallback "
           "path without its HIP library.")
     handle = ctypes.CDLL(LIB_PATH)
-    for name, (res, args) in SIGNATURES.items():
+    for name, (res, args) in {**SIGNATURES, **PACKAGE_SIGNATURES}.items():
       fn = getattr(handle, name)
       fn.restype = res
       fn.argtypes = args

@@ -6,6 +6,7 @@
 
 #include "../../include/rg_lru.h"
 #include "rg_internal.h"
+#include "rg_package_calls.h"
 
 namespace {
 

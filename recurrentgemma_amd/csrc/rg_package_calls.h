@@ -1,0 +1,49 @@
+/* Entry points that this package's own Python calls beside the public C
+ * interface of include/rg_lru.h (same conventions: device pointers, a stream,
+ * RG_OK or an error code, rg_last_error): steps fused the way its modules chain
+ * them, free to change with those. */
+#ifndef RG_PACKAGE_CALLS_H_
+#define RG_PACKAGE_CALLS_H_
+
+#include "../../include/rg_lru.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* first_key of rg_attention_prefill for a prompt's positions [B,T]
+ * (int32/int64): max(last position 0 at or before the query, else 0;
+ * t - window) -- the mask of recurrentgemma/torch/modules.py:86-127. */
+int rg_attention_first_key(const void* positions, int positions_is_i64,
+                           int32_t* first_key, int B, int T, int window,
+                           void* stream);
+
+/* A prompt pass of the local-attention block between its projections
+ * (modules.py:431-476, ring cache :253-283) in two launches: rg_rope_pair on q
+ * and k, rg_attention_prefill, and the cache it leaves.  q, out [B,T,H,256],
+ * k, v [B,T,256] as the projections leave them, inv_freq [64], first_key
+ * [B,T]; ring_keys, ring_values [B,window,256] and num_tokens [B] are written
+ * whole (all three NULL: no cache); workspace of
+ * rg_attention_prompt_workspace_bytes(B, T).  RG_ERR_UNSUPPORTED as for
+ * rg_attention_prefill. */
+size_t rg_attention_prompt_workspace_bytes(int B, int T);
+int rg_attention_prompt(const void* q, const void* k, const void* v,
+                        const void* positions, int positions_is_i64,
+                        const float* inv_freq, const int32_t* first_key,
+                        void* out, void* ring_keys, void* ring_values,
+                        int32_t* num_tokens, void* workspace, int B, int T,
+                        int H, int head_dim, int window, float scale, int dtype,
+                        void* stream);
+
+/* rg_argmax_rows with several workgroups to a row, which need a workspace of
+ * rg_argmax_workspace_bytes (0: one workgroup is enough, and workspace may be
+ * NULL). */
+size_t rg_argmax_workspace_bytes(int rows, int n);
+int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
+                         int n, int dtype, void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif  /* RG_PACKAGE_CALLS_H_ */
