@@ -49,9 +49,10 @@ pack_gate_weights_kernel(const uint16_t* __restrict__ w_x,
 
 // One token per sequence row: the same chain (conv step from the carried conv
 // state, both gate projections, gate arithmetic, one recurrence step) with the
-// 32 rows of a tile being different sequences.  One workgroup per (tile of 32
-// rows, head).  Every state element is read and then written by the same
-// thread, so the outputs may alias the inputs (in-place caches).
+// rows of a tile being different sequences.  One workgroup per (tile of rows,
+// head or share of a head).  With whole heads every state element is read and
+// then written by the same workgroup, loads before stores, so the outputs may
+// alias the inputs (in-place caches).
 //
 // Replaces Conv1D.forward's decode branch (layers.py:469-474, 491-529) and
 // RGLRU.forward / rnn_scan with T == 1 (layers.py:313-365, 170-177).
