@@ -118,13 +118,14 @@ struct TileAt {
 // that alternate between the lane halves) to its outputs: gates, the tile as
 // (prod a, state from zero), the workgroup's barrier, the fold of the pass's
 // TILES tiles, replay, stores.  CH: channels of the workgroup, c0: this wave's
-// first among them, n0: in the head.
+// first among them, n0: in the head.  until: how many tiles after the pass's
+// first the next row opens (0: that one does), kept up to date here.
 template <class L, int TILES, int CH, bool GELU>
 __device__ __forceinline__ void gate_and_scan(
     const FusedArgs& p, lds_byte* const lds3, const int lane, const int wave,
     const int bw, const int h, const int n0, const int c0, const int tt,
     const int buf, const int tiles_per_row, const TileAt at_tile,
-    const f32x16& acc_x, const f32x16& acc_a, float& carry) {
+    const f32x16& acc_x, const f32x16& acc_a, float& carry, int& until) {
   const int T = p.T;
   const int64_t W = p.W;
   const uint32_t row_bytes = 2u * (uint32_t)p.W;
@@ -232,8 +233,7 @@ __device__ __forceinline__ void gate_and_scan(
           th = __builtin_fmaf(run_p[g][s], th, run_h[g][s]);
           tp *= run_p[g][s];
         }
-      // a tile that opens its row cuts it from what came before: its state from
-      // the row's h0 in place of the state from zero, product 0
+      // a tile that opens its row starts from the row's h0 instead of from zero
       if (k_in_row == 0) {
         const float first =
             p.h0 && any && ch_valid
@@ -241,7 +241,6 @@ __device__ __forceinline__ void gate_and_scan(
                       (const char*)(p.h0 + (int64_t)b * W) + state_off)
                 : 0.0f;
         th = __builtin_fmaf(tp, first, th);
-        tp = 0.0f;
         if (any) carry = first;
       }
       {
@@ -259,12 +258,28 @@ __device__ __forceinline__ void gate_and_scan(
 #pragma unroll
         for (int k = 0; k < TILES; ++k) v[k] = all[k * CH + (ln & 31)];
         float s = carry;
-        const bool opens = k_in_row == 0;
+        // (us without the cut: B4 T2048 W5632 129.9, B3 T333 W2560 22.61.  Passes
+        // of two tiles branch past the selections, 129.9 against 131.0; passes of
+        // four, which open a row more often, do them always, 22.64 against 22.72)
+        if (TILES == 2 && __builtin_expect(until >= TILES, 1)) {
 #pragma unroll
-        for (int k = 0; k < TILES; ++k) {
-          if (k == tt && !opens) hin = s;
-          s = __builtin_fmaf(v[k][0], s, v[k][1]);
+          for (int k = 0; k < TILES; ++k) {
+            if (k == tt) hin = s;
+            s = __builtin_fmaf(v[k][0], s, v[k][1]);
+          }
+        } else {
+          // rows open in this pass: cut from the row before by selection (a
+          // product of zero would let that row's NaN or infinity through)
+          const bool opens = k_in_row == 0;
+#pragma unroll
+          for (int k = 0; k < TILES; ++k) {
+            if (k == tt && !opens) hin = s;
+            const float next = __builtin_fmaf(v[k][0], s, v[k][1]);
+            s = k == until ? v[k][1] : next;
+            until += k == until ? tiles_per_row : 0;
+          }
         }
+        until -= TILES;
         carry = s;
       }
       if (active) {
@@ -654,6 +669,7 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
       (uint32_t)(tt * kTile + (lane & 31)) * L::row + 16u * (lane >> 5);
   // state behind the last tile of the pass before, of the row it belongs to
   float carry = 0.0f;
+  int until = 0;
 
   // (the last pass apart: it has no conv to do, and accumulators that two
   // paths lead to would be copied behind their matrix instructions)
@@ -696,7 +712,7 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
     }
     gate_and_scan<L, kTiles, kSlice, GELU>(
         p, lds3, lane, wave, bw, h, n0, half * 32, tt, buf, tiles_per_row,
-        TileAt{b, t0, k_in_row, any, active, starts}, acc_x, acc_a, carry);
+        TileAt{b, t0, k_in_row, any, active, starts}, acc_x, acc_a, carry, until);
     starts = (uint32_t)(mask >> 32);
   };
   for (int i = 0; i + 1 < npasses; ++i) pass(i, std::true_type{});
@@ -920,6 +936,7 @@ block_prefill_narrow_bf16_kernel(FusedArgs p, int slices, int groups) {
     const uint32_t a_lane =
         (uint32_t)(tt * kTile + (lane & 31)) * L::row + 16u * (lane >> 5);
     float carry = 0.0f;
+    int until = 0;
     for (int i = 0; i < npasses; ++i) {
       const int buf = i & 1;
       const At now = asked;
@@ -934,7 +951,7 @@ block_prefill_narrow_bf16_kernel(FusedArgs p, int slices, int groups) {
           p, lds3, lane, wave, bw, h, n0, c0, tt, buf, tiles_per_row,
           TileAt{any ? now.row : row0, now.k * kTile, now.k, any,
                  any && n0 < bw, starts},
-          acc_x, acc_a, carry);
+          acc_x, acc_a, carry, until);
     }
   }
   if (p.cache_out)

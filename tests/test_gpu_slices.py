@@ -86,3 +86,62 @@ def test_slices_without_packed_weights(B, T, bw, H):
       None, ptr(y2), ptr(h2), ptr(c2), None, 0, B, T, W, H, 1,
       torch.cuda.current_stream().cuda_stream))
   assert torch.equal(y1, y2) and torch.equal(h1, h2) and torch.equal(c1, c2)
+
+
+def _core(x, seg, ws, h0=None, packed=True):
+  """recurrent_core, or the same C call without re-laid-out weights."""
+  if packed:
+    return ops.recurrent_core(x, seg, *ws, h0=h0)
+  B, T, W = x.shape
+  H = ws[2].shape[0]
+  lib = _lib.lib()
+  assert lib.rg_recurrent_core_workspace_bytes(B, T, W, H, 1) == 0
+  conv = ws[0] is not None
+  y, c = torch.empty_like(x), x.new_empty(B, 3, W) if conv else None
+  h = torch.empty(B, W, dtype=torch.float32, device=DEV)
+  ptr = lambda t: None if t is None else t.data_ptr()
+  _lib.check(lib.rg_recurrent_core(
+      ptr(x), None, ptr(seg), 1, *[ptr(t) for t in ws[:6]], None, ptr(ws[6]),
+      ptr(h0), ptr(y), ptr(h), ptr(c), None, 0, B, T, W, H, 1,
+      torch.cuda.current_stream().cuda_stream))
+  return y, h, c
+
+
+@pytest.mark.parametrize("B,T,bw,H", [
+    # several rows per workgroup, of one tile, a few and many; whole and cut
+    # last tiles; passes that hold several rows, one, and the end of one and
+    # the start of the next
+    (8, 10, 256, 10), (8, 32, 256, 10), (8, 45, 256, 10), (8, 100, 256, 10),
+    (8, 200, 256, 10), (7, 333, 256, 16), (8, 440, 256, 10), (3, 333, 256, 10),
+    (9, 10, 176, 32), (9, 32, 176, 32), (8, 50, 176, 32), (7, 100, 176, 32),
+    (8, 333, 176, 32), (6, 1000, 176, 32), (8, 70, 200, 12)])
+@pytest.mark.parametrize("packed", [True, False])
+def test_rows_do_not_see_each_other(B, T, bw, H, packed):
+  """A NaN or an infinity in one row's x or h0 leaves every other row's outputs
+  as they are, bit for bit."""
+  W = bw * H
+  p = R.make_params(W, H, torch.bfloat16, seed=41, gate_bias_std=0.4)
+  ws = [p[n].to(DEV) for n in NAMES]
+  g = torch.Generator().manual_seed(42)
+  x = torch.randn(B, T, W, generator=g).bfloat16().to(DEV)
+  h0 = torch.randn(B, W, generator=g).to(DEV)
+  seg = helpers.document_positions(B, T, 60, seed=43).to(DEV)
+  seg[:, 0] = 7  # (rows go on from h0, and no start shields the first token)
+  bare = [None, None] + ws[2:]
+  clean = _core(x, seg, ws, packed=packed)
+  carried = _core(x, seg, bare, h0, packed)
+  assert all(torch.isfinite(t).all() for t in clean + carried[:2])
+  for bad in range(B):
+    value = (float("nan"), float("inf"), float("-inf"))[bad % 3]
+    others = [b for b in range(B) if b != bad]
+    xb, hb = x.clone(), h0.clone()
+    xb[bad, T // 3, ::5] = value
+    hb[bad, ::3] = value
+    got = _core(xb, seg, ws, packed=packed)
+    assert not torch.isfinite(got[0][bad]).all()
+    for a, b in zip(got, clean):
+      assert torch.equal(a[others], b[others]), (bad, value)
+    got = _core(x, seg, bare, hb, packed)
+    assert not torch.isfinite(got[1][bad]).all()
+    for a, b in zip(got[:2], carried[:2]):
+      assert torch.equal(a[others], b[others]), (bad, value, "h0")
