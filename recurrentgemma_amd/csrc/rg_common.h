@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rg_internal.h"
+
 namespace rg {
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -142,10 +144,6 @@ __device__ __forceinline__ float round_act<uint16_t>(float v) {
 }
 
 // ------------------------------------------------------ segment_pos ----
-// How document starts are encoded: int32 / int64 positions (start == 0), or a
-// byte mask (start != 0) as rnn_scan's `reset` argument.
-enum SegKind { kSegI32 = 0, kSegI64 = 1, kSegMaskU8 = 2 };
-
 __device__ __forceinline__ bool is_doc_start(const void* segpos, int kind,
                                              int64_t idx) {
   if (kind == kSegI64) return reinterpret_cast<const int64_t*>(segpos)[idx] == 0;

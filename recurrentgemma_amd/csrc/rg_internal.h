@@ -10,6 +10,10 @@
 
 namespace rg {
 
+// How document starts are encoded: int32 / int64 positions (start == 0), or a
+// byte mask (start != 0) as rnn_scan's `reset` argument.
+enum SegKind { kSegI32 = 0, kSegI64 = 1, kSegMaskU8 = 2 };
+
 // Raises a kernel's dynamic LDS limit the first time it is launched on a
 // device; later launches on that device only read the flag (the attribute is a
 // property of the loaded function, it does not have to be set per launch).
@@ -285,6 +289,10 @@ struct ScanTileArgs {
   float* dlam;           // [B, W], gated backward: each row's share
   float* dbias;          // gated float32 backward, or null: [2][B, W], each
                          // row's sums of the gates' gradients
+  // gated forward, or null: what the backward pass is to read in place of
+  // tensors that the caller may have written to by then
+  uint8_t* starts_out;   // [B, T], 1 where a document starts
+  float* bias_out;       // float32: [2][W]
   int B, T, W;
 };
 enum ScanTileMode { kTilesFwdPlain, kTilesBwdPlain, kTilesFwdGated, kTilesBwdGated };

@@ -200,10 +200,13 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
       lds.sp[tid] = softplus_precise(lambda_of(tid));
       if (kBias) {
 #pragma unroll
-        for (int g = 0; g < 2; ++g)
+        for (int g = 0; g < 2; ++g) {
           lds.bias[g][tid] = p.bias[g] && c0 + tid < p.W
                                  ? load_scalar((const T*)p.bias[g] + c0 + tid)
                                  : 0.0f;
+          if (MODE == kFwdGated && p.bias_out && b == 0 && c0 + tid < p.W)
+            p.bias_out[(int64_t)g * p.W + c0 + tid] = lds.bias[g][tid];
+        }
       }
     }
     __syncthreads();
@@ -280,6 +283,9 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
     {
       const uint64_t mask = __ballot(flag_in && (flag_lo | flag_hi) == 0u);
       starts = (uint32_t)(mask >> ((kBwd ? 7 - q : q) * KL)) & ((1u << KL) - 1u);
+      if (MODE == kFwdGated && p.starts_out && c0 == 0 && flag_in)
+        p.starts_out[(int64_t)b * T_len + first_token(step, wave * 8) + lane] =
+            (flag_lo | flag_hi) == 0u;
     }
     if (more) {
       load_flags(step + 1);

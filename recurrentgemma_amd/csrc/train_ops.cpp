@@ -77,6 +77,14 @@ struct Dims {
 };
 int seg_kind(const Tensor& pos) { return pos.scalar_type() == at::kLong ? 1 : 0; }
 
+// What the backward pass of the RG-LRU reads besides the tensors whose values
+// it may count on (autograd raises if those were written to in between): a
+// caller's positions and biases may hold the next batch's by then.
+struct Kept {
+  Tensor starts;  // [B, T] bool, where documents start
+  Tensor bias;    // [2, W] float32 where the pre-activations are without them
+};
+
 // ---------------------------------------------------------- bare recurrence --
 
 void scan_forward(const Tensor& x, const Tensor& a, const Tensor& reset,
@@ -146,11 +154,18 @@ Tensor by_head(const Tensor& t, int64_t H) {
 
 void gated_forward(const Tensor& x, const Tensor& pos, const GateWeights& g,
                    const Tensor& h0, const Tensor& gx, const Tensor& ga,
-                   const Tensor& y, const Tensor& h) {
+                   const Tensor& y, const Tensor& h, Kept& kept,
+                   bool keep_starts) {
   const Dims d(x);
   const int64_t H = g.w_x.size(0);
   const bool tiles = on_tiles(d);
   const bool f32 = d.code == RG_DTYPE_F32;
+  if (tiles) {  // (written by the recurrence's kernel)
+    if (keep_starts) kept.starts = empty({d.B, d.T}, at::kBool, x);
+    if (f32) kept.bias = empty({2, d.W}, x);
+  } else if (keep_starts) {
+    kept.starts = at::eq(pos, 0);
+  }
   if (f32) {
     if (rg::gates_f32_serves(d.M(), (int)d.W, (int)H)) {
       check_hip(rg::launch_gates_f32(in(x), in(g.w_x), in(g.w_a), out(gx), out(ga),
@@ -181,7 +196,9 @@ void gated_forward(const Tensor& x, const Tensor& pos, const GateWeights& g,
     if (f32) {
       t.bias[0] = in(g.b_x);
       t.bias[1] = in(g.b_a);
+      t.bias_out = (float*)out(kept.bias);
     }
+    t.starts_out = (uint8_t*)out(kept.starts);
     t.init = (const float*)in(h0);
     t.out[0] = out(y);
     t.last = (float*)out(h);
@@ -233,12 +250,15 @@ struct GatedGrads {
   Tensor dx, dlam, dw_x, db_x, dw_a, db_a, dh0;
 };
 
+// kept.starts or, without it, pos
 GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
-                          const Tensor& pos, const GateWeights& g,
-                          const Tensor& gx, const Tensor& ga, const Tensor& y,
-                          const Tensor& h0, const GateNeeds& need_, Sums& sums) {
+                          const Tensor& pos, const Kept& kept,
+                          const Tensor& a_param, const Tensor& w_x,
+                          const Tensor& w_a, const Tensor& gx, const Tensor& ga,
+                          const Tensor& y, const Tensor& h0,
+                          const GateNeeds& need_, Sums& sums) {
   const Dims d(x);
-  const int64_t H = g.w_x.size(0), bw = d.W / H;
+  const int64_t H = w_x.size(0), bw = d.W / H;
   const bool f32 = d.code == RG_DTYPE_F32;
   GatedGrads r;
   r.dx = empty(x.sizes(), x);
@@ -253,12 +273,12 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
     t.in[2] = in(gx);
     t.in[3] = in(ga);
     t.in[4] = in(y);
-    t.flags = in(pos);
-    t.flag_kind = seg_kind(pos);
-    t.a_param = in(g.a_param);
+    t.flags = in(kept.starts.defined() ? kept.starts : pos);
+    t.flag_kind = kept.starts.defined() ? rg::kSegMaskU8 : seg_kind(pos);
+    t.a_param = in(a_param);
     if (f32) {
-      t.bias[0] = in(g.b_x);
-      t.bias[1] = in(g.b_a);
+      t.bias[0] = in(kept.bias);
+      t.bias[1] = kept.bias.const_data_ptr<float>() + d.W;
       bias_rows = empty({2, d.B, d.W}, at::kFloat, x);
       t.dbias = (float*)out(bias_rows);
     }
@@ -274,8 +294,8 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
     t.W = (int)d.W;
     check_hip(rg::launch_scan_tiles(t, rg::kTilesBwdGated, d.code, d.stream));
   } else {
-    Tensor reset = at::eq(pos, 0);
-    check(rg_rglru_backward(in(dy), in(x), in(gx), in(ga), in(g.a_param),
+    Tensor reset = kept.starts.defined() ? kept.starts : at::eq(pos, 0);
+    check(rg_rglru_backward(in(dy), in(x), in(gx), in(ga), in(a_param),
                             in(reset), in(y), in(h0), in(dh), out(r.dx), out(dgx),
                             out(dga), (float*)out(lam_rows), out(r.dh0), (int)d.B,
                             (int)d.T, (int)d.W, d.code, d.stream));
@@ -284,7 +304,7 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
   if (f32) {
     Tensor xs = by_head(x, H), dxs = by_head(r.dx, H);
     Tensor dgs[2] = {by_head(dgx, H), by_head(dga, H)};
-    const Tensor* w[2] = {&g.w_x, &g.w_a};
+    const Tensor* w[2] = {&w_x, &w_a};
     Tensor* dw[2] = {&r.dw_x, &r.dw_a};
     Tensor* db[2] = {&r.db_x, &r.db_a};
     const bool needs_w[2] = {need_.w_x, need_.w_a};
@@ -328,7 +348,7 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
                                 out(r.db_x), out(r.db_a), out(ws), bytes, d.M(),
                                 (int)d.W, (int)H, d.code, d.stream));
   }
-  check_hip(rg::launch_gates_dgrad(in(dgx), in(dga), in(g.w_x), in(g.w_a),
+  check_hip(rg::launch_gates_dgrad(in(dgx), in(dga), in(w_x), in(w_a),
                                    out(r.dx), d.M(), (int)d.W, (int)H, d.stream));
   return r;
 }
@@ -342,21 +362,24 @@ struct Rglru : Function<Rglru> {
     Tensor gx = empty(x.sizes(), x), ga = empty(x.sizes(), x);
     Tensor y = empty(x.sizes(), x);
     Tensor h = empty({x.size(0), x.size(2)}, at::kFloat, x);
-    gated_forward(x, pos, {a_param, w_x, b_x, w_a, b_a}, h0, gx, ga, y, h);
-    ctx->save_for_backward({x, pos, a_param, w_x, b_x, w_a, b_a, h0, gx, ga, y});
+    Kept kept;
+    gated_forward(x, pos, {a_param, w_x, b_x, w_a, b_a}, h0, gx, ga, y, h, kept,
+                  true);
+    ctx->save_for_backward(
+        {x, kept.starts, a_param, w_x, w_a, kept.bias, h0, gx, ga, y});
     return {y, h};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     at::AutoGradMode off(false);
     auto s = ctx->get_saved_variables();
-    const Tensor &x = s[0], &y = s[10];
+    const Tensor &x = s[0], &y = s[9];
     Tensor dy = grads[0].defined() ? dense_grad(grads[0], y.scalar_type())
                                    : at::zeros_like(y);
     Tensor dh;
     if (grads[1].defined()) dh = dense_grad(grads[1], at::kFloat);
     Sums sums;
     GatedGrads r = gated_backward(
-        dy, dh, x, s[1], {s[2], s[3], s[4], s[5], s[6]}, s[8], s[9], y, s[7],
+        dy, dh, x, Tensor(), {s[1], s[5]}, s[2], s[3], s[4], s[7], s[8], y, s[6],
         {ctx->needs_input_grad(3), ctx->needs_input_grad(4),
          ctx->needs_input_grad(5), ctx->needs_input_grad(6)},
         sums);
@@ -390,13 +413,15 @@ struct Block : Function<Block> {
                             d.code, d.stream));
     Tensor gx = empty(lx.sizes(), x), ga = empty(lx.sizes(), x);
     Tensor y = empty(lx.sizes(), x);
-    gated_forward(xc, pos, {a_param, w_x, b_x, w_a, b_a}, Tensor(), gx, ga, y, h);
+    Kept kept;  // (the conv's backward reads the positions themselves)
+    gated_forward(xc, pos, {a_param, w_x, b_x, w_a, b_a}, Tensor(), gx, ga, y, h,
+                  kept, false);
     Tensor join = empty(lx.sizes(), x);
     check(rg_gelu_mul(in(y), in(gate), out(join), d.M() * W, d.code, d.stream));
     Tensor result = at::linear(join.view({B * T, W}), w_out, b_out)
                         .view({B, T, w_out.size(0)});
-    ctx->save_for_backward({x, pos, w_y, w_lx, conv_w, a_param, w_x, b_x, w_a, b_a,
-                            w_out, gate, lx, xc, gx, ga, y, join});
+    ctx->save_for_backward({x, pos, w_y, w_lx, conv_w, a_param, w_x, w_a,
+                            kept.bias, w_out, gate, lx, xc, gx, ga, y, join});
     if (!want_cache) return {result};
     ctx->mark_non_differentiable({conv_state});
     return {result, h, conv_state};
@@ -405,8 +430,8 @@ struct Block : Function<Block> {
     at::AutoGradMode off(false);
     auto s = ctx->get_saved_variables();
     const Tensor &x = s[0], &pos = s[1], &w_y = s[2], &w_lx = s[3], &conv_w = s[4],
-                 &w_out = s[10], &gate = s[11], &lx = s[12], &xc = s[13],
-                 &y = s[16], &join = s[17];
+                 &w_out = s[9], &gate = s[10], &lx = s[11], &xc = s[12],
+                 &y = s[15], &join = s[16];
     const Dims d(lx);
     const int64_t M = d.M(), W = d.W;
     const Tensor x2 = x.view({M, x.size(2)});
@@ -443,8 +468,8 @@ struct Block : Function<Block> {
     if (grads.size() > 1 && grads[1].defined())
       dh = dense_grad(grads[1], at::kFloat);
     GatedGrads g = gated_backward(
-        dy, dh, xc, pos, {s[5], s[6], s[7], s[8], s[9]}, s[14], s[15], y, Tensor(),
-        {needs(9), needs(10), needs(11), needs(12)}, sums);
+        dy, dh, xc, pos, {Tensor(), s[8]}, s[5], s[6], s[7], s[13], s[14], y,
+        Tensor(), {needs(9), needs(10), needs(11), needs(12)}, sums);
     r[8] = g.dlam;
     r[9] = g.dw_x;
     r[10] = g.db_x;

@@ -148,3 +148,52 @@ def test_frozen_parts_and_wrapped_layers():
       block.rg_lru.input_gate.w, block.rg_lru.input_gate.b,
       block.rg_lru.a_gate.w, block.rg_lru.a_gate.b, block.linear_out.weight,
       block.linear_out.bias, False) is None
+
+
+@pytest.mark.parametrize("pos_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("B,T,width,heads,dtype", [
+    (2, 97, 512, 2, BF16), (3, 65, 512, 2, F32), (2, 300, 48, 2, F32),
+    (1, 33, 50, 2, F32)])
+def test_positions_and_biases_may_be_written_to_before_the_backward(
+    B, T, width, heads, dtype, pos_dtype):
+  """The RG-LRU's backward reads the positions and gate biases its forward read,
+  also where a caller has put the next batch's into the same buffers."""
+  block, x, pos = make(B, T, width, heads, dtype)
+  lru, pos = block.rg_lru, pos.to(pos_dtype)
+  dy = torch.randn_like(x)
+  wanted = [x] + list(lru.parameters())
+
+  def gradients(overwrite):
+    with training.differentiable():
+      y, h = lru(x, pos)
+      if overwrite:
+        pos.fill_(1)
+        with torch.no_grad():
+          lru.input_gate.b.add_(1)
+          lru.a_gate.b.add_(1)
+      return torch.autograd.grad((y, h), wanted, (dy, torch.ones_like(h)))
+
+  want = gradients(False)
+  for g, w in zip(gradients(True), want):
+    assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_block_biases_may_be_written_to_before_the_backward(dtype):
+  block, x, pos = make(2, 97, 512, 2, dtype)
+  wanted = [x] + list(block.parameters())
+  dy = torch.randn_like(x)
+
+  def gradients(overwrite):
+    with training.differentiable():
+      y, _ = block(x, pos, return_cache=False)
+      if overwrite:
+        with torch.no_grad():
+          for name, q in block.named_parameters():
+            if name.endswith("bias") or name.endswith(".b"):
+              q.add_(1)
+      return torch.autograd.grad(y, wanted, dy)
+
+  want = gradients(False)
+  for g, w in zip(gradients(True), want):
+    assert torch.equal(g, w)
