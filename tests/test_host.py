@@ -5,6 +5,7 @@ the drop-in modules keep the reference's surface (names, shapes, caches)."""
 import ctypes
 import os
 import re
+import types
 
 import pytest
 import torch
@@ -12,6 +13,7 @@ import torch
 import recurrentgemma_amd as rg
 from oracle import torch_ref as R
 from recurrentgemma_amd import _lib
+from recurrentgemma_amd import modules
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -327,6 +329,42 @@ def test_no_cpu_fallback():
   with pytest.raises(AssertionError):
     rg.rnn_scan(torch.zeros(1, 2, 4), torch.zeros(1, 2, 4, dtype=torch.bfloat16),
                 torch.zeros(1, 2, dtype=torch.bool), None)  # layers.py:163
+
+
+class _Forwarding(torch.nn.Module):
+  """A wrapper that passes attributes through, as torch.compile's and FSDP's."""
+
+  def __init__(self, inner):
+    super().__init__()
+    self.inner = inner
+
+  def __getattr__(self, name):
+    try:
+      return super().__getattr__(name)
+    except AttributeError:
+      return getattr(self.inner, name)
+
+
+@pytest.mark.parametrize("as_module", [False, True])
+def test_recurrent_core_takes_what_has_the_attributes(as_module):
+  """Its layers need not be this package's modules: what has their attributes
+  gets as far as the kernels (which refuse the CPU)."""
+  conv, lru = rg.Conv1D(8, 4), rg.RGLRU(8, 2)
+  if as_module:
+    like = (_Forwarding(conv), _Forwarding(lru))
+  else:
+    gates = [types.SimpleNamespace(w=g.w, b=g.b)
+             for g in (lru.input_gate, lru.a_gate)]
+    like = (types.SimpleNamespace(w=conv.w, b=conv.b, temporal_width=4),
+            types.SimpleNamespace(a_param=lru.a_param, input_gate=gates[0],
+                                  a_gate=gates[1]))
+  want = modules._core_weights(conv, lru)
+  assert all(a is b for a, b in zip(modules._core_weights(*like), want))
+  cache = rg.RecurrentBlock.init_cache(1, 8, torch.float32)
+  for tokens, given in ((5, None), (1, cache)):
+    with pytest.raises(RuntimeError, match="GPU only"):
+      rg.recurrent_core(*like, torch.randn(1, tokens, 8),
+                        torch.arange(tokens)[None], given)
 
 
 def test_missing_library_fails_loudly(monkeypatch):
