@@ -55,12 +55,66 @@ const void* in(const Tensor& t) {
 }
 void* out(const Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
 
-// A gradient from elsewhere in the graph as the kernels take it.
-Tensor dense_grad(const Tensor& t, at::ScalarType dtype) {
+// A tensor from elsewhere in the graph as the kernels take it.
+Tensor dense_tensor(const Tensor& t, at::ScalarType dtype) {
   if (t.scalar_type() == dtype && t.is_contiguous() &&
       !(reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u))
     return t;
   return t.to(dtype).clone(at::MemoryFormat::Contiguous);
+}
+
+// The saved tensors of a backward pass.  Under saved_tensors_hooks they are what
+// a hook returned, which may lie otherwise than what was saved (a copy is made)
+// or be something else (refused: the kernels count on sizes and types).  One of
+// them, [B, T, W], gives the sizes, type and device, the others have to fit.
+struct Saved {
+  variable_list v;
+  Tensor root;
+  int64_t B, T, W;
+  Saved(AutogradContext* ctx, int at) : v(ctx->get_saved_variables()) {
+    const Tensor& r = v[at];
+    fits(r.defined() && r.is_cuda() &&
+         r.device().index() == c10::hip::current_device() &&
+         (r.scalar_type() == at::kBFloat16 || r.scalar_type() == at::kFloat) &&
+         r.dim() == 3 && r.numel() > 0);
+    for (int i = 0; i < 3; ++i) fits(r.size(i) <= INT32_MAX);
+    root = dense_tensor(r, r.scalar_type());
+    B = r.size(0);
+    T = r.size(1);
+    W = r.size(2);
+  }
+  static void fits(bool ok) {
+    if (!ok)
+      throw KernelFailure(
+          "a tensor saved for the backward pass came back from its hook as "
+          "another one");
+  }
+  Tensor get(int i, at::IntArrayRef shape, at::ScalarType t) const {
+    fits(v[i].defined() && v[i].sizes() == shape && v[i].scalar_type() == t &&
+         v[i].device() == root.device());
+    return dense_tensor(v[i], t);
+  }
+  Tensor get(int i, at::IntArrayRef shape) const {
+    return get(i, shape, root.scalar_type());
+  }
+  Tensor like_root(int i) const { return get(i, root.sizes()); }
+  Tensor state(int i) const {  // [B, W], if there is one
+    return v[i].defined() ? get(i, {B, W}, at::kFloat) : Tensor();
+  }
+  // a weight of the gate projections
+  Tensor gate_weight(int i) const {
+    fits(v[i].defined() && v[i].dim() == 3);
+    const int64_t H = v[i].size(0), bw = v[i].size(1);
+    fits(H > 0 && H * bw == W &&
+         (root.scalar_type() == at::kFloat || bw == 256));
+    return get(i, {H, bw, bw});
+  }
+};
+// ... and the gradient of an output of these sizes, if there is one
+Tensor grad_of(const Tensor& grad, at::IntArrayRef shape, at::ScalarType t) {
+  if (!grad.defined()) return grad;
+  Saved::fits(grad.sizes() == shape);
+  return dense_tensor(grad, t);
 }
 
 struct Dims {
@@ -114,13 +168,13 @@ struct Scan : Function<Scan> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     at::AutoGradMode off(false);
-    auto saved = ctx->get_saved_variables();
-    const Tensor &a = saved[0], &reset = saved[1], &y = saved[2], &h0 = saved[3];
+    const Saved s(ctx, 2);
+    const Tensor a = s.like_root(0), reset = s.get(1, {s.B, s.T}, at::kBool),
+                 y = s.root, h0 = s.state(3);
     const Dims d(y);
-    Tensor dy = grads[0].defined() ? dense_grad(grads[0], y.scalar_type())
-                                   : at::zeros_like(y);
-    Tensor dh;
-    if (grads[1].defined()) dh = dense_grad(grads[1], at::kFloat);
+    Tensor dy = grad_of(grads[0], y.sizes(), y.scalar_type());
+    if (!dy.defined()) dy = at::zeros_like(y);
+    const Tensor dh = grad_of(grads[1], {d.B, d.W}, at::kFloat);
     Tensor dx = empty(y.sizes(), y), da = empty(y.sizes(), y), dh0;
     if (h0.defined()) dh0 = empty(h0.sizes(), h0);
     check(rg_linear_scan_backward(in(dy), in(a), in(reset), in(y), in(h0), in(dh),
@@ -144,6 +198,21 @@ bool on_tiles(const Dims& d) {
                               rg::kTilesFwdGated) &&
          rg::scan_tiles_serve((int)d.B, (int)d.T, (int)d.W, d.code,
                               rg::kTilesBwdGated);
+}
+
+// Kept::bias of a backward pass
+Tensor kept_bias(const Saved& s, int i) {
+  const Dims d(s.root);
+  if (d.code != RG_DTYPE_F32 || !on_tiles(d)) return Tensor();
+  return s.get(i, {2, s.W});
+}
+
+// What the block's sums over rows take.
+bool block_sums_serve(int64_t B, int64_t T, int64_t W, int64_t D, int code) {
+  const int per = code == RG_DTYPE_F32 ? 4 : 8;
+  return W % per == 0 && D % per == 0 &&
+         (B * T + rg::kColSumRows - 1) / rg::kColSumRows <= 65535 &&
+         rg::conv1d_backward_sums_dx((int)B, (int)T, (int)W, 4, code);
 }
 
 // [M, W] as a batch of heads [H, M, bw], no copy
@@ -371,15 +440,16 @@ struct Rglru : Function<Rglru> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     at::AutoGradMode off(false);
-    auto s = ctx->get_saved_variables();
-    const Tensor &x = s[0], &y = s[9];
-    Tensor dy = grads[0].defined() ? dense_grad(grads[0], y.scalar_type())
-                                   : at::zeros_like(y);
-    Tensor dh;
-    if (grads[1].defined()) dh = dense_grad(grads[1], at::kFloat);
+    const Saved s(ctx, 0);
+    const Tensor x = s.root, y = s.like_root(9);
+    const Kept kept{s.get(1, {s.B, s.T}, at::kBool), kept_bias(s, 5)};
+    Tensor dy = grad_of(grads[0], y.sizes(), y.scalar_type());
+    if (!dy.defined()) dy = at::zeros_like(y);
+    const Tensor dh = grad_of(grads[1], {s.B, s.W}, at::kFloat);
     Sums sums;
     GatedGrads r = gated_backward(
-        dy, dh, x, Tensor(), {s[1], s[5]}, s[2], s[3], s[4], s[7], s[8], y, s[6],
+        dy, dh, x, Tensor(), kept, s.get(2, {s.W}), s.gate_weight(3),
+        s.gate_weight(4), s.like_root(7), s.like_root(8), y, s.state(6),
         {ctx->needs_input_grad(3), ctx->needs_input_grad(4),
          ctx->needs_input_grad(5), ctx->needs_input_grad(6)},
         sums);
@@ -428,20 +498,28 @@ struct Block : Function<Block> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     at::AutoGradMode off(false);
-    auto s = ctx->get_saved_variables();
-    const Tensor &x = s[0], &pos = s[1], &w_y = s[2], &w_lx = s[3], &conv_w = s[4],
-                 &w_out = s[9], &gate = s[10], &lx = s[11], &xc = s[12],
-                 &y = s[15], &join = s[16];
+    const Saved s(ctx, 11);
+    const Tensor lx = s.root, gate = s.like_root(10), xc = s.like_root(12),
+                 y = s.like_root(15), join = s.like_root(16);
     const Dims d(lx);
     const int64_t M = d.M(), W = d.W;
-    const Tensor x2 = x.view({M, x.size(2)});
+    Saved::fits(s.v[0].defined() && s.v[0].dim() == 3 && s.v[1].defined());
+    const int64_t D = s.v[0].size(2);
+    const Tensor x = s.get(0, {d.B, d.T, D}), w_y = s.get(2, {W, D}),
+                 w_lx = s.get(3, {W, D}), conv_w = s.get(4, {4, W}),
+                 w_out = s.get(9, {D, W}),
+                 pos = s.get(1, {d.B, d.T},
+                             s.v[1].scalar_type() == at::kInt ? at::kInt
+                                                              : at::kLong);
+    Saved::fits(block_sums_serve(d.B, d.T, W, D, d.code));
+    const Tensor x2 = x.view({M, D});
     auto needs = [&](int i) { return ctx->needs_input_grad(i); };
     Sums sums;
     variable_list r(16);  // (the flag takes no gradient)
     Tensor dy, dgate2;
     if (grads[0].defined()) {
       const Tensor dout =
-          dense_grad(grads[0], x.scalar_type()).view({M, w_out.size(0)});
+          grad_of(grads[0], x.sizes(), x.scalar_type()).view({M, D});
       const int64_t parts = (M + rg::kColSumRows - 1) / rg::kColSumRows;
       if (needs(14)) {
         Tensor part = empty({parts, dout.size(1)}, at::kFloat, x);
@@ -465,10 +543,10 @@ struct Block : Function<Block> {
       dy = at::zeros_like(y);  // only the final state is differentiated
     }
     Tensor dh;
-    if (grads.size() > 1 && grads[1].defined())
-      dh = dense_grad(grads[1], at::kFloat);
+    if (grads.size() > 1) dh = grad_of(grads[1], {d.B, W}, at::kFloat);
     GatedGrads g = gated_backward(
-        dy, dh, xc, pos, {Tensor(), s[8]}, s[5], s[6], s[7], s[13], s[14], y,
+        dy, dh, xc, pos, {Tensor(), kept_bias(s, 8)}, s.get(5, {W}),
+        s.gate_weight(6), s.gate_weight(7), s.like_root(13), s.like_root(14), y,
         Tensor(), {needs(9), needs(10), needs(11), needs(12)}, sums);
     r[8] = g.dlam;
     r[9] = g.dw_x;
@@ -642,10 +720,7 @@ PyObject* train_block(PyObject*, PyObject* const* v, Py_ssize_t n) {
     gate_weights(c, v + 8, W);
     c.shaped(v[13], {D, W});
     c.shaped(v[14], {D});
-    const int per = c.code == RG_DTYPE_F32 ? 4 : 8;
-    need(W % per == 0 && D % per == 0 &&
-         (B * T + rg::kColSumRows - 1) / rg::kColSumRows <= 65535 &&
-         rg::conv1d_backward_sums_dx((int)B, (int)T, (int)W, 4, c.code));
+    need(block_sums_serve(B, T, W, D, c.code));
     const bool want_cache = v[15] == Py_True;
     variable_list r;
     {

@@ -197,3 +197,50 @@ def test_block_biases_may_be_written_to_before_the_backward(dtype):
   want = gradients(False)
   for g, w in zip(gradients(True), want):
     assert torch.equal(g, w)
+
+
+def _calls(dtype):
+  """One call of each native autograd function: (outputs, wanted) each."""
+  block, x, pos = make(2, 97, 512, 2, dtype)
+  h0 = torch.randn(2, 512, device="cuda").requires_grad_()
+  a = torch.rand_like(x.detach()).requires_grad_()
+  reset = pos == 0
+  lru = block.rg_lru
+  return {
+      "scan": (lambda: rg.rnn_scan(x, a, reset, h0), [x, a, h0]),
+      "rglru": (lambda: lru(x, pos, h0), [x, h0] + list(lru.parameters())),
+      "block": (lambda: block(x, pos, return_cache=False)[:1],
+                [x] + list(block.parameters()))}
+
+
+def _gradients(call, wanted, pack, unpack):
+  with training.differentiable():
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+      out = call()
+    return torch.autograd.grad(out, wanted, [torch.ones_like(o) for o in out])
+
+
+def _strided(t):
+  return torch.stack([t, t], dim=-1)[..., 0]
+
+
+def _off_by_one(t):
+  flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+  return flat[1:].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("name", ["scan", "rglru", "block"])
+def test_saved_tensors_come_back_as_they_like(dtype, name):
+  """What a hook returns for a saved tensor may lie anyhow; what is another
+  tensor is refused before a kernel runs on it."""
+  call, wanted = _calls(dtype)[name]
+  keep = lambda t: t.detach()
+  want = _gradients(call, wanted, keep, keep)
+  for unpack in (_strided, _off_by_one, lambda t: t.cpu().cuda()):
+    got = _gradients(call, wanted, keep, unpack)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+  for unpack in (lambda t: t[:1], lambda t: t.cpu(), lambda t: t.double(),
+                 lambda t: t.flatten()):
+    with pytest.raises(RuntimeError, match="came back from its hook"):
+      _gradients(call, wanted, keep, unpack)
