@@ -39,14 +39,11 @@ def _parameters(module, *names):
   half a microsecond each, which a decode step with its twenty tensors does
   not have; the dictionary behind it is read instead, and the attribute where
   the name is not in it (a parametrised weight, an object that is no module)."""
-  own = module._parameters if isinstance(module, nn.Module) else ()
+  try:
+    own = module._parameters
+  except AttributeError:
+    own = ()
   return [own[n] if n in own else getattr(module, n) for n in names]
-
-
-def _child(module, name):
-  """A submodule by name, in the same way."""
-  own = module._modules if isinstance(module, nn.Module) else ()
-  return own[name] if name in own else getattr(module, name)
 
 
 def _as_written(module, kind) -> bool:
@@ -68,9 +65,12 @@ def _core_weights(conv_1d, rg_lru):
   if compiled.tracing():
     gx, ga = rg_lru.input_gate, rg_lru.a_gate
     return conv_1d.w, conv_1d.b, gx.w, gx.b, ga.w, ga.b, rg_lru.a_param
-  return (*_parameters(conv_1d, "w", "b"),
-          *_parameters(_child(rg_lru, "input_gate"), "w", "b"),
-          *_parameters(_child(rg_lru, "a_gate"), "w", "b"),
+  try:
+    gx, ga = rg_lru._modules["input_gate"], rg_lru._modules["a_gate"]
+  except (AttributeError, KeyError):  # no module, or one that passes them through
+    gx, ga = rg_lru.input_gate, rg_lru.a_gate
+  return (*_parameters(conv_1d, "w", "b"), *_parameters(gx, "w", "b"),
+          *_parameters(ga, "w", "b"),
           *_parameters(rg_lru, "a_param"))
 
 
@@ -213,9 +213,10 @@ class RecurrentBlock(nn.Module):
           ops.PackedLinear.usable(x, self.width, self.lru_width) and
           ops.PackedLinear.usable(x, self.lru_width, self.width))
       if few_rows:
-        w_y, b_y = _parameters(_child(self, "linear_y"), "weight", "bias")
-        w_x, b_x = _parameters(_child(self, "linear_x"), "weight", "bias")
-        w_out, b_out = _parameters(_child(self, "linear_out"), "weight", "bias")
+        linear = self._modules
+        w_y, b_y = _parameters(linear["linear_y"], "weight", "bias")
+        w_x, b_x = _parameters(linear["linear_x"], "weight", "bias")
+        w_out, b_out = _parameters(linear["linear_out"], "weight", "bias")
         y, x = self._rows_yx(x, (w_y, w_x), (b_y, b_x))
       else:
         y = self.linear_y(x)
@@ -260,8 +261,9 @@ class RecurrentBlock(nn.Module):
     """The whole block as one native autograd function (csrc/train_ops.cpp), or
     None: where a layer has been wrapped, hooked or replaced, or the arguments
     are not as that function takes them."""
-    y, lx, out, conv, lru = (_child(self, n) for n in (
-        "linear_y", "linear_x", "linear_out", "conv_1d", "rg_lru"))
+    own = self._modules
+    y, lx, out = own["linear_y"], own["linear_x"], own["linear_out"]
+    conv, lru = own["conv_1d"], own["rg_lru"]
     if (compiled.tracing() or _global_hooks() or
         not (_as_written(y, nn.Linear) and _as_written(lx, nn.Linear) and
              _as_written(out, nn.Linear) and _as_written(conv, layers.Conv1D) and
