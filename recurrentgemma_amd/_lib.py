@@ -126,7 +126,8 @@ _host = None
 
 
 class KernelError(RuntimeError):
-  """A C-ABI call returned a non-zero status."""
+  """A C-ABI call returned a non-zero status, or was not made because its
+  arguments had changed under way."""
 
 
 def build(force: bool = True) -> str:

@@ -9,10 +9,11 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <memory>
-#include <stdexcept>
+#include <exception>
 #include <unordered_map>
 #include <vector>
 
@@ -24,9 +25,13 @@ inline PyObject* g_kernel_error = nullptr;  // _lib.KernelError
 
 struct Fallback {};  // take the general path
 struct Raised {};    // a Python exception is set
-// a kernel call failed where no Python exception can be set
-struct KernelFailure : std::runtime_error {
-  using std::runtime_error::runtime_error;
+// A kernel call failed where no Python exception can be set.  Torch gives it the
+// type it names where it leaves a backward pass, `guarded` elsewhere.
+struct KernelFailure : torch::PyTorchError {
+  using PyTorchError::PyTorchError;
+  PyObject* python_type() override {
+    return g_kernel_error ? g_kernel_error : PyExc_RuntimeError;
+  }
 };
 
 using at::Tensor;
@@ -139,7 +144,7 @@ inline PyObject* triple(const Tensor& a, const Tensor& b, const Tensor& c) {
 }
 
 // Entry points share this: Fallback becomes None, torch's exceptions become
-// Python's.
+// Python's, and Python's stay what they are.
 template <class F>
 PyObject* guarded(F&& f) {
   try {
@@ -151,8 +156,12 @@ PyObject* guarded(F&& f) {
   } catch (const c10::OutOfMemoryError&) {
     // (the general path asks again and raises torch's own exception)
     Py_RETURN_NONE;
-  } catch (const KernelFailure& e) {
-    PyErr_SetString(g_kernel_error ? g_kernel_error : PyExc_RuntimeError, e.what());
+  } catch (KernelFailure& e) {
+    PyErr_SetString(e.python_type(), e.what());
+    return nullptr;
+  } catch (python_error& e) {
+    // (raised by Python code that torch called, a hook for instance)
+    e.restore();
     return nullptr;
   } catch (const std::exception& e) {
     PyErr_SetString(PyExc_RuntimeError, e.what());

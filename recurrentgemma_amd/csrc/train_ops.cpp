@@ -27,8 +27,7 @@ using torch::autograd::variable_list;
 // (an absent last argument is no input edge: the indices before it stay)
 using OptTensor = std::optional<Tensor>;
 
-// Raised without the GIL, also on autograd's threads; `guarded` makes it the
-// package's exception.
+// Raised without the GIL, also on autograd's threads.
 void check(int rc) {
   if (rc != RG_OK)
     throw KernelFailure("librg_lru status " + std::to_string(rc) + ": " +

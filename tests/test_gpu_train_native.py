@@ -244,3 +244,20 @@ def test_saved_tensors_come_back_as_they_like(dtype, name):
                  lambda t: t.flatten()):
     with pytest.raises(RuntimeError, match="came back from its hook"):
       _gradients(call, wanted, keep, unpack)
+
+
+@pytest.mark.parametrize("name", ["scan", "rglru", "block"])
+def test_failures_keep_their_exception(name):
+  """A kernel's refusal in a backward pass is the package's exception, a hook's
+  own exception stays what it is, in both directions."""
+  call, wanted = _calls(BF16)[name]
+  keep = lambda t: t.detach()
+
+  def broken(t):
+    raise ZeroDivisionError("from a hook")
+
+  with pytest.raises(_lib.KernelError, match="came back from its hook"):
+    _gradients(call, wanted, keep, lambda t: t.flatten())
+  for hooks in ((broken, keep), (keep, broken)):
+    with pytest.raises(ZeroDivisionError, match="from a hook"):
+      _gradients(call, wanted, *hooks)
