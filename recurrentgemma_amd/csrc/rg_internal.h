@@ -295,9 +295,13 @@ struct ScanTileArgs {
   float* bias_out;       // float32: [2][W]
   int B, T, W;
 };
-enum ScanTileMode { kTilesFwdPlain, kTilesBwdPlain, kTilesFwdGated, kTilesBwdGated };
+enum ScanTileMode { kTilesFwdPlain, kTilesBwdPlain, kTilesFwdGated, kTilesBwdGated,
+                    // (a question only) both gated ones of a float32 RG-LRU
+                    kTilesPairGated };
 // whether it takes the shape and is the faster form for it
 bool scan_tiles_serve(int B, int T, int W, int dtype, int mode);
+// whether rg_scan_bwd.hip's kernels give a lane two channels (else one)
+bool scan_backward_two_channels(int B, int W);
 hipError_t launch_scan_tiles(const ScanTileArgs& a, int mode, int dtype,
                              hipStream_t s);
 void scan_split_plan(int B, int T, int W, int granule, int* chunks,

@@ -413,7 +413,7 @@ hipError_t launch_gates_as(const RglruBwdArgs& a, hipStream_t s) {
 
 // Two channels per lane halve the memory instructions, one channel per lane
 // doubles the workgroups: the latter until there is one per CU.
-static bool two_channels_per_lane(int B, int W) {
+bool scan_backward_two_channels(int B, int W) {
   return W % 2 == 0 && (int64_t)B * ((W + 127) / 128) >= 256;
 }
 
@@ -441,7 +441,7 @@ hipError_t launch_rglru_backward(const RglruBwdArgs& a, int dtype,
     t.W = a.W;
     return launch_scan_tiles(t, kTilesBwdGated, dtype, s);
   }
-  const bool two = two_channels_per_lane(a.B, a.W);
+  const bool two = scan_backward_two_channels(a.B, a.W);
   if (dtype == 0)
     return two ? launch_gates_as<float, 2, false>(a, s)
                : launch_gates_as<float, 1, false>(a, s);
@@ -468,7 +468,7 @@ hipError_t launch_linear_scan_backward(const ScanBwdArgs& a, int dtype,
     t.W = a.W;
     return launch_scan_tiles(t, kTilesBwdPlain, dtype, s);
   }
-  const bool two = two_channels_per_lane(a.B, a.W);
+  const bool two = scan_backward_two_channels(a.B, a.W);
   if (dtype == 0) return two ? launch_as<float, 2>(a, s) : launch_as<float, 1>(a, s);
   return two ? launch_as<uint16_t, 2>(a, s) : launch_as<uint16_t, 1>(a, s);
 }

@@ -590,6 +590,29 @@ hipError_t launch_as(const ScanTileArgs& a, hipStream_t s) {
 
 }  // namespace
 
+// The gated backward against rg_scan_bwd.hip's: rounds of 256 workgroups by what
+// one takes, us.  There: 64 channels a workgroup or, two to a lane, 128, by the
+// token; here: steps of 256 tokens.  Both sides as measured (bf16 unless said):
+//   B2 T64 W2560 13, here 17, T256 22 / 18, T1024 62 / 52; B8 T64 W2560 21 / 30,
+//   T384 54 / 56, T512 69 / 57; B8 W4096 (a full round there, two here) T256 38 /
+//   43, T1024 138 / 138, T2048 284 / 329; B16 W4096 T128 43 / 64, T1024 270 / 326,
+//   T4096 1118 / 966; B16 T512 W2560 117 / 100; B24 W4096 T384 157 / 187, T1024
+//   399 / 365; float32 B2 T64 W2560 14 / 16, T128 19 / 17; B16 W4096 T512 272 /
+//   308, T1024 536 / 505; B16 T128 W2560 61 / 75, T256 120 / 97
+static bool gated_backward_pays(int B, int T, int W, int dtype, int64_t blocks) {
+  const auto rounds = [](int64_t n) { return (float)((n + 255) / 256); };
+  const bool two = scan_backward_two_channels(B, W);
+  const float one_there = dtype == 0 ? (two ? 10.0f + 0.25f * T : 8.0f + 0.115f * T)
+                                     : (two ? 12.0f + 0.105f * T : 10.0f + 0.056f * T);
+  const int slabs_there = two ? (W + 127) / 128 : (W + 63) / 64;
+  const float there = rounds((int64_t)B * slabs_there) * one_there;
+  // (a step behind the second costs by its tokens)
+  const float steps = T <= 512 ? (float)((T + 255) / 256) : T / 256.0f;
+  const float here = rounds(blocks) * (9.0f + 13.1f * steps);
+  // (many or long rows, which that kernel reads twice from memory, take it longer)
+  return here < there || T > (blocks <= 1024 ? 2048 : 512);
+}
+
 bool scan_tiles_serve(int B, int T, int W, int dtype, int mode) {
   const int64_t es = dtype == 0 ? 4 : 2;
   if ((int64_t)W * es % 16 != 0 ||
@@ -601,10 +624,16 @@ bool scan_tiles_serve(int B, int T, int W, int dtype, int mode) {
   // kernels cost by the token.  The lines below are where they meet.
   const int64_t slab = dtype == 0 ? TileLds<float>::channels : TileLds<uint16_t>::channels;
   const int64_t blocks = (int64_t)B * ((W + slab - 1) / slab);
-  // The backward forms but for several rounds of short rows (us, B4 T2048 W2560
-  // bf16: plain 77 -> 40, gated 140 -> 118; B16 T8192 W4096: 1555 -> 1104, 2067
-  // -> 1710; but B16 T64 W4096 plain 13, here 19; float32 22, here 28).
-  if (mode == kBwdGated) return true;
+  if (mode == kBwdGated) return gated_backward_pays(B, T, W, dtype, blocks);
+  // Both directions of a float32 RG-LRU, which saves four launches beside the
+  // kernels' own difference: a whole RGLRU step, us, without and with them: B2 T64
+  // W2560 175, 154; B8 W4096 T16 174, 195, T64 188, 175; B16 W2560 T64 252, 259,
+  // T128 359, 325; B16 W4096 T128 399, 432, T256 743, 686.
+  if (mode == kTilesPairGated)
+    return T >= (blocks <= 640 ? 1 : blocks <= 1024 ? 64 : blocks < 2048 ? 100 : 192);
+  // The plain backward but for several rounds of short rows (us, B4 T2048 W2560
+  // bf16 77 -> 40, B16 T8192 W4096 1555 -> 1104; but B16 T64 W4096 13, here 19;
+  // float32 22, here 28).
   if (mode == kBwdPlain)
     return dtype == 0 ? blocks < 800 || T >= 128 : blocks < 512 || T >= 400;
   // The forward ones (B4 T2048 W2560 bf16: plain 52 -> 28, gated 83 -> 44).
@@ -619,7 +648,14 @@ bool scan_tiles_serve(int B, int T, int W, int dtype, int mode) {
     if (T > most) return false;
   }
   const bool cached = 3 * es * (int64_t)B * T * W < ((int64_t)256 << 20);
-  if (mode == kFwdGated) return blocks < (dtype == 0 ? 2048 : 1024) || cached;
+  // Gated: while every slab has a CU of its own; beyond, rows of some length that
+  // the last-level cache holds (bf16, projections included: B16 W2560 T64 32, here
+  // 40, T256 58, 51, T512 92, 77, T2048 267, 284; B8 W4096 T2048 191, 240; B24 W4096
+  // T64 48, 60, T256 96, 84; up to two rounds short rows lose 2 to 6, which the
+  // launch that finds the document starts otherwise costs too).  float32: see above.
+  if (mode == kFwdGated)
+    return dtype == 0 ? blocks < 2048 || cached
+                      : blocks <= 256 || (cached && (blocks <= 512 || T >= 128));
   // Plain: while every slab has a CU of its own; beyond, what the last-level
   // cache holds of a few rounds (bf16 B16 T1024 W2560: 62 -> 47, but T300 21,
   // here 22, and B8 T1600 W4096 61, here 71; float32 B8 T500 W2560 30 -> 24, but

@@ -189,20 +189,27 @@ struct GateWeights {
   Tensor a_param, w_x, b_x, w_a, b_a;
 };
 
-// Where both directions of the recurrence run on the one-pass kernels, they
-// take the document starts from the positions themselves and (float32) add
-// the gates' biases.
-bool on_tiles(const Dims& d) {
-  return rg::scan_tiles_serve((int)d.B, (int)d.T, (int)d.W, d.code,
-                              rg::kTilesFwdGated) &&
-         rg::scan_tiles_serve((int)d.B, (int)d.T, (int)d.W, d.code,
-                              rg::kTilesBwdGated);
+// Which directions of the recurrence run on the one-pass kernels, which take the
+// document starts from the positions themselves and, float32, add the gates'
+// biases to the pre-activations: both directions or neither there.
+struct OnTiles {
+  bool forward, backward;
+};
+OnTiles on_tiles(const Dims& d) {
+  auto serve = [&](rg::ScanTileMode mode) {
+    return rg::scan_tiles_serve((int)d.B, (int)d.T, (int)d.W, d.code, mode);
+  };
+  if (d.code == RG_DTYPE_F32) {
+    const bool both = serve(rg::kTilesFwdGated) && serve(rg::kTilesPairGated);
+    return {both, both};
+  }
+  return {serve(rg::kTilesFwdGated), serve(rg::kTilesBwdGated)};
 }
 
 // Kept::bias of a backward pass
 Tensor kept_bias(const Saved& s, int i) {
   const Dims d(s.root);
-  if (d.code != RG_DTYPE_F32 || !on_tiles(d)) return Tensor();
+  if (d.code != RG_DTYPE_F32 || !on_tiles(d).backward) return Tensor();
   return s.get(i, {2, s.W});
 }
 
@@ -222,16 +229,15 @@ Tensor by_head(const Tensor& t, int64_t H) {
 
 void gated_forward(const Tensor& x, const Tensor& pos, const GateWeights& g,
                    const Tensor& h0, const Tensor& gx, const Tensor& ga,
-                   const Tensor& y, const Tensor& h, Kept& kept,
-                   bool keep_starts) {
+                   const Tensor& y, const Tensor& h, Kept& kept) {
   const Dims d(x);
   const int64_t H = g.w_x.size(0);
-  const bool tiles = on_tiles(d);
+  const bool tiles = on_tiles(d).forward;
   const bool f32 = d.code == RG_DTYPE_F32;
   if (tiles) {  // (written by the recurrence's kernel)
-    if (keep_starts) kept.starts = empty({d.B, d.T}, at::kBool, x);
+    kept.starts = empty({d.B, d.T}, at::kBool, x);
     if (f32) kept.bias = empty({2, d.W}, x);
-  } else if (keep_starts) {
+  } else {
     kept.starts = at::eq(pos, 0);
   }
   if (f32) {
@@ -318,12 +324,10 @@ struct GatedGrads {
   Tensor dx, dlam, dw_x, db_x, dw_a, db_a, dh0;
 };
 
-// kept.starts or, without it, pos
 GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
-                          const Tensor& pos, const Kept& kept,
-                          const Tensor& a_param, const Tensor& w_x,
-                          const Tensor& w_a, const Tensor& gx, const Tensor& ga,
-                          const Tensor& y, const Tensor& h0,
+                          const Kept& kept, const Tensor& a_param,
+                          const Tensor& w_x, const Tensor& w_a, const Tensor& gx,
+                          const Tensor& ga, const Tensor& y, const Tensor& h0,
                           const GateNeeds& need_, Sums& sums) {
   const Dims d(x);
   const int64_t H = w_x.size(0), bw = d.W / H;
@@ -333,7 +337,7 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
   Tensor dgx = empty(x.sizes(), x), dga = empty(x.sizes(), x);
   Tensor lam_rows = empty({d.B, d.W}, at::kFloat, x), bias_rows;
   if (h0.defined()) r.dh0 = empty(h0.sizes(), h0);
-  const bool tiles = on_tiles(d);
+  const bool tiles = on_tiles(d).backward;
   if (tiles) {
     rg::ScanTileArgs t{};
     t.in[0] = in(dy);
@@ -341,8 +345,8 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
     t.in[2] = in(gx);
     t.in[3] = in(ga);
     t.in[4] = in(y);
-    t.flags = in(kept.starts.defined() ? kept.starts : pos);
-    t.flag_kind = kept.starts.defined() ? rg::kSegMaskU8 : seg_kind(pos);
+    t.flags = in(kept.starts);
+    t.flag_kind = rg::kSegMaskU8;
     t.a_param = in(a_param);
     if (f32) {
       t.bias[0] = in(kept.bias);
@@ -362,9 +366,8 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
     t.W = (int)d.W;
     check_hip(rg::launch_scan_tiles(t, rg::kTilesBwdGated, d.code, d.stream));
   } else {
-    Tensor reset = kept.starts.defined() ? kept.starts : at::eq(pos, 0);
     check(rg_rglru_backward(in(dy), in(x), in(gx), in(ga), in(a_param),
-                            in(reset), in(y), in(h0), in(dh), out(r.dx), out(dgx),
+                            in(kept.starts), in(y), in(h0), in(dh), out(r.dx), out(dgx),
                             out(dga), (float*)out(lam_rows), out(r.dh0), (int)d.B,
                             (int)d.T, (int)d.W, d.code, d.stream));
   }
@@ -431,8 +434,7 @@ struct Rglru : Function<Rglru> {
     Tensor y = empty(x.sizes(), x);
     Tensor h = empty({x.size(0), x.size(2)}, at::kFloat, x);
     Kept kept;
-    gated_forward(x, pos, {a_param, w_x, b_x, w_a, b_a}, h0, gx, ga, y, h, kept,
-                  true);
+    gated_forward(x, pos, {a_param, w_x, b_x, w_a, b_a}, h0, gx, ga, y, h, kept);
     ctx->save_for_backward(
         {x, kept.starts, a_param, w_x, w_a, kept.bias, h0, gx, ga, y});
     return {y, h};
@@ -447,7 +449,7 @@ struct Rglru : Function<Rglru> {
     const Tensor dh = grad_of(grads[1], {s.B, s.W}, at::kFloat);
     Sums sums;
     GatedGrads r = gated_backward(
-        dy, dh, x, Tensor(), kept, s.get(2, {s.W}), s.gate_weight(3),
+        dy, dh, x, kept, s.get(2, {s.W}), s.gate_weight(3),
         s.gate_weight(4), s.like_root(7), s.like_root(8), y, s.state(6),
         {ctx->needs_input_grad(3), ctx->needs_input_grad(4),
          ctx->needs_input_grad(5), ctx->needs_input_grad(6)},
@@ -482,15 +484,16 @@ struct Block : Function<Block> {
                             d.code, d.stream));
     Tensor gx = empty(lx.sizes(), x), ga = empty(lx.sizes(), x);
     Tensor y = empty(lx.sizes(), x);
-    Kept kept;  // (the conv's backward reads the positions themselves)
+    Kept kept;
     gated_forward(xc, pos, {a_param, w_x, b_x, w_a, b_a}, Tensor(), gx, ga, y, h,
-                  kept, false);
+                  kept);
     Tensor join = empty(lx.sizes(), x);
     check(rg_gelu_mul(in(y), in(gate), out(join), d.M() * W, d.code, d.stream));
     Tensor result = at::linear(join.view({B * T, W}), w_out, b_out)
                         .view({B, T, w_out.size(0)});
     ctx->save_for_backward({x, pos, w_y, w_lx, conv_w, a_param, w_x, w_a,
-                            kept.bias, w_out, gate, lx, xc, gx, ga, y, join});
+                            kept.bias, w_out, gate, lx, xc, gx, ga, y, join,
+                            kept.starts});
     if (!want_cache) return {result};
     ctx->mark_non_differentiable({conv_state});
     return {result, h, conv_state};
@@ -544,7 +547,7 @@ struct Block : Function<Block> {
     Tensor dh;
     if (grads.size() > 1) dh = grad_of(grads[1], {d.B, W}, at::kFloat);
     GatedGrads g = gated_backward(
-        dy, dh, xc, pos, {Tensor(), kept_bias(s, 8)}, s.get(5, {W}),
+        dy, dh, xc, {s.get(17, {d.B, d.T}, at::kBool), kept_bias(s, 8)}, s.get(5, {W}),
         s.gate_weight(6), s.gate_weight(7), s.like_root(13), s.like_root(14), y,
         Tensor(), {needs(9), needs(10), needs(11), needs(12)}, sums);
     r[8] = g.dlam;

@@ -117,6 +117,16 @@ def test_float32_gate_weight_gradients(B, T, heads):
   test_rglru_gradients(B, T, 256 * heads, heads, F32)
 
 
+# bf16, where each direction picks its own kernel: the backward one-pass (rows that
+# end just before, at and just behind its steps of 256 tokens), neither (many
+# short rows), only the backward (rows the last-level cache does not hold)
+@pytest.mark.parametrize("B,T,width", [
+    (2, 250, 256), (1, 255, 512), (3, 256, 256), (1, 511, 256), (2, 513, 256),
+    (1, 1025, 512), (40, 7, 1024), (36, 100, 1024), (80, 1100, 512)])
+def test_directions_on_kernels_of_their_own(B, T, width):
+  test_rglru_gradients(B, T, width, width // 256, BF16)
+
+
 def test_frozen_parts_and_wrapped_layers():
   """Only what needs a gradient gets one, and a hooked layer is called."""
   block, x, pos = make(2, 70, 512, 2, BF16)
