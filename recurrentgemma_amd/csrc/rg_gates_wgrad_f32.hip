@@ -21,12 +21,20 @@
 // registers) are all resident; their sums are added in a fixed order by a
 // second kernel, so results do not vary from run to run.
 //
-// Measured at M = 3003, W = 2560 (H = 10, 480 workgroups): 78 us + 5 us for the
-// second kernel = 101 TFLOP/s of the fp32 matrix peak's 157, where the
-// library's two batched products on strided views take 141 us (56 TFLOP/s);
-// 512 rows 27 against 235 us, 8192 rows 181 against 312, at width 4096
-// 32 against 235 and 270 against 246.  Error against 64 bits at 8192 rows
-// 4.7e-7 (library 1.6e-6): a wave's chain of sums is a quarter of a row range.
+// Measured against the library's two batched products on strided views, us, and
+// the error of dw against 64 bits (a wave's chain of sums is a quarter of a row
+// range; the second kernel, 5 us of these, included):
+//   rows                  512    1001    2048    3003    4096    8192   16384
+//   10 heads, here         26      38      59      73      96     180     356
+//             library     239     456     106     133     143     313     741
+//             error    1.3e-7  1.7e-7  2.4e-7  2.9e-7  3.4e-7  4.7e-7  6.6e-7
+//             library  4.1e-7  5.7e-7  8.1e-7  9.2e-7  1.1e-6  1.6e-6  2.2e-6
+//   16 heads, here         32      47      81     104     135     270     529
+//             library     238     456      74      98     126     246     506
+//             error    1.5e-7  2.1e-7  2.9e-7  3.5e-7  4.1e-7  5.7e-7  8.1e-7
+//             library  4.1e-7  5.7e-7  8.1e-7  9.8e-7  1.2e-6  1.6e-6  2.3e-6
+// 1 to 4 heads 1.5 to 30 times as fast; 32 heads within 10 % from 2048 rows on.
+// 3003 rows of 10 heads are 108 TFLOP/s of the fp32 matrix peak's 157.
 #include "rg_common.h"
 #include "rg_internal.h"
 
@@ -190,6 +198,9 @@ int64_t rows_for(int64_t M, int splits) {
 
 }  // namespace
 
+// Every shape it can address: from 16 heads and 2048 rows on the library is ahead
+// by up to 10 % (the table above), at three times the error, which is what is
+// paid for there.
 bool gates_wgrad_f32_serves(int64_t M, int W, int H) {
   if (M <= 0 || H <= 0 || W != H * kBW || H > 4096) return false;
   // offsets within a row range, two batches past its end, are 32 bits
