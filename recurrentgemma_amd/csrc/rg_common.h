@@ -354,17 +354,42 @@ __device__ __forceinline__ float sigmoid_fast(float v) {
 }
 
 
-// a * gelu_tanh(g) for bf16 operands held as floats (modules.py:289-291, :644):
-// gelu in fp32 as 0.5 g (1 + tanh u) with tanh u = 2 sigmoid(2u) - 1 rounded
-// to float32 first, so that the negative tail saturates to -0 exactly where a
-// float32 tanh does; gelu is rounded to bf16 like the module output it is in
-// the reference; the caller rounds the product.
-__device__ __forceinline__ float gelu_mul_bf16(float av, float gv) {
-  constexpr float c0 = 0.7978845608028654f;  // sqrt(2/pi)
-  constexpr float c1 = 0.044715f;
-  const float u = c0 * __builtin_fmaf(c1 * gv * gv, gv, gv);
-  const float t = __builtin_fmaf(2.0f, sigmoid_fast(2.0f * u), -1.0f);
-  return av * round_to_bf16(0.5f * gv * (1.0f + t));
+// gelu_tanh(g) in fp32 for the bf16 kernels (modules.py:289-291): g (1 + t) / 2
+// with t / 2 = tanh(u) / 2 = sigmoid(2u) - 1/2 rounded to float32 first, so that
+// the negative tail saturates to -0 exactly where a float32 tanh does.  The
+// factors of u = sqrt(2/pi) (g + 0.044715 g^3) carry the -2 log2(e) of the
+// sigmoid's exponential: eleven issue slots, four fewer than written out.
+__device__ __forceinline__ float gelu_fast(float g) {
+  constexpr float k0 = -2.0f * kLog2e * 0.7978845608028654f;  // sqrt(2/pi)
+  constexpr float k1 = k0 * 0.044715f;
+  const float e =
+      __builtin_amdgcn_exp2f(g * __builtin_fmaf(k1, g * g, k0));  // e^(-2u)
+  const float half_t = __builtin_amdgcn_rcpf(1.0f + e) - 0.5f;
+  return g * (half_t + 0.5f);
+}
+
+// a * gelu_tanh(g) for two bf16 of each operand (modules.py:289-291, :644):
+// gelu is rounded to bf16 like the module output it is in the reference, then
+// the product.
+__device__ __forceinline__ uint32_t gelu_mul_bf16x2(uint32_t a, uint32_t g) {
+  const uint32_t y = pack_bf16x2(gelu_fast(__uint_as_float(g << 16)),
+                                 gelu_fast(__uint_as_float(g & 0xffff0000u)));
+  return pack_bf16x2(
+      __uint_as_float(a << 16) * __uint_as_float(y << 16),
+      __uint_as_float(a & 0xffff0000u) * __uint_as_float(y & 0xffff0000u));
+}
+
+// The recurrence gate's exponent sigmoid(v) * decay with e = exp(-v) as
+// 1 / (e / decay + 1 / decay): one multiply-add where 1 + e and the product
+// with decay were two instructions.  inv is 1 / decay, kept finite: decay = 0
+// (softplus underflowed) gives an exponent of no consequence instead of
+// 0 * infinity.
+__device__ __forceinline__ float inverse_decay(float decay) {
+  const float inv = 1.0f / decay;
+  return __builtin_fabsf(inv) > 0x1p120f ? -0x1p120f : inv;
+}
+__device__ __forceinline__ float gate_exponent(float e, float inv) {
+  return __builtin_amdgcn_rcpf(__builtin_fmaf(e, inv, inv));
 }
 
 // a * gelu_tanh(g) in float32 by the reference's own formula

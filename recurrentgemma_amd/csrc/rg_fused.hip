@@ -319,10 +319,7 @@ block_step_bf16_kernel(StepArgs p) {
     uint32_t y2 = pack_bf16x2(lo, hi);
     if (GELU) {
       const uint32_t g2 = gate2[r >> 1];
-      y2 = pack_bf16x2(gelu_mul_bf16(__uint_as_float(y2 << 16),
-                                     __uint_as_float(g2 << 16)),
-                       gelu_mul_bf16(__uint_as_float(y2 & 0xffff0000u),
-                                     __uint_as_float(g2 & 0xffff0000u)));
+      y2 = gelu_mul_bf16x2(y2, g2);
     }
     __builtin_amdgcn_raw_buffer_store_b32(y2, ry,
                                           pair_ch * 2u + lane_rows * row_bytes,

@@ -200,11 +200,10 @@ linear_rows_kernel(LinearArgs p) {
           up[i] += bu[i];
         }
       }
-      float o[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        o[i] = gelu_mul_bf16(round_to_bf16(up[i]), round_to_bf16(gate[i]));
-      const u32x2 ov = {pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+      const u32x2 ov = {gelu_mul_bf16x2(pack_bf16x2(up[0], up[1]),
+                                        pack_bf16x2(gate[0], gate[1])),
+                        gelu_mul_bf16x2(pack_bf16x2(up[2], up[3]),
+                                        pack_bf16x2(gate[2], gate[3]))};
       *reinterpret_cast<u32x2*>(out + (size_t)row * half + col) = ov;
     }
     return;

@@ -528,7 +528,8 @@ __device__ __forceinline__ void prefill_body(const FusedArgs& p,
   // Finished tokens go through the wave's LDS patch, sixteen at a time, and
   // leave as 16-byte row chunks; the stores are issued a run after the patch
   // was read so that they do not wait for the LDS (y_pending).
-  float bias_x[kNB], bias_a[kNB], decay[kNB];  // times -log2(e), see prologue
+  float bias_x[kNB], bias_a[kNB];  // times -log2(e), see prologue
+  float inv_decay[kNB];
   float hc[kNB] = {0.0f, 0.0f};    // carried state of this lane's channels
   float prod[kNB] = {1.0f, 1.0f};  // kChunkSummary: product of a, own tokens
   u32x4 y_pending[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
@@ -541,12 +542,7 @@ __device__ __forceinline__ void prefill_body(const FusedArgs& p,
       // roundings of the stand-alone gelu_mul pass
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const float lo = gelu_mul_bf16(__uint_as_float(y_pending[j][k] << 16),
-                                       __uint_as_float(g_pending[j][k] << 16));
-        const float hi =
-            gelu_mul_bf16(__uint_as_float(y_pending[j][k] & 0xffff0000u),
-                          __uint_as_float(g_pending[j][k] & 0xffff0000u));
-        y_pending[j][k] = pack_bf16x2(lo, hi);
+        y_pending[j][k] = gelu_mul_bf16x2(y_pending[j][k], g_pending[j][k]);
       }
     }
     buffer_store_16(y_pending[j], ry, y_lane_bytes,
@@ -589,7 +585,8 @@ __device__ __forceinline__ void prefill_body(const FusedArgs& p,
         sa[q] = __builtin_fmaf(acc_a[4 * g + q], -kLog2e, bias_a[nb]);
       }
       pinned(8 * r + 0);
-      // pieces 1, 2: the two sigmoids, eight independent chains
+      // pieces 1, 2: the input gate's sigmoid and the recurrence gate's times
+      // decay, eight independent chains
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         sx[q] = __builtin_amdgcn_exp2f(sx[q]);
@@ -599,17 +596,17 @@ __device__ __forceinline__ void prefill_body(const FusedArgs& p,
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         sx[q] = __builtin_amdgcn_rcpf(1.0f + sx[q]);
-        sa[q] = __builtin_amdgcn_rcpf(1.0f + sa[q]);
+        sa[q] = gate_exponent(sa[q], inv_decay[nb]);
       }
       // the sixteen tokens read back from the patch two runs ago leave now
       if (MODE != kChunkSummary && (r & 3) == 1) flush_y();
       pinned(8 * r + 2);
-      // piece 3: a = exp2(sigmoid(pa) * decay), xc * sigmoid(px); the conv
+      // piece 3: a, xc * sigmoid(px); the conv
       // outputs of the next run are requested here
       float av[4], xn[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        av[q] = __builtin_amdgcn_exp2f(sa[q] * decay[nb]);
+        av[q] = __builtin_amdgcn_exp2f(sa[q]);
         xn[q] = bf16_bits_to_f32(xraw[q]) * sx[q];
       }
       if (r < 7) {
@@ -716,9 +713,9 @@ __device__ __forceinline__ void prefill_body(const FusedArgs& p,
     const int ch = h * kBW + n0 + 32 * nb + (lane & 31);  // this lane's channel
     bias_x[nb] = -kLog2e * bf16_bits_to_f32(((const uint16_t*)p.b[0])[ch]);
     bias_a[nb] = -kLog2e * bf16_bits_to_f32(((const uint16_t*)p.b[1])[ch]);
-    decay[nb] =
+    inv_decay[nb] = inverse_decay(
         (-8.0f * kLog2e) *
-        softplus_precise(bf16_bits_to_f32(((const uint16_t*)p.a_param)[ch]));
+        softplus_precise(bf16_bits_to_f32(((const uint16_t*)p.a_param)[ch])));
     if (MODE == kChunkReplay) {
       // state at the start of this chunk from the summaries of the chunks
       // before it: h <- P[k] h + H[k] (the scan operator of

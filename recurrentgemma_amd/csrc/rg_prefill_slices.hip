@@ -59,7 +59,7 @@ typedef __attribute__((address_space(3))) f32x2 lds_f32x2;
 
 // LDS, in bytes: two conv tiles of TILES x 32 tokens, every matrix wave's
 // output patch, the tiles' (prod a, state) pairs twice, conv taps, and the
-// biases and decays of the workgroup's CH channels.
+// biases and inverse decays of the workgroup's CH channels.
 template <int KS, int TILES, int CH>
 struct Layout {
   static constexpr int row = (KS * 16 + 8) * 2;
@@ -166,7 +166,7 @@ __device__ __forceinline__ void gate_and_scan(
       const f32x4 per_channel = *reinterpret_cast<lds_f32x4*>(
           lds3 + L::gates + (c0 + (ln & 31)) * 16);
       const float bias_x = per_channel[0], bias_a = per_channel[1];
-      const float decay = per_channel[2];
+      const float inv_decay = per_channel[2];
       const uint32_t xc_lane =
           (uint32_t)(tt * kTile + 4 * (ln >> 5)) * L::row + 2u * (uint32_t)(n0 + (ln & 31));
       float av[16], xn[16];
@@ -180,9 +180,9 @@ __device__ __forceinline__ void gate_and_scan(
       for (int e = 0; e < 16; ++e) {
         const float gx = __builtin_amdgcn_rcpf(
             1.0f + __builtin_amdgcn_exp2f(__builtin_fmaf(acc_x[e], -kLog2e, bias_x)));
-        const float ga = __builtin_amdgcn_rcpf(
-            1.0f + __builtin_amdgcn_exp2f(__builtin_fmaf(acc_a[e], -kLog2e, bias_a)));
-        av[e] = __builtin_amdgcn_exp2f(ga * decay);
+        av[e] = __builtin_amdgcn_exp2f(gate_exponent(
+            __builtin_amdgcn_exp2f(__builtin_fmaf(acc_a[e], -kLog2e, bias_a)),
+            inv_decay));
         xn[e] *= gx;
       }
       if (__builtin_expect(starts != 0 || t0 + kTile > T, 0)) {
@@ -318,14 +318,8 @@ __device__ __forceinline__ void gate_and_scan(
             asm volatile("" ::: "memory");
             if (GELU) {
 #pragma unroll
-              for (int k = 0; k < 4; ++k) {
-                const uint32_t gr = gate_rows[g >> 1][k];
-                out[k] = pack_bf16x2(
-                    gelu_mul_bf16(__uint_as_float(out[k] << 16),
-                                  __uint_as_float(gr << 16)),
-                    gelu_mul_bf16(__uint_as_float(out[k] & 0xffff0000u),
-                                  __uint_as_float(gr & 0xffff0000u)));
-              }
+              for (int k = 0; k < 4; ++k)
+                out[k] = gelu_mul_bf16x2(out[k], gate_rows[g >> 1][k]);
             }
             const uint32_t at = (uint32_t)(t0 + 16 * (g >> 1)) * row_bytes;
             buffer_store_16(out, ry, y_valid ? y_lane + at : kBufferOutOfRange, 0);
@@ -415,7 +409,7 @@ __device__ __forceinline__ void fill_taps(const FusedArgs& p,
     tab[1] = u32x4{ub << 16, ub & 0xffff0000u, 0u, 0u};
   }
 }
-// Biases and decay of channels n0 .. n0 + 31: read back in every pass (kept in
+// Biases and inverse decay of channels n0 .. n0 + 31: read back in every pass (kept in
 // registers across the matrix instructions they are three too many).
 template <class L>
 __device__ __forceinline__ void fill_gate_values(const FusedArgs& p,
@@ -429,8 +423,9 @@ __device__ __forceinline__ void fill_gate_values(const FusedArgs& p,
     if (n < bw) {
       v[0] = -kLog2e * bf16_bits_to_f32(((const uint16_t*)p.b[0])[h * bw + n]);
       v[1] = -kLog2e * bf16_bits_to_f32(((const uint16_t*)p.b[1])[h * bw + n]);
-      v[2] = (-8.0f * kLog2e) *
-             softplus_precise(bf16_bits_to_f32(((const uint16_t*)p.a_param)[h * bw + n]));
+      v[2] = inverse_decay(
+          (-8.0f * kLog2e) *
+          softplus_precise(bf16_bits_to_f32(((const uint16_t*)p.a_param)[h * bw + n])));
     }
     *reinterpret_cast<f32x4*>(lds_raw + L::gates + (c0 + lane) * 16) = v;
   }

@@ -120,7 +120,7 @@ template <int MODE, bool GELU>
 __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
                                                    const int chunk) {
   // how much of the gate arithmetic runs at the end of phase M (with the
-  // join, phase G carries 17 more vector slots per element)
+  // join, phase G carries 13 more vector slots per element)
   constexpr int kTailX = GELU ? kTailXJoined : kTailXPlain;
   constexpr int kTailA = GELU ? kTailAJoined : kTailAPlain;
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -315,9 +315,9 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
   const int ch = h * kBW + n0 + (lane & 31);  // this lane's channel
   const float bias_x = -kLog2e * bf16_bits_to_f32(((const uint16_t*)p.b[0])[ch]);
   const float bias_a = -kLog2e * bf16_bits_to_f32(((const uint16_t*)p.b[1])[ch]);
-  const float decay =
+  const float inv_decay = inverse_decay(
       (-8.0f * kLog2e) *
-      softplus_precise(bf16_bits_to_f32(((const uint16_t*)p.a_param)[ch]));
+      softplus_precise(bf16_bits_to_f32(((const uint16_t*)p.a_param)[ch])));
   float hc = 0.0f;    // carried state of this lane's channel
   float prod = 1.0f;  // kChunkSummary: product of a over this lane's tokens
   if (MODE == kChunkReplay) {
@@ -357,10 +357,10 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
       acc_a[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(acc_a[i], -kLog2e, bias_a));
 #pragma unroll
     for (int i = i0; i < i1; ++i)
-      acc_a[i] = __builtin_amdgcn_rcpf(1.0f + acc_a[i]);
+      acc_a[i] = gate_exponent(acc_a[i], inv_decay);
 #pragma unroll
     for (int i = i0; i < i1; ++i)
-      acc_a[i] = __builtin_amdgcn_exp2f(acc_a[i] * decay);
+      acc_a[i] = __builtin_amdgcn_exp2f(acc_a[i]);
   };
   // ---- phase M of block kb ----------------------------------------------------
   auto phase_m = [&](int kb, auto ODD) {
@@ -529,14 +529,8 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float lo = gelu_mul_bf16(__uint_as_float(y_pending[j][k] << 16),
-                                         __uint_as_float(g_pending[j][k] << 16));
-          const float hi =
-              gelu_mul_bf16(__uint_as_float(y_pending[j][k] & 0xffff0000u),
-                            __uint_as_float(g_pending[j][k] & 0xffff0000u));
-          y_pending[j][k] = pack_bf16x2(lo, hi);
-        }
+        for (int k = 0; k < 4; ++k)
+          y_pending[j][k] = gelu_mul_bf16x2(y_pending[j][k], g_pending[j][k]);
     }
     y_pending_row = (uint32_t)t_blk * row_bytes;
   };
