@@ -59,9 +59,11 @@ constexpr int kRawLoads = kRawRows / 2;
 constexpr int kRawLoadsPerWave = (kRawLoads + kWaves - 1) / kWaves;
 constexpr int kRawTileBytes = kRawLoadsPerWave * kWaves * 2 * kRawRowBytes;
 // Per-wave output patch: 16 tokens x 32 channels in bf16, rows padded to 80
-// bytes.
+// bytes; the second eight rows (the upper lanes') another 64 bytes on, in other
+// banks than the first.
 constexpr int kPatchStride = 80;
-constexpr int kPatchBytesPerWave = 16 * kPatchStride;
+constexpr int kPatchUpper = 8 * kPatchStride + 64;
+constexpr int kPatchBytesPerWave = kPatchUpper + 8 * kPatchStride;
 
 constexpr int kXcOff = 0;
 constexpr int kRawOff = kXcOff + kXcRing * kXcBlockBytes;
@@ -73,12 +75,12 @@ static_assert(kTeamsLdsBytes <= 160 * 1024, "LDS of one CU");
 constexpr int kARing = 4;
 // How many of a lane's sixteen tokens have their input-gate sigmoid computed
 // at the end of phase M, the rest at the top of phase G (measured at B16 T8192
-// W4096: 0 -> 778 us, 8 -> 764 us, 12 -> 779 us a launch), and the same for the
-// recurrence gate (any part of it there was slower).
-constexpr int kTailXPlain = 8;
+// W4096: 0 -> 755 us, 4 -> 755 us, 8 -> 765 us, 12 -> 777 us a launch), and the
+// same for the recurrence gate (any part of it there was slower).
+constexpr int kTailXPlain = 0;
 constexpr int kTailAPlain = 0;
-// ... and with the GELU join in phase G (B16 T8192 W4096: 1057-1062 us a launch
-// for 8-16 input-gate and 0-8 recurrence-gate sigmoids here: no difference)
+// ... and with the GELU join in phase G (B8 T4096 W2560 in chunks: 249-256 us for
+// 8-16 input-gate and 0-4 recurrence-gate sigmoids here: no difference)
 constexpr int kTailXJoined = 16;
 constexpr int kTailAJoined = 4;
 // Priority of a wave while it issues its matrix instructions (the wave in
@@ -205,25 +207,42 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
   const uint32_t conv_raw_lane =
       kRawOff + (uint32_t)(rg4 * kConvRows + kRawHalo - 3) * kRawRowBytes +
       conv_pair_of_lane * 4;
+  // Conv output of token t of a block lies in row xc_row(t): the rows are the
+  // A operand's, of whose results a lane gets rows 8 j + 4 (lane / 32) + 0..3,
+  // j = 0..3.  In this order those are tokens 0..15 for lanes 0-31 and tokens
+  // 16..31 for lanes 32-63, a walk of the recurrence in one piece (B16 T8192
+  // W4096: 4 us of 765 against four pieces with the halves in turn).  Summaries
+  // keep the tokens in their order: rg_prefill.hip multiplies its product of a
+  // in the order that gives.
+  constexpr bool halves = MODE != kChunkSummary;
   const uint32_t conv_xc_lane =
-      kXcOff + (uint32_t)(rg4 * kConvRows) * kXcRowBytes + conv_pair_of_lane * 4;
-  // gates: lane -> channel n0 + lane % 32, tokens 4 (lane / 32) + ...
+      kXcOff +
+      (uint32_t)(halves ? 16 * (rg4 & 1) + 4 * (rg4 >> 1) : rg4 * kConvRows) *
+          kXcRowBytes +
+      conv_pair_of_lane * 4;
+  // row of a thread's i-th conv row, relative to its first; likewise the token
+  // of a lane's i-th result, relative to its first
+  auto xc_row = [](int i) { return halves ? 8 * (i >> 2) + (i & 3) : i; };
+  auto token = [](int i) { return halves ? i : 8 * (i >> 2) + (i & 3); };
+  // gates: lane -> channel n0 + lane % 32, tokens 16 (lane / 32) + ...
   const uint32_t xc_lane = kXcOff + 4u * (lane >> 5) * kXcRowBytes +
                            2u * (uint32_t)(n0 + (lane & 31));
   // MFMA A operand: lane -> token lane % 32, k offset 8 (lane / 32)
   const uint32_t a_lane =
       kXcOff + (uint32_t)(lane & 31) * kXcRowBytes + 16u * (lane >> 5);
-  // output patch of this wave: written as token 4 (lane / 32) + q (+ 8 for
-  // odd runs), channel lane % 32; read back as 16-byte row chunks, lane l
-  // taking chunk l % 4 of token l / 4
+  // output patch of this wave: eight tokens of the lower and eight of the upper
+  // lanes at a time, written as row 8 (lane / 32) + ..., channel lane % 32; read
+  // back as 16-byte row chunks, lane l taking chunk l % 4 of row l / 4
   const uint32_t patch_w_lane = kPatchOff + wave * kPatchBytesPerWave +
-                                4u * (lane >> 5) * kPatchStride +
+                                (uint32_t)(lane >> 5) * kPatchUpper +
                                 2u * (lane & 31);
   const uint32_t patch_r_lane = kPatchOff + wave * kPatchBytesPerWave +
-                                (uint32_t)(lane >> 2) * kPatchStride +
+                                (uint32_t)(lane >> 5) * kPatchUpper +
+                                (uint32_t)((lane >> 2) & 7) * kPatchStride +
                                 16u * (lane & 3);
-  const uint32_t y_lane_bytes = (uint32_t)(lane >> 2) * row_bytes +
-                                2u * (uint32_t)(h * kBW + n0) + 16u * (lane & 3);
+  const uint32_t y_lane_bytes =
+      (uint32_t)(16 * (lane >> 5) + ((lane >> 2) & 7)) * row_bytes +
+      2u * (uint32_t)(h * kBW + n0) + 16u * (lane & 3);
 
   // ---- width-4 conv ---------------------------------------------------------
   uint32_t cw10[2], cw32[2];
@@ -271,9 +290,10 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
       cr.e_prev[c] = e[c];
       cr.o_prev[c] = o[c];
     }
-    *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at + (2 * j) * kXcRowBytes) =
+    *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at + xc_row(2 * j) * kXcRowBytes) =
         pack_bf16x2(even[0], even[1]);
-    *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at + (2 * j + 1) * kXcRowBytes) =
+    *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at +
+                                xc_row(2 * j + 1) * kXcRowBytes) =
         pack_bf16x2(odd[0], odd[1]);
   };
   auto conv_with_cuts = [&](const ConvRows& cr, uint32_t cuts) {
@@ -290,7 +310,8 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
       if (i >= 3) {
         float o[2];
         conv4_dot_x2(p2, pt, cw10, cw32, cbias, o);
-        *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at + (i - 3) * kXcRowBytes) =
+        *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at +
+                                    xc_row(i - 3) * kXcRowBytes) =
             pack_bf16x2(o[0], o[1]);
       }
 #pragma unroll
@@ -378,7 +399,7 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
     // the tokens of the block before leave now
     buffer_store_16(y_pending[0], ry, y_lane_bytes, y_pending_row);
     buffer_store_16(y_pending[1], ry, y_lane_bytes,
-                    y_pending_row + 16u * row_bytes);
+                    y_pending_row + 8u * row_bytes);
     const uint32_t cuts = odd ? conv_cuts(kb + 1, m_next, m_cur)
                               : conv_cuts(kb + 1, m_cur, m_prev);
     ConvRows cr;
@@ -431,12 +452,12 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
   };
 
   // ---- phase G of block kb ----------------------------------------------------
-  // The MFMA result gives a lane one channel (lane % 32) and 16 tokens in runs
-  // of four that alternate between the lane halves: run g of lanes 0-31 holds
-  // tokens 8g..8g+3, of lanes 32-63 tokens 8g+4..8g+7.  Per run the recurrence
-  // is walked twice: from the carried state (right for lanes 0-31, whose end
-  // value goes to lanes 32-63 with one permlane32_swap), then again from each
-  // half's own incoming state.
+  // The matrix result gives a lane one channel (lane % 32) and 16 tokens, in a
+  // row (lanes 0-31 the first half of the block, lanes 32-63 the second) or, for
+  // summaries, in runs of four that alternate between the halves.  The recurrence
+  // is walked twice: from the carried state (right for lanes 0-31, whose end value
+  // goes to lanes 32-63 with one permlane32_swap), then again from each half's own
+  // incoming state.
   auto phase_g_as = [&](int kb, auto GENERAL) {
     constexpr bool general = decltype(GENERAL)::value;
     const int t_blk = kb * kBT;
@@ -447,81 +468,80 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
       g_pending[0] = __builtin_amdgcn_raw_buffer_load_b128(
           rgate, y_lane_bytes + (uint32_t)t_blk * row_bytes, 0, 0);
       g_pending[1] = __builtin_amdgcn_raw_buffer_load_b128(
-          rgate, y_lane_bytes + (uint32_t)(t_blk + 16) * row_bytes, 0, 0);
+          rgate, y_lane_bytes + (uint32_t)(t_blk + 8) * row_bytes, 0, 0);
     }
     gate_x(kTailX, 16);
     gate_a(kTailA, 16);
+    float xn[16];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float av[4], xn[4];
+    for (int i = 0; i < 16; ++i) xn[i] = __uint_as_float(xr[i]) * acc_x[i];
+    if (general) {
+      // document start: a = 0; past the end of the sequence: a = 1, no input.
+      // The input scale sqrt(1 - a^2) comes out as 1 at a start.
+      const int first = upper ? (halves ? 16 : 4) : 0;
+      const uint32_t starts = (uint32_t)(m_cur >> ((kb & 1) * 32 + first));
+      const int left = T_len - t_blk - first;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        av[q] = acc_a[4 * g + q];
-        xn[q] = __uint_as_float(xr[4 * g + q]) * acc_x[4 * g + q];
+      for (int i = 0; i < 16; ++i) {
+        acc_a[i] = ((starts >> token(i)) & 1u) ? 0.0f : acc_a[i];
+        acc_a[i] = token(i) < left ? acc_a[i] : 1.0f;
+        xn[i] = token(i) < left ? xn[i] : 0.0f;
       }
-      if (general) {
-        // document start: a = 0; past the end of the sequence: a = 1, no
-        // input.  The input scale sqrt(1 - a^2) comes out as 1 at a start.
-        const int half_rows = upper ? 4 : 0;
-        const int row = (kb & 1) * 32 + 8 * g + half_rows;
-        const uint32_t starts = (uint32_t)(m_cur >> row) & 0xfu;
-        const int t_run = t_blk + 8 * g + half_rows;
+    }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          av[q] = ((starts >> q) & 1u) ? 0.0f : av[q];
-          av[q] = (t_run + q < T_len) ? av[q] : 1.0f;
-          xn[q] = (t_run + q < T_len) ? xn[q] : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        xn[q] = xn[q] *
-                __builtin_amdgcn_sqrtf(__builtin_fmaf(-av[q], av[q], 1.0f));
+    for (int i = 0; i < 16; ++i)
+      xn[i] = xn[i] *
+              __builtin_amdgcn_sqrtf(__builtin_fmaf(-acc_a[i], acc_a[i], 1.0f));
+    // the state from the carried one over elements [i0, i1) of both halves, each
+    // handed to keep(i, state); the end state becomes the carried one
+    auto walk = [&](int i0, int i1, auto&& keep) {
       float e1 = hc;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) e1 = __builtin_fmaf(av[q], e1, xn[q]);
-      float hh;
-      {
-        const auto sw = __builtin_amdgcn_permlane32_swap(
-            __float_as_uint(hc), __float_as_uint(e1), false, false);
-        hh = __uint_as_float(sw[0]);  // lanes 0-31: carry, 32-63: e1 of 0-31
+      for (int i = i0; i < i1; ++i) e1 = __builtin_fmaf(acc_a[i], e1, xn[i]);
+      const auto sw = __builtin_amdgcn_permlane32_swap(
+          __float_as_uint(hc), __float_as_uint(e1), false, false);
+      // lanes 0-31: carry, 32-63: e1 of 0-31
+      float hh = __uint_as_float(sw[0]);
+#pragma unroll
+      for (int i = i0; i < i1; ++i) {
+        hh = __builtin_fmaf(acc_a[i], hh, xn[i]);
+        keep(i, hh);
       }
+      const auto end = __builtin_amdgcn_permlane32_swap(
+          __float_as_uint(hh), __float_as_uint(hh), false, false);
+      hc = __uint_as_float(end[1]);  // all lanes: end value of 32-63
+    };
+    if (MODE == kChunkSummary) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        walk(4 * g, 4 * g + 4, [&](int i, float) { prod *= acc_a[i]; });
+    } else {
       float hv[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        hh = __builtin_fmaf(av[q], hh, xn[q]);
-        hv[q] = hh;
-      }
-      {
-        const auto sw = __builtin_amdgcn_permlane32_swap(
-            __float_as_uint(hh), __float_as_uint(hh), false, false);
-        hc = __uint_as_float(sw[1]);  // all lanes: end value of 32-63
-      }
-      if (MODE == kChunkSummary) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) prod *= av[q];
-        continue;
-      }
-      const uint32_t y01 = pack_bf16x2(hv[0], hv[1]);
-      const uint32_t y23 = pack_bf16x2(hv[2], hv[3]);
-      // the four tokens into the wave's patch: the low halves of the packed
-      // pairs, and the high halves as they are
-      const uint32_t pw = patch_w_lane + (8 * (g & 1)) * kPatchStride;
-      asm volatile(
-          "ds_write_b16 %0, %1\n\t"
-          "ds_write_b16_d16_hi %0, %1 offset:%3\n\t"
-          "ds_write_b16 %0, %2 offset:%4\n\t"
-          "ds_write_b16_d16_hi %0, %2 offset:%5"
-          :
-          : "v"(pw), "v"(y01), "v"(y23), "n"(kPatchStride),
-            "n"(2 * kPatchStride), "n"(3 * kPatchStride)
-          : "memory");
-      if (g & 1) {
-        // sixteen finished tokens are read back as 16-byte row chunks (the
-        // LDS unit executes a wave's instructions in order)
-        y_pending[g >> 1] = *reinterpret_cast<lds_u32x4*>(lds3 + patch_r_lane);
-        asm volatile("" ::: "memory");
-      }
+      walk(0, 16, [&](int i, float hh) {
+        hv[i & 3] = hh;
+        if ((i & 3) != 3) return;
+        const int g = i >> 2;
+        const uint32_t y01 = pack_bf16x2(hv[0], hv[1]);
+        const uint32_t y23 = pack_bf16x2(hv[2], hv[3]);
+        // four tokens into the wave's patch: the low halves of the packed
+        // pairs, and the high halves as they are
+        const uint32_t pw = patch_w_lane + 4 * (g & 1) * kPatchStride;
+        asm volatile(
+            "ds_write_b16 %0, %1\n\t"
+            "ds_write_b16_d16_hi %0, %1 offset:%3\n\t"
+            "ds_write_b16 %0, %2 offset:%4\n\t"
+            "ds_write_b16_d16_hi %0, %2 offset:%5"
+            :
+            : "v"(pw), "v"(y01), "v"(y23), "n"(kPatchStride),
+              "n"(2 * kPatchStride), "n"(3 * kPatchStride)
+            : "memory");
+        if (g & 1) {
+          // sixteen finished tokens are read back as 16-byte row chunks (the
+          // LDS unit executes a wave's instructions in order)
+          y_pending[g >> 1] = *reinterpret_cast<lds_u32x4*>(lds3 + patch_r_lane);
+          asm volatile("" ::: "memory");
+        }
+      });
     }
     if (GELU) {
       // y * gelu(gate branch), each factor a bf16 tensor as in the reference:
@@ -658,7 +678,7 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
     }
   }
   buffer_store_16(y_pending[0], ry, y_lane_bytes, y_pending_row);
-  buffer_store_16(y_pending[1], ry, y_lane_bytes, y_pending_row + 16u * row_bytes);
+  buffer_store_16(y_pending[1], ry, y_lane_bytes, y_pending_row + 8u * row_bytes);
 
   if (MODE == kChunkSummary) {
     // this chunk from a zero state: h_end = prod(a) * h_in + hc
