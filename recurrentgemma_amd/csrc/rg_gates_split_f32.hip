@@ -1,0 +1,519 @@
+// The matrix products of RGLRU's gates in float32 (256-wide heads,
+// recurrentgemma/torch/layers.py:127-137, called twice on the same x at
+// :338-339), forwards and both ways backwards, on the bf16 matrix instructions:
+//   forward   y_g[m, h, j] = sum_i x[m, h, i] w_g[h, i, j]
+//   data      dx[m, h, i] += sum_g sum_j dy_g[m, h, j] w_g[h, i, j]
+//   weights   dw_g[h, i, j] = sum_m x[m, h, i] dy_g[m, h, j]
+//
+// Every operand is cut into three bf16 pieces, each the nearest bf16 to what the
+// pieces before it leave (v = hi + mid + lo to 2^-27 of v), and a product is the
+// six products of pieces that weigh 2^-16 or more: what is left out, mid lo, lo
+// mid and lo lo, is below 2^-26 of it.  v_mfma_f32_32x32x16_bf16 multiplies
+// exactly and adds in float32; hi hi has an accumulator of its own, the five
+// others share one whose roundings are 2^-8 times smaller, so a chain of K / 16
+// roundings counts where the float32 instruction (32x32x2) has K / 2.  Six of
+// them take 192 cycles for what eight of the others need 512, and vector
+// instructions issue beside them.
+//
+// A workgroup of four waves owns 128 x 128 results, a wave 64 x 64 of them (two
+// accumulators for each: half of its registers).  A stage is 16 k: its 2 x 128 x
+// 16 floats are requested two stages ahead, cut between the matrix instructions
+// of the stage before it and laid into the other of two LDS buffers in operand
+// order (rows of 32 bytes padded to 48: eight lanes' 16 bytes meet every bank
+// once); 74 KB, so that two workgroups share a CU.  (Stages of 32 k cut between
+// barriers, one buffer: 3 to 10 % slower.)  An operand whose memory runs along k
+// is fetched eight k a lane with 16-byte loads, one whose memory runs along the
+// result's rows or columns with eight loads of a row of lanes each: either way a
+// lane has eight k of a row, and nothing is transposed.
+//
+// Bound by the matrix pipe at the clock that its power allows: 8192 rows of 10
+// heads are 1.06 PFLOP/s of bf16 products, what large library products reach
+// here.  us (and error of the result against 64 bits) / the float32 instruction's
+// kernels that were here before (data: the library's two batched products):
+//   rows               512         1001        2048        3003        8192
+//   10 heads forward  17 /  20    24 /  34    37 /  51    49 /  65   122 / 162
+//            data     25 /  39    26 /  57    41 /  94    48 /  83   120 / 195
+//            weights  26 /  26    29 /  35    41 /  53    54 /  73   127 / 190
+//   16 heads forward  20 /  22    27 /  36    50 /  67    72 /  97   210 / 267
+//            data     25 /  38    29 /  46    50 /  84    75 / 152   210 / 330
+//            weights  26 /  30    35 /  43    57 /  74    78 / 110   201 / 270
+// errors: forward 8.9e-8 / 2.1e-7, data 1.1e-7 / 2.4e-7, weights 7.7e-8 / 1.3e-7
+// at 512 rows and 2.2e-7 / 4.7e-7 at 8192.
+//
+// Infinities and NaN: a piece of an infinity is no number, and products of
+// pieces may overflow where the product does not.  Either leaves something that
+// is not finite among a wave's results; such a wave computes them again with the
+// float32 instruction and takes those for what was not finite (the others keep
+// their bits whatever their neighbours hold).
+#include <type_traits>
+
+#include "rg_common.h"
+#include "rg_internal.h"
+
+namespace rg {
+namespace {
+
+constexpr int kBW = 256;              // head width
+constexpr int kTile = 128;            // results of a workgroup, each way
+constexpr int kStage = 16;            // k per stage
+constexpr int kThreads = 256;
+constexpr int kRowBytes = 48;         // of an LDS row: 16 bf16, padded
+constexpr int kPieceBytes = kTile * kRowBytes;
+constexpr int kOperandBytes = 3 * kPieceBytes;
+constexpr int kBufferBytes = 2 * kOperandBytes;
+
+enum Kind { kForward = 0, kData = 1, kWeights = 2 };
+
+struct SplitArgs {
+  const float* x;      // [M, W] (kForward, kWeights)
+  const float* dy[2];  // [M, W] per gate (kData, kWeights)
+  const float* w[2];   // [H, 256, 256] per gate (kForward, kData)
+  float* out[2];       // kForward: [M, W] per gate; kData: [M, W];
+                       // kWeights: [H, 256, 256] per gate (one row range)
+  float* part;         // kWeights, several ranges: [splits][2 H][256][256]
+  int64_t M;
+  int W, H;
+  int tiles;           // kForward, kData: of 128 rows
+  int splits, rows_per_split;  // kWeights: row ranges
+};
+
+// One operand: element (r, k) of its 128 rows (of the result's rows or columns)
+// lies at byte r * row + k * step; elements outside the descriptor are zeros.
+struct Source {
+  __amdgpu_buffer_rsrc_t base;
+  uint32_t row, step;
+};
+
+struct Pieces {
+  u32x4 hi, mid, lo;  // eight k
+};
+
+__device__ __forceinline__ void cut(const float (&v)[8], Pieces& p) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+    p.hi[i] = pack_bf16x2(a, b);
+    a -= __uint_as_float(p.hi[i] << 16);
+    b -= __uint_as_float(p.hi[i] & 0xffff0000u);
+    p.mid[i] = pack_bf16x2(a, b);
+    a -= __uint_as_float(p.mid[i] << 16);
+    b -= __uint_as_float(p.mid[i] & 0xffff0000u);
+    p.lo[i] = pack_bf16x2(a, b);
+  }
+}
+
+// A thread's share of one operand's stage: eight k of a row.
+template <bool ALONG_K>
+struct Share {
+  float v[8];
+
+  static __device__ __forceinline__ int row(int tid) {
+    return ALONG_K ? tid >> 1 : tid & (kTile - 1);
+  }
+  static __device__ __forceinline__ int oct(int tid) {
+    return ALONG_K ? tid & 1 : tid / kTile;
+  }
+  // CHECKED: k may lie outside the operand (the descriptor checks the vector
+  // part of an offset, not the scalar one)
+  template <bool CHECKED>
+  __device__ __forceinline__ void request(const Source& s, uint32_t k0,
+                                          int tid) {
+    const uint32_t lane_at =
+        (uint32_t)row(tid) * s.row + 8u * (uint32_t)oct(tid) * s.step;
+    auto word = [&](uint32_t k) {
+      return __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(
+                     s.base, lane_at + (CHECKED ? k * s.step : 0u),
+                     CHECKED ? 0u : k * s.step, 0));
+    };
+    if constexpr (ALONG_K) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const f32x4 t = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(s.base, lane_at + 16u * q,
+                                                         k0 * s.step, 0));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[4 * q + i] = t[i];
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = word(k0 + (uint32_t)k);
+    }
+  }
+  __device__ __forceinline__ void store(unsigned char* lds, int tid) const {
+    unsigned char* const at = lds + row(tid) * kRowBytes + 16 * oct(tid);
+    Pieces p;
+    cut(v, p);
+    *reinterpret_cast<u32x4*>(at) = p.hi;
+    *reinterpret_cast<u32x4*>(at + kPieceBytes) = p.mid;
+    *reinterpret_cast<u32x4*>(at + 2 * kPieceBytes) = p.lo;
+  }
+};
+
+union Frag {
+  u32x4 u;
+  bf16x8 v;
+};
+
+template <int KIND>
+__global__ void __launch_bounds__(kThreads, 2)
+gates_split_f32_kernel(SplitArgs p) {
+  // operand A gives the results' rows, B their columns
+  constexpr bool kAlongKA = KIND != kWeights, kAlongKB = KIND == kData;
+  __shared__ __align__(16) unsigned char lds[2 * kBufferBytes];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // Workgroups go to the eight XCDs in turn: those that share rows of x or dy,
+  // or a head's weights, are dealt to one XCD.
+  int id = blockIdx.x;
+  {
+    const int per_xcd = (int)gridDim.x / 8;
+    if (id < 8 * per_xcd) id = (id & 7) * per_xcd + (id >> 3);
+  }
+  const uint32_t row_bytes = (uint32_t)p.W * 4u;
+  const uint32_t head_row = kBW * 4u;  // of a head's weights
+  constexpr uint32_t head_bytes = kBW * kBW * 4u;
+  Source a, b;
+  __amdgpu_buffer_rsrc_t a2, b2;  // kData: the recurrence gate's
+  int64_t m0 = 0;
+  int head, gate = 0, i0 = 0, j0 = 0, split = 0;
+  uint32_t rows = 0;    // of this workgroup's range (kWeights: along k)
+  uint32_t k_total;
+  if constexpr (KIND == kWeights) {
+    const int which = id & 7;
+    gate = which >> 2;
+    i0 = (which & 1) * kTile;
+    j0 = ((which >> 1) & 1) * kTile;
+    head = (id >> 3) % p.H;
+    split = (id >> 3) / p.H;
+    m0 = (int64_t)split * p.rows_per_split;
+    int64_t left = p.M - m0;
+    if (left > p.rows_per_split) left = p.rows_per_split;
+    rows = left > 0 ? (uint32_t)left : 0u;
+    a = {make_rsrc(p.x + m0 * p.W + head * kBW + i0,
+                   rows ? (rows - 1) * row_bytes + kTile * 4u : 0),
+         4u, row_bytes};
+    b = {make_rsrc((gate ? p.dy[1] : p.dy[0]) + m0 * p.W + head * kBW + j0,
+                   rows ? (rows - 1) * row_bytes + kTile * 4u : 0),
+         4u, row_bytes};
+    k_total = rows;
+  } else {
+    constexpr int kParts = KIND == kForward ? 4 : 2;  // of a head's results
+    const int part = id % kParts;
+    const int tile = (id / kParts) % p.tiles;
+    head = id / kParts / p.tiles;
+    gate = KIND == kForward ? part >> 1 : 0;
+    j0 = (part & 1) * kTile;
+    m0 = (int64_t)tile * kTile;
+    const int64_t left = p.M - m0;
+    rows = (uint32_t)(left < kTile ? left : kTile);
+    // (a descriptor ends with the last row's part of this head)
+    const uint32_t bytes = (rows - 1) * row_bytes + kBW * 4u;
+    if constexpr (KIND == kForward) {
+      a = {make_rsrc(p.x + m0 * p.W + head * kBW, bytes), row_bytes, 4u};
+      b = {make_rsrc((gate ? p.w[1] : p.w[0]) + (int64_t)head * kBW * kBW + j0,
+                     head_bytes - 4u * (uint32_t)j0),
+           4u, head_row};
+      k_total = kBW;
+    } else {
+      a = {make_rsrc(p.dy[0] + m0 * p.W + head * kBW, bytes), row_bytes, 4u};
+      a2 = make_rsrc(p.dy[1] + m0 * p.W + head * kBW, bytes);
+      const int64_t at = ((int64_t)head * kBW + j0) * kBW;
+      b = {make_rsrc(p.w[0] + at, kTile * head_row), head_row, 4u};
+      b2 = make_rsrc(p.w[1] + at, kTile * head_row);
+      k_total = 2 * kBW;
+    }
+  }
+
+  // Two stages of both operands in flight: a stage's floats are requested two
+  // stages ahead and cut during the one before it, between its matrix
+  // instructions.
+  Share<kAlongKA> sa[2];
+  Share<kAlongKB> sb[2];
+  auto request = [&](uint32_t k, auto SLOT) {
+    constexpr int slot = decltype(SLOT)::value;
+    constexpr bool checked = KIND == kWeights;
+    // (past the last stage: the first again, or zeros)
+    if (!checked) k &= k_total - 1;
+    const bool second = KIND == kData && k >= kBW;
+    if (second) k -= kBW;
+    const Source qa = {second ? a2 : a.base, a.row, a.step};
+    const Source qb = {second ? b2 : b.base, b.row, b.step};
+    sa[slot].template request<checked>(qa, k, tid);
+    sb[slot].template request<checked>(qb, k, tid);
+  };
+  // this wave's 64 x 64 results: 2 x 2 blocks
+  const int wr = 64 * (wave >> 1), wc = 64 * (wave & 1);
+  f32x16 big[2][2], small[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) big[i][j][r] = small[i][j][r] = 0.0f;
+  const unsigned char* const la =
+      lds + (wr + (lane & 31)) * kRowBytes + 16 * (lane >> 5);
+  const unsigned char* const lb =
+      lds + kOperandBytes + (wc + (lane & 31)) * kRowBytes + 16 * (lane >> 5);
+  // Stage k from buffer SLOT; the next one's floats are cut into the other
+  // buffer, and their registers take what is asked for of the stage after the
+  // one after it.
+  auto stage = [&](uint32_t k, auto SLOT) {
+    constexpr int slot = decltype(SLOT)::value;
+    Frag fa[2][3], fb[2][3];
+    auto pieces = [&](int q) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        fa[i][q].u = *reinterpret_cast<const u32x4*>(
+            la + slot * kBufferBytes + q * kPieceBytes + 32 * i * kRowBytes);
+        fb[i][q].u = *reinterpret_cast<const u32x4*>(
+            lb + slot * kBufferBytes + q * kPieceBytes + 32 * i * kRowBytes);
+      }
+    };
+    auto multiply = [&](f32x16 (&sum)[2][2], int qa, int qb) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              fa[i][qa].v, fb[j][qb].v, sum[i][j], 0, 0, 0);
+    };
+    pieces(0);
+    pieces(1);
+
+    multiply(big, 0, 0);
+    sa[slot ^ 1].store(lds + (slot ^ 1) * kBufferBytes, tid);
+    multiply(small, 0, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    pieces(2);
+    multiply(small, 1, 0);
+    sb[slot ^ 1].store(lds + (slot ^ 1) * kBufferBytes + kOperandBytes, tid);
+    multiply(small, 1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    request(k + 3 * kStage, std::integral_constant<int, slot ^ 1>{});
+    multiply(small, 0, 2);
+    multiply(small, 2, 0);
+
+    lds_barrier();
+  };
+  request(0, std::integral_constant<int, 0>{});
+  request(kStage, std::integral_constant<int, 1>{});
+  sa[0].store(lds, tid);
+  sb[0].store(lds + kOperandBytes, tid);
+  request(2 * kStage, std::integral_constant<int, 0>{});
+  lds_barrier();
+  for (uint32_t k = 0; k < k_total; k += 2 * kStage) {
+    stage(k, std::integral_constant<int, 0>{});
+    // (an odd number of stages ends with one of zeros)
+    stage(k + kStage, std::integral_constant<int, 1>{});
+  }
+
+  float odd = 0.0f;  // NaN as soon as one result is not finite
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        big[i][j][r] += small[i][j][r];
+        odd = __builtin_fmaf(big[i][j][r], 0.0f, odd);
+      }
+  if (__builtin_expect(__any(odd != 0.0f), 0)) {
+    // infinities, NaN or an overflow: the float32 instruction instead
+    auto element = [&](__amdgpu_buffer_rsrc_t base, const Source& s, uint32_t r,
+                       uint32_t k) {
+      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                           base, r * s.row + k * s.step, 0, 0));
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        f32x16 again;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) again[r] = 0.0f;
+        const uint32_t ra = (uint32_t)(wr + 32 * i + (lane & 31));
+        const uint32_t rb = (uint32_t)(wc + 32 * j + (lane & 31));
+        for (uint32_t k = 0; k < k_total; k += 2) {
+          const bool second = KIND == kData && k >= kBW;
+          const uint32_t kk = (second ? k - kBW : k) + (uint32_t)(lane >> 5);
+          const float va = element(second ? a2 : a.base, a, ra, kk);
+          const float vb = element(second ? b2 : b.base, b, rb, kk);
+          again = __builtin_amdgcn_mfma_f32_32x32x2f32(va, vb, again, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (big[i][j][r] * 0.0f != 0.0f) big[i][j][r] = again[r];
+      }
+  }
+
+  // block (i, j), result r of a lane: row 8 (r / 4) + 4 (lane / 32) + r % 4,
+  // column lane % 32
+  if constexpr (KIND == kWeights) {
+    float* const dst =
+        (p.splits == 1
+             ? (gate ? p.out[1] : p.out[0]) + (int64_t)head * kBW * kBW
+             : p.part + ((int64_t)split * 2 * p.H + gate * p.H + head) * kBW *
+                            kBW) +
+        (i0 + wr) * kBW + j0 + wc + (lane & 31);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) dst[row * kBW + 32 * j] = big[i][j][r];
+      }
+  } else {
+    // (rows past the end fall outside the descriptor)
+    const __amdgpu_buffer_rsrc_t ro =
+        make_rsrc((gate ? p.out[1] : p.out[0]) + m0 * p.W, rows * row_bytes);
+    const uint32_t at = (uint32_t)(wr + 4 * (lane >> 5)) * row_bytes +
+                        4u * (uint32_t)(head * kBW + j0 + wc + (lane & 31));
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        float before[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const uint32_t off =
+              at + (uint32_t)(32 * i + 8 * (r >> 2) + (r & 3)) * row_bytes +
+              128u * j;
+          before[r] = 0.0f;
+          if (KIND == kData)
+            before[r] = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(ro, off, 0, 0));
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const uint32_t off =
+              at + (uint32_t)(32 * i + 8 * (r >> 2) + (r & 3)) * row_bytes +
+              128u * j;
+          const float v = KIND == kData ? before[r] + big[i][j][r] : big[i][j][r];
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ro, off, 0, 0);
+        }
+      }
+  }
+}
+
+// Adds the row ranges' sums in their order.
+__global__ void __launch_bounds__(256)
+gates_wgrad_finish_kernel(const f32x4* __restrict__ part, int splits,
+                          int64_t items, f32x4* __restrict__ dwx,
+                          f32x4* __restrict__ dwa) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= 2 * items) return;
+  f32x4 v = part[e];
+  for (int s = 1; s < splits; ++s) {
+    const f32x4 w = part[(int64_t)s * 2 * items + e];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] += w[k];
+  }
+  if (e < items) dwx[e] = v;
+  else dwa[e - items] = v;
+}
+
+int splits_for(int64_t M, int H) {
+  // as many row ranges as keep every workgroup resident, two to a CU; at least
+  // four stages each
+  int64_t want = 512 / ((int64_t)8 * H);
+  const int64_t most = (M + 8 * kStage - 1) / (8 * kStage);
+  if (want > most) want = most;
+  return want < 1 ? 1 : (int)want;
+}
+
+int64_t rows_for(int64_t M, int splits) {
+  const int64_t rows = (M + splits - 1) / splits;
+  return (rows + 2 * kStage - 1) / (2 * kStage) * (2 * kStage);
+}
+
+template <int KIND>
+hipError_t launch(const SplitArgs& a, int64_t blocks, hipStream_t s) {
+  if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
+  gates_split_f32_kernel<KIND><<<dim3((unsigned)blocks), kThreads, 0, s>>>(a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool gates_f32_serves(int64_t M, int W, int H) {
+  // (128 rows of an operand are 32-bit offsets)
+  return M > 0 && H > 0 && H <= 32768 / 8 && W == H * kBW &&
+         (M + kTile - 1) / kTile * H * 4 <= 0x7fffffff;
+}
+
+hipError_t launch_gates_f32(const void* x, const void* w_x, const void* w_a,
+                            void* gx, void* ga, int64_t M, int W, int H,
+                            hipStream_t s) {
+  if (!gates_f32_serves(M, W, H)) return hipErrorInvalidValue;
+  SplitArgs a{};
+  a.x = (const float*)x;
+  a.w[0] = (const float*)w_x;
+  a.w[1] = (const float*)w_a;
+  a.out[0] = (float*)gx;
+  a.out[1] = (float*)ga;
+  a.M = M;
+  a.W = W;
+  a.H = H;
+  a.tiles = (int)((M + kTile - 1) / kTile);
+  return launch<kForward>(a, (int64_t)a.tiles * H * 4, s);
+}
+
+hipError_t launch_gates_dgrad_f32(const void* dgx, const void* dga,
+                                  const void* w_x, const void* w_a, void* dx,
+                                  int64_t M, int W, int H, hipStream_t s) {
+  if (!gates_f32_serves(M, W, H)) return hipErrorInvalidValue;
+  SplitArgs a{};
+  a.dy[0] = (const float*)dgx;
+  a.dy[1] = (const float*)dga;
+  a.w[0] = (const float*)w_x;
+  a.w[1] = (const float*)w_a;
+  a.out[0] = (float*)dx;
+  a.M = M;
+  a.W = W;
+  a.H = H;
+  a.tiles = (int)((M + kTile - 1) / kTile);
+  return launch<kData>(a, (int64_t)a.tiles * H * 2, s);
+}
+
+bool gates_wgrad_f32_serves(int64_t M, int W, int H) {
+  if (M <= 0 || H <= 0 || W != H * kBW || H > 4096) return false;
+  // offsets within a row range, a stage past its end, are 32 bits
+  return (uint64_t)(rows_for(M, splits_for(M, H)) + 4 * kStage) * (uint64_t)W *
+             4u < 0xffffffffull;
+}
+
+size_t gates_wgrad_f32_workspace_bytes(int64_t M, int W, int H) {
+  const int splits = splits_for(M, H);
+  return splits == 1 ? 0 : (size_t)splits * 2 * H * kBW * kBW * sizeof(float);
+}
+
+hipError_t launch_gates_wgrad_f32(const void* x, const void* dgx,
+                                  const void* dga, void* dwx, void* dwa,
+                                  void* workspace, int64_t M, int W, int H,
+                                  hipStream_t s) {
+  if (!gates_wgrad_f32_serves(M, W, H)) return hipErrorInvalidValue;
+  SplitArgs a{};
+  a.x = (const float*)x;
+  a.dy[0] = (const float*)dgx;
+  a.dy[1] = (const float*)dga;
+  a.out[0] = (float*)dwx;
+  a.out[1] = (float*)dwa;
+  a.part = (float*)workspace;
+  a.M = M;
+  a.W = W;
+  a.H = H;
+  a.splits = splits_for(M, H);
+  a.rows_per_split = (int)rows_for(M, a.splits);
+  hipError_t e = launch<kWeights>(a, (int64_t)H * a.splits * 8, s);
+  if (e != hipSuccess || a.splits == 1) return e;
+  const int64_t items = (int64_t)H * kBW * kBW / 4;
+  gates_wgrad_finish_kernel<<<dim3((unsigned)((2 * items + 255) / 256)), 256, 0,
+                              s>>>((const f32x4*)workspace, a.splits, items,
+                                   (f32x4*)dwx, (f32x4*)dwa);
+  return hipGetLastError();
+}
+
+}  // namespace rg

@@ -398,15 +398,16 @@ struct SumTask {
 constexpr int kMaxSumTasks = 8;
 hipError_t launch_sum_rows(const SumTask* tasks, int count, int dtype,
                            hipStream_t s);
-// rg_gates_f32.hip: both gate projections in float32 (256-wide heads, without
-// the biases).
+// rg_gates_split_f32.hip: both gate projections in float32 (256-wide heads, without
+// the biases); what they give back to x, added to dx; the gradients of their
+// weights (workspace may be null where that needs no bytes).
 bool gates_f32_serves(int64_t M, int W, int H);
 hipError_t launch_gates_f32(const void* x, const void* w_x, const void* w_a,
                             void* gx, void* ga, int64_t M, int W, int H,
                             hipStream_t s);
-
-// rg_gates_wgrad_f32.hip: weight gradients of both gate projections in float32
-// (256-wide heads); workspace may be null where it needs no bytes.
+hipError_t launch_gates_dgrad_f32(const void* dgx, const void* dga,
+                                  const void* w_x, const void* w_a, void* dx,
+                                  int64_t M, int W, int H, hipStream_t s);
 bool gates_wgrad_f32_serves(int64_t M, int W, int H);
 size_t gates_wgrad_f32_workspace_bytes(int64_t M, int W, int H);
 hipError_t launch_gates_wgrad_f32(const void* x, const void* dgx,

@@ -393,9 +393,14 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
                                            out(r.dw_a), out(ws), d.M(), (int)d.W,
                                            (int)H, d.stream));
     }
+    const bool data = rg::gates_f32_serves(d.M(), (int)d.W, (int)H);
+    if (data)  // added to the recurrence's share where it lies
+      check_hip(rg::launch_gates_dgrad_f32(in(dgx), in(dga), in(w_x), in(w_a),
+                                           out(r.dx), d.M(), (int)d.W, (int)H,
+                                           d.stream));
     for (int i = 0; i < 2; ++i) {
-      // added to the recurrence's share where it lies
-      at::baddbmm_out(dxs, dxs, dgs[i], w[i]->transpose(1, 2), 1, 1);
+      if (!data)
+        at::baddbmm_out(dxs, dxs, dgs[i], w[i]->transpose(1, 2), 1, 1);
       if (needs_w[i] && !pair) *dw[i] = at::bmm(xs.transpose(1, 2), dgs[i]);
       if (!needs_b[i]) continue;
       if (tiles)
