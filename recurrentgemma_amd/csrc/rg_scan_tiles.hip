@@ -48,6 +48,25 @@ __device__ __forceinline__ float choose(bool cond, float a, float b) {
   return cond ? a : b;
 }
 
+// 1 - a^2 for a = 2^q, q <= 0, in float32: near a = 1, where the difference of the
+// rounded square would keep few of its digits, -2q (ln 2 + 2q (ln 2)^2 / 2! + ..),
+// eight terms of the exponential's series (the ninth is 2e-8 of the first).  With
+// it the float32 forms can use the hardware's exp2, reciprocal and square root
+// (RG-LRU step B3 T1001 W2560: 254 -> 238 us against expf, sqrtf and divisions)
+// and are closer to 64 bits (y 1.9e-7 -> 1.2e-7, its gradients 2.2e-7 .. 4.0e-7
+// -> 1.4e-7 .. 2.4e-7, the projections' part of that included).
+__device__ __forceinline__ float one_minus_square(float q, float a) {
+  constexpr float kSeries[8] = {0.69314718056f,    0.24022650696f,
+                                5.5504108665e-2f,  9.6181291076e-3f,
+                                1.3333558146e-3f,  1.5403530393e-4f,
+                                1.5252733804e-5f,  1.3215486790e-6f};
+  const float w = 2.0f * q;
+  float s = kSeries[7];
+#pragma unroll
+  for (int k = 6; k >= 0; --k) s = __builtin_fmaf(s, w, kSeries[k]);
+  return w > -0.75f ? -w * s : __builtin_fmaf(-a, a, 1.0f);
+}
+
 constexpr int streams_of(int mode) {
   return mode == kFwdPlain ? 2 : mode == kBwdGated ? 5 : 3;
 }
@@ -106,8 +125,9 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
   constexpr int NS = streams_of(MODE);
   constexpr bool kBwd = MODE == kBwdPlain || MODE == kBwdGated;
   constexpr bool kGated = MODE == kFwdGated || MODE == kBwdGated;
-  constexpr bool kFast = sizeof(T) == 2;  // hardware exp2 / rcp, as in the
-                                          // other bf16 kernels
+  // (both types: the hardware's exp2, reciprocal and square root; float32 forms
+  // 1 - a^2 without the cancellation, see below)
+  constexpr bool kFast = sizeof(T) == 2;
   constexpr bool kBias = kGated && !kFast;
   constexpr int kSegs = kThreads / CH;    // scanning threads of a channel
   constexpr int kPer = kGroups / kSegs;   // pairs each of them takes
@@ -231,8 +251,9 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
       for (int e = 0; e < N; ++e) v[e] += b_[e];
     }
   };
-  auto sigmoid_of = [](float v) {
-    return kFast ? sigmoid_fast(v) : sigmoid_precise(v);
+  // 1 - a^2 with a = 2^q
+  auto rest_of = [](float q, float a) __attribute__((always_inline)) {
+    return kFast ? __builtin_fmaf(-a, a, 1.0f) : one_minus_square(q, a);
   };
 
   // The scanning thread's channel and its state before the step.
@@ -336,18 +357,15 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
         }
 #pragma unroll
         for (int e = 0; e < N; ++e) {
-          const float gate_a = sigmoid_of(ga[e]);
-          coef[i][e] = kFast ? __builtin_amdgcn_exp2f(gate_a * ((-8.0f * kLog2e) * sp[e]))
-                             : expf((-8.0f * gate_a) * sp[e]);
+          const float gate_a = sigmoid_fast(ga[e]);
+          const float log2_a = gate_a * ((-8.0f * kLog2e) * sp[e]);
+          coef[i][e] = __builtin_amdgcn_exp2f(log2_a);
           cf[e] = coef[i][e];
           if constexpr (kKeepGate) kept[i][e] = gate_a;
           if constexpr (MODE == kFwdGated) {
-            const float gate_x = sigmoid_of(gx[e]);
-            float m = kFast
-                          ? __builtin_amdgcn_sqrtf(
-                                __builtin_fmaf(-coef[i][e], coef[i][e], 1.0f))
-                          : sqrtf(1.0f - expf(2.0f * ((-8.0f * gate_a) * sp[e])));
-            m = choose(start, 1.0f, m);
+            const float gate_x = sigmoid_fast(gx[e]);
+            const float m = choose(
+                start, 1.0f, __builtin_amdgcn_sqrtf(rest_of(log2_a, coef[i][e])));
             first[e] = (first[e] * gate_x) * m;
             kept[i][e] = first[e];
           }
@@ -494,22 +512,21 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
 #pragma unroll
           for (int e = 0; e < N; ++e) {
             const float a = coef[i][e];
-            const float gate_a = kKeepGate ? kept[kKeepGate ? i : 0][e] : sigmoid_of(pa[e]);
+            const float gate_a = kKeepGate ? kept[kKeepGate ? i : 0][e] : sigmoid_fast(pa[e]);
             const float c_t =
                 choose(start, 0.0f, choose(t >= T_len, 1.0f, a));
             st[e] = c_t * g[e];
             const float gr = round_act<T>(g[e]);  // the gradient of xn as a tensor
-            const float gate_x = sigmoid_of(px[e]);
-            const float a2 =
-                kFast ? a * a : expf(2.0f * ((-8.0f * gate_a) * sp[e]));
-            const float om = 1.0f - a2;
-            const float m = choose(
-                start, 1.0f, kFast ? __builtin_amdgcn_sqrtf(om) : sqrtf(om));
+            const float gate_x = sigmoid_fast(px[e]);
+            const float om =
+                kFast ? 1.0f - a * a
+                      : one_minus_square(gate_a * ((-8.0f * kLog2e) * sp[e]), a);
+            const float a2 = a * a;
+            const float m = choose(start, 1.0f, __builtin_amdgcn_sqrtf(om));
             const float d_gated = gr * m;
             const float d_m = gr * (x[e] * gate_x);
             const float clipped = fmaxf(4.0f * om, 1e-6f);
-            const float d_om = kFast ? d_m * __builtin_amdgcn_rsqf(clipped)
-                                     : d_m / sqrtf(clipped);
+            const float d_om = d_m * __builtin_amdgcn_rsqf(clipped);
             const float d_log_a = choose(start || !inside, 0.0f,
                                          (gr * hp[e]) * a - 2.0f * a2 * d_om);
             dx[e] = d_gated * gate_x;
