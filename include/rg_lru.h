@@ -302,9 +302,14 @@ int rg_recurrent_prefill_gelu_mul(
  * (recurrentgemma/torch/modules.py:632-643), for every shape and both dtypes,
  * with the choice of kernels made here: a single prefill kernel (bf16, heads
  * of 256 channels: rg_recurrent_prefill_split, but for very many rows of a few
- * tokens; heads of 136 .. 248 channels where that is ahead); for float32 with 256-wide heads and at most 32
- * (row, head) pairs one launch that does the same in float32 (needs no
- * workspace; no entry point of its own); else rg_gates_gemm with the conv
+ * tokens; heads of 136 .. 248 channels where that is ahead); for float32 with
+ * 256-wide heads and at most 32 (row, head) pairs one launch that does the same
+ * in float32 (needs no workspace; no entry point of its own), with more pairs
+ * rg_conv1d_prefill, the projections on the bf16 matrix instruction with every
+ * operand in three pieces (closer to the exact products than rg_gates_gemm) and a
+ * recurrence of its own, conv output and pre-activations living in the workspace
+ * (taken for fewer pairs too where it is faster and the caller brings a workspace
+ * that holds three times x); else rg_gates_gemm with the conv
  * applied on load followed by rg_lru_scan_fused_split, the pre-activations of
  * both gates living in the workspace.  gate_branch (nullable, [B,T,W]): the
  * block's linear_y output; `out` is then rglru(conv1d(x)) * gelu_tanh(
@@ -313,7 +318,7 @@ int rg_recurrent_prefill_gelu_mul(
  * rg_gelu_mul over `out` as a last launch), else the plain RG-LRU output.  `workspace` (16-byte aligned)
  * must hold rg_recurrent_core_workspace_bytes(B, T, W, H, dtype) bytes (0 for
  * whole rows in the single kernel: workspace may then be null).  Same values
- * as the calls it is made of; h0 / h_last / conv_cache_out / w_packed as in
+ * as the calls it is made of (float32 with 256-wide heads: to rounding); h0 / h_last / conv_cache_out / w_packed as in
  * rg_recurrent_prefill (w_packed is only read by the single kernel).
  * conv_w == conv_b == NULL (conv_cache_out then NULL too): x is the conv
  * output already, and the call is RGLRU.forward on its own

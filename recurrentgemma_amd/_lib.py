@@ -119,6 +119,7 @@ PACKAGE_SIGNATURES = {
                             [_i] * 5 + [ctypes.c_float, _i, _vp]),
     "rg_argmax_workspace_bytes": (_sz, [_i, _i]),
     "rg_argmax_rows_split": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
+    "rg_recurrent_core_best_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
 }
 
 _lib = None

@@ -16,6 +16,7 @@
 //
 // Plain C++ on torch's and this library's public interfaces; no device code.
 #include "host_call.h"
+#include "rg_package_calls.h"
 
 namespace {
 
@@ -196,7 +197,7 @@ PyObject* recurrent_core(PyObject*, PyObject* const* v, Py_ssize_t n) {
     Tensor y = c.empty(c.x.sizes()), h, cache, ws;
     if (v[10] == Py_True) h = c.empty({B, W}, at::kFloat);
     if (v[11] == Py_True && conv) cache = c.empty({B, 3, W});
-    const size_t bytes = rg_recurrent_core_workspace_bytes(
+    const size_t bytes = rg_recurrent_core_best_workspace_bytes(
         (int)B, (int)T, (int)W, (int)H, c.code);
     if (bytes) ws = c.empty({(int64_t)bytes}, at::kByte);
     void* yp = y.mutable_data_ptr();

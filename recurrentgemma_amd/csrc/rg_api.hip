@@ -589,16 +589,54 @@ int rg_recurrent_prefill_gelu_mul(
 // scan kernel with the pre-activations of both gates in the workspace.
 struct CorePlan {
   bool small_f32;      // core_f32_small_kernel: everything in one launch
+  bool wide_f32;       // conv, gate projections on bf16 pieces, one-pass scan
   bool single;         // block_prefill_bf16_kernel
   size_t split_bytes;  // chunk summaries of whichever form runs
   size_t gate_bytes;   // one gate's pre-activations (two-kernel form), padded
+  size_t wide_bytes;   // what the wide_f32 form needs where it takes the shape
+  size_t need() const {
+    return small_f32 ? 0 : wide_f32 ? wide_bytes : split_bytes + 2 * gate_bytes;
+  }
 };
+// The float32 form of several launches (conv, gate projections on bf16 pieces,
+// recurrence) for 256-wide heads: which recurrence kernel, and where it is ahead.
+//
+// The one-pass kernel takes 256 tokens of 32 channels a step, one workgroup a CU;
+// many slabs of short rows go to the kernel that costs by the token.  us for the
+// whole call, one-pass / by the token: W2560 B3 T16 20.2 / 20.5, B8 T30 34 / 27,
+// B16 T16 43 / 27, T100 75 / 80, B30 T40 80 / 58, B64 T64 173 / 129, T250 502 / 533
+// (joined); W4096 B3 T128 40 / 46, B16 T100 102 / 92, T1000 719 / 733.
+static bool wide_scan_on_tiles(int B, int T, int W) {
+  const int64_t slabs = (int64_t)B * ((W + 31) / 32);
+  return T >= (slabs <= 256 ? 1 : slabs <= 1024 ? 64 : slabs < 2048 ? 96 : 192);
+}
+// Against one launch for everything (at most 32 pairs, 16 of them at a time, 512
+// tokens in 33 us; the other form about 17 us + 1.1e-5 us an element): us, one
+// launch / several: W2560 T1 35 / 18, T200 34 / 24, T512 34.5 / 33.5, T2048 120 / 78,
+// B2 T64 66 / 22, B3 T512 67 / 52; W4096 T512 35 / 39, T1024 64 / 56; W256 B8 T512
+// 34 / 28.  Against gate GEMM + scan (more pairs) everywhere but a few rows of all:
+// W2560 B64 T1 20.5 / 23, T16 73 / 50, B4 T2048 519 / 240, B8 T2048 joined 878 / 523;
+// W4096 B3 T16 18 / 22, B4 T512 206 / 93; W256 B64 T16 19.2 / 20.5, T64 37 / 29.
+static bool wide_f32_pays(int B, int T, int W, int H, bool one_launch_takes) {
+  const float elements = (float)B * T * W;
+  if (!one_launch_takes) return elements > 3e5f;
+  const float one_launch =
+      33.0f * (((int64_t)B * H + 15) / 16) * ((T + 511) / 512);
+  return 17.0f + 1.1e-5f * elements < 0.95f * one_launch;
+}
+
 static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
   CorePlan p{};
-  // float32 with few rows: one launch, no workspace (a short float32 call is
-  // three launches' worth of latency otherwise)
+  // float32 with few rows: one launch, no workspace; or, with one, the form of
+  // several launches where that is ahead
   p.small_f32 = dtype == RG_DTYPE_F32 && rg::core_f32_small_serves(B, T, W, H);
-  if (p.small_f32) return p;
+  if (dtype == RG_DTYPE_F32 && rg::gates_f32_serves((int64_t)B * T, W, H) &&
+      rg::scan_tiles_take(T, W, dtype) && wide_f32_pays(B, T, W, H, p.small_f32)) {
+    const size_t n = (size_t)B * T * W * sizeof(float);
+    p.wide_bytes = 3 * ((n + 255) & ~(size_t)255);
+    p.wide_f32 = !p.small_f32;
+  }
+  if (p.small_f32 || p.wide_f32) return p;
   const bool fits = dtype == RG_DTYPE_BF16 && single_takes(W / H) &&
                     (int64_t)T * W * 2 < (int64_t)0x7fffffff;
   const size_t chunk_bytes =
@@ -634,8 +672,16 @@ size_t rg_recurrent_core_workspace_bytes(int B, int T, int W, int H,
   if (B <= 0 || T <= 0 || W <= 0 || H <= 0 || W % H != 0 ||
       (dtype != RG_DTYPE_F32 && dtype != RG_DTYPE_BF16))
     return 0;
+  return core_plan(B, T, W, H, dtype).need();
+}
+
+size_t rg_recurrent_core_best_workspace_bytes(int B, int T, int W, int H,
+                                              int dtype) {
+  if (B <= 0 || T <= 0 || W <= 0 || H <= 0 || W % H != 0 ||
+      (dtype != RG_DTYPE_F32 && dtype != RG_DTYPE_BF16))
+    return 0;
   const CorePlan p = core_plan(B, T, W, H, dtype);
-  return p.split_bytes + 2 * p.gate_bytes;
+  return p.wide_bytes ? p.wide_bytes : p.need();
 }
 
 int rg_recurrent_core(const void* x, const void* gate_branch,
@@ -659,14 +705,18 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
   RG_REQUIRE(conv_w != nullptr || conv_cache_out == nullptr,
              "%s: no conv state without a conv", __func__);
   const int conv = conv_w != nullptr;
-  const CorePlan p = core_plan(B, T, W, H, dtype);
-  const size_t need = p.split_bytes + 2 * p.gate_bytes;
+  CorePlan p = core_plan(B, T, W, H, dtype);
+  const size_t need = p.need();
   if (need > 0 && (workspace == nullptr || workspace_bytes < need ||
                    !aligned16(workspace)))
     return fail(RG_ERR_WORKSPACE,
                 "%s: workspace of %zu bytes (16-byte aligned) required, got %zu",
                 __func__, need, workspace ? workspace_bytes : (size_t)0);
-  if (p.small_f32) {
+  // the one-launch form where the caller has brought no more than it needs
+  if (p.small_f32 && p.wide_bytes && workspace != nullptr &&
+      workspace_bytes >= p.wide_bytes && aligned16(workspace))
+    p.wide_f32 = true;
+  if (p.small_f32 || p.wide_f32) {
     RG_CHECK_PTR(x);
     RG_CHECK_PTR(segpos);
     RG_CHECK_OPT_PTR(conv_w);
@@ -681,6 +731,57 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
     RG_CHECK_OPT_PTR(h_last);
     RG_CHECK_OPT_PTR(conv_cache_out);
     RG_REQUIRE(out != x, "%s: out must not alias x", __func__);
+    if (p.wide_f32) {
+      char* const ws = (char*)workspace;
+      const size_t plane = p.wide_bytes / 3;
+      void* const gx = ws;
+      void* const ga = ws + plane;
+      const void* xc = x;
+      if (conv) {
+        xc = ws + 2 * plane;
+        const int rc = rg_conv1d_prefill(x, segpos, segpos_is_i64, conv_w, conv_b,
+                                         ws + 2 * plane, conv_cache_out, B, T, W, 4,
+                                         dtype, stream);
+        if (rc != RG_OK) return rc;
+      }
+      // (the one-pass kernel adds the biases itself, and reads the other branch
+      // where it writes)
+      const bool tiles = wide_scan_on_tiles(B, T, W) || gate_branch == out;
+      int rc = launch_status(
+          __func__, rg::launch_gates_f32(xc, w_x, w_a, tiles ? nullptr : b_x,
+                                         tiles ? nullptr : b_a, gx, ga,
+                                         (int64_t)B * T, W, H,
+                                         (hipStream_t)stream));
+      if (rc != RG_OK) return rc;
+      if (!tiles) {
+        rc = rg_lru_scan_fused(xc, 0, nullptr, nullptr, gx, ga, a_param, segpos,
+                               segpos_is_i64, h0, out, h_last, nullptr, B, T, W,
+                               dtype, stream);
+        if (rc != RG_OK || gate_branch == nullptr) return rc;
+        return launch_status(
+            __func__, rg::launch_gelu_mul(out, gate_branch, out, (int64_t)B * T * W,
+                                          dtype, (hipStream_t)stream));
+      }
+      rg::ScanTileArgs t{};
+      t.in[0] = xc;
+      t.in[1] = gx;
+      t.in[2] = ga;
+      t.in[3] = gate_branch;  // the join is in the kernel's y stores
+      t.flags = segpos;
+      t.flag_kind = segpos_is_i64 ? rg::kSegI64 : rg::kSegI32;
+      t.a_param = a_param;
+      t.bias[0] = b_x;
+      t.bias[1] = b_a;
+      t.init = (const float*)h0;
+      t.out[0] = out;
+      t.last = (float*)h_last;
+      t.B = B;
+      t.T = T;
+      t.W = W;
+      return launch_status(__func__,
+                           rg::launch_scan_tiles(t, rg::kTilesFwdGated, dtype,
+                                                 (hipStream_t)stream));
+    }
     rg::FusedArgs a{};
     a.x = x;
     a.segpos = segpos;

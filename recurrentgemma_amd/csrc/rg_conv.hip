@@ -1,6 +1,8 @@
 // Stand-alone Conv1D kernels (any temporal width): the module-level drop-in
 // for Conv1D.forward.  The fused prefill path does the width-4 conv inside the
 // gate GEMM and the scan kernel instead and does not come through here.
+#include <type_traits>
+
 #include "rg_common.h"
 #include "rg_internal.h"
 
@@ -184,13 +186,14 @@ __device__ __forceinline__ bool conv_row_starts(const void* segpos, int seg_kind
 }
 
 // RUN rows per wave: the longer, the fewer halo rows are read twice (3 per
-// run) and the fewer workgroups are dispatched.
+// run) and the fewer workgroups are dispatched.  The blocks behind the runs, one
+// for every sequence, write its conv state (conv1d_cache_tail_kernel's).
 template <typename T, int RUN>
 __global__ void __launch_bounds__(1024)
 conv1d_prefill_k4_kernel(const T* __restrict__ x, const void* __restrict__ segpos,
                          int seg_kind, const T* __restrict__ w,
                          const T* __restrict__ bias, T* __restrict__ out,
-                         int T_len, int W, int64_t M) {
+                         T* __restrict__ cache_out, int T_len, int W, int64_t M) {
   using V = Vec16<T>;
   constexpr int N = V::N;
   // the waves of a workgroup lie side by side along a row (up to 16 of them:
@@ -198,6 +201,20 @@ conv1d_prefill_k4_kernel(const T* __restrict__ x, const void* __restrict__ segpo
   const int c = ((int)blockIdx.y * (int)blockDim.x + (int)threadIdx.x) * N;
   if (c >= W) return;  // W % N == 0 (launcher): a lane is inside or outside
   const int64_t m0 = (int64_t)blockIdx.x * RUN;
+  if (m0 >= M) {
+    const int64_t b = (int64_t)blockIdx.x - (M + RUN - 1) / RUN;
+    bool cut = false;  // a document starts behind the row
+#pragma unroll
+    for (int k = 2; k >= 0; --k) {
+      const int t = T_len - 3 + k;
+      u32x4 v = {0, 0, 0, 0};
+      if (t >= 0 && !cut)
+        v = *reinterpret_cast<const u32x4*>(x + (b * T_len + t) * W + c);
+      *reinterpret_cast<u32x4*>(cache_out + (b * 3 + k) * W + c) = v;
+      if (t >= 0 && is_doc_start(segpos, seg_kind, b * T_len + t)) cut = true;
+    }
+    return;
+  }
   const int64_t m1 = m0 + RUN < M ? m0 + RUN : M;
   const SeqStarts seq(m0 >= 3 ? m0 - 3 : 0, T_len, RUN + 3);
   auto row = [&](const T* base, int64_t m) {
@@ -547,24 +564,30 @@ hipError_t conv_prefill_t(const ConvArgs& a, hipStream_t s) {
     const unsigned slabs = (unsigned)((a.W / N + 63) / 64);
     const unsigned waves = slabs < 16 ? slabs : 16;  // per workgroup
     const unsigned across = (slabs + waves - 1) / waves;
-    // long runs where that still leaves eight waves for every SIMD
-    constexpr int kLongRun = 128;
-    if ((M / kLongRun) * slabs >= 8192) {
-      const dim3 grid((unsigned)((M + kLongRun - 1) / kLongRun), across);
-      conv1d_prefill_k4_kernel<T, kLongRun><<<grid, waves * 64, 0, s>>>(
-          (const T*)a.x, a.segpos, a.seg_kind, (const T*)a.w,
-          (const T*)a.bias, (T*)a.out, a.T, a.W, M);
-    } else {
-      const dim3 grid((unsigned)((M + kConvRun - 1) / kConvRun), across);
-      conv1d_prefill_k4_kernel<T, kConvRun><<<grid, waves * 64, 0, s>>>(
-          (const T*)a.x, a.segpos, a.seg_kind, (const T*)a.w,
-          (const T*)a.bias, (T*)a.out, a.T, a.W, M);
-    }
-  } else {
-    conv1d_prefill_kernel<T><<<grid_for(total, 256), 256, 0, s>>>(
-        (const T*)a.x, a.segpos, a.seg_kind, (const T*)a.w,
-        (const T*)a.bias, (T*)a.out, a.T, a.W, a.K, total);
+    const int tails = a.cache_out ? a.B : 0;
+    auto launch = [&](auto RUN) {
+      constexpr int run = decltype(RUN)::value;
+      const dim3 grid((unsigned)((M + run - 1) / run + tails), across);
+      conv1d_prefill_k4_kernel<T, run><<<grid, waves * 64, 0, s>>>(
+          (const T*)a.x, a.segpos, a.seg_kind, (const T*)a.w, (const T*)a.bias,
+          (T*)a.out, (T*)a.cache_out, a.T, a.W, M);
+    };
+    // long runs where that still leaves eight waves for every SIMD, short ones
+    // where runs of 32 leave fewer than two: a run's rows come eight at a time,
+    // one memory round trip after the other (B1 T512 W2560 float32: 16 us, 8 rows
+    // 6)
+    constexpr int kLongRun = 128, kShortRun = 8;
+    if ((M / kLongRun) * slabs >= 8192)
+      launch(std::integral_constant<int, kLongRun>{});
+    else if ((M / kConvRun) * slabs >= 2048)
+      launch(std::integral_constant<int, kConvRun>{});
+    else
+      launch(std::integral_constant<int, kShortRun>{});
+    return hipGetLastError();
   }
+  conv1d_prefill_kernel<T><<<grid_for(total, 256), 256, 0, s>>>(
+      (const T*)a.x, a.segpos, a.seg_kind, (const T*)a.w, (const T*)a.bias,
+      (T*)a.out, a.T, a.W, a.K, total);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !a.cache_out) return e;
   const int64_t ctotal = (int64_t)a.B * (a.K - 1) * a.W;

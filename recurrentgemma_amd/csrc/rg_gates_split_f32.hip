@@ -19,12 +19,12 @@
 // accumulators for each: half of its registers).  A stage is 16 k: its 2 x 128 x
 // 16 floats are requested two stages ahead, cut between the matrix instructions
 // of the stage before it and laid into the other of two LDS buffers in operand
-// order (rows of 32 bytes padded to 48: eight lanes' 16 bytes meet every bank
-// once); 74 KB, so that two workgroups share a CU.  (Stages of 32 k cut between
-// barriers, one buffer: 3 to 10 % slower.)  An operand whose memory runs along k
-// is fetched eight k a lane with 16-byte loads, one whose memory runs along the
-// result's rows or columns with eight loads of a row of lanes each: either way a
-// lane has eight k of a row, and nothing is transposed.
+// order; 48 KB, two workgroups a CU.  (Stages of 32 k cut between barriers, one
+// buffer: 3 to 10 % slower.)  An operand whose memory runs along k is fetched
+// eight k a lane with 16-byte loads, one whose memory runs along the result's rows
+// or columns with eight loads of a row of lanes each: either way a lane has eight
+// k of a row, and nothing is transposed.  Few rows: a quarter of the results and
+// twice the k per stage (launch_rows).
 //
 // Bound by the matrix pipe at the clock that its power allows: 8192 rows of 10
 // heads are 1.06 PFLOP/s of bf16 products, what large library products reach
@@ -54,13 +54,26 @@ namespace rg {
 namespace {
 
 constexpr int kBW = 256;              // head width
-constexpr int kTile = 128;            // results of a workgroup, each way
-constexpr int kStage = 16;            // k per stage
 constexpr int kThreads = 256;
-constexpr int kRowBytes = 48;         // of an LDS row: 16 bf16, padded
-constexpr int kPieceBytes = kTile * kRowBytes;
-constexpr int kOperandBytes = 3 * kPieceBytes;
-constexpr int kBufferBytes = 2 * kOperandBytes;
+
+// The two sizes of a workgroup: a wave has BLOCKS x BLOCKS blocks of 32 x 32
+// results, a stage is as many k as give every thread eight of each operand.
+template <int BLOCKS>
+struct Size {
+  static constexpr int tile = 64 * BLOCKS;    // results, each way
+  static constexpr int stage = 32 / BLOCKS;   // k
+  static constexpr int row = 2 * stage;       // bytes of an LDS row
+  static constexpr int piece = tile * row;
+  static constexpr int operand = 3 * piece;
+  static constexpr int buffer = 2 * operand;
+  // Where a row keeps its k-th eight of k (16 bytes): turned so that the same
+  // eight of eight rows in a row, which eight lanes read at once, lie in
+  // different banks.
+  static __host__ __device__ constexpr int at(int row_, int oct) {
+    constexpr int octs = stage / 8;
+    return row_ * row + 16 * (oct ^ (row_ / (8 / octs) % octs));
+  }
+};
 
 enum Kind { kForward = 0, kData = 1, kWeights = 2 };
 
@@ -70,15 +83,15 @@ struct SplitArgs {
   const float* w[2];   // [H, 256, 256] per gate (kForward, kData)
   float* out[2];       // kForward: [M, W] per gate; kData: [M, W];
                        // kWeights: [H, 256, 256] per gate (one row range)
+  const float* bias[2];  // kForward: [W] per gate, or null
   float* part;         // kWeights, several ranges: [splits][2 H][256][256]
   int64_t M;
   int W, H;
-  int tiles;           // kForward, kData: of 128 rows
+  int tiles;           // kForward, kData: of rows
   int splits, rows_per_split;  // kWeights: row ranges
 };
 
-// One operand: element (r, k) of its 128 rows (of the result's rows or columns)
-// lies at byte r * row + k * step; elements outside the descriptor are zeros.
+// One operand: element (r, k) of its rows (of the result's rows or columns) lies at byte r * row + k * step; elements outside the descriptor are zeros.
 struct Source {
   __amdgpu_buffer_rsrc_t base;
   uint32_t row, step;
@@ -103,15 +116,15 @@ __device__ __forceinline__ void cut(const float (&v)[8], Pieces& p) {
 }
 
 // A thread's share of one operand's stage: eight k of a row.
-template <bool ALONG_K>
+template <class S, bool ALONG_K>
 struct Share {
   float v[8];
 
   static __device__ __forceinline__ int row(int tid) {
-    return ALONG_K ? tid >> 1 : tid & (kTile - 1);
+    return ALONG_K ? tid / (S::stage / 8) : tid % S::tile;
   }
   static __device__ __forceinline__ int oct(int tid) {
-    return ALONG_K ? tid & 1 : tid / kTile;
+    return ALONG_K ? tid % (S::stage / 8) : tid / S::tile;
   }
   // CHECKED: k may lie outside the operand (the descriptor checks the vector
   // part of an offset, not the scalar one)
@@ -141,12 +154,12 @@ struct Share {
     }
   }
   __device__ __forceinline__ void store(unsigned char* lds, int tid) const {
-    unsigned char* const at = lds + row(tid) * kRowBytes + 16 * oct(tid);
+    unsigned char* const at = lds + S::at(row(tid), oct(tid));
     Pieces p;
     cut(v, p);
     *reinterpret_cast<u32x4*>(at) = p.hi;
-    *reinterpret_cast<u32x4*>(at + kPieceBytes) = p.mid;
-    *reinterpret_cast<u32x4*>(at + 2 * kPieceBytes) = p.lo;
+    *reinterpret_cast<u32x4*>(at + S::piece) = p.mid;
+    *reinterpret_cast<u32x4*>(at + 2 * S::piece) = p.lo;
   }
 };
 
@@ -155,12 +168,14 @@ union Frag {
   bf16x8 v;
 };
 
-template <int KIND>
-__global__ void __launch_bounds__(kThreads, 2)
+template <int KIND, int BLOCKS>
+__global__ void __launch_bounds__(kThreads, BLOCKS == 1 ? 3 : 2)
 gates_split_f32_kernel(SplitArgs p) {
+  using S = Size<BLOCKS>;
+  constexpr int kTile = S::tile, kStage = S::stage;
   // operand A gives the results' rows, B their columns
   constexpr bool kAlongKA = KIND != kWeights, kAlongKB = KIND == kData;
-  __shared__ __align__(16) unsigned char lds[2 * kBufferBytes];
+  __shared__ __align__(16) unsigned char lds[2 * S::buffer];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -181,12 +196,13 @@ gates_split_f32_kernel(SplitArgs p) {
   uint32_t rows = 0;    // of this workgroup's range (kWeights: along k)
   uint32_t k_total;
   if constexpr (KIND == kWeights) {
-    const int which = id & 7;
-    gate = which >> 2;
-    i0 = (which & 1) * kTile;
-    j0 = ((which >> 1) & 1) * kTile;
-    head = (id >> 3) % p.H;
-    split = (id >> 3) / p.H;
+    constexpr int kSide = kBW / kTile, kParts = 2 * kSide * kSide;
+    const int which = id % kParts;
+    gate = which / (kSide * kSide);
+    i0 = which % kSide * kTile;
+    j0 = which / kSide % kSide * kTile;
+    head = id / kParts % p.H;
+    split = id / kParts / p.H;
     m0 = (int64_t)split * p.rows_per_split;
     int64_t left = p.M - m0;
     if (left > p.rows_per_split) left = p.rows_per_split;
@@ -199,12 +215,13 @@ gates_split_f32_kernel(SplitArgs p) {
          4u, row_bytes};
     k_total = rows;
   } else {
-    constexpr int kParts = KIND == kForward ? 4 : 2;  // of a head's results
+    constexpr int kSide = kBW / kTile;  // parts of a gate's results
+    constexpr int kParts = KIND == kForward ? 2 * kSide : kSide;
     const int part = id % kParts;
-    const int tile = (id / kParts) % p.tiles;
+    const int tile = id / kParts % p.tiles;
     head = id / kParts / p.tiles;
-    gate = KIND == kForward ? part >> 1 : 0;
-    j0 = (part & 1) * kTile;
+    gate = part / kSide;
+    j0 = part % kSide * kTile;
     m0 = (int64_t)tile * kTile;
     const int64_t left = p.M - m0;
     rows = (uint32_t)(left < kTile ? left : kTile);
@@ -229,8 +246,8 @@ gates_split_f32_kernel(SplitArgs p) {
   // Two stages of both operands in flight: a stage's floats are requested two
   // stages ahead and cut during the one before it, between its matrix
   // instructions.
-  Share<kAlongKA> sa[2];
-  Share<kAlongKB> sb[2];
+  Share<S, kAlongKA> sa[2];
+  Share<S, kAlongKB> sb[2];
   auto request = [&](uint32_t k, auto SLOT) {
     constexpr int slot = decltype(SLOT)::value;
     constexpr bool checked = KIND == kWeights;
@@ -243,64 +260,71 @@ gates_split_f32_kernel(SplitArgs p) {
     sa[slot].template request<checked>(qa, k, tid);
     sb[slot].template request<checked>(qb, k, tid);
   };
-  // this wave's 64 x 64 results: 2 x 2 blocks
-  const int wr = 64 * (wave >> 1), wc = 64 * (wave & 1);
-  f32x16 big[2][2], small[2][2];
+  // this wave's results
+  const int wr = kTile / 2 * (wave >> 1), wc = kTile / 2 * (wave & 1);
+  f32x16 big[BLOCKS][BLOCKS], small[BLOCKS][BLOCKS];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < BLOCKS; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < BLOCKS; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) big[i][j][r] = small[i][j][r] = 0.0f;
-  const unsigned char* const la =
-      lds + (wr + (lane & 31)) * kRowBytes + 16 * (lane >> 5);
-  const unsigned char* const lb =
-      lds + kOperandBytes + (wc + (lane & 31)) * kRowBytes + 16 * (lane >> 5);
+  // this lane's eight k of its row in the first block, per 16 k of a stage
+  const unsigned char* la[kStage / 16];
+  const unsigned char* lb[kStage / 16];
+#pragma unroll
+  for (int ks = 0; ks < kStage / 16; ++ks) {
+    la[ks] = lds + S::at(wr + (lane & 31), 2 * ks + (lane >> 5));
+    lb[ks] = lds + S::operand + S::at(wc + (lane & 31), 2 * ks + (lane >> 5));
+  }
   // Stage k from buffer SLOT; the next one's floats are cut into the other
   // buffer, and their registers take what is asked for of the stage after the
   // one after it.
   auto stage = [&](uint32_t k, auto SLOT) {
     constexpr int slot = decltype(SLOT)::value;
-    Frag fa[2][3], fb[2][3];
-    auto pieces = [&](int q) {
+    unsigned char* const other = lds + (slot ^ 1) * S::buffer;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        fa[i][q].u = *reinterpret_cast<const u32x4*>(
-            la + slot * kBufferBytes + q * kPieceBytes + 32 * i * kRowBytes);
-        fb[i][q].u = *reinterpret_cast<const u32x4*>(
-            lb + slot * kBufferBytes + q * kPieceBytes + 32 * i * kRowBytes);
-      }
-    };
-    auto multiply = [&](f32x16 (&sum)[2][2], int qa, int qb) {
+    for (int ks = 0; ks < kStage / 16; ++ks) {
+      const bool first = ks == 0, last = ks == kStage / 16 - 1;
+      Frag fa[BLOCKS][3], fb[BLOCKS][3];
+      auto pieces = [&](int q) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < BLOCKS; ++i) {
+          const int at = slot * S::buffer + q * S::piece + 32 * i * S::row;
+          fa[i][q].u = *reinterpret_cast<const u32x4*>(la[ks] + at);
+          fb[i][q].u = *reinterpret_cast<const u32x4*>(lb[ks] + at);
+        }
+      };
+      auto multiply = [&](f32x16 (&sum)[BLOCKS][BLOCKS], int qa, int qb) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              fa[i][qa].v, fb[j][qb].v, sum[i][j], 0, 0, 0);
-    };
-    pieces(0);
-    pieces(1);
-
-    multiply(big, 0, 0);
-    sa[slot ^ 1].store(lds + (slot ^ 1) * kBufferBytes, tid);
-    multiply(small, 0, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    pieces(2);
-    multiply(small, 1, 0);
-    sb[slot ^ 1].store(lds + (slot ^ 1) * kBufferBytes + kOperandBytes, tid);
-    multiply(small, 1, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    request(k + 3 * kStage, std::integral_constant<int, slot ^ 1>{});
-    multiply(small, 0, 2);
-    multiply(small, 2, 0);
-
+        for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+          for (int j = 0; j < BLOCKS; ++j)
+            sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                fa[i][qa].v, fb[j][qb].v, sum[i][j], 0, 0, 0);
+      };
+      pieces(0);
+      pieces(1);
+      multiply(big, 0, 0);
+      if (first) sa[slot ^ 1].store(other, tid);
+      multiply(small, 0, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      pieces(2);
+      multiply(small, 1, 0);
+      if (last) sb[slot ^ 1].store(other + S::operand, tid);
+      multiply(small, 1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (last)
+        request(k + 3 * kStage, std::integral_constant<int, slot ^ 1>{});
+      multiply(small, 0, 2);
+      multiply(small, 2, 0);
+    }
     lds_barrier();
   };
   request(0, std::integral_constant<int, 0>{});
   request(kStage, std::integral_constant<int, 1>{});
   sa[0].store(lds, tid);
-  sb[0].store(lds + kOperandBytes, tid);
+  sb[0].store(lds + S::operand, tid);
   request(2 * kStage, std::integral_constant<int, 0>{});
   lds_barrier();
   for (uint32_t k = 0; k < k_total; k += 2 * kStage) {
@@ -311,9 +335,9 @@ gates_split_f32_kernel(SplitArgs p) {
 
   float odd = 0.0f;  // NaN as soon as one result is not finite
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < BLOCKS; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < BLOCKS; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         big[i][j][r] += small[i][j][r];
@@ -327,9 +351,9 @@ gates_split_f32_kernel(SplitArgs p) {
                                            base, r * s.row + k * s.step, 0, 0));
     };
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < BLOCKS; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < BLOCKS; ++j) {
         f32x16 again;
 #pragma unroll
         for (int r = 0; r < 16; ++r) again[r] = 0.0f;
@@ -358,12 +382,12 @@ gates_split_f32_kernel(SplitArgs p) {
                             kBW) +
         (i0 + wr) * kBW + j0 + wc + (lane & 31);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < BLOCKS; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) dst[row * kBW + 32 * j] = big[i][j][r];
+        for (int j = 0; j < BLOCKS; ++j) dst[row * kBW + 32 * j] = big[i][j][r];
       }
   } else {
     // (rows past the end fall outside the descriptor)
@@ -372,9 +396,13 @@ gates_split_f32_kernel(SplitArgs p) {
     const uint32_t at = (uint32_t)(wr + 4 * (lane >> 5)) * row_bytes +
                         4u * (uint32_t)(head * kBW + j0 + wc + (lane & 31));
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < BLOCKS; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < BLOCKS; ++j) {
+        float bias = 0.0f;
+        if (KIND == kForward && p.bias[0])
+          bias = (gate ? p.bias[1] : p.bias[0])[head * kBW + j0 + wc + 32 * j +
+                                                (lane & 31)];
         float before[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -391,7 +419,8 @@ gates_split_f32_kernel(SplitArgs p) {
           const uint32_t off =
               at + (uint32_t)(32 * i + 8 * (r >> 2) + (r & 3)) * row_bytes +
               128u * j;
-          const float v = KIND == kData ? before[r] + big[i][j][r] : big[i][j][r];
+          const float v =
+              KIND == kData ? before[r] + big[i][j][r] : big[i][j][r] + bias;
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ro, off, 0, 0);
         }
       }
@@ -417,38 +446,63 @@ gates_wgrad_finish_kernel(const f32x4* __restrict__ part, int splits,
 
 int splits_for(int64_t M, int H) {
   // as many row ranges as keep every workgroup resident, two to a CU; at least
-  // four stages each
+  // 128 rows each
   int64_t want = 512 / ((int64_t)8 * H);
-  const int64_t most = (M + 8 * kStage - 1) / (8 * kStage);
+  const int64_t most = (M + 127) / 128;
   if (want > most) want = most;
   return want < 1 ? 1 : (int)want;
 }
 
 int64_t rows_for(int64_t M, int splits) {
   const int64_t rows = (M + splits - 1) / splits;
-  return (rows + 2 * kStage - 1) / (2 * kStage) * (2 * kStage);
+  return (rows + 31) / 32 * 32;  // (two stages)
 }
 
-template <int KIND>
-hipError_t launch(const SplitArgs& a, int64_t blocks, hipStream_t s) {
+template <int KIND, int BLOCKS>
+hipError_t launch(SplitArgs& a, hipStream_t s) {
+  using S = Size<BLOCKS>;
+  const int64_t side = kBW / S::tile;
+  int64_t blocks;
+  if (KIND == kWeights) {
+    blocks = a.H * a.splits * 2 * side * side;
+  } else {
+    a.tiles = (int)((a.M + S::tile - 1) / S::tile);
+    blocks = (int64_t)a.tiles * a.H * side * (KIND == kForward ? 2 : 1);
+  }
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
-  gates_split_f32_kernel<KIND><<<dim3((unsigned)blocks), kThreads, 0, s>>>(a);
+  gates_split_f32_kernel<KIND, BLOCKS>
+      <<<dim3((unsigned)blocks), kThreads, 0, s>>>(a);
   return hipGetLastError();
+}
+
+// Tiles of 64 x 64 while their workgroups, four for one of 128 x 128, are all
+// resident (three to a CU): us, 64 / 128, forward 10 heads 64 rows 8 / 15, 333 rows
+// (480 workgroups) 12 / 17, 512 (640) 14.9 / 17.1, 768 (960) 19.6 / 18.7; 16 heads
+// 333 rows (768) 15 / 17, 1001 (2048) 35 / 28; data 10 heads 768 rows (480) 18 / 26,
+// 1500 (960) 34 / 29.  Same products in the same order: the same bits.
+template <int KIND>
+hipError_t launch_rows(SplitArgs& a, hipStream_t s) {
+  const int64_t small =
+      (a.M + 63) / 64 * a.H * (KIND == kForward ? 8 : 4);
+  if (small <= 768) return launch<KIND, 1>(a, s);
+  return launch<KIND, 2>(a, s);
 }
 
 }  // namespace
 
 bool gates_f32_serves(int64_t M, int W, int H) {
   // (128 rows of an operand are 32-bit offsets)
-  return M > 0 && H > 0 && H <= 32768 / 8 && W == H * kBW &&
-         (M + kTile - 1) / kTile * H * 4 <= 0x7fffffff;
+  return M > 0 && H > 0 && H <= 4096 && W == H * kBW &&
+         (M + 63) / 64 * H * 8 <= 0x7fffffff;
 }
 
 hipError_t launch_gates_f32(const void* x, const void* w_x, const void* w_a,
-                            void* gx, void* ga, int64_t M, int W, int H,
-                            hipStream_t s) {
+                            const void* b_x, const void* b_a, void* gx, void* ga,
+                            int64_t M, int W, int H, hipStream_t s) {
   if (!gates_f32_serves(M, W, H)) return hipErrorInvalidValue;
   SplitArgs a{};
+  a.bias[0] = (const float*)b_x;
+  a.bias[1] = (const float*)b_a;
   a.x = (const float*)x;
   a.w[0] = (const float*)w_x;
   a.w[1] = (const float*)w_a;
@@ -457,8 +511,7 @@ hipError_t launch_gates_f32(const void* x, const void* w_x, const void* w_a,
   a.M = M;
   a.W = W;
   a.H = H;
-  a.tiles = (int)((M + kTile - 1) / kTile);
-  return launch<kForward>(a, (int64_t)a.tiles * H * 4, s);
+  return launch_rows<kForward>(a, s);
 }
 
 hipError_t launch_gates_dgrad_f32(const void* dgx, const void* dga,
@@ -474,14 +527,13 @@ hipError_t launch_gates_dgrad_f32(const void* dgx, const void* dga,
   a.M = M;
   a.W = W;
   a.H = H;
-  a.tiles = (int)((M + kTile - 1) / kTile);
-  return launch<kData>(a, (int64_t)a.tiles * H * 2, s);
+  return launch_rows<kData>(a, s);
 }
 
 bool gates_wgrad_f32_serves(int64_t M, int W, int H) {
   if (M <= 0 || H <= 0 || W != H * kBW || H > 4096) return false;
   // offsets within a row range, a stage past its end, are 32 bits
-  return (uint64_t)(rows_for(M, splits_for(M, H)) + 4 * kStage) * (uint64_t)W *
+  return (uint64_t)(rows_for(M, splits_for(M, H)) + 64) * (uint64_t)W *
              4u < 0xffffffffull;
 }
 
@@ -507,7 +559,7 @@ hipError_t launch_gates_wgrad_f32(const void* x, const void* dgx,
   a.H = H;
   a.splits = splits_for(M, H);
   a.rows_per_split = (int)rows_for(M, a.splits);
-  hipError_t e = launch<kWeights>(a, (int64_t)H * a.splits * 8, s);
+  hipError_t e = launch<kWeights, 2>(a, s);
   if (e != hipSuccess || a.splits == 1) return e;
   const int64_t items = (int64_t)H * kBW * kBW / 4;
   gates_wgrad_finish_kernel<<<dim3((unsigned)((2 * items + 255) / 256)), 256, 0,

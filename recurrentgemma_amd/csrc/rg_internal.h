@@ -274,7 +274,8 @@ hipError_t launch_rglru_backward(const RglruBwdArgs& a, int dtype,
 // One pass over every element, 16 bytes of channels per lane
 // (rg_scan_tiles.hip).
 struct ScanTileArgs {
-  // forward: x, a | gated: x, input gate, recurrence gate (pre-activations)
+  // forward: x, a | gated: x, input gate, recurrence gate (pre-activations),
+  // float32: the other branch or null
   // backward: dy, a, y | gated: dy, x, input gate, recurrence gate, y
   const void* in[5];
   const void* flags;     // [B, T] document starts
@@ -298,7 +299,8 @@ struct ScanTileArgs {
 enum ScanTileMode { kTilesFwdPlain, kTilesBwdPlain, kTilesFwdGated, kTilesBwdGated,
                     // (a question only) both gated ones of a float32 RG-LRU
                     kTilesPairGated };
-// whether it takes the shape and is the faster form for it
+// whether it takes the shape; ... and is the faster form for it
+bool scan_tiles_take(int T, int W, int dtype);
 bool scan_tiles_serve(int B, int T, int W, int dtype, int mode);
 // whether rg_scan_bwd.hip's kernels give a lane two channels (else one)
 bool scan_backward_two_channels(int B, int W);
@@ -398,13 +400,13 @@ struct SumTask {
 constexpr int kMaxSumTasks = 8;
 hipError_t launch_sum_rows(const SumTask* tasks, int count, int dtype,
                            hipStream_t s);
-// rg_gates_split_f32.hip: both gate projections in float32 (256-wide heads, without
-// the biases); what they give back to x, added to dx; the gradients of their
+// rg_gates_split_f32.hip: both gate projections in float32 (256-wide heads; biases:
+// both or neither); what they give back to x, added to dx; the gradients of their
 // weights (workspace may be null where that needs no bytes).
 bool gates_f32_serves(int64_t M, int W, int H);
 hipError_t launch_gates_f32(const void* x, const void* w_x, const void* w_a,
-                            void* gx, void* ga, int64_t M, int W, int H,
-                            hipStream_t s);
+                            const void* b_x, const void* b_a, void* gx, void* ga,
+                            int64_t M, int W, int H, hipStream_t s);
 hipError_t launch_gates_dgrad_f32(const void* dgx, const void* dga,
                                   const void* w_x, const void* w_a, void* dx,
                                   int64_t M, int W, int H, hipStream_t s);

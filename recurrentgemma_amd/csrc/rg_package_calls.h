@@ -42,6 +42,11 @@ size_t rg_argmax_workspace_bytes(int rows, int n);
 int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
                          int n, int dtype, void* stream);
 
+/* The workspace with which rg_recurrent_core is fastest: what it needs or, for
+ * shapes that one launch without a workspace serves, what its other form takes. */
+size_t rg_recurrent_core_best_workspace_bytes(int B, int T, int W, int H,
+                                              int dtype);
+
 #ifdef __cplusplus
 }
 #endif

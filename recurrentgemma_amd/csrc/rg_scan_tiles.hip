@@ -116,8 +116,11 @@ struct TileLds {
   float bias[2][channels];                // float32: of the gate projections
 };
 
-template <typename T, int MODE, int KL>
+// JOIN (gated forward, float32): y leaves as y * gelu(in[3]), the join of the
+// recurrent block's two branches (recurrentgemma/torch/modules.py:627-628, 644).
+template <typename T, int MODE, int KL, bool JOIN = false>
 __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
+  static_assert(!JOIN || (MODE == kFwdGated && sizeof(T) == 4), "");
   using V = Vec<T>;
   using Lds = TileLds<T>;
   constexpr int N = V::n;
@@ -394,6 +397,17 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
     }
     lds_barrier();
 
+    u32x4 branch[JOIN ? KL : 1];
+    if constexpr (JOIN) {
+      const __amdgpu_buffer_rsrc_t rg = make_rsrc(
+          (const char*)p.in[3] + (int64_t)b * seq_bytes, seq_bytes);
+#pragma unroll
+      for (int i = 0; i < KL; ++i)
+        branch[i] = __builtin_amdgcn_raw_buffer_load_b128(
+            rg, c_ok ? c_off + (uint32_t)(t0 + i) * row_bytes : kBufferOutOfRange,
+            0, 0);
+    }
+
     // ---- 2: scan over the groups ---------------------------------------------
     {
       f32x2 v[kPer];
@@ -477,7 +491,9 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
                          : __builtin_fmaf(cf[e], st[e], in0[e]);
         float y[N];
 #pragma unroll
-        for (int e = 0; e < N; ++e) y[e] = st[e];
+        for (int e = 0; e < N; ++e)
+          y[e] = JOIN ? gelu_mul_f32(st[e], __uint_as_float(branch[JOIN ? i : 0][e & 3]))
+                      : st[e];
         store(0, V::pack(y));
         if (!more && p.last && t == T_len - 1 && c_ok) {
 #pragma unroll
@@ -591,17 +607,19 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
   }
 }
 
-template <typename T, int MODE, int KL>
+template <typename T, int MODE, int KL, bool JOIN = false>
 hipError_t launch_as(const ScanTileArgs& a, hipStream_t s) {
   constexpr int lds = sizeof(TileLds<T>);
   static OncePerDevice once;
   hipError_t e =
-      set_max_dynamic_lds(once, (const void*)scan_tiles_kernel<T, MODE, KL>, lds);
+      set_max_dynamic_lds(once, (const void*)scan_tiles_kernel<T, MODE, KL, JOIN>,
+                          lds);
   if (e != hipSuccess) return e;
   const int64_t blocks =
       (int64_t)a.B * ((a.W + TileLds<T>::channels - 1) / TileLds<T>::channels);
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
-  scan_tiles_kernel<T, MODE, KL><<<dim3((unsigned)blocks), kThreads, lds, s>>>(a);
+  scan_tiles_kernel<T, MODE, KL, JOIN>
+      <<<dim3((unsigned)blocks), kThreads, lds, s>>>(a);
   return hipGetLastError();
 }
 
@@ -630,11 +648,15 @@ static bool gated_backward_pays(int B, int T, int W, int dtype, int64_t blocks) 
   return here < there || T > (blocks <= 1024 ? 2048 : 512);
 }
 
+bool scan_tiles_take(int T, int W, int dtype) {
+  const int64_t es = dtype == 0 ? 4 : 2;
+  return (int64_t)W * es % 16 == 0 &&
+         ((int64_t)T + 1024) * W * es < (int64_t)0x7fffffff;
+}
+
 bool scan_tiles_serve(int B, int T, int W, int dtype, int mode) {
   const int64_t es = dtype == 0 ? 4 : 2;
-  if ((int64_t)W * es % 16 != 0 ||
-      ((int64_t)T + 1024) * W * es >= (int64_t)0x7fffffff)
-    return false;
+  if (!scan_tiles_take(T, W, dtype)) return false;
   // The eight waves of a workgroup walk a slab of channels in steps of 256
   // or 512 tokens, one workgroup per CU: a launch costs a round of the chip per
   // 256 slabs and at least one step, where rg_scan.hip's and rg_scan_bwd.hip's
@@ -687,7 +709,9 @@ hipError_t launch_scan_tiles(const ScanTileArgs& a, int mode, int dtype,
     switch (mode) {
       case kFwdPlain: return launch_as<float, kFwdPlain, 8>(a, s);
       case kBwdPlain: return launch_as<float, kBwdPlain, 4>(a, s);
-      case kFwdGated: return launch_as<float, kFwdGated, 4>(a, s);
+      case kFwdGated:
+        return a.in[3] ? launch_as<float, kFwdGated, 4, true>(a, s)
+                       : launch_as<float, kFwdGated, 4>(a, s);
       default: return launch_as<float, kBwdGated, 4>(a, s);
     }
   }

@@ -242,8 +242,9 @@ void gated_forward(const Tensor& x, const Tensor& pos, const GateWeights& g,
   }
   if (f32) {
     if (rg::gates_f32_serves(d.M(), (int)d.W, (int)H)) {
-      check_hip(rg::launch_gates_f32(in(x), in(g.w_x), in(g.w_a), out(gx), out(ga),
-                                     d.M(), (int)d.W, (int)H, d.stream));
+      check_hip(rg::launch_gates_f32(in(x), in(g.w_x), in(g.w_a), nullptr, nullptr,
+                                     out(gx), out(ga), d.M(), (int)d.W, (int)H,
+                                     d.stream));
     } else {
       // the library's batched products, on strided views: no permuted copies
       Tensor xs = by_head(x, H), gxs = by_head(gx, H), gas = by_head(ga, H);

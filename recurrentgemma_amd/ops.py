@@ -443,7 +443,7 @@ def recurrent_core(x, segment_pos, conv_w, conv_b, w_x, b_x, w_a, b_a, a_param,
             if x.dtype == torch.bfloat16 else None)
   lib = _lib.lib()
   code = _dtype_code(x)
-  need = lib.rg_recurrent_core_workspace_bytes(B, T, W, H, code)
+  need = lib.rg_recurrent_core_best_workspace_bytes(B, T, W, H, code)
   ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
   with _on(x.device):
     _lib.check(lib.rg_recurrent_core(
