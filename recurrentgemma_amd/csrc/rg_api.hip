@@ -593,10 +593,7 @@ struct CorePlan {
   bool single;         // block_prefill_bf16_kernel
   size_t split_bytes;  // chunk summaries of whichever form runs
   size_t gate_bytes;   // one gate's pre-activations (two-kernel form), padded
-  size_t wide_bytes;   // what the wide_f32 form needs where it takes the shape
-  size_t need() const {
-    return small_f32 ? 0 : wide_f32 ? wide_bytes : split_bytes + 2 * gate_bytes;
-  }
+  size_t need() const { return small_f32 ? 0 : split_bytes + 2 * gate_bytes; }
 };
 // The float32 form of several launches (conv, gate projections on bf16 pieces,
 // recurrence) for 256-wide heads: which recurrence kernel, and where it is ahead.
@@ -630,13 +627,15 @@ static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
   // float32 with few rows: one launch, no workspace; or, with one, the form of
   // several launches where that is ahead
   p.small_f32 = dtype == RG_DTYPE_F32 && rg::core_f32_small_serves(B, T, W, H);
-  if (dtype == RG_DTYPE_F32 && rg::gates_f32_serves((int64_t)B * T, W, H) &&
-      rg::scan_tiles_take(T, W, dtype) && wide_f32_pays(B, T, W, H, p.small_f32)) {
+  p.wide_f32 = dtype == RG_DTYPE_F32 &&
+               rg::gates_f32_serves((int64_t)B * T, W, H) &&
+               rg::scan_tiles_take(T, W, dtype) &&
+               wide_f32_pays(B, T, W, H, p.small_f32);
+  if (p.small_f32) {
     const size_t n = (size_t)B * T * W * sizeof(float);
-    p.wide_bytes = 3 * ((n + 255) & ~(size_t)255);
-    p.wide_f32 = !p.small_f32;
+    if (p.wide_f32) p.gate_bytes = (n + 255) & ~(size_t)255;
+    return p;
   }
-  if (p.small_f32 || p.wide_f32) return p;
   const bool fits = dtype == RG_DTYPE_BF16 && single_takes(W / H) &&
                     (int64_t)T * W * 2 < (int64_t)0x7fffffff;
   const size_t chunk_bytes =
@@ -681,7 +680,7 @@ size_t rg_recurrent_core_best_workspace_bytes(int B, int T, int W, int H,
       (dtype != RG_DTYPE_F32 && dtype != RG_DTYPE_BF16))
     return 0;
   const CorePlan p = core_plan(B, T, W, H, dtype);
-  return p.wide_bytes ? p.wide_bytes : p.need();
+  return p.split_bytes + 2 * p.gate_bytes;
 }
 
 int rg_recurrent_core(const void* x, const void* gate_branch,
@@ -705,18 +704,19 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
   RG_REQUIRE(conv_w != nullptr || conv_cache_out == nullptr,
              "%s: no conv state without a conv", __func__);
   const int conv = conv_w != nullptr;
-  CorePlan p = core_plan(B, T, W, H, dtype);
+  const CorePlan p = core_plan(B, T, W, H, dtype);
   const size_t need = p.need();
   if (need > 0 && (workspace == nullptr || workspace_bytes < need ||
                    !aligned16(workspace)))
     return fail(RG_ERR_WORKSPACE,
                 "%s: workspace of %zu bytes (16-byte aligned) required, got %zu",
                 __func__, need, workspace ? workspace_bytes : (size_t)0);
-  // the one-launch form where the caller has brought no more than it needs
-  if (p.small_f32 && p.wide_bytes && workspace != nullptr &&
-      workspace_bytes >= p.wide_bytes && aligned16(workspace))
-    p.wide_f32 = true;
-  if (p.small_f32 || p.wide_f32) {
+  // (the form of several launches keeps the conv output where y goes, and the
+  // pre-activations in a workspace that the one-launch form does not ask for)
+  const bool wide = p.wide_f32 && gate_branch != out && workspace != nullptr &&
+                    workspace_bytes >= p.split_bytes + 2 * p.gate_bytes &&
+                    aligned16(workspace);
+  if (p.small_f32 || wide) {
     RG_CHECK_PTR(x);
     RG_CHECK_PTR(segpos);
     RG_CHECK_OPT_PTR(conv_w);
@@ -731,30 +731,26 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
     RG_CHECK_OPT_PTR(h_last);
     RG_CHECK_OPT_PTR(conv_cache_out);
     RG_REQUIRE(out != x, "%s: out must not alias x", __func__);
-    if (p.wide_f32) {
-      char* const ws = (char*)workspace;
-      const size_t plane = p.wide_bytes / 3;
-      void* const gx = ws;
-      void* const ga = ws + plane;
-      const void* xc = x;
-      if (conv) {
-        xc = ws + 2 * plane;
-        const int rc = rg_conv1d_prefill(x, segpos, segpos_is_i64, conv_w, conv_b,
-                                         ws + 2 * plane, conv_cache_out, B, T, W, 4,
-                                         dtype, stream);
-        if (rc != RG_OK) return rc;
-      }
-      // (the one-pass kernel adds the biases itself, and reads the other branch
-      // where it writes)
-      const bool tiles = wide_scan_on_tiles(B, T, W) || gate_branch == out;
-      int rc = launch_status(
+    if (wide) {
+      void* const gx = (char*)workspace + p.split_bytes;
+      void* const ga = (char*)workspace + p.split_bytes + p.gate_bytes;
+      int rc = RG_OK;
+      if (conv)
+        rc = rg_conv1d_prefill(x, segpos, segpos_is_i64, conv_w, conv_b, out,
+                               conv_cache_out, B, T, W, 4, dtype, stream);
+      if (rc != RG_OK) return rc;
+      const void* const xc = conv ? out : x;
+      // (the one-pass kernel adds the biases itself)
+      const bool tiles = wide_scan_on_tiles(B, T, W);
+      rc = launch_status(
           __func__, rg::launch_gates_f32(xc, w_x, w_a, tiles ? nullptr : b_x,
                                          tiles ? nullptr : b_a, gx, ga,
                                          (int64_t)B * T, W, H,
                                          (hipStream_t)stream));
       if (rc != RG_OK) return rc;
       if (!tiles) {
-        rc = rg_lru_scan_fused(xc, 0, nullptr, nullptr, gx, ga, a_param, segpos,
+        // (from x: this kernel has a conv of its own and takes no y over x)
+        rc = rg_lru_scan_fused(x, conv, conv_w, conv_b, gx, ga, a_param, segpos,
                                segpos_is_i64, h0, out, h_last, nullptr, B, T, W,
                                dtype, stream);
         if (rc != RG_OK || gate_branch == nullptr) return rc;
@@ -762,6 +758,8 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
             __func__, rg::launch_gelu_mul(out, gate_branch, out, (int64_t)B * T * W,
                                           dtype, (hipStream_t)stream));
       }
+      // (over xc in place: every element is read, steps ahead, by the lane that
+      // writes it)
       rg::ScanTileArgs t{};
       t.in[0] = xc;
       t.in[1] = gx;
