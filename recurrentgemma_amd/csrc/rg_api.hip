@@ -739,6 +739,8 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
         rc = rg_conv1d_prefill(x, segpos, segpos_is_i64, conv_w, conv_b, out,
                                conv_cache_out, B, T, W, 4, dtype, stream);
       if (rc != RG_OK) return rc;
+      // (the recurrence runs over it in place: either kernel reads an element, a
+      // step or more ahead, in the lane that writes it)
       const void* const xc = conv ? out : x;
       // (the one-pass kernel adds the biases itself)
       const bool tiles = wide_scan_on_tiles(B, T, W);
@@ -749,17 +751,26 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
                                          (hipStream_t)stream));
       if (rc != RG_OK) return rc;
       if (!tiles) {
-        // (from x: this kernel has a conv of its own and takes no y over x)
-        rc = rg_lru_scan_fused(x, conv, conv_w, conv_b, gx, ga, a_param, segpos,
-                               segpos_is_i64, h0, out, h_last, nullptr, B, T, W,
-                               dtype, stream);
+        rg::ScanArgs s{};
+        s.x = xc;
+        s.gx = gx;
+        s.ga = ga;
+        s.a_param = a_param;
+        s.segpos = segpos;
+        s.seg_kind = segpos_is_i64 ? 1 : 0;
+        s.h0 = (const float*)h0;
+        s.y = out;
+        s.h_last = (float*)h_last;
+        s.B = B;
+        s.T = T;
+        s.W = W;
+        rc = launch_status(__func__,
+                           rg::launch_lru_scan(s, dtype, (hipStream_t)stream));
         if (rc != RG_OK || gate_branch == nullptr) return rc;
         return launch_status(
             __func__, rg::launch_gelu_mul(out, gate_branch, out, (int64_t)B * T * W,
                                           dtype, (hipStream_t)stream));
       }
-      // (over xc in place: every element is read, steps ahead, by the lane that
-      // writes it)
       rg::ScanTileArgs t{};
       t.in[0] = xc;
       t.in[1] = gx;
