@@ -342,6 +342,154 @@ PyObject* rows_partial(PyObject*, PyObject* const* v, Py_ssize_t n) {
   });
 }
 
+// ------------------------------------------------------ the block's step --
+
+// A parameter of an nn.Module, past the attribute lookup that is written in
+// Python; anything but a module that holds it itself takes the general path.
+const Tensor& parameter(PyObject* module, PyObject* name) {
+  static PyObject* const key = PyUnicode_InternFromString("_parameters");
+  PyObject* own = PyObject_GetAttr(module, key);
+  if (!own) {
+    PyErr_Clear();
+    throw Fallback{};
+  }
+  Py_DECREF(own);  // (the module keeps it)
+  need(PyDict_CheckExact(own));
+  PyObject* t = PyDict_GetItemWithError(own, name);
+  if (!t) PyErr_Clear();
+  need(t != nullptr);
+  return tensor_of(t);
+}
+PyObject* child(PyObject* modules, PyObject* name) {
+  need(PyDict_CheckExact(modules));
+  PyObject* m = PyDict_GetItemWithError(modules, name);
+  if (!m) PyErr_Clear();
+  need(m != nullptr);
+  return m;
+}
+PyObject* children(PyObject* module) {
+  static PyObject* const key = PyUnicode_InternFromString("_modules");
+  PyObject* own = PyObject_GetAttr(module, key);
+  if (!own) {
+    PyErr_Clear();
+    throw Fallback{};
+  }
+  Py_DECREF(own);
+  return own;
+}
+const RowsPlan& plan_for(PyObject* capsule,
+                         std::initializer_list<const Tensor*> sources) {
+  need(PyCapsule_IsValid(capsule, kPlanName));
+  const auto& p =
+      *static_cast<RowsPlan*>(PyCapsule_GetPointer(capsule, kPlanName));
+  need(p.sources.size() == sources.size());
+  size_t at = 0;
+  for (const Tensor* t : sources) need(p.sources[at++].matches(*t));
+  return p;
+}
+
+// A cached single-token call of RecurrentBlock (at most 64 rows, bf16, 256-wide
+// heads): its linear layers on the few-row kernels and the step between them,
+// the join written over the gate branch.  As three calls from Python it was 25 us
+// of host time around 17 us of kernels.
+// (the block's _modules, plan of linear_y and linear_x, plan of linear_out, x,
+//  segment_pos, conv_state, h, in_place) -> (out, h, conv_state) | None
+PyObject* block_step(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 8);
+#define RG_NAME(ID, TEXT) \
+  static PyObject* const ID = PyUnicode_InternFromString(TEXT);
+    RG_NAME(k_y, "linear_y") RG_NAME(k_x, "linear_x") RG_NAME(k_out, "linear_out")
+    RG_NAME(k_conv, "conv_1d") RG_NAME(k_lru, "rg_lru")
+    RG_NAME(k_gx, "input_gate") RG_NAME(k_ga, "a_gate") RG_NAME(k_w, "w")
+    RG_NAME(k_b, "b") RG_NAME(k_weight, "weight") RG_NAME(k_bias, "bias")
+    RG_NAME(k_param, "a_param")
+#undef RG_NAME
+    PyObject *m_y = child(v[0], k_y), *m_x = child(v[0], k_x),
+             *m_out = child(v[0], k_out), *m_conv = child(v[0], k_conv),
+             *m_lru = child(v[0], k_lru);
+    PyObject* gates = children(m_lru);
+    PyObject *m_gx = child(gates, k_gx), *m_ga = child(gates, k_ga);
+    const RowsPlan& in_plan =
+        plan_for(v[1], {&parameter(m_y, k_weight), &parameter(m_x, k_weight),
+                        &parameter(m_y, k_bias), &parameter(m_x, k_bias)});
+    const RowsPlan& out_plan = plan_for(
+        v[2], {&parameter(m_out, k_weight), &parameter(m_out, k_bias)});
+    Call c(v[3]);
+    need(c.code == RG_DTYPE_BF16 && c.x.dim() == 3 && c.x.size(1) == 1);
+    const int64_t B = c.x.size(0), D = c.x.size(2), W = out_plan.K;
+    need(B > 0 && B <= 64 && in_plan.K == D && in_plan.groups == 2 &&
+         in_plan.N == 2 * W && !in_plan.gelu_pair && in_plan.bias.defined() &&
+         out_plan.groups == 1 && !out_plan.gelu_pair && out_plan.bias.defined() &&
+         in_plan.packed.device() == c.x.device() &&
+         out_plan.packed.device() == c.x.device());
+    auto shaped = [&](const Tensor& t, std::initializer_list<int64_t> want) {
+      need(shape_is(t, want));
+      return dense(t, c.dtype, c.device);
+    };
+    const Tensor &w_x = parameter(m_gx, k_w), &w_a = parameter(m_ga, k_w);
+    need(w_x.dim() == 3);
+    const int64_t H = w_x.size(0), bw = 256;
+    need(H > 0 && W == H * bw);
+    shaped(w_x, {H, bw, bw});
+    shaped(w_a, {H, bw, bw});
+    void* x = c(v[3]);
+    int is64;
+    void* pos = c.positions(v[4], B, 1, &is64);
+    void* conv_in = c.shaped(v[5], {B, 3, W});
+    void* h_in = c.f32(v[6], {B, W});
+    void* conv_w = shaped(parameter(m_conv, k_w), {4, W});
+    void* conv_b = shaped(parameter(m_conv, k_b), {W});
+    void* b_x = shaped(parameter(m_gx, k_b), {H, bw});
+    void* b_a = shaped(parameter(m_ga, k_b), {H, bw});
+    void* a_param = shaped(parameter(m_lru, k_param), {W});
+    const Tensor packed = packed_for(w_x, w_a);
+    need(packed.device() == c.x.device());
+    const int N = out_plan.N;
+    Tensor yx = c.empty({2, B, W}), out = c.empty({B, 1, N}), ws, h, conv;
+    if (v[7] == Py_True) {
+      h = THPVariable_Unpack(v[6]);
+      conv = THPVariable_Unpack(v[5]);
+    } else {
+      h = c.empty({B, W}, at::kFloat);
+      conv = c.empty({B, 3, W});
+    }
+    const size_t in_bytes =
+        rg_linear_rows_workspace_bytes((int)B, (int)D, (int)(2 * W));
+    const size_t out_bytes = rg_linear_rows_workspace_bytes((int)B, (int)W, N);
+    const size_t bytes = in_bytes > out_bytes ? in_bytes : out_bytes;
+    if (bytes) ws = c.empty({(int64_t)bytes}, at::kByte);
+    void* wp = bytes ? ws.mutable_data_ptr() : nullptr;
+    char* const y = (char*)yx.mutable_data_ptr();  // the gate branch, then the join
+    void* const lx = y + 2 * B * W;
+    void *op = out.mutable_data_ptr(), *hp = h.mutable_data_ptr(),
+         *cp = conv.mutable_data_ptr();
+    const void *in_w = in_plan.packed.const_data_ptr(),
+               *in_b = in_plan.bias.const_data_ptr(),
+               *out_w = out_plan.packed.const_data_ptr(),
+               *out_b = out_plan.bias.const_data_ptr(),
+               *gates_w = packed.const_data_ptr();
+    // (the plans' tensors, which another thread may replace while this one has
+    // let go of the interpreter)
+    const Tensor keep[] = {in_plan.packed, in_plan.bias, out_plan.packed,
+                           out_plan.bias};
+    void* s = c.stream();
+    launch([&] {
+      int rc = rg_linear_rows(x, in_w, in_b, nullptr, y, wp, bytes, (int)B, (int)D,
+                              (int)(2 * W), 2, 0, s);
+      if (rc != RG_OK) return rc;
+      rc = rg_recurrent_step_gelu_mul(lx, y, pos, is64, conv_in, cp,
+                                      (const float*)h_in, (float*)hp, conv_w,
+                                      conv_b, gates_w, b_x, b_a, a_param, y,
+                                      (int)B, (int)W, (int)H, c.code, s);
+      if (rc != RG_OK) return rc;
+      return rg_linear_rows(y, out_w, out_b, nullptr, op, wp, bytes, (int)B,
+                            (int)W, N, 1, 0, s);
+    });
+    return triple(out, h, conv);
+  });
+}
+
 PyObject* set_kernel_error(PyObject*, PyObject* type) {
   Py_INCREF(type);
   Py_XDECREF(g_kernel_error);
@@ -352,6 +500,7 @@ PyObject* set_kernel_error(PyObject*, PyObject* type) {
 PyMethodDef kMethods[] = {
     {"recurrent_step", (PyCFunction)(void*)recurrent_step, METH_FASTCALL, ""},
     {"recurrent_core", (PyCFunction)(void*)recurrent_core, METH_FASTCALL, ""},
+    {"block_step", (PyCFunction)(void*)block_step, METH_FASTCALL, ""},
     {"rows_plan", (PyCFunction)(void*)rows_plan, METH_FASTCALL, ""},
     {"rows_linear", (PyCFunction)(void*)rows_linear, METH_FASTCALL, ""},
     {"rows_partial", (PyCFunction)(void*)rows_partial, METH_FASTCALL, ""},

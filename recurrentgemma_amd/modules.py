@@ -205,6 +205,11 @@ class RecurrentBlock(nn.Module):
     it gets where that saves a pass (a few rows, bf16)."""
     if training.is_enabled():
       return self._forward_differentiable(x, segment_pos, cache, return_cache)
+    if cache is not None and return_cache and not defer_out:
+      done = self._step_natively(x, segment_pos, cache)
+      if done is not None:
+        y, h, conv_state = done
+        return y, RecurrentBlockCache(rg_lru_state=h, conv1d_state=conv_state)
     with torch.no_grad():
       # (a traced program keeps torch's own linear layers: the few-row
       # kernels are reached through ctypes, which a tracer cannot follow)
@@ -237,6 +242,18 @@ class RecurrentBlock(nn.Module):
     if not return_cache:
       return x, None
     return x, new_cache
+
+  def _step_natively(self, x, segment_pos, cache):
+    """A cached single-token call as one native call (csrc/host_ops.cpp), or
+    None: before the linear layers are packed, and where the arguments are not
+    as that call takes them."""
+    yx, out = self._rows_yx._plan, self._rows_out._plan
+    if (yx is None or out is None or compiled.tracing() or
+        self.conv_1d.temporal_width != 4):
+      return None
+    return _lib.host().block_step(
+        self._modules, yx, out, x, segment_pos, cache.conv1d_state,
+        cache.rg_lru_state, self.decode_in_place)
 
   def _forward_differentiable(self, x, segment_pos, cache, return_cache):
     """The reference's op sequence (modules.py:605-655) under autograd."""
