@@ -447,7 +447,8 @@ size_t rg_recurrent_prefill_split_workspace_bytes(int B, int T, int W, int H) {
 
 #undef RG_WHO
 #define RG_WHO who
-static int recurrent_prefill_impl(const char* who, bool narrow, const void* x,
+static int recurrent_prefill_impl(const char* who, bool narrow, bool relay,
+                                  const void* x,
                                   const void* segpos, int segpos_is_i64,
                                   const void* conv_w, const void* conv_b,
                                   const void* w_x, const void* b_x,
@@ -519,6 +520,9 @@ static int recurrent_prefill_impl(const char* who, bool narrow, const void* x,
   a.H = H;
   a.chunks = 1;
   a.tiles_per_chunk = (T + 63) / 64;
+  if (relay)  // (rg_recurrent_core has seen to the workspace)
+    return launch_status(who, rg::launch_block_prefill_relay_bf16(
+                                  a, workspace, (hipStream_t)stream));
   if (split) {
     const size_t need = rg_recurrent_prefill_split_workspace_bytes(B, T, W, H);
     if (need > 0) {
@@ -546,7 +550,7 @@ int rg_recurrent_prefill(const void* x, const void* segpos, int segpos_is_i64,
                          const void* a_param, const void* h0, void* y,
                          void* h_last, void* conv_cache_out, int B, int T,
                          int W, int H, int dtype, void* stream) {
-  return recurrent_prefill_impl(__func__, false, x, segpos, segpos_is_i64, conv_w,
+  return recurrent_prefill_impl(__func__, false, false, x, segpos, segpos_is_i64, conv_w,
                                 conv_b, w_x, b_x, w_a, b_a, w_packed, a_param,
                                 h0, nullptr, y, h_last, conv_cache_out,
                                 nullptr, 0, false, B, T, W, H, dtype, stream);
@@ -561,7 +565,7 @@ int rg_recurrent_prefill_split(const void* x, const void* segpos,
                                void* h_last, void* conv_cache_out,
                                void* workspace, size_t workspace_bytes, int B,
                                int T, int W, int H, int dtype, void* stream) {
-  return recurrent_prefill_impl(__func__, false, x, segpos, segpos_is_i64, conv_w,
+  return recurrent_prefill_impl(__func__, false, false, x, segpos, segpos_is_i64, conv_w,
                                 conv_b, w_x, b_x, w_a, b_a, w_packed, a_param,
                                 h0, nullptr, y, h_last, conv_cache_out,
                                 workspace, workspace_bytes, true, B, T, W, H,
@@ -577,7 +581,7 @@ int rg_recurrent_prefill_gelu_mul(
     int W, int H, int dtype, void* stream) {
   RG_CHECK_PTR(gate_branch);
   RG_REQUIRE(gate_branch != x, "%s: gate_branch must not alias x", __func__);
-  return recurrent_prefill_impl(__func__, false, x, segpos, segpos_is_i64, conv_w,
+  return recurrent_prefill_impl(__func__, false, false, x, segpos, segpos_is_i64, conv_w,
                                 conv_b, w_x, b_x, w_a, b_a, w_packed, a_param,
                                 h0, gate_branch, out, h_last, conv_cache_out,
                                 workspace, workspace_bytes, true, B, T, W, H,
@@ -591,6 +595,9 @@ struct CorePlan {
   bool small_f32;      // core_f32_small_kernel: everything in one launch
   bool wide_f32;       // conv, gate projections on bf16 pieces, one-pass scan
   bool single;         // block_prefill_bf16_kernel
+  // or, for re-laid-out weights and with as large a workspace, by the blocks of
+  // rg_prefill_relay.hip (without and with the join; 0: not)
+  size_t relay_bytes[2];
   size_t split_bytes;  // chunk summaries of whichever form runs
   size_t gate_bytes;   // one gate's pre-activations (two-kernel form), padded
   size_t need() const { return small_f32 ? 0 : split_bytes + 2 * gate_bytes; }
@@ -656,6 +663,10 @@ static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
              (W / H == 256 || rg::prefill_narrow_pays(B, H, T, W));
   if (p.single) {
     p.split_bytes = chunk_bytes;
+    if (W / H == 256)
+      for (int joined = 0; joined < 2; ++joined)
+        if (rg::prefill_relay_pays(B, H, T, joined))
+          p.relay_bytes[joined] = rg::prefill_relay_workspace_bytes(B, W, H);
   } else {
     // (rounded up: the gate planes behind it must stay 16-byte aligned)
     p.split_bytes =
@@ -680,7 +691,10 @@ size_t rg_recurrent_core_best_workspace_bytes(int B, int T, int W, int H,
       (dtype != RG_DTYPE_F32 && dtype != RG_DTYPE_BF16))
     return 0;
   const CorePlan p = core_plan(B, T, W, H, dtype);
-  return p.split_bytes + 2 * p.gate_bytes;
+  size_t n = p.split_bytes + 2 * p.gate_bytes;
+  for (size_t relay : p.relay_bytes)
+    if (n < relay) n = relay;
+  return n;
 }
 
 int rg_recurrent_core(const void* x, const void* gate_branch,
@@ -816,9 +830,13 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
   } else if (p.single) {
     // the join is part of the kernel's output stage, for rows in chunks too
     // (the launches that write y apply it)
+    const size_t relay_bytes = p.relay_bytes[gate_branch != nullptr];
+    const bool relay = relay_bytes > 0 && w_packed != nullptr &&
+                       workspace != nullptr && workspace_bytes >= relay_bytes &&
+                       aligned16(workspace);
     return recurrent_prefill_impl(
-        __func__, true, x, segpos, segpos_is_i64, conv_w, conv_b, w_x, b_x, w_a, b_a,
-        w_packed, a_param, h0, gate_branch, out, h_last, conv_cache_out,
+        __func__, true, relay, x, segpos, segpos_is_i64, conv_w, conv_b, w_x, b_x,
+        w_a, b_a, w_packed, a_param, h0, gate_branch, out, h_last, conv_cache_out,
         workspace, workspace_bytes, true, B, T, W, H, dtype, stream);
   } else {
     char* const ws = (char*)workspace;

@@ -120,6 +120,9 @@ struct FusedArgs {
   int chunks, tiles_per_chunk;
   float* ws_p;
   float* ws_h;
+  // rg_prefill_relay.hip: states between blocks, tickets taken per head
+  uint64_t* relay_words;
+  int* relay_tickets;
   // or null: workgroup (0, 0) leaves here the shader-clock cycles and the
   // 100 MHz ticks its tile loop took (rg_prefill_clock_probe)
   uint64_t* timing;
@@ -312,6 +315,11 @@ void scan_split_plan(int B, int T, int W, int granule, int* chunks,
 int scan_split_granule(int dtype, int W);
 hipError_t launch_block_prefill_bf16(const FusedArgs& a, hipStream_t s);
 hipError_t launch_block_prefill_teams_bf16(const FusedArgs& a, hipStream_t s);
+// the same with blocks of 32 tokens dealt out and states handed on in memory
+bool prefill_relay_pays(int B, int H, int T, bool joined);
+size_t prefill_relay_workspace_bytes(int B, int W, int H);
+hipError_t launch_block_prefill_relay_bf16(FusedArgs a, void* workspace,
+                                           hipStream_t s);
 // the same for heads of 128 .. 256 channels, cut into slices of 64: few (row,
 // head) pairs, short rows, narrower heads (rg_prefill_slices.hip)
 bool prefill_slices_serve(int B, int H, int T, bool joined);  // 256-wide heads

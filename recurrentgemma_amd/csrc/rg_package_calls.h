@@ -42,8 +42,9 @@ size_t rg_argmax_workspace_bytes(int rows, int n);
 int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
                          int n, int dtype, void* stream);
 
-/* The workspace with which rg_recurrent_core is fastest: what it needs or, for
- * shapes that one launch without a workspace serves, what its other form takes. */
+/* The workspace with which rg_recurrent_core is fastest: what it needs or, where a
+ * form with a larger one is ahead (float32 shapes that one launch serves as well, bf16
+ * rows that come out uneven on the CUs), what that takes. */
 size_t rg_recurrent_core_best_workspace_bytes(int B, int T, int W, int H,
                                               int dtype);
 
