@@ -69,7 +69,8 @@ linear_rows_kernel(LinearArgs p) {
   constexpr int kLoads = XR / 8;          // of x per chunk
   constexpr int kMB = XR > 32 ? 2 : 1;    // blocks of 32 result rows
   constexpr int kWaveLds = wave_lds_bytes(NT, kMB);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   const int r = lane & 31, g = lane >> 5;
   const int M = p.M, K = p.K;
   const int chunks = K / 64;
@@ -106,20 +107,18 @@ linear_rows_kernel(LinearArgs p) {
 
   u32x4 xr[kLoads];
   Frag wq[2][NT][4];
-  // loads of the chunk after the last one read the last one again
   auto load_chunk = [&](int c, int slot) {
-    const int cc = min(c, chunks - 1);
 #pragma unroll
     for (int j = 0; j < kLoads; ++j)
-      xr[j] = *reinterpret_cast<const u32x4*>(xg[j] + (size_t)cc * 64);
+      xr[j] = *reinterpret_cast<const u32x4*>(xg[j] + (size_t)c * 64);
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int k = 0; k < 4; ++k)
         wq[slot][t][k].u =
-            __builtin_nontemporal_load(wg[t] + (size_t)(cc * 4 + k) * 64);
+            __builtin_nontemporal_load(wg[t] + (size_t)(c * 4 + k) * 64);
   };
-  auto body = [&](int slot, int c) {
+  auto body = [&](int slot, int c, bool more) {
 #pragma unroll
     for (int j = 0; j < kLoads; ++j)
       *reinterpret_cast<u32x4*>(xs + (8 * j + xrow) * kXStride + 8 * xseg) =
@@ -131,7 +130,7 @@ linear_rows_kernel(LinearArgs p) {
       for (int m = 0; m < kMB; ++m)
         xf[k][m].u = *reinterpret_cast<const u32x4*>(
             xs + (32 * m + r) * kXStride + 16 * k + 8 * g);
-    load_chunk(c + 1, slot ^ 1);
+    if (more) load_chunk(c + 1, slot ^ 1);
     // (the next chunk's loads stay in front of this one's products)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -146,11 +145,22 @@ linear_rows_kernel(LinearArgs p) {
   if (c0 < c1) {
     load_chunk(c0, 0);
     int c = c0;
-    for (; c + 1 < c1; c += 2) {
-      body(0, c);
-      body(1, c + 1);
+    for (; c + 2 < c1; c += 2) {
+      body(0, c, true);
+      body(1, c + 1, true);
     }
-    if (c < c1) body(0, c);
+    // The last one or two: nothing is loaded behind them.  (A load of the last chunk
+    // once more, as an even number of chunks a wave used to have it, is an eighth of
+    // the weights at K 4096: us a layer, with / without it, N 8192 at 1, 16, 32, 64
+    // rows 15.1 / 14.5, 15.5 / 14.4, 16.7 / 15.4, 19.7 / 18.5; N 24576 in pairs
+    // 47.5 / 44; K 2048, N 2560 6.6 / 6.0; odd numbers the same.  More chunks on their
+    // way, 3 to 5 of them, are no faster: a CU takes about 40 GB/s whatever waits.)
+    if (c + 1 < c1) {
+      body(0, c, true);
+      body(1, c + 1, false);
+    } else {
+      body(0, c, false);
+    }
   }
 
   // the waves' partial sums meet in LDS (each wave's region is its own x tile)
@@ -327,7 +337,7 @@ hipError_t launch_rows_of(const LinearArgs& a, dim3 grid, hipStream_t s) {
 //   K 2560, N 2560     8.7 /  6.5   8.7 /  7.6   9.9 /  9.1  11.8 / 11.3
 //   K 2560, N 5120    10.6 /  7.6  10.8 /  9.3  10.3 / 10.1  12.6 / 12.1
 //   K 7680, N 2560    12.7 / 11.2  13.1 / 12.0  14.6 / 13.6  17.1 / 16.2
-//   K 4096, N 8192    17.8 / 15.1  17.9 / 15.4  17.9 / 16.7  20.7 / 20.0
+//   K 4096, N 8192    17.8 / 14.5  17.9 / 14.4  17.9 / 15.4  20.7 / 18.5
 // (8 staged rows are within 2 % of 16.  Fewer rows without the barrier are
 // slower than 64, 10.0 us for one row at 2560 x 2560: the compiler moves the
 // loads behind the products.)
