@@ -887,14 +887,32 @@ static int linear_scan_impl(const char* who, const void* x, const void* a,
   s.T = T;
   s.W = W;
   if (split) {
-    const int rc = plan_scan_split(who, &s, dtype, workspace, workspace_bytes);
-    if (rc != RG_OK) return rc;
+    const size_t deal =
+        workspace == nullptr || !aligned16(workspace)
+            ? 0
+            : rg::scan_tiles_deal_bytes(B, T, W, dtype, rg::kTilesFwdPlain);
+    if (deal > 0 && workspace_bytes >= deal) {
+      s.deal = workspace;
+    } else {
+      const int rc = plan_scan_split(who, &s, dtype, workspace, workspace_bytes);
+      if (rc != RG_OK) return rc;
+    }
   }
   return launch_status(who, rg::launch_lru_scan(s, dtype, (hipStream_t)stream));
 }
 
 #undef RG_WHO
 #define RG_WHO __func__
+
+size_t rg_linear_scan_best_workspace_bytes(int B, int T, int W, int dtype,
+                                           int backward) {
+  if (B <= 0 || T <= 0 || W <= 0) return 0;
+  const size_t deal = rg::scan_tiles_deal_bytes(
+      B, T, W, dtype, backward ? rg::kTilesBwdPlain : rg::kTilesFwdPlain);
+  if (backward) return deal;
+  const size_t split = rg_scan_split_workspace_bytes(B, T, W);
+  return split < deal ? deal : split;
+}
 
 int rg_linear_scan(const void* x, const void* a, const void* reset,
                    const void* h0, void* y, void* h_last, int B, int T, int W,
@@ -911,13 +929,17 @@ int rg_linear_scan_split(const void* x, const void* a, const void* reset,
                           workspace_bytes, true, B, T, W, dtype, stream);
 }
 
-int rg_linear_scan_backward(const void* dy, const void* a, const void* reset,
-                            const void* y, const void* h0, const void* dh_last,
-                            void* dx, void* da, void* dh0, int B, int T, int W,
-                            int dtype, void* stream) {
+#undef RG_WHO
+#define RG_WHO who
+static int linear_scan_backward_impl(const char* who, const void* dy, const void* a,
+                                     const void* reset, const void* y,
+                                     const void* h0, const void* dh_last, void* dx,
+                                     void* da, void* dh0, void* workspace,
+                                     size_t workspace_bytes, int B, int T, int W,
+                                     int dtype, void* stream) {
   RG_CHECK_DTYPE(dtype);
   RG_REQUIRE(B > 0 && T > 0 && W > 0, "%s: B=%d T=%d W=%d must be positive",
-             __func__, B, T, W);
+             who, B, T, W);
   RG_CHECK_PTR(dy);
   RG_CHECK_PTR(a);
   RG_CHECK_PTR(reset);
@@ -929,7 +951,7 @@ int rg_linear_scan_backward(const void* dy, const void* a, const void* reset,
   RG_CHECK_OPT_PTR(dh0);
   RG_REQUIRE(dx != a && dx != y && da != a && da != y && da != dy && dx != da,
              "%s: dx and da must not alias a, y or each other (da nor dy)",
-             __func__);
+             who);
   rg::ScanBwdArgs s{};
   s.dy = dy;
   s.a = a;
@@ -943,8 +965,33 @@ int rg_linear_scan_backward(const void* dy, const void* a, const void* reset,
   s.B = B;
   s.T = T;
   s.W = W;
-  return launch_status(__func__, rg::launch_linear_scan_backward(
-                                     s, dtype, (hipStream_t)stream));
+  const size_t deal =
+      workspace == nullptr || !aligned16(workspace)
+          ? 0
+          : rg::scan_tiles_deal_bytes(B, T, W, dtype, rg::kTilesBwdPlain);
+  if (deal > 0 && workspace_bytes >= deal) s.deal = workspace;
+  return launch_status(
+      who, rg::launch_linear_scan_backward(s, dtype, (hipStream_t)stream));
+}
+#undef RG_WHO
+#define RG_WHO __func__
+
+int rg_linear_scan_backward(const void* dy, const void* a, const void* reset,
+                            const void* y, const void* h0, const void* dh_last,
+                            void* dx, void* da, void* dh0, int B, int T, int W,
+                            int dtype, void* stream) {
+  return linear_scan_backward_impl(__func__, dy, a, reset, y, h0, dh_last, dx, da,
+                                   dh0, nullptr, 0, B, T, W, dtype, stream);
+}
+
+int rg_linear_scan_backward_best(const void* dy, const void* a, const void* reset,
+                                 const void* y, const void* h0, const void* dh_last,
+                                 void* dx, void* da, void* dh0, void* workspace,
+                                 size_t workspace_bytes, int B, int T, int W,
+                                 int dtype, void* stream) {
+  return linear_scan_backward_impl("rg_linear_scan_backward", dy, a, reset, y, h0,
+                                   dh_last, dx, da, dh0, workspace, workspace_bytes,
+                                   B, T, W, dtype, stream);
 }
 
 int rg_rglru_backward(const void* dy, const void* x, const void* gx_pre,

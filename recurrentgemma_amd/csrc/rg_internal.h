@@ -94,6 +94,7 @@ struct ScanArgs {
   int chunks, t_chunk;
   float* ws_p;
   float* ws_h;
+  void* deal;  // plain: as in ScanTileArgs
 };
 
 struct FusedArgs {
@@ -252,6 +253,7 @@ struct ScanBwdArgs {
   void* da;              // [B, T, W]
   float* dh0;            // [B, W] or null
   int B, T, W;
+  void* deal;            // as in ScanTileArgs
 };
 hipError_t launch_linear_scan_backward(const ScanBwdArgs& a, int dtype,
                                        hipStream_t s);
@@ -298,7 +300,14 @@ struct ScanTileArgs {
   uint8_t* starts_out;   // [B, T], 1 where a document starts
   float* bias_out;       // float32: [2][W]
   int B, T, W;
+  // or null: scan_tiles_deal_bytes of workspace (16-byte aligned), and the steps of
+  // all rows are dealt out to one workgroup per CU; dlam and dbias are then
+  // [B * scan_tiles_steps, W] and [2][B * scan_tiles_steps, W], a row per step
+  void* deal;
 };
+// what it takes; 0 where a slab by the workgroup is the faster form
+size_t scan_tiles_deal_bytes(int B, int T, int W, int dtype, int mode);
+int scan_tiles_steps(int T, int mode);
 enum ScanTileMode { kTilesFwdPlain, kTilesBwdPlain, kTilesFwdGated, kTilesBwdGated,
                     // (a question only) both gated ones of a float32 RG-LRU
                     kTilesPairGated };

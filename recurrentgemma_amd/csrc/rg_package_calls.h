@@ -48,6 +48,16 @@ int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
 size_t rg_recurrent_core_best_workspace_bytes(int B, int T, int W, int H,
                                               int dtype);
 
+/* The bare recurrence with the workspace that it is fastest with, forward by
+ * rg_linear_scan_split and backward by rg_linear_scan_backward_best (0: none). */
+size_t rg_linear_scan_best_workspace_bytes(int B, int T, int W, int dtype,
+                                           int backward);
+int rg_linear_scan_backward_best(const void* dy, const void* a, const void* reset,
+                                 const void* y, const void* h0, const void* dh_last,
+                                 void* dx, void* da, void* dh0, void* workspace,
+                                 size_t workspace_bytes, int B, int T, int W,
+                                 int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

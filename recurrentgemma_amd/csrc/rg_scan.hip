@@ -900,7 +900,8 @@ int scan_split_granule(int dtype, int W) {
 }
 
 hipError_t launch_lru_scan(const ScanArgs& a, int dtype, hipStream_t s) {
-  if (a.plain && scan_tiles_serve(a.B, a.T, a.W, dtype, kTilesFwdPlain)) {
+  if (a.plain &&
+      (a.deal || scan_tiles_serve(a.B, a.T, a.W, dtype, kTilesFwdPlain))) {
     ScanTileArgs t{};
     t.in[0] = a.x;
     t.in[1] = a.ga;
@@ -912,6 +913,7 @@ hipError_t launch_lru_scan(const ScanArgs& a, int dtype, hipStream_t s) {
     t.B = a.B;
     t.T = a.T;
     t.W = a.W;
+    t.deal = a.deal;
     return launch_scan_tiles(t, kTilesFwdPlain, dtype, s);
   }
   // Channels per lane: 8 bytes per lane where the width allows it (every row

@@ -451,7 +451,7 @@ hipError_t launch_rglru_backward(const RglruBwdArgs& a, int dtype,
 
 hipError_t launch_linear_scan_backward(const ScanBwdArgs& a, int dtype,
                                        hipStream_t s) {
-  if (scan_tiles_serve(a.B, a.T, a.W, dtype, kTilesBwdPlain)) {
+  if (a.deal || scan_tiles_serve(a.B, a.T, a.W, dtype, kTilesBwdPlain)) {
     ScanTileArgs t{};
     t.in[0] = a.dy;
     t.in[1] = a.a;
@@ -466,6 +466,7 @@ hipError_t launch_linear_scan_backward(const ScanBwdArgs& a, int dtype,
     t.B = a.B;
     t.T = a.T;
     t.W = a.W;
+    t.deal = a.deal;
     return launch_scan_tiles(t, kTilesBwdPlain, dtype, s);
   }
   const bool two = scan_backward_two_channels(a.B, a.W);

@@ -21,6 +21,20 @@
 //   3  every lane replays its tokens from that state and stores.
 // Rows are asked for as early as the registers allow (see below), so that the
 // memory pipe works while a step computes.
+//
+// A workgroup walks one slab of channels of one row, or (DEAL) the steps of all slabs
+// are dealt out: few rows leave most CUs without a slab, and slabs beyond a multiple
+// of the CUs take a round of their own.  One workgroup per CU takes steps from a
+// counter, the first step of all slabs, then the second, ..; the state behind a step
+// is one word per channel, value and number of the step, that goes through memory
+// (agent-scope stores and loads of the whole word: no fence) to whoever has the next
+// one, between that step's 2 and 3.  Two words per row and channel: the state of step
+// s - 2 has been read when the one of s - 1 arrives.  Every wait ends: a workgroup
+// works on its tickets in order, a step waits for one with a smaller ticket, and only
+// a workgroup that runs takes tickets.  Sums over tokens leave a row per step.
+// us, B1 T8192 W2560 bf16, slabs / dealt: plain forward 82 / 38, backward 130 / 49,
+// gated 152 / 63 and 389 / 112; a step costs as much as before, the rest is the first
+// launch (states and counter cleared), the first tickets and loads: 14 us.
 // The kernels this replaces where it runs (rg_scan.hip, rg_scan_bwd.hip) keep
 // one or two channels per lane: 80 .. 160 workgroups with 2- and 4-byte
 // accesses at B4 W2560, and the backward ones read their inputs twice and
@@ -112,14 +126,32 @@ struct TileLds {
   // lie channels / 8 rows apart, then start on different banks)
   float pair[kGroups][2 * channels + 2];  // P, H per channel
   float in[kGroups][channels + 4];        // state before the group
-  float sp[channels];                     // softplus of a_param
-  float bias[2][channels];                // float32: of the gate projections
+  // (dealt out: of this step's slab and the next one's)
+  float sp[2][channels];                  // softplus of a_param
+  float slope[2][channels];               // and its derivative
+  float bias[2][2][channels];             // float32: of the gate projections
+  int ticket[4];                          // dealt out: the last four
+};
+
+// Dealt out: polls of a state before a wave gives up with NaN (seconds; it cannot
+// happen, see below).
+constexpr int kMaxPolls = 1 << 21;
+
+// What the dealt form has beside: states between steps, [B][2][W] words of value and
+// number of the step; the tickets taken; total = steps x chains, chains = B x slabs.
+struct DealArgs {
+  uint64_t* words;
+  float* soft;  // [2][W]: softplus of a_param, its derivative
+  int* counter;
+  int chains, slabs, total;
+  uint32_t inv_chains, inv_slabs;
 };
 
 // JOIN (gated forward, float32): y leaves as y * gelu(in[3]), the join of the
 // recurrent block's two branches (recurrentgemma/torch/modules.py:627-628, 644).
-template <typename T, int MODE, int KL, bool JOIN = false>
-__global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
+template <typename T, int MODE, int KL, bool JOIN, bool DEAL>
+__global__ void __launch_bounds__(kThreads)
+scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
   static_assert(!JOIN || (MODE == kFwdGated && sizeof(T) == 4), "");
   using V = Vec<T>;
   using Lds = TileLds<T>;
@@ -141,35 +173,81 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Workgroups go to the eight XCDs in turn: neighbouring slabs of channels,
-  // which share cache lines where W is no multiple of a slab, to one of them.
-  int block = blockIdx.x;
-  {
-    const int per_xcd = (int)gridDim.x / 8;
-    if (block < 8 * per_xcd) block = (block & 7) * per_xcd + (block >> 3);
-  }
-  const int slabs = (p.W + CH - 1) / CH;
-  const int b = block / slabs;
-  const int c0 = (block - b * slabs) * CH;
   const int T_len = p.T;
   const int oct = lane % kLanes, q = lane / kLanes;
   const int group = wave * (64 / kLanes) + q;
-  const int c = c0 + oct * N;
-  const bool c_ok = c < p.W;  // W % N == 0: all of the vector or nothing
-
   const uint32_t row_bytes = (uint32_t)p.W * sizeof(T);
   const uint32_t seq_bytes = (uint32_t)T_len * row_bytes;  // < 2^31 (launcher)
-  __amdgpu_buffer_rsrc_t rs[NS];
-#pragma unroll
-  for (int s = 0; s < NS; ++s)
-    rs[s] = make_rsrc((const char*)p.in[s] + (int64_t)b * seq_bytes, seq_bytes);
-  // which of them is y (read one row before the token): backward only
+  // which of the streams is y (read one row before the token): backward only
   constexpr int kY = MODE == kBwdPlain ? 2 : 4;
-  const uint32_t c_off = (uint32_t)c * sizeof(T);
 
   // Blocks of KL tokens in the order of the recurrence.
   const int blocks = (T_len + KL - 1) / KL;
   const int steps = (blocks + kGroups - 1) / kGroups;
+
+  // A step of a slab of channels.
+  struct Place {
+    int b, c0, step;
+    bool any;
+  };
+  // (dealt out: scalar divisions, an inverse gives the quotient or one less)
+  auto quotient = [](uint32_t n, uint32_t by, uint32_t inverse, uint32_t& rest) {
+    uint32_t k = (uint32_t)(((uint64_t)n * inverse) >> 32);
+    rest = n - k * by;
+    k += rest >= by ? 1u : 0u;
+    rest -= rest >= by ? by : 0u;
+    return k;
+  };
+  auto place_of = [&](int ticket) {
+    Place z;
+    z.any = ticket < d.total;
+    uint32_t chain, slab;
+    z.step = (int)quotient(z.any ? (uint32_t)ticket : 0u, (uint32_t)d.chains,
+                           d.inv_chains, chain);
+    z.b = (int)quotient(chain, (uint32_t)d.slabs, d.inv_slabs, slab);
+    z.c0 = (int)slab * CH;
+    return z;
+  };
+  auto place_at = [&](int k) {  // of this workgroup's k-th ticket
+    return place_of(__builtin_amdgcn_readfirstlane(lds.ticket[k & 3]));
+  };
+  auto take = [&]() { return atomicAdd(d.counter, 1); };
+  Place now, ahead;
+  int asked = 0;  // (thread 0) the ticket after `ahead`'s
+  if (DEAL) {
+    if (tid == 0) {
+      const int first = take(), second = take();
+      asked = take();
+      lds.ticket[0] = first;
+      lds.ticket[1] = second;
+    }
+    __syncthreads();
+    now = place_at(0);
+    ahead = place_at(1);
+  } else {
+    // Workgroups go to the eight XCDs in turn: neighbouring slabs of channels,
+    // which share cache lines where W is no multiple of a slab, to one of them.
+    int block = blockIdx.x;
+    const int per_xcd = (int)gridDim.x / 8;
+    if (block < 8 * per_xcd) block = (block & 7) * per_xcd + (block >> 3);
+    const int slabs = (p.W + CH - 1) / CH;
+    now.b = block / slabs;
+    now.c0 = (block - now.b * slabs) * CH;
+    now.step = 0;
+    now.any = true;
+    ahead = now;
+    ahead.step = 1;
+  }
+  // this lane's byte offset in a place's rows, which start at its slab (W % N == 0:
+  // all of the vector or nothing)
+  auto lane_off = [&](const Place& z) {
+    return z.c0 + oct * N < p.W ? (uint32_t)(oct * N * sizeof(T)) : kBufferOutOfRange;
+  };
+  auto rows_of = [&](const void* base, const Place& z) {
+    const uint32_t before = (uint32_t)z.c0 * sizeof(T);
+    return make_rsrc((const char*)base + (int64_t)z.b * seq_bytes + before,
+                     z.any ? seq_bytes - before : 0u);
+  };
   auto first_token = [&](int step, int g) {
     const int o = step * kGroups + g;
     return (kBwd ? blocks - 1 - o : o) * KL;  // (may lie before or past the row)
@@ -186,20 +264,44 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
     return MODE == kFwdPlain || s == 0 || (kBwd && s == kCoef);
   };
   u32x4 next[kReload ? 1 : 2][KL];
-  auto fetch = [&](int s, int t0, int i) {
+  // (dealt out: this step's streams and, those that are asked for a step ahead, the
+  // next one's)
+  __amdgpu_buffer_rsrc_t rs[NS], rs_ahead[NS];
+  uint32_t off_now = lane_off(now), off_ahead = off_now;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) rs[s] = rs_ahead[s] = rows_of(p.in[s], now);
+  auto look_ahead = [&]() __attribute__((always_inline)) {
+    if (DEAL) {
+      off_ahead = lane_off(ahead);
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        if (kReload || is_early(s)) rs_ahead[s] = rows_of(p.in[s], ahead);
+    }
+  };
+  auto fetch_from = [&](const __amdgpu_buffer_rsrc_t (&from)[NS], uint32_t off, int s,
+                        int t0, int i) __attribute__((always_inline)) {
     const int t = kBwd && s == kY ? t0 + i - 1 : t0 + i;
     // (a row before or past the sequence falls outside the descriptor)
     return __builtin_amdgcn_raw_buffer_load_b128(
-        rs[s], c_ok ? c_off + (uint32_t)t * row_bytes : kBufferOutOfRange, 0, 0);
+        from[s],
+        off != kBufferOutOfRange ? off + (uint32_t)t * row_bytes : kBufferOutOfRange,
+        0, 0);
+  };
+  auto fetch = [&](int s, int t0, int i) __attribute__((always_inline)) {
+    return fetch_from(rs, off_now, s, t0, i);
+  };
+  auto fetch_ahead = [&](int s, int t0, int i) __attribute__((always_inline)) {
+    return DEAL ? fetch_from(rs_ahead, off_ahead, s, t0, i)
+                : fetch_from(rs, off_now, s, t0, i);
   };
   // Document starts of the wave's 8 KL tokens, one token per lane.
   uint32_t flag_lo = 1, flag_hi = 0;
   bool flag_in = false;
-  auto load_flags = [&](int step) {
-    const int lo = first_token(step, kBwd ? wave * 8 + 7 : wave * 8);
+  auto load_flags = [&](const Place& z) {
+    const int lo = first_token(z.step, kBwd ? wave * 8 + 7 : wave * 8);
     const int t = lo + lane;
     flag_in = lane < 8 * KL && t >= 0 && t < T_len;
-    const int64_t at = (int64_t)b * T_len + (flag_in ? t : 0);
+    const int64_t at = (int64_t)z.b * T_len + (flag_in ? t : 0);
     if (p.flag_kind == kSegMaskU8) {
       flag_lo = reinterpret_cast<const uint8_t*>(p.flags)[at] == 0;
       flag_hi = 0;
@@ -215,23 +317,46 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
 
   // softplus of a_param, log2 a = -8 log2(e) sp sigmoid(.): read from LDS
   // twice a step (no registers to keep it in)
-  auto lambda_of = [&](int ch) {  // a_param of the workgroup's channel ch
-    return c0 + ch < p.W ? load_scalar((const T*)p.a_param + c0 + ch) : 0.0f;
+  auto channel_value = [&](const void* v, int ch) {
+    return ch < p.W ? load_scalar((const T*)v + ch) : 0.0f;
   };
-  if (kGated) {
-    if (tid < CH) {
-      lds.sp[tid] = softplus_precise(lambda_of(tid));
+  // (thread ch < CH) its channel's values of a place, asked for and laid into LDS
+  float soft[2] = {0.0f, 0.0f}, biases[2] = {0.0f, 0.0f};
+  auto ask_channel = [&](const Place& z) __attribute__((always_inline)) {
+    if (kGated && tid < CH) {
+      const int ch = z.c0 + tid;
+      if (DEAL) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          soft[g] = ch < p.W ? d.soft[(int64_t)g * p.W + ch] : 0.0f;
+      } else {
+        soft[0] = softplus_precise(channel_value(p.a_param, ch));
+      }
+      if (kBias) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          biases[g] = p.bias[g] ? channel_value(p.bias[g], ch) : 0.0f;
+      }
+    }
+  };
+  auto lay_channel = [&](const Place& z, int k) __attribute__((always_inline)) {
+    if (kGated && tid < CH) {
+      lds.sp[k & 1][tid] = soft[0];
+      if (DEAL) lds.slope[k & 1][tid] = soft[1];
       if (kBias) {
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-          lds.bias[g][tid] = p.bias[g] && c0 + tid < p.W
-                                 ? load_scalar((const T*)p.bias[g] + c0 + tid)
-                                 : 0.0f;
-          if (MODE == kFwdGated && p.bias_out && b == 0 && c0 + tid < p.W)
-            p.bias_out[(int64_t)g * p.W + c0 + tid] = lds.bias[g][tid];
+          lds.bias[k & 1][g][tid] = biases[g];
+          if (MODE == kFwdGated && p.bias_out && z.any && z.b == 0 && z.step == 0 &&
+              z.c0 + tid < p.W)
+            p.bias_out[(int64_t)g * p.W + z.c0 + tid] = biases[g];
         }
       }
     }
+  };
+  if (kGated) {
+    ask_channel(now);
+    lay_channel(now, 0);
     __syncthreads();
   }
   auto read_row = [&](const float* row, float (&v)[N]) __attribute__((always_inline)) {
@@ -242,14 +367,14 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
       for (int k = 0; k < 4; ++k) v[e + k] = r[k];
     }
   };
-  auto read_sp = [&](float (&sp)[N]) __attribute__((always_inline)) {
-    read_row(lds.sp, sp);
+  auto read_sp = [&](int k, float (&sp)[N]) __attribute__((always_inline)) {
+    read_row(lds.sp[DEAL ? k & 1 : 0], sp);
   };
   // a gate's pre-activations (0: input, 1: recurrence), the bias included
-  auto add_bias = [&](int g, float (&v)[N]) __attribute__((always_inline)) {
+  auto add_bias = [&](int k, int g, float (&v)[N]) __attribute__((always_inline)) {
     if constexpr (kBias) {
       float b_[N];
-      read_row(lds.bias[g], b_);
+      read_row(lds.bias[DEAL ? k & 1 : 0][g], b_);
 #pragma unroll
       for (int e = 0; e < N; ++e) v[e] += b_[e];
     }
@@ -262,38 +387,90 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
   // The scanning thread's channel and its state before the step.
   const int seg = lane / kSegLane;
   const int scan_ch = wave * kSegLane + lane % kSegLane;
-  float carry = 0.0f;
-  if (p.init && c0 + scan_ch < p.W)
-    carry = p.init[(int64_t)b * p.W + c0 + scan_ch];
+  auto initial = [&](const Place& z) {
+    return p.init && z.c0 + scan_ch < p.W ? p.init[(int64_t)z.b * p.W + z.c0 + scan_ch]
+                                          : 0.0f;
+  };
+  float carry = DEAL ? 0.0f : initial(now);
 
   float lam_acc[MODE == kBwdGated ? N : 1];
   // float32: also the sums of the gates' gradients (bf16 has no registers for
   // them, and its weight gradients' kernel forms them)
   constexpr bool kBiasGrads = MODE == kBwdGated && kBias;
   float bias_acc[2][kBiasGrads ? N : 1];
-  if (MODE == kBwdGated) {
+  // What a row's (dealt out: a block's) tokens make of the sums over tokens.
+  auto zero_sums = [&]() __attribute__((always_inline)) {
+    if (MODE == kBwdGated) {
 #pragma unroll
-    for (int e = 0; e < N; ++e) lam_acc[e] = 0.0f;
-  }
-  if (kBiasGrads) {
+      for (int e = 0; e < N; ++e) lam_acc[e] = 0.0f;
+    }
+    if (kBiasGrads) {
 #pragma unroll
-    for (int e = 0; e < N; ++e) bias_acc[0][e] = bias_acc[1][e] = 0.0f;
-  }
+      for (int e = 0; e < N; ++e) bias_acc[0][e] = bias_acc[1][e] = 0.0f;
+    }
+  };
+  auto write_sums = [&](const Place& z, int k) __attribute__((always_inline)) {
+    if constexpr (MODE == kBwdGated) {
+      // over the groups in order
+      auto total = [&](const float (&v)[N]) __attribute__((always_inline)) {
+        lds_barrier();
+#pragma unroll
+        for (int e = 0; e < N; e += 4)
+          *reinterpret_cast<f32x4*>(&lds.in[group][oct * N + e]) =
+              f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
+        lds_barrier();
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) sum += lds.in[seg * kPer + i][scan_ch];
+#pragma unroll
+        for (int d_ = 1; d_ < kSegs; d_ *= 2) sum += __shfl_xor(sum, d_ * kSegLane);
+        return sum;
+      };
+      const bool writes = seg == 0 && z.c0 + scan_ch < p.W;
+      const int64_t rows = DEAL ? (int64_t)p.B * steps : p.B;
+      const int64_t row = DEAL ? (int64_t)z.b * steps + z.step : z.b;
+      const int64_t at = row * p.W + z.c0 + scan_ch;
+      const float lam = total(lam_acc);
+      if (writes)
+        p.dlam[at] = lam * (DEAL ? lds.slope[k & 1][scan_ch]
+                                 : sigmoid_precise(channel_value(p.a_param,
+                                                                 z.c0 + scan_ch)));
+      if constexpr (kBiasGrads) {
+        if (p.dbias != nullptr) {
+#pragma unroll
+          for (int g = 0; g < 2; ++g) {
+            const float sum = total(bias_acc[g]);
+            if (writes) p.dbias[(int64_t)g * rows * p.W + at] = sum;
+          }
+        }
+      }
+    }
+  };
 
-  load_flags(0);
+  load_flags(now);
   {
-    const int t0 = first_token(0, group);
+    const int t0 = first_token(now.step, group);
 #pragma unroll
     for (int i = 0; i < KL; ++i)
 #pragma unroll
       for (int s = 0; s < NS; ++s)
         if (kReload || is_early(s)) raw[s][i] = fetch(s, t0, i);
   }
-  // (the last step apart: only it can hold the row's end)
-  auto one_step = [&](int step, auto LAST) __attribute__((always_inline)) {
-    constexpr bool more = !decltype(LAST)::value;
-    const int t0 = first_token(step, group);
-    const int next_t0 = first_token(step + 1, group);
+  // (a row's last step apart: only it can hold the row's end, and undealt nothing
+  // comes behind it)
+  auto one_step = [&](int k, const Place& now, const Place& ahead,
+                      auto LAST) __attribute__((always_inline)) {
+    constexpr bool last = decltype(LAST)::value;
+    constexpr bool more = DEAL || !last;
+    const int t0 = first_token(now.step, group);
+    const int next_t0 = first_token(ahead.step, group);
+    const int c = now.c0 + oct * N;
+    const uint32_t c_off = off_now;
+    const bool c_ok = c_off != kBufferOutOfRange;
+    if (DEAL) {
+      zero_sums();
+      ask_channel(ahead);
+    }
     if (!kReload) {
 #pragma unroll
       for (int j = 0; j < KL; ++j) {
@@ -307,18 +484,18 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
     {
       const uint64_t mask = __ballot(flag_in && (flag_lo | flag_hi) == 0u);
       starts = (uint32_t)(mask >> ((kBwd ? 7 - q : q) * KL)) & ((1u << KL) - 1u);
-      if (MODE == kFwdGated && p.starts_out && c0 == 0 && flag_in)
-        p.starts_out[(int64_t)b * T_len + first_token(step, wave * 8) + lane] =
+      if (MODE == kFwdGated && p.starts_out && now.c0 == 0 && flag_in)
+        p.starts_out[(int64_t)now.b * T_len + first_token(now.step, wave * 8) + lane] =
             (flag_lo | flag_hi) == 0u;
     }
     if (more) {
-      load_flags(step + 1);
+      load_flags(ahead);
       if (!kReload) {
 #pragma unroll
         for (int j = 0; j < KL; ++j) {
           const int i = kBwd ? KL - 1 - j : j;
-          next[0][i] = fetch(0, next_t0, i);
-          next[kReload ? 0 : 1][i] = fetch(kCoef, next_t0, i);
+          next[0][i] = fetch_ahead(0, next_t0, i);
+          next[kReload ? 0 : 1][i] = fetch_ahead(kCoef, next_t0, i);
         }
       }
     }
@@ -333,7 +510,7 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
     float coef[kGated ? KL : 1][N];
     float kept[MODE == kFwdGated || kKeepGate ? KL : 1][N];
     float P[N], H[N], sp[N];
-    if (kGated) read_sp(sp);
+    if (kGated) read_sp(k, sp);
 #pragma unroll
     for (int e = 0; e < N; ++e) {
       P[e] = 1.0f;
@@ -352,11 +529,11 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
       } else {
         float ga[N];
         V::unpack(raw[MODE == kFwdGated ? 2 : 3][i], ga);
-        add_bias(1, ga);
+        add_bias(k, 1, ga);
         float gx[N];
         if (MODE == kFwdGated) {
           V::unpack(raw[1][i], gx);
-          add_bias(0, gx);
+          add_bias(k, 0, gx);
         }
 #pragma unroll
         for (int e = 0; e < N; ++e) {
@@ -384,7 +561,7 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
       }
       if (kReload && more) {
 #pragma unroll
-        for (int s = 0; s < NS; ++s) raw[s][i] = fetch(s, next_t0, i);
+        for (int s = 0; s < NS; ++s) raw[s][i] = fetch_ahead(s, next_t0, i);
       }
     }
 #pragma unroll
@@ -396,11 +573,17 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
           f32x2{P[e + 1], H[e + 1]};
     }
     lds_barrier();
+    if (DEAL) {
+      if (tid == 0) {  // (asked for a step ago, there by now)
+        lds.ticket[(k + 2) & 3] = asked;
+        asked = take();
+      }
+      lay_channel(ahead, k + 1);
+    }
 
     u32x4 branch[JOIN ? KL : 1];
     if constexpr (JOIN) {
-      const __amdgpu_buffer_rsrc_t rg = make_rsrc(
-          (const char*)p.in[3] + (int64_t)b * seq_bytes, seq_bytes);
+      const __amdgpu_buffer_rsrc_t rg = rows_of(p.in[3], now);
 #pragma unroll
       for (int i = 0; i < KL; ++i)
         branch[i] = __builtin_amdgcn_raw_buffer_load_b128(
@@ -410,16 +593,32 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
 
     // ---- 2: scan over the groups ---------------------------------------------
     {
+      // (dealt out) the state behind the step before, from whoever had it: number
+      // and value
+      uint64_t* words = nullptr;
+      uint64_t word = 0;
+      bool there = false;
+      auto poll = [&]() __attribute__((always_inline)) {
+        word = (uint64_t)(uint32_t)now.step << 32;
+        if (there)
+          word = __hip_atomic_load(words + (int64_t)((now.step + 1) & 1) * p.W,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      };
+      if (DEAL) {
+        words = d.words + ((int64_t)now.b * 2) * p.W + now.c0 + scan_ch;
+        there = now.c0 + scan_ch < p.W;
+        if (now.step > 0) poll();
+      }
       f32x2 v[kPer];
 #pragma unroll
-      for (int k = 0; k < kPer; ++k)
-        v[k] = *reinterpret_cast<const f32x2*>(
-            &lds.pair[seg * kPer + k][2 * scan_ch]);
+      for (int i = 0; i < kPer; ++i)
+        v[i] = *reinterpret_cast<const f32x2*>(
+            &lds.pair[seg * kPer + i][2 * scan_ch]);
       float sp_ = 1.0f, sh = 0.0f;
 #pragma unroll
-      for (int k = 0; k < kPer; ++k) {
-        sh = __builtin_fmaf(v[k][0], sh, v[k][1]);
-        sp_ *= v[k][0];
+      for (int i = 0; i < kPer; ++i) {
+        sh = __builtin_fmaf(v[i][0], sh, v[i][1]);
+        sp_ *= v[i][0];
       }
 #pragma unroll
       for (int d = 1; d < kSegs; d *= 2) {
@@ -435,20 +634,42 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
         ep = 1.0f;
         eh = 0.0f;
       }
+      if constexpr (DEAL) {
+        if (now.step == 0) {
+          carry = initial(now);
+        } else {
+          for (int polls = 0; !__all((uint32_t)(word >> 32) == (uint32_t)now.step);
+               ++polls) {
+            if (polls == kMaxPolls) {
+              word = 0x7fc00000u;
+              break;
+            }
+            poll();
+          }
+          carry = __uint_as_float((uint32_t)word);
+        }
+        // this step's to whoever has the next
+        if (seg == kSegs - 1 && there && now.step + 1 < steps)
+          __hip_atomic_store(
+              words + (int64_t)(now.step & 1) * p.W,
+              ((uint64_t)(uint32_t)(now.step + 1) << 32) |
+                  __float_as_uint(__builtin_fmaf(sp_, carry, sh)),
+              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
       float s = __builtin_fmaf(ep, carry, eh);
 #pragma unroll
-      for (int k = 0; k < kPer; ++k) {
-        lds.in[seg * kPer + k][scan_ch] = s;
-        s = __builtin_fmaf(v[k][0], s, v[k][1]);
+      for (int i = 0; i < kPer; ++i) {
+        lds.in[seg * kPer + i][scan_ch] = s;
+        s = __builtin_fmaf(v[i][0], s, v[i][1]);
       }
-      carry = __shfl(s, (kSegs - 1) * kSegLane + lane % kSegLane);
+      if (!DEAL) carry = __shfl(s, (kSegs - 1) * kSegLane + lane % kSegLane);
     }
     lds_barrier();
 
     // ---- 3: replay ------------------------------------------------------------
     if (MODE == kBwdGated) {
       asm volatile("" ::: "memory");
-      read_sp(sp);
+      read_sp(k, sp);
     }
     float st[N];  // h, or the u that comes in from behind
 #pragma unroll
@@ -467,8 +688,7 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
                               ? c_off + (uint32_t)t * row_bytes
                               : kBufferOutOfRange;
       auto store = [&](int o, u32x4 v) {
-        buffer_store_16(v, make_rsrc((char*)p.out[o] + (int64_t)b * seq_bytes,
-                                     seq_bytes), at, 0);
+        buffer_store_16(v, rows_of(p.out[o], now), at, 0);
       };
       // (out of the compiler's sight: it would keep what it unpacked in step 1
       // in registers instead of the packed rows)
@@ -495,9 +715,9 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
           y[e] = JOIN ? gelu_mul_f32(st[e], __uint_as_float(branch[JOIN ? i : 0][e & 3]))
                       : st[e];
         store(0, V::pack(y));
-        if (!more && p.last && t == T_len - 1 && c_ok) {
+        if (last && p.last && t == T_len - 1 && c_ok) {
 #pragma unroll
-          for (int e = 0; e < N; ++e) p.last[(int64_t)b * p.W + c + e] = st[e];
+          for (int e = 0; e < N; ++e) p.last[(int64_t)now.b * p.W + c + e] = st[e];
         }
       } else {
         float hp[N];
@@ -505,7 +725,7 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
         if (i == 0 && t == 0) {  // (t0 is a multiple of KL)
 #pragma unroll
           for (int e = 0; e < N; ++e)  // h_{-1} in the activation dtype
-            hp[e] = p.h0 && c_ok ? round_act<T>(p.h0[(int64_t)b * p.W + c + e])
+            hp[e] = p.h0 && c_ok ? round_act<T>(p.h0[(int64_t)now.b * p.W + c + e])
                                  : 0.0f;
         }
         float g[N];
@@ -524,7 +744,7 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
           if (!kKeepGate) V::unpack(raw[3][i], pa);
           V::unpack(raw[1][i], x);
           V::unpack(raw[2][i], px);
-          add_bias(0, px);
+          add_bias(k, 0, px);
 #pragma unroll
           for (int e = 0; e < N; ++e) {
             const float a = coef[i][e];
@@ -560,7 +780,7 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
         }
         if (i == 0 && p.last && t == 0 && c_ok) {  // dh0
 #pragma unroll
-          for (int e = 0; e < N; ++e) p.last[(int64_t)b * p.W + c + e] = st[e];
+          for (int e = 0; e < N; ++e) p.last[(int64_t)now.b * p.W + c + e] = st[e];
         }
       }
     }
@@ -572,55 +792,88 @@ __global__ void __launch_bounds__(kThreads) scan_tiles_kernel(ScanTileArgs p) {
       }
     }
   };
-  for (int step = 0; step + 1 < steps; ++step) one_step(step, std::false_type{});
-  one_step(steps - 1, std::true_type{});
-
-  if constexpr (MODE == kBwdGated) {
-    // sums over the row: over the groups in order
-    auto total = [&](const float (&v)[N]) __attribute__((always_inline)) {
-      __syncthreads();
-#pragma unroll
-      for (int e = 0; e < N; e += 4)
-        *reinterpret_cast<f32x4*>(&lds.in[group][oct * N + e]) =
-            f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
-      __syncthreads();
-      float sum = 0.0f;
-#pragma unroll
-      for (int k = 0; k < kPer; ++k) sum += lds.in[seg * kPer + k][scan_ch];
-#pragma unroll
-      for (int d = 1; d < kSegs; d *= 2) sum += __shfl_xor(sum, d * kSegLane);
-      return sum;
-    };
-    const bool writes = seg == 0 && c0 + scan_ch < p.W;
-    const int64_t at = (int64_t)b * p.W + c0 + scan_ch;
-    const float lam = total(lam_acc);
-    if (writes) p.dlam[at] = lam * sigmoid_precise(lambda_of(scan_ch));
-    if constexpr (kBiasGrads) {
-      if (p.dbias != nullptr) {
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          const float sum = total(bias_acc[g]);
-          if (writes) p.dbias[(int64_t)g * p.B * p.W + at] = sum;
-        }
+  if constexpr (DEAL) {
+    look_ahead();
+    for (int k = 0; now.any; ++k) {
+      if (kBwd || now.step + 1 < steps) {
+        one_step(k, now, ahead, std::false_type{});
+      } else {
+        one_step(k, now, ahead, std::true_type{});
       }
+      write_sums(now, k);
+      now = ahead;
+      off_now = off_ahead;
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        rs[s] = kReload || is_early(s) ? rs_ahead[s] : rows_of(p.in[s], now);
+      ahead = place_at(k + 2);
+      look_ahead();
     }
+  } else {
+    zero_sums();
+    for (; now.step + 1 < steps; ++now.step, ++ahead.step)
+      one_step(0, now, ahead, std::false_type{});
+    one_step(0, now, ahead, std::true_type{});
+    write_sums(now, 0);
   }
+}
+
+// Before a dealt launch: no state valid, no ticket taken; softplus of a_param and its
+// derivative.
+template <typename T>
+__global__ void __launch_bounds__(256)
+deal_begin_kernel(u32x4* words, int64_t n, const T* a_param, float* soft, int W) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) words[i] = u32x4{0, 0, 0, 0};
+  if (a_param != nullptr && i < W) {
+    const float v = load_scalar(a_param + i);
+    soft[i] = softplus_precise(v);
+    soft[W + i] = sigmoid_precise(v);
+  }
+}
+
+// Tokens of a step.
+int step_tokens(int mode) { return (mode == kFwdPlain ? 8 : 4) * kGroups; }
+
+template <typename T, int MODE, int KL, bool JOIN, bool DEAL>
+hipError_t launch_form(const ScanTileArgs& a, hipStream_t s) {
+  constexpr int lds = sizeof(TileLds<T>);
+  static OncePerDevice once;
+  hipError_t e = set_max_dynamic_lds(
+      once, (const void*)scan_tiles_kernel<T, MODE, KL, JOIN, DEAL>, lds);
+  if (e != hipSuccess) return e;
+  const int slabs = (a.W + TileLds<T>::channels - 1) / TileLds<T>::channels;
+  int64_t blocks = (int64_t)a.B * slabs;
+  if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
+  DealArgs d{};
+  if (DEAL) {
+    const int64_t steps = scan_tiles_steps(a.T, MODE);
+    if (steps * blocks > (1 << 30)) return hipErrorInvalidValue;
+    d.words = (uint64_t*)a.deal;
+    const int64_t words = (int64_t)a.B * 2 * a.W;
+    d.counter = (int*)(d.words + words);  // (16 bytes of its own)
+    d.soft = (float*)(d.counter + 4);
+    d.chains = (int)blocks;
+    d.slabs = slabs;
+    d.inv_chains = 0xffffffffu / (uint32_t)blocks;
+    d.inv_slabs = 0xffffffffu / (uint32_t)slabs;
+    d.total = (int)(steps * blocks);
+    const int64_t items = words / 2 + 1;  // (at least W)
+    deal_begin_kernel<T><<<dim3((unsigned)((items + 255) / 256)), 256, 0, s>>>(
+        (u32x4*)a.deal, items, (const T*)a.a_param, d.soft, a.W);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    blocks = d.total < 256 ? d.total : 256;
+  }
+  scan_tiles_kernel<T, MODE, KL, JOIN, DEAL>
+      <<<dim3((unsigned)blocks), kThreads, lds, s>>>(a, d);
+  return hipGetLastError();
 }
 
 template <typename T, int MODE, int KL, bool JOIN = false>
 hipError_t launch_as(const ScanTileArgs& a, hipStream_t s) {
-  constexpr int lds = sizeof(TileLds<T>);
-  static OncePerDevice once;
-  hipError_t e =
-      set_max_dynamic_lds(once, (const void*)scan_tiles_kernel<T, MODE, KL, JOIN>,
-                          lds);
-  if (e != hipSuccess) return e;
-  const int64_t blocks =
-      (int64_t)a.B * ((a.W + TileLds<T>::channels - 1) / TileLds<T>::channels);
-  if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
-  scan_tiles_kernel<T, MODE, KL, JOIN>
-      <<<dim3((unsigned)blocks), kThreads, lds, s>>>(a);
-  return hipGetLastError();
+  return a.deal ? launch_form<T, MODE, KL, JOIN, true>(a, s)
+                : launch_form<T, MODE, KL, JOIN, false>(a, s);
 }
 
 }  // namespace
@@ -678,13 +931,14 @@ bool scan_tiles_serve(int B, int T, int W, int dtype, int mode) {
   // The forward ones (B4 T2048 W2560 bf16: plain 52 -> 28, gated 83 -> 44).
   // One or two long rows rg_scan.hip cuts into chunks (bf16 plain: B1 T4096
   // W512 26, here 32, W4096 60, here 41; gated from 4096 tokens on: T8192 105,
-  // here 146; float32 plain B1 T8192 W512 60, here 49).
+  // here 146; float32 plain B1 T8192 W512 60, here 49, gated W2560 T4096 103, here 65,
+  // T8192 181, here 152).
   int chunks, t_chunk;
   scan_split_plan(B, T, W, 64, &chunks, &t_chunk);
   if (chunks > 1) {
     const int64_t few = blocks * 64 > 2048 ? blocks * 64 : 2048;
     const int64_t most = mode == kFwdGated ? 4096 : dtype == 0 ? 8192 : few;
-    if (T > most) return false;
+    if (T > most && !(mode == kFwdGated && dtype == 0)) return false;
   }
   const bool cached = 3 * es * (int64_t)B * T * W < ((int64_t)256 << 20);
   // Gated: while every slab has a CU of its own; beyond, rows of some length that
@@ -701,6 +955,60 @@ bool scan_tiles_serve(int B, int T, int W, int dtype, int mode) {
   // T180 13, here 14, and B16 T500 W2048 35, here 35).
   if (blocks <= (dtype == 0 ? 512 : 256)) return true;
   return cached && (dtype == 0 ? blocks < 800 && T >= 400 : blocks > 512 && T >= 500);
+}
+
+int scan_tiles_steps(int T, int mode) {
+  return (T + step_tokens(mode) - 1) / step_tokens(mode);
+}
+
+// Dealt out against a slab by the workgroup: us, what a step of a full round and of
+// half a round takes (up to 128 slabs leave the memory to each other); dealt, what the
+// launches and the first step take, a round of 256 steps, and a step of one row, of
+// which the next one waits for its state.  Fitted to 18 shapes a kernel, 1 to 16 rows
+// of 1000 to 16000 tokens, 512 to 4096 wide, and within 15 % of them but where the
+// planes leave the last-level cache, which slows both alike (slab / dealt: bf16 gated
+// backward B1 T2048 W2560 85 / 43, T8192 389 / 112, B4 T2048 118 / 102, B7 T2000
+// 206 / 165, but B4 T1024 49 / 58; gated forward B1 T8192 152 / 63, B3 T4096 80 / 73;
+// plain backward B1 T8192 130 / 49; float32 gated backward B1 T8192 328 / 163).
+static bool dealing_pays(int B, int T, int W, int dtype, int mode) {
+  struct Cost {
+    float half, full, start, round, row;
+  };
+  static constexpr Cost kCost[2][4] = {
+      // float32: plain forward and backward, gated forward and backward
+      {{4.2f, 8.0f, 17.0f, 6.8f, 0.75f}, {3.4f, 6.0f, 17.0f, 5.6f, 0.75f},
+       {4.1f, 6.2f, 22.0f, 7.0f, 0.75f}, {7.5f, 15.6f, 22.0f, 13.5f, 0.85f}},
+      {{5.2f, 9.0f, 18.0f, 7.6f, 0.75f}, {4.2f, 7.4f, 17.0f, 6.6f, 0.75f},
+       {4.8f, 6.8f, 20.0f, 7.6f, 0.75f}, {10.6f, 17.4f, 20.0f, 16.5f, 0.85f}}};
+  const int64_t slab = dtype == 0 ? TileLds<float>::channels : TileLds<uint16_t>::channels;
+  const int64_t slabs = (int64_t)B * ((W + slab - 1) / slab);
+  const int64_t steps = scan_tiles_steps(T, mode);
+  if (steps < 2 || steps * slabs > (1 << 30)) return false;
+  const Cost& c = kCost[dtype != 0][mode];
+  const int64_t rest = slabs % 256;
+  const float last =
+      rest == 0 ? 0.0f
+                : c.half + (c.full - c.half) *
+                               sqrtf(fmaxf(0.0f, (float)(rest - 128) / 128.0f));
+  const float whole = 2.0f + (float)steps * ((float)(slabs / 256) * c.full + last);
+  const float rounds = (float)(steps * slabs) / 256.0f;
+  const float dealt = c.start + fmaxf(c.round * rounds, c.row * (float)steps);
+  // (its one launch more is time of the host, which short rows are waiting for)
+  const bool backward = mode == kBwdPlain || mode == kBwdGated;
+  if (whole < (backward ? 55.0f : 30.0f)) return false;
+  // (what rg_scan.hip cuts into chunks takes it 0.7 of a slab by the workgroup's time
+  // and more: bf16 B1 T8192 W2560 plain 75, gated 100, dealt 38 and 63; B1 T16000 W512
+  // 229 and 242, dealt 41 and 65)
+  const bool served = scan_tiles_serve(B, T, W, dtype, mode);
+  return dealt < (served ? 0.95f : backward ? 0.0f : 0.7f) * whole;
+}
+
+size_t scan_tiles_deal_bytes(int B, int T, int W, int dtype, int mode) {
+  if (B <= 0 || T <= 0 || W <= 0 || !scan_tiles_take(T, W, dtype) ||
+      !dealing_pays(B, T, W, dtype, mode))
+    return 0;
+  // states, the counter, softplus of a_param and its derivative
+  return (size_t)B * 2 * W * 8 + 16 + (((size_t)W * 8 + 15) & ~(size_t)15);
 }
 
 hipError_t launch_scan_tiles(const ScanTileArgs& a, int mode, int dtype,

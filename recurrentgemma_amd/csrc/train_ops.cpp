@@ -17,6 +17,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 
 #include "rg_internal.h"
+#include "rg_package_calls.h"
 
 namespace rg_host {
 namespace {
@@ -143,8 +144,8 @@ struct Kept {
 void scan_forward(const Tensor& x, const Tensor& a, const Tensor& reset,
                   const Tensor& h0, const Tensor& y, const Tensor& h) {
   const Dims d(x);
-  const size_t bytes =
-      rg_scan_split_workspace_bytes((int)d.B, (int)d.T, (int)d.W);
+  const size_t bytes = rg_linear_scan_best_workspace_bytes(
+      (int)d.B, (int)d.T, (int)d.W, d.code, 0);
   Tensor ws;
   if (bytes) ws = empty({(int64_t)bytes}, at::kByte, x);
   check(bytes ? rg_linear_scan_split(in(x), in(a), in(reset), in(h0), out(y),
@@ -176,9 +177,14 @@ struct Scan : Function<Scan> {
     const Tensor dh = grad_of(grads[1], {d.B, d.W}, at::kFloat);
     Tensor dx = empty(y.sizes(), y), da = empty(y.sizes(), y), dh0;
     if (h0.defined()) dh0 = empty(h0.sizes(), h0);
-    check(rg_linear_scan_backward(in(dy), in(a), in(reset), in(y), in(h0), in(dh),
-                                  out(dx), out(da), out(dh0), (int)d.B, (int)d.T,
-                                  (int)d.W, d.code, d.stream));
+    const size_t bytes = rg_linear_scan_best_workspace_bytes(
+        (int)d.B, (int)d.T, (int)d.W, d.code, 1);
+    Tensor ws;
+    if (bytes) ws = empty({(int64_t)bytes}, at::kByte, y);
+    check(rg_linear_scan_backward_best(in(dy), in(a), in(reset), in(y), in(h0),
+                                       in(dh), out(dx), out(da), out(dh0), out(ws),
+                                       bytes, (int)d.B, (int)d.T, (int)d.W, d.code,
+                                       d.stream));
     return {dx, da, Tensor(), dh0};
   }
 };
@@ -203,7 +209,16 @@ OnTiles on_tiles(const Dims& d) {
     const bool both = serve(rg::kTilesFwdGated) && serve(rg::kTilesPairGated);
     return {both, both};
   }
-  return {serve(rg::kTilesFwdGated), serve(rg::kTilesBwdGated)};
+  const bool dealt = rg::scan_tiles_deal_bytes((int)d.B, (int)d.T, (int)d.W, d.code,
+                                               rg::kTilesFwdGated) > 0;
+  return {dealt || serve(rg::kTilesFwdGated), serve(rg::kTilesBwdGated)};
+}
+
+// Workspace of the one-pass kernels' dealt form, where that is the faster one.
+Tensor deal_workspace(const Dims& d, rg::ScanTileMode mode, const Tensor& like) {
+  const size_t bytes =
+      rg::scan_tiles_deal_bytes((int)d.B, (int)d.T, (int)d.W, d.code, mode);
+  return bytes ? empty({(int64_t)bytes}, at::kByte, like) : Tensor();
 }
 
 // Kept::bias of a backward pass
@@ -280,6 +295,8 @@ void gated_forward(const Tensor& x, const Tensor& pos, const GateWeights& g,
     t.B = (int)d.B;
     t.T = (int)d.T;
     t.W = (int)d.W;
+    const Tensor ws = deal_workspace(d, rg::kTilesFwdGated, x);
+    t.deal = out(ws);
     check_hip(rg::launch_scan_tiles(t, rg::kTilesFwdGated, d.code, d.stream));
     return;
   }
@@ -336,11 +353,17 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
   GatedGrads r;
   r.dx = empty(x.sizes(), x);
   Tensor dgx = empty(x.sizes(), x), dga = empty(x.sizes(), x);
-  Tensor lam_rows = empty({d.B, d.W}, at::kFloat, x), bias_rows;
-  if (h0.defined()) r.dh0 = empty(h0.sizes(), h0);
   const bool tiles = on_tiles(d).backward;
+  Tensor ws_deal, bias_rows;
+  if (tiles) ws_deal = deal_workspace(d, rg::kTilesBwdGated, x);
+  // (dealt out: a row of sums per step)
+  const int64_t rows =
+      d.B * (ws_deal.defined() ? rg::scan_tiles_steps((int)d.T, rg::kTilesBwdGated) : 1);
+  Tensor lam_rows = empty({rows, d.W}, at::kFloat, x);
+  if (h0.defined()) r.dh0 = empty(h0.sizes(), h0);
   if (tiles) {
     rg::ScanTileArgs t{};
+    t.deal = out(ws_deal);
     t.in[0] = in(dy);
     t.in[1] = in(x);
     t.in[2] = in(gx);
@@ -352,7 +375,7 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
     if (f32) {
       t.bias[0] = in(kept.bias);
       t.bias[1] = kept.bias.const_data_ptr<float>() + d.W;
-      bias_rows = empty({2, d.B, d.W}, at::kFloat, x);
+      bias_rows = empty({2, rows, d.W}, at::kFloat, x);
       t.dbias = (float*)out(bias_rows);
     }
     t.init = (const float*)in(dh);
@@ -372,7 +395,7 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
                             out(dga), (float*)out(lam_rows), out(r.dh0), (int)d.B,
                             (int)d.T, (int)d.W, d.code, d.stream));
   }
-  r.dlam = sums.add(lam_rows, 0, d.B, d.W, d.W, {d.W}, x);
+  r.dlam = sums.add(lam_rows, 0, rows, d.W, d.W, {d.W}, x);
   if (f32) {
     Tensor xs = by_head(x, H), dxs = by_head(r.dx, H);
     Tensor dgs[2] = {by_head(dgx, H), by_head(dga, H)};
@@ -405,7 +428,7 @@ GatedGrads gated_backward(const Tensor& dy, const Tensor& dh, const Tensor& x,
       if (needs_w[i] && !pair) *dw[i] = at::bmm(xs.transpose(1, 2), dgs[i]);
       if (!needs_b[i]) continue;
       if (tiles)
-        *db[i] = sums.add(bias_rows, i * d.B * d.W, d.B, d.W, d.W, {H, bw}, x);
+        *db[i] = sums.add(bias_rows, i * rows * d.W, rows, d.W, d.W, {H, bw}, x);
       else
         *db[i] = (i ? dga : dgx).view({-1, H, bw}).sum(0);
     }
