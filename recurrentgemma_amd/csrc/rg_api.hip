@@ -598,6 +598,7 @@ struct CorePlan {
   // or, for re-laid-out weights and with as large a workspace, by the blocks of
   // rg_prefill_relay.hip (without and with the join; 0: not)
   size_t relay_bytes[2];
+  size_t deal_bytes;   // wide_f32: behind the rest, the one-pass kernel dealt out
   size_t split_bytes;  // chunk summaries of whichever form runs
   size_t gate_bytes;   // one gate's pre-activations (two-kernel form), padded
   size_t need() const { return small_f32 ? 0 : split_bytes + 2 * gate_bytes; }
@@ -638,6 +639,8 @@ static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
                rg::gates_f32_serves((int64_t)B * T, W, H) &&
                rg::scan_tiles_take(T, W, dtype) &&
                wide_f32_pays(B, T, W, H, p.small_f32);
+  if (p.wide_f32 && wide_scan_on_tiles(B, T, W))
+    p.deal_bytes = rg::scan_tiles_deal_bytes(B, T, W, dtype, rg::kTilesFwdGated);
   if (p.small_f32) {
     const size_t n = (size_t)B * T * W * sizeof(float);
     if (p.wide_f32) p.gate_bytes = (n + 255) & ~(size_t)255;
@@ -691,7 +694,7 @@ size_t rg_recurrent_core_best_workspace_bytes(int B, int T, int W, int H,
       (dtype != RG_DTYPE_F32 && dtype != RG_DTYPE_BF16))
     return 0;
   const CorePlan p = core_plan(B, T, W, H, dtype);
-  size_t n = p.split_bytes + 2 * p.gate_bytes;
+  size_t n = p.split_bytes + 2 * p.gate_bytes + p.deal_bytes;
   for (size_t relay : p.relay_bytes)
     if (n < relay) n = relay;
   return n;
@@ -801,6 +804,9 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
       t.B = B;
       t.T = T;
       t.W = W;
+      const size_t used = p.split_bytes + 2 * p.gate_bytes;
+      if (p.deal_bytes > 0 && workspace_bytes >= used + p.deal_bytes)
+        t.deal = (char*)workspace + used;
       return launch_status(__func__,
                            rg::launch_scan_tiles(t, rg::kTilesFwdGated, dtype,
                                                  (hipStream_t)stream));

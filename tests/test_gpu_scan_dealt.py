@@ -10,6 +10,7 @@ import torch
 
 from recurrentgemma_amd import _lib
 from recurrentgemma_amd import ops
+from tests import test_gpu_core_f32_wide as core_f32
 from tests import test_gpu_scan_tiles as one_pass
 from tests import test_gpu_training as trained
 
@@ -44,6 +45,14 @@ def test_plain_recurrence(dtype, B, T, W, with_state):
 def test_gated_recurrence(dtype, B, T, W, H):
   assert _dealt(B, T, W, dtype, 3)
   trained._rglru_against_float64(dtype, B, T, W, H, DEV)
+
+
+@pytest.mark.parametrize("B,T,H,mean_doc,joined,with_h0,with_conv", [
+    (1, 2049, 2, 200, True, True, True), (2, 2303, 1, 0, False, False, True),
+    (1, 2560, 3, 60, True, False, False)])
+def test_core_of_float32(B, T, H, mean_doc, joined, with_h0, with_conv):
+  assert _dealt(B, T, 256 * H, F32, 2)
+  core_f32.test_against_the_oracle(B, T, H, mean_doc, joined, with_h0, with_conv)
 
 
 def _inputs(B, T, W, dtype, seed):
