@@ -361,8 +361,14 @@ conv1d_prefill_k4_kernel(const T* __restrict__ x, const void* __restrict__ segpo
 // dw), a window of dout[m .. m+3] slides ahead of it (for dx), with the starts
 // of rows m+1 .. m+3 deciding which of them a tap may use.  Sums for dw and
 // dbias go to the chunk's plane of `partial` like the general kernel's.
-template <typename T>
-__global__ void __launch_bounds__(64)
+//
+// A chunk's rows are shared by the WAVES waves of a workgroup, whose sums meet in LDS.
+// What bounds it: a wave waits for its batch of rows, then works on it, and its
+// registers (200) leave no room for the next batch; so the waves of a CU have to
+// cover each other, of which one a chunk makes five (B4 T2048 W2560 bf16).  Figures
+// beside the launch.
+template <typename T, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
 conv1d_backward_k4_kernel(const T* __restrict__ dout, const T* __restrict__ x,
                           const void* __restrict__ segpos, int seg_kind,
                           const T* __restrict__ w, T* __restrict__ dx,
@@ -371,114 +377,148 @@ conv1d_backward_k4_kernel(const T* __restrict__ dout, const T* __restrict__ x,
                           int64_t M, int rows) {
   using V = Vec16<T>;
   constexpr int N = V::N;
-  const int c = ((int)blockIdx.y * 64 + (int)threadIdx.x) * N;
-  if (c >= W) return;
-  const int64_t m0 = (int64_t)blockIdx.x * rows;
-  const int64_t m1 = m0 + rows < M ? m0 + rows : M;
-  const SeqStarts seq(m0 >= 3 ? m0 - 3 : 0, T_len, rows + 6);
-  auto row = [&](const T* base, int64_t m) {
-    return *reinterpret_cast<const u32x4*>(base + m * W + c);
-  };
-  // a row behind the last one counts as a start (nothing beyond it is used)
-  auto starts = [&](int64_t m) {
-    return m >= M || conv_row_starts(segpos, seg_kind, seq, m);
-  };
-  float w0[N], w1[N], w2[N], w3[N];
-  V::unpack(row(w, 0), w0);
-  V::unpack(row(w, 1), w1);
-  V::unpack(row(w, 2), w2);
-  V::unpack(row(w, 3), w3);
-  float h1[N], h2[N], h3[N], d0[N], d1[N], d2[N], d3[N], db[N], dxs[N];
+  __shared__ float others[WAVES > 1 ? WAVES - 1 : 1][WAVES > 1 ? 6 * N : 1][64];
+  const int lane = (int)threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int c = ((int)blockIdx.y * 64 + lane) * N;
+  if (WAVES == 1 && c >= W) return;
+  const int share = rows / WAVES;
+  const int64_t m0 = (int64_t)blockIdx.x * rows + wave * share;
+  const int64_t m1 = m0 + share < M ? m0 + share : M;
+  float d0[N], d1[N], d2[N], d3[N], db[N], dxs[N];
 #pragma unroll
   for (int e = 0; e < N; ++e)
-    h1[e] = h2[e] = h3[e] = d0[e] = d1[e] = d2[e] = d3[e] = db[e] = dxs[e] = 0.0f;
-  for (int64_t j = m0 - 3; j < m0; ++j) {
-    if (j < 0) continue;
-    if (conv_row_starts(segpos, seg_kind, seq, j)) {
+    d0[e] = d1[e] = d2[e] = d3[e] = db[e] = dxs[e] = 0.0f;
+  if (WAVES == 1 || (c < W && m0 < M)) {
+    const SeqStarts seq(m0 >= 3 ? m0 - 3 : 0, T_len, share + 6);
+    auto row = [&](const T* base, int64_t m) {
+      return *reinterpret_cast<const u32x4*>(base + m * W + c);
+    };
+    // a row behind the last one counts as a start (nothing beyond it is used)
+    auto starts = [&](int64_t m) {
+      return m >= M || conv_row_starts(segpos, seg_kind, seq, m);
+    };
+    float w0[N], w1[N], w2[N], w3[N];
+    V::unpack(row(w, 0), w0);
+    V::unpack(row(w, 1), w1);
+    V::unpack(row(w, 2), w2);
+    V::unpack(row(w, 3), w3);
+    float h1[N], h2[N], h3[N];
 #pragma unroll
-      for (int e = 0; e < N; ++e) h1[e] = h2[e] = 0.0f;
+    for (int e = 0; e < N; ++e) h1[e] = h2[e] = h3[e] = 0.0f;
+    for (int64_t j = m0 - 3; j < m0; ++j) {
+      if (j < 0) continue;
+      if (conv_row_starts(segpos, seg_kind, seq, j)) {
+#pragma unroll
+        for (int e = 0; e < N; ++e) h1[e] = h2[e] = 0.0f;
+      }
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        h3[e] = h2[e];
+        h2[e] = h1[e];
+      }
+      V::unpack(row(x, j), h1);
     }
+    // g0 = dout[m], g1 .. g3 the rows after it; f1 .. f3: those rows start
+    float g0[N], g1[N], g2[N], g3[N];
+    bool f1, f2, f3;
+    auto dout_row = [&](int64_t m, float (&v)[N]) {
+      if (m < M) {
+        V::unpack(row(dout, m), v);
+      } else {
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
-      h3[e] = h2[e];
-      h2[e] = h1[e];
-    }
-    V::unpack(row(x, j), h1);
-  }
-  // g0 = dout[m], g1 .. g3 the rows after it; f1 .. f3: those rows start
-  float g0[N], g1[N], g2[N], g3[N];
-  bool f1, f2, f3;
-  auto dout_row = [&](int64_t m, float (&v)[N]) {
-    if (m < M) {
-      V::unpack(row(dout, m), v);
-    } else {
+        for (int e = 0; e < N; ++e) v[e] = 0.0f;
+      }
+    };
+    dout_row(m0, g0);
+    dout_row(m0 + 1, g1);
+    dout_row(m0 + 2, g2);
+    f1 = starts(m0 + 1);
+    f2 = starts(m0 + 2);
+    for (int64_t mb = m0; mb < m1; mb += kConvBatch) {
+      u32x4 xr[kConvBatch], gr[kConvBatch];
+      bool st[kConvBatch], fa[kConvBatch];
 #pragma unroll
-      for (int e = 0; e < N; ++e) v[e] = 0.0f;
-    }
-  };
-  dout_row(m0, g0);
-  dout_row(m0 + 1, g1);
-  dout_row(m0 + 2, g2);
-  f1 = starts(m0 + 1);
-  f2 = starts(m0 + 2);
-  for (int64_t mb = m0; mb < m1; mb += kConvBatch) {
-    u32x4 xr[kConvBatch], gr[kConvBatch];
-    bool st[kConvBatch], fa[kConvBatch];
+      for (int u = 0; u < kConvBatch; ++u) {
+        const int64_t m = mb + u < m1 ? mb + u : m1 - 1;
+        xr[u] = row(x, m);
+        gr[u] = row(dout, m + 3 < M ? m + 3 : M - 1);
+        st[u] = conv_row_starts(segpos, seg_kind, seq, m);
+        fa[u] = starts(m + 3);
+      }
 #pragma unroll
-    for (int u = 0; u < kConvBatch; ++u) {
-      const int64_t m = mb + u < m1 ? mb + u : m1 - 1;
-      xr[u] = row(x, m);
-      gr[u] = row(dout, m + 3 < M ? m + 3 : M - 1);
-      st[u] = conv_row_starts(segpos, seg_kind, seq, m);
-      fa[u] = starts(m + 3);
-    }
+      for (int u = 0; u < kConvBatch; ++u) {
+        const int64_t m = mb + u;
+        if (m < m1) {
+          if (m + 3 < M) {
+            V::unpack(gr[u], g3);
+          } else {
 #pragma unroll
-    for (int u = 0; u < kConvBatch; ++u) {
-      const int64_t m = mb + u;
-      if (m < m1) {
-        if (m + 3 < M) {
-          V::unpack(gr[u], g3);
-        } else {
+            for (int e = 0; e < N; ++e) g3[e] = 0.0f;
+          }
+          f3 = fa[u];
+          if (st[u]) {
 #pragma unroll
-          for (int e = 0; e < N; ++e) g3[e] = 0.0f;
+            for (int e = 0; e < N; ++e) h1[e] = h2[e] = h3[e] = 0.0f;
+          }
+          float cur[N], o[N];
+          V::unpack(xr[u], cur);
+          const bool ok1 = !f1, ok2 = ok1 && !f2, ok3 = ok2 && !f3;
+#pragma unroll
+          for (int e = 0; e < N; ++e) {
+            float acc = w3[e] * g0[e];
+            acc = __builtin_fmaf(w2[e], ok1 ? g1[e] : 0.0f, acc);
+            acc = __builtin_fmaf(w1[e], ok2 ? g2[e] : 0.0f, acc);
+            acc = __builtin_fmaf(w0[e], ok3 ? g3[e] : 0.0f, acc);
+            o[e] = acc;
+            d3[e] = __builtin_fmaf(cur[e], g0[e], d3[e]);  // w[3] meets x[t]
+            d2[e] = __builtin_fmaf(h1[e], g0[e], d2[e]);
+            d1[e] = __builtin_fmaf(h2[e], g0[e], d1[e]);
+            d0[e] = __builtin_fmaf(h3[e], g0[e], d0[e]);
+            db[e] += g0[e];
+            h3[e] = h2[e];
+            h2[e] = h1[e];
+            h1[e] = cur[e];
+            g0[e] = g1[e];
+            g1[e] = g2[e];
+            g2[e] = g3[e];
+          }
+          f1 = f2;
+          f2 = f3;
+          const u32x4 packed = V::pack(o);
+          *reinterpret_cast<u32x4*>(dx + m * W + c) = packed;
+          // (of what is stored: the bias gradient of the layer in front)
+          V::unpack(packed, o);
+#pragma unroll
+          for (int e = 0; e < N; ++e) dxs[e] += o[e];
         }
-        f3 = fa[u];
-        if (st[u]) {
-#pragma unroll
-          for (int e = 0; e < N; ++e) h1[e] = h2[e] = h3[e] = 0.0f;
-        }
-        float cur[N], o[N];
-        V::unpack(xr[u], cur);
-        const bool ok1 = !f1, ok2 = ok1 && !f2, ok3 = ok2 && !f3;
-#pragma unroll
-        for (int e = 0; e < N; ++e) {
-          float acc = w3[e] * g0[e];
-          acc = __builtin_fmaf(w2[e], ok1 ? g1[e] : 0.0f, acc);
-          acc = __builtin_fmaf(w1[e], ok2 ? g2[e] : 0.0f, acc);
-          acc = __builtin_fmaf(w0[e], ok3 ? g3[e] : 0.0f, acc);
-          o[e] = acc;
-          d3[e] = __builtin_fmaf(cur[e], g0[e], d3[e]);  // w[3] meets x[t]
-          d2[e] = __builtin_fmaf(h1[e], g0[e], d2[e]);
-          d1[e] = __builtin_fmaf(h2[e], g0[e], d1[e]);
-          d0[e] = __builtin_fmaf(h3[e], g0[e], d0[e]);
-          db[e] += g0[e];
-          h3[e] = h2[e];
-          h2[e] = h1[e];
-          h1[e] = cur[e];
-          g0[e] = g1[e];
-          g1[e] = g2[e];
-          g2[e] = g3[e];
-        }
-        f1 = f2;
-        f2 = f3;
-        const u32x4 packed = V::pack(o);
-        *reinterpret_cast<u32x4*>(dx + m * W + c) = packed;
-        // (of what is stored: the bias gradient of the layer in front)
-        V::unpack(packed, o);
-#pragma unroll
-        for (int e = 0; e < N; ++e) dxs[e] += o[e];
       }
     }
+  }
+  if constexpr (WAVES > 1) {
+    auto meet = [&](int i, float (&v)[N]) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        if (wave > 0) {
+          others[wave - 1][i * N + e][lane] = v[e];
+        } else {
+#pragma unroll
+          for (int k = 0; k < WAVES - 1; ++k) v[e] += others[k][i * N + e][lane];
+        }
+      }
+    };
+    auto meet_all = [&]() {
+      meet(0, d0);
+      meet(1, d1);
+      meet(2, d2);
+      meet(3, d3);
+      meet(4, db);
+      meet(5, dxs);
+    };
+    if (wave > 0) meet_all();
+    __syncthreads();
+    if (wave > 0 || c >= W) return;
+    meet_all();
   }
   if (dx_sums != nullptr) {
 #pragma unroll
@@ -648,18 +688,27 @@ hipError_t launch_conv1d_backward(const ConvBwdArgs& a, int dtype,
     return hipErrorInvalidValue;
   if (dtype == 0 ? conv_k4_fits<float>(a.K, a.W, M)
                  : conv_k4_fits<uint16_t>(a.K, a.W, M)) {
-    if (dtype == 0)
-      conv1d_backward_k4_kernel<float>
-          <<<dim3((unsigned)chunks, (unsigned)((a.W / 4 + 63) / 64)), 64, 0, s>>>(
-              (const float*)a.dout, (const float*)a.x, a.segpos, a.seg_kind,
-              (const float*)a.w, (float*)a.dx, a.partial, a.dx_sums, a.T, a.W, M,
-              rows);
-    else
-      conv1d_backward_k4_kernel<uint16_t>
-          <<<dim3((unsigned)chunks, (unsigned)((a.W / 8 + 63) / 64)), 64, 0, s>>>(
-              (const uint16_t*)a.dout, (const uint16_t*)a.x, a.segpos,
-              a.seg_kind, (const uint16_t*)a.w, (uint16_t*)a.dx, a.partial,
-              a.dx_sums, a.T, a.W, M, rows);
+    // waves of a chunk: as many as there is room for on the CUs (us, one / two / four:
+    // bf16 B1 T300 W2560 26 / 17 / 12, B2 T1000 W4096 30 / 23 / 18, B4 T2048 W2560
+    // 40 / 43 / 42, B8 T2048 W4096 108 / 115 / 126; float32 19 / 12 / 8, 23 / 20 / 23,
+    // 49 / 47 / 48)
+    auto run = [&](auto* tag, auto waves) {
+      typedef std::remove_pointer_t<decltype(tag)> T;
+      constexpr int w = decltype(waves)::value;
+      conv1d_backward_k4_kernel<T, w>
+          <<<dim3((unsigned)chunks, (unsigned)((a.W / Vec16<T>::N + 63) / 64)), 64 * w,
+             0, s>>>((const T*)a.dout, (const T*)a.x, a.segpos, a.seg_kind,
+                     (const T*)a.w, (T*)a.dx, a.partial, a.dx_sums, a.T, a.W, M, rows);
+    };
+    auto pick = [&](auto* tag) {
+      typedef std::remove_pointer_t<decltype(tag)> T;
+      const int64_t blocks = chunks * ((a.W / Vec16<T>::N + 63) / 64);
+      if (blocks <= 512) run(tag, std::integral_constant<int, 4>{});
+      else if (blocks <= 1024) run(tag, std::integral_constant<int, 2>{});
+      else run(tag, std::integral_constant<int, 1>{});
+    };
+    if (dtype == 0) pick((float*)nullptr);
+    else pick((uint16_t*)nullptr);
     return hipGetLastError();
   }
   if (a.dx_sums != nullptr) return hipErrorInvalidValue;
