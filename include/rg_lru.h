@@ -210,7 +210,9 @@ int rg_rglru_backward(const void* dy, const void* x, const void* gx_pre,
  * that gain nothing (then the calls behave exactly like the plain ones and
  * workspace may be null); otherwise workspace (16-byte aligned, that many
  * bytes) is required.  Same arguments and results otherwise (fp32 1e-5, the
- * float32 state is combined in a different order). */
+ * float32 state is combined in a different order).  With B * W * 16 + W * 8 + 16
+ * bytes or more, and few long rows, rg_linear_scan_split hands the state from
+ * workgroup to workgroup instead and reads once. */
 size_t rg_scan_split_workspace_bytes(int B, int T, int W);
 int rg_lru_scan_fused_split(const void* x, int apply_conv, const void* conv_w,
                             const void* conv_b, const void* gx_pre,
@@ -318,7 +320,10 @@ int rg_recurrent_prefill_gelu_mul(
  * rg_gelu_mul over `out` as a last launch), else the plain RG-LRU output.  `workspace` (16-byte aligned)
  * must hold rg_recurrent_core_workspace_bytes(B, T, W, H, dtype) bytes (0 for
  * whole rows in the single kernel: workspace may then be null).  Same values
- * as the calls it is made of (float32 with 256-wide heads: to rounding); h0 / h_last / conv_cache_out / w_packed as in
+ * as the calls it is made of (float32 with 256-wide heads: to rounding; so are bf16
+ * rows with 256-wide heads that do not come out even on the CUs where the workspace
+ * has B * W * 16 + H * 4 bytes or more, padded to 16: blocks of 32 tokens, whose
+ * states go from workgroup to workgroup through it); h0 / h_last / conv_cache_out / w_packed as in
  * rg_recurrent_prefill (w_packed is only read by the single kernel).
  * conv_w == conv_b == NULL (conv_cache_out then NULL too): x is the conv
  * output already, and the call is RGLRU.forward on its own
