@@ -14,12 +14,14 @@
 //     the wave are joined, and as soon as the incoming state h is there the state
 //     behind the block, P h + H, goes out to the next one: one multiply-add between
 //     receiving and passing on.  Then the tokens are replayed from h;
-//   * a state is one 8-byte word per channel, value and block number, written with an
-//     agent-scope store of the whole word and polled by agent-scope loads into LDS: no
-//     fence, no flag apart.  (A load into a register on one of two paths makes the
-//     compiler wait for all loads and stores on both.)  Two words per row and channel
-//     are enough: the word of block t - 2 has been read when the state of block t - 1
-//     arrives.
+//   * a state is one 8-byte word per channel: each of its halves has 16 bits of the
+//     value and the 16 low bits of the block's number, written with an agent-scope
+//     store of the whole word and polled by agent-scope loads into LDS, four bytes a
+//     lane: a half vouches for itself, so it does not matter that two lanes fetch a
+//     word; no fence, no flag apart.  (A load into a register on one of two paths, or
+//     one for some lanes only, makes the compiler wait for loads and stores it need
+//     not wait for.)  Two words per row and channel are enough: the word of block
+//     t - 2 has been read when the state of block t - 1 arrives.
 // Every wait ends: a workgroup takes tickets in order and works on them in order, a
 // block waits only for a block of a smaller ticket (and its team's earlier phases),
 // and a ticket is taken only by a workgroup that runs, however many of them do.
@@ -331,7 +333,9 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
   u32x4 y_pending[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
   int y_row = 0;  // where they belong
   uint32_t y_pending_row = kBufferOutOfRange;
-  // states between blocks: [B][2][W] words, value and block number + 1
+  // states between blocks: [B][2][W] words.  Block t leaves its number + 1 in both
+  // halves, mod 2^16: what it replaces has t - 1 there, or the zeros from before the
+  // first two blocks
   // (lane-dependent addresses of phase G are made where they are used, out of the
   // compiler's sight: kept across phase M they are registers too many)
   auto lane_channel = [&]() {
@@ -342,6 +346,10 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
   auto word_at = [&](int b, int t) {
     return p.relay_words + ((int64_t)b * 2 + (t & 1)) * W + h * kBW + n0 +
            lane_channel();
+  };
+  auto word_of = [](float value, int t) {
+    const uint32_t v = __float_as_uint(value), number = (uint32_t)(t + 1) & 0xffffu;
+    return (uint64_t)(v << 16 | number) << 32 | (v & 0xffff0000u) | number;
   };
   // the words that come into a block, into LDS (four bytes a lane)
   auto fetch_words = [&](const Place& q, int slot) {
@@ -470,13 +478,18 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
     // for again now and behind the gates, and then until it is, two polls in flight.
     // (All of it by way of LDS: a load into registers on one of two paths makes the
     // compiler wait for everything on both.)
-    uint64_t word = 0;
+    uint32_t state = 0;
     auto arrived = [&](int slot) {
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      word = *reinterpret_cast<lds_u64*>(lds3 + kWordOff + wave * kWordBytesPerWave +
-                                         slot * kWordBytes + 8 * lane_channel());
-      return (bool)__all((uint32_t)(word >> 32) == (uint32_t)q.t);  // block before
+      const uint64_t word =
+          *reinterpret_cast<lds_u64*>(lds3 + kWordOff + wave * kWordBytesPerWave +
+                                      slot * kWordBytes + 8 * lane_channel());
+      const uint32_t low = (uint32_t)word, high = (uint32_t)(word >> 32);
+      state = __builtin_amdgcn_perm(low, high, 0x07060302u);
+      // both halves from the block before
+      return (bool)__all(__builtin_amdgcn_perm(low, high, 0x05040100u) ==
+                         ((uint32_t)q.t & 0xffffu) * 0x10001u);
     };
     wait_vmcnt<GELU ? 9 : 7>();
     bool there = q.t == 0 || arrived(0);
@@ -522,13 +535,13 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
         wait_vmcnt<1>();
         if (arrived(polls & 1)) break;
         if (polls == kMaxPolls) {
-          word = 0x7fc00000u;
+          state = 0x7fc00000u;
           break;
         }
         fetch_words(q, polls & 1);
       }
     }
-    float h_in = __uint_as_float((uint32_t)word);
+    float h_in = __uint_as_float(state);
     if (q.t == 0)
       h_in = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
           state_row(p.h0, q.b), 4u * lane_channel(), 0, 0));
@@ -537,10 +550,8 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
     const float h_out = __builtin_fmaf(p_up, h_mid, e_up);
     if (!upper) {
       if (q.t + 1 < blocks)
-        __hip_atomic_store(word_at(q.b, q.t),
-                           ((uint64_t)(uint32_t)(q.t + 1) << 32) |
-                               __float_as_uint(h_out),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(word_at(q.b, q.t), word_of(h_out, q.t), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
       else  // (no descriptor, no store)
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(h_out),
                                               state_row(p.h_last, q.b),

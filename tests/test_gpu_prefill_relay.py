@@ -92,6 +92,41 @@ def test_against_the_oracle():
   assert helpers.max_rel(y.cpu().float(), yo) < 3e-2
 
 
+def test_halves_of_a_state_word_vouch_for_themselves():
+  """Two lanes fetch a word, four bytes each: each half has to say by itself which
+  block it is from.  The words a call leaves in its workspace, and the states in
+  them: those that a call ends with whose rows end there."""
+  B, T, H = 40, 1056, 1
+  W = 256 * H
+  _, (x, seg, cw, cb, wx, bx, wa, ba, ap), kw = _case(B, T, H, 90, True, False)
+  lib = _lib.lib()
+  packed = ops.packed_gate_weights(wx, wa)
+  ends = {}
+  for n in (T, 1024):
+    xn, sn = x[:, :n].contiguous(), seg[:, :n].contiguous()
+    gate = kw["gate_branch"][:, :n].contiguous()
+    need = lib.rg_recurrent_core_best_workspace_bytes(B, n, W, H, 1)
+    assert need >= B * 2 * W * 8
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    y, h = torch.empty_like(xn), torch.empty(B, W, device=DEV)
+    ptr = lambda t: None if t is None else t.data_ptr()
+    _lib.check(lib.rg_recurrent_core(
+        *map(ptr, (xn, gate, sn)), 0, *map(ptr, (
+            cw, cb, wx, bx, wa, ba, packed, ap, None, y, h, None, ws)), need, B, n, W,
+        H, 1, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    ends[n] = h, ws[:B * 2 * W * 8].cpu().view(torch.int32).view(B, 2, W, 2)
+  # 33 blocks: the last word is block 31's, the state behind 1024 tokens; the other
+  # one is block 30's
+  low, high = (ends[T][1][..., i].to(torch.int64) & 0xffffffff for i in range(2))
+  for block in (31, 30):
+    assert bool((low[:, block & 1] & 0xffff == block + 1).all())
+    assert bool((high[:, block & 1] & 0xffff == block + 1).all())
+  bits = (low[:, 1] & 0xffff0000) | high[:, 1] >> 16
+  want = ends[1024][0].cpu().view(torch.int32).to(torch.int64) & 0xffffffff
+  assert torch.equal(bits, want)
+
+
 def test_rows_apart():
   """NaN and infinities in one row's input or state stay in that row."""
   _, args, kw = _case(40, 1000, 1, 90, True, True)
