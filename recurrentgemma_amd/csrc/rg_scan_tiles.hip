@@ -66,9 +66,13 @@ __device__ __forceinline__ float choose(bool cond, float a, float b) {
 // rounded square would keep few of its digits, -2q (ln 2 + 2q (ln 2)^2 / 2! + ..),
 // eight terms of the exponential's series (the ninth is 2e-8 of the first).  With
 // it the float32 forms can use the hardware's exp2, reciprocal and square root
-// (RG-LRU step B3 T1001 W2560: 254 -> 238 us against expf, sqrtf and divisions)
-// and are closer to 64 bits (y 1.9e-7 -> 1.2e-7, its gradients 2.2e-7 .. 4.0e-7
-// -> 1.4e-7 .. 2.4e-7, the projections' part of that included).
+// (RG-LRU step B3 T1001 W2560: 254 -> 240 us against expf, sqrtf and divisions;
+// sigmoids: sigmoid_f32).  Errors against 64 bits, projections included, before and
+// now: gates around 0 y 1.0e-7 .. 1.6e-7 -> 7.2e-8 .. 1.2e-7, gradients 1.5e-7 ..
+// 3.3e-7 -> 1.0e-7 .. 2.1e-7; input gates at -12 .. -8 y 4.0e-7 -> 3.4e-7; recurrence
+// gates there y 4e-5 -> 6e-7.  Of this kernel alone (exact pre-activations): y and the
+// gradients of x and the input gate as before, the recurrence gate's bias up to 1.1
+// times (1.7e-7 -> 1.9e-7).
 __device__ __forceinline__ float one_minus_square(float q, float a) {
   constexpr float kSeries[8] = {0.69314718056f,    0.24022650696f,
                                 5.5504108665e-2f,  9.6181291076e-3f,
@@ -160,8 +164,8 @@ scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
   constexpr int NS = streams_of(MODE);
   constexpr bool kBwd = MODE == kBwdPlain || MODE == kBwdGated;
   constexpr bool kGated = MODE == kFwdGated || MODE == kBwdGated;
-  // (both types: the hardware's exp2, reciprocal and square root; float32 forms
-  // 1 - a^2 without the cancellation, see below)
+  // (both types: the hardware's exp2, reciprocal and square root; float32 1 - a^2
+  // without the cancellation and sigmoids without the exponent's rounding)
   constexpr bool kFast = sizeof(T) == 2;
   constexpr bool kBias = kGated && !kFast;
   constexpr int kSegs = kThreads / CH;    // scanning threads of a channel
@@ -379,6 +383,9 @@ scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
       for (int e = 0; e < N; ++e) v[e] += b_[e];
     }
   };
+  auto sigmoid_of = [](float v) __attribute__((always_inline)) {
+    return kFast ? sigmoid_fast(v) : sigmoid_f32(v);
+  };
   // 1 - a^2 with a = 2^q
   auto rest_of = [](float q, float a) __attribute__((always_inline)) {
     return kFast ? __builtin_fmaf(-a, a, 1.0f) : one_minus_square(q, a);
@@ -537,13 +544,13 @@ scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
         }
 #pragma unroll
         for (int e = 0; e < N; ++e) {
-          const float gate_a = sigmoid_fast(ga[e]);
+          const float gate_a = sigmoid_of(ga[e]);
           const float log2_a = gate_a * ((-8.0f * kLog2e) * sp[e]);
           coef[i][e] = __builtin_amdgcn_exp2f(log2_a);
           cf[e] = coef[i][e];
           if constexpr (kKeepGate) kept[i][e] = gate_a;
           if constexpr (MODE == kFwdGated) {
-            const float gate_x = sigmoid_fast(gx[e]);
+            const float gate_x = sigmoid_of(gx[e]);
             const float m = choose(
                 start, 1.0f, __builtin_amdgcn_sqrtf(rest_of(log2_a, coef[i][e])));
             first[e] = (first[e] * gate_x) * m;
@@ -748,12 +755,12 @@ scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
 #pragma unroll
           for (int e = 0; e < N; ++e) {
             const float a = coef[i][e];
-            const float gate_a = kKeepGate ? kept[kKeepGate ? i : 0][e] : sigmoid_fast(pa[e]);
+            const float gate_a = kKeepGate ? kept[kKeepGate ? i : 0][e] : sigmoid_of(pa[e]);
             const float c_t =
                 choose(start, 0.0f, choose(t >= T_len, 1.0f, a));
             st[e] = c_t * g[e];
             const float gr = round_act<T>(g[e]);  // the gradient of xn as a tensor
-            const float gate_x = sigmoid_fast(px[e]);
+            const float gate_x = sigmoid_of(px[e]);
             const float om =
                 kFast ? 1.0f - a * a
                       : one_minus_square(gate_a * ((-8.0f * kLog2e) * sp[e]), a);

@@ -56,3 +56,85 @@ def test_plain_recurrence(dtype, B, T, W, with_state):
   # run to run the same bits, and the inference call's
   y2, h2 = ops.linear_scan(x, a, reset, h0)
   assert torch.equal(y2, y) and torch.equal(h2, h)
+
+
+def _gated(x, gate_x, gate_a, a_param):
+  """y of the RG-LRU from pre-activations [W], in float64."""
+  log_a = -8.0 * torch.sigmoid(gate_a) * torch.nn.functional.softplus(a_param)
+  a, m = torch.exp(log_a), torch.sqrt(-torch.expm1(2 * log_a))
+  state, ys = torch.zeros_like(x[:, 0]), []
+  for t in range(x.shape[1]):
+    xn = x[:, t] * torch.sigmoid(gate_x)
+    state = a * state + m * xn if t else xn
+    ys.append(state)
+  return torch.stack(ys, 1)
+
+
+def _layer(width, heads, gate_x, gate_a, softplus):
+  """A float32 layer whose pre-activations are its biases."""
+  layer = rg.RGLRU(width=width, num_heads=heads, device=DEV, dtype=torch.float32)
+  with torch.no_grad():
+    layer.a_param.fill_(softplus).expm1_().log_()
+    for gate, bias in ((layer.input_gate, gate_x), (layer.a_gate, gate_a)):
+      gate.w.zero_()
+      gate.b.copy_(bias.view_as(gate.b))
+  return layer
+
+
+@pytest.mark.parametrize("low,high", [(-1, 1), (-6, -3), (-12, -8), (-25, -15), (3, 12)])
+@pytest.mark.parametrize("native", [True, False])
+def test_float32_gates_far_from_zero(low, high, native):
+  """A sigmoid of float32 is as good where it is small as elsewhere: y and dx within
+  2^-23 of their norm.  A term of y is x gate m, two products of 2^-24 each at most,
+  and gate and m are off by about one unit in the last place, 2^-24 at most and half
+  of that in the mean: together 2^-24 in the mean square.  (a is 0.02 here: nothing
+  adds up over time.)"""
+  B, T, W, heads = 3, 130, 512, 2
+  g = torch.Generator(device=DEV).manual_seed(7)
+  uniform = lambda lo, hi: lo + (hi - lo) * torch.rand(W, generator=g, device=DEV)
+  gate_x, gate_a = uniform(low, high), uniform(-1, 1)
+  layer = _layer(W, heads, gate_x, gate_a, 1.0)
+  x = torch.randn(B, T, W, generator=g, device=DEV)
+  dy = torch.randn(B, T, W, generator=g, device=DEV)
+  pos = torch.arange(T, device=DEV, dtype=torch.int32).repeat(B, 1)
+  xd = x.double().requires_grad_()
+  want = _gated(xd, gate_x.double(), gate_a.double(), layer.a_param.detach().double())
+  if native:
+    x.requires_grad_()
+    with training.differentiable():
+      y, _ = layer(x, pos, return_cache=False)
+    pairs = [(y, want)] + list(zip(torch.autograd.grad(y, x, dy),
+                                   torch.autograd.grad(want, xd, dy.double())))
+  else:  # a prompt pass by several launches
+    x, pos, want = (t.repeat(6, 1, 1)[..., :T, :] if t.dim() == 3 else t.repeat(6, 1)
+                    for t in (x, pos, want))
+    y, _, _ = ops.recurrent_core(
+        x, pos, None, None, layer.input_gate.w.detach(), layer.input_gate.b.detach(),
+        layer.a_gate.w.detach(), layer.a_gate.b.detach(), layer.a_param.detach())
+    pairs = [(y, want)]
+  for got, exact in pairs:
+    assert (got.double() - exact).norm() <= 2.0**-23 * exact.norm()
+
+
+def test_float32_gates_beyond_range():
+  """Pre-activations that saturate a gate, infinite ones among them, and NaN, which
+  stays in its channel."""
+  B, T, W = 2, 70, 256
+  values = [float("inf"), 1e30, 200.0, 89.0, -89.0, -200.0, -1e30, -float("inf")]
+  gate_x = torch.zeros(W, device=DEV)
+  gate_x[:8] = torch.tensor(values)
+  gate_a = torch.zeros(W, device=DEV)
+  gate_a[8:16] = torch.tensor(values)
+  gate_x[16], gate_a[17] = float("nan"), float("nan")
+  layer = _layer(W, 1, gate_x, gate_a, 1.0)
+  x = torch.randn(B, T, W, device=DEV)
+  pos = torch.arange(T, device=DEV, dtype=torch.int32).repeat(B, 1)
+  with training.differentiable():
+    y, _ = layer(x, pos, return_cache=False)
+  want = _gated(x.double(), gate_x.double(), gate_a.double(),
+                layer.a_param.detach().double())
+  assert bool(y[..., 16].isnan().all()) and bool(y[:, 1:, 17].isnan().all())
+  keep = [c for c in range(W) if c not in (16, 17)]
+  assert bool(torch.isfinite(y[..., keep]).all())
+  # (e^-89 is below float32's normal numbers: 2^-126 of x)
+  assert float((y.detach()[..., keep].double() - want[..., keep]).abs().max()) <= 1e-6
