@@ -6,14 +6,24 @@
 //   weights   dw_g[h, i, j] = sum_m x[m, h, i] dy_g[m, h, j]
 //
 // Every operand is cut into three bf16 pieces, each the nearest bf16 to what the
-// pieces before it leave (v = hi + mid + lo to 2^-27 of v), and a product is the
-// six products of pieces that weigh 2^-16 or more: what is left out, mid lo, lo
-// mid and lo lo, is below 2^-26 of it.  v_mfma_f32_32x32x16_bf16 multiplies
+// pieces before it leave (v = hi + mid + lo: three times eight bits, all of a
+// float32), and a product is the six products of pieces that weigh 2^-16 or more: what
+// is left out, mid lo, lo mid and lo lo, is below 2^-26 of it.  v_mfma_f32_32x32x16_bf16 multiplies
 // exactly and adds in float32; hi hi has an accumulator of its own, the five
 // others share one whose roundings are 2^-8 times smaller, so a chain of K / 16
 // roundings counts where the float32 instruction (32x32x2) has K / 2.  Six of
 // them take 192 cycles for what eight of the others need 512, and vector
 // instructions issue beside them.
+//
+// A piece has float32's range of exponents, so the last one of a value below 2^-110 =
+// 8e-34 is no normal number any more and, further down, loses its digits.  Gradients
+// (and x, where it meets them) are therefore cut 2^24 times as large, which makes every
+// piece of every normal float32 a normal number or zero, and the results are scaled
+// back, both exactly: dx of gradients of 1e-35 was off by 6e-6 of its norm and is as
+// good as others now.  x and weights in the forward products and weights behind
+// gradients are cut as they are: what they would gain lies 1e-34 below the bias, or the
+// other share of dx, that it is added to.  (These scaled as well: float32 prefill of 8 x
+// 2048 tokens, 2560 wide, 532 -> 539 us; as it is the kernels take what they took.)
 //
 // A workgroup of four waves owns 128 x 128 results, a wave 64 x 64 of them (two
 // accumulators for each: half of its registers).  A stage is 16 k: its 2 x 128 x
@@ -40,9 +50,9 @@
 // errors: forward 8.9e-8 / 2.1e-7, data 1.1e-7 / 2.4e-7, weights 7.7e-8 / 1.3e-7
 // at 512 rows and 2.2e-7 / 4.7e-7 at 8192.
 //
-// Infinities and NaN: a piece of an infinity is no number, and products of
-// pieces may overflow where the product does not.  Either leaves something that
-// is not finite among a wave's results; such a wave computes them again with the
+// Infinities and NaN: a piece of an infinity is no number, and scaled operands (from
+// 2^104 = 2e31 on) or products of pieces (scaled: from 2^80 = 1e24 on) may overflow
+// where the product does not.  Either leaves something that is not finite among a wave's results; such a wave computes them again with the
 // float32 instruction and takes those for what was not finite (the others keep
 // their bits whatever their neighbours hold).
 #include <type_traits>
@@ -100,6 +110,7 @@ struct Source {
 struct Pieces {
   u32x4 hi, mid, lo;  // eight k
 };
+constexpr float kScale = 0x1p24f;
 
 __device__ __forceinline__ void cut(const float (&v)[8], Pieces& p) {
 #pragma unroll
@@ -116,7 +127,7 @@ __device__ __forceinline__ void cut(const float (&v)[8], Pieces& p) {
 }
 
 // A thread's share of one operand's stage: eight k of a row.
-template <class S, bool ALONG_K>
+template <class S, bool ALONG_K, bool SCALED>
 struct Share {
   float v[8];
 
@@ -153,8 +164,12 @@ struct Share {
       for (int k = 0; k < 8; ++k) v[k] = word(k0 + (uint32_t)k);
     }
   }
-  __device__ __forceinline__ void store(unsigned char* lds, int tid) const {
+  __device__ __forceinline__ void store(unsigned char* lds, int tid) {
     unsigned char* const at = lds + S::at(row(tid), oct(tid));
+    if (SCALED) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] *= kScale;
+    }
     Pieces p;
     cut(v, p);
     *reinterpret_cast<u32x4*>(at) = p.hi;
@@ -175,6 +190,10 @@ gates_split_f32_kernel(SplitArgs p) {
   constexpr int kTile = S::tile, kStage = S::stage;
   // operand A gives the results' rows, B their columns
   constexpr bool kAlongKA = KIND != kWeights, kAlongKB = KIND == kData;
+  // operands cut kScale times as large
+  constexpr bool kScaledA = KIND != kForward, kScaledB = KIND == kWeights;
+  constexpr float kBack = (kScaledA ? 1.0f / kScale : 1.0f) *
+                          (kScaledB ? 1.0f / kScale : 1.0f);
   __shared__ __align__(16) unsigned char lds[2 * S::buffer];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -246,8 +265,8 @@ gates_split_f32_kernel(SplitArgs p) {
   // Two stages of both operands in flight: a stage's floats are requested two
   // stages ahead and cut during the one before it, between its matrix
   // instructions.
-  Share<S, kAlongKA> sa[2];
-  Share<S, kAlongKB> sb[2];
+  Share<S, kAlongKA, kScaledA> sa[2];
+  Share<S, kAlongKB, kScaledB> sb[2];
   auto request = [&](uint32_t k, auto SLOT) {
     constexpr int slot = decltype(SLOT)::value;
     constexpr bool checked = KIND == kWeights;
@@ -340,8 +359,9 @@ gates_split_f32_kernel(SplitArgs p) {
     for (int j = 0; j < BLOCKS; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        big[i][j][r] += small[i][j][r];
-        odd = __builtin_fmaf(big[i][j][r], 0.0f, odd);
+        const float sum = big[i][j][r] + small[i][j][r];
+        odd = __builtin_fmaf(sum, 0.0f, odd);
+        big[i][j][r] = sum * kBack;
       }
   if (__builtin_expect(__any(odd != 0.0f), 0)) {
     // infinities, NaN or an overflow: the float32 instruction instead
