@@ -298,25 +298,30 @@ scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
     return DEAL ? fetch_from(rs_ahead, off_ahead, s, t0, i)
                 : fetch_from(rs, off_now, s, t0, i);
   };
-  // Document starts of the wave's 8 KL tokens, one token per lane.
-  uint32_t flag_lo = 1, flag_hi = 0;
+  // Document starts of the wave's 8 KL tokens, one token per lane.  (Loads of every
+  // kind of flag, those that it is not out of range: a branch per kind, or a comparison
+  // here, makes the wave wait for them, and for the rows asked for before, at once.)
+  const bool flag_bytes = p.flag_kind == kSegMaskU8;
+  const uint32_t flag_size = flag_bytes ? 1u : p.flag_kind == kSegI32 ? 4u : 8u;
+  uint32_t flag_lo = 0, flag_hi = 0, flag_byte = 0;
   bool flag_in = false;
   auto load_flags = [&](const Place& z) {
     const int lo = first_token(z.step, kBwd ? wave * 8 + 7 : wave * 8);
     const int t = lo + lane;
     flag_in = lane < 8 * KL && t >= 0 && t < T_len;
-    const int64_t at = (int64_t)z.b * T_len + (flag_in ? t : 0);
-    if (p.flag_kind == kSegMaskU8) {
-      flag_lo = reinterpret_cast<const uint8_t*>(p.flags)[at] == 0;
-      flag_hi = 0;
-    } else if (p.flag_kind == kSegI32) {
-      flag_lo = reinterpret_cast<const uint32_t*>(p.flags)[at];
-      flag_hi = 0;
-    } else {
-      const u32x2 v = reinterpret_cast<const u32x2*>(p.flags)[at];
-      flag_lo = v[0];
-      flag_hi = v[1];
-    }
+    const uint32_t row = (uint32_t)T_len * flag_size;  // < 2^31 (scan_tiles_take)
+    const __amdgpu_buffer_rsrc_t r =
+        make_rsrc((const char*)p.flags + (int64_t)z.b * row, row);
+    const uint32_t at = flag_in ? (uint32_t)t * flag_size : kBufferOutOfRange;
+    flag_byte = __builtin_amdgcn_raw_buffer_load_b8(
+        r, flag_bytes ? at : kBufferOutOfRange, 0, 0);
+    flag_lo = __builtin_amdgcn_raw_buffer_load_b32(
+        r, flag_bytes ? kBufferOutOfRange : at, 0, 0);
+    flag_hi = __builtin_amdgcn_raw_buffer_load_b32(
+        r, flag_size == 8u ? at + 4u : kBufferOutOfRange, 0, 0);
+  };
+  auto is_start = [&]() {
+    return flag_in && (flag_bytes ? flag_byte != 0u : (flag_lo | flag_hi) == 0u);
   };
 
   // softplus of a_param, log2 a = -8 log2(e) sp sigmoid(.): read from LDS
@@ -489,14 +494,20 @@ scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
     }
     uint32_t starts;
     {
-      const uint64_t mask = __ballot(flag_in && (flag_lo | flag_hi) == 0u);
+      const uint64_t mask = __ballot(is_start());
       starts = (uint32_t)(mask >> ((kBwd ? 7 - q : q) * KL)) & ((1u << KL) - 1u);
       if (MODE == kFwdGated && p.starts_out && now.c0 == 0 && flag_in)
         p.starts_out[(int64_t)now.b * T_len + first_token(now.step, wave * 8) + lane] =
-            (flag_lo | flag_hi) == 0u;
+            is_start();
     }
     if (more) {
       load_flags(ahead);
+      // The plain backward does wait for what it has asked for so far before it asks
+      // for the next step's rows.  Forward and backward of B4 T2048 W2560 bf16 with the
+      // rows in memory: 91.2 us, without this wait 91.7 (in the last-level cache 64.5
+      // and 63.8; both kernels waiting, as they did, 92.2 and 65.8).
+      if (MODE == kBwdPlain && !DEAL)
+        asm volatile("" : "+v"(flag_byte), "+v"(flag_lo), "+v"(flag_hi));
       if (!kReload) {
 #pragma unroll
         for (int j = 0; j < KL; ++j) {
@@ -730,10 +741,17 @@ scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
         float hp[N];
         V::unpack(raw[kY][i], hp);
         if (i == 0 && t == 0) {  // (t0 is a multiple of KL)
+          // h_{-1} in the activation dtype, 16 bytes a load and one wait
+          const __amdgpu_buffer_rsrc_t rh =
+              make_rsrc(p.h0 + (int64_t)now.b * p.W, p.h0 ? (uint32_t)p.W * 4u : 0u);
+          u32x4 h0[N / 4];
 #pragma unroll
-          for (int e = 0; e < N; ++e)  // h_{-1} in the activation dtype
-            hp[e] = p.h0 && c_ok ? round_act<T>(p.h0[(int64_t)now.b * p.W + c + e])
-                                 : 0.0f;
+          for (int e = 0; e < N; e += 4)
+            h0[e / 4] = __builtin_amdgcn_raw_buffer_load_b128(
+                rh, c_ok ? 4u * (uint32_t)(c + e) : kBufferOutOfRange, 0, 0);
+#pragma unroll
+          for (int e = 0; e < N; ++e)
+            hp[e] = round_act<T>(__uint_as_float(h0[e / 4][e & 3]));
         }
         float g[N];
 #pragma unroll

@@ -138,3 +138,26 @@ def test_float32_gates_beyond_range():
   assert bool(torch.isfinite(y[..., keep]).all())
   # (e^-89 is below float32's normal numbers: 2^-126 of x)
   assert float((y.detach()[..., keep].double() - want[..., keep]).abs().max()) <= 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [5, 257, 514])
+def test_kinds_of_document_starts(dtype, T):
+  """Positions of 32 and of 64 bits, only whole zeros of which are starts, rows that
+  begin at any byte of a mask: the same outputs and gradients."""
+  B, W, heads = 3, 256, 1
+  g = torch.Generator(device=DEV).manual_seed(T)
+  torch.manual_seed(T)
+  layer = rg.RGLRU(width=W, num_heads=heads, device=DEV, dtype=dtype)
+  x = torch.randn(B, T, W, generator=g, device=DEV).to(dtype).requires_grad_()
+  dy = torch.randn(B, T, W, generator=g, device=DEV).to(dtype)
+  starts = torch.rand(B, T, generator=g, device=DEV) < 0.1
+  got = []
+  for far in (7, 2**32, -2**32):
+    kind = torch.int32 if far == 7 else torch.int64
+    pos = torch.where(starts, 0, far).to(kind)
+    with training.differentiable():
+      y, _ = layer(x, pos, return_cache=False)
+    got.append((y.detach(), *torch.autograd.grad(y, (x, *layer.parameters()), dy)))
+  for other in got[1:]:
+    assert all(torch.equal(a, b) for a, b in zip(got[0], other))
