@@ -453,6 +453,14 @@ def recurrent_core(x, segment_pos, conv_w, conv_b, w_x, b_x, w_a, b_a, a_param,
   return y, h_last, cache
 
 
+def _linear_scan_workspace(x, backward):
+  """What the bare recurrence is fastest with (csrc/train_ops.cpp brings the same:
+  one shape, one form of the call and one set of bits), or None."""
+  need = _lib.lib().rg_linear_scan_best_workspace_bytes(*x.shape, _dtype_code(x),
+                                                        int(backward))
+  return torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+
+
 def linear_scan(x, a, reset, h0=None, split=True):
   if split:
     got = _lib.host().linear_scan(x, a, reset, h0)
@@ -471,7 +479,7 @@ def linear_scan(x, a, reset, h0=None, split=True):
     return y, h_last
   y = torch.empty_like(x)
   h_last = torch.empty((B, W), dtype=torch.float32, device=x.device)
-  ws = _scan_workspace(B, T, W, x.device, split)
+  ws = _linear_scan_workspace(x, backward=False) if split else None
   with _on(x.device):
     if ws is None:
       _lib.check(_lib.lib().rg_linear_scan(
@@ -486,7 +494,7 @@ def linear_scan(x, a, reset, h0=None, split=True):
 
 def linear_scan_backward(dy, a, reset, y, h0=None, dh_last=None):
   """Gradients of linear_scan: (dx, da, dh0 | None) from the gradient of y
-  (and of the final state); one kernel, no flipped copies."""
+  (and of the final state); one pass, no flipped copies."""
   B, T, W = y.shape
   y = _dev(y, "y")
   _same(y.dtype, y.device, dy=dy, a=a)
@@ -503,10 +511,12 @@ def linear_scan_backward(dy, a, reset, y, h0=None, dh_last=None):
   dx, da = torch.empty_like(y), torch.empty_like(y)
   dh0 = (torch.empty((B, W), dtype=torch.float32, device=y.device)
          if h0 is not None else None)
+  ws = _linear_scan_workspace(y, backward=True)
   with _on(y.device):
-    _lib.check(_lib.lib().rg_linear_scan_backward(
+    _lib.check(_lib.lib().rg_linear_scan_backward_best(
         _p(dy), _p(a), _p(reset), _p(y), _p(h0), _p(dh_last), _p(dx), _p(da),
-        _p(dh0), B, T, W, _dtype_code(y), _stream(y)))
+        _p(dh0), _p(ws), 0 if ws is None else ws.numel(), B, T, W, _dtype_code(y),
+        _stream(y)))
   return dx, da, dh0
 
 

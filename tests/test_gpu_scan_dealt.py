@@ -8,8 +8,10 @@ import ctypes
 import pytest
 import torch
 
+import recurrentgemma_amd as rg
 from recurrentgemma_amd import _lib
 from recurrentgemma_amd import ops
+from recurrentgemma_amd import training
 from tests import test_gpu_core_f32_wide as core_f32
 from tests import test_gpu_scan_tiles as one_pass
 from tests import test_gpu_training as trained
@@ -80,6 +82,25 @@ def test_rows_apart_and_against_slabs():
   yn, hn = ops.linear_scan(x, a, reset, h0)
   assert torch.equal(yn[0], y[0]) and torch.equal(hn[0], h[0])
   assert torch.equal(yn[1, :3], y[1, :3]) and bool(yn[1, 700].isnan().all())
+
+
+@pytest.mark.parametrize("dtype,B,T,W", [(BF16, 1, 8000, 512), (F32, 2, 6000, 1024),
+                                         (F32, 1, 6145, 2560)])
+def test_general_path_is_the_same_call(dtype, B, T, W):
+  """Inputs that do not lie densely take the Python path, forward and backward: the
+  same form of the call, the same bits."""
+  x, a, reset, h0 = _inputs(B, T, W, dtype, 4)
+  dy = torch.randn_like(x)
+  assert _dealt(B, T, W, dtype, 0, 1)
+  leaves = [t.clone().requires_grad_() for t in (x, a, h0)]
+  with training.differentiable():
+    y, h = rg.rnn_scan(leaves[0], leaves[1], reset, leaves[2])
+  grads = torch.autograd.grad(y, leaves, dy)
+  wide = torch.empty(B, T, 2 * W, device=DEV, dtype=dtype)[..., :W]
+  yg, hg = ops.linear_scan(wide.copy_(x), a, reset, h0)
+  assert torch.equal(yg, y) and torch.equal(hg, h)
+  got = ops.linear_scan_backward(dy, a, reset, y.detach(), h0)
+  assert all(torch.equal(g, w) for g, w in zip(got, grads))
 
 
 def test_captured_and_side_by_side():
