@@ -120,6 +120,7 @@ PACKAGE_SIGNATURES = {
     "rg_argmax_workspace_bytes": (_sz, [_i, _i]),
     "rg_argmax_rows_split": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
     "rg_recurrent_core_best_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "rg_scan_deal_bytes": (_sz, [_i] * 5),
     "rg_linear_scan_best_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "rg_linear_scan_backward_best": (_i, [_vp] * 10 + [_sz, _i, _i, _i, _i, _vp]),
 }

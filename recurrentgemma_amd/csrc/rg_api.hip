@@ -910,6 +910,11 @@ static int linear_scan_impl(const char* who, const void* x, const void* a,
 #undef RG_WHO
 #define RG_WHO __func__
 
+size_t rg_scan_deal_bytes(int B, int T, int W, int dtype, int mode) {
+  if (mode < rg::kTilesFwdPlain || mode > rg::kTilesBwdGated) return 0;
+  return rg::scan_tiles_deal_bytes(B, T, W, dtype, mode);
+}
+
 size_t rg_linear_scan_best_workspace_bytes(int B, int T, int W, int dtype,
                                            int backward) {
   if (B <= 0 || T <= 0 || W <= 0) return 0;

@@ -58,6 +58,10 @@ int rg_linear_scan_backward_best(const void* dy, const void* a, const void* rese
                                  size_t workspace_bytes, int B, int T, int W,
                                  int dtype, void* stream);
 
+/* Bytes with which a recurrence's one-pass kernel is dealt out in steps, 0 where it is
+ * not: mode 0 the plain forward, 1 the plain backward, 2 and 3 the gated ones. */
+size_t rg_scan_deal_bytes(int B, int T, int W, int dtype, int mode);
+
 #ifdef __cplusplus
 }
 #endif

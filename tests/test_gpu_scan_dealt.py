@@ -3,8 +3,6 @@
 steps of 256 and 512 tokens, slabs of channels that are not full, one slab to more
 than there are CUs."""
 
-import ctypes
-
 import pytest
 import torch
 
@@ -23,8 +21,7 @@ BF16, F32 = torch.bfloat16, torch.float32
 
 def _dealt(B, T, W, dtype, *modes):
   """Whether the plain forward and backward, the gated ones are dealt out."""
-  f = _lib.lib()._ZN2rg21scan_tiles_deal_bytesEiiiii
-  f.restype = ctypes.c_size_t
+  f = _lib.lib().rg_scan_deal_bytes
   return all(f(B, T, W, int(dtype == BF16), m) > 0 for m in modes)
 
 

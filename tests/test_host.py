@@ -223,6 +223,15 @@ def test_c_side_validation_without_launch():
   assert lib.rg_scan_split_workspace_bytes(16, 8192, 4096) == 0
   assert lib.rg_scan_split_workspace_bytes(1, 500, 2560) == 0
   assert lib.rg_scan_split_workspace_bytes(1, 8192, 2560) == 2 * 22 * 2560 * 4
+  # few long rows are dealt out in steps: states and numbers of two steps, a counter,
+  # softplus of a_param and its derivative; nothing for many short rows, and for what
+  # is no recurrence
+  assert lib.rg_scan_deal_bytes(1, 8192, 2560, 1, 0) == 2 * 2560 * 8 + 16 + 2560 * 8
+  assert all(lib.rg_scan_deal_bytes(1, 8192, 2560, d, m) > 0
+             for d in (0, 1) for m in range(4))
+  assert lib.rg_scan_deal_bytes(16, 64, 4096, 1, 0) == 0
+  assert lib.rg_scan_deal_bytes(1, 8192, 2560, 1, -1) == 0
+  assert lib.rg_scan_deal_bytes(1, 8192, 2560, 1, 4) == 0
   rc = lib.rg_lru_scan_fused_split(ok, 0, None, None, ok, ok, ok, ok, 1, None, y,
                                    None, None, None, 0, 1, 8192, 2560, 1, None)
   assert rc == -4 and b"rg_lru_scan_fused_split: workspace" in lib.rg_last_error()
