@@ -18,6 +18,11 @@
  *  - Return value: RG_OK or a negative RG_ERR_* code; rg_last_error() then
  *    gives a thread-local, human-readable reason.  No C++ exception crosses
  *    this boundary.  Arguments are validated before anything is launched.
+ *  - Kernels that hand a row's state from workgroup to workgroup (rg_linear_scan_split
+ *    and rg_recurrent_core with the larger workspaces named there) wait for it a second
+ *    or two at most.  That bound is there for mistakes and is not reached by shapes or
+ *    load; a wait that reaches it leaves NaN in everything of its row from there on and
+ *    in the row's h_last, whatever document starts follow, and no other row is touched.
  *  - Inputs are never modified (the reference's Conv1D multiplies its input by
  *    the document mask in place, layers.py:497-508; that side effect is NOT
  *    reproduced, the masked conv state it leads to is).

@@ -338,6 +338,16 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// ------------------------------------------- states between workgroups ----
+// Polls of a state in memory (rg_prefill_relay.hip, rg_scan_tiles.hip) before a wave
+// gives up: half a microsecond to one each, so a second or two.  It cannot happen while
+// the kernels' waits are what they say they are; it is there so that a mistake in them
+// ends.  The wave then goes on with NaN as the state, which no document start clears:
+// everything of that row from there on and its last state are NaN (include/rg_lru.h),
+// which is how a caller hears of it.
+constexpr int kMaxStatePolls = 1 << 21;
+constexpr uint32_t kNoState = 0x7fc00000u;  // NaN
+
 // ------------------------------------------------------------- math ----
 constexpr float kLog2e = 1.4426950408889634f;
 

@@ -90,9 +90,6 @@ constexpr int kMatrixPriority = 1;
 // Input- and recurrence-gate sigmoids at the end of phase M, with the join and
 // without.
 constexpr int kTailXPlain = 0, kTailXJoined = 16, kTailAJoined = 4;
-// Polls of a state word before a wave gives up with NaN (about a second; it cannot
-// happen, see above).
-constexpr int kMaxPolls = 1 << 21;
 
 typedef __attribute__((address_space(3))) unsigned char lds_byte;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
@@ -534,8 +531,8 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
       for (int polls = 0; ; ++polls) {
         wait_vmcnt<1>();
         if (arrived(polls & 1)) break;
-        if (polls == kMaxPolls) {
-          state = 0x7fc00000u;
+        if (polls == kMaxStatePolls) {
+          state = kNoState;
           break;
         }
         fetch_words(q, polls & 1);

@@ -137,10 +137,6 @@ struct TileLds {
   int ticket[4];                          // dealt out: the last four
 };
 
-// Dealt out: polls of a state before a wave gives up with NaN (seconds; it cannot
-// happen, see below).
-constexpr int kMaxPolls = 1 << 21;
-
 // What the dealt form has beside: states between steps, [B][2][W] words of value and
 // number of the step; the tickets taken; total = steps x chains, chains = B x slabs.
 struct DealArgs {
@@ -658,8 +654,8 @@ scan_tiles_kernel(ScanTileArgs p, DealArgs d) {
         } else {
           for (int polls = 0; !__all((uint32_t)(word >> 32) == (uint32_t)now.step);
                ++polls) {
-            if (polls == kMaxPolls) {
-              word = 0x7fc00000u;
+            if (polls == kMaxStatePolls) {
+              word = kNoState;
               break;
             }
             poll();
