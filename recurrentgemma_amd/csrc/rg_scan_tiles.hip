@@ -63,26 +63,24 @@ __device__ __forceinline__ float choose(bool cond, float a, float b) {
 }
 
 // 1 - a^2 for a = 2^q, q <= 0, in float32: near a = 1, where the difference of the
-// rounded square would keep few of its digits, -2q (ln 2 + 2q (ln 2)^2 / 2! + ..),
-// eight terms of the exponential's series (the ninth is 2e-8 of the first).  With
-// it the float32 forms can use the hardware's exp2, reciprocal and square root
-// (RG-LRU step B3 T1001 W2560: 254 -> 240 us against expf, sqrtf and divisions;
-// sigmoids: sigmoid_f32).  Errors against 64 bits, projections included, before and
+// rounded square would keep few of its digits, -q p(q) with p the polynomial of degree
+// five through (2^2q - 1) / q at the Chebyshev nodes of -0.375 .. 0 (off by 2e-9 of it,
+// as eight terms of the exponential's own series are by 2e-8).  With it the float32
+// forms can use the hardware's exp2, reciprocal and square root (sigmoids: sigmoid_f32).
+// Errors against 64 bits, projections included, before (expf, sqrtf and divisions) and
 // now: gates around 0 y 1.0e-7 .. 1.6e-7 -> 7.2e-8 .. 1.2e-7, gradients 1.5e-7 ..
 // 3.3e-7 -> 1.0e-7 .. 2.1e-7; input gates at -12 .. -8 y 4.0e-7 -> 3.4e-7; recurrence
 // gates there y 4e-5 -> 6e-7.  Of this kernel alone (exact pre-activations): y and the
 // gradients of x and the input gate as before, the recurrence gate's bias up to 1.1
 // times (1.7e-7 -> 1.9e-7).
 __device__ __forceinline__ float one_minus_square(float q, float a) {
-  constexpr float kSeries[8] = {0.69314718056f,    0.24022650696f,
-                                5.5504108665e-2f,  9.6181291076e-3f,
-                                1.3333558146e-3f,  1.5403530393e-4f,
-                                1.5252733804e-5f,  1.3215486790e-6f};
-  const float w = 2.0f * q;
-  float s = kSeries[7];
+  constexpr float kNear[6] = {0.69314718246f * 0x1p1f,   0.24022640288f * 0x1p2f,
+                              0.055502466857f * 0x1p3f,  0.0096086980775f * 0x1p4f,
+                              0.0013086448889f * 0x1p5f, 0.00012355708168f * 0x1p6f};
+  float s = kNear[5];
 #pragma unroll
-  for (int k = 6; k >= 0; --k) s = __builtin_fmaf(s, w, kSeries[k]);
-  return w > -0.75f ? -w * s : __builtin_fmaf(-a, a, 1.0f);
+  for (int k = 4; k >= 0; --k) s = __builtin_fmaf(s, q, kNear[k]);
+  return q > -0.375f ? -q * s : __builtin_fmaf(-a, a, 1.0f);
 }
 
 constexpr int streams_of(int mode) {
