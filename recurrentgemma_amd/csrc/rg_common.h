@@ -368,8 +368,8 @@ __device__ __forceinline__ float sigmoid_fast(float v) {
 // along with what the reciprocal is off by.  (Where c or u is no number, at infinite v
 // or e^-v, its factor is 0: the medians of three are only to make them finite.)
 // RG-LRU whose input gates lie at -12 .. -8, softplus(a_param) 1: error of y against
-// 64 bits 2.4e-7 -> 6.1e-8, as with expf and a division.  Twelve issue slots instead of
-// four; a training step at B3 T1001 W2560 240.1 -> 241.6 us.
+// 64 bits 2.4e-7 -> 6.1e-8, as with expf and a division.  Eight issue slots more; of a
+// training step's 240 us at B3 T1001 W2560 1.5.
 __device__ __forceinline__ float sigmoid_f32(float v) {
   constexpr float kLn2 = 0.693147182464599609375f, kLn2Rest = -1.904654299957768e-9f;
   const float p = -kLog2e * v;
