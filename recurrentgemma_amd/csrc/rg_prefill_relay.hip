@@ -43,38 +43,26 @@
 
 #include "rg_common.h"
 #include "rg_internal.h"
-#include "rg_weight_frags.h"
+#include "rg_two_teams.h"
 
 namespace rg {
 namespace {
 
-constexpr int kBW = 256;   // head width (K and per-gate N)
-constexpr int kBT = 32;    // tokens per block
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * 64;
-// Conv output of a block (the MFMA A operand), bf16, rows padded to 264 elements; a
-// ring of three blocks.
-constexpr int kXcRowBytes = 264 * 2;
-constexpr int kXcBlockBytes = kBT * kXcRowBytes;
+using namespace two_teams;
+
 // Raw x of a block as the memory pipe writes it into LDS: rows -4 .. 31, 512 bytes
 // each, two rows a load, three loads a wave (the six beyond 18 are sent out of
 // range); a ring of three blocks.
-constexpr int kRawHalo = 4;
-constexpr int kRawRowBytes = kBW * 2;
 constexpr int kRawLoads = (kBT + kRawHalo) / 2;
 constexpr int kRawLoadsPerWave = (kRawLoads + kWaves - 1) / kWaves;
 constexpr int kRawBlockBytes = kRawLoadsPerWave * kWaves * 2 * kRawRowBytes;
-constexpr int kRing = 3;
-// Per-wave output patch, as in rg_prefill_teams.hip.
-constexpr int kPatchStride = 80;
-constexpr int kPatchUpper = 8 * kPatchStride + 64;
-constexpr int kPatchBytesPerWave = kPatchUpper + 8 * kPatchStride;
+constexpr int kRing = kXcRing;
 
 constexpr int kXcOff = 0;
 constexpr int kRawOff = kXcOff + kRing * kXcBlockBytes;
 constexpr int kPatchOff = kRawOff + kRing * kRawBlockBytes;
 constexpr int kConvTabOff = kPatchOff + kWaves * kPatchBytesPerWave;
-constexpr int kTicketOff = kConvTabOff + 128 * 32;  // the last eight tickets
+constexpr int kTicketOff = kConvTabOff + kConvTabBytes;  // the last eight tickets
 // Per wave: the 32 state words that come into its block, as the memory pipe writes
 // them, two polls of them; and the gate-branch values of its part of the block.
 constexpr int kWordOff = kTicketOff + 8 * 4;
@@ -84,29 +72,7 @@ constexpr int kBranchOff = kWordOff + kWaves * kWordBytesPerWave;
 constexpr int kBranchBytesPerWave = 2 * 1024;
 constexpr int kRelayLdsBytes = kBranchOff + kWaves * kBranchBytesPerWave;
 static_assert(kRelayLdsBytes <= 160 * 1024, "LDS of one CU");
-constexpr int kARing = 4;
-constexpr int kConvRows = 8;
-constexpr int kMatrixPriority = 1;
-// Input- and recurrence-gate sigmoids at the end of phase M, with the join and
-// without.
-constexpr int kTailXPlain = 0, kTailXJoined = 16, kTailAJoined = 4;
-
-typedef __attribute__((address_space(3))) unsigned char lds_byte;
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-typedef __attribute__((address_space(3))) uint64_t lds_u64;
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 constexpr int kAgentScope = 16;  // sc1 of a buffer instruction (gfx950)
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-__device__ __forceinline__ void phase_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
 
 // GELU: y is written as y * gelu(gate_branch), the join of the recurrent block's two
 // branches (recurrentgemma/torch/modules.py:627-628, 644).
@@ -114,7 +80,7 @@ template <bool GELU>
 __global__ void __launch_bounds__(kThreads)
 block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
   constexpr int kTailX = GELU ? kTailXJoined : kTailXPlain;
-  constexpr int kTailA = GELU ? kTailAJoined : 0;
+  constexpr int kTailA = GELU ? kTailAJoined : kTailAPlain;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   lds_byte* const lds3 = (lds_byte*)lds_raw;
 
@@ -237,78 +203,10 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
       2u * (uint32_t)(h * kBW + n0) + 16u * (lane & 3);
 
   // ---- width-4 conv ---------------------------------------------------------
-  uint32_t cw10[2], cw32[2];
-  float cbias[2];
-  auto pair_rows = [&](uint32_t earlier, uint32_t later, uint32_t (&out)[2]) {
-    pair_up(earlier, later, out[0], out[1]);
-  };
-  // rows 8 rg4 .. +7 of block kb, raw rows -> conv output, in steps that the
-  // caller spreads between its matrix instructions: the eleven raw rows
-  // (three of them history), then four row pairs.  The rows are convolved as
-  // if no document started among them; where one does they are redone with
-  // the history cut (bit i of `cuts`: row i - 3 of these rows starts a
-  // document), the same dot products in the same order.
-  struct ConvRows {
-    uint32_t raw[kConvRows + 3];
-    uint32_t e_prev[2], o_prev[2];
-    uint32_t xc_at;
-  };
-  auto conv_load = [&](int kb, ConvRows& cr) {
-    const uint32_t raw_at =
-        conv_raw_lane + (uint32_t)(kb % kRing) * kRawBlockBytes;
-    cr.xc_at = conv_xc_lane + (uint32_t)(kb % kRing) * kXcBlockBytes;
-#pragma unroll
-    for (int i = 0; i < kConvRows + 3; ++i)
-      cr.raw[i] = *reinterpret_cast<lds_u32*>(lds3 + raw_at + i * kRawRowBytes);
-  };
-  auto conv_pair = [&](ConvRows& cr, int j) {
-    if (j == 0) {
-      pair_rows(cr.raw[0], cr.raw[1], cr.o_prev);
-      pair_rows(cr.raw[1], cr.raw[2], cr.e_prev);
-    }
-    uint32_t e[2], o[2];
-    pair_rows(cr.raw[3 + 2 * j], cr.raw[4 + 2 * j], e);
-    float even[2], odd[2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-      o[c] = __builtin_amdgcn_alignbit(e[c], cr.e_prev[c], 16);
-    conv4_dot_row_pair(cr.o_prev, o, cr.e_prev, e, cw10, cw32, cbias, even, odd);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      cr.e_prev[c] = e[c];
-      cr.o_prev[c] = o[c];
-    }
-    *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at + xc_row(2 * j) * kXcRowBytes) =
-        pack_bf16x2(even[0], even[1]);
-    *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at +
-                                xc_row(2 * j + 1) * kXcRowBytes) =
-        pack_bf16x2(odd[0], odd[1]);
-  };
-  auto conv_with_cuts = [&](const ConvRows& cr, uint32_t cuts) {
-    uint32_t r_prev = 0, p1[2] = {0, 0}, p2[2] = {0, 0};
-#pragma unroll
-    for (int i = 0; i < kConvRows + 3; ++i) {
-      const uint32_t r = cr.raw[i];
-      if ((cuts >> i) & 1u) {
-        r_prev = 0;
-        p1[0] = p1[1] = p2[0] = p2[1] = 0;
-      }
-      uint32_t pt[2];
-      pair_rows(r_prev, r, pt);
-      if (i >= 3) {
-        float o[2];
-        conv4_dot_x2(p2, pt, cw10, cw32, cbias, o);
-        *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at +
-                                    xc_row(i - 3) * kXcRowBytes) =
-            pack_bf16x2(o[0], o[1]);
-      }
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        p2[c] = p1[c];
-        p1[c] = pt[c];
-      }
-      r_prev = r;
-    }
+  Conv conv;
+  auto load_rows = [&](int kb, ConvRows& cr) {  // of block kb
+    conv_load(lds3, conv_raw_lane + (uint32_t)(kb % kRing) * kRawBlockBytes,
+              conv_xc_lane + (uint32_t)(kb % kRing) * kXcBlockBytes, cr);
   };
   // Document starts among this thread group's rows (3 before + its own) of the block
   // with this mask
@@ -439,9 +337,9 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
         a[(ks + kARing - 1) % kARing] = a_read(ks + kARing - 1);
       mfma_weight_frag(2 * ks, ks == 0, a[ks % kARing], acc_x);
       mfma_weight_frag(2 * ks + 1, ks == 0, a[ks % kARing], acc_a);
-      if (ks == 0) conv_load(k + 1, cr);
+      if (ks == 0) load_rows(k + 1, cr);
       if (ks >= 3 && ks % 3 == 0 && ks / 3 - 1 < kConvRows / 2)
-        conv_pair(cr, ks / 3 - 1);
+        conv_pair(lds3, conv, cr, ks / 3 - 1, xc_row);
       if (ks == 1) dma_block(third, k + 3, 0);
       if (ks == 2) dma_block(third, k + 3, 1);
       if (ks == 3) dma_block(third, k + 3, 2);
@@ -455,7 +353,7 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
     }
 #undef RG_XR
     __builtin_amdgcn_s_setprio(0);
-    if (__builtin_expect(cuts != 0, 0)) conv_with_cuts(cr, cuts);
+    if (__builtin_expect(cuts != 0, 0)) conv_with_cuts(lds3, conv, cr, cuts, xc_row);
     // the last matrix results land (19 issue slots); every reader of the
     // accumulators is ordered behind this statement
     asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc_x), "+v"(acc_a));
@@ -664,14 +562,15 @@ block_prefill_relay_bf16_kernel(FusedArgs p, int per_head, uint32_t inverse) {
                                                      conv_pair_of_lane * 32);
     const u32x2 t1 = *reinterpret_cast<const u32x2*>(lds_raw + kConvTabOff +
                                                      conv_pair_of_lane * 32 + 16);
-    cw10[0] = t0[0]; cw32[0] = t0[1]; cw10[1] = t0[2]; cw32[1] = t0[3];
-    cbias[0] = __uint_as_float(t1[0]);
-    cbias[1] = __uint_as_float(t1[1]);
+    conv.w10[0] = t0[0]; conv.w32[0] = t0[1];
+    conv.w10[1] = t0[2]; conv.w32[1] = t0[3];
+    conv.bias[0] = __uint_as_float(t1[0]);
+    conv.bias[1] = __uint_as_float(t1[1]);
   }
   {
     ConvRows cr;
-    conv_load(0, cr);
-    conv_with_cuts(cr, conv_cuts(mask_now));
+    load_rows(0, cr);
+    conv_with_cuts(lds3, conv, cr, conv_cuts(mask_now), xc_row);
   }
   phase_barrier();
 

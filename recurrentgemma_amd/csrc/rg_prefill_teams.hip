@@ -33,76 +33,26 @@
 
 #include "rg_common.h"
 #include "rg_internal.h"
-#include "rg_weight_frags.h"
+#include "rg_two_teams.h"
 
 namespace rg {
 namespace {
 
-constexpr int kBW = 256;   // head width (K and per-gate N)
-constexpr int kBT = 32;    // tokens per block
+using namespace two_teams;
+
 constexpr int kTM = 64;    // tokens per raw tile (two blocks)
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * 64;
-// Conv output of a block (the MFMA A operand), bf16, rows padded to 264
-// elements; a ring of three blocks (a block is written over two phases, read
-// over the three after them, and a new one starts every second phase).
-constexpr int kXcStride = 264;
-constexpr int kXcRowBytes = kXcStride * 2;
-constexpr int kXcBlockBytes = kBT * kXcRowBytes;
-constexpr int kXcRing = 3;
 // Raw x of a 64-token tile as the memory pipe writes it into LDS: rows -4 ..
 // 63 of the tile, 512 bytes each; two tiles.
-constexpr int kRawHalo = 4;
 constexpr int kRawRows = kTM + kRawHalo;
-constexpr int kRawRowBytes = kBW * 2;
 constexpr int kRawLoads = kRawRows / 2;
 constexpr int kRawLoadsPerWave = (kRawLoads + kWaves - 1) / kWaves;
 constexpr int kRawTileBytes = kRawLoadsPerWave * kWaves * 2 * kRawRowBytes;
-// Per-wave output patch: 16 tokens x 32 channels in bf16, rows padded to 80
-// bytes; the second eight rows (the upper lanes') another 64 bytes on, in other
-// banks than the first.
-constexpr int kPatchStride = 80;
-constexpr int kPatchUpper = 8 * kPatchStride + 64;
-constexpr int kPatchBytesPerWave = kPatchUpper + 8 * kPatchStride;
-
 constexpr int kXcOff = 0;
 constexpr int kRawOff = kXcOff + kXcRing * kXcBlockBytes;
 constexpr int kPatchOff = kRawOff + 2 * kRawTileBytes;
 constexpr int kConvTabOff = kPatchOff + kWaves * kPatchBytesPerWave;
-constexpr int kTeamsLdsBytes = kConvTabOff + 128 * 32;
+constexpr int kTeamsLdsBytes = kConvTabOff + kConvTabBytes;
 static_assert(kTeamsLdsBytes <= 160 * 1024, "LDS of one CU");
-// Ring of MFMA A operands read ahead of their matrix instruction.
-constexpr int kARing = 4;
-// How many of a lane's sixteen tokens have their input-gate sigmoid computed
-// at the end of phase M, the rest at the top of phase G (measured at B16 T8192
-// W4096: 0 -> 755 us, 4 -> 755 us, 8 -> 765 us, 12 -> 777 us a launch), and the
-// same for the recurrence gate (any part of it there was slower).
-constexpr int kTailXPlain = 0;
-constexpr int kTailAPlain = 0;
-// ... and with the GELU join in phase G (B8 T4096 W2560 in chunks: 249-256 us for
-// 8-16 input-gate and 0-4 recurrence-gate sigmoids here: no difference)
-constexpr int kTailXJoined = 16;
-constexpr int kTailAJoined = 4;
-// Priority of a wave while it issues its matrix instructions (the wave in
-// phase G stays at 0 and fills the gaps).
-constexpr int kMatrixPriority = 1;
-
-typedef __attribute__((address_space(3))) unsigned char lds_byte;
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-typedef __attribute__((address_space(3))) uint16_t lds_u16;
-typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-__device__ __forceinline__ void phase_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
 
 // What one workgroup does with its tiles.  A row cut into chunks takes two
 // launches: the first runs chunk 0 as kChunkHead and chunks 1 .. n-2 as
@@ -203,7 +153,6 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
   // before the group's first.
   const int rg4 = team * 2 + (in_team >> 1);  // 0..3
   const int conv_pair_of_lane = (in_team & 1) * 64 + lane;
-  constexpr int kConvRows = 8;
   const uint32_t conv_raw_lane =
       kRawOff + (uint32_t)(rg4 * kConvRows + kRawHalo - 3) * kRawRowBytes +
       conv_pair_of_lane * 4;
@@ -245,82 +194,12 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
       2u * (uint32_t)(h * kBW + n0) + 16u * (lane & 3);
 
   // ---- width-4 conv ---------------------------------------------------------
-  uint32_t cw10[2], cw32[2];
-  float cbias[2];
-  constexpr uint32_t kSelLo = 0x05040100u;
-  constexpr uint32_t kSelHi = 0x07060302u;
-  auto pair_rows = [&](uint32_t earlier, uint32_t later, uint32_t (&out)[2]) {
-    out[0] = __builtin_amdgcn_perm(later, earlier, kSelLo);
-    out[1] = __builtin_amdgcn_perm(later, earlier, kSelHi);
-  };
-  // rows 8 rg4 .. +7 of block kb, raw rows -> conv output, in steps that the
-  // caller spreads between its matrix instructions: the eleven raw rows
-  // (three of them history), then four row pairs.  The rows are convolved as
-  // if no document started among them; where one does they are redone with
-  // the history cut (bit i of `cuts`: row i - 3 of these rows starts a
-  // document), the same dot products in the same order.
-  struct ConvRows {
-    uint32_t raw[kConvRows + 3];
-    uint32_t e_prev[2], o_prev[2];
-    uint32_t xc_at;
-  };
-  auto conv_load = [&](int kb, ConvRows& cr) {
-    const uint32_t raw_at = conv_raw_lane +
-                            (uint32_t)((kb >> 1) & 1) * kRawTileBytes +
-                            (uint32_t)(kb & 1) * (32 * kRawRowBytes);
-    cr.xc_at = conv_xc_lane + (uint32_t)(kb % kXcRing) * kXcBlockBytes;
-#pragma unroll
-    for (int i = 0; i < kConvRows + 3; ++i)
-      cr.raw[i] = *reinterpret_cast<lds_u32*>(lds3 + raw_at + i * kRawRowBytes);
-  };
-  auto conv_pair = [&](ConvRows& cr, int j) {
-    if (j == 0) {
-      pair_rows(cr.raw[0], cr.raw[1], cr.o_prev);
-      pair_rows(cr.raw[1], cr.raw[2], cr.e_prev);
-    }
-    uint32_t e[2], o[2];
-    pair_rows(cr.raw[3 + 2 * j], cr.raw[4 + 2 * j], e);
-    float even[2], odd[2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-      o[c] = __builtin_amdgcn_alignbit(e[c], cr.e_prev[c], 16);
-    conv4_dot_row_pair(cr.o_prev, o, cr.e_prev, e, cw10, cw32, cbias, even, odd);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      cr.e_prev[c] = e[c];
-      cr.o_prev[c] = o[c];
-    }
-    *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at + xc_row(2 * j) * kXcRowBytes) =
-        pack_bf16x2(even[0], even[1]);
-    *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at +
-                                xc_row(2 * j + 1) * kXcRowBytes) =
-        pack_bf16x2(odd[0], odd[1]);
-  };
-  auto conv_with_cuts = [&](const ConvRows& cr, uint32_t cuts) {
-    uint32_t r_prev = 0, p1[2] = {0, 0}, p2[2] = {0, 0};
-#pragma unroll
-    for (int i = 0; i < kConvRows + 3; ++i) {
-      const uint32_t r = cr.raw[i];
-      if ((cuts >> i) & 1u) {
-        r_prev = 0;
-        p1[0] = p1[1] = p2[0] = p2[1] = 0;
-      }
-      uint32_t pt[2];
-      pair_rows(r_prev, r, pt);
-      if (i >= 3) {
-        float o[2];
-        conv4_dot_x2(p2, pt, cw10, cw32, cbias, o);
-        *reinterpret_cast<lds_u32*>(lds3 + cr.xc_at +
-                                    xc_row(i - 3) * kXcRowBytes) =
-            pack_bf16x2(o[0], o[1]);
-      }
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        p2[c] = p1[c];
-        p1[c] = pt[c];
-      }
-      r_prev = r;
-    }
+  Conv conv;
+  auto load_rows = [&](int kb, ConvRows& cr) {  // of block kb
+    conv_load(lds3,
+              conv_raw_lane + (uint32_t)((kb >> 1) & 1) * kRawTileBytes +
+                  (uint32_t)(kb & 1) * (32 * kRawRowBytes),
+              conv_xc_lane + (uint32_t)(kb % kXcRing) * kXcBlockBytes, cr);
   };
   // Document starts among this thread group's rows (3 before + its own) of
   // block kb: m_tile is the start mask of the block's tile, m_before that of
@@ -421,9 +300,9 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
         a[(ks + kARing - 1) % kARing] = a_read(ks + kARing - 1);
       mfma_weight_frag(2 * ks, ks == 0, a[ks % kARing], acc_x);
       mfma_weight_frag(2 * ks + 1, ks == 0, a[ks % kARing], acc_a);
-      if (ks == 0) conv_load(kb + 1, cr);
+      if (ks == 0) load_rows(kb + 1, cr);
       if (ks >= 3 && ks % 3 == 0 && ks / 3 - 1 < kConvRows / 2)
-        conv_pair(cr, ks / 3 - 1);
+        conv_pair(lds3, conv, cr, ks / 3 - 1, xc_row);
       // (late in the loop, when the conv rows have left their registers)
       if (ks == 13) { RG_XR(0) RG_XR(1) RG_XR(2) RG_XR(3) RG_XR(4) }
       if (ks == 14) { RG_XR(5) RG_XR(6) RG_XR(7) RG_XR(8) RG_XR(9) RG_XR(10) }
@@ -439,7 +318,7 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
     }
 #undef RG_XR
     __builtin_amdgcn_s_setprio(0);
-    if (__builtin_expect(cuts != 0, 0)) conv_with_cuts(cr, cuts);
+    if (__builtin_expect(cuts != 0, 0)) conv_with_cuts(lds3, conv, cr, cuts, xc_row);
     // the last matrix results land (19 issue slots); every reader of the
     // accumulators is ordered behind this statement
     asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc_x), "+v"(acc_a));
@@ -637,14 +516,15 @@ __device__ __forceinline__ void prefill_teams_body(const FusedArgs& p,
                                                      conv_pair_of_lane * 32);
     const u32x2 t1 = *reinterpret_cast<const u32x2*>(lds_raw + kConvTabOff +
                                                      conv_pair_of_lane * 32 + 16);
-    cw10[0] = t0[0]; cw32[0] = t0[1]; cw10[1] = t0[2]; cw32[1] = t0[3];
-    cbias[0] = __uint_as_float(t1[0]);
-    cbias[1] = __uint_as_float(t1[1]);
+    conv.w10[0] = t0[0]; conv.w32[0] = t0[1];
+    conv.w10[1] = t0[2]; conv.w32[1] = t0[3];
+    conv.bias[0] = __uint_as_float(t1[0]);
+    conv.bias[1] = __uint_as_float(t1[1]);
   }
   {
     ConvRows cr;
-    conv_load(2 * tile_begin, cr);
-    conv_with_cuts(cr, conv_cuts(2 * tile_begin, m_cur, m_prev));
+    load_rows(2 * tile_begin, cr);
+    conv_with_cuts(lds3, conv, cr, conv_cuts(2 * tile_begin, m_cur, m_prev), xc_row);
   }
   phase_barrier();
 
