@@ -209,15 +209,14 @@ OnTiles on_tiles(const Dims& d) {
     const bool both = serve(rg::kTilesFwdGated) && serve(rg::kTilesPairGated);
     return {both, both};
   }
-  const bool dealt = rg::scan_tiles_deal_bytes((int)d.B, (int)d.T, (int)d.W, d.code,
-                                               rg::kTilesFwdGated) > 0;
+  const bool dealt = rg_scan_deal_bytes((int)d.B, (int)d.T, (int)d.W, d.code,
+                                        rg::kTilesFwdGated) > 0;
   return {dealt || serve(rg::kTilesFwdGated), serve(rg::kTilesBwdGated)};
 }
 
 // Workspace of the one-pass kernels' dealt form, where that is the faster one.
 Tensor deal_workspace(const Dims& d, rg::ScanTileMode mode, const Tensor& like) {
-  const size_t bytes =
-      rg::scan_tiles_deal_bytes((int)d.B, (int)d.T, (int)d.W, d.code, mode);
+  const size_t bytes = rg_scan_deal_bytes((int)d.B, (int)d.T, (int)d.W, d.code, mode);
   return bytes ? empty({(int64_t)bytes}, at::kByte, like) : Tensor();
 }
 
