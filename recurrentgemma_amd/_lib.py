@@ -121,6 +121,13 @@ PACKAGE_SIGNATURES = {
     "rg_argmax_rows_split": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
     "rg_recurrent_core_best_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "rg_scan_deal_bytes": (_sz, [_i] * 5),
+    "rg_linear_many_pays": (_i, [_i64, _i, _i, _vp, _i]),
+    "rg_linear_many": (_i, [_vp, _i64, _i, _i, _vp, _vp, _vp, _vp, _i, _vp]),
+    "rg_linear_back_pays": (_i, [_i64, _i, _i, _i, _i]),
+    "rg_linear_back": (_i, [_vp] * 5 + [_i64, _i, _i, _i, _vp]),
+    "rg_linear_weight_grads": (_i, [_vp] * 5 + [_i, _i64, _i, _vp]),
+    "rg_linear_gelu_pair_pays": (_i, [_i64, _i, _i, _i]),
+    "rg_linear_gelu_pair": (_i, [_vp] * 4 + [_i64, _i, _i, _i, _vp]),
     "rg_linear_scan_best_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "rg_linear_scan_backward_best": (_i, [_vp] * 10 + [_sz, _i, _i, _i, _i, _vp]),
 }

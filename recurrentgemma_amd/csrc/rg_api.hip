@@ -1192,6 +1192,183 @@ size_t rg_argmax_workspace_bytes(int rows, int n) {
   return rows > 0 && n > 0 ? rg::argmax_workspace_bytes(rows, n) : 0;
 }
 
+// x [M, K] and weights [N_i, K] as one launch of products, or nothing where they do not
+// fit one
+static bool linear_many_args(const void* x, int64_t M, int K, int count,
+                             const void* const* w, const void* const* bias,
+                             void* const* out, const int* N, rg::MatmulArgs* a) {
+  *a = rg::MatmulArgs{};
+  if (count < 1 || count > rg::kMaxMatmuls || M > INT32_MAX) return false;
+  a->count = count;
+  for (int i = 0; i < count; ++i) {
+    rg::MatmulProblem& p = a->p[i];
+    p.m = x;
+    if (w) p.n = w[i];
+    if (bias) p.bias = bias[i];
+    if (out) p.c = out[i];
+    p.M = (int)M;
+    p.N = N[i];
+    p.K = K;
+    p.ldm = p.ldn = K;
+    p.ldc = N[i];
+  }
+  return true;
+}
+
+int rg_linear_many_pays(int64_t M, int K, int count, const int* N, int dtype) {
+  rg::MatmulArgs a;
+  return dtype == RG_DTYPE_BF16 && N &&
+         linear_many_args(nullptr, M, K, count, nullptr, nullptr, nullptr, N, &a) &&
+         rg::matmul_pays(a, rg::kMatmulForward);
+}
+
+int rg_linear_many(const void* x, int64_t M, int K, int count, const void* const* w,
+                   const void* const* bias, void* const* out, const int* N, int dtype,
+                   void* stream) {
+  RG_CHECK_DTYPE(dtype);
+  RG_REQUIRE(M > 0 && K > 0 && count > 0 && w && out && N,
+             "%s: M=%lld K=%d count=%d must be positive, the lists present", __func__,
+             (long long)M, K, count);
+  RG_CHECK_PTR(x);
+  for (int i = 0; i < count; ++i) {
+    RG_REQUIRE(N[i] > 0, "%s: N[%d]=%d must be positive", __func__, i, N[i]);
+    RG_CHECK_PTR(w[i]);
+    RG_CHECK_PTR(out[i]);
+    if (bias) RG_CHECK_OPT_PTR(bias[i]);
+  }
+  rg::MatmulArgs a;
+  if (dtype != RG_DTYPE_BF16 ||
+      !linear_many_args(x, M, K, count, w, bias, out, N, &a) ||
+      !rg::matmul_serves(a, rg::kMatmulForward))
+    return fail(RG_ERR_UNSUPPORTED, "%s: M=%lld K=%d", __func__, (long long)M, K);
+  return launch_status(__func__,
+                       rg::launch_matmul(a, rg::kMatmulForward, (hipStream_t)stream));
+}
+
+static bool linear_back_args(const void* dy, const void* w, const void* dy2,
+                             const void* w2, void* dx, int64_t M, int K, int N,
+                             rg::MatmulArgs* a) {
+  *a = rg::MatmulArgs{};
+  if (M > INT32_MAX) return false;
+  a->count = 1;
+  rg::MatmulProblem& p = a->p[0];
+  p.m = dy;
+  p.n = w;
+  p.m2 = dy2;
+  p.n2 = w2;
+  p.c = dx;
+  p.M = (int)M;
+  p.N = N;
+  p.K = K;
+  p.ldm = K;
+  p.ldn = p.ldc = N;
+  return true;
+}
+
+int rg_linear_back_pays(int64_t M, int K, int N, int two, int dtype) {
+  rg::MatmulArgs a;
+  // (the second pair only counts as being there)
+  alignas(16) static const char some = 0;
+  const void* second = two ? &some : nullptr;
+  return dtype == RG_DTYPE_BF16 &&
+         linear_back_args(nullptr, nullptr, second, second, nullptr, M, K, N, &a) &&
+         rg::matmul_pays(a, rg::kMatmulBack);
+}
+
+int rg_linear_back(const void* dy, const void* w, const void* dy2, const void* w2,
+                   void* dx, int64_t M, int K, int N, int dtype, void* stream) {
+  RG_CHECK_DTYPE(dtype);
+  RG_REQUIRE(M > 0 && K > 0 && N > 0, "%s: M=%lld K=%d N=%d must be positive", __func__,
+             (long long)M, K, N);
+  RG_CHECK_PTR(dy);
+  RG_CHECK_PTR(w);
+  RG_REQUIRE(!dy2 == !w2, "%s: dy2 and w2 come together", __func__);
+  RG_CHECK_OPT_PTR(dy2);
+  RG_CHECK_OPT_PTR(w2);
+  RG_CHECK_PTR(dx);
+  rg::MatmulArgs a;
+  if (dtype != RG_DTYPE_BF16 || !linear_back_args(dy, w, dy2, w2, dx, M, K, N, &a) ||
+      !rg::matmul_serves(a, rg::kMatmulBack))
+    return fail(RG_ERR_UNSUPPORTED, "%s: M=%lld K=%d N=%d", __func__, (long long)M, K, N);
+  return launch_status(__func__,
+                       rg::launch_matmul(a, rg::kMatmulBack, (hipStream_t)stream));
+}
+
+int rg_linear_weight_grads(const void* const* dy, const void* const* x, void* const* dw,
+                           const int* out_features, const int* in_features, int count,
+                           int64_t M, int dtype, void* stream) {
+  RG_CHECK_DTYPE(dtype);
+  RG_REQUIRE(M > 0 && count > 0 && dy && x && dw && out_features && in_features,
+             "%s: M=%lld count=%d must be positive, the lists present", __func__,
+             (long long)M, count);
+  rg::MatmulArgs a{};
+  bool fits = dtype == RG_DTYPE_BF16 && count <= rg::kMaxMatmuls && M <= INT32_MAX;
+  for (int i = 0; i < count; ++i) {
+    RG_REQUIRE(out_features[i] > 0 && in_features[i] > 0,
+               "%s: features %d, %d must be positive", __func__, out_features[i],
+               in_features[i]);
+    RG_CHECK_PTR(dy[i]);
+    RG_CHECK_PTR(x[i]);
+    RG_CHECK_PTR(dw[i]);
+    if (!fits) continue;
+    rg::MatmulProblem& p = a.p[a.count++];
+    p.m = dy[i];
+    p.n = x[i];
+    p.c = dw[i];
+    p.M = p.ldm = out_features[i];
+    p.N = p.ldn = p.ldc = in_features[i];
+    p.K = (int)M;
+  }
+  if (!fits || !rg::matmul_serves(a, rg::kMatmulWeights))
+    return fail(RG_ERR_UNSUPPORTED, "%s: M=%lld count=%d", __func__, (long long)M, count);
+  return launch_status(__func__,
+                       rg::launch_matmul(a, rg::kMatmulWeights, (hipStream_t)stream));
+}
+
+static bool gelu_pair_args(const void* x, const void* w, const void* bias, void* out,
+                           int64_t M, int K, int N, rg::MatmulArgs* a) {
+  *a = rg::MatmulArgs{};
+  if (M > INT32_MAX) return false;
+  a->count = 1;
+  rg::MatmulProblem& p = a->p[0];
+  p.m = x;
+  p.n = w;
+  p.n2 = w ? (const char*)w + 2ll * K * N : nullptr;
+  p.bias = bias;
+  p.bias2 = bias ? (const char*)bias + 2ll * N : nullptr;
+  p.c = out;
+  p.M = (int)M;
+  p.N = N;
+  p.K = K;
+  p.ldm = K;
+  p.ldn = p.ldc = N;
+  return true;
+}
+
+int rg_linear_gelu_pair_pays(int64_t M, int K, int N, int dtype) {
+  rg::MatmulArgs a;
+  return dtype == RG_DTYPE_BF16 &&
+         gelu_pair_args(nullptr, nullptr, nullptr, nullptr, M, K, N, &a) &&
+         rg::matmul_pays(a, rg::kMatmulGeluPair);
+}
+
+int rg_linear_gelu_pair(const void* x, const void* w, const void* bias, void* out,
+                        int64_t M, int K, int N, int dtype, void* stream) {
+  RG_CHECK_DTYPE(dtype);
+  RG_REQUIRE(M > 0 && K > 0 && N > 0, "%s: M=%lld K=%d N=%d must be positive", __func__,
+             (long long)M, K, N);
+  RG_CHECK_PTR(x);
+  RG_CHECK_PTR(w);
+  RG_CHECK_OPT_PTR(bias);
+  RG_CHECK_PTR(out);
+  rg::MatmulArgs a;
+  if (dtype != RG_DTYPE_BF16 || !gelu_pair_args(x, w, bias, out, M, K, N, &a) ||
+      !rg::matmul_serves(a, rg::kMatmulGeluPair))
+    return fail(RG_ERR_UNSUPPORTED, "%s: M=%lld K=%d N=%d", __func__, (long long)M, K, N);
+  return launch_status(__func__,
+                       rg::launch_matmul(a, rg::kMatmulGeluPair, (hipStream_t)stream));
+}
+
 int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
                          int n, int dtype, void* stream) {
   RG_CHECK_DTYPE(dtype);

@@ -241,6 +241,31 @@ hipError_t launch_gemm_mfma_bf16(const GemmArgs& a, hipStream_t s);
 hipError_t launch_gemm_mfma_f32(const GemmArgs& a, hipStream_t s);
 hipError_t launch_lru_scan(const ScanArgs& a, int dtype, hipStream_t s);
 
+// Linear layers of many rows, bf16 (rg_matmul.hip): up to kMaxMatmuls products of one
+// kind as one launch.
+enum MatmulKind {
+  kMatmulForward = 0,   // m [M, K], n [N, K]: c = m n^T + bias
+  kMatmulBack = 1,      // m [M, K], n [K, N]: c = m n (+ m2 n2, the same sizes)
+  kMatmulWeights = 2,   // m [K, M], n [K, N]: c = m^T n
+  kMatmulGeluPair = 3   // m [M, K], n, n2 [K, N]: c = gelu(m n + bias) * (m n2 + bias2)
+};
+constexpr int kMaxMatmuls = 4;
+struct MatmulProblem {
+  const void *m, *n, *m2, *n2, *bias, *bias2;
+  void* c;                 // [M, N]
+  int M, N, K;
+  int ldm, ldn, ldc;       // elements from one row of a tensor to the next
+  int first_tile;          // (the launcher's)
+};
+struct MatmulArgs {
+  MatmulProblem p[kMaxMatmuls];
+  int count;
+};
+// Whether the launch can be made; and whether it is ahead of the library's products.
+bool matmul_serves(const MatmulArgs& a, int kind);
+bool matmul_pays(const MatmulArgs& a, int kind);
+hipError_t launch_matmul(MatmulArgs a, int kind, hipStream_t s);
+
 // Backward pass of rnn_scan (rg_scan_bwd.hip).
 struct ScanBwdArgs {
   const void* dy;        // [B, T, W] gradient of y

@@ -1,0 +1,580 @@
+// Linear layers of many rows in bf16 (the nn.Linear and stacked layers of
+// recurrentgemma/torch/modules.py:605-760 and :404-476 on prompts and training
+// batches): C[m, n] = sum_k of an M-side times an N-side operand, float32 sums, one
+// rounding.  Each side comes with the contraction as its contiguous dimension
+// (activations [rows, features], weights [out, in]) or as its slow one (weights
+// [in, out]; both sides of a weight gradient), so the three directions of a layer are
+// one kernel:
+//   kMatmulForward   x [M, K] . w [N, K]^T (+ bias)
+//   kMatmulBack      dy [M, K] . w [K, N], the contraction in one stretch or two
+//                    (two layers that share an input: one product over both)
+//   kMatmulWeights   dy [K, M]^T . x [K, N]
+//   kMatmulGeluPair  gelu(x . w [K, N] + bias) * (x . w2 [K, N] + bias2)
+// Up to kMaxMatmuls products go out as one launch, tile after tile.
+//
+// One workgroup of four waves, one per SIMD, per tile of 32 MB x 64 NB outputs (256 x
+// 320 for a large product).  Both operands go global -> LDS by the memory pipe in steps
+// of 64 along the contraction, two stages; a wave multiplies a quarter of the tile from
+// LDS with v_mfma_f32_16x16x32_bf16, operand fragments of the next half step on their
+// way while those of this one are multiplied.  A side whose contraction is the slow
+// dimension is staged as it lies and read with ds_read_b64_tr_b16, which hands out
+// columns.
+//
+// What bounds it is power: the matrix pipe is busy 82-86 % of the main loop's cycles
+// and the clock gives way to 1.6-1.85 GHz under it (with zeros for operands the same
+// loop runs at 2.25).  So what costs energy decides:
+//  - 16x16x32 instructions instead of 32x32x16 (half the accumulator traffic for the
+//    same product; 1.40-1.55 GHz at 94 % busy): 8192 x 5120 x 2560 168 -> 156 us.
+//  - Tiles 320 wide: fewer LDS reads per product than 256 x 256, and the widths that
+//    are multiples of 320 come out even on 256 CUs (8192 x 2560: 256 tiles for 320).
+//  - 16-byte chunks of an LDS row permuted by the row's number, so that operand reads
+//    meet no bank twice; full 128-byte lines per row in every load.
+// A stage's lines are asked into L2 one step before the stage is loaded (each
+// workgroup its share of the panels that the workgroups of its XCD read together): a
+// stage has one step to arrive, which a miss in L2 does not make (8192 x 5120 x 2560
+// 176 -> 168 us).
+// Rates in TFLOP/s, operands in memory, against the library's: rows 8192, 5120 x 2560
+// forward 1370 (870); back through two 2560 x 2560 layers 1370 (930); three weight
+// gradients of 2560 x 2560 over 8192 rows 1340 (770).
+#include <utility>
+
+#include "rg_common.h"
+#include "rg_internal.h"
+
+namespace rg {
+namespace {
+
+typedef __attribute__((address_space(3))) unsigned char lds_byte;
+typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+constexpr int kStep = 64;           // of the contraction, per stage
+constexpr int kPanelBytes = 8192;   // 64 x 64 values of one operand
+constexpr int kAccBlocks = 64;      // 16 x 16 results in a[0:255], the rest in VGPRs
+
+// The first 64 result blocks of a wave live in the accumulation registers, which are
+// numbered by hand (the build checks that the compiler takes none for itself).
+template <int N>
+__device__ __forceinline__ float acc_read() {
+  float t;
+  asm volatile("v_accvgpr_read_b32 %0, a[%c1]" : "=v"(t) : "n"(N));
+  return t;
+}
+template <int N>
+__device__ __forceinline__ void acc_zero() {
+  asm volatile("v_accvgpr_write_b32 a[%c0], 0" ::"n"(N) : "a255");
+}
+template <int BLK>
+__device__ __forceinline__ void acc_mfma(const f32x4& a, const f32x4& b) {
+  asm volatile(
+      "v_mfma_f32_16x16x32_bf16 a[%c2:%c2+3], %0, %1, a[%c2:%c2+3]" ::"v"(a),
+      "v"(b), "n"(4 * BLK));
+}
+
+template <int... I, class F>
+__device__ __forceinline__ void for_each(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void for_n(F&& f) {
+  for_each(std::make_integer_sequence<int, N>{}, f);
+}
+
+// A buffer descriptor in scalar registers, for inline assembly.
+__device__ __forceinline__ u32x4 scalar_rsrc(const void* base, int64_t bytes) {
+  const uint64_t at = (uint64_t)base;
+  return u32x4{
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at),
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) & 0xffffu,
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+
+// KIND as in rg_internal.h; wave tile 16 MB x 32 NB.
+template <int KIND, int MB, int NB>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+matmul_bf16_kernel(MatmulArgs args) {
+  constexpr bool kPair = KIND == kMatmulGeluPair;
+  // sides whose contraction is the slow dimension
+  constexpr bool kSlowM = KIND == kMatmulWeights;
+  constexpr bool kSlowN = KIND != kMatmulForward;
+  constexpr bool kTwoStretches = KIND == kMatmulBack;
+  constexpr int kPanelsM = MB / 2, kPanelsN = NB;
+  constexpr int kTileM = 32 * MB;
+  constexpr int kTileN = kPair ? 32 * NB : 64 * NB;  // columns of C
+  constexpr int kStage = (kPanelsM + kPanelsN) * kPanelBytes;
+  constexpr int kLoads = 2 * (kPanelsM + kPanelsN);  // per wave and stage
+  constexpr int kLoadsEarly = kLoads / 2;            // behind the barrier at once
+  constexpr int kBlocksN = 2 * NB;                   // of 16, per wave
+  constexpr int kMfmas = MB * kBlocksN;              // per half step and wave
+  constexpr int kReads = MB + kBlocksN;
+  extern __shared__ __align__(16) unsigned char matmul_lds[];
+  lds_byte* const lds = (lds_byte*)matmul_lds;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wm = wave & 1, wn = wave >> 1;
+
+  // Tiles: contiguous runs per XCD (workgroups go to the eight XCDs in turn); inside a
+  // product eight tile rows side by side, so that the 32 workgroups of an XCD read
+  // eight panels of rows and four of columns between them.
+  unsigned id = blockIdx.x;
+  {
+    const unsigned per_xcd = gridDim.x / 8;
+    if (id < 8 * per_xcd) id = (id & 7) * per_xcd + (id >> 3);
+  }
+  int which = 0;
+  while (which + 1 < args.count && (int)id >= args.p[which + 1].first_tile) ++which;
+  const MatmulProblem& p = args.p[which];
+  id -= p.first_tile;
+  const int tiles_n = (p.N + kTileN - 1) / kTileN;
+  const int tiles_m = (p.M + kTileM - 1) / kTileM;
+  const int group = (int)id / (8 * tiles_n), in_group = (int)id % (8 * tiles_n);
+  const int group_m = tiles_m - 8 * group < 8 ? tiles_m - 8 * group : 8;
+  const int tm = 8 * group + in_group % group_m, tn = in_group / group_m;
+  const int m0 = tm * kTileM, n0 = tn * kTileN;
+
+  // ---- operands: descriptors from the tile's first row (column) to the tensor's end --
+  const int ldm2 = 2 * p.ldm, ldn2 = 2 * p.ldn;  // bytes
+  auto operand = [&](const void* base, bool slow, int first, int rows, int ld) {
+    const int64_t skip = slow ? 2ll * first : 2ll * first * ld;
+    const int64_t all =
+        slow ? 2 * ((int64_t)(p.K - 1) * ld + rows) : 2 * ((int64_t)(rows - 1) * ld + p.K);
+    return scalar_rsrc((const char*)base + skip, all - skip);
+  };
+  u32x4 rm = operand(p.m, kSlowM, m0, p.M, p.ldm);
+  u32x4 rn = operand(p.n, kSlowN, n0, p.N, p.ldn);
+  u32x4 rn_up = rn;
+  if (kPair) rn_up = operand(p.n2, kSlowN, n0, p.N, p.ldn);
+  const int steps_one = (p.K + kStep - 1) / kStep;
+  const int steps = kTwoStretches && p.m2 ? 2 * steps_one : steps_one;
+
+  // A load instruction fills 1 KB: eight rows of a panel (rows of the operand, or of
+  // the contraction where that is the slow dimension), 128 bytes each, their 16-byte
+  // chunks permuted by the row's number.
+  const int lr = lane >> 3, lc = lane & 7;
+  auto lane_offset = [&](bool slow, int ld2) {
+    return (uint32_t)(lr * ld2 + 16 * (slow ? lc ^ ((lr & 3) << 1) : lc ^ lr));
+  };
+  const uint32_t vm0 = lane_offset(kSlowM, ldm2), vn0 = lane_offset(kSlowN, ldn2);
+  const uint32_t step_m = kSlowM ? kStep * ldm2 : 2 * kStep;
+  const uint32_t step_n = kSlowN ? kStep * ldn2 : 2 * kStep;
+  uint32_t vm = vm0, vn = vn0;
+  // wave's part of panel i / 2: rows 32 (i % 2) + 8 wave .. + 7
+  int scalar_offset[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int row = 32 * (i & 1) + 8 * wave;
+    const bool is_m = i / 2 < kPanelsM;
+    int panel = is_m ? i / 2 : i / 2 - kPanelsM;
+    if (kPair && !is_m) panel %= NB / 2;
+    scalar_offset[i] = (is_m ? kSlowM : kSlowN)
+                           ? row * (is_m ? ldm2 : ldn2) + 128 * panel
+                           : (64 * panel + row) * (is_m ? ldm2 : ldn2);
+  }
+  auto load = [&](uint32_t stage, auto I) {
+    constexpr int i = decltype(I)::value;
+    constexpr bool is_m = i / 2 < kPanelsM;
+    constexpr bool is_up = kPair && i / 2 - kPanelsM >= NB / 2;
+    const u32x4 r = is_m ? rm : is_up ? rn_up : rn;
+    // (inline assembly: behind the builtin the compiler has every transposing LDS read
+    // wait for all loads on their way)
+    const uint32_t to = stage + 1024 * (uint32_t)wave, v = is_m ? vm : vn;
+    const int at = scalar_offset[i];
+    asm volatile("s_add_u32 m0, %0, %c1\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds" ::"s"(to),
+                 "n"(i / 2 * kPanelBytes + (i & 1) * 4096), "v"(v), "s"(r), "s"(at)
+                 : "scc");
+  };
+
+  // ---- lines of the step after a stage's, asked into L2 ------------------------------
+  // wave 0: this workgroup's quarter of the M panels' lines, wave 1: its eighth of the
+  // N panels'; what arrives goes to a corner of LDS that nobody reads.
+  uint32_t vp0 = kBufferOutOfRange;
+  if (wave == 0 && lane < 8 * MB) {
+    constexpr int kLines = kTileM / 64;  // a row of the contraction is this many lines
+    vp0 = kSlowM ? (uint32_t)((16 * (tn & 3) + lane / kLines) * ldm2 + 128 * (lane % kLines))
+                 : (uint32_t)((8 * MB * (tn & 3) + lane) * ldm2);
+  }
+  if (wave == 1 && lane < 8 * NB) {
+    constexpr int kLines = kTileN / 64;
+    vp0 = kSlowN ? (uint32_t)((8 * (tm & 7) + lane % (8 * kLines) / kLines) * ldn2 +
+                              128 * (lane % kLines))
+                 : (uint32_t)((8 * NB * (tm & 7) + lane) * ldn2);
+  }
+  // (the pair's second weight is asked for by wave 2)
+  if (kPair && wave == 2 && lane < 8 * NB)
+    vp0 = (uint32_t)((8 * (tm & 7) + lane % (8 * (kTileN / 64)) / (kTileN / 64)) * ldn2 +
+                     128 * (lane % (kTileN / 64)));
+  u32x4 rp = wave == 0 ? rm : kPair && wave == 2 ? rn_up : rn;
+  const uint32_t step_p = wave == 0 ? step_m : step_n;
+  uint32_t vp = vp0 + step_p;
+  auto prefetch = [&] {
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(
+                     (uint32_t)(uintptr_t)lds + 2 * kStage + 256 * (uint32_t)wave),
+                 "v"(vp), "s"(rp));
+  };
+  int load_step = 0;
+  auto advance = [&] {  // a stage's loads are out: on to the next step's
+    ++load_step;
+    vm += step_m;
+    vn += step_n;
+    vp += step_p;
+    if (kTwoStretches && load_step == steps_one && steps > steps_one) {
+      rm = operand(p.m2, kSlowM, m0, p.M, p.ldm);
+      rn = operand(p.n2, kSlowN, n0, p.N, p.ldn);
+      rp = wave == 0 ? rm : rn;
+      vm = vm0;
+      vn = vn0;
+      vp = vp0 + step_p;
+    }
+    if (load_step >= steps) rm[2] = rn[2] = rn_up[2] = 0;  // nothing more is read
+    if (load_step + 1 >= steps) rp[2] = 0;
+  };
+
+  // ---- operand fragments ---------------------------------------------------------------
+  // Lane (n = lane % 16, quarter = lane / 16) holds row n of a 16-row block, contraction
+  // indices 8 quarter .. + 7 of a half step.
+  const int n = lane & 15, quarter = lane >> 4;
+  auto lane_address = [&](bool slow, uint32_t base, uint32_t (&a)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (!slow) {  // i: half step
+        a[i] = base + (uint32_t)(128 * n + 16 * ((4 * i + quarter) ^ (n & 7)));
+      } else {  // i: block of a panel; rows 8 quarter + n / 4 and four on
+        const int row = 8 * quarter + (n >> 2);
+        a[i] = base + (uint32_t)(128 * row + 16 * ((2 * i + ((n & 3) >> 1)) ^ ((n >> 2) << 1)) +
+                                 8 * (n & 1));
+      }
+    }
+  };
+  const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+  uint32_t am[4], an[4];
+  lane_address(kSlowM, lds0 + wm * (MB / 4) * kPanelBytes, am);
+  // The N side's blocks of a wave: 16 kBlocksN in a row, or (slow: whole panels are
+  // wanted, for constant offsets) every second pair of blocks, or of each weight of a
+  // pair the same panel.
+  lane_address(kSlowN,
+               lds0 + kPanelsM * kPanelBytes +
+                   (kPair ? wn * kPanelBytes : kSlowN ? 0 : wn * NB * 4096),
+               an);
+  if (kSlowN && !kPair && wn) {
+    an[0] = an[2];
+    an[1] = an[3];
+  }
+  auto fragment = [&](bool slow, const uint32_t (&a)[4], uint32_t stage, int block,
+                      int panel, int half_step) -> f32x4 {
+    if (!slow)
+      return *reinterpret_cast<const lds_f32x4*>((lds_byte*)(uintptr_t)(a[half_step] + stage) +
+                                                 2048 * block);
+    union {
+      s16x4 h[2];
+      f32x4 v;
+    } u;
+    lds_byte* const at = (lds_byte*)(uintptr_t)(a[block] + stage) + panel * kPanelBytes +
+                         4096 * half_step;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 512));
+    return u.v;
+  };
+  f32x4 fm[2][MB], fn[2][kBlocksN];
+  auto read = [&](uint32_t stage, int half_step, auto I) {
+    constexpr int i = decltype(I)::value;
+    if constexpr (i < MB) {
+      fm[half_step][i] = kSlowM ? fragment(true, am, stage, i & 3, i >> 2, half_step)
+                                : fragment(false, am, stage, i, 0, half_step);
+    } else {
+      constexpr int j = i - MB;
+      fn[half_step][j] =
+          kPair ? fragment(true, an, stage, j & 3, (j >> 2) * (NB / 2), half_step)
+          : kSlowN ? fragment(true, an, stage, j & 1, j >> 1, half_step)
+                   : fragment(false, an, stage, j, 0, half_step);
+    }
+  };
+
+  // ---- main loop -----------------------------------------------------------------------
+  constexpr int kInVgprs = MB * kBlocksN > kAccBlocks ? MB * kBlocksN - kAccBlocks : 0;
+  f32x4 extra[kInVgprs > 0 ? kInVgprs : 1];
+#pragma unroll
+  for (int i = 0; i < kInVgprs; ++i) extra[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for_n<4 * (MB * kBlocksN - kInVgprs)>([&](auto I) { acc_zero<decltype(I)::value>(); });
+
+  // a half step's matrix instructions, with what `between` issues behind each
+  auto multiply = [&](auto HALF, auto&& between) {
+    constexpr int half_step = decltype(HALF)::value;
+    for_n<kMfmas>([&](auto I) {
+      constexpr int i = decltype(I)::value, nb = i / MB, mb = i % MB;
+      const f32x4 &a = fn[half_step][nb], &b = fm[half_step][mb];
+      if constexpr (i < kAccBlocks) {
+        acc_mfma<i>(a, b);
+      } else {
+        f32x4& c = extra[i - kAccBlocks];
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      between(I);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  constexpr int kReadEvery = kMfmas / kReads > 2 ? kMfmas / kReads - 1 : 2;
+  constexpr int kEarlyEvery = kMfmas / kLoadsEarly;
+  constexpr int kLateEvery = kMfmas / 20 > 2 ? kMfmas / 20 : 2;
+  static_assert(kReadEvery * (kReads - 1) < kMfmas, "reads of a half step");
+  static_assert(kLateEvery * (kLoads - kLoadsEarly) + 1 < kMfmas, "loads of a half step");
+  using Zero = std::integral_constant<int, 0>;
+  using One = std::integral_constant<int, 1>;
+
+  for_n<kLoads>([&](auto I) { load(lds0, I); });
+  advance();
+  for_n<kLoadsEarly>([&](auto I) { load(lds0 + kStage, I); });
+  asm volatile("s_waitcnt vmcnt(%c0)\n\ts_barrier" ::"n"(kLoadsEarly) : "memory");
+  for_n<kReads>([&](auto I) { read(0, 0, I); });
+  uint32_t stage = 0;
+  for (int step = 0; step < steps; ++step) {
+    // First half step: this stage's second half is read, the next stage's loads end.
+    const uint32_t next = kStage - stage;
+    multiply(Zero{}, [&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if constexpr (i % kReadEvery == 0 && i / kReadEvery < kReads)
+        read(stage, 1, std::integral_constant<int, i / kReadEvery>{});
+      if constexpr (i % kLateEvery == 1 && kLoadsEarly + i / kLateEvery < kLoads)
+        load(lds0 + next, std::integral_constant<int, kLoadsEarly + i / kLateEvery>{});
+      if constexpr (i == kLateEvery * (kLoads - kLoadsEarly) + 1) prefetch();
+    });
+    advance();
+    // This wave has read all of this stage and its share of the next one is there
+    // (everything but the prefetch): behind the barrier that holds for all four.
+    asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    multiply(One{}, [&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if constexpr (i % kReadEvery == 0 && i / kReadEvery < kReads)
+        read(next, 0, std::integral_constant<int, i / kReadEvery>{});
+      if constexpr (i % kEarlyEvery == 1 && i / kEarlyEvery < kLoadsEarly)
+        load(lds0 + stage, std::integral_constant<int, i / kEarlyEvery>{});
+    });
+    stage = next;
+  }
+  // (no load outlives the workgroup's LDS; the last ones were out of range)
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 7" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < kInVgprs; ++i) asm volatile("" : "+v"(extra[i]));
+
+  // ---- results: lane (n, quarter) has row n of a block of 16 rows of C, columns
+  //      4 quarter .. + 3 of one of 16 columns -------------------------------------------
+  auto value = [&](auto BLK, auto R) -> float {
+    constexpr int b = decltype(BLK)::value, r = decltype(R)::value;
+    if constexpr (b < kAccBlocks) return acc_read<4 * b + r>();
+    else return extra[b - kAccBlocks][r];
+  };
+  const int64_t c_skip = 2ll * m0 * p.ldc;
+  const __amdgpu_buffer_rsrc_t rc =
+      make_rsrc((char*)p.c + c_skip,
+                (uint32_t)(2 * ((int64_t)(p.M - 1) * p.ldc + p.N) - c_skip));
+  const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.bias, p.bias ? 2u * (uint32_t)p.N : 0u);
+  const __amdgpu_buffer_rsrc_t rb2 =
+      make_rsrc(p.bias2, kPair && p.bias2 ? 2u * (uint32_t)p.N : 0u);
+  const uint32_t row0 = (uint32_t)(16 * MB * wm + n);
+  struct Four {
+    float v[4];
+  };
+  auto bias_at = [&](__amdgpu_buffer_rsrc_t r, int col) {
+    const u32x2 b = __builtin_amdgcn_raw_buffer_load_b64(r, 2u * (uint32_t)col, 0, 0);
+    return Four{{__uint_as_float(b[0] << 16), __uint_as_float(b[0] & 0xffff0000u),
+                 __uint_as_float(b[1] << 16), __uint_as_float(b[1] & 0xffff0000u)}};
+  };
+  // two blocks of 16 columns side by side: a quarter trades one of its two runs of four
+  // columns for its neighbour's and has eight in a row
+  constexpr int kPairsOfBlocks = (kPair ? kBlocksN / 2 : kBlocksN) / 2;
+  for_n<kPairsOfBlocks>([&](auto PB) {
+    constexpr int nb = 2 * decltype(PB)::value;
+    const int col = n0 + (kPair ? 64 * wn + 16 * nb
+                          : kSlowN ? 32 * (nb + wn)
+                                   : 32 * NB * wn + 16 * nb);
+    Four bias[2], bias2[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      bias[e] = bias_at(rb, col + 16 * e + 4 * quarter);
+      if (kPair) bias2[e] = bias_at(rb2, col + 16 * e + 4 * quarter);
+    }
+    const int at = col + 16 * (quarter & 1) + 4 * (quarter & 2);
+    for_n<MB>([&](auto MBI) {
+      constexpr int mb = decltype(MBI)::value;
+      auto two = [&](auto E, auto R, const Four* b) {
+        constexpr int e = decltype(E)::value, r = decltype(R)::value;
+        return pack_bf16x2(
+            value(std::integral_constant<int, (nb + e) * MB + mb>{},
+                  std::integral_constant<int, r>{}) + b[e].v[r],
+            value(std::integral_constant<int, (nb + e) * MB + mb>{},
+                  std::integral_constant<int, r + 1>{}) + b[e].v[r + 1]);
+      };
+      uint32_t w[2][2];
+      for_n<2>([&](auto E) {
+        for_n<2>([&](auto R) {
+          constexpr int e = decltype(E)::value, r = 2 * decltype(R)::value;
+          const uint32_t one = two(E, std::integral_constant<int, r>{}, bias);
+          if constexpr (kPair) {
+            constexpr int b = (kBlocksN / 2 + nb + e) * MB + mb;
+            using Blk = std::integral_constant<int, b>;
+            const uint32_t up = pack_bf16x2(
+                value(Blk{}, std::integral_constant<int, r>{}) + bias2[e].v[r],
+                value(Blk{}, std::integral_constant<int, r + 1>{}) + bias2[e].v[r + 1]);
+            w[e][r / 2] = gelu_mul_bf16x2(up, one);
+          } else {
+            w[e][r / 2] = one;
+          }
+        });
+      });
+      const auto s0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+      const auto s1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+      buffer_store_16(u32x4{s0[0], s1[0], s0[1], s1[1]}, rc,
+                      at < p.N ? (row0 + 16 * mb) * 2u * (uint32_t)p.ldc + 2u * (uint32_t)at
+                               : kBufferOutOfRange,
+                      0);
+    });
+  });
+}
+
+constexpr int kCus = 256;
+
+template <int KIND, int MB, int NB>
+hipError_t launch_tiles(MatmulArgs& a, hipStream_t s) {
+  constexpr int kTileN = KIND == kMatmulGeluPair ? 32 * NB : 64 * NB;
+  constexpr int kLds = 2 * (MB / 2 + NB) * kPanelBytes + 4 * 256;
+  static OncePerDevice once;
+  hipError_t e = set_max_dynamic_lds(
+      once, (const void*)matmul_bf16_kernel<KIND, MB, NB>, kLds);
+  if (e != hipSuccess) return e;
+  int64_t tiles = 0;
+  for (int i = 0; i < a.count; ++i) {
+    a.p[i].first_tile = (int)tiles;
+    tiles += (int64_t)((a.p[i].M + 32 * MB - 1) / (32 * MB)) *
+             ((a.p[i].N + kTileN - 1) / kTileN);
+  }
+  matmul_bf16_kernel<KIND, MB, NB><<<dim3((unsigned)tiles), 256, kLds, s>>>(a);
+  return hipGetLastError();
+}
+
+template <int KIND>
+hipError_t launch_kind(MatmulArgs& a, int tile, hipStream_t s) {
+  if (tile == 0) return launch_tiles<KIND, 8, 4>(a, s);
+  if (tile == 2) return launch_tiles<KIND, 4, 4>(a, s);
+  if constexpr (KIND != kMatmulGeluPair) {
+    if (tile == 1) return launch_tiles<KIND, 8, 5>(a, s);
+    if (tile == 3) return launch_tiles<KIND, 4, 5>(a, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+// A tile's time in microseconds: per step of the contraction and beside it (measured at
+// 8192 and 16000 rows of 2560 to 7680 and 8192 x 4096 x 4096).
+struct Tile {
+  int rows, cols;
+  float step_us, fixed_us;
+};
+constexpr Tile kTiles[4] = {{256, 256, 1.37f, 9.0f},
+                            {256, 320, 1.78f, 10.0f},
+                            {128, 256, 0.80f, 7.0f},
+                            {128, 320, 1.00f, 7.0f}};
+
+int64_t tiles_of(const MatmulProblem& p, int rows, int cols) {
+  return (int64_t)((p.M + rows - 1) / rows) * ((p.N + cols - 1) / cols);
+}
+int steps_of(const MatmulProblem& p, int kind) {
+  const int one = (p.K + kStep - 1) / kStep;
+  return kind == kMatmulBack && p.m2 ? 2 * one : one;
+}
+float rounds(int64_t tiles) { return (float)((tiles + kCus - 1) / kCus); }
+
+// The tile with which a launch takes least, in whole rounds of the chip.
+float best_tile(const MatmulArgs& a, int kind, int* tile) {
+  float best = 0.0f;
+  *tile = -1;
+  for (int t = 0; t < 4; ++t) {
+    if (kind == kMatmulGeluPair && (t & 1)) continue;
+    const int cols = kind == kMatmulGeluPair ? kTiles[t].cols / 2 : kTiles[t].cols;
+    int64_t tiles = 0;
+    int steps = 0;
+    for (int i = 0; i < a.count; ++i) {
+      tiles += tiles_of(a.p[i], kTiles[t].rows, cols);
+      const int n = steps_of(a.p[i], kind);
+      if (n > steps) steps = n;
+    }
+    const float us = rounds(tiles) * (kTiles[t].fixed_us + steps * kTiles[t].step_us);
+    if (*tile < 0 || us < best) {
+      best = us;
+      *tile = t;
+    }
+  }
+  return best;
+}
+
+bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+}  // namespace
+
+// What the kernel can address: 16-byte loads and stores, offsets below 2^31.
+bool matmul_serves(const MatmulArgs& a, int kind) {
+  if (a.count < 1 || a.count > kMaxMatmuls) return false;
+  for (int i = 0; i < a.count; ++i) {
+    const MatmulProblem& p = a.p[i];
+    if (p.M < 1 || p.N < 8 || p.K < 1 || p.N % 8) return false;
+    if (kind == kMatmulWeights ? p.M % 8 : p.K % kStep) return false;
+    if ((p.ldm | p.ldn | p.ldc) % 8) return false;
+    const int64_t rows_m = kind == kMatmulWeights ? p.K : p.M;
+    const int64_t rows_n = kind == kMatmulForward ? p.N : p.K;
+    // (a step past the end is asked for, and found out of range)
+    if (rows_m >= (1 << 30) || rows_n >= (1 << 30) ||
+        (rows_m + 512) * p.ldm >= (1ll << 30) || (rows_n + 512) * p.ldn >= (1ll << 30) ||
+        ((int64_t)p.M + 512) * p.ldc >= (1ll << 30))
+      return false;
+    for (const void* t : {p.m, p.n, p.m2, p.n2, p.bias, p.bias2, (const void*)p.c})
+      if (!aligned(t)) return false;
+    if (tiles_of(p, 128, 128) > (1 << 28)) return false;
+  }
+  return true;
+}
+
+// Whether a launch is ahead of the library's products, one by one.  Their time: whole
+// rounds of 256 x 256 tiles at 1.3 us a step, or (few tiles) some 1.2 PFLOP/s, and what a
+// launch costs; with the weights [in, out] 1.35 and 12 us.  Measured over 256 to 32768
+// rows, widths 2560 and 4096 (library / this, us): forward 8192 x 2560 x 2560 93 / 74,
+// two of them 189 / 147, 16376 rows 233 / 149, 2048 rows 31 / 39, two of them 60 / 44,
+// 8192 x 4096 x 4096 171 / 184 (its 256 x 256 tiles come out even); back 8192 x 2560 x
+// 2560 109 / 74, through two layers 230 / 138, 1500 rows 56 / 72.  Weight gradients, whose
+// contraction fills every tile whatever the rows, and the pair with its join (8192 rows,
+// 2560 -> 7680: 494 + 60 / 481) are ahead at all sizes: three of 2560 x 2560 over 256
+// rows 60 / 21, 1000 rows 87 / 37, 8192 rows 407 / 211, one of 4096 x 4096 over 8192 rows
+// 237 / 181 (one of 2560 x 2560 alone 113 / 114).
+bool matmul_pays(const MatmulArgs& a, int kind) {
+  if (!matmul_serves(a, kind)) return false;
+  if (kind == kMatmulWeights) return true;
+  int tile;
+  const float own = best_tile(a, kind, &tile);
+  float library = 0.0f;
+  for (int i = 0; i < a.count; ++i) {
+    const MatmulProblem& p = a.p[i];
+    const float gflop = 2e-9f * (float)p.M * (float)p.N * (float)p.K;
+    const int steps = (p.K + kStep - 1) / kStep;
+    if (kind == kMatmulForward) {
+      const float whole = rounds(tiles_of(p, 256, 256)) * (6.0f + 1.3f * steps);
+      const float few = 6.0f + gflop / 1.2f;
+      library += whole < few ? whole : few;
+    } else {
+      library += (p.n2 ? 2.0f : 1.0f) * (12.0f + gflop / 1.35f);
+      if (kind == kMatmulGeluPair) library += 3.0f + 1.2e-6f * (float)p.M * (float)p.N;
+    }
+  }
+  return own < library;
+}
+
+hipError_t launch_matmul(MatmulArgs a, int kind, hipStream_t s) {
+  if (!matmul_serves(a, kind)) return hipErrorInvalidValue;
+  int tile;
+  best_tile(a, kind, &tile);
+  if (kind == kMatmulForward) return launch_kind<kMatmulForward>(a, tile, s);
+  if (kind == kMatmulBack) return launch_kind<kMatmulBack>(a, tile, s);
+  if (kind == kMatmulWeights) return launch_kind<kMatmulWeights>(a, tile, s);
+  if (kind == kMatmulGeluPair) return launch_kind<kMatmulGeluPair>(a, tile, s);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace rg

@@ -62,6 +62,32 @@ int rg_linear_scan_backward_best(const void* dy, const void* a, const void* rese
  * not: mode 0 the plain forward, 1 the plain backward, 2 and 3 the gated ones. */
 size_t rg_scan_deal_bytes(int B, int T, int W, int dtype, int mode);
 
+/* Linear layers of many rows that share their input, as one launch (bf16): out[i]
+ * [M,N[i]] = x [M,K] . w[i] [N[i],K]^T + bias[i] (bias or an entry of it NULL: none), and
+ * the stacked layer of the MLP with its join, out [M,N] = gelu(x . w[0] + bias[0]) *
+ * (x . w[1] + bias[1]) with w [2,K,N], bias [2,N] or NULL.  Float32 sums, each product
+ * rounded once; K a multiple of 64, N of 8, else RG_ERR_UNSUPPORTED.  *_pays: whether
+ * that is ahead of the library's products. */
+int rg_linear_many_pays(int64_t M, int K, int count, const int* N, int dtype);
+int rg_linear_many(const void* x, int64_t M, int K, int count, const void* const* w,
+                   const void* const* bias, void* const* out, const int* N, int dtype,
+                   void* stream);
+int rg_linear_gelu_pair_pays(int64_t M, int K, int N, int dtype);
+int rg_linear_gelu_pair(const void* x, const void* w, const void* bias, void* out,
+                        int64_t M, int K, int N, int dtype, void* stream);
+
+/* What such layers give back: dx [M,N] = dy [M,K] . w [K,N] (+ dy2 . w2 of the same
+ * sizes: two layers that read the same x; both NULL: none), one rounding; and dw[i]
+ * [out_features[i], in_features[i]] = dy[i] [M,out]^T . x[i] [M,in], up to four as one
+ * launch, which is ahead of the library's products wherever it is supported (features in
+ * multiples of 8, any M). */
+int rg_linear_back_pays(int64_t M, int K, int N, int two, int dtype);
+int rg_linear_back(const void* dy, const void* w, const void* dy2, const void* w2,
+                   void* dx, int64_t M, int K, int N, int dtype, void* stream);
+int rg_linear_weight_grads(const void* const* dy, const void* const* x, void* const* dw,
+                           const int* out_features, const int* in_features, int count,
+                           int64_t M, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -489,6 +489,81 @@ struct Rglru : Function<Rglru> {
 
 // --------------------------------------------------------- recurrent block --
 
+// x [M, K] through layers that share it, each [M, N] of `out` written: one launch where
+// that is ahead of the library's products.
+void linear_forward(const Tensor& x, std::initializer_list<const Tensor*> w,
+                    std::initializer_list<const Tensor*> b,
+                    std::initializer_list<const Tensor*> out_, const Dims& d) {
+  const void *ws[rg::kMaxMatmuls], *bs[rg::kMaxMatmuls];
+  void* outs[rg::kMaxMatmuls];
+  int n[rg::kMaxMatmuls];
+  const int count = (int)w.size();
+  for (int i = 0; i < count; ++i) {
+    ws[i] = in(*w.begin()[i]);
+    bs[i] = in(*b.begin()[i]);
+    outs[i] = out(*out_.begin()[i]);
+    n[i] = (int)w.begin()[i]->size(0);
+  }
+  const int K = (int)x.size(1);
+  if (rg_linear_many_pays(x.size(0), K, count, n, d.code)) {
+    check(rg_linear_many(in(x), x.size(0), K, count, ws, bs, outs, n, d.code, d.stream));
+    return;
+  }
+  for (int i = 0; i < count; ++i) {
+    Tensor y = *out_.begin()[i];
+    at::addmm_out(y, *b.begin()[i], x, w.begin()[i]->t());
+  }
+}
+
+// dy [M, N] back through w [N, K], and dy2 through w2 where there is one (two layers
+// that read the same input).
+Tensor linear_back(const Tensor& dy, const Tensor& w, const Tensor& dy2, const Tensor& w2,
+                   const Dims& d) {
+  const int64_t M = dy.size(0);
+  const int N = (int)dy.size(1), K = (int)w.size(1);
+  Tensor dx = empty({M, K}, dy);
+  if (rg_linear_back_pays(M, N, K, dy2.defined(), d.code)) {
+    check(rg_linear_back(in(dy), in(w), in(dy2), dy2.defined() ? in(w2) : nullptr,
+                         out(dx), M, N, K, d.code, d.stream));
+    return dx;
+  }
+  at::mm_out(dx, dy, w);
+  if (dy2.defined()) dx.addmm_(dy2, w2);
+  return dx;
+}
+
+// The weights' gradients of layers side by side: 100 tiles of a 2560 x 2560 each, whose
+// contraction is the rows, leave the chip half idle one by one.
+struct LinearWeights {
+  std::vector<Tensor> dy, x;
+  std::vector<Tensor*> dw;
+  void add(const Tensor& dy_, const Tensor& x_, Tensor* to) {
+    dy.push_back(dy_);
+    x.push_back(x_);
+    dw.push_back(to);
+  }
+  void launch(const Dims& d) {
+    const void *dys[rg::kMaxMatmuls], *xs[rg::kMaxMatmuls];
+    void* dws[rg::kMaxMatmuls];
+    int n[rg::kMaxMatmuls], k[rg::kMaxMatmuls];
+    for (size_t i = 0; i < dw.size(); ++i) {
+      n[i] = (int)dy[i].size(1);
+      k[i] = (int)x[i].size(1);
+      *dw[i] = empty({n[i], k[i]}, x[i]);
+      dys[i] = in(dy[i]);
+      xs[i] = in(x[i]);
+      dws[i] = out(*dw[i]);
+    }
+    if (dw.empty()) return;
+    int rc = RG_ERR_UNSUPPORTED;
+    if (d.code == RG_DTYPE_BF16)
+      rc = rg_linear_weight_grads(dys, xs, dws, n, k, (int)dw.size(), d.M(), d.code,
+                                  d.stream);
+    if (rc != RG_ERR_UNSUPPORTED) return check(rc);
+    for (size_t i = 0; i < dw.size(); ++i) at::mm_out(*dw[i], dy[i].t(), x[i]);
+  }
+};
+
 // (modules.py:605-655 of the reference, without a cache)
 struct Block : Function<Block> {
   static variable_list forward(AutogradContext* ctx, Tensor x, Tensor pos,
@@ -498,9 +573,12 @@ struct Block : Function<Block> {
                                Tensor w_out, Tensor b_out, bool want_cache) {
     ctx->set_materialize_grads(false);
     const int64_t B = x.size(0), T = x.size(1), W = w_y.size(0);
-    Tensor x2 = x.view({B * T, x.size(2)});
-    Tensor gate = at::linear(x2, w_y, b_y).view({B, T, W});
-    Tensor lx = at::linear(x2, w_lx, b_lx).view({B, T, W});
+    const int64_t D = x.size(2);
+    Tensor x2 = x.view({B * T, D});
+    Tensor gate = empty({B * T, W}, x), lx = empty({B * T, W}, x);
+    linear_forward(x2, {&w_y, &w_lx}, {&b_y, &b_lx}, {&gate, &lx}, Dims(x));
+    gate = gate.view({B, T, W});
+    lx = lx.view({B, T, W});
     const Dims d(lx);
     Tensor xc = empty(lx.sizes(), x), conv_state, h;
     if (want_cache) {
@@ -517,8 +595,9 @@ struct Block : Function<Block> {
                   kept);
     Tensor join = empty(lx.sizes(), x);
     check(rg_gelu_mul(in(y), in(gate), out(join), d.M() * W, d.code, d.stream));
-    Tensor result = at::linear(join.view({B * T, W}), w_out, b_out)
-                        .view({B, T, w_out.size(0)});
+    Tensor result = empty({B * T, D}, x);
+    linear_forward(join.view({B * T, W}), {&w_out}, {&b_out}, {&result}, d);
+    result = result.view({B, T, D});
     ctx->save_for_backward({x, pos, w_y, w_lx, conv_w, a_param, w_x, w_a,
                             kept.bias, w_out, gate, lx, xc, gx, ga, y, join,
                             kept.starts});
@@ -546,10 +625,9 @@ struct Block : Function<Block> {
     auto needs = [&](int i) { return ctx->needs_input_grad(i); };
     Sums sums;
     variable_list r(16);  // (the flag takes no gradient)
-    Tensor dy, dgate2;
+    Tensor dy, dgate2, dout;
     if (grads[0].defined()) {
-      const Tensor dout =
-          grad_of(grads[0], x.sizes(), x.scalar_type()).view({M, D});
+      dout = grad_of(grads[0], x.sizes(), x.scalar_type()).view({M, D});
       const int64_t parts = (M + rg::kColSumRows - 1) / rg::kColSumRows;
       if (needs(14)) {
         Tensor part = empty({parts, dout.size(1)}, at::kFloat, x);
@@ -558,8 +636,7 @@ struct Block : Function<Block> {
         r[14] = sums.add(part, 0, parts, dout.size(1), dout.size(1),
                          {dout.size(1)}, x);
       }
-      if (needs(13)) r[13] = at::mm(dout.t(), join.view({M, W}));
-      Tensor djoin = at::mm(dout, w_out);
+      const Tensor djoin = linear_back(dout, w_out, Tensor(), Tensor(), d);
       dy = empty(lx.sizes(), x);
       dgate2 = empty({M, W}, x);
       Tensor part = empty({parts, W}, at::kFloat, x);
@@ -567,8 +644,6 @@ struct Block : Function<Block> {
           in(djoin), in(y), in(gate), out(dy), out(dgate2), (float*)out(part), M,
           (int)W, d.code, d.stream));
       if (needs(3)) r[3] = sums.add(part, 0, parts, W, W, {W}, x);
-      if (needs(2)) r[2] = at::mm(dgate2.t(), x2);
-      if (needs(0)) r[0] = at::mm(dgate2, w_y);
     } else {
       dy = at::zeros_like(y);  // only the final state is differentiated
     }
@@ -605,14 +680,13 @@ struct Block : Function<Block> {
     if (needs(7)) r[7] = sums.add(part, 4 * W, chunks, W, 5 * W, {W}, x);
     if (needs(5)) r[5] = sums.add(dlx_part, 0, chunks, W, W, {W}, x);
     sums.launch(d);
-    if (needs(4)) r[4] = at::mm(dlx2.t(), x2);
-    if (needs(0)) {
-      if (r[0].defined())
-        r[0].addmm_(dlx2, w_lx);
-      else
-        r[0] = at::mm(dlx2, w_lx);
-      r[0] = r[0].view(x.sizes());
-    }
+    LinearWeights dw;
+    if (dout.defined() && needs(13)) dw.add(dout, join.view({M, W}), &r[13]);
+    if (dout.defined() && needs(2)) dw.add(dgate2, x2, &r[2]);
+    if (needs(4)) dw.add(dlx2, x2, &r[4]);
+    dw.launch(d);
+    if (needs(0))
+      r[0] = linear_back(dlx2, w_lx, dgate2, w_y, d).view(x.sizes());
     return r;
   }
 };
