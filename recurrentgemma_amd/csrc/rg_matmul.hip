@@ -559,7 +559,7 @@ bool matmul_pays(const MatmulArgs& a, int kind) {
       const float few = 6.0f + gflop / 1.2f;
       library += whole < few ? whole : few;
     } else {
-      library += (p.n2 ? 2.0f : 1.0f) * (12.0f + gflop / 1.35f);
+      library += (kind == kMatmulGeluPair || p.n2 ? 2.0f : 1.0f) * (12.0f + gflop / 1.35f);
       if (kind == kMatmulGeluPair) library += 3.0f + 1.2e-6f * (float)p.M * (float)p.N;
     }
   }

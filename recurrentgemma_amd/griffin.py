@@ -8,10 +8,10 @@ same constructor arguments, parameter names (reference state dicts load
 unchanged), forward signatures and cache tuples.  On this package's kernels:
 the recurrent block, RMSNorm (with the residual sums in front of it), the two
 gelu(a) * b joins, the rotary embedding, the prompt attention and the decode
-step of the attention block (bf16, head_dim 256), the linear layers of a
-decode step of at most 64 rows, the logits' soft cap and the greedy pick.
-Library calls: linear layers with more rows and the logits projection
-(hipBLASLt), attention in other dtypes and head sizes
+step of the attention block (bf16, head_dim 256), the linear layers (bf16: a
+decode step of at most 64 rows; many rows where the library is behind), the
+logits' soft cap and the greedy pick.  Library calls: other linear layers and
+the logits projection (hipBLASLt), attention in other dtypes and head sizes
 (scaled_dot_product_attention / batched products).  It exists so that the
 recurrent path can be exercised and measured inside the model it belongs to.
 Inference only (no autograd through the kernels).
@@ -29,6 +29,7 @@ from typing import Any, NamedTuple
 import torch
 from torch import nn
 
+from recurrentgemma_amd import compiled
 from recurrentgemma_amd import modules
 from recurrentgemma_amd import ops
 
@@ -209,8 +210,15 @@ class MLPBlock(nn.Module):
                                        (self.ffw_down.bias,), addend=residual)
       return self._rows_down(hidden, (self.ffw_down.weight,),
                              (self.ffw_down.bias,), residual=residual)
-    gate, up = self.ffw_up(x)
-    out = self.ffw_down(ops.gelu_mul(up, gate))  # gelu(gate) * up, one pass
+    hidden = None
+    if (not compiled.tracing() and not modules._global_hooks() and
+        modules._as_written(self.ffw_up, _StackedLinear)):
+      hidden = ops.linear_gelu_pair(
+          x, *modules._parameters(self.ffw_up, "w", "b"))
+    if hidden is None:
+      gate, up = self.ffw_up(x)
+      hidden = ops.gelu_mul(up, gate)  # gelu(gate) * up, one pass
+    out, = modules.linears(hidden, self.ffw_down)
     if residual is None:
       return out
     # (many rows: the norm that reads the sum next adds the two in its pass)
@@ -383,7 +391,7 @@ class LocalAttentionBlock(nn.Module):
       q = self._rows_q(x, (self.proj_q.weight,))
       k, v = self._rows_kv(x, (self.proj_k.weight, self.proj_v.weight))
     else:
-      q, k, v = self.proj_q(x), self.proj_k(x), self.proj_v(x)
+      q, k, v = modules.linears(x, self.proj_q, self.proj_k, self.proj_v)
     q = q.reshape(b, t, self.num_heads, self.head_dim)
     k = k.reshape(b, t, 1, self.head_dim)
     v = v.reshape(b, t, 1, self.head_dim)
@@ -455,7 +463,7 @@ class LocalAttentionBlock(nn.Module):
       return self._rows_final.partial(x, weights, biases)
     if ops.PackedLinear.usable(x, self.width, self.width):
       return self._rows_final(x, weights, biases)
-    return self.proj_final(x)
+    return modules.linears(x, self.proj_final)[0]
 
   def _ring_positions(self, num_tokens, t):
     """Positions held by the ring (slot j keeps the largest position congruent

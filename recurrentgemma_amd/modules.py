@@ -3,7 +3,8 @@
 RecurrentBlock / RecurrentBlockCache mirror
 recurrentgemma/torch/modules.py:32-37 and :496-680 (same constructor,
 parameter names, forward signature and cache tuple).  linear_x / linear_y /
-linear_out stay torch.nn.Linear (hipBLASLt); conv_1d -> rg_lru runs as
+linear_out stay torch.nn.Linear, whose products run on this package's kernels
+where those are ahead of hipBLASLt's (linears below, and a few rows); conv_1d -> rg_lru runs as
   prefill: rg_recurrent_core (the single prefill kernel, or rg_gates_gemm with
            the conv on load + rg_lru_scan_fused: the library picks)
   decode : rg_recurrent_step
@@ -58,6 +59,20 @@ def _global_hooks() -> bool:
   m = nn.modules.module
   return bool(m._global_forward_hooks or m._global_forward_pre_hooks or
               m._global_backward_hooks or m._global_backward_pre_hooks)
+
+
+def linears(x, *layers):
+  """The outputs of nn.Linear layers that read x.  Many rows in bf16: one
+  launch (ops.linear_many) where that is ahead of the library, as long as
+  calling the layers is nothing but their products (and no program is being
+  traced: the kernels are reached through ctypes)."""
+  if (not compiled.tracing() and not _global_hooks() and
+      all(_as_written(layer, nn.Linear) for layer in layers)):
+    parts = [_parameters(layer, "weight", "bias") for layer in layers]
+    out = ops.linear_many(x, [w for w, _ in parts], [b for _, b in parts])
+    if out is not None:
+      return out
+  return [layer(x) for layer in layers]
 
 
 def _core_weights(conv_1d, rg_lru):
@@ -225,8 +240,7 @@ class RecurrentBlock(nn.Module):
         w_out, b_out = _parameters(linear["linear_out"], "weight", "bias")
         y, x = self._rows_yx(x, (w_y, w_x), (b_y, b_x))
       else:
-        y = self.linear_y(x)
-        x = self.linear_x(x)
+        y, x = linears(x, self.linear_y, self.linear_x)
       # x * gelu(y) (modules.py:627-628, 644) is part of the core call: inside
       # the prefill kernel where that runs, one pass after it elsewhere
       x, new_cache = recurrent_core(
@@ -239,7 +253,7 @@ class RecurrentBlock(nn.Module):
       elif few_rows:
         x = self._rows_out(x, (w_out,), (b_out,))
       else:
-        x = self.linear_out(x)
+        x, = linears(x, self.linear_out)
     if not return_cache:
       return x, None
     return x, new_cache

@@ -7,6 +7,7 @@ HIP stream.  Nothing here computes on the CPU.
 
 from __future__ import annotations
 
+import ctypes
 import functools
 
 import torch
@@ -554,6 +555,80 @@ def gelu_mul_backward(dout, a, g):
         _p(dout), _p(a), _p(g), _p(d_a), _p(d_g), a.numel(), _dtype_code(a),
         _stream(a)))
   return d_a, d_g
+
+
+@functools.lru_cache(maxsize=1024)
+def _linear_many_pays(M, K, n) -> bool:
+  sizes = (ctypes.c_int * len(n))(*n)
+  return bool(_lib.lib().rg_linear_many_pays(M, K, len(n), sizes,
+                                             _lib.RG_DTYPE_BF16))
+
+
+@functools.lru_cache(maxsize=1024)
+def _linear_gelu_pair_pays(M, K, N) -> bool:
+  return bool(_lib.lib().rg_linear_gelu_pair_pays(M, K, N,
+                                                  _lib.RG_DTYPE_BF16))
+
+
+def _as_they_lie(x, *others) -> bool:
+  """Whether kernels may read x (bf16) and the others where they lie instead
+  of torch's operators: plain dense tensors of one device and dtype, nothing
+  that autograd or autocast would see."""
+  grad = torch.is_grad_enabled()
+  return not torch.is_autocast_enabled("cuda") and all(
+      t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and
+                    t.dtype == torch.bfloat16 and t.device == x.device and
+                    t.is_contiguous() and not (grad and t.requires_grad) and
+                    t.data_ptr() % 16 == 0)
+      for t in (x, *others))
+
+
+def _rows(x) -> int:
+  """Rows of x [..., K] that a many-row linear layer may take, else 0."""
+  if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() and x.numel()):
+    return 0
+  return x.numel() // x.shape[-1]
+
+
+def linear_many(x, weights, biases):
+  """x [..., K] through layers that read it (weights [N_i, K], biases [N_i] or
+  None): one launch (rg_linear_many) where that is ahead of the library's
+  products and the tensors are as the kernel takes them, else None."""
+  M = _rows(x)
+  if not M or any(w.dim() != 2 for w in weights):
+    return None
+  K = x.shape[-1]
+  n = tuple(w.shape[0] for w in weights)
+  if (not _linear_many_pays(M, K, n) or any(w.shape[1] != K for w in weights) or
+      any(b is not None and b.shape != (m,) for b, m in zip(biases, n)) or
+      not _as_they_lie(x, *weights, *biases)):
+    return None
+  out = [torch.empty((*x.shape[:-1], m), dtype=x.dtype, device=x.device)
+         for m in n]
+  pointers = ctypes.c_void_p * len(n)
+  with _on(x.device):
+    _lib.check(_lib.lib().rg_linear_many(
+        _p(x), M, K, len(n), pointers(*map(_p, weights)),
+        pointers(*map(_p, biases)), pointers(*map(_p, out)),
+        (ctypes.c_int * len(n))(*n), _lib.RG_DTYPE_BF16, _stream(x)))
+  return out
+
+
+def linear_gelu_pair(x, w, b):
+  """gelu(x w[0] + b[0]) * (x w[1] + b[1]) for x [..., K], w [2, K, N], b of
+  2 N values (modules.py:752-757) as one launch, else None, as linear_many."""
+  M = _rows(x)
+  if not M or w.dim() != 3 or w.shape[:2] != (2, x.shape[-1]):
+    return None
+  K, N = w.shape[1:]
+  if (not _linear_gelu_pair_pays(M, K, N) or b.numel() != 2 * N or N % 8 or
+      not _as_they_lie(x, w, b)):
+    return None
+  out = torch.empty((*x.shape[:-1], N), dtype=x.dtype, device=x.device)
+  with _on(x.device):
+    _lib.check(_lib.lib().rg_linear_gelu_pair(
+        _p(x), _p(w), _p(b), _p(out), M, K, N, _lib.RG_DTYPE_BF16, _stream(x)))
+  return out
 
 
 def rms_norm(x, scale, eps=1e-6):

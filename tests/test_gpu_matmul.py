@@ -144,3 +144,47 @@ def test_what_does_not_fit_is_refused():
   assert rc != _lib.RG_OK  # 96 is no multiple of 64
   assert not _lib.lib().rg_linear_many_pays(64, 96, 1, ints([64]), _lib.RG_DTYPE_BF16)
   assert not _lib.lib().rg_linear_many_pays(8192, 2560, 1, ints([2560]), _lib.RG_DTYPE_F32)
+
+
+def test_layers_of_the_modules(monkeypatch):
+  """Calls that take the launches, and those that must not: a hooked layer, a
+  layer under autocast, weights that want gradients, a view."""
+  from recurrentgemma_amd import griffin, modules
+  layers = [torch.nn.Linear(2560, n, device="cuda", dtype=BF16) for n in (2560, 2560)]
+  mlp = griffin.MLPBlock(512, 1536, device="cuda", dtype=BF16)
+  x, xm = normal(1, 8, 512, 2560), normal(2, 2, 2048, 512)
+  taken = []
+  many, pair = ops.linear_many, ops.linear_gelu_pair
+  note = lambda f: lambda *a: (taken.append(f(*a) is not None), f(*a))[1]
+  monkeypatch.setattr(ops, "linear_many", note(many))
+  monkeypatch.setattr(ops, "linear_gelu_pair", note(pair))
+
+  def run(want):
+    taken.clear()
+    out = modules.linears(x, *layers)
+    assert taken == want
+    for y, layer in zip(out, layers):
+      ref = x.double() @ layer.weight.double().t() + layer.bias.double()
+      assert ((y.double() - ref).norm() / ref.norm()).item() < 4e-3  # one rounding
+    return out
+
+  with torch.no_grad():
+    run([True])
+    called = []
+    h = layers[1].register_forward_hook(lambda *a: called.append(1))
+    run([])
+    assert called
+    h.remove()
+    with torch.autocast("cuda", dtype=BF16):
+      run([False])
+    x = normal(1, 8, 512, 2568)[..., 8:]
+    run([False])
+    taken.clear()
+    out = mlp(xm)
+    assert taken[0]
+    gate, up = mlp.ffw_up(xm)
+    ref = mlp.ffw_down(ops.gelu_mul(up, gate))
+    assert ((out.double() - ref.double()).norm() / ref.double().norm()).item() < 6e-3
+  x = normal(1, 8, 512, 2560)
+  run([False])
+  assert all(y.requires_grad for y in modules.linears(x, *layers))
