@@ -1489,7 +1489,7 @@ int rg_attention_prefill(const void* q, const void* k, const void* v_t,
   rg::AttnPrefillArgs a{};
   a.q = q;
   a.k = k;
-  a.v_t = v_t;
+  a.v = v_t;
   a.lo = first_key;
   a.out = out;
   a.B = B;
@@ -1518,9 +1518,8 @@ int rg_attention_first_key(const void* positions, int positions_is_i64,
 
 size_t rg_attention_prompt_workspace_bytes(int B, int T) {
   if (B <= 0 || T <= 0) return 0;
-  const size_t t_pad = ((size_t)T + 63) / 64 * 64;
-  // rotated keys, transposed values, sines and cosines
-  return (size_t)B * ((size_t)T * 512 + t_pad * 512 + (size_t)T * 256);
+  // rotated keys, sines and cosines
+  return (size_t)B * T * (512 + 256);
 }
 
 int rg_attention_prompt(const void* q, const void* k, const void* v,
@@ -1538,9 +1537,7 @@ int rg_attention_prompt(const void* q, const void* k, const void* v,
     return fail(RG_ERR_UNSUPPORTED,
                 "%s: needs bf16 and head_dim == 256 (dtype=%d head_dim=%d)",
                 __func__, dtype, head_dim);
-  const int64_t t_pad = ((int64_t)T + 63) / 64 * 64;
-  RG_REQUIRE((int64_t)T * H * 512 < ((int64_t)1 << 31) &&
-                 t_pad * 512 < ((int64_t)1 << 31),
+  RG_REQUIRE((int64_t)T * H * 512 < ((int64_t)1 << 31),
              "%s: T=%d H=%d: a row's queries exceed 2 GiB", __func__, T, H);
   RG_CHECK_PTR(q);
   RG_CHECK_PTR(k);
@@ -1564,26 +1561,23 @@ int rg_attention_prompt(const void* q, const void* k, const void* v,
   p.pos_kind = positions_is_i64 ? 1 : 0;
   p.inv_freq = inv_freq;
   p.k_rot = (uint16_t*)workspace;
-  p.v_t = p.k_rot + (int64_t)B * T * 256;
-  p.rope_table = (uint32_t*)(p.v_t + (int64_t)B * t_pad * 256);
+  p.rope_table = (uint32_t*)(p.k_rot + (int64_t)B * T * 256);
   p.ring_k = (uint16_t*)ring_keys;
   p.ring_v = (uint16_t*)ring_values;
   p.num_tokens = num_tokens;
   p.B = B;
   p.T = T;
-  p.T_pad = (int)t_pad;
   p.window = window;
   hipError_t e = rg::launch_attn_prompt_prepare(p, (hipStream_t)stream);
   if (e != hipSuccess) return launch_status(__func__, e);
   rg::AttnPrefillArgs a{};
   a.q = q;
   a.k = p.k_rot;
-  a.v_t = p.v_t;
+  a.v = p.v;
   a.lo = first_key;
   a.out = out;
   a.B = B;
   a.T = T;
-  a.T_pad = (int)t_pad;
   a.H = H;
   a.scale = scale;
   a.rope_table = p.rope_table;

@@ -8,25 +8,38 @@
 // lo[t] = max(first token of t's document, t - window) is supplied by the
 // caller (non-decreasing in t).
 //
-// One workgroup of four waves per (row, head, 128 queries); a wave owns 32
-// queries.  Keys and values come by in tiles of 64 keys, staged in LDS for the
-// four waves.  Both products are v_mfma_f32_32x32x16_bf16 with the QUERIES as
-// the 32 columns of the result:
-//   S^T [32 keys x 32 queries]  = K tile [32 x 256]   x Q^T [256 x 32]
-//   O^T [256 x 32 queries]     += V^T tile [256 x 32] x P^T [32 keys x 32]
-// so a lane (query l % 32, half l / 32) holds, of every result, one query's
-// values: the softmax statistics of a query are per-lane scalars (one exchange
-// between the two halves per tile), the 16 scores a lane holds become, as they
-// lie, its operand of the second product, and rescaling O is a multiplication
-// by a per-lane scalar.  Which keys sit in which contraction slot of the second
-// product is free as long as both operands agree: the S^T result gives half h
-// of a lane the keys 8 j + 4 h + i (j = 0..3, i = 0..3), so the values are laid
-// out in LDS in that order.  The values arrive transposed ([row, 256, T]: the
-// caller's one extra pass over them), which makes the contraction index the
-// contiguous one of both operands of both products.
+// A wave owns 48 queries of one head, a workgroup four such waves: heads of the same queries first, since all heads read the same keys and
+// values.  They come by in blocks of 32 keys, global -> LDS by the memory pipe, three
+// blocks ahead (a ring of four each), one barrier per block.  Both products are
+// v_mfma_f32_16x16x32_bf16 with the QUERIES as the 16 columns of the result:
+//   S^T [16 keys x 16 queries]  = K [16 x 256]     x Q^T [256 x 16]
+//   O^T [16 dims x 16 queries] += V^T [16 x 32 keys] x P^T [32 keys x 16]
+// so a lane (query l % 16, quarter l / 16) holds, of every result, one query's values:
+// the softmax statistics of a query are per-lane scalars, the 8 scores a lane holds of
+// a query become, as they lie, its operand of the second product, and rescaling O is a
+// multiplication by a per-lane scalar.  Which keys sit in which contraction slot of the
+// second product is free as long as both operands agree: the S^T results give quarter g
+// the keys 4 g + i and 16 + 4 g + i (i = 0..3), and so the values are read from LDS, by
+// ds_read_b64_tr_b16 where they lie key by key.
 //
-// What a block does around that for a prompt -- rotary embedding, the values'
-// transposition, the ring cache it leaves -- is attn_prompt_prepare_kernel at
+// One wave per SIMD, so what it overlaps it overlaps by its own order: the scores of
+// block j + 1 are multiplied while block j's go through their exponentials (phase A, 48
+// matrix instructions with two steps of the softmax behind each), then the values of
+// block j with the maxima of block j + 1 and the next loads between (phase B).  48
+// queries a wave because LDS is the tightest resource: a key or value read from it is
+// multiplied by three times 16 queries.  (64 queries are 256 accumulators, 128 registers of
+// queries and 48 of scores, more than there are.)
+//
+// 8 x 2047 tokens, 10 heads: 185-200 us where all rows are full (0.9 PFLOP/s of the visible
+// pairs), 155 left-padded by 0 to half; 290-320 and 290 with 32 queries a wave on
+// v_mfma_f32_32x32x16_bf16, tiles of 64 keys through registers, scores, softmax and values
+// one after the other, a row to an XCD.  What is left: a block takes 2450 cycles where its
+// matrix instructions take 1540 (what is issued between them counts in full from two
+// instructions on), and 18000 before the first (the queries' way from memory, all
+// workgroups at once, and their rotation).
+//
+// What a block does around that for a prompt -- rotary embedding, the ring cache
+// it leaves -- is attn_prompt_prepare_kernel at
 // the end of this file; the queries take their rotary embedding inside the
 // attention kernel.
 #include <utility>
@@ -37,18 +50,18 @@
 namespace rg {
 namespace {
 
+#define RG_INLINE __attribute__((always_inline))
 constexpr int kAttnHd = 256;
-constexpr int kAttnQ = 128;  // queries per workgroup
-constexpr int kAttnK = 64;   // keys per tile
-constexpr int kAttnKB = kAttnK / 32;  // blocks of 32 keys (one S^T result each)
-constexpr int kAttnChunks = kAttnK * 32 / 256;  // 16-byte chunks per thread, tile and tensor
-// K tile rows (one key, 512 B) padded to 528 B, V^T tile rows (one of the 256
-// dimensions, 64 keys = 128 B) to 144 B: the 16-byte operand reads of 16
-// consecutive rows fall on distinct banks.
-constexpr int kKRowBytes = 528;
-constexpr int kVRowBytes = 2 * kAttnK + 16;
-constexpr int kKTileBytes = kAttnK * kKRowBytes;
-constexpr int kVTileBytes = kAttnHd * kVRowBytes;
+constexpr int kBlockKeys = 32;
+constexpr int kBlockBytes = kBlockKeys * kAttnHd * 2;
+constexpr int kRing = 4;  // blocks of keys, and of values, in LDS
+constexpr int kAttnLds = 2 * kRing * kBlockBytes;
+
+typedef __attribute__((address_space(3))) unsigned char lds_byte;
+typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 union AFrag {
   bf16x8 v;
@@ -56,16 +69,13 @@ union AFrag {
   uint32_t u[4];
 };
 
-// The 128 output accumulators of a lane (O^T: 8 blocks of 32 dimensions, 16
-// registers each) live in the accumulation registers a[0:127] for the whole
-// kernel, written and read by inline assembly with the register numbers
-// spelled out: the second product accumulates into them tile after tile, and
-// nothing else touches them but the rare rescaling and the final store (left
-// to the register allocator they were moved between the two register files
-// every tile, 256 moves for 32 matrix instructions).  The build checks that
-// the compiler allocates no accumulation register of its own in this file.
-#define RG_ATTN_LAST_AGPR "a127"
-
+// The output accumulators of a lane (O^T: 16 blocks of 16 dimensions by QB blocks of 16
+// queries, 4 registers each) live in the accumulation registers a[0:255] for the whole
+// kernel, written and read by inline assembly with the register numbers spelled out:
+// nothing but the second product, the rare rescaling and the final store touches them
+// (left to the register allocator they were moved between the two register files every
+// block).  The build checks that the compiler allocates no accumulation register of its
+// own in this file.
 template <int N>
 __device__ __forceinline__ float acc_read() {
   float t;
@@ -74,44 +84,54 @@ __device__ __forceinline__ float acc_read() {
 }
 template <int N>
 __device__ __forceinline__ void acc_write(float t) {
-  asm volatile("v_accvgpr_write_b32 a[%c1], %0" ::"v"(t), "n"(N)
-               : RG_ATTN_LAST_AGPR);
+  asm volatile("v_accvgpr_write_b32 a[%c1], %0" ::"v"(t), "n"(N));
 }
-template <int... I>
-__device__ __forceinline__ void acc_fill(float v,
-                                         std::integer_sequence<int, I...>) {
-  (acc_write<I>(v), ...);
-}
-template <int... I>
-__device__ __forceinline__ void acc_scale(float f,
-                                          std::integer_sequence<int, I...>) {
-  (acc_write<I>(acc_read<I>() * f), ...);
+template <int N>
+__device__ __forceinline__ void acc_zero() {
+  asm volatile("v_accvgpr_write_b32 a[%c0], 0" ::"n"(N));
 }
 // block BLK of O^T += a x b
 template <int BLK>
 __device__ __forceinline__ void acc_mfma(const f32x4& a, const f32x4& b) {
-  asm volatile(
-      "v_mfma_f32_32x32x16_bf16 a[%c2:%c2+15], %0, %1, a[%c2:%c2+15]" ::"v"(a),
-      "v"(b), "n"(16 * BLK)
-      : RG_ATTN_LAST_AGPR);
+  asm volatile("v_mfma_f32_16x16x32_bf16 a[%c2:%c2+3], %0, %1, a[%c2:%c2+3]" ::"v"(a),
+               "v"(b), "n"(4 * BLK));
+}
+template <int... I, class F>
+__device__ __forceinline__ void for_each(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void for_n(F&& f) {
+  for_each(std::make_integer_sequence<int, N>{}, f);
+}
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
 }
 // The compiler does not count the wait states between a matrix instruction in
 // inline assembly and a read of its result.
 __device__ __forceinline__ void wait_for_matrix_results() {
   asm volatile("s_nop 15\n\ts_nop 7");
 }
+__device__ __forceinline__ u32x4 scalar_rsrc(const void* base, uint32_t bytes) {
+  const uint64_t at = (uint64_t)base;
+  return u32x4{
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at),
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) & 0xffffu,
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
 
 // Rotary embedding of the first half of a query's dimensions (elements i and
-// i + 64, i < 64) where the query lies as operand fragments: k-steps 0..3 hold
-// this lane's elements 16 ks + 8 half + 0..7, k-steps 4..7 their partners.
-// `table` is the query's row of sines and cosines (see
+// i + 64, i < 64) where the query lies as operand fragments: k-steps 0 and 1 hold
+// this lane's elements 32 ks + 8 quarter + 0..7, k-steps 2 and 3 their partners.
+// `table` is the lane's share of the query's row of sines and cosines (see
 // attn_prompt_prepare_kernel).  The arithmetic of rg_rope_pair, element for
 // element: products and sums rounded one by one.
-__device__ __forceinline__ void rotate_query(AFrag (&qf)[16],
-                                             const u32x4 (&table)[8]) {
+__device__ __forceinline__ void rotate_query(AFrag (&qf)[8], const u32x4 (&table)[4]) {
 #pragma clang fp contract(off)
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
+  for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       float vlo[2], vhi[2];
@@ -120,354 +140,457 @@ __device__ __forceinline__ void rotate_query(AFrag (&qf)[16],
         const uint32_t sc = table[2 * ks + (w >> 1)][2 * (w & 1) + e];
         const float sn = __uint_as_float(sc << 16);
         const float cs = __uint_as_float(sc & 0xffff0000u);
-        const uint32_t l = qf[ks].u[w], h = qf[ks + 4].u[w];
+        const uint32_t l = qf[ks].u[w], h = qf[ks + 2].u[w];
         const float lo = __uint_as_float(e == 0 ? l << 16 : l & 0xffff0000u);
         const float hi = __uint_as_float(e == 0 ? h << 16 : h & 0xffff0000u);
         vlo[e] = round_to_bf16(lo * cs) - round_to_bf16(hi * sn);
         vhi[e] = round_to_bf16(hi * cs) + round_to_bf16(lo * sn);
       }
       qf[ks].u[w] = pack_bf16x2(vlo[0], vlo[1]);
-      qf[ks + 4].u[w] = pack_bf16x2(vhi[0], vhi[1]);
+      qf[ks + 2].u[w] = pack_bf16x2(vhi[0], vhi[1]);
     }
   }
 }
+
+// Below every score that is a number, in units of log2: the running maximum before a
+// query's first visible key (a masked score is minus infinity).
+constexpr float kNoMaximum = -3.0e38f;
 
 // ROPE: the queries come before their rotary embedding and take it here, in
 // the registers they are loaded to (p.rope_table); a pass of its own over them
 // reads and writes every query once more (8 x 2047 tokens, 10 heads: 43 us).
-template <bool ROPE>
-__global__ void __launch_bounds__(256)
+// COLUMNS: the values come transposed, [row, 256, T_pad], else key by key.
+// QB: blocks of 16 queries per wave.
+template <bool ROPE, bool COLUMNS, int QB>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 attn_prefill_bf16_kernel(AttnPrefillArgs p) {
   extern __shared__ __align__(16) unsigned char attn_lds[];
-  unsigned char* const k_tile = attn_lds;                    // two buffers
-  unsigned char* const v_tile = attn_lds + 2 * kKTileBytes;  // two buffers
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_byte*)attn_lds;
+  constexpr int kQ = 16 * QB;       // queries per wave
+  constexpr int kMfmas = 16 * QB;   // of either product, per block of keys
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n = lane & 31, half = lane >> 5;
-  const int qtiles = (p.T + kAttnQ - 1) / kAttnQ;
-  // Workgroups go to the eight XCDs in turn (linear id modulo 8), each with an
-  // L2 of its own: the ids are dealt out so that one XCD gets a contiguous run
-  // of (row, head, query tile) triples, i.e. a row's keys and values are
-  // pulled through one L2 instead of all eight.
-  unsigned id = blockIdx.x;
-  {
-    const unsigned per_xcd = gridDim.x / 8;
-    if (id < 8 * per_xcd) id = (id & 7) * per_xcd + (id >> 3);
-  }
-  // the longest workgroups (last query tiles) first
-  const int qt = qtiles - 1 - (int)(id % qtiles);
-  const int head = (int)(id / qtiles) % p.H;
-  const int b = (int)(id / qtiles) / p.H;
-  const int T = p.T;
-  const int q0 = qt * kAttnQ;
-  const int qw0 = q0 + 32 * wave;  // this wave's first query
-  const int q = qw0 + n;           // this lane's query
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int n = lane & 15, quarter = lane >> 4;
+  const int T = p.T, H = p.H;
+  const int units = (T + kQ - 1) / kQ * H;  // (query tile, head) pairs of a row
+  const int groups = (units + 3) / 4;
+  // The longest workgroups (last query tiles) of all rows first.  Workgroups go to the
+  // eight XCDs in turn, each with an L2 of its own; which row an XCD gets turns every
+  // eight ranks: its 32 workgroups read a few rows' keys and values, and the XCDs'
+  // shares come out alike where rows differ (8 x 2047 tokens, left-padded by 0 to 966:
+  // 174 -> 155 us; a row to an XCD is 2 % better where all are full).
+  const int rank = (int)(blockIdx.x / p.B);
+  const int b = (int)((blockIdx.x % p.B + rank / 8) % p.B);
+  const int first_unit = 4 * (groups - 1 - rank);
+  const int last_unit = first_unit + 3 < units ? first_unit + 3 : units - 1;
+  const int unit = first_unit + wave;
+  const bool works = unit < units;
+  const int q0 = (works ? unit : units - 1) / H * kQ;  // this wave's first query
+  const int head = (works ? unit : units - 1) % H;
 
   // descriptors over this row's tensors
-  const uint32_t q_row_bytes = (uint32_t)p.H * kAttnHd * 2u;
+  const uint32_t q_row_bytes = (uint32_t)H * kAttnHd * 2u;
   const __amdgpu_buffer_rsrc_t rq =
       make_rsrc((const char*)p.q + (int64_t)b * T * q_row_bytes,
                 (uint32_t)T * q_row_bytes);
-  const __amdgpu_buffer_rsrc_t ro = make_rsrc(
-      (char*)p.out + (int64_t)b * T * q_row_bytes, (uint32_t)T * q_row_bytes);
-  const __amdgpu_buffer_rsrc_t rk =
-      make_rsrc((const char*)p.k + (int64_t)b * T * (kAttnHd * 2),
-                (uint32_t)T * (kAttnHd * 2u));
-  const uint32_t vt_row_bytes = (uint32_t)p.T_pad * 2u;
-  const __amdgpu_buffer_rsrc_t rv =
-      make_rsrc((const char*)p.v_t + (int64_t)b * kAttnHd * vt_row_bytes,
-                (uint32_t)kAttnHd * vt_row_bytes);
   const __amdgpu_buffer_rsrc_t rlo = make_rsrc(
       (const char*)p.lo + (int64_t)b * T * 4, (uint32_t)T * 4u);
+  const u32x4 rk = scalar_rsrc((const char*)p.k + (int64_t)b * T * (kAttnHd * 2),
+                               (uint32_t)T * (kAttnHd * 2u));
+  const uint32_t v_row_bytes = COLUMNS ? (uint32_t)p.T_pad * 2u : kAttnHd * 2u;
+  const uint32_t v_bytes = (COLUMNS ? (uint32_t)kAttnHd : (uint32_t)T) * v_row_bytes;
+  const u32x4 rv = scalar_rsrc((const char*)p.v + (int64_t)b * v_bytes, v_bytes);
 
-  // first visible key of this lane's query, and of the tile's / wave's first
-  // query (lo is non-decreasing: they bound the keys the tile / wave needs)
-  auto lo_at = [&](int t) {
+  // ---- everything that is asked for at once: which keys are seen, the queries (the B
+  //      operand of the first product, 8 k-steps of 32 dimensions) and their rotation;
+  //      queries past the end read as zero ------------------------------------------
+  auto lo_at = [&](int t) RG_INLINE {
     return (int)__builtin_amdgcn_raw_buffer_load_b32(
         rlo, t < T ? (uint32_t)t * 4u : kBufferOutOfRange, 0, 0);
   };
-  const int lo_q = q < T ? lo_at(q) : 0x7fffffff;
-  const int lo_tile = __builtin_amdgcn_readfirstlane(lo_at(q0));
-  const int lo_wave =
-      __builtin_amdgcn_readfirstlane(qw0 < T ? lo_at(qw0) : 0x7fffffff);
-  const int q_last_tile = q0 + kAttnQ - 1 < T - 1 ? q0 + kAttnQ - 1 : T - 1;
-  const int q_last_wave = qw0 + 31 < T - 1 ? qw0 + 31 : T - 1;
-  const int kt_begin = lo_tile / kAttnK;
-  const int kt_end = q_last_tile / kAttnK;  // inclusive
-
-  // (after the bounds, which the first tile's addresses wait for: loads return
-  // in order, and the tile is requested with the queries on their way)
-  // this lane's query as the B operand of the first product: 16 k-steps of
-  // 8 dimensions (16 bytes); queries past the end read as zero
-  AFrag qf[16];
-  {
-    const uint32_t off = (uint32_t)q * q_row_bytes + (uint32_t)head * 512u +
-                         16u * (uint32_t)half;
+  const int q_last = q0 + kQ - 1 < T - 1 ? q0 + kQ - 1 : T - 1;
+  const int lo_raw[3] = {lo_at(first_unit / H * kQ), lo_at(q0), lo_at(q_last)};
+  __builtin_amdgcn_sched_barrier(0);
+  AFrag qf[QB][8];
+  u32x4 table[ROPE ? QB : 1][4];
+  int lo_q[QB];
+  const __amdgpu_buffer_rsrc_t rt =
+      make_rsrc((const char*)p.rope_table + (int64_t)b * T * 256, ROPE ? (uint32_t)T * 256u : 0u);
 #pragma unroll
-    for (int ks = 0; ks < 16; ++ks)
-      qf[ks].q = __builtin_bit_cast(
+  for (int qb = 0; qb < QB; ++qb) {
+    const int q = q0 + 16 * qb + n;
+    const uint32_t off = (uint32_t)q * q_row_bytes + (uint32_t)head * 512u + 16u * quarter;
+    lo_q[qb] = lo_at(q);
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+      qf[qb][ks].q = __builtin_bit_cast(
           f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     rq, q < T ? off + 32u * ks : kBufferOutOfRange, 0, 0));
-  }
-  u32x4 table[ROPE ? 8 : 1];  // this lane's share of the query's sines, cosines
-  if (ROPE) {
-    const __amdgpu_buffer_rsrc_t rt =
-        make_rsrc((const char*)p.rope_table + (int64_t)b * T * 256,
-                  (uint32_t)T * 256u);
-    const uint32_t off = (uint32_t)q * 256u + 32u * (uint32_t)half;
+                     rq, q < T ? off + 64u * ks : kBufferOutOfRange, 0, 0));
+    if constexpr (ROPE) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      table[i] = __builtin_amdgcn_raw_buffer_load_b128(
-          rt, q < T ? off + 64u * (i >> 1) + 16u * (i & 1) : kBufferOutOfRange,
-          0, 0);
+      for (int i = 0; i < 4; ++i)
+        table[qb][i] = __builtin_amdgcn_raw_buffer_load_b128(
+            rt,
+            q < T ? (uint32_t)q * 256u + 32u * quarter + 128u * (i >> 1) + 16u * (i & 1)
+                  : kBufferOutOfRange,
+            0, 0);
+    }
   }
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "a255");  // (the kernel has them)
+  for_n<64 * QB>([&](auto I) RG_INLINE { acc_zero<decltype(I)::value>(); });
 
-  acc_fill(0.0f, std::make_integer_sequence<int, 128>{});
-  float m_run = -__builtin_inff();  // running maximum, in units of log2
-  float l_run = 0.0f;               // running sum over this half's keys
-  const float scale_log2 = p.scale * kLog2e;
+  // first visible key of a query (non-decreasing in it): what bounds the blocks that
+  // the workgroup and this wave need
+  auto uniform = [](int v) RG_INLINE { return __builtin_amdgcn_readfirstlane(v); };
+  const int lo_group = uniform(lo_raw[0]), lo_first = uniform(lo_raw[1]);
+  const int lo_last = uniform(lo_raw[2]);
+  const int group_last = last_unit / H * kQ + kQ - 1;
+  const int j_begin = lo_group / kBlockKeys;
+  const int j_end = (group_last < T - 1 ? group_last : T - 1) / kBlockKeys;  // inclusive
+  const int j_first = works ? lo_first / kBlockKeys : 0x7fffffff;
+  const int j_last = works ? q_last / kBlockKeys : -1;
 
-  // staging: 16-byte chunks, kAttnChunks per thread, tile and tensor; the
-  // chunks of tile kt + 1 are requested as soon as tile kt is in LDS and
-  // arrive while it is worked on
-  u32x4 kc[kAttnChunks], vc[kAttnChunks];
-  auto request_tile = [&](int kt) {
-    const int key0 = kt * kAttnK;
-#pragma unroll
-    for (int i = 0; i < kAttnChunks; ++i) {
-      const int c = tid + 256 * i;
-      const int krow = c >> 5, kcol = c & 31;
-      const int key = key0 + krow;
-      kc[i] = __builtin_amdgcn_raw_buffer_load_b128(
-          rk, key < T ? (uint32_t)key * 512u + 16u * kcol : kBufferOutOfRange,
-          0, 0);
-      const int d = c / (kAttnK / 8), part = c % (kAttnK / 8);
-      vc[i] = __builtin_amdgcn_raw_buffer_load_b128(
-          rv, (uint32_t)d * vt_row_bytes + (uint32_t)(key0 + 8 * part) * 2u, 0,
-          0);
+  // ---- blocks of keys and values into LDS ------------------------------------------
+  // A load instruction fills 1 KB.  Keys (and values key by key): two rows, 32 chunks of
+  // 16 bytes each, permuted by the row's number; a wave's four instructions take rows
+  // 8 r + 2 wave and the next.  Values in columns: 16 rows of a dimension, 64 bytes.
+  const int row2 = 2 * wave + (lane >> 5);
+  const uint32_t vk = (uint32_t)(row2 * 512 + 16 * ((lane & 31) ^ row2));
+  const uint32_t vv =
+      COLUMNS ? (uint32_t)(16 * wave + (lane >> 2)) * v_row_bytes +
+                    16u * ((lane & 3) ^ ((lane >> 3) & 3))
+              : (uint32_t)(row2 * 512 + 16 * ((lane & 31) ^ ((row2 & 3) << 1)));
+  auto load_one = [&](int to, int r, uint32_t v, u32x4 rsrc, int at) RG_INLINE {
+    const uint32_t m0 = lds0 + (uint32_t)to + 4096u * (uint32_t)r + 1024u * (uint32_t)wave;
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(m0),
+                 "v"(v), "s"(rsrc), "s"(at));
+  };
+  // (past the last key the descriptor's end: nothing is read)
+  auto load_keys = [&](int j, int r) RG_INLINE {
+    load_one((j & (kRing - 1)) * kBlockBytes, r, vk, rk, (j * kBlockKeys + 8 * r) * 512);
+  };
+  auto load_values = [&](int j, int r) RG_INLINE {
+    const int to = (kRing + (j & (kRing - 1))) * kBlockBytes;
+    if (COLUMNS) {
+      // (columns behind T_pad belong to the next dimension: not asked for)
+      const bool there = j * kBlockKeys < p.T_pad;
+      load_one(to, r, there ? vv : kBufferOutOfRange, rv,
+               there ? 64 * r * (int)v_row_bytes + j * kBlockKeys * 2 : 0);
+    } else {
+      load_one(to, r, vv, rv, (j * kBlockKeys + 8 * r) * 512);
     }
   };
-  auto stage_tile = [&](int buf) {
-    unsigned char* const kt_ = k_tile + buf * kKTileBytes;
-    unsigned char* const vt_ = v_tile + buf * kVTileBytes;
+
 #pragma unroll
-    for (int i = 0; i < kAttnChunks; ++i) {
-      const int c = tid + 256 * i;
-      const int krow = c >> 5, kcol = c & 31;
-      *reinterpret_cast<u32x4*>(kt_ + krow * kKRowBytes + 16 * kcol) = kc[i];
-      const int d = c / (kAttnK / 8), part = c % (kAttnK / 8);
-      // keys 8 part .. 8 part + 7 of the tile: group s = part / 2 of 16 keys,
-      // stored as [keys 0-3, 8-11 | keys 4-7, 12-15] of the group
-      unsigned char* const vb =
-          vt_ + d * kVRowBytes + 32 * (part >> 1) + 8 * (part & 1);
-      *reinterpret_cast<u32x2*>(vb) = u32x2{vc[i][0], vc[i][1]};
-      *reinterpret_cast<u32x2*>(vb + 16) = u32x2{vc[i][2], vc[i][3]};
+  for (int i = 0; i < 20; ++i) {
+    const int r = i & 3;
+    if (i < 8) load_keys(j_begin + i / 4, r);
+    else if (i < 12) load_values(j_begin, r);
+    else if (i < 16) load_keys(j_begin + 2, r);
+    else load_values(j_begin + 1, r);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (i < 4) load_keys(j_begin + 3, i);
+    else load_values(j_begin + 2, i - 4);
+  if constexpr (ROPE)
+    for_n<QB>([&](auto I) RG_INLINE {
+      rotate_query(qf[decltype(I)::value], table[decltype(I)::value]);
+    });
+  float m_run[QB], l_run[QB];  // running maximum (units of log2), this quarter's sum
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    m_run[qb] = kNoMaximum;
+    l_run[qb] = 0.0f;
+  }
+  const float scale_log2 = __uint_as_float(
+      (uint32_t)uniform((int)__float_as_uint(p.scale * kLog2e)));
+
+  // ---- operands from LDS ---------------------------------------------------------------
+  // (kept from being spread over a register per constant offset)
+  uint32_t k_lane = lds0 + (uint32_t)(512 * n + 16 * (quarter ^ (n & 7)));
+  uint32_t v_lane =
+      lds0 + kRing * kBlockBytes +
+      (COLUMNS ? (uint32_t)(64 * n + 16 * ((quarter >> 1) ^ ((n >> 1) & 3)) + 8 * (quarter & 1))
+               : (uint32_t)(512 * (4 * quarter + (n >> 2)) +
+                            16 * (((n & 3) >> 1) ^ ((n >> 2) << 1)) + 8 * (n & 1)));
+  constexpr int kAhead = 3;  // fragments on their way
+  constexpr int kFrags = kAhead + 1;
+  f32x4 ring[kFrags];
+  // fragment f of a block of keys: keys 16 (f / 8) .., k-step f % 8 (the second 16 keys'
+  // scores are started when half of the block before has left its registers)
+  auto read_keys = [&](int j, auto F) RG_INLINE {
+    constexpr int f = decltype(F)::value, ks = f % 8;
+    const uint32_t at = (k_lane ^ (64u * (ks & 1))) + (uint32_t)((j & (kRing - 1)) * kBlockBytes);
+    ring[f % kFrags] = *reinterpret_cast<const lds_f32x4*>(
+        (lds_byte*)(uintptr_t)at + 128 * (ks >> 1) + 8192 * (f / 8));
+  };
+  // fragment d of a block of values: dimensions 16 d ..
+  auto read_values = [&](int j, auto D) RG_INLINE {
+    constexpr int d = decltype(D)::value;
+    const uint32_t to = (uint32_t)((j & (kRing - 1)) * kBlockBytes);
+    if constexpr (COLUMNS) {
+      union {
+        u32x2 h[2];
+        f32x4 v;
+      } u;
+      const uint32_t at = v_lane + to;
+      u.h[0] = *reinterpret_cast<const lds_u32x2*>((lds_byte*)(uintptr_t)at + 1024 * d);
+      u.h[1] = *reinterpret_cast<const lds_u32x2*>((lds_byte*)(uintptr_t)(at ^ 32u) + 1024 * d);
+      ring[d % kFrags] = u.v;
+    } else {
+      union {
+        s16x4 h[2];
+        f32x4 v;
+      } u;
+      lds_byte* const at =
+          (lds_byte*)(uintptr_t)((v_lane ^ (32u * (d & 3))) + to) + 128 * (d >> 2);
+      u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
+      u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 8192));
+      ring[d % kFrags] = u.v;
     }
   };
-  // Two LDS buffers: while tile kt is worked on out of one, tile kt + 1
-  // arrives in registers and is written to the other afterwards; one barrier
-  // per tile.
-  request_tile(kt_begin);
-  if constexpr (ROPE) rotate_query(qf, table);
-  stage_tile(0);
-  __syncthreads();
-  if (kt_begin < kt_end) request_tile(kt_begin + 1);
-  // last query of this wave sees from lo_last_wave on (lo is non-decreasing)
-  const int lo_last_wave = __builtin_amdgcn_readfirstlane(lo_at(q_last_wave));
-  for (int kt = kt_begin; kt <= kt_end; ++kt) {
-    const int key0 = kt * kAttnK;
-    const int buf = (kt - kt_begin) & 1;
-    const unsigned char* const kt_ = k_tile + buf * kKTileBytes;
-    const unsigned char* const vt_ = v_tile + buf * kVTileBytes;
 
-    // tiles outside what this wave's queries can see are skipped (wave-uniform)
-    if (!(key0 > q_last_wave || key0 + kAttnK - 1 < lo_wave)) {
-      // ---- S^T = K tile x Q^T ----------------------------------------------
-      // (inline assembly with the results in ordinary registers: a matrix
-      // builtin lets the compiler pick accumulation registers for the result,
-      // and it picks a[0:15].  The compiler moves no LDS read across such a
-      // statement, so the operands are requested by hand, four fragments
-      // ahead of the instructions that use them.)
-      f32x16 s[kAttnKB];
-      {
-        constexpr int kFrags = 16 * kAttnKB, kBatch = 4;
-        auto k_frag = [&](int f) {  // fragment f: k-step f / KB, key block f % KB
-          return *reinterpret_cast<const f32x4*>(
-              kt_ + (32 * (f % kAttnKB) + n) * kKRowBytes + 32 * (f / kAttnKB) +
-              16 * half);
-        };
-        f32x4 fr[2][kBatch];
-#pragma unroll
-        for (int i = 0; i < kBatch; ++i) fr[0][i] = k_frag(i);
-#pragma unroll
-        for (int bt = 0; bt < kFrags / kBatch; ++bt) {
-          if (bt + 1 < kFrags / kBatch) {
-#pragma unroll
-            for (int i = 0; i < kBatch; ++i)
-              fr[(bt + 1) & 1][i] = k_frag((bt + 1) * kBatch + i);
-          }
-#pragma unroll
-          for (int i = 0; i < kBatch; ++i) {
-            const int f = bt * kBatch + i;
-            const int ks = f / kAttnKB, kb = f % kAttnKB;
-            if (ks == 0)
-              asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0"
-                           : "=&v"(s[kb])
-                           : "v"(fr[bt & 1][i]), "v"(qf[ks].q));
-            else
-              asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
-                           : "+v"(s[kb])
-                           : "v"(fr[bt & 1][i]), "v"(qf[ks].q));
-          }
-        }
-      }
-      // (tied to the scores: nothing that reads them may be scheduled above
-      // the wait)
-#pragma unroll
-      for (int kb = 0; kb < kAttnKB; ++kb) asm volatile("" : "+v"(s[kb]));
-      wait_for_matrix_results();
-#pragma unroll
-      for (int kb = 0; kb < kAttnKB; ++kb) asm volatile("" : "+v"(s[kb]));
-      // ---- mask (only where the band's edges cross the tile) ----------------
-      const bool interior = key0 + kAttnK - 1 <= qw0 && key0 >= lo_last_wave;
-      if (!interior) {
-#pragma unroll
-        for (int kb = 0; kb < kAttnKB; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = key0 + 32 * kb + 8 * (r >> 2) + 4 * half + (r & 3);
-            s[kb][r] = (key >= lo_q && key <= q) ? s[kb][r] : -__builtin_inff();
-          }
-      }
-      // ---- running maximum (in units of log2), moved only when the tile's
-      //      exceeds it by more than 2^8: the accumulators are rescaled rarely --
-      float tile_max = s[0][0];
-#pragma unroll
-      for (int kb = 0; kb < kAttnKB; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tile_max = fmaxf(tile_max, s[kb][r]);
-      {
-        const auto sw = __builtin_amdgcn_permlane32_swap(
-            __float_as_uint(tile_max), __float_as_uint(tile_max), false, false);
-        tile_max = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-      }
-      tile_max *= scale_log2;  // (the scale is positive)
-      if (__ballot(tile_max > m_run + 8.0f) != 0) {
-        const float m_new = fmaxf(m_run, tile_max);
-        // (no visible key so far: keep every exponent finite)
-        const float alpha = __builtin_amdgcn_exp2f(
-            m_run - (m_new == -__builtin_inff() ? 0.0f : m_new));
-        // (before a query's first visible key its accumulators are zeros)
-        const bool started = __ballot(m_run != -__builtin_inff()) != 0;
-        m_run = m_new;
-        l_run *= alpha;
-        if (started) {
-          wait_for_matrix_results();
-          acc_scale(alpha, std::make_integer_sequence<int, 128>{});
-        }
-      }
-      const float m_sub = m_run == -__builtin_inff() ? 0.0f : m_run;
-      AFrag pf[2 * kAttnKB];
-#pragma unroll
-      for (int kb = 0; kb < kAttnKB; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(
-              __builtin_fmaf(s[kb][r], scale_log2, -m_sub));
-          const float p1 = __builtin_amdgcn_exp2f(
-              __builtin_fmaf(s[kb][r + 1], scale_log2, -m_sub));
-          l_run += p0 + p1;
-          pf[2 * kb + (r >> 3)].u[(r & 7) >> 1] = pack_bf16x2(p0, p1);
-        }
-      // ---- O^T += V^T tile x P^T: the eight blocks of a 16-key step one after
-      //      the other (independent accumulators), the operands of the next
-      //      step requested before ------------------------------------------------
-      {
-        auto v_frag = [&](int ss, int blk) {
-          return *reinterpret_cast<const f32x4*>(
-              vt_ + (32 * blk + n) * kVRowBytes + 32 * ss + 16 * half);
-        };
-        // batch bt: 16-key step bt / 2, blocks 4 (bt % 2) .. + 3
-        f32x4 fr[2][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) fr[0][i] = v_frag(0, i);
-#pragma unroll
-        for (int bt = 0; bt < 4 * kAttnKB; ++bt) {
-          if (bt + 1 < 4 * kAttnKB) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              fr[(bt + 1) & 1][i] = v_frag((bt + 1) >> 1, 4 * ((bt + 1) & 1) + i);
-          }
-          const f32x4& pq = pf[bt >> 1].q;
-          if (bt & 1) {
-            acc_mfma<4>(fr[bt & 1][0], pq);
-            acc_mfma<5>(fr[bt & 1][1], pq);
-            acc_mfma<6>(fr[bt & 1][2], pq);
-            acc_mfma<7>(fr[bt & 1][3], pq);
-          } else {
-            acc_mfma<0>(fr[bt & 1][0], pq);
-            acc_mfma<1>(fr[bt & 1][1], pq);
-            acc_mfma<2>(fr[bt & 1][2], pq);
-            acc_mfma<3>(fr[bt & 1][3], pq);
-          }
-        }
-      }
+  // ---- one block of keys -------------------------------------------------------------
+  // s[kb][qb]: S^T of 16 keys by 16 queries
+  using Scores = f32x4[2][QB];
+  auto score_mfma = [&](Scores& s, auto I) RG_INLINE {
+    constexpr int i = decltype(I)::value, f = i / QB, qb = i % QB, ks = f % 8;
+    f32x4& c = s[f / 8][qb];
+    const f32x4 &k = ring[f % kFrags], &q = qf[qb][ks].q;
+    if constexpr (ks == 0)
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(k), "v"(q));
+    else
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(k), "v"(q));
+  };
+  AFrag pf[QB];
+  // Scores 2 i and 2 i + 1 of a query block, i = 0..3, to probabilities, in seven steps:
+  // a matrix instruction leaves room for two others before the next, and a longer run
+  // of them leaves the matrix pipe idle (all seven behind every fourth: a block's loop
+  // 2630 cycles).
+  constexpr int kSteps = 7 * 4 * QB;
+  float p0, p1;
+  auto probability_step = [&](const Scores& s, auto I) RG_INLINE {
+    constexpr int o = decltype(I)::value / 7, step = decltype(I)::value % 7;
+    constexpr int qb = o / 2 % QB, i = o % 2 + 2 * (o / (2 * QB));  // 16 keys after 16
+    if constexpr (step < 2) {
+      float& x = step ? p1 : p0;
+      x = __builtin_fmaf(s[i >> 1][qb][2 * (i & 1) + step], scale_log2, -m_run[qb]);
     }
-    if (kt < kt_end) {
-      stage_tile(buf ^ 1);  // tile kt + 1; that buffer's readers passed the
-      __syncthreads();      // barrier of the previous round
-      if (kt + 1 < kt_end) request_tile(kt + 2);
+    if constexpr (step == 2) p0 = __builtin_amdgcn_exp2f(p0);
+    if constexpr (step == 3) p1 = __builtin_amdgcn_exp2f(p1);
+    if constexpr (step == 4) l_run[qb] += p0;
+    if constexpr (step == 5) l_run[qb] += p1;
+    if constexpr (step == 6) pf[qb].u[i] = pack_bf16x2(p0, p1);
+  };
+  auto value_mfma = [&](auto I) RG_INLINE {
+    constexpr int i = decltype(I)::value;
+    acc_mfma<i>(ring[i / QB % kFrags], pf[i % QB].q);
+  };
+  auto mask = [&](Scores& s, int j) RG_INLINE {  // where the band's edges cross the block
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int n = ln & 15, quarter = ln >> 4;
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      const int q = q0 + 16 * qb + n, lo = lo_q[qb];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = j * kBlockKeys + 16 * kb + 4 * quarter + r;
+          s[kb][qb][r] = key >= lo && key <= q ? s[kb][qb][r] : -__builtin_inff();
+        }
     }
+  };
+  auto interior = [&](int j) RG_INLINE {
+    return j * kBlockKeys + kBlockKeys - 1 <= q0 && j * kBlockKeys >= lo_last;
+  };
+  // The running maximum moves only when a block's exceeds it by more than 2^8: the
+  // accumulators are rescaled rarely.
+  float most[QB];  // the next block's maxima, of this lane's scores
+  auto maximum = [&](const Scores& s, auto QBI) RG_INLINE {
+    constexpr int qb = decltype(QBI)::value;
+    const f32x4 &a = s[0][qb], &c = s[1][qb];
+    most[qb] = max3(max3(a[0], a[1], a[2]), max3(a[3], c[0], c[1]), fmaxf(c[2], c[3]));
+  };
+  auto rescale_where_needed = [&](bool first_block) RG_INLINE {
+    float over = __builtin_fmaf(most[0], scale_log2, -m_run[0]);
+#pragma unroll
+    for (int qb = 1; qb < QB; ++qb)
+      over = fmaxf(over, __builtin_fmaf(most[qb], scale_log2, -m_run[qb]));
+    if (__builtin_expect(__ballot(over > 8.0f) == 0, 1)) return;
+    float alpha[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      float m = most[qb] * scale_log2;  // (the scale is positive)
+      m = fmaxf(m, __shfl_xor(m, 16));
+      m = fmaxf(m, __shfl_xor(m, 32));
+      m = fmaxf(m, m_run[qb]);
+      alpha[qb] = __builtin_amdgcn_exp2f(m_run[qb] - m);
+      m_run[qb] = m;
+      l_run[qb] *= alpha[qb];
+    }
+    if (first_block) return;  // (the accumulators are zeros)
+    wait_for_matrix_results();
+    for_n<64 * QB>([&](auto I) RG_INLINE {
+      constexpr int i = decltype(I)::value;
+      acc_write<i>(acc_read<i>() * alpha[i / 4 % QB]);
+    });
+  };
+  auto settle = [&](Scores& s) RG_INLINE {  // results of the matrix instructions before this
+    wait_for_matrix_results();
+#pragma unroll
+    for (int i = 0; i < 2 * QB; ++i) asm volatile("" : "+v"(s[i / QB][i % QB]));
+  };
+  auto scores_alone = [&](Scores& s, int j) RG_INLINE {
+    for_n<kAhead>([&](auto F) RG_INLINE { read_keys(j, F); });
+    for_n<16>([&](auto F) RG_INLINE {
+      constexpr int f = decltype(F)::value;
+      if constexpr (f + kAhead < 16) read_keys(j, std::integral_constant<int, f + kAhead>{});
+      for_n<QB>([&](auto K) RG_INLINE {
+        score_mfma(s, std::integral_constant<int, f * QB + decltype(K)::value>{});
+      });
+    });
+    settle(s);
+    if (!interior(j)) mask(s, j);
+    for_n<QB>([&](auto I) RG_INLINE { maximum(s, I); });
+  };
+  // Behind this every wave is done with the keys of block j + 1 and the values of
+  // j - 1, and keys j + 2 and values j + 1 are in LDS (the loads of one round may be on
+  // their way).
+  auto block_barrier = [&] RG_INLINE { asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory"); };
+  auto load = [&](int j, int i) RG_INLINE {  // the i-th of a round's eight
+    if (i < 4) load_keys(j + 4, i);
+    else load_values(j + 3, i - 4);
+  };
+  // Probabilities and values of block j, scores of block j + 1.
+  auto block = [&](int j, Scores& now, Scores& next) RG_INLINE {
+    const bool values = j >= j_first && j <= j_last;
+    const bool scores = j + 1 >= j_first && j + 1 <= j_last;
+    asm volatile("" : "+v"(k_lane), "+v"(v_lane));
+    if (__builtin_expect(values && scores, 1)) {
+      for_n<kMfmas>([&](auto I) RG_INLINE {
+        constexpr int i = decltype(I)::value, f = i / QB;
+        score_mfma(next, I);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (i % QB == 0) {
+          if constexpr (f + kAhead < 16) read_keys(j + 1, std::integral_constant<int, f + kAhead>{});
+          else read_values(j, std::integral_constant<int, f + kAhead - 16>{});
+        }
+        constexpr int from = i * kSteps / kMfmas, to = (i + 1) * kSteps / kMfmas;
+        for_n<to - from>([&](auto S) RG_INLINE {
+          probability_step(now, std::integral_constant<int, from + decltype(S)::value>{});
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      const bool edge = !interior(j + 1);
+      for_n<kMfmas>([&](auto I) RG_INLINE {
+        constexpr int i = decltype(I)::value, d = i / QB;
+        value_mfma(I);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (i == 8 * QB) block_barrier();
+        if constexpr (i % QB == 0) {
+          if constexpr (d + kAhead < 16) read_values(j, std::integral_constant<int, d + kAhead>{});
+          else read_keys(j + 2, std::integral_constant<int, d + kAhead - 16>{});
+        }
+        if constexpr (i == 6 * QB) {
+#pragma unroll
+          for (int k = 0; k < 2 * QB; ++k) asm volatile("" : "+v"(next[k / QB][k % QB]));
+          if (__builtin_expect(edge, 0)) mask(next, j + 1);
+        }
+        if constexpr (i > 6 * QB && i % 2 == 1 && (i - 6 * QB) / 2 < QB)
+          maximum(next, std::integral_constant<int, (i - 6 * QB) / 2>{});
+        if constexpr (i > 8 * QB && i <= 8 * QB + 16 && i % 2 == 1)
+          load(j, (i - 8 * QB) / 2);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    } else {
+      if (values) {
+        for_n<kSteps>([&](auto I) RG_INLINE { probability_step(now, I); });
+        for_n<kAhead>([&](auto D) RG_INLINE { read_values(j, D); });
+        for_n<16>([&](auto D) RG_INLINE {
+          constexpr int d = decltype(D)::value;
+          if constexpr (d + kAhead < 16) read_values(j, std::integral_constant<int, d + kAhead>{});
+          for_n<QB>([&](auto K) RG_INLINE {
+            value_mfma(std::integral_constant<int, d * QB + decltype(K)::value>{});
+          });
+        });
+      }
+      if (scores) scores_alone(next, j + 1);
+      block_barrier();
+      for (int i = 0; i < 8; ++i) load(j, i);
+      for_n<kAhead>([&](auto F) RG_INLINE { read_keys(j + 2, F); });
+    }
+    if (scores) rescale_where_needed(j + 1 == j_first);
+  };
+
+  Scores even, odd;
+#pragma unroll
+  for (int i = 0; i < 2 * QB; ++i)
+    even[i / QB][i % QB] = odd[i / QB][i % QB] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
+  if (j_first == j_begin) {
+    scores_alone(even, j_begin);
+    rescale_where_needed(true);
   }
+  for_n<kAhead>([&](auto F) RG_INLINE { read_keys(j_begin + 1, F); });
+  for (int j = j_begin; j <= j_end; j += 2) {
+    block(j, even, odd);
+    if (j + 1 > j_end) break;
+    block(j + 1, odd, even);
+  }
+  // (no load outlives the workgroup's LDS)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (!works) return;
 
-  // ---- normalise and store: this lane's query, dimensions
-  //      32 blk + 8 j + 4 half + i ---------------------------------------------
+  // ---- normalise and store: a lane's query of each block, dimensions 16 d + 4 quarter
+  //      .. + 3; two neighbouring quarters trade runs of two blocks for eight in a row --
   wait_for_matrix_results();
-  float l_total;
-  {
-    const auto sw = __builtin_amdgcn_permlane32_swap(
-        __float_as_uint(l_run), __float_as_uint(l_run), false, false);
-    l_total = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-  }
-  const float inv = l_total > 0.0f ? 1.0f / l_total : 0.0f;
-  const uint32_t out_off = (uint32_t)q * q_row_bytes + (uint32_t)head * 512u;
-  auto store4 = [&](int d0, float o0, float o1, float o2, float o3) {
-    __builtin_amdgcn_raw_buffer_store_b64(
-        u32x2{pack_bf16x2(o0 * inv, o1 * inv), pack_bf16x2(o2 * inv, o3 * inv)},
-        ro, q < T ? out_off + (uint32_t)(d0 + 4 * half) * 2u : kBufferOutOfRange,
-        0, 0);
-  };
-#define RG_ATTN_STORE(BLK, J)                                              \
-  store4(32 * BLK + 8 * J, acc_read<16 * BLK + 4 * J>(),                   \
-         acc_read<16 * BLK + 4 * J + 1>(), acc_read<16 * BLK + 4 * J + 2>(), \
-         acc_read<16 * BLK + 4 * J + 3>());
-#define RG_ATTN_STORE_BLK(BLK) \
-  RG_ATTN_STORE(BLK, 0) RG_ATTN_STORE(BLK, 1) RG_ATTN_STORE(BLK, 2) RG_ATTN_STORE(BLK, 3)
-  RG_ATTN_STORE_BLK(0) RG_ATTN_STORE_BLK(1) RG_ATTN_STORE_BLK(2) RG_ATTN_STORE_BLK(3)
-  RG_ATTN_STORE_BLK(4) RG_ATTN_STORE_BLK(5) RG_ATTN_STORE_BLK(6) RG_ATTN_STORE_BLK(7)
-#undef RG_ATTN_STORE_BLK
-#undef RG_ATTN_STORE
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  const __amdgpu_buffer_rsrc_t ro = make_rsrc(
+      (char*)p.out + (int64_t)b * T * q_row_bytes, (uint32_t)T * q_row_bytes);
+  for_n<QB>([&](auto QBI) RG_INLINE {
+    constexpr int qb = decltype(QBI)::value;
+    float l = l_run[qb];
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const int q = q0 + 16 * qb + (ln & 15);
+    const uint32_t off = (uint32_t)q * q_row_bytes + (uint32_t)head * 512u +
+                         2u * (uint32_t)(ln & 16) + 8u * (uint32_t)(ln >> 4 & 2);
+    for_n<8>([&](auto P) RG_INLINE {
+      constexpr int pair = decltype(P)::value;
+      uint32_t w[2][2];
+      for_n<4>([&](auto E) RG_INLINE {
+        constexpr int e = decltype(E)::value, at = 4 * ((2 * pair + e / 2) * QB + qb) + 2 * (e % 2);
+        w[e / 2][e % 2] = pack_bf16x2(acc_read<at>() * inv, acc_read<at + 1>() * inv);
+      });
+      const auto s0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+      const auto s1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+      buffer_store_16(u32x4{s0[0], s1[0], s0[1], s1[1]}, ro,
+                      q < T ? off + 64u * pair : kBufferOutOfRange, 0);
+    });
+  });
 }
 
 // ---------------------------------------------------------------- prepare --
 // Everything of the block between its projections and the attention kernel,
-// in one pass over the keys and values (recurrentgemma/torch/modules.py:431-440
+// in one pass over the keys (recurrentgemma/torch/modules.py:431-440
 // and the ring cache of a prompt, :253-283): rotary embedding of the keys, the
 // sines and cosines the queries are rotated with (one word per token and pair:
-// sine in the low half, cosine in the high half, bf16), the values transposed
-// for the second product (zeros behind the last token), the last min(window, T)
+// sine in the low half, cosine in the high half, bf16), the last min(window, T)
 // keys and values in their ring slots, zeros in the slots never written, and
 // the token count.
 //
 // One workgroup per (row, 32 tokens and 32 ring slots), which leaves the chip
 // full from 8 x 1024 tokens on.  Bound by memory (8 x 2047 tokens: 17 MB in,
-// 38 MB out); the tensor operations it replaces were ten launches, 146 us
-// there.  32 tokens make runs of 64 bytes of a transposed row; with 64 a single
-// prompt fills half as many CUs.
+// 30 MB out); the tensor operations it replaces were ten launches, 146 us
+// there.
 constexpr int kPrepTokens = 32;
-constexpr int kPrepStride = kAttnHd + 8;  // of a token's values in LDS
 
 __device__ __forceinline__ int64_t position_at(const AttnPromptArgs& p,
                                                int64_t i) {
@@ -479,7 +602,6 @@ __device__ __forceinline__ int64_t position_at(const AttnPromptArgs& p,
 __global__ void __launch_bounds__(256)
 attn_prompt_prepare_kernel(AttnPromptArgs p) {
 #pragma clang fp contract(off)
-  __shared__ __align__(16) uint16_t values[kPrepTokens * kPrepStride];
   const int tid = threadIdx.x;
   const int T = p.T, b = (int)(blockIdx.x / p.groups);
   const int t0 = (int)(blockIdx.x % p.groups) * kPrepTokens;
@@ -564,19 +686,16 @@ attn_prompt_prepare_kernel(AttnPromptArgs p) {
         *reinterpret_cast<u32x4*>(ring_k + (int64_t)slot * kAttnHd + d) = w;
     }
   }
-  // values: to their ring slots, and through LDS into transposed rows
+  // values, to their ring slots
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int i = 8 * j + tid / 32, t = t0 + i;
-    const int d = 8 * (tid % 32);
-    u32x4 w = {0, 0, 0, 0};
-    if (t < T) {
-      w = *reinterpret_cast<const u32x4*>(v + (int64_t)t * kAttnHd + d);
-      const int slot = slot_of(t);
-      if (slot >= 0)
-        *reinterpret_cast<u32x4*>(ring_v + (int64_t)slot * kAttnHd + d) = w;
+    const int t = t0 + 8 * j + tid / 32;
+    const int slot = t < T ? slot_of(t) : -1;
+    if (slot >= 0) {
+      const int d = 8 * (tid % 32);
+      *reinterpret_cast<u32x4*>(ring_v + (int64_t)slot * kAttnHd + d) =
+          *reinterpret_cast<const u32x4*>(v + (int64_t)t * kAttnHd + d);
     }
-    *reinterpret_cast<u32x4*>(values + i * kPrepStride + d) = w;
   }
   // ring slots that no token of the prompt fills
   if (cache) {
@@ -588,22 +707,6 @@ attn_prompt_prepare_kernel(AttnPromptArgs p) {
         *reinterpret_cast<u32x4*>(ring_k + at) = u32x4{0, 0, 0, 0};
         *reinterpret_cast<u32x4*>(ring_v + at) = u32x4{0, 0, 0, 0};
       }
-    }
-  }
-  __syncthreads();
-  if (t0 < p.T_pad) {  // (T_pad is a multiple of 64: all 32 columns exist)
-    uint16_t* const vt = p.v_t + (int64_t)b * kAttnHd * p.T_pad + t0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = 64 * j + tid / 4, part = tid % 4;
-      u32x4 w;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint16_t* const c =
-            values + (8 * part + 2 * e) * kPrepStride + d;
-        w[e] = (uint32_t)c[0] | ((uint32_t)c[kPrepStride] << 16);
-      }
-      *reinterpret_cast<u32x4*>(vt + (int64_t)d * p.T_pad + 8 * part) = w;
     }
   }
 }
@@ -648,7 +751,7 @@ first_key_kernel(const void* pos, int pos_kind, int32_t* __restrict__ first,
 hipError_t launch_attn_prompt_prepare(const AttnPromptArgs& args,
                                       hipStream_t s) {
   AttnPromptArgs a = args;
-  const int64_t tokens = a.ring_k && a.window > a.T_pad ? a.window : a.T_pad;
+  const int64_t tokens = a.ring_k && a.window > a.T ? a.window : a.T;
   const int64_t groups = (tokens + kPrepTokens - 1) / kPrepTokens;
   if (groups <= 0 || a.B <= 0 || groups * a.B > 0x7fffffff)
     return hipErrorInvalidValue;
@@ -664,25 +767,28 @@ hipError_t launch_first_key(const void* pos, int pos_kind, int32_t* first,
   return hipGetLastError();
 }
 
-hipError_t launch_attn_prefill_bf16(const AttnPrefillArgs& a, hipStream_t s) {
-  // needs head dimension 256, T_pad a multiple of 64 >= T, and rows whose byte
-  // offsets fit 32 bits (checked by the caller)
-  const int64_t qtiles = (a.T + kAttnQ - 1) / kAttnQ;
-  const int64_t blocks = qtiles * a.H * a.B;
-  if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
-  constexpr size_t lds = 2 * (size_t)(kKTileBytes + kVTileBytes);
-  static_assert(lds <= 160 * 1024, "LDS of one CU");
-  static OncePerDevice once[2];
-  const bool rope = a.rope_table != nullptr;
-  hipError_t e = set_max_dynamic_lds(
-      once[rope], rope ? (const void*)attn_prefill_bf16_kernel<true>
-                       : (const void*)attn_prefill_bf16_kernel<false>, lds);
+namespace {
+template <bool ROPE, bool COLUMNS, int QB>
+hipError_t launch_prefill(const AttnPrefillArgs& a, hipStream_t s) {
+  const int64_t units = (int64_t)((a.T + 16 * QB - 1) / (16 * QB)) * a.H;
+  const int64_t blocks = (units + 3) / 4 * a.B;
+  if (blocks <= 0 || blocks > 0x7fffffff || units > 0x7ffffff0) return hipErrorInvalidValue;
+  static OncePerDevice once;
+  const auto kernel = attn_prefill_bf16_kernel<ROPE, COLUMNS, QB>;
+  hipError_t e = set_max_dynamic_lds(once, (const void*)kernel, kAttnLds);
   if (e != hipSuccess) return e;
-  if (rope)
-    attn_prefill_bf16_kernel<true><<<dim3((unsigned)blocks), 256, lds, s>>>(a);
-  else
-    attn_prefill_bf16_kernel<false><<<dim3((unsigned)blocks), 256, lds, s>>>(a);
+  kernel<<<dim3((unsigned)blocks), 256, kAttnLds, s>>>(a);
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_attn_prefill_bf16(const AttnPrefillArgs& a, hipStream_t s) {
+  // needs head dimension 256 and rows whose byte offsets fit 32 bits (checked by the
+  // caller); values in columns T_pad (a multiple of 64) long, or key by key (T_pad 0)
+  if (a.T_pad == 0)
+    return a.rope_table ? launch_prefill<true, false, 3>(a, s)
+                        : launch_prefill<false, false, 3>(a, s);
+  return launch_prefill<false, true, 3>(a, s);
 }
 
 }  // namespace rg

@@ -154,7 +154,7 @@ struct AttnPrefillArgs {
   const void* q;    // [B, T, H, 256] bf16, after the rotary embedding
                     // (before it where rope_table is given)
   const void* k;    // [B, T, 256] bf16, after the rotary embedding
-  const void* v_t;  // [B, 256, T_pad] bf16: the values transposed, zeros
+  const void* v;    // [B, T, 256] bf16, or (T_pad > 0) [B, 256, T_pad]: transposed, zeros
                     // behind token T - 1 (T_pad a multiple of 64)
   const void* lo;   // [B, T] int32: first key each query sees (non-decreasing)
   void* out;        // [B, T, H, 256] bf16
@@ -171,12 +171,11 @@ struct AttnPromptArgs {
   int pos_kind;
   const float* inv_freq;  // [64]
   uint16_t* k_rot;        // [B, T, 256]
-  uint16_t* v_t;          // [B, 256, T_pad]
   uint32_t* rope_table;   // [B, T, 64]
   uint16_t* ring_k;       // [B, window, 256], null: no cache wanted
   uint16_t* ring_v;
   int32_t* num_tokens;    // [B]
-  int B, T, T_pad, window;
+  int B, T, window;
   unsigned groups;        // workgroups per row (set by the launch)
 };
 hipError_t launch_attn_prompt_prepare(const AttnPromptArgs& a, hipStream_t s);

@@ -66,7 +66,9 @@ def linears(x, *layers):
   launch (ops.linear_many) where that is ahead of the library, as long as
   calling the layers is nothing but their products (and no program is being
   traced: the kernels are reached through ctypes)."""
-  if (not compiled.tracing() and not _global_hooks() and
+  # (few rows never pay, and their callers wait for the host)
+  if (x.dim() > 1 and x.numel() >= 1024 * x.shape[-1] and
+      not compiled.tracing() and not _global_hooks() and
       all(_as_written(layer, nn.Linear) for layer in layers)):
     parts = [_parameters(layer, "weight", "bias") for layer in layers]
     out = ops.linear_many(x, [w for w, _ in parts], [b for _, b in parts])

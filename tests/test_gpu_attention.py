@@ -67,6 +67,15 @@ def test_attention_prefill_kernel(B, T, H, window, mean_doc):
                                    what="attention")
 
 
+@pytest.mark.parametrize("T", [31, 32, 47, 48, 49, 95, 97, 145])
+@pytest.mark.parametrize("H,window,mean_doc", [(1, 2048, None), (5, 16, 20),
+                                               (10, 31, None), (3, 2048, 33)])
+def test_attention_prefill_tile_edges(T, H, window, mean_doc):
+  """Around 48 queries of a wave, 32 keys of a block, four (query tile, head)
+  pairs of a workgroup, with bands that open and close inside them."""
+  test_attention_prefill_kernel(2, T, H, window, mean_doc)
+
+
 def test_attention_prefill_left_padded_rows():
   """Rows padded on the left with position -1, as the sampler lays out
   prompts of different lengths (sampler.py:234-238): the first real token
