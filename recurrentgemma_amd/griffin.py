@@ -211,7 +211,7 @@ class MLPBlock(nn.Module):
       return self._rows_down(hidden, (self.ffw_down.weight,),
                              (self.ffw_down.bias,), residual=residual)
     hidden = None
-    if (x.dim() > 1 and x.numel() >= 256 * self.width and
+    if (x.dim() > 1 and x.numel() > 64 * self.width and
         not compiled.tracing() and not modules._global_hooks() and
         modules._as_written(self.ffw_up, _StackedLinear)):
       hidden = ops.linear_gelu_pair(

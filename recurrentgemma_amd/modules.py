@@ -62,13 +62,16 @@ def _global_hooks() -> bool:
 
 
 def linears(x, *layers):
-  """The outputs of nn.Linear layers that read x.  Many rows in bf16: one
-  launch (ops.linear_many) where that is ahead of the library, as long as
-  calling the layers is nothing but their products (and no program is being
-  traced: the kernels are reached through ctypes)."""
-  # (few rows never pay, and their callers wait for the host)
-  if (x.dim() > 1 and x.numel() >= 1024 * x.shape[-1] and
-      not compiled.tracing() and not _global_hooks() and
+  """The outputs of nn.Linear layers that read x.  More rows than a decode
+  step's in bf16: one launch (ops.linear_many) where that is ahead of the
+  library, as long as calling the layers is nothing but their products (and no
+  program is being traced: the kernels are reached through ctypes)."""
+  # (what mostly says no comes first: the callers of few rows wait for the host)
+  if (x.dtype is torch.bfloat16 and x.dim() > 1 and
+      x.numel() > 64 * x.shape[-1] and not compiled.tracing() and
+      all(type(layer) is nn.Linear for layer in layers) and
+      ops.linear_many_pays(x, *[layer.out_features for layer in layers]) and
+      not _global_hooks() and
       all(_as_written(layer, nn.Linear) for layer in layers)):
     parts = [_parameters(layer, "weight", "bias") for layer in layers]
     out = ops.linear_many(x, [w for w, _ in parts], [b for _, b in parts])

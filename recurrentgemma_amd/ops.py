@@ -590,6 +590,13 @@ def _rows(x) -> int:
   return x.numel() // x.shape[-1]
 
 
+def linear_many_pays(x, *features) -> bool:
+  """Whether layers of so many output features are better run by linear_many
+  (sizes alone)."""
+  return (x.is_cuda and x.numel() > 0 and
+          _linear_many_pays(x.numel() // x.shape[-1], x.shape[-1], features))
+
+
 def linear_many(x, weights, biases):
   """x [..., K] through layers that read it (weights [N_i, K], biases [N_i] or
   None): one launch (rg_linear_many) where that is ahead of the library's

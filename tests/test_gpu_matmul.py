@@ -1,6 +1,6 @@
 """Linear layers of many rows (csrc/rg_matmul.hip) against float64, through the C calls
 that the modules make: forward, both directions back, the MLP's pair.  Sizes at the edges
-of the tiles (128 and 256 rows, 256 and 320 columns), of the steps (64 of the contraction)
+of the tiles (64, 128 and 256 rows, 64 to 320 columns), of the steps (64 of the contraction)
 and of the 8 values of a load."""
 
 import ctypes
@@ -52,8 +52,10 @@ def check(got, terms, buf, extra=0.0):
 
 
 # rows, features in, features out
-FORWARD = [(1, 64, 8), (127, 128, 264), (129, 192, 256), (256, 64, 320), (257, 320, 328),
-           (1000, 2560, 512), (4097, 512, 2560)]
+FORWARD = [(1, 64, 8), (63, 64, 72), (65, 448, 136), (127, 128, 264), (129, 192, 256),
+           (256, 64, 320), (257, 320, 328), (1000, 2560, 512), (999, 512, 2560),
+           # tiles of 128 x 320, 256 x 320, 128 x 256 and 256 x 256
+           (4095, 192, 2560), (8191, 192, 2560), (2049, 1024, 2560), (4097, 1024, 2568)]
 
 
 @pytest.mark.parametrize("M,K,N", FORWARD)
@@ -87,7 +89,7 @@ def test_back(M, K, N, two):
 # rows; features out, features in
 @pytest.mark.parametrize("M", [1, 63, 64, 65, 191, 1003])
 @pytest.mark.parametrize("shapes", [[(8, 8)], [(264, 328)], [(256, 320), (8, 264), (512, 256)],
-                                    [(2560, 2560)] * 3])
+                                    [(2560, 2560)] * 3, [(4096, 4104)]])
 def test_weight_gradients(M, shapes):
   dy = [normal(1 + i, M, n) for i, (n, _) in enumerate(shapes)]
   x = [normal(9 + i, M, k) for i, (_, k) in enumerate(shapes)]
