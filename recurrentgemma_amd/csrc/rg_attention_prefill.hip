@@ -8,7 +8,7 @@
 // lo[t] = max(first token of t's document, t - window) is supplied by the
 // caller (non-decreasing in t).
 //
-// A wave owns 48 queries of one head, a workgroup four such waves: heads of the same queries first, since all heads read the same keys and
+// A wave owns 48 queries of one head (32 in short prompts), a workgroup four such waves: heads of the same queries first, since all heads read the same keys and
 // values.  They come by in blocks of 32 keys, global -> LDS by the memory pipe, three
 // blocks ahead (a ring of four each), one barrier per block.  Both products are
 // v_mfma_f32_16x16x32_bf16 with the QUERIES as the 16 columns of the result:
@@ -782,13 +782,28 @@ hipError_t launch_prefill(const AttnPrefillArgs& a, hipStream_t s) {
 }
 }  // namespace
 
+namespace {
+template <int QB>
+hipError_t launch_queries(const AttnPrefillArgs& a, hipStream_t s) {
+  if (a.T_pad == 0)
+    return a.rope_table ? launch_prefill<true, false, QB>(a, s)
+                        : launch_prefill<false, false, QB>(a, s);
+  return launch_prefill<false, true, QB>(a, s);
+}
+// 32 queries a wave up to two rounds of the chip of them: half as many workgroups again,
+// each with two thirds of the work (us with 48 / 32, 10 heads: 1 x 300 tokens 28 / 22,
+// 1 x 2047 86 / 67, 4 x 1000 58 / 47, 8 x 700 50 / 47; 16 heads 1 x 1000 52 / 41, 4 x 1000
+// 60 / 59, 3 x 1500 78 / 79).
+bool short_tiles(const AttnPrefillArgs& a) {
+  const int64_t units = (int64_t)((a.T + 31) / 32) * a.H;
+  return (units + 3) / 4 * a.B <= 512;
+}
+}  // namespace
+
 hipError_t launch_attn_prefill_bf16(const AttnPrefillArgs& a, hipStream_t s) {
   // needs head dimension 256 and rows whose byte offsets fit 32 bits (checked by the
   // caller); values in columns T_pad (a multiple of 64) long, or key by key (T_pad 0)
-  if (a.T_pad == 0)
-    return a.rope_table ? launch_prefill<true, false, 3>(a, s)
-                        : launch_prefill<false, false, 3>(a, s);
-  return launch_prefill<false, true, 3>(a, s);
+  return short_tiles(a) ? launch_queries<2>(a, s) : launch_queries<3>(a, s);
 }
 
 }  // namespace rg

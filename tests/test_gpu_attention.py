@@ -71,9 +71,18 @@ def test_attention_prefill_kernel(B, T, H, window, mean_doc):
 @pytest.mark.parametrize("H,window,mean_doc", [(1, 2048, None), (5, 16, 20),
                                                (10, 31, None), (3, 2048, 33)])
 def test_attention_prefill_tile_edges(T, H, window, mean_doc):
-  """Around 48 queries of a wave, 32 keys of a block, four (query tile, head)
+  """Around 32 queries of a wave, 32 keys of a block, four (query tile, head)
   pairs of a workgroup, with bands that open and close inside them."""
   test_attention_prefill_kernel(2, T, H, window, mean_doc)
+
+
+@pytest.mark.parametrize("T,window,mean_doc", [(31, 2048, None), (47, 16, 20),
+                                               (48, 2048, None), (49, 31, None),
+                                               (97, 2048, 33)])
+def test_attention_prefill_tile_edges_many_rows(T, window, mean_doc):
+  """The same with 48 queries of a wave, which more than 512 workgroups of 32
+  queries a wave get."""
+  test_attention_prefill_kernel(264, T, 5, window, mean_doc)
 
 
 def test_attention_prefill_left_padded_rows():
