@@ -1025,15 +1025,15 @@ def run_prefill(args, torch, rg, R, ops, workload, steps, warmup, extras,
         "frac_of_bf16_mfma_peak": gemm_flops / (first_ms * 1e-3) / 2.5e15}
   elif f32_single:
     # float32 with few rows: rg_recurrent_core is ONE launch that does the
-    # conv, both gate projections (true float32 products on the float32
-    # matrix instruction), the gates and the recurrence
+    # conv, both gate projections (float32 products as six bf16 products of
+    # three pieces of either operand), the gates and the recurrence
     algo = single_algorithmic_bytes(B, T, W, H, 4, seg_bytes, has_h0=False)
     tf = gemm_flops / (first_ms * 1e-3) / 1e12
     roofline = {
-        "kernel": "core_f32_small_kernel (conv + gate GEMMs on "
-                  "v_mfma_f32_16x16x4_f32 + gates + scan, one launch)",
-        "bound": "mfma", "achieved": tf, "peak": 157.3, "unit": "TFLOP/s",
-        "frac": tf / 157.3, "traffic": None, "algorithmic_bytes": algo,
+        "kernel": "core_f32_small_kernel (conv + gate GEMMs on six "
+                  "v_mfma_f32_16x16x32_bf16 + gates + scan, one launch)",
+        "bound": "mfma", "achieved": tf, "peak": 2500.0 / 6, "unit": "TFLOP/s",
+        "frac": tf / (2500.0 / 6), "traffic": None, "algorithmic_bytes": algo,
         "avg_launch_ms": first_ms, "launch_ms": per_launch["main"][0],
         "gbs": algo / (first_ms * 1e-3) / 1e9}
   else:

@@ -312,11 +312,11 @@ int rg_recurrent_prefill_gelu_mul(
  * tokens; heads of 136 .. 248 channels where that is ahead); for float32 with
  * 256-wide heads and at most 32 (row, head) pairs one launch that does the same
  * in float32 (needs no workspace; no entry point of its own), with more pairs
- * rg_conv1d_prefill, the projections on the bf16 matrix instruction with every
- * operand in three pieces (closer to the exact products than rg_gates_gemm) and a
- * recurrence of its own, the pre-activations living in the workspace (taken for
- * fewer pairs too where it is faster and the caller brings a workspace that holds
- * x twice); else rg_gates_gemm with the conv
+ * rg_conv1d_prefill, the projections and a recurrence of its own, the
+ * pre-activations living in the workspace (taken for fewer pairs too where it is
+ * faster and the caller brings a workspace that holds x twice), the projections of
+ * either on the bf16 matrix instruction with every operand in three pieces (closer to
+ * the exact products than rg_gates_gemm); else rg_gates_gemm with the conv
  * applied on load followed by rg_lru_scan_fused_split, the pre-activations of
  * both gates living in the workspace.  gate_branch (nullable, [B,T,W]): the
  * block's linear_y output; `out` is then rglru(conv1d(x)) * gelu_tanh(

@@ -615,19 +615,36 @@ static bool wide_scan_on_tiles(int B, int T, int W) {
   const int64_t slabs = (int64_t)B * ((W + 31) / 32);
   return T >= (slabs <= 256 ? 1 : slabs <= 1024 ? 64 : slabs < 2048 ? 96 : 192);
 }
-// Against one launch for everything (at most 32 pairs, 16 of them at a time, 512
-// tokens in 33 us; the other form about 17 us + 1.1e-5 us an element): us, one
-// launch / several: W2560 T1 35 / 18, T200 34 / 24, T512 34.5 / 33.5, T2048 120 / 78,
-// B2 T64 66 / 22, B3 T512 67 / 52; W4096 T512 35 / 39, T1024 64 / 56; W256 B8 T512
-// 34 / 28.  Against gate GEMM + scan (more pairs) everywhere but a few rows of all:
-// W2560 B64 T1 20.5 / 23, T16 73 / 50, B4 T2048 519 / 240, B8 T2048 joined 878 / 523;
-// W4096 B3 T16 18 / 22, B4 T512 206 / 93; W256 B64 T16 19.2 / 20.5, T64 37 / 29.
-static bool wide_f32_pays(int B, int T, int W, int H, bool one_launch_takes) {
+// Against one launch for everything (at most 32 pairs, 16 of them at a time).  us from
+// a graph, one launch / several: W2560 T1 10 / 18, T200 17 / 24, T512 27 / 34, T1024
+// 46 / 54, T1536 67 / 64, T2048 87 / 84, B2 T64 19 / 22, T300 34 / 40, T512 49 / 48,
+// T1024 89 / 70, B3 T512 51 / 53, T1024 96 / 91; W4096 T512 27 / 39, T2048 94 / 100, B2
+// T512 50 / 54, T1536 142 / 135; W256 T300 18 / 22, T640 31 / 27, T2048 86 / 31, B8 T512
+// 25 / 28, T1536 65 / 61.  One launch takes a round of 16 pairs for its turns of 128
+// tokens and, past 512, another segment; several take a fixed part, the bytes, and the
+// recurrence along a row.  (While one launch ran on the float32 matrix instruction it
+// took 33 for up to 512 tokens, whatever there was of them, 65 for 1024.)
+static bool wide_f32_ahead(int B, int T, int W, int H) {
+  const float elements = (float)B * T * W;
+  const int rounds = (int)(((int64_t)B * H + 15) / 16);
+  const float one_launch = rounds * ((T > 512 ? 6.5f : 4.5f) +
+                                     (rounds == 1 ? 0.04f : 0.044f) * T);
+  const float several =
+      (elements < 3e5f ? 18.0f : 22.0f) + 0.85e-5f * elements + 0.005f * T;
+  return several < one_launch;
+}
+// Where the workspace of the form of several launches is asked for.  With more pairs
+// it is the form unless there are a few rows of all (against gate GEMM + scan: W2560
+// B64 T1 20.5 / 23, T16 73 / 50, B4 T2048 519 / 240, B8 T2048 joined 878 / 523; W4096
+// B3 T16 18 / 22, B4 T512 206 / 93; W256 B64 T16 19.2 / 20.5, T64 37 / 29).  With few
+// it is asked for where it may be ahead and further down, as it always was, so that a
+// caller's sizes stay what they are; wide_f32_ahead decides.
+static bool wide_f32_room(int B, int T, int W, int H, bool one_launch_takes) {
   const float elements = (float)B * T * W;
   if (!one_launch_takes) return elements > 3e5f;
-  const float one_launch =
+  const float rounds =
       33.0f * (((int64_t)B * H + 15) / 16) * ((T + 511) / 512);
-  return 17.0f + 1.1e-5f * elements < 0.95f * one_launch;
+  return 17.0f + 1.1e-5f * elements < 0.95f * rounds;
 }
 
 static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
@@ -638,7 +655,7 @@ static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
   p.wide_f32 = dtype == RG_DTYPE_F32 &&
                rg::gates_f32_serves((int64_t)B * T, W, H) &&
                rg::scan_tiles_take(T, W, dtype) &&
-               wide_f32_pays(B, T, W, H, p.small_f32);
+               wide_f32_room(B, T, W, H, p.small_f32);
   if (p.wide_f32 && wide_scan_on_tiles(B, T, W))
     p.deal_bytes = rg::scan_tiles_deal_bytes(B, T, W, dtype, rg::kTilesFwdGated);
   if (p.small_f32) {
@@ -730,7 +747,8 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
                 __func__, need, workspace ? workspace_bytes : (size_t)0);
   // (the form of several launches keeps the conv output where y goes, and the
   // pre-activations in a workspace that the one-launch form does not ask for)
-  const bool wide = p.wide_f32 && gate_branch != out && workspace != nullptr &&
+  const bool wide = p.wide_f32 && (!p.small_f32 || wide_f32_ahead(B, T, W, H)) &&
+                    gate_branch != out && workspace != nullptr &&
                     workspace_bytes >= p.split_bytes + 2 * p.gate_bytes &&
                     aligned16(workspace);
   if (p.small_f32 || wide) {

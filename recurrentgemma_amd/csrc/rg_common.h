@@ -165,6 +165,18 @@ __device__ __forceinline__ float conv4(float x0, float x1, float x2, float x3,
   return acc;
 }
 
+// Two float32 as three bf16 pieces each, every piece the nearest bf16 to what the
+// pieces before it leave: (first value's, second value's) in one register per piece.
+__device__ __forceinline__ void cut_bf16x2(float a, float b, uint32_t (&piece)[3]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    piece[i] = pack_bf16x2(a, b);
+    a -= __uint_as_float(piece[i] << 16);
+    b -= __uint_as_float(piece[i] & 0xffff0000u);
+  }
+  piece[2] = pack_bf16x2(a, b);
+}
+
 // The bf16 kernels' width-4 conv, one arithmetic everywhere (gate GEMM with
 // the conv on load, scan kernel, single prefill kernel, stand-alone conv,
 // decode step), so that all of them see bit-identical conv outputs: per

@@ -117,14 +117,11 @@ constexpr float kScale = 0x1p24f;
 __device__ __forceinline__ void cut(const float (&v)[8], Pieces& p) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float a = v[2 * i], b = v[2 * i + 1];
-    p.hi[i] = pack_bf16x2(a, b);
-    a -= __uint_as_float(p.hi[i] << 16);
-    b -= __uint_as_float(p.hi[i] & 0xffff0000u);
-    p.mid[i] = pack_bf16x2(a, b);
-    a -= __uint_as_float(p.mid[i] << 16);
-    b -= __uint_as_float(p.mid[i] & 0xffff0000u);
-    p.lo[i] = pack_bf16x2(a, b);
+    uint32_t piece[3];
+    cut_bf16x2(v[2 * i], v[2 * i + 1], piece);
+    p.hi[i] = piece[0];
+    p.mid[i] = piece[1];
+    p.lo[i] = piece[2];
   }
 }
 

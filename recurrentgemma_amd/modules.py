@@ -152,7 +152,7 @@ def _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
     # head), per chunk of one (few pairs) or by blocks of 32 tokens (pairs that
     # do not come out even on the CUs); many rows of a few tokens and every
     # other dtype or head width: gate GEMM + scan; float32 with 256-wide heads:
-    # one launch for one short row, else conv, projections and recurrence; and
+    # one launch for few short rows, else conv, projections and recurrence; and
     # the join with the gate branch inside those kernels (after the two-kernel
     # form it is a pass of its own).
     if compiled.tracing():
