@@ -355,6 +355,8 @@ hipError_t launch_block_prefill_relay_bf16(FusedArgs a, void* workspace,
                                            hipStream_t s);
 // the same for heads of 128 .. 256 channels, cut into slices of 64: few (row,
 // head) pairs, short rows, narrower heads (rg_prefill_slices.hip)
+bool prefill_short_serves(int B, int H, int T);  // 256-wide heads
+hipError_t launch_block_prefill_short_bf16(const FusedArgs& a, hipStream_t s);
 bool prefill_slices_serve(int B, int H, int T, bool joined);  // 256-wide heads
 bool prefill_narrow_pays(int B, int H, int T, int W);         // narrower ones
 hipError_t launch_block_prefill_slices_bf16(const FusedArgs& a, hipStream_t s);

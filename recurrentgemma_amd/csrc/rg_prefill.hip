@@ -998,6 +998,10 @@ hipError_t launch_block_prefill_bf16(const FusedArgs& a, hipStream_t s) {
   // fit 31-bit byte offsets (checked by the caller)
   const int64_t blocks = (int64_t)a.B * a.H;
   if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
+  // few pairs, rows that are not long: tiles of a row side by side
+  if (a.W / a.H == 256 && a.timing == nullptr &&
+      prefill_short_serves(a.B, a.H, a.T))
+    return launch_block_prefill_short_bf16(a, s);
   // narrow heads, few pairs, short rows: heads in slices
   if (a.W / a.H != 256 ||
       (a.chunks <= 1 &&
