@@ -437,7 +437,7 @@ def run_training(args, torch, rg, ops, wl):
                  "documents": "geometric mean %d" % wl["mean_doc"],
                  "path": "training.differentiable(): kernels for conv, gate "
                          "projections, RG-LRU and the gelu join in both "
-                         "directions; linear layers torch autograd"},
+                         "directions; linear layers rg_matmul.hip"},
       "forward_only_ms": forward_only * 1e3,
       "roofline": {"kernel": "rglru_backward_kernel (rg_rglru_backward)",
                    "bound": "hbm", "achieved": main["achieved_gbs"],

@@ -27,7 +27,7 @@
 // us from a graph, on the float32 matrix instruction (which keeps the SIMD's vector
 // unit busy: matrix and vector work added up, and four tiles a wave were worked off
 // whatever there was of a sequence) / now: W2560 1 x 16 tokens 33.7 / 10, 1 x 128
-// 33.7 / 11.6, 1 x 512 35.8 / 27.8, 1 x 1024 66 / 50, 2 x 300 65.6 / 35; W4096 1 x 512
+// 33.7 / 11.6, 1 x 512 35.8 / 27.8, 1 x 1024 66 / 47, 2 x 300 65.6 / 35; W4096 1 x 512
 // 36.4 / 30.  A turn of eight tiles takes 5.4 us, launch, weights and scan 6.  Without
 // the matrix instructions 24.2 of 27.8, without the cutting 26.5, without the row loads
 // 29.2 of 29.7, the reads of a pass all in front of its products 27.6 with no register
