@@ -126,6 +126,7 @@ PACKAGE_SIGNATURES = {
     "rg_linear_back_pays": (_i, [_i64, _i, _i, _i, _i]),
     "rg_linear_back": (_i, [_vp] * 5 + [_i64, _i, _i, _i, _vp]),
     "rg_linear_weight_grads": (_i, [_vp] * 5 + [_i, _i64, _i, _vp]),
+    "rg_linear_rows_beside": (_i, [_vp] * 4 + [_i] * 4 + [_vp, _vp, _i64, _vp]),
     "rg_linear_gelu_pair_pays": (_i, [_i64, _i, _i, _i]),
     "rg_linear_gelu_pair": (_i, [_vp] * 4 + [_i64, _i, _i, _i, _vp]),
     "rg_linear_scan_best_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),

@@ -84,10 +84,10 @@ PyObject* remember_packed(PyObject*, PyObject* const* v, Py_ssize_t n) {
 // --------------------------------------------------------- recurrent core --
 
 // (x, segment_pos, conv_state, h, conv_w, conv_b, w_x, b_x, w_a, b_a, a_param,
-//  in_place, gate_branch | None) -> (y, h, conv_state) | None
+//  in_place, gate_branch | None, [copy of conv_state | None]) -> (y, h, conv_state) | None
 PyObject* recurrent_step(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    need(n == 13);
+    need(n == 13 || n == 14);
     Call c(v[0]);
     need(c.x.dim() == 3 && c.x.size(1) == 1);
     const int64_t B = c.x.size(0), W = c.x.size(2);
@@ -117,6 +117,8 @@ PyObject* recurrent_step(PyObject*, PyObject* const* v, Py_ssize_t n) {
     }
     const bool in_place = v[11] == Py_True;
     void* gate = v[12] == Py_None ? nullptr : c.shaped(v[12], {B, 1, W});
+    // (read from the copy, the conv state is written while heads are shared)
+    if (n == 14 && v[13] != Py_None) conv_in = c.shaped(v[13], {B, 3, W});
     Tensor y = c.empty(c.x.sizes());
     Tensor h, conv;
     if (in_place) {
@@ -276,10 +278,11 @@ std::vector<int64_t> lead_of(const Call& c, int K, int64_t* M) {
   return lead;
 }
 
-// (plan, x, weights, biases | None, residual | None) -> out | tuple | None
+// (plan, x, weights, biases | None, residual | None[, state]) -> out | tuple | None;
+// with a state (layers packed together): (outputs .., a copy of the state made beside them)
 PyObject* rows_linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    need(n == 5);
+    need(n == 5 || n == 6);
     const RowsPlan& p = plan_of(v[0], v[2], v[3]);
     Call c(v[1]);
     int64_t M;
@@ -305,15 +308,30 @@ PyObject* rows_linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const void* pk = p.packed.const_data_ptr();
     const void* bias = p.bias.defined() ? p.bias.const_data_ptr() : nullptr;
     void* s = c.stream();
-    launch([&] {
-      return rg_linear_rows(x, pk, bias, residual, op, wp, bytes, (int)M, p.K,
-                            p.N, grouped ? p.groups : 1, p.gelu_pair, s);
-    });
+    Tensor aside;
+    if (n == 6) {
+      const Tensor& state = tensor_of(v[5]);
+      const void* from = dense(state, c.dtype, c.device);
+      const int64_t copied = (int64_t)state.nbytes();
+      need(grouped && !residual && !bytes && copied > 0 && copied % 16 == 0);
+      aside = c.empty(state.sizes());
+      void* to = aside.mutable_data_ptr();
+      launch([&] {
+        return rg_linear_rows_beside(x, pk, bias, op, (int)M, p.K, p.N, p.groups, from,
+                                     to, copied, s);
+      });
+    } else {
+      launch([&] {
+        return rg_linear_rows(x, pk, bias, residual, op, wp, bytes, (int)M, p.K,
+                              p.N, grouped ? p.groups : 1, p.gelu_pair, s);
+      });
+    }
     if (!grouped) return wrap(out);
-    PyObject* t = PyTuple_New(p.groups);
+    PyObject* t = PyTuple_New(p.groups + (n == 6));
     if (!t) throw Raised{};
     for (int i = 0; i < p.groups; ++i)
       PyTuple_SET_ITEM(t, i, wrap(out.select(0, i)));
+    if (n == 6) PyTuple_SET_ITEM(t, p.groups, wrap(aside));
     return t;
   });
 }

@@ -1824,6 +1824,45 @@ int rg_linear_rows(const void* x, const void* w_packed, const void* bias,
       __func__, rg::launch_linear_rows(a, gelu_pair != 0, (hipStream_t)stream));
 }
 
+int rg_linear_rows_beside(const void* x, const void* w_packed, const void* bias, void* out,
+                          int M, int K, int N, int groups, const void* from, void* to,
+                          int64_t bytes, void* stream) {
+  RG_REQUIRE(M > 0 && K > 0 && N > 0, "%s: M=%d K=%d N=%d must be positive",
+             __func__, M, K, N);
+  if (M > 64 || rg_linear_packed_bytes(N, K, 0) == 0 ||
+      rg_linear_rows_workspace_bytes(M, K, N) > 0)
+    return fail(RG_ERR_UNSUPPORTED,
+                "%s: needs M <= 64, K %% 64 == 0, N %% 32 == 0 and a K that is not "
+                "split, got M=%d K=%d N=%d", __func__, M, K, N);
+  RG_REQUIRE(groups >= 1 && N % groups == 0 && (N / groups) % 4 == 0,
+             "%s: N=%d / groups=%d must be a multiple of 4", __func__, N,
+             groups);
+  RG_REQUIRE(bytes > 0 && bytes % 16 == 0, "%s: bytes=%lld is no multiple of 16",
+             __func__, (long long)bytes);
+  RG_CHECK_PTR(x);
+  RG_CHECK_PTR(w_packed);
+  RG_CHECK_PTR(out);
+  RG_CHECK_PTR(from);
+  RG_CHECK_PTR(to);
+  RG_CHECK_OPT_PTR(bias);
+  RG_REQUIRE(out != x && to != x && to != from && to != out,
+             "%s: out, to and the inputs must not alias", __func__);
+  rg::LinearArgs a{};
+  a.x = x;
+  a.w_packed = w_packed;
+  a.bias = bias;
+  a.out = out;
+  a.M = M;
+  a.K = K;
+  a.N = N;
+  a.group_width = N / groups;
+  a.copy_from = from;
+  a.copy_to = to;
+  a.copy_items = bytes / 16;
+  return launch_status(__func__,
+                       rg::launch_linear_rows_beside(a, (hipStream_t)stream));
+}
+
 int rg_linear_rows_partial(const void* x, const void* w_packed, void* partial,
                            int M, int K, int N, int slices, void* stream) {
   RG_REQUIRE(M > 0 && K > 0 && N > 0, "%s: M=%d K=%d N=%d must be positive",

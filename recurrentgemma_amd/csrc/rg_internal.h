@@ -214,6 +214,10 @@ struct LinearArgs {
   float* partial;        // [slices, M, N] when K is split over the grid
   int M, K, N;
   int group_width;       // N / G
+  // launch_linear_rows_beside: 16-byte items that workgroups behind the layer's copy
+  const void* copy_from;
+  void* copy_to;
+  int64_t copy_items;
 };
 
 // Each returns hipSuccess or the launch error.  dtype: 0 = f32, 1 = bf16.
@@ -407,6 +411,7 @@ hipError_t launch_linear_pack(const void* w, void* packed, int N, int K,
                               int layout, int groups, int pair, hipStream_t s);
 hipError_t launch_linear_rows(const LinearArgs& a, int gelu_pair,
                               hipStream_t s);
+hipError_t launch_linear_rows_beside(const LinearArgs& a, hipStream_t s);
 // Only the fp32 partial sums a.partial[slices][M][N] of x @ W^T, K split in
 // `slices`; rg_elementwise.hip's norm kernel takes them from there.
 hipError_t launch_linear_rows_partial(const LinearArgs& a, int slices,

@@ -62,10 +62,23 @@ __device__ __forceinline__ size_t out_index(int m, int n, int M, int gw) {
 // XR: rows of x that are loaded and staged (M rounded up to 16, 32 or 64).
 // Every workgroup draws all of x beside its weights: 64 rows are twice the
 // bytes of one tile's weights, whether the rows exist or not.
-template <int NT, int MODE, int XR>
+// BESIDE: the grid goes on behind the layer's workgroups with kCopiers that copy
+// p.copy_items: what the next launch reads while it overwrites the original.
+constexpr int kCopiers = 16;
+
+template <int NT, int MODE, int XR, bool BESIDE>
 __global__ void __launch_bounds__(kWaves * 64)
 linear_rows_kernel(LinearArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  if (BESIDE && blockIdx.x >= gridDim.x - kCopiers) {
+    const u32x4* from = reinterpret_cast<const u32x4*>(p.copy_from);
+    u32x4* to = reinterpret_cast<u32x4*>(p.copy_to);
+    constexpr int64_t step = kCopiers * kWaves * 64;
+    for (int64_t i = (int64_t)(gridDim.x - 1 - blockIdx.x) * (kWaves * 64) + threadIdx.x;
+         i < p.copy_items; i += step)
+      to[i] = from[i];
+    return;
+  }
   constexpr int kLoads = XR / 8;          // of x per chunk
   constexpr int kMB = XR > 32 ? 2 : 1;    // blocks of 32 result rows
   constexpr int kWaveLds = wave_lds_bytes(NT, kMB);
@@ -319,14 +332,14 @@ linear_pack_kernel(const uint16_t* __restrict__ w, u32x4* __restrict__ packed,
   packed[idx] = v;
 }
 
-template <int NT, int MODE, int XR>
+template <int NT, int MODE, int XR, bool BESIDE>
 hipError_t launch_rows_of(const LinearArgs& a, dim3 grid, hipStream_t s) {
   constexpr int lds = kWaves * wave_lds_bytes(NT, XR > 32 ? 2 : 1);
   static OncePerDevice once;  // one per instantiation of this launcher
   hipError_t e = set_max_dynamic_lds(
-      once, (const void*)linear_rows_kernel<NT, MODE, XR>, lds);
+      once, (const void*)linear_rows_kernel<NT, MODE, XR, BESIDE>, lds);
   if (e != hipSuccess) return e;
-  linear_rows_kernel<NT, MODE, XR><<<grid, kWaves * 64, lds, s>>>(a);
+  linear_rows_kernel<NT, MODE, XR, BESIDE><<<grid, kWaves * 64, lds, s>>>(a);
   return hipGetLastError();
 }
 
@@ -341,12 +354,15 @@ hipError_t launch_rows_of(const LinearArgs& a, dim3 grid, hipStream_t s) {
 // (8 staged rows are within 2 % of 16.  Fewer rows without the barrier are
 // slower than 64, 10.0 us for one row at 2560 x 2560: the compiler moves the
 // loads behind the products.)
-template <int NT, int MODE>
+template <int NT, int MODE, bool BESIDE = false>
 hipError_t launch_rows(const LinearArgs& a, dim3 grid, hipStream_t s) {
-  if (a.M <= 16) return launch_rows_of<NT, MODE, 16>(a, grid, s);
-  if (a.M <= 32) return launch_rows_of<NT, MODE, 32>(a, grid, s);
-  return launch_rows_of<NT, MODE, 64>(a, grid, s);
+  if (a.M <= 16) return launch_rows_of<NT, MODE, 16, BESIDE>(a, grid, s);
+  if (a.M <= 32) return launch_rows_of<NT, MODE, 32, BESIDE>(a, grid, s);
+  return launch_rows_of<NT, MODE, 64, BESIDE>(a, grid, s);
 }
+
+// two tiles per workgroup once that still leaves a workgroup for most CUs
+bool two_tiles(int tiles) { return tiles % 2 == 0 && tiles / 2 >= 200; }
 
 }  // namespace
 
@@ -384,10 +400,17 @@ hipError_t launch_linear_rows(const LinearArgs& a, int gelu_pair,
     linear_finish_kernel<<<dim3((quads + 255) / 256), 256, 0, s>>>(a, slices);
     return hipGetLastError();
   }
-  // two tiles per workgroup once that still leaves a workgroup for most CUs
-  if (tiles % 2 == 0 && tiles / 2 >= 200)
-    return launch_rows<2, kStore>(a, dim3(tiles / 2, 1), s);
+  if (two_tiles(tiles)) return launch_rows<2, kStore>(a, dim3(tiles / 2, 1), s);
   return launch_rows<1, kStore>(a, dim3(tiles, 1), s);
+}
+
+// A layer whose K is not split (the caller has seen to it), and the copy beside it:
+// 160 workgroups at N 5120 leave the CUs that do it idle otherwise.
+hipError_t launch_linear_rows_beside(const LinearArgs& a, hipStream_t s) {
+  const int tiles = a.N / 32;
+  if (two_tiles(tiles))
+    return launch_rows<2, kStore, true>(a, dim3(tiles / 2 + kCopiers, 1), s);
+  return launch_rows<1, kStore, true>(a, dim3(tiles + kCopiers, 1), s);
 }
 
 }  // namespace rg

@@ -88,6 +88,13 @@ int rg_linear_weight_grads(const void* const* dy, const void* const* x, void* co
                            const int* out_features, const int* in_features, int count,
                            int64_t M, int dtype, void* stream);
 
+/* rg_linear_rows without a residual, and bytes (a multiple of 16) copied from `from` to
+ * `to` beside it: a state that the next launch on the stream reads from the copy while it
+ * overwrites the original.  RG_ERR_UNSUPPORTED where rg_linear_rows wants a workspace. */
+int rg_linear_rows_beside(const void* x, const void* w_packed, const void* bias, void* out,
+                          int M, int K, int N, int groups, const void* from, void* to,
+                          int64_t bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -115,7 +115,7 @@ def recurrent_core(conv_1d: layers.Conv1D, rg_lru: layers.RGLRU, x,
 
 
 def _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
-                    in_place, gate_branch):
+                    in_place, gate_branch, conv_aside=None):
   bs, l, _ = x.shape
   assert segment_pos.shape == (bs, l)
   fused = conv_1d.temporal_width == 4
@@ -134,7 +134,7 @@ def _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
       else:
         y, h, conv_state = ops.recurrent_step(
             x, segment_pos, cache.conv1d_state, cache.rg_lru_state, *weights,
-            in_place=in_place, gate_branch=gate_branch)
+            in_place=in_place, gate_branch=gate_branch, conv_aside=conv_aside)
       if not return_cache:
         return y, None
       return y, RecurrentBlockCache(rg_lru_state=h, conv1d_state=conv_state)
@@ -231,6 +231,8 @@ class RecurrentBlock(nn.Module):
       if done is not None:
         y, h, conv_state = done
         return y, RecurrentBlockCache(rg_lru_state=h, conv1d_state=conv_state)
+    in_place = self.decode_in_place and cache is not None and return_cache
+    aside = None
     with torch.no_grad():
       # (a traced program keeps torch's own linear layers: the few-row
       # kernels are reached through ctypes, which a tracer cannot follow)
@@ -243,15 +245,23 @@ class RecurrentBlock(nn.Module):
         w_y, b_y = _parameters(linear["linear_y"], "weight", "bias")
         w_x, b_x = _parameters(linear["linear_x"], "weight", "bias")
         w_out, b_out = _parameters(linear["linear_out"], "weight", "bias")
-        y, x = self._rows_yx(x, (w_y, w_x), (b_y, b_x))
+        # (a step in place: the conv state copied beside the layers, so that
+        # the step's workgroups may share heads while they overwrite it)
+        done = None
+        if in_place and self.conv_1d.temporal_width == 4:
+          done = self._rows_yx.beside(x, (w_y, w_x), (b_y, b_x),
+                                      cache.conv1d_state)
+        if done is not None:
+          y, x, aside = done
+        else:
+          y, x = self._rows_yx(x, (w_y, w_x), (b_y, b_x))
       else:
         y, x = linears(x, self.linear_y, self.linear_x)
       # x * gelu(y) (modules.py:627-628, 644) is part of the core call: inside
       # the prefill kernel where that runs, one pass after it elsewhere
-      x, new_cache = recurrent_core(
+      x, new_cache = _recurrent_core(
           self.conv_1d, self.rg_lru, x, segment_pos, cache, return_cache,
-          in_place=self.decode_in_place and cache is not None and return_cache,
-          gate_branch=y)
+          in_place, y, aside)
       if few_rows and defer_out and ops.PackedLinear.partial_slices(
           x, self.lru_width, self.width):
         x = self._rows_out.partial(x, (w_out,), (b_out,))

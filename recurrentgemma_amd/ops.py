@@ -1188,6 +1188,15 @@ class PackedLinear:
     return PartialSums(sums, self._bias, (*x.shape[:-1], N), x.dtype, addend)
 
   @torch.no_grad()
+  def beside(self, x, weights, biases, state):
+    """The outputs of layers packed together and, made in the same launch, a copy
+    of `state`, which the next launch may then overwrite while it reads the copy:
+    (outputs .., copy), or None where that is not to be had."""
+    if self._plan is None:
+      return None
+    return _lib.host().rows_linear(self._plan, x, weights, biases, None, state)
+
+  @torch.no_grad()
   def __call__(self, x, weights, biases=None, residual=None):
     """x [..., K].  Returns out [..., N] (one layer), a tuple of outputs
     (several layers / a stacked weight), or the gelu pair product [..., N/2].
@@ -1235,16 +1244,19 @@ class PackedLinear:
 
 
 def recurrent_step(x, segment_pos, conv_cache, h, conv_w, conv_b, w_x, b_x, w_a,
-                   b_a, a_param, in_place=False, gate_branch=None):
+                   b_a, a_param, in_place=False, gate_branch=None,
+                   conv_aside=None):
   """One decode step of conv -> RG-LRU.  Returns (y, h_new, conv_cache_new).
 
   bf16 with 256-wide heads runs as one launch on re-laid-out gate weights
   (packed once per weight version); other shapes as conv step + gate GEMM +
   scan step.  gate_branch: the block's linear_y output [B,1,W]; y is then
-  y * gelu(gate_branch) (inside the one launch where that runs)."""
+  y * gelu(gate_branch) (inside the one launch where that runs).  conv_aside: a
+  copy of conv_cache made earlier on the stream (PackedLinear.beside); reading
+  it, a step in place may share heads among workgroups."""
   done = _lib.host().recurrent_step(x, segment_pos, conv_cache, h, conv_w,
                                     conv_b, w_x, b_x, w_a, b_a, a_param,
-                                    in_place, gate_branch)
+                                    in_place, gate_branch, conv_aside)
   if done is not None:  # (None: not the ordinary case, see host_ops.cpp)
     return done
   B, n_tok, W = x.shape
