@@ -134,7 +134,7 @@ def _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
       else:
         y, h, conv_state = ops.recurrent_step(
             x, segment_pos, cache.conv1d_state, cache.rg_lru_state, *weights,
-            in_place=in_place, gate_branch=gate_branch, conv_aside=conv_aside)
+            in_place, gate_branch, conv_aside)
       if not return_cache:
         return y, None
       return y, RecurrentBlockCache(rg_lru_state=h, conv1d_state=conv_state)
@@ -149,7 +149,8 @@ def _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
   else:
     # One call; the library picks the kernels (rg_recurrent_core): for bf16
     # and 256-wide heads the single-launch kernel, one workgroup per (row,
-    # head), per chunk of one (few pairs) or by blocks of 32 tokens (pairs that
+    # head), per 32 channels of one (few rows of some hundred tokens), per
+    # chunk of one (few long ones) or by blocks of 32 tokens (pairs that
     # do not come out even on the CUs); many rows of a few tokens and every
     # other dtype or head width: gate GEMM + scan; float32 with 256-wide heads:
     # one launch for few short rows, else conv, projections and recurrence; and
