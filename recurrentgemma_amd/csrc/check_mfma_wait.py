@@ -1,5 +1,6 @@
 #!/usr/bin/env python3
-"""Build check for kernels whose matrix instructions are inline assembly.
+"""Build check for kernels whose matrix instructions or loads to LDS are inline
+assembly.
 
 The compiler does not know that such a statement is a matrix instruction and
 counts no wait states behind it: a vector, LDS or memory instruction that
@@ -11,6 +12,12 @@ instruction touches a matrix instruction's destination registers within
 WINDOW instructions of it without such a wait in between -- which is what a
 register copy that the compiler decided to insert there would look like.
 
+Nor does it count wait states in front of a load in such a statement.  Reported
+too are a load to LDS right behind the write of M0, which says where to (one
+wait state: the compiler puts an instruction there for its own), and a memory
+instruction that reads a scalar register within five wait states of the vector
+instruction that wrote it (a descriptor made with v_readfirstlane).
+
 usage: check_mfma_wait.py file.s
 """
 import re
@@ -18,6 +25,9 @@ import sys
 
 WINDOW = 20  # instructions; 16 passes need at most 18 wait states
 REG = re.compile(r'\b([va])(?:(\d+)\b|\[([^\]]+)\])')
+SCALAR_REG = re.compile(r'\b(s)(?:(\d+)\b|\[([^\]]+)\])')
+SCALAR_WINDOW = 5  # wait states from a vector write to a memory read
+MEMORY = ('buffer_', 'global_', 'flat_', 'scratch_')
 
 
 def _value(expr):
@@ -26,10 +36,10 @@ def _value(expr):
   return int(eval(expr))  # digits, +, * only (checked above)
 
 
-def registers(text):
+def registers(text, kinds=REG):
   """{('v', 3), ...} named in an operand string."""
   out = set()
-  for kind, single, inner in REG.findall(text):
+  for kind, single, inner in kinds.findall(text):
     if single:
       out.add((kind, int(single)))
     elif ':' in inner:
@@ -40,9 +50,39 @@ def registers(text):
   return out
 
 
+def early_loads(path):
+  """How many loads come too soon behind what they read (see above)."""
+  written = []  # [scalar registers, wait states left]
+  m0 = False    # the last instruction wrote it
+  bad = 0
+  for number, line in enumerate(open(path), 1):
+    text = line.split(';')[0].strip()
+    if not text or text.startswith('.') or text.endswith(':'):
+      continue
+    op, _, operands = text.partition(' ')
+    waits = 1
+    if op.startswith('s_nop'):
+      waits += _value(operands.strip())
+    elif op.startswith(MEMORY):
+      if m0 and re.search(r'\blds\b', operands):
+        print(f'{path}:{number}: `{text}` right behind the write of M0')
+        bad += 1
+      used = registers(operands, SCALAR_REG)
+      if any(d & used for d, _ in written):
+        print(f'{path}:{number}: `{text}` reads a scalar register written by a '
+              f'vector instruction fewer than {SCALAR_WINDOW} wait states before')
+        bad += 1
+    first = operands.split(',')[0].strip()
+    m0 = first == 'm0'
+    written = [[d, n - waits] for d, n in written if n > waits]
+    if op.startswith('v_') and first.startswith('s'):
+      written.append([registers(first, SCALAR_REG), SCALAR_WINDOW])
+  return bad
+
+
 def main(path):
   pending = []  # [destination registers, instructions left]
-  bad = 0
+  bad = early_loads(path)
   for number, line in enumerate(open(path), 1):
     text = line.split(';')[0].strip()
     if not text or text.startswith('.') or text.endswith(':'):

@@ -42,10 +42,9 @@
 // it leaves -- is attn_prompt_prepare_kernel at
 // the end of this file; the queries take their rotary embedding inside the
 // attention kernel.
-#include <utility>
-
 #include "rg_common.h"
 #include "rg_internal.h"
+#include "rg_matrix_asm.h"
 
 namespace rg {
 namespace {
@@ -57,11 +56,8 @@ constexpr int kBlockBytes = kBlockKeys * kAttnHd * 2;
 constexpr int kRing = 4;  // blocks of keys, and of values, in LDS
 constexpr int kAttnLds = 2 * kRing * kBlockBytes;
 
-typedef __attribute__((address_space(3))) unsigned char lds_byte;
-typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+using namespace matrix_asm;
 typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 union AFrag {
   bf16x8 v;
@@ -76,52 +72,11 @@ union AFrag {
 // (left to the register allocator they were moved between the two register files every
 // block).  The build checks that the compiler allocates no accumulation register of its
 // own in this file.
-template <int N>
-__device__ __forceinline__ float acc_read() {
-  float t;
-  asm volatile("v_accvgpr_read_b32 %0, a[%c1]" : "=v"(t) : "n"(N));
-  return t;
-}
-template <int N>
-__device__ __forceinline__ void acc_write(float t) {
-  asm volatile("v_accvgpr_write_b32 a[%c1], %0" ::"v"(t), "n"(N));
-}
-template <int N>
-__device__ __forceinline__ void acc_zero() {
-  asm volatile("v_accvgpr_write_b32 a[%c0], 0" ::"n"(N));
-}
-// block BLK of O^T += a x b
-template <int BLK>
-__device__ __forceinline__ void acc_mfma(const f32x4& a, const f32x4& b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 a[%c2:%c2+3], %0, %1, a[%c2:%c2+3]" ::"v"(a),
-               "v"(b), "n"(4 * BLK));
-}
-template <int... I, class F>
-__device__ __forceinline__ void for_each(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void for_n(F&& f) {
-  for_each(std::make_integer_sequence<int, N>{}, f);
-}
 __device__ __forceinline__ float max3(float a, float b, float c) {
   float r;
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
-// The compiler does not count the wait states between a matrix instruction in
-// inline assembly and a read of its result.
-__device__ __forceinline__ void wait_for_matrix_results() {
-  asm volatile("s_nop 15\n\ts_nop 7");
-}
-__device__ __forceinline__ u32x4 scalar_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t at = (uint64_t)base;
-  return u32x4{
-      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at),
-      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) & 0xffffu,
-      (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-
 // Rotary embedding of the first half of a query's dimensions (elements i and
 // i + 64, i < 64) where the query lies as operand fragments: k-steps 0 and 1 hold
 // this lane's elements 32 ks + 8 quarter + 0..7, k-steps 2 and 3 their partners.
@@ -238,7 +193,7 @@ attn_prefill_bf16_kernel(AttnPrefillArgs p) {
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "a255");  // (the kernel has them)
+  take_accumulators();
   for_n<64 * QB>([&](auto I) RG_INLINE { acc_zero<decltype(I)::value>(); });
 
   // first visible key of a query (non-decreasing in it): what bounds the blocks that
@@ -263,9 +218,8 @@ attn_prefill_bf16_kernel(AttnPrefillArgs p) {
                     16u * ((lane & 3) ^ ((lane >> 3) & 3))
               : (uint32_t)(row2 * 512 + 16 * ((lane & 31) ^ ((row2 & 3) << 1)));
   auto load_one = [&](int to, int r, uint32_t v, u32x4 rsrc, int at) RG_INLINE {
-    const uint32_t m0 = lds0 + (uint32_t)to + 4096u * (uint32_t)r + 1024u * (uint32_t)wave;
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(m0),
-                 "v"(v), "s"(rsrc), "s"(at));
+    const uint32_t where = lds0 + (uint32_t)to + 4096u * (uint32_t)r + 1024u * (uint32_t)wave;
+    load_lds_16<0>(where, v, rsrc, at);
   };
   // (past the last key the descriptor's end: nothing is read)
   auto load_keys = [&](int j, int r) RG_INLINE {

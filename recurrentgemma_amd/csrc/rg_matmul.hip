@@ -38,59 +38,18 @@
 // gradients of 2560 x 2560 over 8192 rows 1340 (770).
 #include <math.h>
 
-#include <utility>
-
 #include "rg_common.h"
 #include "rg_internal.h"
+#include "rg_matrix_asm.h"
 
 namespace rg {
 namespace {
 
-typedef __attribute__((address_space(3))) unsigned char lds_byte;
-typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+using namespace matrix_asm;
 
 constexpr int kStep = 64;           // of the contraction, per stage
 constexpr int kPanelBytes = 8192;   // 64 x 64 values of one operand
 constexpr int kAccBlocks = 64;      // 16 x 16 results in a[0:255], the rest in VGPRs
-
-// The first 64 result blocks of a wave live in the accumulation registers, which are
-// numbered by hand (the build checks that the compiler takes none for itself).
-template <int N>
-__device__ __forceinline__ float acc_read() {
-  float t;
-  asm volatile("v_accvgpr_read_b32 %0, a[%c1]" : "=v"(t) : "n"(N));
-  return t;
-}
-template <int N>
-__device__ __forceinline__ void acc_zero() {
-  asm volatile("v_accvgpr_write_b32 a[%c0], 0" ::"n"(N) : "a255");
-}
-template <int BLK>
-__device__ __forceinline__ void acc_mfma(const f32x4& a, const f32x4& b) {
-  asm volatile(
-      "v_mfma_f32_16x16x32_bf16 a[%c2:%c2+3], %0, %1, a[%c2:%c2+3]" ::"v"(a),
-      "v"(b), "n"(4 * BLK));
-}
-
-template <int... I, class F>
-__device__ __forceinline__ void for_each(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void for_n(F&& f) {
-  for_each(std::make_integer_sequence<int, N>{}, f);
-}
-
-// A buffer descriptor in scalar registers, for inline assembly.
-__device__ __forceinline__ u32x4 scalar_rsrc(const void* base, int64_t bytes) {
-  const uint64_t at = (uint64_t)base;
-  return u32x4{
-      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at),
-      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) & 0xffffu,
-      (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
 
 // Which tile a workgroup has: contiguous runs of tiles per XCD (workgroups go to the
 // eight XCDs in turn); inside a product eight tile rows side by side, so that the 32
@@ -279,13 +238,8 @@ matmul_bf16_kernel(MatmulArgs args) {
     constexpr bool is_m = i / 2 < kPanelsM;
     constexpr bool is_up = kPair && i / 2 - kPanelsM >= NB / 2;
     const u32x4 r = is_m ? rm : is_up ? rn_up : rn;
-    // (inline assembly: behind the builtin the compiler has every transposing LDS read
-    // wait for all loads on their way)
-    const uint32_t to = stage + 1024 * (uint32_t)wave, v = is_m ? vm : vn;
-    const int at = scalar_offset[i];
-    asm volatile("s_add_u32 m0, %0, %c1\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds" ::"s"(to),
-                 "n"(i / 2 * kPanelBytes + (i & 1) * 4096), "v"(v), "s"(r), "s"(at)
-                 : "scc");
+    load_lds_16<i / 2 * kPanelBytes + (i & 1) * 4096>(
+        stage + 1024 * (uint32_t)wave, is_m ? vm : vn, r, scalar_offset[i]);
   };
 
   // ---- lines of the step after a stage's, asked into L2 ------------------------------
@@ -311,9 +265,7 @@ matmul_bf16_kernel(MatmulArgs args) {
   const uint32_t step_p = wave == 0 ? step_m : step_n;
   uint32_t vp = vp0 + step_p;
   auto prefetch = [&] {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(
-                     (uint32_t)(uintptr_t)lds + 2 * kStage + 256 * (uint32_t)wave),
-                 "v"(vp), "s"(rp));
+    load_lds_4((uint32_t)(uintptr_t)lds + 2 * kStage + 256 * (uint32_t)wave, vp, rp);
   };
   int load_step = 0;
   auto advance = [&] {  // a stage's loads are out: on to the next step's
@@ -367,6 +319,7 @@ matmul_bf16_kernel(MatmulArgs args) {
   f32x4 extra[kInVgprs > 0 ? kInVgprs : 1];
 #pragma unroll
   for (int i = 0; i < kInVgprs; ++i) extra[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  take_accumulators();
   for_n<4 * (MB * kBlocksN - kInVgprs)>([&](auto I) { acc_zero<decltype(I)::value>(); });
 
   // a half step's matrix instructions, with what `between` issues behind each
@@ -489,10 +442,7 @@ __global__ void __launch_bounds__(256) matmul_small_bf16_kernel(MatmulArgs args)
       const int where = (is_m ? kSlowM : kSlowN) ? row * ld2 + 128 * panel
                                                  : (64 * panel + row) * ld2;
       const u32x4 r = is_m ? rm : is_up ? rn_up : rn;
-      const uint32_t v = is_m ? vm : vn, to = load_stage;
-      asm volatile("s_add_u32 m0, %0, %c1\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds" ::"s"(to),
-                   "n"(i / 2 * kPanelBytes + (i & 1) * 4096), "v"(v), "s"(r), "s"(where)
-                   : "scc");
+      load_lds_16<i / 2 * kPanelBytes + (i & 1) * 4096>(load_stage, is_m ? vm : vn, r, where);
     });
     load_stage += kStage;
     if (load_stage == stages_end) load_stage -= STAGES * kStage;

@@ -310,6 +310,34 @@ def test_build_check_for_early_reads_of_matrix_results(tmp_path):
     assert rc == want, name
 
 
+def test_build_check_for_early_loads(tmp_path):
+  """check_mfma_wait.py: a load to LDS right behind the write of M0, and a memory
+  instruction close behind the vector instruction that wrote a scalar register it
+  reads, are reported; with the wait states in between they are not."""
+  import subprocess
+  import sys
+  script = os.path.join(_lib.CSRC, "check_mfma_wait.py")
+  load = "\tbuffer_load_dwordx4 v1, s[4:7], s9 offen lds\n"
+  lane = "\tv_readfirstlane_b32 s5, v8\n"
+  cases = {
+      "at_once": ("\ts_add_u32 m0, s8, 0x400\n" + load, 1),
+      "moved_at_once": ("\ts_mov_b32 m0, s8\n\t;;#ASMEND\n" + load, 1),
+      "one_wait": ("\ts_add_u32 m0, s8, 0x400\n\ts_nop 0\n" + load, 0),
+      "one_instruction": ("\ts_mov_b32 m0, s8\n\ts_movk_i32 s9, 0x1000\n" + load, 0),
+      "not_to_lds": ("\ts_mov_b32 m0, s8\n"
+                     "\tbuffer_load_dwordx4 v[0:3], v1, s[4:7], 0 offen\n", 0),
+      "descriptor": (lane + "\ts_nop 3\n" + load, 1),
+      "descriptor_later": (lane + "\ts_nop 4\n" + load, 0),
+      "other_scalar": ("\tv_readfirstlane_b32 s10, v8\n" + load, 0),
+  }
+  for name, (text, want) in cases.items():
+    path = tmp_path / (name + ".s")
+    path.write_text(text)
+    rc = subprocess.run([sys.executable, script, str(path)],
+                        stdout=subprocess.DEVNULL).returncode
+    assert rc == want, name
+
+
 def test_bench_refuses_more_than_one_gpu():
   """bench.py measures one GPU; any other --gpus ends with a message, not a
   number."""
