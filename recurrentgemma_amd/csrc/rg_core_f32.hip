@@ -147,6 +147,9 @@ __device__ __forceinline__ void cut_rows(float a, float b, uint32_t (&piece)[3])
   b -= __uint_as_float(piece[1] & 0xffff0000u);
   piece[2] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), upper);
 }
+// From here on the pieces of a value hold all of it: the last of its 24 bits is worth
+// 2^-133, the least that a bf16 has.  (Below 2^-134, 5e-41, they are zeros.)
+constexpr float kExactOwn = 0x1p-110f;
 // A lane's number that nothing is worked out from ahead of a loop: what is worked out
 // from it is worked out again where it is used, instead of being kept in registers.
 template <class V>
@@ -390,7 +393,7 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
         }
         __builtin_amdgcn_wave_barrier();
         // the conv output of the workgroup's own channels, which the gate arithmetic
-        // multiplies, put together again (exactly)
+        // multiplies, put together again: exactly from kExactOwn on
         if (pass == (s >> 2)) {
           const int g = fresh(lane) >> 4, n = fresh(lane) & 15;
           const int own_at = g * 4 * kRow + (g & 1) * kRow +
@@ -437,12 +440,19 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
       });
       f32x4 pre_x = hi_x + low_x, pre_a = hi_a + low_a;
       // A piece of an infinity is no number, and a product of pieces may overflow
-      // where the product does not: what is not finite is computed again in float32
+      // where the product does not: what is not finite is computed again in float32,
+      // and so is a conv output whose last digits the third piece cannot hold (zero is
+      // none: one less than it is the largest of all).
       float none = 0.0f;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         none = __builtin_fmaf(pre_a[q], 0.0f, __builtin_fmaf(pre_x[q], 0.0f, none));
-      if (__builtin_expect(__ballot(none != 0.0f) != 0, 0)) {
+      uint32_t least = 0xffffffffu;  // of the magnitudes' bits, twice, less one
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        least = min(least, (__float_as_uint(own[q]) << 1) - 1u);
+      const bool small = least < (__builtin_bit_cast(uint32_t, kExactOwn) << 1) - 1u;
+      if (__builtin_expect(__ballot(none != 0.0f || small) != 0, 0)) {
         const float b_x = fresh(bias_x), b_a = fresh(bias_a);
         f32x4 full_x = {b_x, b_x, b_x, b_x}, full_a = {b_a, b_a, b_a, b_a};
         float* const rows = reinterpret_cast<float*>(stage);

@@ -95,6 +95,24 @@ def test_a_value_whose_pieces_overflow(value):
   assert torch.equal(torch.isinf(y), torch.isinf(yo))
 
 
+@pytest.mark.parametrize("scale", [1e-30, 1e-34, 1e-36])
+def test_small_inputs_keep_their_digits(scale):
+  """Inputs whose last digits no bf16 piece can hold: y is as close to 64 bits as at
+  ordinary sizes (the float32 bar; pieces put together again are off by 4e-6 at 1e-35
+  and 3e-4 at 1e-37, which is where the conv takes 1e-36)."""
+  B, T, H = 1, 70, 2
+  W = 256 * H
+  p = R.make_params(W, H, torch.float32, seed=9, gate_bias_std=0.3)
+  p["conv_b"] = torch.zeros_like(p["conv_b"])
+  g = torch.Generator().manual_seed(10)
+  x = torch.randn(B, T, W, generator=g) * scale
+  seg = torch.arange(T).repeat(B, 1)
+  y, h, _ = one_launch(x, seg, p)
+  yo, ho, _ = wanted(x.double(), seg, {k: v.double() for k, v in p.items()})
+  got, want = (y.double() / scale, h.double() / scale), (yo / scale, ho / scale)
+  assert all(helpers.max_rel(a, b) < 1e-5 for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("B,T,H,several", [
     (1, 500, 10, False), (2, 300, 10, False), (1, 2048, 1, True), (2, 640, 10, True)])
 def test_the_form_is_chosen_by_the_time_it_takes(B, T, H, several):
