@@ -1210,6 +1210,13 @@ size_t rg_argmax_workspace_bytes(int rows, int n) {
   return rows > 0 && n > 0 ? rg::argmax_workspace_bytes(rows, n) : 0;
 }
 
+// Whether a tensor that a launch writes is one of those that it reads.
+static bool among(const void* p, const void* const* list, int n) {
+  for (int i = 0; list && i < n; ++i)
+    if (list[i] == p) return true;
+  return false;
+}
+
 // x [M, K] and weights [N_i, K] as one launch of products, or nothing where they do not
 // fit one
 static bool linear_many_args(const void* x, int64_t M, int K, int count,
@@ -1253,6 +1260,9 @@ int rg_linear_many(const void* x, int64_t M, int K, int count, const void* const
     RG_CHECK_PTR(w[i]);
     RG_CHECK_PTR(out[i]);
     if (bias) RG_CHECK_OPT_PTR(bias[i]);
+    RG_REQUIRE(out[i] != x && !among(out[i], w, count) && !among(out[i], bias, count) &&
+                   !among(out[i], out, i),
+               "%s: outputs must not alias an input or each other", __func__);
   }
   rg::MatmulArgs a;
   if (dtype != RG_DTYPE_BF16 ||
@@ -1304,6 +1314,8 @@ int rg_linear_back(const void* dy, const void* w, const void* dy2, const void* w
   RG_CHECK_OPT_PTR(dy2);
   RG_CHECK_OPT_PTR(w2);
   RG_CHECK_PTR(dx);
+  RG_REQUIRE(dx != dy && dx != w && dx != dy2 && dx != w2,
+             "%s: dx must not alias an input", __func__);
   rg::MatmulArgs a;
   if (dtype != RG_DTYPE_BF16 || !linear_back_args(dy, w, dy2, w2, dx, M, K, N, &a) ||
       !rg::matmul_serves(a, rg::kMatmulBack))
@@ -1328,6 +1340,8 @@ int rg_linear_weight_grads(const void* const* dy, const void* const* x, void* co
     RG_CHECK_PTR(dy[i]);
     RG_CHECK_PTR(x[i]);
     RG_CHECK_PTR(dw[i]);
+    RG_REQUIRE(!among(dw[i], dy, count) && !among(dw[i], x, count) && !among(dw[i], dw, i),
+               "%s: gradients must not alias an input or each other", __func__);
     if (!fits) continue;
     rg::MatmulProblem& p = a.p[a.count++];
     p.m = dy[i];
@@ -1379,6 +1393,8 @@ int rg_linear_gelu_pair(const void* x, const void* w, const void* bias, void* ou
   RG_CHECK_PTR(w);
   RG_CHECK_OPT_PTR(bias);
   RG_CHECK_PTR(out);
+  RG_REQUIRE(out != x && out != w && out != bias, "%s: out must not alias an input",
+             __func__);
   rg::MatmulArgs a;
   if (dtype != RG_DTYPE_BF16 || !gelu_pair_args(x, w, bias, out, M, K, N, &a) ||
       !rg::matmul_serves(a, rg::kMatmulGeluPair))
@@ -1845,8 +1861,11 @@ int rg_linear_rows_beside(const void* x, const void* w_packed, const void* bias,
   RG_CHECK_PTR(from);
   RG_CHECK_PTR(to);
   RG_CHECK_OPT_PTR(bias);
-  RG_REQUIRE(out != x && to != x && to != from && to != out,
-             "%s: out, to and the inputs must not alias", __func__);
+  for (const void* written : {(const void*)out, (const void*)to})
+    RG_REQUIRE(written != x && written != w_packed && written != from &&
+                   written != bias,
+               "%s: out and to must not alias an input", __func__);
+  RG_REQUIRE(to != out, "%s: out and to must not alias", __func__);
   rg::LinearArgs a{};
   a.x = x;
   a.w_packed = w_packed;

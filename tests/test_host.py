@@ -265,6 +265,36 @@ def test_c_side_validation_without_launch():
   assert lib.rg_packed_gate_weights_bytes(4096, 8, 1) == 0  # 512-wide heads
 
 
+def test_products_refuse_an_output_that_is_an_input():
+  """The linear layers of many rows and the layer with a copy beside it, as their
+  neighbours: an output that is an input, or another output, is refused before
+  anything is launched."""
+  lib = _lib.lib()
+  BAD = -1  # RG_ERR_BAD_ARG
+  x, w, b, out, more, last = (256 * i for i in range(1, 7))  # never dereferenced
+  some = lambda *p: (ctypes.c_void_p * len(p))(*p)
+  ints = lambda *v: (ctypes.c_int * len(v))(*v)
+  many = lambda bias, *outs: lib.rg_linear_many(
+      x, 64, 64, 2, some(w, more), bias, some(*outs), ints(64, 64), 1, None)
+  for outs in ((x, out), (out, x), (w, out), (out, w), (more, out), (out, out)):
+    assert many(None, *outs) == BAD, outs
+  assert many(some(b, None), out, b) == BAD and many(some(None, b), b, out) == BAD
+  for dx in (x, w, more, last):
+    assert lib.rg_linear_back(x, w, more, last, dx, 64, 64, 64, 1, None) == BAD
+  for dws in ((x, out), (out, w), (b, out), (out, more), (out, out)):
+    assert lib.rg_linear_weight_grads(
+        some(x, w), some(b, more), some(*dws), ints(64, 64), ints(64, 64), 2, 64, 1,
+        None) == BAD, dws
+  for o in (x, w, b):
+    assert lib.rg_linear_gelu_pair(x, w, b, o, 64, 64, 64, 1, None) == BAD
+  beside = lambda o, to: lib.rg_linear_rows_beside(
+      x, w, b, o, 8, 64, 64, 1, more, to, 256, None)
+  for taken in (x, w, b, more):
+    assert beside(taken, last) == BAD and beside(out, taken) == BAD
+  assert beside(out, out) == BAD
+  assert b"alias" in lib.rg_last_error()
+
+
 def test_prefill_kernel_keeps_its_hand_numbered_registers():
   """The prefill kernel's gate weights sit in accumulation registers that the
   source numbers itself; the compiled kernels may touch those registers only
