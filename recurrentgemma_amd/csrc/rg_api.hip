@@ -633,29 +633,20 @@ static bool wide_f32_ahead(int B, int T, int W, int H) {
       (elements < 3e5f ? 18.0f : 22.0f) + 0.85e-5f * elements + 0.005f * T;
   return several < one_launch;
 }
-// Where the workspace of the form of several launches is asked for.  With more pairs
-// it is the form unless there are a few rows of all (against gate GEMM + scan: W2560
-// B64 T1 20.5 / 23, T16 73 / 50, B4 T2048 519 / 240, B8 T2048 joined 878 / 523; W4096
-// B3 T16 18 / 22, B4 T512 206 / 93; W256 B64 T16 19.2 / 20.5, T64 37 / 29).  With few
-// it is asked for where it may be ahead and further down, as it always was, so that a
-// caller's sizes stay what they are; wide_f32_ahead decides.
-static bool wide_f32_room(int B, int T, int W, int H, bool one_launch_takes) {
-  const float elements = (float)B * T * W;
-  if (!one_launch_takes) return elements > 3e5f;
-  const float rounds =
-      33.0f * (((int64_t)B * H + 15) / 16) * ((T + 511) / 512);
-  return 17.0f + 1.1e-5f * elements < 0.95f * rounds;
-}
 
 static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
   CorePlan p{};
   // float32 with few rows: one launch, no workspace; or, with one, the form of
-  // several launches where that is ahead
+  // several launches where that is ahead.  With more pairs that is the form unless
+  // there are a few rows of all (against gate GEMM + scan: W2560 B64 T1 20.5 / 23, T16
+  // 73 / 50, B4 T2048 519 / 240, B8 T2048 joined 878 / 523; W4096 B3 T16 18 / 22, B4
+  // T512 206 / 93; W256 B64 T16 19.2 / 20.5, T64 37 / 29).
   p.small_f32 = dtype == RG_DTYPE_F32 && rg::core_f32_small_serves(B, T, W, H);
   p.wide_f32 = dtype == RG_DTYPE_F32 &&
                rg::gates_f32_serves((int64_t)B * T, W, H) &&
                rg::scan_tiles_take(T, W, dtype) &&
-               wide_f32_room(B, T, W, H, p.small_f32);
+               (p.small_f32 ? wide_f32_ahead(B, T, W, H)
+                            : (float)B * T * W > 3e5f);
   if (p.wide_f32 && wide_scan_on_tiles(B, T, W))
     p.deal_bytes = rg::scan_tiles_deal_bytes(B, T, W, dtype, rg::kTilesFwdGated);
   if (p.small_f32) {
@@ -747,8 +738,7 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
                 __func__, need, workspace ? workspace_bytes : (size_t)0);
   // (the form of several launches keeps the conv output where y goes, and the
   // pre-activations in a workspace that the one-launch form does not ask for)
-  const bool wide = p.wide_f32 && (!p.small_f32 || wide_f32_ahead(B, T, W, H)) &&
-                    gate_branch != out && workspace != nullptr &&
+  const bool wide = p.wide_f32 && gate_branch != out && workspace != nullptr &&
                     workspace_bytes >= p.split_bytes + 2 * p.gate_bytes &&
                     aligned16(workspace);
   if (p.small_f32 || wide) {

@@ -16,10 +16,14 @@ NAMES = ("conv_w", "conv_b", "w_x", "b_x", "w_a", "b_a", "a_param")
 
 
 @pytest.mark.parametrize("B,T,H,mean_doc,joined,with_h0,with_conv", [
-    # at most 32 pairs, where the workspace that is brought makes the choice
+    # at most 32 pairs: one launch, which asks for no workspace
     (1, 1, 1, 0, True, True, True), (1, 2, 10, 0, False, False, True),
     (2, 31, 10, 7, True, True, True), (3, 64, 10, 20, False, True, False),
     (1, 257, 2, 60, True, False, True), (2, 700, 4, 100, False, True, True),
+    # ... and several with the workspace that is brought, where they are ahead
+    (1, 641, 1, 70, True, True, True), (2, 1041, 2, 0, False, True, True),
+    (3, 401, 7, 100, True, False, True), (20, 513, 1, 60, False, True, False),
+    (1, 2047, 10, 300, True, True, True),
     # more pairs: one-pass recurrence, and by the token
     (12, 64, 3, 15, True, True, True), (4, 130, 10, 50, False, False, True),
     (40, 33, 1, 10, True, False, True), (9, 45, 8, 0, False, True, True),
@@ -30,7 +34,9 @@ def test_against_the_oracle(B, T, H, mean_doc, joined, with_h0, with_conv):
   W = 256 * H
   lib = _lib.lib()
   best = lib.rg_recurrent_core_best_workspace_bytes(B, T, W, H, 0)
-  assert best >= 2 * 4 * B * T * W
+  several = (B, T, H) not in [(1, 1, 1), (1, 2, 10), (2, 31, 10), (3, 64, 10),
+                              (1, 257, 2), (2, 700, 4)]
+  assert best >= 2 * 4 * B * T * W if several else best == 0
   assert lib.rg_recurrent_core_workspace_bytes(B, T, W, H, 0) == (
       0 if B * H <= 32 else best)
   p = R.make_params(W, H, torch.float32, seed=T + H, gate_bias_std=0.3)

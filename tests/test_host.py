@@ -295,6 +295,17 @@ def test_products_refuse_an_output_that_is_an_input():
   assert b"alias" in lib.rg_last_error()
 
 
+@pytest.mark.parametrize("B,T,H,several", [
+    (1, 1, 1, False), (1, 512, 10, False), (2, 300, 10, False), (3, 64, 10, False),
+    (2, 700, 4, False), (1, 641, 1, True), (2, 640, 10, True), (1, 2048, 10, True),
+    (20, 513, 1, True), (33, 64, 1, True)])
+def test_float32_workspace_only_where_it_is_used(B, T, H, several):
+  """The workspace that the package brings to a float32 prefill: what the form of
+  several launches takes where that form runs, nothing where one launch does."""
+  best = _lib.lib().rg_recurrent_core_best_workspace_bytes(B, T, 256 * H, H, 0)
+  assert best >= 2 * 4 * B * T * 256 * H if several else best == 0
+
+
 def test_prefill_kernel_keeps_its_hand_numbered_registers():
   """The prefill kernel's gate weights sit in accumulation registers that the
   source numbers itself; the compiled kernels may touch those registers only
