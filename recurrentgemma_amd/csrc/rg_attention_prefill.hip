@@ -114,7 +114,8 @@ constexpr float kNoMaximum = -3.0e38f;
 // ROPE: the queries come before their rotary embedding and take it here, in
 // the registers they are loaded to (p.rope_table); a pass of its own over them
 // reads and writes every query once more (8 x 2047 tokens, 10 heads: 43 us).
-// COLUMNS: the values come transposed, [row, 256, T_pad], else key by key.
+// COLUMNS: the values come transposed, [row, 256, T_pad], else key by key.  Launched as
+// rotated and key by key, or as neither.
 // QB: blocks of 16 queries per wave.
 template <bool ROPE, bool COLUMNS, int QB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
@@ -739,10 +740,9 @@ hipError_t launch_prefill(const AttnPrefillArgs& a, hipStream_t s) {
 namespace {
 template <int QB>
 hipError_t launch_queries(const AttnPrefillArgs& a, hipStream_t s) {
-  if (a.T_pad == 0)
-    return a.rope_table ? launch_prefill<true, false, QB>(a, s)
-                        : launch_prefill<false, false, QB>(a, s);
-  return launch_prefill<false, true, QB>(a, s);
+  if (a.T_pad > 0) return launch_prefill<false, true, QB>(a, s);
+  if (!a.rope_table) return hipErrorInvalidValue;
+  return launch_prefill<true, false, QB>(a, s);
 }
 // 32 queries a wave up to two rounds of the chip of them: half as many workgroups again,
 // each with two thirds of the work (us with 48 / 32, 10 heads: 1 x 300 tokens 28 / 22,
@@ -756,7 +756,8 @@ bool short_tiles(const AttnPrefillArgs& a) {
 
 hipError_t launch_attn_prefill_bf16(const AttnPrefillArgs& a, hipStream_t s) {
   // needs head dimension 256 and rows whose byte offsets fit 32 bits (checked by the
-  // caller); values in columns T_pad (a multiple of 64) long, or key by key (T_pad 0)
+  // caller); values in columns T_pad (a multiple of 64) long, or key by key (T_pad 0):
+  // then the queries take their rotary embedding here
   return short_tiles(a) ? launch_queries<2>(a, s) : launch_queries<3>(a, s);
 }
 

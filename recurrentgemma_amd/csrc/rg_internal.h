@@ -264,7 +264,8 @@ struct MatmulArgs {
   MatmulProblem p[kMaxMatmuls];
   int count;
 };
-// Whether the launch can be made; and whether it is ahead of the library's products.
+// Whether the launch can be made; and (but for weight gradients) whether it is ahead of
+// the library's products.
 bool matmul_serves(const MatmulArgs& a, int kind);
 bool matmul_pays(const MatmulArgs& a, int kind);
 hipError_t launch_matmul(MatmulArgs a, int kind, hipStream_t s);

@@ -648,22 +648,25 @@ bool matmul_serves(const MatmulArgs& a, int kind) {
   return true;
 }
 
-// Whether a launch is ahead of the library's products, one by one.  Their time: whole
-// rounds of 256 x 256 tiles at 1.3 us a step, or (few tiles) some 1.25 PFLOP/s and the way
-// along the contraction; with the weights [in, out] 1.35 and more beside; and never less
-// than 14 us (a call of the library's takes the host 20, one here 6 to 12).  Measured
-// over 64 to 32768 rows, widths 2560 and 4096 (library / this, us): forward 8192 x 2560 x
-// 2560 93 / 74, two of them 189 / 147, 16376 rows 233 / 149, 2048 rows 33 / 38, two of them
-// 65 / 48, 300 rows 13 (host 21) / 12, three of them 60 / 27, 1000 rows 24 / 25, 8192 x
-// 4096 x 4096 171 / 184 (its 256 x 256 tiles come out even); back 8192 x 2560 x 2560 109 /
-// 74, through two layers 230 / 138, 300 rows 17 / 14, 1500 rows 56 / 57 through two.  Weight
-// gradients, whose contraction fills every tile whatever the rows, and the pair with its
-// join (8192 rows, 2560 -> 7680: 494 + 60 / 481) are ahead at all sizes: three of 2560 x
-// 2560 over 256 rows 60 / 21, 1000 rows 87 / 37, 8192 rows 407 / 211, one of 4096 x 4096
-// over 8192 rows 237 / 181 (one of 2560 x 2560 alone 113 / 114).
+// Whether a launch is ahead of the library's products, one by one (weight gradients: at
+// rg_linear_weight_grads).  Their time: whole rounds of 256 x 256 tiles at 1.3 us a step,
+// or (few tiles) some 1.25 PFLOP/s and the way along the contraction; with the weights
+// [in, out] 1.35 and more beside.  Measured over 64 to 32768 rows, widths 64 to 7680
+// (library / this, us): forward 8192 x 2560 x 2560 93 / 74, two of them 189 / 147, 16376
+// rows 233 / 149, 2048 rows 33 / 38, two of them 65 / 48, 300 rows 13 / 12, three of them
+// 37 / 27, 1000 rows 24 / 25, 8192 x 4096 x 4096 171 / 184 (its 256 x 256 tiles come out
+// even); back 8192 x 2560 x 2560 109 / 74, through two layers 230 / 138, 300 rows 17 / 14,
+// 1500 rows 56 / 57 through two; the pair with its join, 8192 rows, 2560 -> 7680 494 + 60 /
+// 481.
+// Never less than 14 us, which counts the host's time and is right where calls are made
+// one by one: nn.Linear keeps it for 21, a call here for 14 (three layers: 62 / 22), with
+// 70, 300 or 1000 rows alike.  From a graph no host time counts, and a single layer with
+// a long contraction and few tiles is behind there: 70 rows 2560 -> 2560 8.7 / 11.4 (100
+// rows 10.8 / 11.3), 70 to 300 rows 2560 -> 256 7 / 11 and back 8 / 13.5, the pair so 17 /
+// 19; of the other calls of a block 70 rows 2560 -> 2560 twice 17 / 12, thrice 30 / 13, the
+// pair 2560 -> 7680 34 / 20, so that a captured step of more than 64 sequences gains.
 bool matmul_pays(const MatmulArgs& a, int kind) {
   if (!matmul_serves(a, kind)) return false;
-  if (kind == kMatmulWeights) return true;
   int tile;
   const float own = best_tile(a, kind, &tile);
   constexpr float kCall = 14.0f;
