@@ -180,6 +180,48 @@ def test_attention_prompt_equals_its_parts(B, T, H, window, layout,
   assert count.dtype == torch.int32 and torch.equal(count, want.num_tokens)
 
 
+# more than 512 workgroups of 32 queries a wave: 48 queries a wave
+MANY_QUERIES = [(264, 47, 5, 2048, "padded"), (264, 48, 5, 16, "documents"),
+                (264, 49, 5, 2048, "one"), (264, 97, 5, 33, "padded"),
+                (8, 2047, 10, 2048, "padded"), (8, 2047, 10, 700, "documents")]
+
+
+@pytest.mark.parametrize("B,T,H,window,layout", MANY_QUERIES)
+def test_attention_prompt_equals_its_parts_many_rows(B, T, H, window, layout):
+  """The same with 48 queries of a wave."""
+  assert (((T + 31) // 32 * H + 3) // 4) * B > 512
+  test_attention_prompt_equals_its_parts(B, T, H, window, layout, True)
+
+
+@pytest.mark.parametrize("B,T,H,window,layout", MANY_QUERIES)
+def test_attention_prompt_many_rows_against_the_reference(B, T, H, window, layout):
+  """... and against the reference's sequence of operators: rotary embedding as
+  ops.rope_pair has it, the rest in tensor operators, a few rows at a time."""
+  hd = 256
+  g = torch.Generator().manual_seed(B * 1000 + T + 1)
+  q, k, v = (torch.randn(B, T, n, hd, generator=g).bfloat16().cuda()
+             for n in (H, 1, 1))
+  at = torch.arange(T).expand(B, T)
+  seg = at.clone()
+  if layout == "padded":
+    seg = (at - torch.randint(0, T // 2 + 1, (B, 1), generator=g)).clamp(min=-1)
+  elif layout == "documents":
+    starts = torch.rand(B, T, generator=g) < 0.02
+    seg = at - torch.cummax(torch.where(starts, at, 0), dim=1).values
+  seg = seg.to("cuda", torch.int32)
+  inv = griffin._inv_frequencies(hd, "cuda")
+  first = ops.attention_first_key(seg, window)
+  got = ops.attention_prompt(q, k, v, seg, inv, first, window, hd ** -0.5, False)[0]
+  qr, kr = ops.rope_pair(q, k, seg, inv)
+  rows = B if T < 100 else 1
+  for b in range(0, B, rows):
+    r = slice(b, b + rows)
+    want = reference(qr[r], kr[r], v[r], seg[r], window, hd ** -0.5)
+    real = (seg[r] >= 0)[..., None, None]  # (pads see only each other)
+    helpers.assert_close_elementwise(got[r] * real, want * real, rtol=2e-2,
+                                     atol_of_max=2e-2, what=f"rows {b} ..")
+
+
 def test_attention_prefill_refuses_other_shapes():
   q = torch.zeros(1, 8, 2, 128, dtype=torch.bfloat16, device=DEV)
   assert not ops.attention_prefill_supported(q)
