@@ -290,10 +290,12 @@ int rg_recurrent_prefill_split(const void* x, const void* segpos,
  * activation, both [B,T,W]; out feeds linear_out.  rg_recurrent_prefill_split
  * (whole rows or rows in chunks: same workspace rule, workspace may be null
  * when rg_recurrent_prefill_split_workspace_bytes is 0) with the join of the
- * two branches applied where y is stored: same values, bit for bit, as that
- * call followed by rg_gelu_mul(y, gate_branch) (gelu rounded to `dtype` like
- * the tensor it is in the reference, then the product rounded), without the
- * pass over y in between.  out may alias gate_branch (every element is read
+ * two branches applied where y is stored: the values of that call followed by
+ * rg_gelu_mul(y, gate_branch) (gelu rounded to `dtype` like the tensor it is in
+ * the reference, then the product rounded), without the pass over y in between.
+ * The same bits where both run the same form of the kernel; some sizes (256-wide
+ * heads, 8 rows of 200 tokens in 10 heads) run another with the join than
+ * without, which adds up the float32 state in another order.  out may alias gate_branch (every element is read
  * before it is written, by the same lane); neither may alias x.  h_last and
  * conv_cache_out as in rg_recurrent_prefill.  RG_ERR_UNSUPPORTED for the
  * shapes rg_recurrent_prefill refuses: callers then use the separate calls. */

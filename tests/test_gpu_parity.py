@@ -698,6 +698,11 @@ def test_recurrent_block_module_joined_kernel(monkeypatch):
     (3, 1540, 256, 1, 7, torch.int64, False),
     (1, 8192, 256, 1, 1024, torch.int64, True),  # 64 chunks of two tiles
     (2, 1700, 256, 1, -300, torch.int32, False),  # chunks, left padding
+    # ... of 449 to 1000 tokens in more than 32 pairs (fewer: rg_prefill_short.hip)
+    (17, 449, 512, 2, 60, torch.int64, True),
+    (33, 700, 256, 1, -300, torch.int32, False),
+    (12, 1000, 768, 3, 250, torch.int64, False),
+    (100, 150, 512, 2, 30, torch.int32, True),    # whole rows, a workgroup a pair
 ])
 def test_recurrent_prefill_single_launch(B, T, W, H, mean_doc, seg_dtype,
                                          with_h0):
@@ -760,8 +765,10 @@ def test_recurrent_prefill_single_launch(B, T, W, H, mean_doc, seg_dtype,
     (1, 2048, 512, 2, 300),    # rows in chunks
     (3, 1600, 768, 3, None),
     (40, 130, 1024, 4, 50),    # 160 (row, head) pairs
-    (2, 449, 512, 2, 60),      # the shortest rows that are cut into chunks
+    (17, 449, 512, 2, 60),     # the shortest rows that are cut into chunks
+    (2, 449, 512, 2, 60),      # ... and in at most 32 pairs, where they are not
     (1, 513, 256, 1, None),
+    (33, 513, 256, 1, None),
     (1, 4096, 2560, 10, 1024), # chunks at the 2B width
     (5, 3000, 2560, 10, 5),    # ... ragged, documents of a few tokens
     (6, 1500, 768, 3, 300),
@@ -870,14 +877,18 @@ def test_recurrent_step_single_launch(B, W, H, in_place):
 
 @pytest.mark.parametrize("B,T,W,H,mean_doc,with_h0", [
     (3, 150, 512, 2, 40, False), (2, 1000, 768, 3, 100, True),
-    (1, 31, 256, 1, 5, False), (2, 4096, 1024, 4, 500, True)])
+    (1, 31, 256, 1, 5, False), (2, 4096, 1024, 4, 500, True),
+    # whole rows, a workgroup a pair: two kernels
+    (100, 150, 512, 2, 40, False), (60, 201, 768, 3, 100, True),
+    (33, 1000, 768, 3, 300, True)])
 def test_recurrent_prefill_without_packed_weights(B, T, W, H, mean_doc, with_h0):
   """rg_recurrent_prefill with w_packed == NULL re-lays the gate weights out
   inside the kernel: same result, bit for bit, as with the packed buffer.
 
-  The two calls also run two different kernels -- with packed weights whole
-  rows go to the form with two waves per SIMD, without them to the form with
-  one -- so this is the check that the two forms compute the same thing."""
+  Where a workgroup takes a whole row the two calls also run two different
+  kernels -- with packed weights the form with two waves per SIMD, without them
+  the form with one -- so this is the check that the two forms compute the same
+  thing (few pairs run one kernel of slices or of short rows either way)."""
   p = R.make_params(W, H, torch.bfloat16, seed=61, gate_bias_std=0.5)
   P = {k: _dev(v) for k, v in p.items()}
   g = torch.Generator().manual_seed(62)
@@ -901,7 +912,8 @@ def test_recurrent_prefill_without_packed_weights(B, T, W, H, mean_doc, with_h0)
 
 @pytest.mark.parametrize("B,T,W,H,mean_doc,with_h0", [
     (1, 8192, 2560, 10, 0, False), (4, 4096, 512, 2, 300, True),
-    (2, 3000, 768, 3, 50, True)])
+    (2, 3000, 768, 3, 50, True), (17, 449, 512, 2, 60, True),
+    (12, 768, 768, 3, 0, False), (4, 640, 2560, 10, 100, True)])
 def test_recurrent_prefill_in_chunks_without_packed_weights(B, T, W, H,
                                                             mean_doc, with_h0):
   """Rows cut into chunks (rg_recurrent_prefill_split): with and without the
@@ -935,7 +947,11 @@ def test_recurrent_prefill_in_chunks_without_packed_weights(B, T, W, H,
   assert torch.equal(y1, y2) and torch.equal(h1, h2) and torch.equal(c1, c2)
 
 
-@pytest.mark.parametrize("B,T,W,H", [(3, 150, 512, 2), (1, 2048, 512, 2)])
+@pytest.mark.parametrize("B,T,W,H", [
+    (3, 150, 512, 2), (1, 2048, 512, 2),
+    # whole rows through the forms with one and two waves per SIMD, chunks
+    # through both, slices of rows longer than a pass
+    (100, 150, 512, 2), (17, 500, 512, 2), (4, 200, 2560, 10)])
 def test_recurrent_prefill_joined_without_packed_weights(B, T, W, H):
   """The block's GELU join inside the kernel (rg_recurrent_prefill_gelu_mul),
   whole rows and rows in chunks, through both kernel forms: same bits."""

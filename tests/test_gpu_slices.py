@@ -26,7 +26,11 @@ NAMES = ("conv_w", "conv_b", "w_x", "b_x", "w_a", "b_a", "a_param")
     (2, 70, 136, 2, 20), (2, 70, 168, 3, 20), (3, 150, 184, 2, 50),
     (3, 150, 200, 1, 50), (2, 70, 248, 3, 20),
     # long rows, left padding
-    (2, 700, 176, 4, -200), (3, 333, 256, 10, 80)])
+    (2, 700, 176, 4, -200), (3, 333, 256, 10, 80),
+    # 256-wide heads, rows longer than a pass: more than 32 pairs (fewer go to
+    # rg_prefill_short.hip)
+    (33, 129, 256, 1, 3), (4, 200, 256, 10, 40), (4, 333, 256, 10, -200),
+    (17, 300, 256, 2, 1000)])
 @pytest.mark.parametrize("joined", [False, True])
 def test_prefill_in_slices(B, T, bw, H, mean_doc, joined):
   W = bw * H
@@ -66,26 +70,39 @@ def test_prefill_in_slices(B, T, bw, H, mean_doc, joined):
 
 
 @pytest.mark.parametrize("B,T,bw,H", [(3, 100, 176, 2), (2, 300, 256, 2),
-                                      (5, 40, 200, 3)])
-def test_slices_without_packed_weights(B, T, bw, H):
-  """w_packed == NULL: the weights fetched from the reference layout, same bits."""
+                                      (5, 40, 200, 3), (4, 200, 256, 10),
+                                      (33, 129, 256, 1), (5, 333, 256, 7),
+                                      (8, 200, 256, 10)])
+@pytest.mark.parametrize("joined", [False, True])
+def test_slices_without_packed_weights(B, T, bw, H, joined):
+  """w_packed == NULL: the weights fetched from the reference layout, same bits
+  (2 rows of 300 tokens in 2 heads of 256: in rg_prefill_short.hip; 80 pairs of 200
+  tokens: in slices only joined)."""
   W = bw * H
   p = R.make_params(W, H, torch.bfloat16, seed=31, gate_bias_std=0.4)
   ws = [p[n].to(DEV) for n in NAMES]
   g = torch.Generator().manual_seed(32)
   x = torch.randn(B, T, W, generator=g).bfloat16().to(DEV)
   seg = helpers.document_positions(B, T, 30, seed=33).to(DEV)
-  y1, h1, c1 = ops.recurrent_core(x, seg, *ws)
+  gate = torch.randn(B, T, W, generator=g).bfloat16().to(DEV) if joined else None
+  y1, h1, c1 = ops.recurrent_core(x, seg, *ws, gate_branch=gate)
   lib = _lib.lib()
   assert lib.rg_recurrent_core_workspace_bytes(B, T, W, H, 1) == 0
   y2, c2 = torch.empty_like(x), x.new_empty(B, 3, W)
   h2 = torch.empty(B, W, dtype=torch.float32, device=DEV)
   ptr = lambda t: t.data_ptr()
   _lib.check(lib.rg_recurrent_core(
-      ptr(x), None, ptr(seg), 1, *[ptr(t) for t in ws[:6]], None, ptr(ws[6]),
+      ptr(x), ptr(gate) if joined else None, ptr(seg), 1,
+      *[ptr(t) for t in ws[:6]], None, ptr(ws[6]),
       None, ptr(y2), ptr(h2), ptr(c2), None, 0, B, T, W, H, 1,
       torch.cuda.current_stream().cuda_stream))
   assert torch.equal(y1, y2) and torch.equal(h1, h2) and torch.equal(c1, c2)
+  yo, co = R.widened_recurrent_core(x.cpu(), seg.cpu(), p, None)
+  if joined:
+    yo = (yo.float() * torch.nn.functional.gelu(
+        gate.cpu().float(), approximate="tanh").bfloat16().float()).bfloat16()
+  assert helpers.max_rel(y2, yo) < 1e-2
+  assert helpers.max_rel(h2, co.rg_lru_state) < 2e-3
 
 
 def _core(x, seg, ws, h0=None, packed=True):
