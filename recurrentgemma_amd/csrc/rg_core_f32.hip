@@ -37,18 +37,18 @@
 // Replaces the chain Conv1D.forward -> RGLRU.forward of
 // recurrentgemma/torch/modules.py:632-643 (layers.py:447-529, 313-365,
 // 140-191) for such shapes.
-#include <type_traits>
-#include <utility>
-
 #include "rg_common.h"
 #include "rg_internal.h"
+#include "rg_row_tiles.h"
 
 namespace rg {
 namespace {
 
+using namespace row_tiles;
+
 constexpr int kBW = 256;      // head width
 constexpr int kCh = 16;       // output channels per workgroup
-constexpr int kTile = 16;     // tokens per matrix tile
+constexpr int kSlices = kBW / kCh;
 constexpr int kSeg = 512;     // tokens per segment
 constexpr int kWaves = 8;     // two per SIMD
 constexpr int kThreads = kWaves * 64;
@@ -150,20 +150,6 @@ __device__ __forceinline__ void cut_rows(float a, float b, uint32_t (&piece)[3])
 // From here on the pieces of a value hold all of it: the last of its 24 bits is worth
 // 2^-133, the least that a bf16 has.  (Below 2^-134, 5e-41, they are zeros.)
 constexpr float kExactOwn = 0x1p-110f;
-// A lane's number that nothing is worked out from ahead of a loop: what is worked out
-// from it is worked out again where it is used, instead of being kept in registers.
-template <class V>
-__device__ __forceinline__ V fresh(V lane) {
-  asm volatile("" : "+v"(lane));
-  return lane;
-}
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
 
 // GELU: y is written as y * gelu(gate_branch), the join of the recurrent
 // block's two branches (recurrentgemma/torch/modules.py:627-628, 644).
@@ -175,17 +161,9 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // 16 workgroups per (row, head).  Workgroups go to the eight XCDs in turn
-  // (linear id modulo 8), each with an L2 of its own: the 16 workgroups of a
-  // pair are dealt to ONE of them, so that the head's rows and weights, which
-  // all 16 read, come through one L2 (pair p runs on XCD p % 8; the grid is
-  // rounded up to whole rounds of eight pairs and the surplus exits).
-  constexpr int slices = kBW / kCh;
-  const int xcd = blockIdx.x & 7;
-  const int in_xcd = blockIdx.x >> 3;
-  const int pair = (in_xcd / slices) * 8 + xcd;
+  const Slice own_slice = slice_of_workgroup<kSlices>();
+  const int pair = own_slice.pair, s = own_slice.s;
   if (pair >= p.B * p.H) return;
-  const int s = in_xcd % slices;
   const int h = pair % p.H;
   const int b = pair / p.H;
   const int T = p.T;
@@ -288,7 +266,7 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
     // Rows 4 g - 3 .. 4 g + 3 of a tile.  The rows of a pass are requested when the
     // pass before it has consumed its own, and arrive while it multiplies.
     f32x4 xr[7];
-    uint32_t seg_lo = 1, seg_hi = 0;
+    Positions positions;
     auto request_rows = [&](int t0, int pass) __attribute__((always_inline)) {
       const uint32_t at = lane_at + (uint32_t)t0 * row_bytes + 4u * kPass * pass;
 #pragma unroll
@@ -296,18 +274,8 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
         xr[r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                                               rx, at + r * row_bytes, 0, 0));
     };
-    // positions of rows t0-2 .. t0+15 (lane j looks at row t0 - 2 + j)
-    auto request_positions = [&](int t0) __attribute__((always_inline)) {
-      const int t = t0 - 2 + lane;
-      const bool in = lane < kTile + 2 && t >= 0 && t < T;
-      const uint32_t off = in ? (uint32_t)t * seg_esize : kBufferOutOfRange;
-      seg_lo = __builtin_amdgcn_raw_buffer_load_b32(rseg, off, 0, 0);
-      seg_hi = __builtin_amdgcn_raw_buffer_load_b32(
-          rseg, seg_is64 ? off + 4u : kBufferOutOfRange, 0, 0);
-    };
-    // The conv of a pass's 64 channels: put(r, four channels of row 4 g + r).  Tap k
-    // of a row reads the row k before it, which counts only if no document starts in
-    // between or at the row itself (bit j of `starts` is row j - 2 of the tile).
+    // The conv of a pass's 64 channels: put(r, four channels of row 4 g + r) (bit j of
+    // `starts` is row j - 2 of the tile).
     auto convolve = [&](int pass, uint32_t starts, auto&& put)
         __attribute__((always_inline)) {
       asm volatile("" : "+s"(starts));  // (the cuts below are made where they are used)
@@ -331,16 +299,13 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
       } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const uint32_t near = (starts >> (4 * g + r)) & 7u;  // rows r-2, r-1, r
-          const bool cut1 = (near & 4u) != 0;          // start at r
-          const bool cut2 = cut1 || (near & 2u) != 0;  // ... or at r-1
-          const bool cut3 = cut2 || (near & 1u) != 0;  // ... or at r-2
+          const Cuts cut = cuts_of_row(starts >> (4 * g), r);
           f32x4 o;
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            o[e] = has_conv ? conv4(xr[r + 3][e], cut1 ? 0.0f : xr[r + 2][e],
-                                    cut2 ? 0.0f : xr[r + 1][e],
-                                    cut3 ? 0.0f : xr[r][e], cw[0][e], cw[1][e],
+            o[e] = has_conv ? conv4(xr[r + 3][e], cut.one ? 0.0f : xr[r + 2][e],
+                                    cut.two ? 0.0f : xr[r + 1][e],
+                                    cut.three ? 0.0f : xr[r][e], cw[0][e], cw[1][e],
                                     cw[2][e], cw[3][e], cw[4][e])
                             : xr[r + 3][e];
           put(r, o);
@@ -350,20 +315,13 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
     const int first = seg * kSeg + wave * kTile;
     const int end = min(T, (seg + 1) * kSeg);
     if (first < end) {
-      request_positions(first);
+      positions.request(rseg, seg_is64, first, lane, T);
       request_rows(first, 0);
     }
 #pragma unroll 1
     for (int t0 = first; t0 < end; t0 += kWaves * kTile) {
       const int next_t0 = t0 + kWaves * kTile;
-      // document starts among rows t0-2 .. t0+15 (rows before the sequence or
-      // past its end: no start)
-      uint32_t starts;
-      {
-        const int t = t0 - 2 + lane;
-        const bool in = lane < kTile + 2 && t >= 0 && t < T;
-        starts = (uint32_t)__ballot(in && (seg_lo | seg_hi) == 0u);
-      }
+      const uint32_t starts = positions.starts(t0, lane, T);
       // both gates' pre-activations of tokens t0 .. t0+15, channels c0 .. +15:
       // lane (g, n) ends up with channel n of tokens 4 g .. 4 g + 3; the products of
       // the first pieces in one accumulator, the five smaller ones in another
@@ -389,7 +347,7 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
           request_rows(t0, pass + 1);
         } else if (next_t0 < end) {
           request_rows(next_t0, 0);
-          request_positions(next_t0);
+          positions.request(rseg, seg_is64, next_t0, lane, T);
         }
         __builtin_amdgcn_wave_barrier();
         // the conv output of the workgroup's own channels, which the gate arithmetic
@@ -555,31 +513,7 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
         lds.chunk_h[chunk][ch] = hh;
       }
       __syncthreads();
-      // The state every chunk starts from: a scan over the 32 chunk summaries
-      // with the operator of recurrentgemma/jax/scan.py:161-187, by lane
-      // shifts inside a wave (lane = 2 chunk + channel; a wave takes 2 of the
-      // 16 channels), left where the chunk's own summary was.
-      {
-        const int sc = lane >> 1;               // chunk
-        const int sch = 2 * wave + (lane & 1);  // channel
-        float sp = lds.chunk_p[sc][sch], sh = lds.chunk_h[sc][sch];
-#pragma unroll
-        for (int d = 1; d < kChunks; d *= 2) {
-          const float pp = __shfl_up(sp, 2 * d, 64);
-          const float hp = __shfl_up(sh, 2 * d, 64);
-          if (sc >= d) {
-            sh = __builtin_fmaf(sp, hp, sh);
-            sp *= pp;
-          }
-        }
-        // (sp, sh): chunks 0 .. sc from a zero state; the state after chunk sc
-        // is sp * carry + sh, and chunk sc starts from its neighbour's
-        const float carry = lds.carry[sch];
-        const float after = __builtin_fmaf(sp, carry, sh);
-        const float before = __shfl_up(after, 2, 64);
-        lds.chunk_h[sc][sch] = sc == 0 ? carry : before;
-        if (sc == kChunks - 1) lds.carry[sch] = after;
-      }
+      chunk_starts(lds.chunk_p, lds.chunk_h, lds.carry, wave, lane);
       __syncthreads();
       float hin = lds.chunk_h[chunk][ch];
       const int64_t y_at = ((int64_t)b * T + seg * kSeg + i0) * W + c0 + ch;
@@ -605,22 +539,7 @@ __global__ void __launch_bounds__(kThreads) core_f32_small_kernel(FusedArgs p) {
 
   if (p.h_last && tid < kCh) p.h_last[(int64_t)b * W + c0 + tid] = lds.carry[tid];
 
-  // Masked conv state: rows T-3..T-1 of x, each zeroed if a document starts in
-  // a later position of the row; rows before the sequence start are zero.
-  if (p.cache_out && tid < kCh) {
-    float* cache = (float*)p.cache_out + (int64_t)b * 3 * W + c0 + tid;
-    bool later_start = false;
-#pragma unroll
-    for (int kk = 2; kk >= 0; --kk) {
-      const int t = T - 3 + kk;
-      float v = 0.0f;
-      if (t >= 0 && !later_start)
-        v = ((const float*)p.x)[((int64_t)b * T + t) * W + c0 + tid];
-      cache[(int64_t)kk * W] = v;
-      if (t >= 0 && is_doc_start(p.segpos, p.seg_kind, (int64_t)b * T + t))
-        later_start = true;
-    }
-  }
+  if (p.cache_out && tid < kCh) leave_conv_state<float>(p, b, c0 + tid);
 }
 
 }  // namespace
@@ -646,8 +565,7 @@ static hipError_t launch_core_f32_small_as(const FusedArgs& a, dim3 grid,
 }
 
 hipError_t launch_core_f32_small(const FusedArgs& a, hipStream_t s) {
-  const int rounds = (a.B * a.H + 7) / 8;
-  const dim3 grid((unsigned)(rounds * 8 * (kBW / kCh)));
+  const dim3 grid = slices_grid((int64_t)a.B * a.H, kSlices);
   if (a.conv_w)
     return a.gate_branch ? launch_core_f32_small_as<true, true>(a, grid, s)
                          : launch_core_f32_small_as<true, false>(a, grid, s);

@@ -25,18 +25,18 @@
 // Replaces the chain Conv1D.forward -> RGLRU.forward of
 // recurrentgemma/torch/modules.py:632-643 (layers.py:447-529, 313-365,
 // 140-191) for such shapes.
-#include <type_traits>
-
 #include "rg_common.h"
 #include "rg_internal.h"
+#include "rg_row_tiles.h"
 
 namespace rg {
 namespace {
 
+using namespace row_tiles;
+
 constexpr int kBW = 256;    // head width
 constexpr int kCh = 32;     // output channels per workgroup
 constexpr int kSlices = kBW / kCh;
-constexpr int kTile = 16;   // tokens per matrix tile
 constexpr int kWaves = 8;   // two per SIMD
 constexpr int kThreads = kWaves * 64;
 constexpr int kTurns = 3;   // of kWaves tiles in a segment
@@ -109,21 +109,6 @@ __device__ __forceinline__ void mfma_last(u32x4 a, const u32x4 (&w)[4], f32x4 (&
       : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])
       : "v"(a), "a"(w[0]), "a"(w[1]), "a"(w[2]), "a"(w[3]));
 }
-// A value that nothing is worked out from ahead of a loop: what is worked out from it is
-// worked out again where it is used, instead of being kept in registers.
-template <class V>
-__device__ __forceinline__ V fresh(V v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
-#define RG_INLINE __attribute__((always_inline))
 
 // GELU: y leaves as y * gelu(gate_branch), the join of the recurrent block's two
 // branches (recurrentgemma/torch/modules.py:627-628, 644).  PACKED: gate weights in
@@ -137,14 +122,9 @@ block_prefill_short_bf16_kernel(FusedArgs p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Workgroups go to the eight XCDs in turn: the eight of a pair, which read the same
-  // rows and one head's weights, are dealt to one XCD (the grid is rounded up to whole
-  // rounds of eight pairs, the surplus exits).
-  const int xcd = blockIdx.x & 7;
-  const int in_xcd = blockIdx.x >> 3;
-  const int pair = (in_xcd / kSlices) * 8 + xcd;
+  const Slice own_slice = slice_of_workgroup<kSlices>();
+  const int pair = own_slice.pair, s = own_slice.s;
   if (pair >= p.B * p.H) return;
-  const int s = in_xcd % kSlices;
   const int h = pair % p.H;
   const int b = pair / p.H;
   const int T = p.T;
@@ -246,26 +226,15 @@ block_prefill_short_bf16_kernel(FusedArgs p) {
     // Rows 4 g - 3 .. 4 g + 3 of a tile.  The rows of a pass are requested when the
     // pass before it has consumed its own, and arrive while it multiplies.
     u32x4 xr[7];
-    uint32_t seg_lo = 1, seg_hi = 0;
+    Positions positions;
     auto request_rows = [&](int t0, int pass) RG_INLINE {
       const uint32_t at = lane_at + (uint32_t)t0 * row_bytes + 2u * kPass * pass;
 #pragma unroll
       for (int r = HAS_CONV ? 0 : 3; r < 7; ++r)
         xr[r] = __builtin_amdgcn_raw_buffer_load_b128(rx, at + r * row_bytes, 0, 0);
     };
-    // positions of rows t0-2 .. t0+15 (lane j looks at row t0 - 2 + j)
-    auto request_positions = [&](int t0) RG_INLINE {
-      const int t = t0 - 2 + lane;
-      const bool in = lane < kTile + 2 && t >= 0 && t < T;
-      const uint32_t off = in ? (uint32_t)t * seg_esize : kBufferOutOfRange;
-      seg_lo = __builtin_amdgcn_raw_buffer_load_b32(rseg, off, 0, 0);
-      seg_hi = __builtin_amdgcn_raw_buffer_load_b32(
-          rseg, seg_is64 ? off + 4u : kBufferOutOfRange, 0, 0);
-    };
     // The conv of a pass's 128 channels into the stage, a channel pair of the lane's
-    // four rows at a time.  Tap k of a row reads the row k before it, which counts only
-    // if no document starts in between or at the row itself (bit j of `starts` is row
-    // j - 2 of the tile).
+    // four rows at a time (bit j of `starts` is row j - 2 of the tile).
     auto convolve = [&](int pass, uint32_t starts) RG_INLINE {
       asm volatile("" : "+s"(starts));  // (the cuts below are made where they are used)
       // (in place: the outputs of rows 0 .. 3 take the registers of these rows)
@@ -307,12 +276,11 @@ block_prefill_short_bf16_kernel(FusedArgs p) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               // rows r, r - 1, r - 2, r - 3 without what a start cuts off
-              const bool cut1 = (near >> (r + 2)) & 1u;
-              const bool cut2 = cut1 || ((near >> (r + 1)) & 1u);
-              const bool cut3 = cut2 || ((near >> r) & 1u);
+              const Cuts cut = cuts_of_row(near, r);
               uint32_t p_old[2], p_new[2];
-              pair_up(cut1 ? 0u : xr[r + 2][i], xr[r + 3][i], p_new[0], p_new[1]);
-              pair_up(cut3 ? 0u : xr[r][i], cut2 ? 0u : xr[r + 1][i], p_old[0], p_old[1]);
+              pair_up(cut.one ? 0u : xr[r + 2][i], xr[r + 3][i], p_new[0], p_new[1]);
+              pair_up(cut.three ? 0u : xr[r][i], cut.two ? 0u : xr[r + 1][i], p_old[0],
+                      p_old[1]);
               conv4_dot_x2(p_old, p_new, w10, w32, bias, o[r]);
             }
           });
@@ -326,20 +294,13 @@ block_prefill_short_bf16_kernel(FusedArgs p) {
     const int first = seg * kSeg + wave * kTile;
     const int end = min(T, (seg + 1) * kSeg);
     if (first < end) {
-      request_positions(first);
+      positions.request(rseg, seg_is64, first, lane, T);
       request_rows(first, 0);
     }
 #pragma unroll 1
     for (int t0 = first; t0 < end; t0 += kWaves * kTile) {
       const int next_t0 = t0 + kWaves * kTile;
-      // document starts among rows t0-2 .. t0+15 (rows before the sequence or
-      // past its end: no start)
-      uint32_t starts;
-      {
-        const int t = t0 - 2 + lane;
-        const bool in = lane < kTile + 2 && t >= 0 && t < T;
-        starts = (uint32_t)__ballot(in && (seg_lo | seg_hi) == 0u);
-      }
+      const uint32_t starts = positions.starts(t0, lane, T);
       // pre-activations of tokens t0 .. t0+15: lane (g, n) ends up with channels n and
       // 16 + n of tokens 4 g .. 4 g + 3
       f32x4 acc[4];
@@ -356,7 +317,7 @@ block_prefill_short_bf16_kernel(FusedArgs p) {
           request_rows(t0, 1);
         } else if (next_t0 < end) {
           request_rows(next_t0, 0);
-          request_positions(next_t0);
+          positions.request(rseg, seg_is64, next_t0, lane, T);
         }
         __builtin_amdgcn_wave_barrier();
         if (pass == (s >> 2)) {
@@ -469,31 +430,7 @@ block_prefill_short_bf16_kernel(FusedArgs p) {
         lds.chunk_h[chunk][ch] = hh;
       }
       __syncthreads();
-      // The state every chunk starts from: a scan over the 16 chunk summaries
-      // with the operator of recurrentgemma/jax/scan.py:161-187, by lane
-      // shifts inside a wave (lane = 4 chunk + channel; a wave takes 4 of the
-      // 32 channels), left where the chunk's own summary was.
-      {
-        const int sc = lane >> 2;               // chunk
-        const int sch = 4 * wave + (lane & 3);  // channel
-        float sp = lds.chunk_p[sc][sch], sh = lds.chunk_h[sc][sch];
-#pragma unroll
-        for (int d = 1; d < kChunks; d *= 2) {
-          const float pp = __shfl_up(sp, 4 * d, 64);
-          const float hp = __shfl_up(sh, 4 * d, 64);
-          if (sc >= d) {
-            sh = __builtin_fmaf(sp, hp, sh);
-            sp *= pp;
-          }
-        }
-        // (sp, sh): chunks 0 .. sc from a zero state; the state after chunk sc
-        // is sp * carry + sh, and chunk sc starts from its neighbour's
-        const float carry = lds.carry[sch];
-        const float after = __builtin_fmaf(sp, carry, sh);
-        const float before = __shfl_up(after, 4, 64);
-        lds.chunk_h[sc][sch] = sc == 0 ? carry : before;
-        if (sc == kChunks - 1) lds.carry[sch] = after;
-      }
+      chunk_starts(lds.chunk_p, lds.chunk_h, lds.carry, wave, lane);
       __syncthreads();
       // replay, a token's state where its a was; then eight channels of a token a
       // thread, out with 16 bytes
@@ -527,22 +464,7 @@ block_prefill_short_bf16_kernel(FusedArgs p) {
 
   if (p.h_last && tid < kCh) p.h_last[(int64_t)b * W + c0 + tid] = lds.carry[tid];
 
-  // Masked conv state: rows T-3..T-1 of x, each zeroed if a document starts in
-  // a later position of the row; rows before the sequence start are zero.
-  if (p.cache_out && tid < kCh) {
-    uint16_t* cache = (uint16_t*)p.cache_out + (int64_t)b * 3 * W + c0 + tid;
-    bool later_start = false;
-#pragma unroll
-    for (int kk = 2; kk >= 0; --kk) {
-      const int t = T - 3 + kk;
-      uint16_t v = 0;
-      if (t >= 0 && !later_start)
-        v = ((const uint16_t*)p.x)[((int64_t)b * T + t) * W + c0 + tid];
-      cache[(int64_t)kk * W] = v;
-      if (t >= 0 && is_doc_start(p.segpos, p.seg_kind, (int64_t)b * T + t))
-        later_start = true;
-    }
-  }
+  if (p.cache_out && tid < kCh) leave_conv_state<uint16_t>(p, b, c0 + tid);
 }
 
 template <bool HAS_CONV, bool PACKED, bool GELU>
@@ -579,11 +501,11 @@ bool prefill_short_serves(int B, int H, int T) {
 }
 
 hipError_t launch_block_prefill_short_bf16(const FusedArgs& a, hipStream_t s) {
-  const int64_t rounds = ((int64_t)a.B * a.H + 7) / 8;
-  if (a.W / a.H != kBW || rounds <= 0 || rounds * 8 * kSlices > 0x7fffffff ||
+  const int64_t pairs = (int64_t)a.B * a.H;
+  if (a.W / a.H != kBW || pairs <= 0 || (pairs + 7) * kSlices > 0x7fffffff ||
       (int64_t)a.T * a.W * 2 >= (int64_t)0x7fffffff)
     return hipErrorInvalidValue;
-  const dim3 grid((unsigned)(rounds * 8 * kSlices));
+  const dim3 grid = slices_grid(pairs, kSlices);
   if (a.conv_w)
     return a.w_packed ? launch_with<true, true>(a, grid, s)
                       : launch_with<true, false>(a, grid, s);
