@@ -327,7 +327,8 @@ def run_attention(args, torch, ops, wl):
                  "query_heads": H, "kv_heads": 1, "head_dim": hd,
                  "window": window,
                  "path": "rg_attention_prefill (+ the transposed copy of v)"},
-      "roofline": {"kernel": "attn_prefill_bf16_kernel", "bound": "mfma",
+      "roofline": {"kernel": "attn_prefill_bf16_kernel (avg_launch_ms covers "
+                             "the copy as well)", "bound": "mfma",
                    "achieved": achieved, "peak": 2500.0, "unit": "TFLOP/s",
                    "frac": achieved / 2500.0, "traffic": None,
                    "algorithmic_flops": flops, "avg_launch_ms": ms},
@@ -337,8 +338,8 @@ def run_attention(args, torch, ops, wl):
 def run_training(args, torch, rg, ops, wl):
   """RecurrentBlock.forward and the backward pass through it inside
   training.differentiable(): conv, gate projections (bf16), RG-LRU gating and
-  recurrence on kernels in both directions, the block's three linear layers
-  as torch autograd.  A step = forward + loss + backward.  The backward
+  recurrence and the block's three linear layers on kernels in both
+  directions.  A step = forward + loss + backward.  The backward
   kernels of the recurrent path are then timed alone on the same shapes."""
   from recurrentgemma_amd import training
   dev = torch.device("cuda:0")

@@ -981,9 +981,9 @@ void prefill_chunk_plan(int B, int H, int T, int* chunks, int* tiles_per_chunk) 
   // (measured at W2560 H10 with the two-wave kernel, us, chunks / whole rows:
   // T384 10-120 pairs even; T512 10 pairs 35/43, 80 pairs 45/49, 120 pairs
   // 54/51; T768 10 pairs 37/61, 120 pairs 69/73; T1024 10 pairs 38/78, 120
-  // pairs 89/92; T4096 10 pairs 58/288, 80 pairs 231/298, 120 pairs 307/314; up to 1000 tokens in at most 32
-  // pairs the plan only sizes the workspace that callers bring: rg_prefill_short.hip
-  // runs there)
+  // pairs 89/92; T4096 10 pairs 58/288, 80 pairs 231/298, 120 pairs 307/314; up to
+  // 1000 tokens in at most 32 pairs the plan only sizes the workspace that callers
+  // bring, as it always did: rg_prefill_short.hip runs there)
   if (groups > 128 || ntiles < 8 || (ntiles < 12 && groups > 96)) return;
   int want = (int)(256 / groups) + 1;  // workgroups per launch and row, + 1
   if (want > ntiles / 2) want = ntiles / 2;

@@ -495,7 +495,11 @@ hipError_t launch_with(const FusedArgs& a, dim3 grid, hipStream_t s) {
 // 36 / 30 (42 / 32), T900 44 / 38 (54 / 42), T1024 37 / 39 (43 / 42), T1536 39 / 56
 // (46 / 61), B3 T333 20 / 18 (22 / 19), T512 36 / 25 (43 / 27), T1024 42 / 41 (48 / 44);
 // W4096 B2 T512 35 / 24 (41 / 26); two rounds: W4096 B3 T333 21 / 32 (23 / 34), T512
-// 35 / 44 (43 / 49), T768 40 / 56 (47 / 62).
+// 35 / 44 (43 / 49), T768 40 / 56 (47 / 62).  One line with the join and without, so that a
+// joined call has the plain one's bits: 961 to 1000 tokens are 37 / 38.5 (44 / 42).  Weights
+// as the reference lays them out cost 1.3 here and much more in the other forms, W2560 B1
+// T129 28 / 14 (29 / 15), T333 33 / 19 (35 / 20), T512 65 / 26 (73 / 28), T1000 69 / 41 (81 /
+// 46), 1 to 32 heads alike: the line is the packed weights'.
 bool prefill_short_serves(int B, int H, int T) {
   return (int64_t)B * H * kSlices <= 256 && T > 128 && T <= 1000;
 }
