@@ -69,10 +69,12 @@ __device__ __forceinline__ u32x4 scalar_rsrc(const void* base, int64_t bytes) {
 }
 
 // 16 bytes a lane, lane after lane, to LDS bytes to + OFFSET ..: of `rsrc` at byte
-// v + at.  M0, which says where to, is read one wait state behind its write at the
-// earliest: the compiler, which writes M0 for the builtin, puts an instruction between,
-// and the build fails where one of these has none (check_mfma_wait.py).  (Nothing else
-// in the kernels that use these reads M0.)
+// v + at.  What lies behind the descriptor's end is zero, also where the scalar offset
+// alone does (tried with scalar offsets of 0 to 128 times the descriptor's size, in a
+// buffer that held them all).  M0, which says where to, is read one wait state behind its
+// write at the earliest: the compiler, which writes M0 for the builtin, puts an instruction
+// between, and the build fails where one of these has none (check_mfma_wait.py).  (Nothing
+// else in the kernels that use these reads M0.)
 template <int OFFSET>
 __device__ __forceinline__ void load_lds_16(uint32_t to, uint32_t v, u32x4 rsrc, int at) {
   asm volatile(
