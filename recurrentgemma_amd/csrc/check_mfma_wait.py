@@ -12,11 +12,13 @@ instruction touches a matrix instruction's destination registers within
 WINDOW instructions of it without such a wait in between -- which is what a
 register copy that the compiler decided to insert there would look like.
 
-Nor does it count wait states in front of a load in such a statement.  Reported
-too are a load to LDS right behind the write of M0, which says where to (one
-wait state: the compiler puts an instruction there for its own), and a memory
-instruction that reads a scalar register within five wait states of the vector
-instruction that wrote it (a descriptor made with v_readfirstlane).
+Nor does it count wait states in front of such a statement.  Reported too are a
+load to LDS right behind the write of M0, which says where to (one wait state:
+the compiler puts an instruction there for its own), a memory instruction that
+reads a scalar register within five wait states of the vector instruction that
+wrote it (a descriptor made with v_readfirstlane), and a matrix instruction that
+reads a register within two wait states of the vector instruction that wrote it
+(an accumulator's zeros, a packed operand).
 
 usage: check_mfma_wait.py file.s
 """
@@ -27,6 +29,7 @@ WINDOW = 20  # instructions; 16 passes need at most 18 wait states
 REG = re.compile(r'\b([va])(?:(\d+)\b|\[([^\]]+)\])')
 SCALAR_REG = re.compile(r'\b(s)(?:(\d+)\b|\[([^\]]+)\])')
 SCALAR_WINDOW = 5  # wait states from a vector write to a memory read
+OPERAND_WINDOW = 2  # wait states from a vector write to a matrix instruction's read
 MEMORY = ('buffer_', 'global_', 'flat_', 'scratch_')
 
 
@@ -50,9 +53,10 @@ def registers(text, kinds=REG):
   return out
 
 
-def early_loads(path):
-  """How many loads come too soon behind what they read (see above)."""
-  written = []  # [scalar registers, wait states left]
+def too_soon(path):
+  """How many loads and matrix instructions come too soon behind what they read
+  (see above)."""
+  written = []  # [registers, wait states left]
   m0 = False    # the last instruction wrote it
   bad = 0
   for number, line in enumerate(open(path), 1):
@@ -72,17 +76,28 @@ def early_loads(path):
         print(f'{path}:{number}: `{text}` reads a scalar register written by a '
               f'vector instruction fewer than {SCALAR_WINDOW} wait states before')
         bad += 1
-    first = operands.split(',')[0].strip()
+    # (operands are apart at commas outside a[..])
+    parts = [p.strip() for p in re.split(r',(?![^\[]*\])', operands)]
+    first = parts[0]
+    if op.startswith('v_mfma'):
+      used = registers(', '.join(parts[1:4]))
+      if any(d & used for d, _ in written):
+        print(f'{path}:{number}: `{text}` reads a register written by a vector '
+              f'instruction fewer than {OPERAND_WINDOW} wait states before')
+        bad += 1
     m0 = first == 'm0'
     written = [[d, n - waits] for d, n in written if n > waits]
     if op.startswith('v_') and first.startswith('s'):
       written.append([registers(first, SCALAR_REG), SCALAR_WINDOW])
+    elif op.startswith('v_') and not op.startswith('v_mfma'):
+      both = ', '.join(parts[:2]) if 'swap' in op else first
+      written.append([registers(both), OPERAND_WINDOW])
   return bad
 
 
 def main(path):
   pending = []  # [destination registers, instructions left]
-  bad = early_loads(path)
+  bad = too_soon(path)
   for number, line in enumerate(open(path), 1):
     text = line.split(';')[0].strip()
     if not text or text.startswith('.') or text.endswith(':'):

@@ -351,15 +351,18 @@ def test_build_check_for_early_reads_of_matrix_results(tmp_path):
     assert rc == want, name
 
 
-def test_build_check_for_early_loads(tmp_path):
-  """check_mfma_wait.py: a load to LDS right behind the write of M0, and a memory
+def test_build_check_for_what_comes_too_soon(tmp_path):
+  """check_mfma_wait.py: a load to LDS right behind the write of M0, a memory
   instruction close behind the vector instruction that wrote a scalar register it
-  reads, are reported; with the wait states in between they are not."""
+  reads, and a matrix instruction close behind the one that wrote an operand, are
+  reported; with the wait states in between they are not."""
   import subprocess
   import sys
   script = os.path.join(_lib.CSRC, "check_mfma_wait.py")
   load = "\tbuffer_load_dwordx4 v1, s[4:7], s9 offen lds\n"
   lane = "\tv_readfirstlane_b32 s5, v8\n"
+  mfma = "\tv_mfma_f32_16x16x32_bf16 v[4:7], v[8:11], v[12:15], v[4:7]\n"
+  other = "\ts_add_u32 s0, s0, 1\n"
   cases = {
       "at_once": ("\ts_add_u32 m0, s8, 0x400\n" + load, 1),
       "moved_at_once": ("\ts_mov_b32 m0, s8\n\t;;#ASMEND\n" + load, 1),
@@ -369,6 +372,14 @@ def test_build_check_for_early_loads(tmp_path):
                      "\tbuffer_load_dwordx4 v[0:3], v1, s[4:7], 0 offen\n", 0),
       "descriptor": (lane + "\ts_nop 3\n" + load, 1),
       "descriptor_later": (lane + "\ts_nop 4\n" + load, 0),
+      "accumulator": ("\tv_mov_b32_e32 v7, 0\n" + mfma, 1),
+      "hand_numbered": ("\tv_accvgpr_write_b32 a[2], 0\n\ts_nop 0\n"
+                        "\tv_mfma_f32_16x16x32_bf16 a[0*4:0*4+3], v[8:11], v[12:15], "
+                        "a[0*4:0*4+3]\n", 1),
+      "operand": ("\tv_permlane32_swap_b32_e32 v1, v9\n" + other + mfma, 1),
+      "operand_later": ("\tv_permlane32_swap_b32_e32 v1, v9\n\ts_nop 1\n" + mfma, 0),
+      "two_others": ("\tv_mov_b32_e32 v7, 0\n" + other * 2 + mfma, 0),
+      "not_an_operand": ("\tv_mov_b32_e32 v1, 0\n" + mfma, 0),
       "other_scalar": ("\tv_readfirstlane_b32 s10, v8\n" + load, 0),
   }
   for name, (text, want) in cases.items():
