@@ -18,9 +18,10 @@
 // A product is the six products of pieces that weigh most, what is left out below
 // 2^-22 of it; the products of the first pieces have an accumulator of their own, the
 // others' is 2^-7 times smaller.  Error of y against 64 bits, relative norm, with the
-// float32 matrix instruction / now: 1 x 512 tokens, W2560 2.06e-7 / 2.0e-7, W4096
-// 1.80e-7 / 1.81e-7, 1 x 1000 3.08e-7 / 2.99e-7, 1 x 100 9.5e-8 / 9.3e-8; 24 sets of 200
-// tokens (inputs as large, a twentieth and eight times) 0.96 of it in the mean.  Same conv4() tap
+// float32 matrix instruction / now, mean of 16 sets each (inputs as large, a twentieth and
+// eight times): 1 x 33 tokens, W4096 9.6e-8 / 8.6e-8, 1 x 200 W2560 and W4096 1.28e-7 /
+// 1.22e-7, 1 x 512 1.73e-7 / 1.69e-7, 1 x 1000 2.16e-7 / 2.14e-7; set by set 0.80 to 1.02 of
+// what it was, in the mean 0.91 (33 tokens) to 0.99 (1000).  Same conv4() tap
 // chain as the other float32 kernels, conv state identical; exp2, reciprocal and
 // square root of the gate arithmetic are the hardware's.
 //
