@@ -410,12 +410,17 @@ __device__ __forceinline__ float gelu_fast(float g) {
 // a * gelu_tanh(g) for two bf16 of each operand (modules.py:289-291, :644):
 // gelu is rounded to bf16 like the module output it is in the reference, then
 // the product.
-__device__ __forceinline__ uint32_t gelu_mul_bf16x2(uint32_t a, uint32_t g) {
-  const uint32_t y = pack_bf16x2(gelu_fast(__uint_as_float(g << 16)),
-                                 gelu_fast(__uint_as_float(g & 0xffff0000u)));
+__device__ __forceinline__ uint32_t gelu_bf16x2(uint32_t g) {
+  return pack_bf16x2(gelu_fast(__uint_as_float(g << 16)),
+                     gelu_fast(__uint_as_float(g & 0xffff0000u)));
+}
+__device__ __forceinline__ uint32_t mul_bf16x2(uint32_t a, uint32_t b) {
   return pack_bf16x2(
-      __uint_as_float(a << 16) * __uint_as_float(y << 16),
-      __uint_as_float(a & 0xffff0000u) * __uint_as_float(y & 0xffff0000u));
+      __uint_as_float(a << 16) * __uint_as_float(b << 16),
+      __uint_as_float(a & 0xffff0000u) * __uint_as_float(b & 0xffff0000u));
+}
+__device__ __forceinline__ uint32_t gelu_mul_bf16x2(uint32_t a, uint32_t g) {
+  return mul_bf16x2(a, gelu_bf16x2(g));
 }
 
 // The recurrence gate's exponent sigmoid(v) * decay with e = exp(-v) as

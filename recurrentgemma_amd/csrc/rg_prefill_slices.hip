@@ -57,19 +57,19 @@ typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 typedef __attribute__((address_space(3))) f32x2 lds_f32x2;
 
-// LDS, in bytes: two conv tiles of TILES x 32 tokens, every matrix wave's
+// LDS, in bytes: two conv tiles of four times 32 tokens, every matrix wave's
 // output patch, the tiles' (prod a, state) pairs twice, conv taps, and the
-// biases and inverse decays of the workgroup's CH channels.
-template <int KS, int TILES, int CH>
+// biases and inverse decays of the workgroup's channels.
+template <int KS>
 struct Layout {
   static constexpr int row = (KS * 16 + 8) * 2;
-  static constexpr int buffer = kTile * TILES * row;
+  static constexpr int buffer = kTile * kTiles * row;
   static constexpr int patch = 2 * buffer;
   static constexpr int pairs = patch + kWaves * kPatchBytes;
-  static constexpr int pairs_one = TILES * CH * 8;
+  static constexpr int pairs_one = kTiles * kSlice * 8;
   static constexpr int taps = pairs + 2 * pairs_one;
   static constexpr int gates = taps + 128 * 32;
-  static constexpr int total = gates + CH * 16;
+  static constexpr int total = gates + kSlice * 16;
   static_assert(total <= 160 * 1024, "LDS of one CU");
 };
 
@@ -117,10 +117,10 @@ struct TileAt {
 // From a tile's pre-activations (a lane: 16 tokens of one channel, runs of four
 // that alternate between the lane halves) to its outputs: gates, the tile as
 // (prod a, state from zero), the workgroup's barrier, the fold of the pass's
-// TILES tiles, replay, stores.  CH: channels of the workgroup, c0: this wave's
-// first among them, n0: in the head.  until: how many tiles after the pass's
+// four tiles, replay, stores.  c0: this wave's first channel among the workgroup's,
+// n0: in the head.  until: how many tiles after the pass's
 // first the next row opens (0: that one does), kept up to date here.
-template <class L, int TILES, int CH, bool GELU>
+template <class L, bool GELU>
 __device__ __forceinline__ void gate_and_scan(
     const FusedArgs& p, lds_byte* const lds3, const int lane, const int wave,
     const int bw, const int h, const int n0, const int c0, const int tt,
@@ -245,7 +245,7 @@ __device__ __forceinline__ void gate_and_scan(
       }
       {
         lds_f32x2* const mine = reinterpret_cast<lds_f32x2*>(
-            lds3 + L::pairs + buf * L::pairs_one + (tt * CH + c0) * 8);
+            lds3 + L::pairs + buf * L::pairs_one + (tt * kSlice + c0) * 8);
         if (ln < 32) mine[ln] = f32x2{tp, th};
       }
       lds_barrier();
@@ -254,32 +254,22 @@ __device__ __forceinline__ void gate_and_scan(
       {
         const lds_f32x2* const all = reinterpret_cast<const lds_f32x2*>(
             lds3 + L::pairs + buf * L::pairs_one + c0 * 8);
-        f32x2 v[TILES];
+        f32x2 v[kTiles];
 #pragma unroll
-        for (int k = 0; k < TILES; ++k) v[k] = all[k * CH + (ln & 31)];
+        for (int k = 0; k < kTiles; ++k) v[k] = all[k * kSlice + (ln & 31)];
         float s = carry;
-        // (us without the cut: B4 T2048 W5632 129.9, B3 T333 W2560 22.61.  Passes
-        // of two tiles branch past the selections, 129.9 against 131.0; passes of
-        // four, which open a row more often, do them always, 22.64 against 22.72)
-        if (TILES == 2 && __builtin_expect(until >= TILES, 1)) {
+        // rows open in this pass: cut from the row before by selection (a product of
+        // zero would let that row's NaN or infinity through; B3 T333 W2560 without the
+        // cut 22.61 us, with it 22.64)
+        const bool opens = k_in_row == 0;
 #pragma unroll
-          for (int k = 0; k < TILES; ++k) {
-            if (k == tt) hin = s;
-            s = __builtin_fmaf(v[k][0], s, v[k][1]);
-          }
-        } else {
-          // rows open in this pass: cut from the row before by selection (a
-          // product of zero would let that row's NaN or infinity through)
-          const bool opens = k_in_row == 0;
-#pragma unroll
-          for (int k = 0; k < TILES; ++k) {
-            if (k == tt && !opens) hin = s;
-            const float next = __builtin_fmaf(v[k][0], s, v[k][1]);
-            s = k == until ? v[k][1] : next;
-            until += k == until ? tiles_per_row : 0;
-          }
+        for (int k = 0; k < kTiles; ++k) {
+          if (k == tt && !opens) hin = s;
+          const float next = __builtin_fmaf(v[k][0], s, v[k][1]);
+          s = k == until ? v[k][1] : next;
+          until += k == until ? tiles_per_row : 0;
         }
-        until -= TILES;
+        until -= kTiles;
         carry = s;
       }
       if (active) {
@@ -474,7 +464,7 @@ __device__ __forceinline__ void store_conv_state(const FusedArgs& p,
 template <int KS, bool PACKED, bool GELU>
 __global__ void __launch_bounds__(kThreads)
 block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
-  using L = Layout<KS, kTiles, kSlice>;
+  using L = Layout<KS>;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   lds_byte* const lds3 = (lds_byte*)lds_raw;
 
@@ -705,7 +695,7 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
     } else {
       matrix_tile<KS>(lds3, a_lane + buf * L::buffer, acc_x, acc_a, [](auto) RG_INLINE {});
     }
-    gate_and_scan<L, kTiles, kSlice, GELU>(
+    gate_and_scan<L, GELU>(
         p, lds3, lane, wave, bw, h, n0, half * 32, tt, buf, tiles_per_row,
         TileAt{b, t0, k_in_row, any, active, starts}, acc_x, acc_a, carry, until);
     starts = (uint32_t)(mask >> 32);
@@ -718,19 +708,72 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
 }
 
 // Heads of at most 176 channels (the paper presets): two slices of 96, and the
-// waves of a workgroup specialised.  Six of them multiply -- two tiles of 32
-// tokens by three groups of 32 channels -- and two do nothing but the conv of
-// the next pass's two tiles, one of them beside each of the four multiplying
-// waves that share a SIMD in pairs otherwise: 32 heads x 2 slices x 4 rows are
-// exactly one workgroup per CU where slices of 64 are one and a half.
-constexpr int kNarrowKS = 11, kNarrowTiles = 2, kNarrowGroups = 3;
+// waves of a workgroup specialised.  Six of them multiply, two teams of three groups
+// of 32 channels that take the row's tiles of 32 tokens in turn, one phase apart: while
+// one team has its matrix instructions (phase M) the other, on the same SIMDs, has its
+// gates and the recurrence (phase G), as in rg_prefill_teams.hip.  Two do nothing but
+// the conv of the tiles to come, beside the multiplying waves that have a SIMD to
+// themselves otherwise: 32 heads x 2 slices x 4 rows are exactly one workgroup per CU
+// where slices of 64 are one and a half.
+//
+// Phase p: M of tile p, G of tile p - 1; conv of tile p + 2's first 128 channels and of
+// tile p + 1's others.  A workgroup barrier behind every phase; the state goes from
+// tile to tile through LDS, and so the tokens are walked in their order.
+//
+// What bounds it: vector issue on the two SIMDs with two multiplying waves, which is
+// busy all of the time with the join (840 slots a phase, 22 matrix instructions among
+// them, of 1.6 us) and three quarters of it without (1.25 us); the other two have a
+// tenth less.  us, all four multiplying and both converting waves of a tile pair in the
+// same phases, the state by (prod a, state from zero) as in the form above / now, W5632
+// H32: B4 T2048 115 / 88, joined 126 / 109; B16 T2048 433 / 329, joined 476 / 414; B40
+// T300 183 / 144, joined 201 / 173; B64 T33 75 / 66, joined 82 / 73; B16 T100 38 / 34,
+// joined 42 / 38.
+constexpr int kNarrowKS = 11, kNarrowTeams = 2, kNarrowGroups = 3;
 constexpr int kNarrowSlice = 32 * kNarrowGroups;
 constexpr int kNarrowPairs = kNarrowKS * 8;  // channel pairs of a head
+constexpr int kNarrowRing = 4;  // conv tiles: two being made, one in M, one done with
+constexpr int kNarrowRaw = 6;   // tiles of raw rows: four on their way, two being read
+struct NarrowLayout {
+  static constexpr int row = (kNarrowKS * 16 + 8) * 2;
+  static constexpr int tile = kTile * row;
+  static constexpr int patch = kNarrowRing * tile;
+  // (a wave's output patch: 16 tokens x 32 channels; the upper lanes' eight rows
+  // another 64 bytes on, in other banks)
+  static constexpr int patch_upper = 8 * kPatchStride + 64;
+  static constexpr int patch_wave = patch_upper + 8 * kPatchStride;
+  // raw rows, 35 of a tile
+  static constexpr int raw_pieces = kNarrowKS * 2, raw_row = 16 * raw_pieces;
+  static constexpr int raw_loads = ((kTile + 3) * raw_pieces + 63) / 64;
+  static constexpr int raw_tile = raw_loads * 1024;
+  static constexpr int raw = patch + kNarrowTeams * kNarrowGroups * patch_wave;
+  static constexpr int state = raw + kNarrowRaw * raw_tile;
+  static constexpr int taps = state + kNarrowSlice * 4;
+  static constexpr int gates = taps + 128 * 32;
+  static constexpr int total = gates + kNarrowSlice * 16;
+  static_assert(taps % 16 == 0 && total <= 160 * 1024, "LDS of one CU");
+};
+
+// 16 bytes a lane from memory into LDS, 1 KB in a row.
+__device__ __forceinline__ void load_to_lds(const __amdgpu_buffer_rsrc_t from,
+                                            lds_byte* const to, const uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to, 16, off, 0, 0, 0);
+}
+
+// A bf16 value of LDS into the high half of a zeroed register: as a float without a
+// shift.  (The wait for it is the reader's.)
+template <int OFFSET>
+__device__ __forceinline__ uint32_t read_bf16_high(uint32_t at) {
+  uint32_t v;
+  asm volatile("v_mov_b32 %0, 0\n\tds_read_u16_d16_hi %0, %1 offset:%2"
+               : "=&v"(v)
+               : "v"(at), "n"(OFFSET));
+  return v;
+}
 
 template <bool PACKED, bool GELU>
 __global__ void __launch_bounds__(kThreads)
 block_prefill_narrow_bf16_kernel(FusedArgs p, int slices, int groups) {
-  using L = Layout<kNarrowKS, kNarrowTiles, kNarrowSlice>;
+  using L = NarrowLayout;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   lds_byte* const lds3 = (lds_byte*)lds_raw;
 
@@ -747,22 +790,23 @@ block_prefill_narrow_bf16_kernel(FusedArgs p, int slices, int groups) {
   const int row0 = (int)((int64_t)group * p.B / groups);
   const int row1 = (int)((int64_t)(group + 1) * p.B / groups);
   const int T = p.T;
+  const int64_t W = p.W;
   const int tiles_per_row = (T + kTile - 1) / kTile;
   const int ntiles = (row1 - row0) * tiles_per_row;
-  const int npasses = (ntiles + kNarrowTiles - 1) / kNarrowTiles;
   const uint32_t row_bytes = 2u * (uint32_t)p.W;
   const uint32_t seq_bytes = (uint32_t)T * row_bytes;  // < 2^31 (launcher)
   const bool seg_is64 = p.seg_kind == kSegI64;
   const uint32_t seg_esize = seg_is64 ? 8u : 4u;
 
-  const bool convolves = wave >= kNarrowTiles * kNarrowGroups;
-  const int tt = convolves ? wave - kNarrowTiles * kNarrowGroups
-                           : wave / kNarrowGroups;
-  struct At {
+  const bool convolves = wave >= kNarrowTeams * kNarrowGroups;
+  // this wave's tiles: every second, from this one on
+  const int first = convolves ? wave - kNarrowTeams * kNarrowGroups
+                              : wave / kNarrowGroups;
+  struct At {  // a tile: row (past the range: none), and which of the row's
     int row, k;
   };
-  const int step_rows = kNarrowTiles / tiles_per_row;
-  const int step_k = kNarrowTiles % tiles_per_row;
+  const int step_rows = kNarrowTeams / tiles_per_row;
+  const int step_k = kNarrowTeams % tiles_per_row;
   auto step = [&](At& at) RG_INLINE {
     at.row += step_rows;
     at.k += step_k;
@@ -771,69 +815,93 @@ block_prefill_narrow_bf16_kernel(FusedArgs p, int slices, int groups) {
       ++at.row;
     }
   };
-  At asked = {row0 + tt / tiles_per_row, tt % tiles_per_row};
+  const At begin = {row0 + first / tiles_per_row, first % tiles_per_row};
   // positions of rows t0 - 32 .. t0 + 31 of the tile a wave asks for
   uint32_t seg_lo = 1, seg_hi = 0;
   bool seg_in = false;
+  // (no branch: a load on one of two paths is waited for, with all before it, on both)
   auto request_positions = [&](const At& at) RG_INLINE {
     const bool any = at.row < row1;
+    const uint32_t bytes = (uint32_t)T * seg_esize;
+    const __amdgpu_buffer_rsrc_t rseg = make_rsrc(
+        (const char*)p.segpos + (int64_t)(any ? at.row : row0) * bytes, any ? bytes : 0u);
     const int t = at.k * kTile + lane - 32;
-    seg_in = any && t >= 0 && t < T;
-    const char* seg_row = (const char*)p.segpos +
-                          (int64_t)(any ? at.row : row0) * T * seg_esize;
-    const uint32_t off = (uint32_t)(seg_in ? t : 0) * seg_esize;
-    seg_lo = *reinterpret_cast<const uint32_t*>(seg_row + off);
-    seg_hi = seg_is64 ? *reinterpret_cast<const uint32_t*>(seg_row + off + 4) : 0u;
+    seg_in = any && (uint32_t)t < (uint32_t)T;
+    const uint32_t off = seg_in ? (uint32_t)t * seg_esize : kBufferOutOfRange;
+    seg_lo = __builtin_amdgcn_raw_buffer_load_b32(rseg, off, 0, 0);
+    seg_hi = __builtin_amdgcn_raw_buffer_load_b32(
+        rseg, seg_is64 ? off + 4u : kBufferOutOfRange, 0, 0);
   };
   auto starts_mask = [&]() RG_INLINE -> uint64_t {
     return __ballot(seg_in && (seg_lo | seg_hi) == 0u);
   };
+  // Where a token's conv output lies in its tile: a lane of the matrix result has
+  // rows 0-3, 8-11, .. (upper lanes 4-7, 12-15, ..), and gets sixteen tokens in a row.
+  auto conv_row = [](int t) RG_INLINE {
+    return 8 * ((t & 15) >> 2) + (t & 3) + 4 * (t >> 4);
+  };
+  auto conv_at = [](int tile) RG_INLINE {
+    return (uint32_t)((tile % kNarrowRing) * L::tile);
+  };
   fill_taps<L>(p, lds_raw, tid, bw, h);
+  // Behind every phase.  (lds_barrier would wait for the raw rows on their way into
+  // LDS, too: whoever reads them waits for them, two phases on.)
+  auto phase_barrier = []() RG_INLINE {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto wait_loads = []() RG_INLINE {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L::raw_loads) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
   if (convolves) {
     // ---- conv: channel pairs 0-63 of the head, 32 rows a lane; then the 24
     //      others, 16 rows a lane (the upper lanes the later ones) -------------
     const int pair_b = 64 + (lane & 31);
     const bool lane_b = pair_b < kNarrowPairs;
-    const uint32_t off_a = 2u * (uint32_t)(h * bw + 2 * lane);
     const int row_b = (lane >> 5) * 16;
-    const uint32_t off_b = lane_b && 2 * pair_b < bw
-                               ? 2u * (uint32_t)(h * bw + 2 * pair_b)
-                               : kBufferOutOfRange;
     constexpr int kRowsB = 16;
-    uint32_t raw_a[kTile + 3], raw_b[kRowsB + 3];
-    auto request = [&]() RG_INLINE {
+    // Raw rows t0 - 3 .. t0 + 31 of a tile as the memory pipe writes them into LDS,
+    // 22 pieces of 16 bytes each (zeros beyond the head and the sequence), two tiles
+    // of each of the two waves.  (As 54 loads of four bytes a lane into registers, two
+    // rows a load at best, the conv took longer than the other waves' phases: B4 T2048
+    // W5632 110 us, joined 124.)
+    uint32_t piece[L::raw_loads];
+#pragma unroll
+    for (int j = 0; j < L::raw_loads; ++j) {
+      const int q = 64 * j + lane, r = q / L::raw_pieces, c = q % L::raw_pieces;
+      piece[j] = r < kTile + 3 && 8 * c < bw
+                     ? (uint32_t)((r - 3) * (int)row_bytes) +
+                           2u * (uint32_t)(h * bw) + 16u * c
+                     : kBufferOutOfRange;
+    }
+    At asked = begin, asked_positions = begin;
+    auto raw_at = [](int tile) RG_INLINE {
+      return (uint32_t)(L::raw + (tile % kNarrowRaw) * L::raw_tile);
+    };
+    auto request = [&](int tile) RG_INLINE {  // (the one that `asked` stands at)
       const bool any = asked.row < row1;
-      const int b = any ? asked.row : row0;
-      const int t0 = asked.k * kTile;
-      const char* base = (const char*)p.x + (int64_t)b * seq_bytes;
-      const __amdgpu_buffer_rsrc_t rx = make_rsrc(base, any ? seq_bytes : 0);
-      const __amdgpu_buffer_rsrc_t rhalo =
-          make_rsrc(base, any && t0 ? seq_bytes : 0);
+      const uint32_t before = (uint32_t)(asked.k * kTile) * row_bytes;
+      const __amdgpu_buffer_rsrc_t rx = make_rsrc(
+          (const char*)p.x + (int64_t)(any ? asked.row : row0) * seq_bytes,
+          any ? seq_bytes : 0);
 #pragma unroll
-      for (int r = 0; r < kTile + 3; ++r)
-        raw_a[r] = __builtin_amdgcn_raw_buffer_load_b32(
-            r < 3 ? rhalo : rx,
-            off_a + (uint32_t)(r < 3 && t0 == 0 ? 0 : t0 + r - 3) * row_bytes, 0,
-            0);
-#pragma unroll
-      for (int r = 0; r < kRowsB + 3; ++r) {
-        const int t = t0 + row_b + r - 3;  // (before the row's start: zeros)
-        raw_b[r] = __builtin_amdgcn_raw_buffer_load_b32(
-            rx,
-            off_b == kBufferOutOfRange || t < 0
-                ? kBufferOutOfRange
-                : off_b + (uint32_t)t * row_bytes,
-            0, 0);
-      }
-      request_positions(asked);
+      for (int j = 0; j < L::raw_loads; ++j)
+        load_to_lds(rx, lds3 + raw_at(tile) + 1024 * j, piece[j] + before);
       step(asked);
     };
     // ROWS rows from raw rows; bit j of `cuts`: raw row j starts a document
-    auto convolve = [&](auto& raw, auto ROWS, const int pair_of_lane,
+    auto convolve = [&](const uint32_t raw_from, auto ROWS, const int pair_of_lane,
                         const uint32_t out, const bool store,
                         const uint64_t cuts) RG_INLINE {
       constexpr int rows = decltype(ROWS)::value;
+      uint32_t raw[rows + 3];
+#pragma unroll
+      for (int r = 0; r < rows + 3; ++r)
+        raw[r] = *reinterpret_cast<lds_u32*>(lds3 + raw_from + r * L::raw_row);
       uint32_t w10[2], w32[2];
       float bias[2];
       const u32x4 t0 =
@@ -848,7 +916,7 @@ block_prefill_narrow_bf16_kernel(FusedArgs p, int slices, int groups) {
       }
       auto put = [&](int r, const float (&o)[2]) RG_INLINE {
         if (store)
-          *reinterpret_cast<lds_u32*>(lds3 + out + r * L::row) =
+          *reinterpret_cast<lds_u32*>(lds3 + out + conv_row(r) * L::row) =
               pack_bf16x2(o[0], o[1]);
       };
       uint32_t p1[2], p2[2];
@@ -899,55 +967,252 @@ block_prefill_narrow_bf16_kernel(FusedArgs p, int slices, int groups) {
         }
       }
     };
-    auto convolve_tile = [&](int buf) RG_INLINE {
-      const uint64_t mask = starts_mask();
-      const uint32_t tile = (uint32_t)(buf * L::buffer + tt * kTile * L::row);
-      convolve(raw_a, std::integral_constant<int, kTile>{}, lane,
-               tile + lane * 4, true, mask >> 29);
-      convolve(raw_b, std::integral_constant<int, kRowsB>{},
-               lane_b ? pair_b : 64, tile + row_b * L::row + pair_b * 4, lane_b,
+    uint64_t mask = 0;  // of the tile whose first part was made last
+    auto make_a = [&](int tile) RG_INLINE {
+      // the tile's raw rows, asked for three phases ago, and its positions (the rows of
+      // the next tile of this wave may still be on their way)
+      wait_loads();
+      mask = starts_mask();
+      request_positions(asked_positions);
+      step(asked_positions);
+      convolve(raw_at(tile) + lane * 4, std::integral_constant<int, kTile>{}, lane,
+               conv_at(tile) + lane * 4, true, mask >> 29);
+    };
+    // (the wave that shares the SIMD has its phase G then: the loads, which hold a wave
+    // 50 to 100 cycles each, where there is less of the conv)
+    auto make_b = [&](int tile) RG_INLINE {
+      request(tile + 2 * kNarrowTeams);
+      convolve(raw_at(tile) + row_b * L::raw_row + pair_b * 4,
+               std::integral_constant<int, kRowsB>{}, lane_b ? pair_b : 64,
+               conv_at(tile) + 4 * (lane >> 5) * L::row + pair_b * 4, lane_b,
                (mask >> (29 + row_b)) & ((1u << (kRowsB + 3)) - 1u));
     };
-    request();
+    request(first);
+    request_positions(asked_positions);
+    step(asked_positions);
+    request(first + kNarrowTeams);
     __syncthreads();  // taps
-    convolve_tile(0);
-    if (npasses > 1) request();
-    lds_barrier();
-    for (int i = 0; i < npasses; ++i) {
-      if (i + 1 < npasses) {
-        convolve_tile((i & 1) ^ 1);
-        if (i + 2 < npasses) request();
-      }
-      lds_barrier();  // (the multiplying waves' one in gate_and_scan)
+    make_a(first);
+    if (first == 0) make_b(0);
+    phase_barrier();
+    int phase = 0, tile = 2;
+    if (first == 1) {
+      make_b(1);
+      phase_barrier();
+      phase = 1;
+      tile = 3;
+    }
+    for (; phase < ntiles; phase += 2, tile += 2) {
+      if (tile < ntiles) make_a(tile);
+      phase_barrier();
+      if (tile < ntiles) make_b(tile);
+      if (phase + 1 < ntiles) phase_barrier();
     }
   } else {
+    const int team = first;
     const int c0 = 32 * (wave % kNarrowGroups);
     const int n0 = slice * kNarrowSlice + c0;
     load_weights<kNarrowKS, PACKED>(p, lane, bw, h, n0);
-    request_positions(asked);
-    if (tt == 0) fill_gate_values<L>(p, lds_raw, lane, bw, h, n0, c0);
+    if (team == 0) fill_gate_values<L>(p, lds_raw, lane, bw, h, n0, c0);
     __syncthreads();  // taps
-    lds_barrier();    // the first conv tiles, the gate values
-    const uint32_t a_lane =
-        (uint32_t)(tt * kTile + (lane & 31)) * L::row + 16u * (lane >> 5);
-    float carry = 0.0f;
-    int until = 0;
-    for (int i = 0; i < npasses; ++i) {
-      const int buf = i & 1;
-      const At now = asked;
-      const bool any = now.row < row1;
-      f32x16 acc_x, acc_a;
-      matrix_tile<kNarrowKS>(lds3, a_lane + buf * L::buffer, acc_x, acc_a,
-                             [](auto) RG_INLINE {});
+    phase_barrier();  // the first conv tiles, the gate values
+    const f32x4 per_channel = *reinterpret_cast<lds_f32x4*>(
+        lds3 + L::gates + (c0 + (lane & 31)) * 16);
+    const float bias_x = per_channel[0], bias_a = per_channel[1];
+    const float inv_decay = per_channel[2];
+    const uint32_t a_lane = (uint32_t)(lane & 31) * L::row + 16u * (lane >> 5);
+    const uint32_t xc_lane = 4u * (lane >> 5) * L::row + 2u * (uint32_t)(n0 + (lane & 31));
+    const uint32_t patch_at = L::patch + wave * L::patch_wave + (lane >> 5) * L::patch_upper;
+    const uint32_t patch_w = patch_at + 2u * (lane & 31);
+    const uint32_t patch_r =
+        patch_at + (uint32_t)((lane >> 2) & 7) * kPatchStride + 16u * (lane & 3);
+    const bool ch_valid = n0 + (lane & 31) < bw;
+    // (8 channels a lane: all of them channels of the head or none)
+    const uint32_t y_lane =
+        n0 + 8 * (lane & 3) < bw
+            ? (uint32_t)(16 * (lane >> 5) + ((lane >> 2) & 7)) * row_bytes +
+                  2u * (uint32_t)(h * bw + n0) + 16u * (lane & 3)
+            : kBufferOutOfRange;
+    const uint32_t state_at = L::state + 4u * (uint32_t)(c0 + (lane & 31));
+    const uint32_t ch_bytes = ch_valid ? 4u * (uint32_t)(h * bw + n0 + (lane & 31))
+                                       : kBufferOutOfRange;
+    auto state_row = [&](const float* base, int b, bool any) RG_INLINE {
+      return make_rsrc(base + (int64_t)b * W, base && any ? 4u * (uint32_t)p.W : 0u);
+    };
+    float h0 = 0.0f;  // of a tile that opens its row
+
+    f32x16 acc_x, acc_a;
+    uint32_t xr[16];  // conv outputs, this lane's tokens, as floats
+    u32x4 y_pending[2];
+    int y_row = -1;  // where they belong: row (none yet) and first token
+    uint32_t y_at = 0;
+    At at = begin;
+
+    auto rows_of = [&](const void* base, int b, bool any) RG_INLINE {
+      return make_rsrc((const char*)base + (int64_t)b * seq_bytes, any ? seq_bytes : 0u);
+    };
+    // (a lane past the head's channels keeps its offset out of every descriptor)
+    auto y_offset = [&](uint32_t before) RG_INLINE {
+      return y_lane == kBufferOutOfRange ? kBufferOutOfRange : y_lane + before;
+    };
+    auto store_pending = [&]() RG_INLINE {
+      const __amdgpu_buffer_rsrc_t ry = rows_of(p.y, y_row < 0 ? row0 : y_row, y_row >= 0);
+      buffer_store_16(y_pending[0], ry, y_offset(y_at), 0);
+      buffer_store_16(y_pending[1], ry, y_offset(y_at + 8u * row_bytes), 0);
+    };
+    y_pending[0] = y_pending[1] = u32x4{0, 0, 0, 0};
+    u32x4 gate_rows[2];  // the gate branch's values, then gelu of them
+
+    // What phase G reads of tile `at`, asked for a tile of this team ahead and in front
+    // of the outputs of the tile before (loads and stores are waited for in order).
+    auto request = [&]() RG_INLINE {
+      const bool any = at.row < row1;
+      request_positions(at);
+      h0 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+          state_row(p.h0, any ? at.row : row0, any && at.k == 0), ch_bytes, 0, 0));
+      if (GELU) {
+        const __amdgpu_buffer_rsrc_t rgate =
+            rows_of(p.gate_branch, any ? at.row : row0, any);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          gate_rows[j] = __builtin_amdgcn_raw_buffer_load_b128(
+              rgate, y_offset((uint32_t)(at.k * kTile + 8 * j) * row_bytes), 0, 0);
+      }
+    };
+
+    // ---- phase M: the tile's matrix instructions; y of this team's tile before ----
+    auto phase_m = [&](int tile) RG_INLINE {
+      const uint32_t tile_at = conv_at(tile);
+      store_pending();
+      const uint32_t x_at = tile_at + xc_lane;
+      __builtin_amdgcn_s_setprio(1);
+      matrix_tile<kNarrowKS>(lds3, tile_at + a_lane, acc_x, acc_a, [&](auto KSTEP) RG_INLINE {
+        constexpr int ks = decltype(KSTEP)::value;
+        // the conv outputs for the gate arithmetic (in phase G)
+        if constexpr (ks >= kNarrowKS - 4) {
+          static_for<4 * (ks - kNarrowKS + 4), 4 * (ks - kNarrowKS + 5)>([&](auto I) RG_INLINE {
+            constexpr int i = decltype(I)::value;
+            xr[i] = read_bf16_high<(8 * (i >> 2) + (i & 3)) * L::row>(x_at);
+          });
+        }
+      });
+      __builtin_amdgcn_s_setprio(0);
+      // gelu here, the gates in phase G.  (us, B4 T2048 W5632: joined 112.1, with gelu in
+      // phase G 115.4; plain 90.4, with 4, 8 or 16 of the lane's input gates here 91.1,
+      // 92.3, 98.4)
+      if (GELU) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) gate_rows[j][k] = gelu_bf16x2(gate_rows[j][k]);
+        asm volatile("" : "+v"(gate_rows[0]), "+v"(gate_rows[1]));
+      }
+    };
+    // ---- phase G: gates, recurrence, outputs ---------------------------------------
+    auto phase_g = [&](auto GENERAL, uint32_t tile_starts) RG_INLINE {
+      constexpr bool general = decltype(GENERAL)::value;
+      const int t0 = at.k * kTile;
+      // the state before the tile
+      float before = *reinterpret_cast<__attribute__((address_space(3))) float*>(
+          lds3 + state_at);
+      before = at.k == 0 ? h0 : before;
+      float xn[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float gx = __builtin_amdgcn_rcpf(
+            1.0f + __builtin_amdgcn_exp2f(__builtin_fmaf(acc_x[i], -kLog2e, bias_x)));
+        acc_a[i] = __builtin_amdgcn_exp2f(gate_exponent(
+            __builtin_amdgcn_exp2f(__builtin_fmaf(acc_a[i], -kLog2e, bias_a)),
+            inv_decay));
+        xn[i] = __uint_as_float(xr[i]) * gx;
+      }
+      if (general) {
+        // document start: a = 0; past the end of the row: identity
+        int token0 = (lane >> 5) * 16;
+        asm volatile("" : "+v"(token0));
+        const uint32_t mine = tile_starts >> token0;
+        const int left = T - t0 - token0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          acc_a[i] = (mine >> i) & 1u ? 0.0f : acc_a[i];
+          acc_a[i] = i < left ? acc_a[i] : 1.0f;
+          xn[i] = i < left ? xn[i] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        xn[i] *= __builtin_amdgcn_sqrtf(__builtin_fmaf(-acc_a[i], acc_a[i], 1.0f));
+      // walked twice: right for the lower lanes, whose end goes to the upper ones,
+      // then from each half's own incoming state
+      float e1 = before;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) e1 = __builtin_fmaf(acc_a[i], e1, xn[i]);
+      const auto sw = __builtin_amdgcn_permlane32_swap(
+          __float_as_uint(before), __float_as_uint(e1), false, false);
+      float hh = __uint_as_float(sw[0]);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float hv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          hh = __builtin_fmaf(acc_a[4 * g + q], hh, xn[4 * g + q]);
+          hv[q] = hh;
+        }
+        const uint32_t y01 = pack_bf16x2(hv[0], hv[1]);
+        const uint32_t y23 = pack_bf16x2(hv[2], hv[3]);
+        asm volatile(
+            "ds_write_b16 %0, %1 offset:%3\n\t"
+            "ds_write_b16_d16_hi %0, %1 offset:%4\n\t"
+            "ds_write_b16 %0, %2 offset:%5\n\t"
+            "ds_write_b16_d16_hi %0, %2 offset:%6"
+            :
+            : "v"(patch_w), "v"(y01), "v"(y23), "n"((4 * (g & 1)) * kPatchStride),
+              "n"((4 * (g & 1) + 1) * kPatchStride),
+              "n"((4 * (g & 1) + 2) * kPatchStride),
+              "n"((4 * (g & 1) + 3) * kPatchStride)
+            : "memory");
+        if (g & 1) {
+          // (the LDS unit executes a wave's instructions in order)
+          y_pending[g >> 1] = *reinterpret_cast<lds_u32x4*>(lds3 + patch_r);
+          asm volatile("" ::: "memory");
+        }
+      }
+      // the state behind the tile: the upper lanes' end
+      if (lane >= 32) {
+        *reinterpret_cast<__attribute__((address_space(3))) float*>(lds3 + state_at) = hh;
+        if (at.k == tiles_per_row - 1)
+          __builtin_amdgcn_raw_buffer_store_b32(
+              __float_as_uint(hh), state_row(p.h_last, at.row, true), ch_bytes, 0, 0);
+      }
+      if (GELU) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            y_pending[j][k] = mul_bf16x2(y_pending[j][k], gate_rows[j][k]);
+      }
+      // (done here: behind the loads of the next tile they would be waited for)
+      asm volatile("" : "+v"(y_pending[0]), "+v"(y_pending[1]));
+      __builtin_amdgcn_sched_barrier(0);
+      y_row = at.row;
+      y_at = (uint32_t)t0 * row_bytes;
+    };
+
+    request();
+    if (team == 1) phase_barrier();
+    for (int tile = team; tile < ntiles; tile += kNarrowTeams) {
+      phase_m(tile);
+      phase_barrier();
       const uint32_t starts = (uint32_t)(starts_mask() >> 32);
-      step(asked);
-      request_positions(asked);
-      gate_and_scan<L, kNarrowTiles, kNarrowSlice, GELU>(
-          p, lds3, lane, wave, bw, h, n0, c0, tt, buf, tiles_per_row,
-          TileAt{any ? now.row : row0, now.k * kTile, now.k, any,
-                 any && n0 < bw, starts},
-          acc_x, acc_a, carry, until);
+      if (__builtin_expect(starts != 0 || (at.k + 1) * kTile > T, 0))
+        phase_g(std::true_type{}, starts);
+      else
+        phase_g(std::false_type{}, starts);
+      step(at);
+      request();
+      if (tile + 1 < ntiles) phase_barrier();
     }
+    store_pending();
   }
   if (p.cache_out)
     store_conv_state<kNarrowSlice>(p, tid, bw, h, slice * kNarrowSlice, row0, row1);
@@ -1003,13 +1268,13 @@ Plan plan(int B, int H, int T, int bw, bool joined) {
     return Plan{kSlices16, slices,
                 best_split(B, H, T, slices, kTiles, joined ? 5.8f : 6.2f,
                            joined ? 6.3f : 5.2f)};
-  // narrow heads: four tiles at once while that fills no more than one round
-  // (few rows), else the specialised waves
-  const Split wide = best_split(B, H, T, slices, kTiles, 6.2f,
-                                joined ? 5.2f : 4.3f);
+  // Narrow heads: four tiles at once for few rows of up to 128 tokens, else the
+  // specialised waves (whose walk in the tokens' order rounds states differently: the
+  // form does not depend on the join, so that a joined call is a plain one and the join,
+  // bit for bit).
+  const Split wide = best_split(B, H, T, slices, kTiles, 6.2f, 5.2f);
   const int pairs = (bw + kNarrowSlice - 1) / kNarrowSlice;
-  const Split roles = best_split(B, H, T, pairs, kNarrowTiles, 7.0f,
-                                 joined ? 3.8f : 3.2f);
+  const Split roles = best_split(B, H, T, pairs, kNarrowTeams, 7.0f, 3.2f);
   if (wide.us <= roles.us) return Plan{kSlices11, slices, wide};
   return Plan{kNarrow, pairs, roles};
 }
@@ -1020,15 +1285,15 @@ hipError_t launch_as(const FusedArgs& a, const Plan& p, hipStream_t s) {
   switch (p.form) {
     case kNarrow:
       return launch_one(block_prefill_narrow_bf16_kernel<PACKED, GELU>, once[0],
-                        Layout<kNarrowKS, kNarrowTiles, kNarrowSlice>::total, a,
+                        NarrowLayout::total, a,
                         p.slices, p.split.groups, s);
     case kSlices11:
       return launch_one(block_prefill_slices_bf16_kernel<11, PACKED, GELU>,
-                        once[1], Layout<11, kTiles, kSlice>::total, a, p.slices,
+                        once[1], Layout<11>::total, a, p.slices,
                         p.split.groups, s);
     default:
       return launch_one(block_prefill_slices_bf16_kernel<16, PACKED, GELU>,
-                        once[2], Layout<16, kTiles, kSlice>::total, a, p.slices,
+                        once[2], Layout<16>::total, a, p.slices,
                         p.split.groups, s);
   }
 }

@@ -25,6 +25,10 @@ NAMES = ("conv_w", "conv_b", "w_x", "b_x", "w_a", "b_a", "a_param")
     # head widths between the presets': padding in k, in channels, in both
     (2, 70, 136, 2, 20), (2, 70, 168, 3, 20), (3, 150, 184, 2, 50),
     (3, 150, 200, 1, 50), (2, 70, 248, 3, 20),
+    # narrow heads, two teams of waves: odd and even numbers of tiles, several rows per
+    # workgroup, whole and cut last tiles
+    (16, 33, 176, 32, 20), (12, 97, 176, 32, -50), (20, 64, 160, 32, 40),
+    (9, 31, 176, 32, 6), (5, 193, 128, 60, 70),
     # long rows, left padding
     (2, 700, 176, 4, -200), (3, 333, 256, 10, 80),
     # 256-wide heads, rows longer than a pass: more than 32 pairs (fewer go to
@@ -131,7 +135,9 @@ def _core(x, seg, ws, h0=None, packed=True):
     (8, 10, 256, 10), (8, 32, 256, 10), (8, 45, 256, 10), (8, 100, 256, 10),
     (8, 200, 256, 10), (7, 333, 256, 16), (8, 440, 256, 10), (3, 333, 256, 10),
     (9, 10, 176, 32), (9, 32, 176, 32), (8, 50, 176, 32), (7, 100, 176, 32),
-    (8, 333, 176, 32), (6, 1000, 176, 32), (8, 70, 200, 12)])
+    (8, 333, 176, 32), (6, 1000, 176, 32), (8, 70, 200, 12),
+    # narrow heads of two teams: a row per tile, rows that end in either team's
+    (9, 20, 160, 64), (8, 64, 176, 32), (7, 65, 176, 32), (6, 97, 176, 64)])
 @pytest.mark.parametrize("packed", [True, False])
 def test_rows_do_not_see_each_other(B, T, bw, H, packed):
   """A NaN or an infinity in one row's x or h0 leaves every other row's outputs
