@@ -127,6 +127,10 @@ PACKAGE_SIGNATURES = {
     "rg_linear_back": (_i, [_vp] * 5 + [_i64, _i, _i, _i, _vp]),
     "rg_linear_weight_grads": (_i, [_vp] * 5 + [_i, _i64, _i, _vp]),
     "rg_linear_rows_beside": (_i, [_vp] * 4 + [_i] * 4 + [_vp, _vp, _i64, _vp]),
+    "rg_linear_rows_partial_flags": (_i, [_vp] * 4 + [_i] * 4 + [_vp]),
+    "rg_linear_rows_normed_serve": (_i, [_i] * 4),
+    "rg_linear_rows_normed": (_i, [_vp, _i, _vp, _vp, _vp, ctypes.c_float] + [_vp] * 6 +
+                              [_i] * 5 + [_vp, _vp, _i64, _i, _vp]),
     "rg_linear_gelu_pair_pays": (_i, [_i64, _i, _i, _i]),
     "rg_linear_gelu_pair": (_i, [_vp] * 4 + [_i64, _i, _i, _i, _vp]),
     "rg_linear_scan_best_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),

@@ -348,13 +348,16 @@ PyObject* rows_partial(PyObject*, PyObject* const* v, Py_ssize_t n) {
     void* x = c(v[1]);
     const long slices = PyLong_AsLong(v[4]);
     need(slices > 0);
-    Tensor sums = c.empty({slices, M, (int64_t)p.N}, at::kFloat);
-    void* op = sums.mutable_data_ptr();
+    // (the flags of rg_linear_rows_normed behind the sums)
+    const int64_t n = slices * M * p.N;
+    Tensor all = c.empty({n + RG_NORM_FLAGS}, at::kFloat);
+    void* op = all.mutable_data_ptr();
+    Tensor sums = all.narrow(0, 0, n).view({slices, M, (int64_t)p.N});
     const void* pk = p.packed.const_data_ptr();
     void* s = c.stream();
     launch([&] {
-      return rg_linear_rows_partial(x, pk, (float*)op, (int)M, p.K, p.N,
-                                    (int)slices, s);
+      return rg_linear_rows_partial_flags(x, pk, (float*)op, (uint32_t*)((float*)op + n),
+                                          (int)M, p.K, p.N, (int)slices, s);
     });
     return wrap(sums);
   });

@@ -1815,7 +1815,7 @@ int rg_linear_rows(const void* x, const void* w_packed, const void* bias,
     return fail(RG_ERR_WORKSPACE,
                 "%s: workspace of %zu bytes (16-byte aligned) required, got %zu",
                 __func__, need, workspace ? workspace_bytes : (size_t)0);
-  rg::LinearArgs a;
+  rg::LinearArgs a{};
   a.x = x;
   a.w_packed = w_packed;
   a.bias = bias;
@@ -1872,8 +1872,9 @@ int rg_linear_rows_beside(const void* x, const void* w_packed, const void* bias,
                        rg::launch_linear_rows_beside(a, (hipStream_t)stream));
 }
 
-int rg_linear_rows_partial(const void* x, const void* w_packed, void* partial,
-                           int M, int K, int N, int slices, void* stream) {
+int rg_linear_rows_partial_flags(const void* x, const void* w_packed, void* partial,
+                                 uint32_t* flags, int M, int K, int N, int slices,
+                                 void* stream) {
   RG_REQUIRE(M > 0 && K > 0 && N > 0, "%s: M=%d K=%d N=%d must be positive",
              __func__, M, K, N);
   if (M > 64 || rg_linear_packed_bytes(N, K, 0) == 0)
@@ -1886,7 +1887,9 @@ int rg_linear_rows_partial(const void* x, const void* w_packed, void* partial,
   RG_CHECK_PTR(w_packed);
   RG_CHECK_PTR(partial);
   RG_REQUIRE(partial != x, "%s: partial must not alias x", __func__);
+  RG_REQUIRE(((uintptr_t)flags & 3) == 0, "%s: flags is not 4-byte aligned", __func__);
   rg::LinearArgs a{};
+  a.clear = flags;
   a.x = x;
   a.w_packed = w_packed;
   a.partial = (float*)partial;
@@ -1896,6 +1899,88 @@ int rg_linear_rows_partial(const void* x, const void* w_packed, void* partial,
   a.group_width = N;
   return launch_status(__func__, rg::launch_linear_rows_partial(
                                      a, slices, (hipStream_t)stream));
+}
+
+int rg_linear_rows_partial(const void* x, const void* w_packed, void* partial,
+                           int M, int K, int N, int slices, void* stream) {
+  return rg_linear_rows_partial_flags(x, w_packed, partial, nullptr, M, K, N, slices,
+                                      stream);
+}
+
+static_assert(RG_NORM_FLAGS == rg::kNormFlags, "");
+int rg_linear_rows_normed_serve(int M, int K, int N, int gelu_pair) {
+  return M <= 64 && N > 0 && rg_linear_packed_bytes(N, K, gelu_pair) > 0 &&
+         rg::linear_rows_normed_serve(M, K, N, gelu_pair);
+}
+
+int rg_linear_rows_normed(const void* partial, int slices, const void* partial_bias,
+                          const void* addend, const void* scale, float eps, void* sum_out,
+                          void* normed, uint32_t* flags, const void* w_packed,
+                          const void* bias, void* out, int M, int K, int N, int groups,
+                          int gelu_pair, const void* from, void* to, int64_t bytes,
+                          int patience, void* stream) {
+  RG_REQUIRE(M > 0 && K > 0 && N > 0, "%s: M=%d K=%d N=%d must be positive",
+             __func__, M, K, N);
+  if (!rg_linear_rows_normed_serve(M, K, N, gelu_pair))
+    return fail(RG_ERR_UNSUPPORTED, "%s: M=%d K=%d N=%d gelu_pair=%d is not served",
+                __func__, M, K, N, gelu_pair);
+  RG_REQUIRE(slices >= 1 && slices <= 8, "%s: slices=%d not in 1..8", __func__, slices);
+  RG_REQUIRE(groups >= 1 && N % groups == 0 && (N / groups) % 4 == 0 &&
+                 (!gelu_pair || groups == 1),
+             "%s: N=%d / groups=%d must be a multiple of 4, gelu pairs one group",
+             __func__, N, groups);
+  RG_REQUIRE(bytes >= 0 && bytes % 16 == 0 && (bytes == 0 || !gelu_pair),
+             "%s: bytes=%lld is no multiple of 16, or beside gelu pairs", __func__,
+             (long long)bytes);
+  RG_REQUIRE(patience >= 0, "%s: patience=%d is negative", __func__, patience);
+  RG_CHECK_PTR(partial);
+  RG_CHECK_PTR(scale);
+  RG_CHECK_PTR(sum_out);
+  RG_CHECK_PTR(normed);
+  RG_CHECK_PTR(w_packed);
+  RG_CHECK_PTR(out);
+  RG_CHECK_OPT_PTR(partial_bias);
+  RG_CHECK_OPT_PTR(addend);
+  RG_CHECK_OPT_PTR(bias);
+  if (bytes) {
+    RG_CHECK_PTR(from);
+    RG_CHECK_PTR(to);
+  }
+  RG_REQUIRE(flags != nullptr && ((uintptr_t)flags & 3) == 0,
+             "%s: flags is null or not 4-byte aligned", __func__);
+  const void* const in[] = {partial, partial_bias, addend, scale, w_packed, bias,
+                            bytes ? from : nullptr};
+  const void* const written[] = {sum_out, normed, out, flags, bytes ? to : nullptr};
+  for (size_t i = 0; i < sizeof(written) / sizeof(*written); ++i) {
+    RG_REQUIRE(!written[i] || !among(written[i], in, sizeof(in) / sizeof(*in)),
+               "%s: an output must not alias an input", __func__);
+    RG_REQUIRE(!written[i] || !among(written[i], written, (int)i),
+               "%s: outputs must not alias each other", __func__);
+  }
+  rg::NormedLinearArgs a{};
+  a.layer.x = normed;
+  a.layer.w_packed = w_packed;
+  a.layer.bias = bias;
+  a.layer.out = out;
+  a.layer.M = M;
+  a.layer.K = K;
+  a.layer.N = N;
+  a.layer.group_width = N / groups;
+  a.layer.copy_from = from;
+  a.layer.copy_to = to;
+  a.layer.copy_items = bytes / 16;
+  a.sums = (const float*)partial;
+  a.bias = partial_bias;
+  a.addend = addend;
+  a.scale = scale;
+  a.sum_out = sum_out;
+  a.normed = normed;
+  a.flags = flags;
+  a.slices = slices;
+  a.patience = patience;
+  a.eps = eps;
+  return launch_status(__func__,
+                       rg::launch_linear_rows_normed(a, gelu_pair, (hipStream_t)stream));
 }
 
 int rg_add_rms_norm_partial(const void* partial, int slices, const void* bias,

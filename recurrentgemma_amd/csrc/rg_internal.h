@@ -218,6 +218,23 @@ struct LinearArgs {
   const void* copy_from;
   void* copy_to;
   int64_t copy_items;
+  // with partial sums: kNormFlags words set to zero for launch_linear_rows_normed
+  uint32_t* clear;
+};
+constexpr int kNormFlags = 64;
+
+// A layer whose x is the norm of what the layer before left as partial sums.
+struct NormedLinearArgs {
+  LinearArgs layer;  // x = normed
+  const float* sums;  // [slices, M, K]
+  const void* bias;   // [K] or null: of the layer before
+  const void* addend;  // [M, K] or null
+  const void* scale;   // [K]
+  void* sum_out;       // [M, K]
+  void* normed;        // [M, K]
+  uint32_t* flags;     // kNormFlags words, zero: row m is there
+  int slices, patience;
+  float eps;
 };
 
 // Each returns hipSuccess or the launch error.  dtype: 0 = f32, 1 = bf16.
@@ -415,6 +432,9 @@ hipError_t launch_linear_rows(const LinearArgs& a, int gelu_pair,
 hipError_t launch_linear_rows_beside(const LinearArgs& a, hipStream_t s);
 // Only the fp32 partial sums a.partial[slices][M][N] of x @ W^T, K split in
 // `slices`; rg_elementwise.hip's norm kernel takes them from there.
+bool linear_rows_normed_serve(int M, int K, int N, int gelu_pair);
+hipError_t launch_linear_rows_normed(const NormedLinearArgs& a, int gelu_pair,
+                                     hipStream_t s);
 hipError_t launch_linear_rows_partial(const LinearArgs& a, int slices,
                                       hipStream_t s);
 hipError_t launch_rms_norm_partial(const float* sums, int slices,

@@ -25,6 +25,7 @@
 // stacked up-projection (modules.py:752-757).
 #include "rg_common.h"
 #include "rg_internal.h"
+#include "rg_norm_row.h"
 
 namespace rg {
 namespace {
@@ -36,6 +37,7 @@ union Frag {
 
 constexpr int kXStride = 72;  // elements per staged x row: 64 + 8 of padding
 constexpr int kWaves = 8;
+constexpr int kAgentScope = 16;  // sc1 of a buffer instruction (gfx950)
 
 // LDS of a wave: its x tile (whole blocks of 32 rows) or its sums.
 __host__ __device__ constexpr int wave_lds_bytes(int nt, int blocks) {
@@ -59,26 +61,128 @@ __device__ __forceinline__ size_t out_index(int m, int n, int M, int gw) {
   return ((size_t)grp * M + m) * gw + (n - grp * gw);
 }
 
+// From the waves' accumulators to the layer's outputs: the sums over K meet in LDS, then
+// the epilogue.  block: which NT tiles of weight rows.
+template <int NT, int MODE, int XR>
+__device__ __forceinline__ void add_up_and_store(
+    const LinearArgs& p, unsigned char* const smem, const int wave, const int lane,
+    const int block, const f32x16 (&acc)[NT][XR > 32 ? 2 : 1]) {
+  constexpr int kMB = XR > 32 ? 2 : 1;
+  constexpr int kWaveLds = wave_lds_bytes(NT, kMB);
+  const int M = p.M;
+  // the waves' partial sums meet in LDS (each wave's region is its own x tile)
+  float* mine = reinterpret_cast<float*>(smem + (size_t)wave * kWaveLds);
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int m = 0; m < kMB; ++m)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        mine[((t * kMB + m) * 16 + i) * 64 + lane] = acc[t][m][i];
+  lds_barrier();
+  const float* red = reinterpret_cast<const float*>(smem);
+  // sum of accumulator registers 4 q .. 4 q + 3 of (tile t, half m, lane l):
+  // result rows 32 m + l % 32, weight rows 32 t + 8 q + 4 (l / 32) + 0..3
+  auto gather = [&](int t, int m, int q, int l, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = 0.0f;
+    for (int wv = 0; wv < kWaves; ++wv) {
+      const float* src = red + (size_t)wv * (kWaveLds / 4) +
+                         ((t * kMB + m) * 16 + q * 4) * 64 + l;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += src[i * 64];
+    }
+  };
+  const uint16_t* bias = reinterpret_cast<const uint16_t*>(p.bias);
+  uint16_t* out = reinterpret_cast<uint16_t*>(p.out);
+  if (MODE == kGeluPair) {
+    // tile 0 = 32 rows of the gate half, tile 1 = the same rows of the up half
+    static_assert(MODE != kGeluPair || NT == 2, "pairs need two tiles");
+    const int half = p.N / 2;
+    for (int qd = threadIdx.x; qd < kMB * 4 * 64; qd += kWaves * 64) {
+      const int l = qd & 63, q = (qd >> 6) & 3, m = qd >> 8;
+      const int row = 32 * m + (l & 31);
+      const int col = block * 32 + 8 * q + 4 * (l >> 5);
+      if (row >= M) continue;
+      float gate[4], up[4];
+      gather(0, m, q, l, gate);
+      gather(NT - 1, m, q, l, up);
+      if (bias) {
+        float bg[4], bu[4];
+        unpack4(*reinterpret_cast<const u32x2*>(bias + col), bg);
+        unpack4(*reinterpret_cast<const u32x2*>(bias + half + col), bu);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          gate[i] += bg[i];
+          up[i] += bu[i];
+        }
+      }
+      const u32x2 ov = {gelu_mul_bf16x2(pack_bf16x2(up[0], up[1]),
+                                        pack_bf16x2(gate[0], gate[1])),
+                        gelu_mul_bf16x2(pack_bf16x2(up[2], up[3]),
+                                        pack_bf16x2(gate[2], gate[3]))};
+      *reinterpret_cast<u32x2*>(out + (size_t)row * half + col) = ov;
+    }
+    return;
+  }
+  for (int qd = threadIdx.x; qd < NT * kMB * 4 * 64; qd += kWaves * 64) {
+    const int l = qd & 63, q = (qd >> 6) & 3, m = (qd >> 8) % kMB;
+    const int t = (qd >> 8) / kMB;
+    const int row = 32 * m + (l & 31);
+    const int col = (block * NT + t) * 32 + 8 * q + 4 * (l >> 5);
+    if (row >= M) continue;
+    float v[4];
+    gather(t, m, q, l, v);
+    if (MODE == kPartial) {
+      const f32x4 o = {v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<f32x4*>(p.partial +
+                                ((size_t)blockIdx.y * M + row) * p.N + col) = o;
+      continue;
+    }
+    if (bias) {
+      float b[4];
+      unpack4(*reinterpret_cast<const u32x2*>(bias + col), b);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += b[i];
+    }
+    const size_t at = out_index(row, col, M, p.group_width);
+    if (p.residual) {
+      float res[4];
+      unpack4(*reinterpret_cast<const u32x2*>(
+                  reinterpret_cast<const uint16_t*>(p.residual) + at), res);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = round_to_bf16(v[i]) + res[i];
+    }
+    const u32x2 ov = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    *reinterpret_cast<u32x2*>(out + at) = ov;
+  }
+}
+
 // XR: rows of x that are loaded and staged (M rounded up to 16, 32 or 64).
 // Every workgroup draws all of x beside its weights: 64 rows are twice the
 // bytes of one tile's weights, whether the rows exist or not.
 // BESIDE: the grid goes on behind the layer's workgroups with kCopiers that copy
 // p.copy_items: what the next launch reads while it overwrites the original.
 constexpr int kCopiers = 16;
+__device__ __forceinline__ void copy_beside(const LinearArgs& p) {
+  const u32x4* from = reinterpret_cast<const u32x4*>(p.copy_from);
+  u32x4* to = reinterpret_cast<u32x4*>(p.copy_to);
+  constexpr int64_t step = kCopiers * kWaves * 64;
+  for (int64_t i = (int64_t)(gridDim.x - 1 - blockIdx.x) * (kWaves * 64) + threadIdx.x;
+       i < p.copy_items; i += step)
+    to[i] = from[i];
+}
 
 template <int NT, int MODE, int XR, bool BESIDE>
 __global__ void __launch_bounds__(kWaves * 64)
 linear_rows_kernel(LinearArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   if (BESIDE && blockIdx.x >= gridDim.x - kCopiers) {
-    const u32x4* from = reinterpret_cast<const u32x4*>(p.copy_from);
-    u32x4* to = reinterpret_cast<u32x4*>(p.copy_to);
-    constexpr int64_t step = kCopiers * kWaves * 64;
-    for (int64_t i = (int64_t)(gridDim.x - 1 - blockIdx.x) * (kWaves * 64) + threadIdx.x;
-         i < p.copy_items; i += step)
-      to[i] = from[i];
+    copy_beside(p);
     return;
   }
+  if (MODE == kPartial && p.clear && blockIdx.x + blockIdx.y == 0 && threadIdx.x < kNormFlags)
+    p.clear[threadIdx.x] = 0;
   constexpr int kLoads = XR / 8;          // of x per chunk
   constexpr int kMB = XR > 32 ? 2 : 1;    // blocks of 32 result rows
   constexpr int kWaveLds = wave_lds_bytes(NT, kMB);
@@ -176,92 +280,170 @@ linear_rows_kernel(LinearArgs p) {
     }
   }
 
-  // the waves' partial sums meet in LDS (each wave's region is its own x tile)
-  float* mine = reinterpret_cast<float*>(smem + (size_t)wave * kWaveLds);
+  add_up_and_store<NT, MODE, XR>(p, smem, wave, lane, blockIdx.x, acc);
+}
+
+// The norm in front of such layers and the layers as one launch: what a decode step has
+// twice in a block.  As launches of their own the norm is 2.5 us of launch and 2 of
+// latencies in which nothing else happens, and the layer's first weights are asked for
+// behind it.  Here the first M workgroups norm a row each (of what the layer before left
+// as partial sums), while the others have all of their weights on their way -- the CPW
+// chunks of 64 that a wave has of K, in registers -- and wait for the rows, which the norms'
+// workgroups report in a.flags.  Rows and flags are written and read at agent
+// scope (a row's stores have arrived before its flag is stored): no fence, which cost 0.3
+// to 0.7 us.
+// Every wait ends: a workgroup that has looked `patience` times in vain (the norms'
+// workgroups, the first of the grid, are not running) norms all rows itself, which writes
+// the same bytes once more.
+// What bounds it: launch, norm, stores, flag, loads of x one behind the other, 9 us, and
+// from 12 MB or so of weights on those.  us a norm and layer, K 2560, replayed from a graph
+// over 16 sets of weights, two launches / one: N 5120 at 1, 16, 32 rows 9.9 / 7.9, 11.7 /
+// 8.9, 13.4 / 10.3; N 3072 10.3 / 7.9, 11.6 / 8.7, 12.7 / 9.9; pairs of N 15360 18.8 /
+// 16.2, 18.1 / 16.5, 19.6 / 18.6.
+template <int NT, int MODE, int XR, int CPW, bool BESIDE>
+__global__ void __launch_bounds__(kWaves * 64)
+linear_rows_normed_kernel(NormedLinearArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ float norm_sums[4];
+  __shared__ int all_there;
+  const LinearArgs& p = a.layer;
+  const int M = p.M;
+  const int tid = threadIdx.x;
+  constexpr int K = CPW * kWaves * 64;
+  const auto norm_row = [&](int row) {
+    PartialRows part;
+    part.sums = reinterpret_cast<const f32x4*>(a.sums);
+    part.slices = a.slices;
+    part.slice_stride = (int64_t)M * K / 4;
+    part.bias = reinterpret_cast<const u32x4*>(a.bias);
+    const u32x4* const scale = reinterpret_cast<const u32x4*>(a.scale);
+    u32x4* const sum_out = reinterpret_cast<u32x4*>(a.sum_out);
+    u32x4* const out = reinterpret_cast<u32x4*>(a.normed);
+    if (a.addend)
+      rms_norm_row<true, true, true>(tid, row, norm_sums, nullptr, part,
+                                     reinterpret_cast<const u32x4*>(a.addend), scale,
+                                     sum_out, out, K / 8, 1.0f / (float)K, a.eps);
+    else
+      rms_norm_row<false, true, true>(tid, row, norm_sums, nullptr, part, nullptr, scale,
+                                      sum_out, out, K / 8, 1.0f / (float)K, a.eps);
+    // (the agent-scope stores have arrived when they are counted)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+  if ((int)blockIdx.x < M) {
+    if (tid >= 256) return;
+    norm_row(blockIdx.x);
+    __syncthreads();
+    if (tid == 0)
+      __hip_atomic_store(a.flags + blockIdx.x, 1u, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  if (BESIDE && blockIdx.x >= gridDim.x - kCopiers) {
+    copy_beside(p);
+    return;
+  }
+  const int block = blockIdx.x - M;
+  constexpr int kLoads = XR / 8;
+  constexpr int kMB = XR > 32 ? 2 : 1;
+  constexpr int kWaveLds = wave_lds_bytes(NT, kMB);
+  // chunks of x on their way beside the weights
+  constexpr int kAhead = XR == 16 ? (NT == 1 ? CPW : 3) : XR == 32 ? 2 : 1;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int r = lane & 31, g = lane >> 5;
+  const int c0 = wave * CPW;
+  uint16_t* xs = reinterpret_cast<uint16_t*>(smem + (size_t)wave * kWaveLds);
+  const u32x4* wg[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    wg[t] = reinterpret_cast<const u32x4*>(p.w_packed) +
+            ((size_t)(block * NT + t) * (K / 16) + c0 * 4) * 64 + lane;
+  Frag wq[CPW][NT][4];
+  auto load_weights = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        wq[c][t][k].u = __builtin_nontemporal_load(wg[t] + (c * 4 + k) * 64);
+  };
+#pragma unroll
+  for (int c = 0; c < CPW; ++c) load_weights(c);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- the rows ------------------------------------------------------------------
+  if (wave == 0) {
+    int polls = 0;
+    bool there = false;
+    for (;;) {
+      uint32_t flag = 1;
+      if (lane < M)
+        flag = __hip_atomic_load(a.flags + lane, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+      there = __all(flag != 0);
+      if (there || ++polls > a.patience) break;
+    }
+    if (lane == 0) all_there = there;
+  }
+  lds_barrier();
+  if (__builtin_expect(!all_there, 0)) {
+    for (int row = 0; row < M; ++row) {
+      if (tid < 256)
+        norm_row(row);
+      else
+        __syncthreads();  // (the norm's one)
+      __syncthreads();
+    }
+    // (once more: kept across the norm they are registers too many)
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) load_weights(c);
+  }
+
+  const int xrow = lane >> 3, xseg = lane & 7;
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, (uint32_t)M * K * 2u);
+  u32x4 xr[kAhead][kLoads];
+  // (rows past the last read as zeros)
+  auto load_x = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j)
+      xr[c % kAhead][j] = __builtin_amdgcn_raw_buffer_load_b128(
+          rx, (uint32_t)((8 * j + xrow) * K + (c0 + c) * 64 + 8 * xseg) * 2u, 0,
+          kAgentScope);
+  };
+  f32x16 acc[NT][kMB];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int m = 0; m < kMB; ++m)
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        mine[((t * kMB + m) * 16 + i) * 64 + lane] = acc[t][m][i];
-  lds_barrier();
-  const float* red = reinterpret_cast<const float*>(smem);
-  // sum of accumulator registers 4 q .. 4 q + 3 of (tile t, half m, lane l):
-  // result rows 32 m + l % 32, weight rows 32 t + 8 q + 4 (l / 32) + 0..3
-  auto gather = [&](int t, int m, int q, int l, float (&v)[4]) {
+      for (int i = 0; i < 16; ++i) acc[t][m][i] = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = 0.0f;
-    for (int wv = 0; wv < kWaves; ++wv) {
-      const float* src = red + (size_t)wv * (kWaveLds / 4) +
-                         ((t * kMB + m) * 16 + q * 4) * 64 + l;
+  for (int c = 0; c < kAhead; ++c) load_x(c);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] += src[i * 64];
-    }
-  };
-  const uint16_t* bias = reinterpret_cast<const uint16_t*>(p.bias);
-  uint16_t* out = reinterpret_cast<uint16_t*>(p.out);
-  if (MODE == kGeluPair) {
-    // tile 0 = 32 rows of the gate half, tile 1 = the same rows of the up half
-    static_assert(MODE != kGeluPair || NT == 2, "pairs need two tiles");
-    const int half = p.N / 2;
-    for (int qd = threadIdx.x; qd < kMB * 4 * 64; qd += kWaves * 64) {
-      const int l = qd & 63, q = (qd >> 6) & 3, m = qd >> 8;
-      const int row = 32 * m + (l & 31);
-      const int col = blockIdx.x * 32 + 8 * q + 4 * (l >> 5);
-      if (row >= M) continue;
-      float gate[4], up[4];
-      gather(0, m, q, l, gate);
-      gather(NT - 1, m, q, l, up);
-      if (bias) {
-        float bg[4], bu[4];
-        unpack4(*reinterpret_cast<const u32x2*>(bias + col), bg);
-        unpack4(*reinterpret_cast<const u32x2*>(bias + half + col), bu);
+  for (int c = 0; c < CPW; ++c) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          gate[i] += bg[i];
-          up[i] += bu[i];
-        }
-      }
-      const u32x2 ov = {gelu_mul_bf16x2(pack_bf16x2(up[0], up[1]),
-                                        pack_bf16x2(gate[0], gate[1])),
-                        gelu_mul_bf16x2(pack_bf16x2(up[2], up[3]),
-                                        pack_bf16x2(gate[2], gate[3]))};
-      *reinterpret_cast<u32x2*>(out + (size_t)row * half + col) = ov;
-    }
-    return;
+    for (int j = 0; j < kLoads; ++j)
+      *reinterpret_cast<u32x4*>(xs + (8 * j + xrow) * kXStride + 8 * xseg) =
+          xr[c % kAhead][j];
+    Frag xf[4][kMB];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int m = 0; m < kMB; ++m)
+        xf[k][m].u = *reinterpret_cast<const u32x4*>(
+            xs + (32 * m + r) * kXStride + 16 * k + 8 * g);
+    if (c + kAhead < CPW) load_x(c + kAhead);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int m = 0; m < kMB; ++m)
+          acc[t][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              wq[c][t][k].v, xf[k][m].v, acc[t][m], 0, 0, 0);
   }
-  for (int qd = threadIdx.x; qd < NT * kMB * 4 * 64; qd += kWaves * 64) {
-    const int l = qd & 63, q = (qd >> 6) & 3, m = (qd >> 8) % kMB;
-    const int t = (qd >> 8) / kMB;
-    const int row = 32 * m + (l & 31);
-    const int col = (blockIdx.x * NT + t) * 32 + 8 * q + 4 * (l >> 5);
-    if (row >= M) continue;
-    float v[4];
-    gather(t, m, q, l, v);
-    if (MODE == kPartial) {
-      const f32x4 o = {v[0], v[1], v[2], v[3]};
-      *reinterpret_cast<f32x4*>(p.partial +
-                                ((size_t)blockIdx.y * M + row) * p.N + col) = o;
-      continue;
-    }
-    if (bias) {
-      float b[4];
-      unpack4(*reinterpret_cast<const u32x2*>(bias + col), b);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] += b[i];
-    }
-    const size_t at = out_index(row, col, M, p.group_width);
-    if (p.residual) {
-      float res[4];
-      unpack4(*reinterpret_cast<const u32x2*>(
-                  reinterpret_cast<const uint16_t*>(p.residual) + at), res);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = round_to_bf16(v[i]) + res[i];
-    }
-    const u32x2 ov = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-    *reinterpret_cast<u32x2*>(out + at) = ov;
-  }
+  add_up_and_store<NT, MODE, XR>(p, smem, wave, lane, block, acc);
 }
 
 // Sum of the K slices (in slice order), bias, optional residual; four columns
@@ -364,6 +546,28 @@ hipError_t launch_rows(const LinearArgs& a, dim3 grid, hipStream_t s) {
 // two tiles per workgroup once that still leaves a workgroup for most CUs
 bool two_tiles(int tiles) { return tiles % 2 == 0 && tiles / 2 >= 200; }
 
+template <int NT, int MODE, int XR, int CPW, bool BESIDE>
+hipError_t launch_normed_of(const NormedLinearArgs& a, int blocks, hipStream_t s) {
+  constexpr int lds = kWaves * wave_lds_bytes(NT, XR > 32 ? 2 : 1);
+  static OncePerDevice once;
+  const auto kernel = linear_rows_normed_kernel<NT, MODE, XR, CPW, BESIDE>;
+  hipError_t e = set_max_dynamic_lds(once, (const void*)kernel, lds);
+  if (e != hipSuccess) return e;
+  kernel<<<dim3((unsigned)(a.layer.M + blocks + (BESIDE ? kCopiers : 0))), kWaves * 64,
+           lds, s>>>(a);
+  return hipGetLastError();
+}
+constexpr int kNormedChunks = 5;  // of a wave: K 2560
+template <int NT, int MODE, bool BESIDE>
+hipError_t launch_normed_rows(const NormedLinearArgs& a, int blocks, hipStream_t s) {
+  constexpr int CPW = kNormedChunks;
+  if (a.layer.M <= 16) return launch_normed_of<NT, MODE, 16, CPW, BESIDE>(a, blocks, s);
+  if (NT == 2 || a.layer.M <= 32)
+    return launch_normed_of<NT, MODE, 32, CPW, BESIDE>(a, blocks, s);
+  // (pairs end at 32 rows: linear_rows_normed_serve)
+  return launch_normed_of<1, MODE == kGeluPair ? kStore : MODE, 64, CPW, BESIDE>(a, blocks, s);
+}
+
 }  // namespace
 
 // How many slices of K the grid takes: more than one only where the weight
@@ -411,6 +615,25 @@ hipError_t launch_linear_rows_beside(const LinearArgs& a, hipStream_t s) {
   if (two_tiles(tiles))
     return launch_rows<2, kStore, true>(a, dim3(tiles / 2 + kCopiers, 1), s);
   return launch_rows<1, kStore, true>(a, dim3(tiles + kCopiers, 1), s);
+}
+
+// Whether a layer (or layers packed together) with the norm in front of it is one launch:
+// K as the kernel is made for (a wave's weights fill its registers), single tiles, pairs
+// for up to 32 rows (us, two launches / one: N 5120 at 40, 64 rows 14.2 / 12.5, 16.2 /
+// 13.5, N 3072 14.1 / 12.1, 15.7 / 13.4; pairs of N 15360 21.6 / 22.0, 23.1 / 23.1: the
+// workgroups are more than the CUs).
+bool linear_rows_normed_serve(int M, int K, int N, int gelu_pair) {
+  return M > 0 && M <= (gelu_pair ? 32 : kNormFlags) &&
+         K == kNormedChunks * kWaves * 64 && N % 32 == 0 &&
+         (gelu_pair || !two_tiles(N / 32));
+}
+
+hipError_t launch_linear_rows_normed(const NormedLinearArgs& a, int gelu_pair,
+                                     hipStream_t s) {
+  const int tiles = a.layer.N / 32;
+  if (gelu_pair) return launch_normed_rows<2, kGeluPair, false>(a, tiles / 2, s);
+  return a.layer.copy_items ? launch_normed_rows<1, kStore, true>(a, tiles, s)
+                            : launch_normed_rows<1, kStore, false>(a, tiles, s);
 }
 
 }  // namespace rg

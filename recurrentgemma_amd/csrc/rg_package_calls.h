@@ -99,6 +99,25 @@ int rg_linear_rows_beside(const void* x, const void* w_packed, const void* bias,
                           int M, int K, int N, int groups, const void* from, void* to,
                           int64_t bytes, void* stream);
 
+/* rg_linear_rows_partial that also sets the RG_NORM_FLAGS words of `flags` to zero, for
+ * rg_linear_rows_normed: rg_add_rms_norm_partial of such sums (M rows of K; sum_out and
+ * normed are written whole) and rg_linear_rows of normed, without a residual, as one
+ * launch, with `bytes` copied as in rg_linear_rows_beside (0: none).  The flags serve one
+ * such launch.  patience: how often its workgroups look for the rows' norm before they
+ * form it themselves, at least a microsecond each.  out has the same bits as the two
+ * calls.  RG_ERR_UNSUPPORTED where *_serve says 0. */
+#define RG_NORM_FLAGS 64
+int rg_linear_rows_partial_flags(const void* x, const void* w_packed, void* partial,
+                                 uint32_t* flags, int M, int K, int N, int slices,
+                                 void* stream);
+int rg_linear_rows_normed_serve(int M, int K, int N, int gelu_pair);
+int rg_linear_rows_normed(const void* partial, int slices, const void* partial_bias,
+                          const void* addend, const void* scale, float eps, void* sum_out,
+                          void* normed, uint32_t* flags, const void* w_packed,
+                          const void* bias, void* out, int M, int K, int N, int groups,
+                          int gelu_pair, const void* from, void* to, int64_t bytes,
+                          int patience, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -211,6 +211,7 @@ class MLPBlock(nn.Module):
       return self._rows_down(hidden, (self.ffw_down.weight,),
                              (self.ffw_down.bias,), residual=residual)
     hidden = None
+    x = ops.formed(x)
     if (x.dim() > 1 and x.numel() > 64 * self.width and
         not compiled.tracing() and not modules._global_hooks() and
         modules._as_written(self.ffw_up, _StackedLinear)):
@@ -392,6 +393,7 @@ class LocalAttentionBlock(nn.Module):
       q = self._rows_q(x, (self.proj_q.weight,))
       k, v = self._rows_kv(x, (self.proj_k.weight, self.proj_v.weight))
     else:
+      x = ops.formed(x)
       q, k, v = modules.linears(x, self.proj_q, self.proj_k, self.proj_v)
     q = q.reshape(b, t, self.num_heads, self.head_dim)
     k = k.reshape(b, t, 1, self.head_dim)
@@ -534,6 +536,20 @@ class LocalAttentionBlock(nn.Module):
         num_tokens=torch.zeros([batch_size], dtype=torch.int32, device=device))
 
 
+def _norm_for(reader, norm, x, addend):
+  """(x + addend, norm of it) for a block that reads the norm: of partial sums,
+  left to the block's first layers to form in their own launch, as long as
+  nobody but the block's own code gets to see it."""
+  if (isinstance(x, ops.PartialSums) and x.flags is not None and
+      type(norm) is RMSNorm and "add_then_norm" not in norm.__dict__ and
+      not modules._global_hooks() and
+      any(modules._as_written(reader, kind) for kind in
+          (modules.RecurrentBlock, LocalAttentionBlock, MLPBlock))):
+    pending = ops.PendingNorm(x, addend, norm.scale, norm.eps)
+    return pending.total, pending
+  return norm.add_then_norm(x, addend)
+
+
 class ResidualBlock(nn.Module):
   """norm -> temporal block -> +x -> norm -> MLP -> +  (modules.py:763-932)."""
 
@@ -587,7 +603,7 @@ class ResidualBlock(nn.Module):
     that way for a decode step) -- or, with many rows, ops.PendingSum: that
     output and the skip connection before they are added."""
     if isinstance(x, ops.PartialSums):
-      x, normed = self.temporal_pre_norm.add_then_norm(x, None)
+      x, normed = _norm_for(self.temporal_block, self.temporal_pre_norm, x, None)
     elif isinstance(x, ops.PendingSum):
       x, normed = self.temporal_pre_norm.add_then_norm(x.a, x.b)
     else:
@@ -595,9 +611,11 @@ class ResidualBlock(nn.Module):
     mixed, new_cache = self.temporal_block(normed, segment_pos, cache,
                                            return_cache=return_cache,
                                            defer_out=True)
-    residual, normed = self.channel_pre_norm.add_then_norm(mixed, x)
-    return (self.mlp_block(normed, residual=residual, defer_out=defer_out),
-            new_cache)
+    ops.formed(normed)  # (and x with it, whoever has read it)
+    residual, normed = _norm_for(self.mlp_block, self.channel_pre_norm, mixed, x)
+    out = self.mlp_block(normed, residual=residual, defer_out=defer_out)
+    ops.formed(normed)
+    return out, new_cache
 
   @classmethod
   def init_cache(cls, batch_size, width, num_heads, attention_window_size,

@@ -257,7 +257,7 @@ class RecurrentBlock(nn.Module):
         else:
           y, x = self._rows_yx(x, (w_y, w_x), (b_y, b_x))
       else:
-        y, x = linears(x, self.linear_y, self.linear_x)
+        y, x = linears(ops.formed(x), self.linear_y, self.linear_x)
       # x * gelu(y) (modules.py:627-628, 644) is part of the core call: inside
       # the prefill kernel where that runs, one pass after it elsewhere
       x, new_cache = _recurrent_core(

@@ -698,24 +698,34 @@ def argmax_last(x):
   return out
 
 
-def _add_rms_norm_partial(ps, addend, scale, eps):
+def _partial_norm_args(ps, addend, scale):
+  """addend, scale of a norm of PartialSums, checked."""
   if ps.addend is not None:
     if addend is not None:
       raise ValueError("the partial sums already carry an addend")
     addend = ps.addend
-  slices, rows, width = ps.sums.shape
   scale = _dev(scale, "scale")
-  assert scale.shape == (width,) and scale.dtype == ps.dtype
+  assert scale.shape == ps.sums.shape[2:] and scale.dtype == ps.dtype
   if addend is not None:
     assert tuple(addend.shape) == tuple(ps.shape)
     _same(ps.dtype, ps.sums.device, addend=addend)
     addend = _dev(addend, "addend")
-  total = torch.empty(ps.shape, dtype=ps.dtype, device=ps.sums.device)
-  out = torch.empty_like(total)
+  return addend, scale
+
+
+def _launch_partial_norm(ps, addend, scale, total, out, eps):
+  slices, rows, width = ps.sums.shape
   with _on(total.device):
     _lib.check(_lib.lib().rg_add_rms_norm_partial(
         _p(ps.sums), slices, _p(ps.bias), _p(addend), _p(scale), _p(total),
         _p(out), rows, width, eps, _DTYPES[ps.dtype], _stream(total)))
+
+
+def _add_rms_norm_partial(ps, addend, scale, eps):
+  addend, scale = _partial_norm_args(ps, addend, scale)
+  total = torch.empty(ps.shape, dtype=ps.dtype, device=ps.sums.device)
+  out = torch.empty_like(total)
+  _launch_partial_norm(ps, addend, scale, total, out, eps)
   return total, out
 
 
@@ -1025,22 +1035,72 @@ def packed_gate_weights(w_x, w_a):
   return packed
 
 
+NORM_FLAGS = 64  # RG_NORM_FLAGS
+# How often a workgroup looks for a norm that others of its launch form, before
+# it forms the norm itself: some 0.3 ms.
+NORM_PATIENCE = 512
+
+
 class PartialSums:
   """The output of a linear layer that has not been added up yet: fp32 partial
   sums over slices of K (PackedLinear.partial), its bias, and optionally a
   tensor still to be added (a skip connection).  `add_rms_norm` takes it in
   place of a tensor; `materialize()` gives the tensor it stands for."""
 
-  def __init__(self, sums, bias, shape, dtype, addend=None):
+  def __init__(self, sums, bias, shape, dtype, addend=None, flags=None):
     self.sums, self.bias = sums, bias    # [slices, M, N] float32, [N] | None
     self.shape, self.dtype = shape, dtype  # of the tensor this stands for
     self.addend = addend
+    # address of NORM_FLAGS words, kept by `sums`, that the launch set to zero:
+    # for one PendingNorm
+    self.flags = flags
+
+  def take_flags(self):
+    flags, self.flags = self.flags, None
+    return flags
 
   def materialize(self):
     out = (self.sums.sum(0) if self.bias is None
            else self.sums.sum(0) + self.bias.float())
     out = out.to(self.dtype).reshape(self.shape)
     return out if self.addend is None else out + self.addend
+
+
+class PendingNorm:
+  """add_rms_norm of PartialSums, not formed yet: the few-row layers that read
+  the norm next do it in their own launch (PackedLinear), `tensor()` in one of
+  its own.  total: the sum that was normed, good from then on."""
+
+  is_cuda = True
+
+  def __init__(self, sums, addend, scale, eps):
+    self.args = _partial_norm_args(sums, addend, scale)
+    self.sums, self.eps = sums, eps
+    self.shape, self.dtype = torch.Size(sums.shape), sums.dtype
+    self.device = sums.sums.device
+    self.flags = sums.take_flags()
+    self.total = torch.empty(self.shape, dtype=self.dtype, device=self.device)
+    self.out = torch.empty_like(self.total)
+    self.formed = False
+
+  def numel(self):
+    return self.out.numel()
+
+  def dim(self):
+    return len(self.shape)
+
+  def tensor(self):
+    if not self.formed:
+      addend, scale = self.args
+      _launch_partial_norm(self.sums, addend, scale, self.total, self.out,
+                           self.eps)
+      self.formed = True
+    return self.out
+
+
+def formed(x):
+  """x, or what a PendingNorm stands for."""
+  return x.tensor() if isinstance(x, PendingNorm) else x
 
 
 class PendingSum:
@@ -1173,7 +1233,7 @@ class PackedLinear:
                                       self.partial_slices(x, K, N))
       if sums is not None:
         return PartialSums(sums, self._bias, (*x.shape[:-1], N), x.dtype,
-                           addend)
+                           addend, sums.data_ptr() + 4 * sums.numel())
     x = _dev(x, "x")
     self._prepare(weights, biases)
     N, K, groups = self._shape
@@ -1181,11 +1241,59 @@ class PackedLinear:
     slices = self.partial_slices(x, K, N)
     assert slices > 0
     M = x.numel() // K
-    sums = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+    n = slices * M * N
+    every = torch.empty(n + NORM_FLAGS, dtype=torch.float32, device=x.device)
+    sums = every[:n].view(slices, M, N)
     with _on(x.device):
-      _lib.check(_lib.lib().rg_linear_rows_partial(
-          _p(x), _p(self._packed), _p(sums), M, K, N, slices, _stream(x)))
-    return PartialSums(sums, self._bias, (*x.shape[:-1], N), x.dtype, addend)
+      _lib.check(_lib.lib().rg_linear_rows_partial_flags(
+          _p(x), _p(self._packed), _p(sums), sums.data_ptr() + 4 * n, M, K, N,
+          slices, _stream(x)))
+    return PartialSums(sums, self._bias, (*x.shape[:-1], N), x.dtype, addend,
+                       sums.data_ptr() + 4 * n)
+
+  @torch.no_grad()
+  def _with_norm(self, x, weights, biases, state=None):
+    """The layers' outputs, as __call__ and beside return them, and x's norm in
+    one launch, or None where that is not one."""
+    if x.formed or x.flags is None:
+      return None
+    self._prepare(weights, biases)
+    N, K, groups = self._shape
+    M = x.numel() // K
+    lib = _lib.lib()
+    if (x.shape[-1] != K or x.dtype != weights[0].dtype or
+        x.device != weights[0].device or
+        not lib.rg_linear_rows_normed_serve(M, K, N, int(self.gelu_pair))):
+      return None
+    copied, aside = 0, None
+    if state is not None:
+      copied = state.numel() * state.element_size()
+      if (self.gelu_pair or groups == 1 or copied == 0 or copied % 16 or
+          not state.is_contiguous() or state.device != x.device or
+          state.data_ptr() % 16):
+        return None
+      aside = torch.empty_like(state)
+    lead = x.shape[:-1]
+    stacked = groups > 1 and not self.gelu_pair
+    if stacked:
+      shape = (groups, *lead, N // groups)
+    else:
+      shape = (*lead, N // 2 if self.gelu_pair else N)
+    out = torch.empty(shape, dtype=x.dtype, device=x.device)
+    addend, scale = x.args
+    sums = x.sums
+    with _on(x.device):
+      _lib.check(lib.rg_linear_rows_normed(
+          _p(sums.sums), sums.sums.shape[0], _p(sums.bias), _p(addend),
+          _p(scale), x.eps, _p(x.total), _p(x.out), x.flags, _p(self._packed),
+          _p(self._bias), _p(out), M, K, N, groups if stacked else 1,
+          int(self.gelu_pair), _p(state), _p(aside), copied, NORM_PATIENCE,
+          _stream(out)))
+    x.formed = True
+    outs = tuple(out[i] for i in range(groups)) if stacked else (out,)
+    if state is not None:
+      return (*outs, aside)
+    return outs if stacked else out
 
   @torch.no_grad()
   def beside(self, x, weights, biases, state):
@@ -1194,13 +1302,24 @@ class PackedLinear:
     (outputs .., copy), or None where that is not to be had."""
     if self._plan is None:
       return None
+    if isinstance(x, PendingNorm):
+      out = self._with_norm(x, weights, biases, state)
+      if out is not None:
+        return out
+      x = x.tensor()
     return _lib.host().rows_linear(self._plan, x, weights, biases, None, state)
 
   @torch.no_grad()
   def __call__(self, x, weights, biases=None, residual=None):
     """x [..., K].  Returns out [..., N] (one layer), a tuple of outputs
     (several layers / a stacked weight), or the gelu pair product [..., N/2].
-    residual (one layer only): added after the output is rounded."""
+    residual (one layer only): added after the output is rounded.  x may be a
+    PendingNorm, which is formed on the way."""
+    if isinstance(x, PendingNorm):
+      out = None if residual is not None else self._with_norm(x, weights, biases)
+      if out is not None:
+        return out
+      x = x.tensor()
     if self._plan is not None:
       out = _lib.host().rows_linear(self._plan, x, weights, biases, residual)
       if out is not None:
