@@ -37,7 +37,8 @@ union Frag {
 
 constexpr int kXStride = 72;  // elements per staged x row: 64 + 8 of padding
 constexpr int kWaves = 8;
-constexpr int kAgentScope = 16;  // sc1 of a buffer instruction (gfx950)
+// of buffer instructions (gfx950)
+constexpr int kAgentScope = 16, kNonTemporal = 2;
 
 // LDS of a wave: its x tile (whole blocks of 32 rows) or its sums.
 __host__ __device__ constexpr int wave_lds_bytes(int nt, int blocks) {
@@ -62,8 +63,8 @@ __device__ __forceinline__ size_t out_index(int m, int n, int M, int gw) {
 }
 
 // From the waves' accumulators to the layer's outputs: the sums over K meet in LDS, then
-// the epilogue.  block: which NT tiles of weight rows.
-template <int NT, int MODE, int XR>
+// the epilogue.  block: which NT tiles of weight rows or, HALF, which half of a tile.
+template <int NT, int MODE, int XR, bool HALF>
 __device__ __forceinline__ void add_up_and_store(
     const LinearArgs& p, unsigned char* const smem, const int wave, const int lane,
     const int block, const f32x16 (&acc)[NT][XR > 32 ? 2 : 1]) {
@@ -125,11 +126,14 @@ __device__ __forceinline__ void add_up_and_store(
     }
     return;
   }
-  for (int qd = threadIdx.x; qd < NT * kMB * 4 * 64; qd += kWaves * 64) {
-    const int l = qd & 63, q = (qd >> 6) & 3, m = (qd >> 8) % kMB;
-    const int t = (qd >> 8) / kMB;
+  static_assert(!HALF || (NT == 1 && MODE == kStore), "");
+  constexpr int kQuads = HALF ? 2 : 4;  // of 8 weight rows
+  for (int qd = threadIdx.x; qd < NT * kMB * kQuads * 64; qd += kWaves * 64) {
+    const int l = qd & 63, m = qd / (64 * kQuads) % kMB;
+    const int q = (qd >> 6) % kQuads + (HALF ? (block & 1) * 2 : 0);
+    const int t = qd / (64 * kQuads) / kMB;
     const int row = 32 * m + (l & 31);
-    const int col = (block * NT + t) * 32 + 8 * q + 4 * (l >> 5);
+    const int col = (HALF ? block >> 1 : block * NT + t) * 32 + 8 * q + 4 * (l >> 5);
     if (row >= M) continue;
     float v[4];
     gather(t, m, q, l, v);
@@ -173,7 +177,9 @@ __device__ __forceinline__ void copy_beside(const LinearArgs& p) {
     to[i] = from[i];
 }
 
-template <int NT, int MODE, int XR, bool BESIDE>
+// HALF: a workgroup has half a tile of weight rows (the matrix instructions run with zeros
+// in place of the others, which gives the same bits).
+template <int NT, int MODE, int XR, bool BESIDE, bool HALF>
 __global__ void __launch_bounds__(kWaves * 64)
 linear_rows_kernel(LinearArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -212,7 +218,13 @@ linear_rows_kernel(LinearArgs p) {
 #pragma unroll
   for (int t = 0; t < NT; ++t)
     wg[t] = reinterpret_cast<const u32x4*>(p.w_packed) +
-            ((size_t)(blockIdx.x * NT + t) * (K / 16)) * 64 + lane;
+            ((size_t)((HALF ? blockIdx.x >> 1 : blockIdx.x) * NT + t) * (K / 16)) * 64 +
+            lane;
+  // (the other half's lanes lie outside the descriptor: zeros, and nothing is fetched)
+  const __amdgpu_buffer_rsrc_t tile_rows =
+      make_rsrc(wg[0] - lane, HALF ? (uint32_t)K * 64u : 0u);
+  const uint32_t in_tile =
+      (r >> 4) == (int)(blockIdx.x & 1) ? 16u * (uint32_t)lane : kBufferOutOfRange;
 
   f32x16 acc[NT][kMB];
 #pragma unroll
@@ -233,7 +245,9 @@ linear_rows_kernel(LinearArgs p) {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
         wq[slot][t][k].u =
-            __builtin_nontemporal_load(wg[t] + (size_t)(c * 4 + k) * 64);
+            HALF ? __builtin_amdgcn_raw_buffer_load_b128(
+                       tile_rows, in_tile + (uint32_t)(c * 4 + k) * 1024u, 0, kNonTemporal)
+                 : __builtin_nontemporal_load(wg[t] + (size_t)(c * 4 + k) * 64);
   };
   auto body = [&](int slot, int c, bool more) {
 #pragma unroll
@@ -280,7 +294,7 @@ linear_rows_kernel(LinearArgs p) {
     }
   }
 
-  add_up_and_store<NT, MODE, XR>(p, smem, wave, lane, blockIdx.x, acc);
+  add_up_and_store<NT, MODE, XR, HALF>(p, smem, wave, lane, blockIdx.x, acc);
 }
 
 // The norm in front of such layers and the layers as one launch: what a decode step has
@@ -443,7 +457,7 @@ linear_rows_normed_kernel(NormedLinearArgs a) {
           acc[t][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               wq[c][t][k].v, xf[k][m].v, acc[t][m], 0, 0, 0);
   }
-  add_up_and_store<NT, MODE, XR>(p, smem, wave, lane, block, acc);
+  add_up_and_store<NT, MODE, XR, false>(p, smem, wave, lane, block, acc);
 }
 
 // Sum of the K slices (in slice order), bias, optional residual; four columns
@@ -514,14 +528,14 @@ linear_pack_kernel(const uint16_t* __restrict__ w, u32x4* __restrict__ packed,
   packed[idx] = v;
 }
 
-template <int NT, int MODE, int XR, bool BESIDE>
+template <int NT, int MODE, int XR, bool BESIDE, bool HALF>
 hipError_t launch_rows_of(const LinearArgs& a, dim3 grid, hipStream_t s) {
   constexpr int lds = kWaves * wave_lds_bytes(NT, XR > 32 ? 2 : 1);
   static OncePerDevice once;  // one per instantiation of this launcher
   hipError_t e = set_max_dynamic_lds(
-      once, (const void*)linear_rows_kernel<NT, MODE, XR, BESIDE>, lds);
+      once, (const void*)linear_rows_kernel<NT, MODE, XR, BESIDE, HALF>, lds);
   if (e != hipSuccess) return e;
-  linear_rows_kernel<NT, MODE, XR, BESIDE><<<grid, kWaves * 64, lds, s>>>(a);
+  linear_rows_kernel<NT, MODE, XR, BESIDE, HALF><<<grid, kWaves * 64, lds, s>>>(a);
   return hipGetLastError();
 }
 
@@ -536,15 +550,23 @@ hipError_t launch_rows_of(const LinearArgs& a, dim3 grid, hipStream_t s) {
 // (8 staged rows are within 2 % of 16.  Fewer rows without the barrier are
 // slower than 64, 10.0 us for one row at 2560 x 2560: the compiler moves the
 // loads behind the products.)
-template <int NT, int MODE, bool BESIDE = false>
+template <int NT, int MODE, bool BESIDE = false, bool HALF = false>
 hipError_t launch_rows(const LinearArgs& a, dim3 grid, hipStream_t s) {
-  if (a.M <= 16) return launch_rows_of<NT, MODE, 16, BESIDE>(a, grid, s);
-  if (a.M <= 32) return launch_rows_of<NT, MODE, 32, BESIDE>(a, grid, s);
-  return launch_rows_of<NT, MODE, 64, BESIDE>(a, grid, s);
+  if (a.M <= 16) return launch_rows_of<NT, MODE, 16, BESIDE, HALF>(a, grid, s);
+  if (a.M <= 32) return launch_rows_of<NT, MODE, 32, BESIDE, HALF>(a, grid, s);
+  return launch_rows_of<NT, MODE, 64, BESIDE, HALF>(a, grid, s);
 }
 
 // two tiles per workgroup once that still leaves a workgroup for most CUs
 bool two_tiles(int tiles) { return tiles % 2 == 0 && tiles / 2 >= 200; }
+// Half a tile while there is a CU for each: what a workgroup draws is what bounds it.  us a
+// layer, replayed from a graph over 16 sets of weights, whole / half tiles:
+//   rows                     1           16           32           64
+//   K 2560, N 2560     6.0 /  5.5   7.1 /  6.1   8.4 /  7.4  10.6 /  9.8
+//   K 2560, N 4096     6.4 /  5.9   7.4 /  6.4   8.8 /  7.8  11.0 / 10.3
+//   K 4096, N 4096     9.6 /  8.5   9.9 /  8.5  11.5 / 10.1  14.6 / 13.6
+//   K 1024, N 2048     4.1 /  3.8   4.2 /  3.9   4.7 /  4.3   5.8 /  5.6
+bool half_tiles(int tiles) { return 2 * tiles <= 256; }
 
 template <int NT, int MODE, int XR, int CPW, bool BESIDE>
 hipError_t launch_normed_of(const NormedLinearArgs& a, int blocks, hipStream_t s) {
@@ -605,6 +627,8 @@ hipError_t launch_linear_rows(const LinearArgs& a, int gelu_pair,
     return hipGetLastError();
   }
   if (two_tiles(tiles)) return launch_rows<2, kStore>(a, dim3(tiles / 2, 1), s);
+  if (half_tiles(tiles))
+    return launch_rows<1, kStore, false, true>(a, dim3(2 * tiles, 1), s);
   return launch_rows<1, kStore>(a, dim3(tiles, 1), s);
 }
 

@@ -124,6 +124,23 @@ def test_layers_packed_together():
     ops.PackedLinear()(x, (w1, w2[:40]), (b1, b2[:40]))
 
 
+@pytest.mark.parametrize("N", [32, 2560, 4096])
+@pytest.mark.parametrize("M", [1, 16, 17, 64])
+@pytest.mark.parametrize("K", [64, 2560])
+def test_half_tiles_equal_whole_ones(M, K, N):
+  """Up to 4096 weight rows a workgroup has 16 of them, beyond 32: a layer alone
+  and the same one packed in front of another."""
+  g = torch.Generator().manual_seed(M + K + N)
+  x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+  w = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+  more = (torch.randn(4160, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+  b, c = (torch.randn(n, generator=g).bfloat16().to(DEV) for n in (N, 4160))
+  alone = ops.PackedLinear()(x, (w,), (b,))
+  both = ops.PackedLinear()(x, (w, more), (b, c))
+  assert torch.equal(alone, both[:, :N])
+  _check(alone, x.cpu(), w.cpu(), b.cpu())
+
+
 @pytest.mark.parametrize("M,K,E", [(64, 2560, 7680), (3, 128, 96)])
 def test_stacked_weight_and_gelu_pairs(M, K, E):
   """The MLP's stacked up-projection [2, K, E] (Einsum "cdD" layout): plain
