@@ -127,6 +127,8 @@ PACKAGE_SIGNATURES = {
     "rg_linear_back": (_i, [_vp] * 5 + [_i64, _i, _i, _i, _vp]),
     "rg_linear_weight_grads": (_i, [_vp] * 5 + [_i, _i64, _i, _vp]),
     "rg_linear_rows_beside": (_i, [_vp] * 4 + [_i] * 4 + [_vp, _vp, _i64, _vp]),
+    "rg_recurrent_step_join": (_i, [_vp, _vp, _vp, _i] + [_vp] * 13 +
+                               [_sz, _i, _i, _i, _i, _vp]),
     "rg_linear_rows_partial_flags": (_i, [_vp] * 4 + [_i] * 4 + [_vp]),
     "rg_linear_rows_normed_serve": (_i, [_i] * 4),
     "rg_linear_rows_normed": (_i, [_vp, _i, _vp, _vp, _vp, ctypes.c_float] + [_vp] * 6 +

@@ -137,12 +137,15 @@ PyObject* recurrent_step(PyObject*, PyObject* const* v, Py_ssize_t n) {
       ws = c.empty({(int64_t)bytes}, at::kByte);
       void* wp = ws.mutable_data_ptr();
       launch([&] {
-        const int rc = rg_recurrent_step(
+        if (gate)
+          return rg_recurrent_step_join(
+              x, gate, pos, is64, conv_in, cp, (const float*)h_in, (float*)hp, conv_w,
+              conv_b, wx, b_x, wa, b_a, a_param, yp, wp, bytes, (int)B, (int)W, (int)H,
+              c.code, s);
+        return rg_recurrent_step(
             x, pos, is64, conv_in, cp, (const float*)h_in, (float*)hp, conv_w,
             conv_b, wx, b_x, wa, b_a, a_param, yp, wp, bytes, (int)B, (int)W,
             (int)H, c.code, s);
-        if (rc != RG_OK || !gate) return rc;
-        return rg_gelu_mul(yp, gate, yp, B * W, c.code, s);
       });
       return triple(y, h, conv);
     }

@@ -1072,6 +1072,45 @@ size_t rg_recurrent_step_workspace_bytes(int B, int W, int dtype) {
   return 3 * one;
 }
 
+// The float32 step as one launch, where the arguments are as that takes them (any other
+// call, those with an argument that is refused among them, takes the three).
+static bool step_f32_args(const void* x, const void* gate_branch, const void* segpos,
+                          int segpos_is_i64, const void* conv_cache_in,
+                          void* conv_cache_out, const void* h_in, void* h_out,
+                          const void* conv_w, const void* conv_b, const void* w_x,
+                          const void* b_x, const void* w_a, const void* b_a,
+                          const void* a_param, void* y, int B, int W, int H, int dtype,
+                          rg::StepF32Args* a) {
+  if (dtype != RG_DTYPE_F32 || B <= 0 || H <= 0) return false;
+  const void* const all[] = {x,   segpos, conv_cache_in, conv_cache_out, h_in,
+                             h_out, conv_w, conv_b,      w_x,            b_x,
+                             w_a, b_a,    a_param,       y};
+  for (const void* p : all)
+    if (p == nullptr || !aligned16(p)) return false;
+  if (!aligned16(gate_branch)) return false;
+  *a = rg::StepF32Args{};
+  a->x = (const float*)x;
+  a->segpos = segpos;
+  a->seg_kind = segpos_is_i64 ? 1 : 0;
+  a->cache_in = (const float*)conv_cache_in;
+  a->cache_out = (float*)conv_cache_out;
+  a->h_in = (const float*)h_in;
+  a->h_out = (float*)h_out;
+  a->conv_w = (const float*)conv_w;
+  a->conv_b = (const float*)conv_b;
+  a->w[0] = (const float*)w_x;
+  a->w[1] = (const float*)w_a;
+  a->b[0] = (const float*)b_x;
+  a->b[1] = (const float*)b_a;
+  a->a_param = (const float*)a_param;
+  a->y = (float*)y;
+  a->gate_branch = (const float*)gate_branch;
+  a->B = B;
+  a->W = W;
+  a->H = H;
+  return rg::block_step_f32_serves(*a);
+}
+
 int rg_recurrent_step(const void* x, const void* segpos, int segpos_is_i64,
                       const void* conv_cache_in, void* conv_cache_out,
                       const void* h_in, void* h_out, const void* conv_w,
@@ -1092,6 +1131,11 @@ int rg_recurrent_step(const void* x, const void* segpos, int segpos_is_i64,
     return fail(RG_ERR_WORKSPACE,
                 "%s: workspace of %zu bytes (16-byte aligned) required, got %zu",
                 __func__, need, workspace ? workspace_bytes : (size_t)0);
+  rg::StepF32Args a;
+  if (step_f32_args(x, nullptr, segpos, segpos_is_i64, conv_cache_in, conv_cache_out, h_in,
+                    h_out, conv_w, conv_b, w_x, b_x, w_a, b_a, a_param, y, B, W, H, dtype,
+                    &a))
+    return launch_status(__func__, rg::launch_block_step_f32(a, (hipStream_t)stream));
   const size_t one = need / 3;
   char* ws = (char*)workspace;
   void* xc = ws;
@@ -1106,6 +1150,28 @@ int rg_recurrent_step(const void* x, const void* segpos, int segpos_is_i64,
   return rg_lru_scan_fused(xc, 0, nullptr, nullptr, gx, ga, a_param, segpos,
                            segpos_is_i64, h_in, y, h_out, nullptr, B, 1, W,
                            dtype, stream);
+}
+
+int rg_recurrent_step_join(const void* x, const void* gate_branch, const void* segpos,
+                           int segpos_is_i64, const void* conv_cache_in,
+                           void* conv_cache_out, const void* h_in, void* h_out,
+                           const void* conv_w, const void* conv_b, const void* w_x,
+                           const void* b_x, const void* w_a, const void* b_a,
+                           const void* a_param, void* y, void* workspace,
+                           size_t workspace_bytes, int B, int W, int H, int dtype,
+                           void* stream) {
+  RG_CHECK_PTR(gate_branch);
+  rg::StepF32Args a;
+  if (W > 0 &&
+      step_f32_args(x, gate_branch, segpos, segpos_is_i64, conv_cache_in, conv_cache_out,
+                    h_in, h_out, conv_w, conv_b, w_x, b_x, w_a, b_a, a_param, y, B, W, H,
+                    dtype, &a))
+    return launch_status(__func__, rg::launch_block_step_f32(a, (hipStream_t)stream));
+  const int rc = rg_recurrent_step(x, segpos, segpos_is_i64, conv_cache_in, conv_cache_out,
+                                   h_in, h_out, conv_w, conv_b, w_x, b_x, w_a, b_a,
+                                   a_param, y, workspace, workspace_bytes, B, W, H, dtype,
+                                   stream);
+  return rc == RG_OK ? rg_gelu_mul(y, gate_branch, y, (int64_t)B * W, dtype, stream) : rc;
 }
 
 int rg_recurrent_step_static(const void* x, const void* segpos,

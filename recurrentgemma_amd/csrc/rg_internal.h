@@ -149,6 +149,25 @@ struct StepArgs {
   int B, W, H;
 };
 
+// The float32 step in one launch (rg_step_f32.hip): as StepArgs, weights [H, 256, 256].
+struct StepF32Args {
+  const float* x;
+  const void* segpos;
+  int seg_kind;
+  const float* cache_in;
+  float* cache_out;
+  const float* h_in;
+  float* h_out;
+  const float* conv_w;
+  const float* conv_b;
+  const float* w[2];
+  const float* b[2];
+  const float* a_param;
+  float* y;
+  const float* gate_branch;
+  int B, W, H;
+};
+
 // Prompt-pass attention (rg_attention_prefill.hip).
 struct AttnPrefillArgs {
   const void* q;    // [B, T, H, 256] bf16, after the rotary embedding
@@ -432,6 +451,8 @@ hipError_t launch_linear_rows(const LinearArgs& a, int gelu_pair,
 hipError_t launch_linear_rows_beside(const LinearArgs& a, hipStream_t s);
 // Only the fp32 partial sums a.partial[slices][M][N] of x @ W^T, K split in
 // `slices`; rg_elementwise.hip's norm kernel takes them from there.
+bool block_step_f32_serves(const StepF32Args& a);
+hipError_t launch_block_step_f32(const StepF32Args& a, hipStream_t s);
 bool linear_rows_normed_serve(int M, int K, int N, int gelu_pair);
 hipError_t launch_linear_rows_normed(const NormedLinearArgs& a, int gelu_pair,
                                      hipStream_t s);

@@ -99,6 +99,17 @@ int rg_linear_rows_beside(const void* x, const void* w_packed, const void* bias,
                           int M, int K, int N, int groups, const void* from, void* to,
                           int64_t bytes, void* stream);
 
+/* rg_recurrent_step and rg_gelu_mul of its y with gate_branch [B,1,W], one launch where
+ * the step is one (float32, 256-wide heads, nothing written that is read). */
+int rg_recurrent_step_join(const void* x, const void* gate_branch, const void* segpos,
+                           int segpos_is_i64, const void* conv_cache_in,
+                           void* conv_cache_out, const void* h_in, void* h_out,
+                           const void* conv_w, const void* conv_b, const void* w_x,
+                           const void* b_x, const void* w_a, const void* b_a,
+                           const void* a_param, void* y, void* workspace,
+                           size_t workspace_bytes, int B, int W, int H, int dtype,
+                           void* stream);
+
 /* rg_linear_rows_partial that also sets the RG_NORM_FLAGS words of `flags` to zero, for
  * rg_linear_rows_normed: rg_add_rms_norm_partial of such sums (M rows of K; sum_out and
  * normed are written whole) and rg_linear_rows of normed, without a residual, as one
