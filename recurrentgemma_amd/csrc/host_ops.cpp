@@ -15,6 +15,8 @@
 // has to.
 //
 // Plain C++ on torch's and this library's public interfaces; no device code.
+#include <ATen/autocast_mode.h>
+
 #include "host_call.h"
 #include "rg_package_calls.h"
 
@@ -370,7 +372,7 @@ PyObject* rows_partial(PyObject*, PyObject* const* v, Py_ssize_t n) {
 
 // A parameter of an nn.Module, past the attribute lookup that is written in
 // Python; anything but a module that holds it itself takes the general path.
-const Tensor& parameter(PyObject* module, PyObject* name) {
+PyObject* parameters(PyObject* module) {
   static PyObject* const key = PyUnicode_InternFromString("_parameters");
   PyObject* own = PyObject_GetAttr(module, key);
   if (!own) {
@@ -378,6 +380,10 @@ const Tensor& parameter(PyObject* module, PyObject* name) {
     throw Fallback{};
   }
   Py_DECREF(own);  // (the module keeps it)
+  return own;
+}
+const Tensor& parameter(PyObject* module, PyObject* name) {
+  PyObject* own = parameters(module);
   need(PyDict_CheckExact(own));
   PyObject* t = PyDict_GetItemWithError(own, name);
   if (!t) PyErr_Clear();
@@ -514,6 +520,116 @@ PyObject* block_step(PyObject*, PyObject* const* v, Py_ssize_t n) {
   });
 }
 
+// ------------------------------------------------- a prompt's attention --
+
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+// LocalAttentionBlock on a prompt without a cache (bf16, 256-wide heads, more rows than
+// the few-row kernels take): projections, rotary embedding, attention, ring cache and
+// proj_final, each where and as modules.linears and ops.attention_prompt would run it.
+// As calls from Python it was 75 to 90 us of host time, which prompts of up to some 900
+// tokens in all waited for: us a call, before and after, width 2560, 1 x 135 tokens
+// 77 / 42, 7 x 72 88 / 54, 10 x 91 89 / 70, 7 x 739 165 / 164; width 4096, 1 x 300 89 / 69.
+// (the block's _modules, x, segment_pos, inv_freq, first_key, heads, window, scale,
+//  return_cache) -> (out, ring keys | None, ring values | None, num_tokens | None) | None
+PyObject* attention_prompt(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    need(n == 9);
+#define RG_NAME(ID, TEXT) \
+  static PyObject* const ID = PyUnicode_InternFromString(TEXT);
+    RG_NAME(k_q, "proj_q") RG_NAME(k_k, "proj_k") RG_NAME(k_v, "proj_v")
+    RG_NAME(k_final, "proj_final") RG_NAME(k_weight, "weight") RG_NAME(k_bias, "bias")
+#undef RG_NAME
+    PyObject *m_q = child(v[0], k_q), *m_k = child(v[0], k_k), *m_v = child(v[0], k_v),
+             *m_final = child(v[0], k_final);
+    for (PyObject* m : {m_q, m_k, m_v}) need(child(parameters(m), k_bias) == Py_None);
+    const Tensor &w_q = parameter(m_q, k_weight), &w_k = parameter(m_k, k_weight),
+                 &w_v = parameter(m_v, k_weight), &w_o = parameter(m_final, k_weight),
+                 &b_o = parameter(m_final, k_bias);
+    Call c(v[1]);
+    need(c.code == RG_DTYPE_BF16 && c.x.dim() == 3 && c.x.numel() > 0 &&
+         !at::autocast::is_autocast_enabled(at::kCUDA));
+    const int64_t B = c.x.size(0), T = c.x.size(1), W = c.x.size(2), rows = B * T;
+    const long H = PyLong_AsLong(v[5]), window = PyLong_AsLong(v[6]);
+    const double scale = PyFloat_AsDouble(v[7]);
+    if (PyErr_Occurred()) throw Raised{};
+    constexpr int64_t kHead = 256;
+    need(H > 0 && window > 0 && W == H * kHead && B <= INT32_MAX && T * H * 512 < INT32_MAX &&
+         window <= INT32_MAX);
+    need(shape_is(w_q, {W, W}) && shape_is(w_k, {kHead, W}) && shape_is(w_v, {kHead, W}) &&
+         shape_is(w_o, {W, W}) && shape_is(b_o, {W}));
+    void* x = c(v[1]);
+    int is64;
+    void* pos = c.positions(v[2], B, T, &is64);
+    const float* inv = (const float*)c.f32(v[3], {kHead / 4});
+    const Tensor& first = tensor_of(v[4]);
+    need(shape_is(first, {B, T}));
+    const int32_t* first_key = (const int32_t*)dense(first, at::kInt, c.device);
+    for (const Tensor* t : {&w_q, &w_k, &w_v, &w_o, &b_o}) dense(*t, c.dtype, c.device);
+    void* s = c.stream();
+
+    const int n_qkv[3] = {(int)W, (int)kHead, (int)kHead}, n_out[1] = {(int)W};
+    const bool qkv_ours = rg_linear_many_pays(rows, (int)W, 3, n_qkv, c.code);
+    const bool out_ours = rg_linear_many_pays(rows, (int)W, 1, n_out, c.code);
+    Tensor q, k, val, attended = c.empty({B, T, W}), out, ring_k, ring_v, count;
+    if (qkv_ours) {
+      q = c.empty({B, T, W});
+      k = c.empty({B, T, kHead});
+      val = c.empty({B, T, kHead});
+    } else {
+      NoGil free;
+      q = at::linear(c.x, w_q);
+      k = at::linear(c.x, w_k);
+      val = at::linear(c.x, w_v);
+    }
+    if (v[8] == Py_True) {
+      ring_k = c.empty({B, window, 1, kHead});
+      ring_v = c.empty({B, window, 1, kHead});
+      count = c.empty({B}, at::kInt);
+    }
+    if (out_ours) out = c.empty({B, T, W});
+    Tensor ws = c.empty({(int64_t)rg_attention_prompt_workspace_bytes((int)B, (int)T)},
+                        at::kByte);
+    auto at_of = [](Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; };
+    void *qp = at_of(q), *kp = at_of(k), *vp = at_of(val), *ap = at_of(attended),
+         *op = at_of(out), *rk = at_of(ring_k), *rv = at_of(ring_v), *np = at_of(count),
+         *wp = at_of(ws);
+    const void* const w3[3] = {w_q.const_data_ptr(), w_k.const_data_ptr(),
+                               w_v.const_data_ptr()};
+    const void* const w1[1] = {w_o.const_data_ptr()};
+    const void* const b1[1] = {b_o.const_data_ptr()};
+    // (another thread may replace a parameter while this one is without the interpreter)
+    const Tensor keep[] = {w_q, w_k, w_v, w_o, b_o};
+    launch([&] {
+      if (qkv_ours) {
+        void* const to[3] = {qp, kp, vp};
+        const int rc =
+            rg_linear_many(x, rows, (int)W, 3, w3, nullptr, to, n_qkv, c.code, s);
+        if (rc != RG_OK) return rc;
+      }
+      const int rc = rg_attention_prompt(
+          qp, kp, vp, pos, is64, inv, first_key, ap, rk, rv, (int32_t*)np, wp, (int)B,
+          (int)T, (int)H, (int)kHead, (int)window, (float)scale, c.code, s);
+      if (rc != RG_OK || !out_ours) return rc;
+      void* const to[1] = {op};
+      return rg_linear_many(ap, rows, (int)W, 1, w1, b1, to, n_out, c.code, s);
+    });
+    if (!out_ours) {
+      NoGil free;
+      out = at::linear(attended, keep[3], keep[4]);
+    }
+    PyObject* t = PyTuple_New(4);
+    if (!t) throw Raised{};
+    int i = 0;
+    for (const Tensor* each : {&out, &ring_k, &ring_v, &count})
+      PyTuple_SET_ITEM(t, i++, wrap(*each));
+    return t;
+  });
+}
+
 PyObject* set_kernel_error(PyObject*, PyObject* type) {
   Py_INCREF(type);
   Py_XDECREF(g_kernel_error);
@@ -525,6 +641,7 @@ PyMethodDef kMethods[] = {
     {"recurrent_step", (PyCFunction)(void*)recurrent_step, METH_FASTCALL, ""},
     {"recurrent_core", (PyCFunction)(void*)recurrent_core, METH_FASTCALL, ""},
     {"block_step", (PyCFunction)(void*)block_step, METH_FASTCALL, ""},
+    {"attention_prompt", (PyCFunction)(void*)attention_prompt, METH_FASTCALL, ""},
     {"rows_plan", (PyCFunction)(void*)rows_plan, METH_FASTCALL, ""},
     {"rows_linear", (PyCFunction)(void*)rows_linear, METH_FASTCALL, ""},
     {"rows_partial", (PyCFunction)(void*)rows_partial, METH_FASTCALL, ""},

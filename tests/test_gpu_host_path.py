@@ -5,6 +5,7 @@ weights that were written to."""
 import pytest
 import torch
 
+import recurrentgemma_amd as rg
 from oracle import torch_ref as R
 from recurrentgemma_amd import _lib
 from recurrentgemma_amd import ops
@@ -78,3 +79,39 @@ def test_native_linear_rows_follow_their_weights():
   assert _lib.host().rows_linear(layer._plan, x, (w,), (b,), None) is None
   want = (x.double() @ w.double().T + b.double())
   assert helpers.max_rel(layer(x, (w,), (b,)), want) < 1e-2
+
+
+@pytest.mark.parametrize("B,T,H,window,positions", [
+    (1, 65, 10, 2048, torch.int32), (7, 72, 10, 64, torch.int64),
+    (3, 43, 2, 2048, torch.int32), (130, 1, 2, 8, torch.int32),
+    (1, 700, 16, 500, torch.int32), (2, 1201, 1, 2048, torch.int64)])
+def test_attention_prompts_natively(B, T, H, window, positions):
+  W = 256 * H
+  torch.manual_seed(8)
+  block = rg.LocalAttentionBlock(width=W, num_heads=H, window_size=window,
+                                 device=DEV, dtype=torch.bfloat16)
+  with torch.no_grad():
+    block.proj_final.bias.normal_()
+  x = torch.randn(B, T, W, device=DEV).bfloat16()
+  pos = helpers.document_positions(B, T, 40, seed=9).to(positions).to(DEV)
+  with pytest.MonkeyPatch.context() as patch:
+    patch.setattr(rg.LocalAttentionBlock, "_prompt_natively",
+                  lambda *a: None)
+    general = block(x, pos)
+  assert block._prompt_natively(_strided(x), pos, True) is None
+  assert block._prompt_natively(x, pos, True) is not None
+  out, cache = block(x, pos)
+  assert torch.equal(out, general[0])
+  for got, want in zip(cache, general[1]):
+    assert got.dtype == want.dtype and torch.equal(got, want)
+  alone, none = block(x, pos, return_cache=False)
+  assert none is None and torch.equal(alone, general[0])
+  # what is not a plain layer of the block's own takes the general path
+  seen = []
+  hook = block.proj_k.register_forward_hook(lambda *a: seen.append(1))
+  # (other sums in front of four bf16 roundings, 2^-8 of the largest each)
+  assert helpers.max_rel(block(x, pos)[0], general[0]) < 4 * 2**-8
+  assert seen
+  hook.remove()
+  block.proj_q.bias = torch.nn.Parameter(torch.ones(W, device=DEV).bfloat16())
+  assert block._prompt_natively(x, pos, True) is None
