@@ -113,9 +113,16 @@ constexpr size_t kEpiBytesPerWave = 32ull * kEpiStride;
 constexpr size_t kBiasLdsOffset = kStageLdsBytes + 8 * kEpiBytesPerWave;
 constexpr size_t kMfmaLdsBytes = kBiasLdsOffset + 8 * 64 * sizeof(float);
 
+// LDS row of weights (elements) while they are laid out: 16 banks beyond a multiple
+// of all 64.
+constexpr int kWeightStride = 288;
+static_assert(128 * kWeightStride * sizeof(uint16_t) <= kMfmaLdsBytes, "");
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 union Frag {
   bf16x8 v;
-  uint16_t u[8];
+  s16x4 h[2];
   f32x4 q;
 };
 
@@ -147,41 +154,6 @@ __global__ void __launch_bounds__(512) gates_mfma_bf16_kernel(GemmArgs p) {
                       (!NARROW || (wave & 3) * 64 < p.bw);
   const int ksteps = NARROW ? (p.bw + 15) / 16 : 16;  // k-steps with a row < bw
   const int n0 = (wave & 3) * 64;     // first output column inside the gate
-  // The weights are [k][n] with n contiguous, the MFMA B operand wants 8
-  // consecutive k per lane: transpose through LDS, 128 k-rows of one gate at
-  // a time (coalesced 16-byte global reads, 2-byte LDS reads).
-  Frag bfrag[16][2];
-#pragma unroll
-  for (int g = 0; g < (ONE ? 1 : 2); ++g) {
-#pragma unroll
-    for (int kh = 0; kh < 2; ++kh) {
-      // (a head narrower than the 256 x 256 tile -- bw a multiple of 8 --
-      // is padded with zeros: rows and columns from bw on)
-      const uint16_t* src =
-          (const uint16_t*)p.w[g] + ((int64_t)h * bw + kh * 128) * bw;
-      for (int e = tid; e < 128 * 32; e += 512) {
-        const int r = e >> 5, q = e & 31;
-        f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (kh * 128 + r < bw && q * 8 < bw)
-          v = *reinterpret_cast<const f32x4*>(src + (size_t)r * bw + q * 8);
-        *reinterpret_cast<f32x4*>(lds + (size_t)r * kLdsStride + q * 8) = v;
-      }
-      __syncthreads();
-      if (gate == g) {
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
-#pragma unroll
-          for (int nt = 0; nt < 2; ++nt) {
-            const int n = n0 + nt * 32 + (lane & 31);
-            const int kb = ks * 16 + 8 * (lane >> 5);
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              bfrag[kh * 8 + ks][nt].u[e] = lds[(size_t)(kb + e) * kLdsStride + n];
-          }
-      }
-      __syncthreads();
-    }
-  }
   // The MFMAs compute the transposed block (weights as the A operand): lane l
   // then holds, for x row l%32, the channels 8*g + 4*(l/32) + 0..3 of each
   // 32-channel block, g = 0..3, i.e. four adjacent channels per register
@@ -385,6 +357,59 @@ __global__ void __launch_bounds__(512) gates_mfma_bf16_kernel(GemmArgs p) {
   if (tile < ntiles) {
     fetch_seg(tile);
     fetch_rows(tile);
+  }
+  // The weights are [k][n] with n contiguous, the MFMA B operand wants 8
+  // consecutive k per lane: transposed on their way through LDS, 128 k-rows of
+  // one gate at a time, by reads that hand out columns (four rows by 16 columns
+  // to 16 lanes; rows of LDS 16 banks apart, so that the 32 lanes of a k-half
+  // meet no bank twice).  The next 128 rows are on their way meanwhile.  (With
+  // 2-byte reads this was most of a launch over few rows.)
+  Frag bfrag[16][2];
+  {
+    constexpr int kRounds = ONE ? 2 : 4;
+    f32x4 v[8];
+    auto request = [&](int round) {
+      // (a head narrower than the 256 x 256 tile -- bw a multiple of 8 --
+      // is padded with zeros: rows and columns from bw on)
+      const int k0 = (round & 1) * 128;
+      const uint16_t* src =
+          (const uint16_t*)p.w[round >> 1] + ((int64_t)h * bw + k0) * bw;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = (tid >> 5) + 16 * i, q = tid & 31;
+        v[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (k0 + r < bw && q * 8 < bw)
+          v[i] = *reinterpret_cast<const f32x4*>(src + (size_t)r * bw + q * 8);
+      }
+    };
+    request(0);
+#pragma unroll
+    for (int round = 0; round < kRounds; ++round) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        *reinterpret_cast<f32x4*>(
+            lds + ((tid >> 5) + 16 * i) * kWeightStride + (tid & 31) * 8) = v[i];
+      if (round + 1 < kRounds) request(round + 1);
+      lds_barrier();
+      if (gate == round >> 1) {
+        const uint16_t* const at =
+            lds + (8 * (lane >> 5) + ((lane & 15) >> 2)) * kWeightStride + n0 +
+            (lane & 16) + 4 * (lane & 3);
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+              bfrag[(round & 1) * 8 + ks][nt].h[half] =
+                  __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                      (lds_s16x4*)(at + (16 * ks + 4 * half) * kWeightStride +
+                                   32 * nt));
+      }
+      lds_barrier();
+    }
+  }
+  if (tile < ntiles) {
     stage_begin(tile);
 #pragma unroll
     for (int j = 0; j < kRaw; ++j) stage_row(j, 0, WithCuts{});

@@ -53,24 +53,6 @@ gates_dgrad_kernel(const uint16_t* __restrict__ dgx,
   const int range = blockIdx.x / H;
   const int64_t tiles = (M + kRows - 1) / kRows;
 
-  // weights: fragment f = 16 gate + k-step
-#pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    const uint16_t* src = (half ? w_a : w_x) +
-                          ((int64_t)h * kBW + 32 * wave + (lane & 31)) * kBW +
-                          8 * (lane >> 5);
-    f32x4 w[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-      w[k] = *reinterpret_cast<const f32x4*>(src + 16 * k);
-    asm volatile("" ::"v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]),
-                 "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]),
-                 "v"(w[10]), "v"(w[11]), "v"(w[12]), "v"(w[13]), "v"(w[14]),
-                 "v"(w[15]));
-#pragma unroll
-    for (int k = 0; k < 16; ++k) set_weight_frag(16 * half + k, w[k]);
-  }
-
   const uint32_t row_bytes = 2u * (uint32_t)W;
   // rows of one tile -> LDS: a wave-wide load covers one row's 512 bytes of
   // either gate in one half of the lanes each; chunk p of row r holds the
@@ -101,6 +83,23 @@ gates_dgrad_kernel(const uint16_t* __restrict__ dgx,
   int64_t tile = range;
   int buf = 0;
   request(tile, 0);
+  // weights: fragment f = 16 gate + k-step
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    const uint16_t* src = (half ? w_a : w_x) +
+                          ((int64_t)h * kBW + 32 * wave + (lane & 31)) * kBW +
+                          8 * (lane >> 5);
+    f32x4 w[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+      w[k] = *reinterpret_cast<const f32x4*>(src + 16 * k);
+    asm volatile("" ::"v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]),
+                 "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]),
+                 "v"(w[10]), "v"(w[11]), "v"(w[12]), "v"(w[13]), "v"(w[14]),
+                 "v"(w[15]));
+#pragma unroll
+    for (int k = 0; k < 16; ++k) set_weight_frag(16 * half + k, w[k]);
+  }
   const uint32_t patch = kPatchOff + wave * 16 * kPatchFloats * 4;
   for (; tile < tiles; tile += ranges, buf ^= 1) {
     // this tile's rows are in LDS (every wave waits for its own loads), and
