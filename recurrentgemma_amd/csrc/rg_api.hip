@@ -665,10 +665,12 @@ static CorePlan core_plan(int B, int T, int W, int H, int dtype) {
   // again for every pair it runs, and with a few tokens per row that
   // outweighs the rest (us, single / pair: 640 pairs T1 37/28, T16 40/36, T32
   // 42/48; 1280 pairs T16 68/47, T32 70/66, T48 72/85; 2560 pairs T1 122/28,
-  // T32 136/112, T48 138/146).
+  // T32 136/112, T48 138/146).  Narrower heads are in slices there, and rows of up to 16
+  // tokens, with re-laid-out weights, several to a tile (prefill_many_serve; W5632 H32 B64
+  // T27 81 apart, 46 in slices).
   const int64_t pairs = (int64_t)B * H;
   const bool many_short_rows =
-      (pairs > 512 && T <= 16) || (pairs > 1024 && T <= 32);
+      (pairs > 512 && T <= 16) || (W / H == 256 && pairs > 1024 && T <= 32);
   // (narrower heads: where the form in slices is ahead of gate GEMM + scan)
   p.single = fits && !many_short_rows &&
              (W / H == 256 || rg::prefill_narrow_pays(B, H, T, W));
@@ -841,7 +843,9 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
     a.H = H;
     return launch_status(
         __func__, rg::launch_core_f32_small(a, (hipStream_t)stream));
-  } else if (p.single) {
+  } else if (p.single || (w_packed != nullptr && dtype == RG_DTYPE_BF16 &&
+                          rg::prefill_many_serve(B, H, T, W / H,
+                                                 gate_branch != nullptr))) {
     // the join is part of the kernel's output stage, for rows in chunks too
     // (the launches that write y apply it)
     const size_t relay_bytes = p.relay_bytes[gate_branch != nullptr];

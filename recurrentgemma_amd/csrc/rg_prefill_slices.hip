@@ -112,6 +112,14 @@ struct TileAt {
   bool any;     // false: past the workgroup's rows
   bool active;  // ... and this wave's channels are channels of the head
   uint32_t starts;
+  int tokens;   // of its row (MANY: of the rows that lie in it)
+};
+
+// Several whole rows to a tile (MANY): how many, and of the tile's tokens those that
+// open a row and those that end one; token i is in the tile's row i * inverse >> 16.
+struct RowsOfTile {
+  int rows;
+  uint32_t opens, ends, inverse;
 };
 
 // From a tile's pre-activations (a lane: 16 tokens of one channel, runs of four
@@ -120,16 +128,18 @@ struct TileAt {
 // four tiles, replay, stores.  c0: this wave's first channel among the workgroup's,
 // n0: in the head.  until: how many tiles after the pass's
 // first the next row opens (0: that one does), kept up to date here.
-template <class L, bool GELU>
+template <class L, bool GELU, bool MANY>
 __device__ __forceinline__ void gate_and_scan(
-    const FusedArgs& p, lds_byte* const lds3, const int lane, const int wave,
+    const FusedArgs& p, const RowsOfTile& many, lds_byte* const lds3, const int lane, const int wave,
     const int bw, const int h, const int n0, const int c0, const int tt,
     const int buf, const int tiles_per_row, const TileAt at_tile,
     const f32x16& acc_x, const f32x16& acc_a, float& carry, int& until) {
-  const int T = p.T;
+  const int T = MANY ? at_tile.tokens : p.T;
   const int64_t W = p.W;
   const uint32_t row_bytes = 2u * (uint32_t)p.W;
   const uint32_t seq_bytes = (uint32_t)T * row_bytes;
+  const int64_t seq_at =
+      (int64_t)at_tile.row * (MANY ? many.rows * p.T : p.T) * row_bytes;
   const int b = at_tile.row, t0 = at_tile.t0, k_in_row = at_tile.k_in_row;
   const bool any = at_tile.any, active = at_tile.active;
   const uint32_t starts = at_tile.starts;
@@ -153,7 +163,7 @@ __device__ __forceinline__ void gate_and_scan(
       u32x4 gate_rows[2];
       if (GELU) {
         const __amdgpu_buffer_rsrc_t rgate =
-            make_rsrc((const char*)p.gate_branch + (int64_t)b * seq_bytes,
+            make_rsrc((const char*)p.gate_branch + seq_at,
                       is_gelu_row ? seq_bytes : 0);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -204,16 +214,55 @@ __device__ __forceinline__ void gate_and_scan(
 #pragma unroll
       for (int e = 0; e < 16; ++e)
         xn[e] *= __builtin_amdgcn_sqrtf(__builtin_fmaf(-av[e], av[e], 1.0f));
+      // MANY: a row that opens in the tile starts from its h0, and is cut from the row
+      // before by selection, here and below (runs of four tokens: uniformly).
+      // (masks of this lane's tokens, made where they are used: a comparison per
+      // element kept across the pass is scalar registers too many)
+      uint32_t opens = 0, first_token = 0;
+      auto lane_masks = [&]() RG_INLINE {
+        if (MANY) {
+          first_token = (uint32_t)(ln >> 5) * 4u;
+          asm volatile("" : "+v"(first_token));
+          opens = many.opens >> first_token;
+        }
+      };
+      if (MANY) {
+        if (p.h0) {
+          lane_masks();
+          const __amdgpu_buffer_rsrc_t rh0 =
+              make_rsrc(p.h0 + (int64_t)b * many.rows * W,
+                        active ? (uint32_t)(T / p.T) * 2u * row_bytes : 0u);
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const uint32_t row = 8 * (e >> 2) + (e & 3);
+            const uint32_t in_tile = (row + first_token) * many.inverse >> 16;
+            if (e % 4 == 0) asm volatile("" ::: "memory");
+            const float h0 = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(
+                           rh0,
+                           (opens >> row) & 1u
+                               ? in_tile * 2u * row_bytes + state_off
+                               : kBufferOutOfRange,
+                           0, 0));
+            xn[e] = (opens >> row) & 1u ? __builtin_fmaf(av[e], h0, xn[e]) : xn[e];
+          }
+        }
+      }
+      auto walk = [&](int e, float state) RG_INLINE {
+        const float next = __builtin_fmaf(av[e], state, xn[e]);
+        return MANY && ((opens >> (8 * (e >> 2) + (e & 3))) & 1u) ? xn[e] : next;
+      };
 
       // ---- the tile as (prod a, state from zero): runs of four tokens, of the
       //      lower and the upper lanes in turn ---------------------------------
       float run_p[4][2], run_h[4][2];  // [run][lane half]
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
+        lane_masks();
         float ph = xn[4 * g], pp = av[4 * g];
 #pragma unroll
         for (int q = 1; q < 4; ++q) {
-          ph = __builtin_fmaf(av[4 * g + q], ph, xn[4 * g + q]);
+          ph = walk(4 * g + q, ph);
           pp *= av[4 * g + q];
         }
         const auto sp = __builtin_amdgcn_permlane32_swap(
@@ -225,18 +274,22 @@ __device__ __forceinline__ void gate_and_scan(
         run_h[g][0] = __uint_as_float(sh[0]);
         run_h[g][1] = __uint_as_float(sh[1]);
       }
+      auto walk_run = [&](int g, int s, float state) RG_INLINE {
+        const float next = __builtin_fmaf(run_p[g][s], state, run_h[g][s]);
+        return MANY && ((many.opens >> (8 * g + 4 * s)) & 15u) ? run_h[g][s] : next;
+      };
       float tp = 1.0f, th = 0.0f;
 #pragma unroll
       for (int g = 0; g < 4; ++g)
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-          th = __builtin_fmaf(run_p[g][s], th, run_h[g][s]);
+          th = walk_run(g, s, th);
           tp *= run_p[g][s];
         }
       // a tile that opens its row starts from the row's h0 instead of from zero
       if (k_in_row == 0) {
         const float first =
-            p.h0 && any && ch_valid
+            !MANY && p.h0 && any && ch_valid
                 ? *reinterpret_cast<const float*>(
                       (const char*)(p.h0 + (int64_t)b * W) + state_off)
                 : 0.0f;
@@ -275,20 +328,35 @@ __device__ __forceinline__ void gate_and_scan(
       if (active) {
         // ---- replay -------------------------------------------------------------
         const __amdgpu_buffer_rsrc_t ry =
-            make_rsrc((char*)p.y + (int64_t)b * seq_bytes, seq_bytes);
+            make_rsrc((char*)p.y + seq_at, seq_bytes);
+        const __amdgpu_buffer_rsrc_t rlast =
+            make_rsrc(p.h_last + (MANY ? (int64_t)b * many.rows * W : 0),
+                      MANY && p.h_last ? (uint32_t)(T / p.T) * 2u * row_bytes : 0u);
         float s = hin;
         float behind = hin;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const float before = s;
-          s = __builtin_fmaf(run_p[g][0], s, run_h[g][0]);
+          s = walk_run(g, 0, s);
           float hh = ln >= 32 ? s : before;
-          s = __builtin_fmaf(run_p[g][1], s, run_h[g][1]);
+          s = walk_run(g, 1, s);
           float hv[4];
+          lane_masks();
+          const uint32_t ends = MANY ? many.ends >> first_token : 0u;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            hh = __builtin_fmaf(av[4 * g + q], hh, xn[4 * g + q]);
+            hh = walk(4 * g + q, hh);
             hv[q] = hh;
+            if (MANY) {  // (rows past the last, tokens that end none: dropped)
+              const uint32_t row = 8 * g + q;
+              const uint32_t in_tile = (row + first_token) * many.inverse >> 16;
+              __builtin_amdgcn_raw_buffer_store_b32(
+                  __float_as_uint(hh), rlast,
+                  ((ends >> row) & 1u) && ch_valid
+                      ? in_tile * 2u * row_bytes + state_off
+                      : kBufferOutOfRange,
+                  0, 0);
+            }
           }
           behind = hh;
           const uint32_t y01 = pack_bf16x2(hv[0], hv[1]);
@@ -317,7 +385,7 @@ __device__ __forceinline__ void gate_and_scan(
         }
         // the row's last tile: its end state (identity past the end) -- the
         // upper lanes' last run is the tile's last
-        if (p.h_last && k_in_row == tiles_per_row - 1 && ln >= 32 &&
+        if (!MANY && p.h_last && k_in_row == tiles_per_row - 1 && ln >= 32 &&
             ch_valid)
           *reinterpret_cast<float*>((char*)(p.h_last + (int64_t)b * W) +
                                     state_off) = behind;
@@ -461,9 +529,13 @@ __device__ __forceinline__ void store_conv_state(const FusedArgs& p,
 // PACKED: gate weights in operand order (launch_pack_gate_weights), else as
 // the reference lays them out.  GELU: y leaves as y * gelu(gate_branch), the
 // block's join (recurrentgemma/torch/modules.py:627-628, 644).
-template <int KS, bool PACKED, bool GELU>
+// MANY: rows of at most 16 tokens, as many whole ones to a tile as go into it; what is
+// a row of the batch elsewhere is a tile here.  (A row to a tile leaves most of it empty:
+// figures at prefill_many_serve.)
+template <int KS, bool PACKED, bool GELU, bool MANY>
 __global__ void __launch_bounds__(kThreads)
-block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
+block_prefill_slices_bf16_kernel(FusedArgs p, RowsOfTile many, int slices, int groups) {
+  static_assert(PACKED || !MANY, "");
   using L = Layout<KS>;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   lds_byte* const lds3 = (lds_byte*)lds_raw;
@@ -481,15 +553,18 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
   const int slice = in_xcd % slices;
   const int h = pair / groups;
   const int group = pair - h * groups;
-  const int row0 = (int)((int64_t)group * p.B / groups);
-  const int row1 = (int)((int64_t)(group + 1) * p.B / groups);
-  const int T = p.T;
-  const int tiles_per_row = (T + kTile - 1) / kTile;
+  const int rows = MANY ? (p.B + many.rows - 1) / many.rows : p.B;
+  const int row0 = (int)((int64_t)group * rows / groups);
+  const int row1 = (int)((int64_t)(group + 1) * rows / groups);
+  const int row_tokens = MANY ? many.rows * p.T : p.T;
+  const int tiles_per_row = MANY ? 1 : (row_tokens + kTile - 1) / kTile;
   const int ntiles = (row1 - row0) * tiles_per_row;
   const int npasses = (ntiles + kTiles - 1) / kTiles;
+  auto tokens_of = [&](int row) {  // (the last tile of MANY may hold fewer rows)
+    return MANY && row + 1 == rows ? (p.B - row * many.rows) * p.T : row_tokens;
+  };
 
   const uint32_t row_bytes = 2u * (uint32_t)p.W;
-  const uint32_t seq_bytes = (uint32_t)T * row_bytes;  // < 2^31 (launcher)
   const bool seg_is64 = p.seg_kind == kSegI64;
   const uint32_t seg_esize = seg_is64 ? 8u : 4u;
 
@@ -530,7 +605,9 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
     const int b = any ? asked.row : row0;
     const int t0 = asked.k * kTile;
     step(asked);
-    const char* base = (const char*)p.x + (int64_t)b * seq_bytes;
+    const int T = tokens_of(b);
+    const uint32_t seq_bytes = (uint32_t)T * row_bytes;  // < 2^31 (launcher)
+    const char* base = (const char*)p.x + (int64_t)b * row_tokens * row_bytes;
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(base, any ? seq_bytes : 0);
     const __amdgpu_buffer_rsrc_t rhalo = make_rsrc(base, any && t0 ? seq_bytes : 0);
     // (the whole offset in the vector part, which the descriptor checks: rows
@@ -545,7 +622,7 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
     const int t = t0 + lane - 32;
     seg_in = any && t >= 0 && t < T;
     const char* seg_row =
-        (const char*)p.segpos + (int64_t)b * T * seg_esize;  // (uniform)
+        (const char*)p.segpos + (int64_t)b * row_tokens * seg_esize;  // (uniform)
     const uint32_t at = (uint32_t)(seg_in ? t : 0) * seg_esize;
     seg_lo = *reinterpret_cast<const uint32_t*>(seg_row + at);
     seg_hi = seg_is64 ? *reinterpret_cast<const uint32_t*>(seg_row + at + 4) : 0u;
@@ -555,9 +632,15 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
     return __ballot(seg_in && (seg_lo | seg_hi) == 0u);
   };
 
-  if (!PACKED) load_weights<KS, false>(p, lane, bw, h, n0);
+  // Where the conv is cut: bit j, row j - 3 of the tile
+  auto cuts_of = [&](uint64_t mask) RG_INLINE -> uint64_t {
+    return mask >> 29 | (MANY ? (uint64_t)many.opens << 3 : 0);
+  };
+
+  // (MANY: beside the first rows its registers do not suffice for the weights)
+  if (!PACKED || MANY) load_weights<KS, PACKED>(p, lane, bw, h, n0);
   request();
-  if (PACKED) load_weights<KS, true>(p, lane, bw, h, n0);
+  if (PACKED && !MANY) load_weights<KS, true>(p, lane, bw, h, n0);
   fill_taps<L>(p, lds_raw, tid, bw, h);
   if (tt == 0) fill_gate_values<L>(p, lds_raw, lane, bw, h, n0, half * 32);
   __syncthreads();  // taps, per-channel values
@@ -645,9 +728,9 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
       for (int j = 0; j < kConvRows / 2; ++j) conv_rows(c, buf, j);
     }
   };
-  convolve(0, mask >> 29);
+  convolve(0, cuts_of(mask));
   uint32_t starts = (uint32_t)(mask >> 32);
-  if (PACKED && npasses > 1) request();
+  if (PACKED && !MANY && npasses > 1) request();
   lds_barrier();
 
   const uint32_t a_lane =
@@ -669,17 +752,17 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
     step(now);
     // the next pass's conv between the matrix instructions, then the rows of
     // the one after
-    // (weights in the reference layout: the rare form, whose conv runs before
-    // the matrix instructions -- between them its registers do not suffice)
-    if (!PACKED && more) {
+    // (weights in the reference layout, and MANY, which has one pass or two: the conv
+    // runs before the matrix instructions -- between them registers do not suffice)
+    if ((!PACKED || MANY) && more) {
       request();
       mask = starts_mask();
-      convolve(buf ^ 1, mask >> 29);
+      convolve(buf ^ 1, cuts_of(mask));
     }
     f32x16 acc_x, acc_a;
-    if constexpr (PACKED && more) {
+    if constexpr (PACKED && !MANY && more) {
       mask = starts_mask();
-      const uint64_t cuts = mask >> 29;
+      const uint64_t cuts = cuts_of(mask);
       Conv c;
       conv_begin(c);
       matrix_tile<KS>(lds3, a_lane + buf * L::buffer, acc_x, acc_a, [&](auto KSTEP) RG_INLINE {
@@ -695,16 +778,19 @@ block_prefill_slices_bf16_kernel(FusedArgs p, int slices, int groups) {
     } else {
       matrix_tile<KS>(lds3, a_lane + buf * L::buffer, acc_x, acc_a, [](auto) RG_INLINE {});
     }
-    gate_and_scan<L, GELU>(
-        p, lds3, lane, wave, bw, h, n0, half * 32, tt, buf, tiles_per_row,
-        TileAt{b, t0, k_in_row, any, active, starts}, acc_x, acc_a, carry, until);
+    gate_and_scan<L, GELU, MANY>(
+        p, many, lds3, lane, wave, bw, h, n0, half * 32, tt, buf, tiles_per_row,
+        TileAt{b, t0, k_in_row, any, active, starts, tokens_of(b)}, acc_x, acc_a,
+        carry, until);
     starts = (uint32_t)(mask >> 32);
   };
   for (int i = 0; i + 1 < npasses; ++i) pass(i, std::true_type{});
   pass(npasses - 1, std::false_type{});
 
   if (p.cache_out)
-    store_conv_state<kSlice>(p, tid, bw, h, slice * kSlice, row0, row1);
+    store_conv_state<kSlice>(p, tid, bw, h, slice * kSlice,
+                             MANY ? row0 * many.rows : row0,
+                             MANY ? min(row1 * many.rows, p.B) : row1);
 }
 
 // Heads of at most 176 channels (the paper presets): two slices of 96, and the
@@ -1241,15 +1327,15 @@ Split best_split(int B, int H, int T, int slices, int tiles, float fixed_us,
   return best;
 }
 
-template <class K>
+template <class K, class... Extra>
 hipError_t launch_one(K kernel, OncePerDevice& once, int lds, const FusedArgs& a,
-                      int slices, int groups, hipStream_t s) {
+                      int slices, int groups, hipStream_t s, Extra... extra) {
   hipError_t e = set_max_dynamic_lds(once, (const void*)kernel, lds);
   if (e != hipSuccess) return e;
   const int64_t rounds = ((int64_t)groups * a.H + 7) / 8;
   if (rounds * 8 * slices > 0x7fffffff) return hipErrorInvalidValue;
-  kernel<<<dim3((unsigned)(rounds * 8 * slices)), kThreads, lds, s>>>(a, slices,
-                                                                      groups);
+  kernel<<<dim3((unsigned)(rounds * 8 * slices)), kThreads, lds, s>>>(
+      a, extra..., slices, groups);
   return hipGetLastError();
 }
 
@@ -1288,14 +1374,38 @@ hipError_t launch_as(const FusedArgs& a, const Plan& p, hipStream_t s) {
                         NarrowLayout::total, a,
                         p.slices, p.split.groups, s);
     case kSlices11:
-      return launch_one(block_prefill_slices_bf16_kernel<11, PACKED, GELU>,
+      return launch_one(block_prefill_slices_bf16_kernel<11, PACKED, GELU, false>,
                         once[1], Layout<11>::total, a, p.slices,
-                        p.split.groups, s);
+                        p.split.groups, s, RowsOfTile{});
     default:
-      return launch_one(block_prefill_slices_bf16_kernel<16, PACKED, GELU>,
+      return launch_one(block_prefill_slices_bf16_kernel<16, PACKED, GELU, false>,
                         once[2], Layout<16>::total, a, p.slices,
-                        p.split.groups, s);
+                        p.split.groups, s, RowsOfTile{});
   }
+}
+
+// Rows of at most 16 tokens, several to a tile.
+constexpr int kManyTokens = kTile / 2;
+Plan many_plan(int B, int H, int T, int bw) {
+  const int rows = kTile / T, slices = (bw + kSlice - 1) / kSlice;
+  return Plan{bw > kNarrowKS * 16 ? kSlices16 : kSlices11, slices,
+              best_split((int)(((int64_t)B + rows - 1) / rows), H, kTile, slices, kTiles,
+                         7.0f, 6.3f)};
+}
+template <bool GELU>
+hipError_t launch_many(const FusedArgs& a, hipStream_t s) {
+  const Plan p = many_plan(a.B, a.H, a.T, a.W / a.H);
+  RowsOfTile many{kTile / a.T, 0u, 0u, 65536u / (uint32_t)a.T + 1u};
+  for (int r = 0; r < many.rows; ++r) {
+    many.opens |= 1u << (r * a.T);
+    many.ends |= 1u << (r * a.T + a.T - 1);
+  }
+  static OncePerDevice once[2];
+  if (p.form == kSlices11)
+    return launch_one(block_prefill_slices_bf16_kernel<11, true, GELU, true>, once[0],
+                      Layout<11>::total, a, p.slices, p.split.groups, s, many);
+  return launch_one(block_prefill_slices_bf16_kernel<16, true, GELU, true>, once[1],
+                    Layout<16>::total, a, p.slices, p.split.groups, s, many);
 }
 
 }  // namespace
@@ -1303,16 +1413,38 @@ hipError_t launch_as(const FusedArgs& a, const Plan& p, hipStream_t s) {
 // k-steps of 16 the packed weights of a head of bw channels are laid out for.
 int gate_k_steps(int bw) { return bw <= kNarrowKS * 16 ? kNarrowKS : 16; }
 
-bool prefill_slices_serve(int B, int H, int T, bool joined) {
-  // the whole-head form (rg_prefill_teams.hip): one workgroup per pair, 64
-  // tokens in 4.35 us (joined 6.65)
+// The whole-head form (rg_prefill_teams.hip): one workgroup per pair, 64 tokens in 4.35
+// us (joined 6.65).
+static float whole_heads_us(int B, int H, int T, bool joined) {
   const int64_t rounds = ((int64_t)B * H + 255) / 256;
   const int64_t tiles = (T + 63) / 64;
-  const float whole = rounds * (joined ? 8.3f + 6.65f * tiles : 8.8f + 4.35f * tiles);
+  return rounds * (joined ? 8.3f + 6.65f * tiles : 8.8f + 4.35f * tiles);
+}
+
+bool prefill_slices_serve(int B, int H, int T, bool joined) {
+  const int64_t rounds = ((int64_t)B * H + 255) / 256;
+  const float whole = whole_heads_us(B, H, T, joined);
   // (beyond two rounds of pairs four times as many workgroups read the rows
   // anew from memory, which the estimate does not know: B46 T48 W4096 39, here
   // 44)
   return plan(B, H, T, 256, joined).split.us < (rounds > 2 ? 0.75f : 1.0f) * whole;
+}
+
+// Rows of a few tokens, several to a tile, where that takes fewer passes than a row to a
+// tile (its own pass is 0.5 to 1 us longer), or than whole heads by the workgroup.  us,
+// joined, otherwise / so: W4096 B24 T1 18.7 / 12.3, T9 19.5 / 14.0, W5632 H32 B24 T3 27.1 /
+// 13.0, T9 34.8 / 13.9, B64 T1 26.1 / 13.3, T9 50 / 31; with one pass either way W2560 B24
+// T9 13.2 / 14.2, B2 T1 11.0 / 11.8.
+bool prefill_many_serve(int B, int H, int T, int bw, bool joined) {
+  if (B < 2 || T > kManyTokens || bw <= 128 || bw > 256 || bw % 8) return false;
+  const float here = many_plan(B, H, T, bw).split.us;
+  // (beyond 512 pairs rg_recurrent_core's form is gate GEMM + scan.  256-wide heads stay
+  // there: its outputs are those of the two calls, bit for bit)
+  if ((int64_t)B * H > 512) return bw < 256;
+  const float apart = plan(B, H, T, bw, joined).split.us;
+  return here < (bw < 256 || prefill_slices_serve(B, H, T, joined)
+                     ? apart
+                     : whole_heads_us(B, H, T, joined));
 }
 
 bool prefill_narrow_pays(int B, int H, int T, int W) {
@@ -1334,6 +1466,9 @@ hipError_t launch_block_prefill_slices_bf16(const FusedArgs& a, hipStream_t s) {
   if (bw < 128 || bw > 256 || bw % 8 || a.B <= 0 ||
       (int64_t)a.T * a.W * 2 >= (int64_t)0x7fffffff)
     return hipErrorInvalidValue;
+  if (a.w_packed &&
+      prefill_many_serve(a.B, a.H, a.T, bw, a.gate_branch != nullptr))
+    return a.gate_branch ? launch_many<true>(a, s) : launch_many<false>(a, s);
   const Plan p = plan(a.B, a.H, a.T, bw, a.gate_branch != nullptr);
   if (a.w_packed)
     return a.gate_branch ? launch_as<true, true>(a, p, s)

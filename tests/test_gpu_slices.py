@@ -168,3 +168,22 @@ def test_rows_do_not_see_each_other(B, T, bw, H, packed):
     assert not torch.isfinite(got[1][bad]).all()
     for a, b in zip(got[:2], carried[:2]):
       assert torch.equal(a[others], b[others]), (bad, value, "h0")
+
+
+# several whole rows to a tile: one token each, numbers that leave tokens of the tile
+# over, the longest, last tiles with one row and with all, one tile and many
+MANY = [(2, 1, 256, 1), (33, 1, 176, 2), (300, 1, 256, 10), (64, 3, 256, 10),
+        (11, 5, 200, 3), (65, 9, 176, 32), (23, 11, 256, 2), (2, 16, 256, 2),
+        (129, 16, 248, 3), (40, 15, 136, 4)]
+
+
+@pytest.mark.parametrize("B,T,bw,H", MANY)
+@pytest.mark.parametrize("mean_doc", [4, -9])
+def test_rows_of_a_few_tokens(B, T, bw, H, mean_doc):
+  test_prefill_in_slices(B, T, bw, H, mean_doc, True)
+
+
+@pytest.mark.parametrize("B,T,bw,H", [(9, 1, 256, 2), (12, 3, 176, 4),
+                                      (7, 16, 256, 10), (9, 7, 200, 3)])
+def test_rows_of_a_few_tokens_do_not_see_each_other(B, T, bw, H):
+  test_rows_do_not_see_each_other(B, T, bw, H, True)
