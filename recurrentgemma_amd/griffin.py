@@ -663,6 +663,7 @@ class Embedder(nn.Module):
     self.vocab_size = vocab_size
     self.embed_dim = embed_dim
     self.scale_by_sqrt_dim = scale_by_sqrt_dim
+    self._rows_logits = ops.PackedLinear()
     self.input_embedding = nn.Parameter(
         torch.empty([vocab_size, embed_dim], device=device, dtype=dtype))
     self.reset_parameters()
@@ -679,7 +680,17 @@ class Embedder(nn.Module):
     return x
 
   def decode(self, x):
-    return x @ self.input_embedding.T
+    """Logits.  A few rows: the table streamed by the few-row kernel, from a
+    copy of its own in operand order (1.3 GB at 256000 x 2560).  us, library /
+    this, replayed from a graph: 1 row 217 / 192, 8 220 / 195, 16 223 / 205, 24
+    228 / 219, but 32 230 / 233, 64 246 / 279."""
+    table = self.input_embedding
+    if (0 < x.numel() <= 24 * self.embed_dim and
+        x.shape[-1:] == table.shape[1:] and not compiled.tracing() and
+        ops.PackedLinear.usable(x, self.embed_dim, self.vocab_size) and
+        ops._as_they_lie(x, table)):
+      return self._rows_logits(x, (table,))
+    return x @ table.T
 
 
 class Griffin(nn.Module):

@@ -191,3 +191,21 @@ def test_config5_full_shape_graph_equals_eager():
   # (other batch sizes take other kernels for the linear layers: the logits
   # agree to rounding, the greedy tokens almost always)
   assert (alone_t == want_t[:4]).float().mean().item() >= 0.75
+
+
+@pytest.mark.parametrize("rows", [1, 3, 16, 24, 25])
+def test_logits_of_a_few_rows(rows):
+  """The token table on the few-row kernel: one rounding of float32 sums, again
+  after the table has changed, and not where a gradient is asked for."""
+  torch.manual_seed(5)
+  e = G.Embedder(1024, 256, True, device="cuda", dtype=torch.bfloat16)
+  x = torch.randn(rows, 1, 256, device="cuda").bfloat16()
+  for _ in range(2):
+    with torch.no_grad():
+      got = e.decode(x)
+      want = x.double() @ e.input_embedding.double().T
+      # (half a unit in the last place of bf16, and the float32 sums' order)
+      assert ((got.double() - want).abs() <=
+              want.abs() * 2**-8 + 1e-5).all()
+      e.input_embedding.neg_()
+  assert e.decode(x).requires_grad
