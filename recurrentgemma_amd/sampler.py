@@ -128,6 +128,18 @@ class Sampler:
       return ops.argmax_last(logits)
     return torch.distributions.Categorical(logits=logits).sample()
 
+  def _step_for(self, batch_size, steps):
+    """The captured step of a batch, where this sampler replays one that was
+    captured with the parameters as they are."""
+    if not self.use_graph or steps <= 2:
+      return None
+    captured = self._captured.get(batch_size)
+    stamp = _parameter_stamp(self.model)
+    if (captured is None or captured.stamp != stamp or
+        any(s[1] is None for s in stamp)):  # (no version counter: recapture)
+      return None
+    return captured
+
   @torch.no_grad()
   def sample_tokens(self, padded_tokens, input_lengths,
                     total_generation_steps: int, echo: bool = False,
@@ -149,7 +161,7 @@ class Sampler:
     positions = torch.clip(positions, min=-1)
     model = self.model
 
-    prev_logits = logits = cache = None
+    prev_logits = logits = cache = captured = None
     if total_generation_steps == 0:
       prev_logits, _ = model(padded_tokens, positions, None,
                              return_logits=return_logits and echo,
@@ -161,12 +173,20 @@ class Sampler:
     else:
       # the logits of the first L-1 prompt tokens are never formed unless
       # they are asked for
-      prev_logits, cache = model(padded_tokens[:, :-1], positions[:, :-1],
-                                 None, return_logits=return_logits and echo,
+      before = positions[:, :-1].contiguous()
+      prev_logits, cache = model(padded_tokens[:, :-1], before, None,
+                                 return_logits=return_logits and echo,
                                  return_cache=True)
-      logits, cache = model(padded_tokens[:, -1:], positions[:, -1:], cache,
-                            return_logits=True,
-                            return_cache=total_generation_steps > 1)
+      captured = self._step_for(bsz, total_generation_steps)
+      # (2B model, 16 rows: 3.9 -> 1.5 ms.  Not a step captured for this call: the
+      # eager one in front of a capture lays the weights out on this stream)
+      if captured is not None:
+        captured.load(cache, positions[:, -1:])
+        logits = captured.step(padded_tokens[:, -1:])
+      else:
+        logits, cache = model(padded_tokens[:, -1:], positions[:, -1:], cache,
+                              return_logits=True,
+                              return_cache=total_generation_steps > 1)
 
     tokens_buffer = torch.full((bsz, total_generation_steps), pad_id, **ints)
     logits_buffer = None
@@ -188,12 +208,9 @@ class Sampler:
 
     pos = positions[:, -1:] + 1
     done = False
-    captured = None
-    if self.use_graph and total_generation_steps > 2:
-      captured = self._captured.get(bsz)
-      stamp = _parameter_stamp(model)
-      if (captured is None or captured.stamp != stamp or
-          any(s[1] is None for s in stamp)):  # (no version counter: recapture)
+    if captured is None and self.use_graph and total_generation_steps > 2:
+      captured = self._step_for(bsz, total_generation_steps)
+      if captured is None:
         captured = self._captured[bsz] = _CapturedStep(model, bsz, self.dtype,
                                                        dev)
       captured.load(cache, pos)
