@@ -1307,30 +1307,62 @@ int rg_linear_many_pays(int64_t M, int K, int count, const int* N, int dtype) {
          rg::matmul_pays(a, rg::kMatmulForward);
 }
 
-int rg_linear_many(const void* x, int64_t M, int K, int count, const void* const* w,
-                   const void* const* bias, void* const* out, const int* N, int dtype,
-                   void* stream) {
+static bool runs_fit(int64_t rows, const int32_t* runs, int count) {
+  return !runs || (count > 0 && count <= INT32_MAX / 8 && rows >= 8 && rows <= INT32_MAX &&
+                   (reinterpret_cast<uintptr_t>(runs) & 3u) == 0);
+}
+static bool with_runs(rg::MatmulArgs* a, int64_t rows, const int32_t* runs) {
+  a->runs = runs;
+  a->rows = runs ? (int)rows : 0;
+  return true;
+}
+
+// (runs: of M rows those in run_count runs of eight)
+#undef RG_WHO
+#define RG_WHO who
+static int linear_many_impl(const char* who, const void* x, int64_t M, const int32_t* runs,
+                            int run_count, int K, int count, const void* const* w,
+                            const void* const* bias, void* const* out, const int* N,
+                            int dtype, void* stream) {
   RG_CHECK_DTYPE(dtype);
   RG_REQUIRE(M > 0 && K > 0 && count > 0 && w && out && N,
-             "%s: M=%lld K=%d count=%d must be positive, the lists present", __func__,
+             "%s: M=%lld K=%d count=%d must be positive, the lists present", who,
              (long long)M, K, count);
   RG_CHECK_PTR(x);
   for (int i = 0; i < count; ++i) {
-    RG_REQUIRE(N[i] > 0, "%s: N[%d]=%d must be positive", __func__, i, N[i]);
+    RG_REQUIRE(N[i] > 0, "%s: N[%d]=%d must be positive", who, i, N[i]);
     RG_CHECK_PTR(w[i]);
     RG_CHECK_PTR(out[i]);
     if (bias) RG_CHECK_OPT_PTR(bias[i]);
     RG_REQUIRE(out[i] != x && !among(out[i], w, count) && !among(out[i], bias, count) &&
                    !among(out[i], out, i),
-               "%s: outputs must not alias an input or each other", __func__);
+               "%s: outputs must not alias an input or each other", who);
   }
   rg::MatmulArgs a;
-  if (dtype != RG_DTYPE_BF16 ||
-      !linear_many_args(x, M, K, count, w, bias, out, N, &a) ||
-      !rg::matmul_serves(a, rg::kMatmulForward))
-    return fail(RG_ERR_UNSUPPORTED, "%s: M=%lld K=%d", __func__, (long long)M, K);
-  return launch_status(__func__,
+  if (dtype != RG_DTYPE_BF16 || !runs_fit(M, runs, run_count) ||
+      !linear_many_args(x, runs ? 8ll * run_count : M, K, count, w, bias, out, N, &a) ||
+      !with_runs(&a, M, runs) || !rg::matmul_serves(a, rg::kMatmulForward))
+    return fail(RG_ERR_UNSUPPORTED, "%s: M=%lld K=%d", who, (long long)M, K);
+  return launch_status(who,
                        rg::launch_matmul(a, rg::kMatmulForward, (hipStream_t)stream));
+}
+
+#undef RG_WHO
+#define RG_WHO __func__
+
+int rg_linear_many(const void* x, int64_t M, int K, int count, const void* const* w,
+                   const void* const* bias, void* const* out, const int* N, int dtype,
+                   void* stream) {
+  return linear_many_impl(__func__, x, M, nullptr, 0, K, count, w, bias, out, N, dtype,
+                          stream);
+}
+
+int rg_linear_many_runs(const void* x, int64_t rows, const int32_t* runs, int count, int K,
+                        int layers, const void* const* w, const void* const* bias,
+                        void* const* out, const int* N, int dtype, void* stream) {
+  RG_REQUIRE(runs != nullptr, "%s: runs is null", __func__);
+  return linear_many_impl(__func__, x, rows, runs, count, K, layers, w, bias, out, N, dtype,
+                          stream);
 }
 
 static bool linear_back_args(const void* dy, const void* w, const void* dy2,
@@ -1444,23 +1476,42 @@ int rg_linear_gelu_pair_pays(int64_t M, int K, int N, int dtype) {
          rg::matmul_pays(a, rg::kMatmulGeluPair);
 }
 
-int rg_linear_gelu_pair(const void* x, const void* w, const void* bias, void* out,
-                        int64_t M, int K, int N, int dtype, void* stream) {
+#undef RG_WHO
+#define RG_WHO who
+static int gelu_pair_impl(const char* who, const void* x, const void* w, const void* bias,
+                          void* out, int64_t M, const int32_t* runs, int run_count, int K,
+                          int N, int dtype, void* stream) {
   RG_CHECK_DTYPE(dtype);
-  RG_REQUIRE(M > 0 && K > 0 && N > 0, "%s: M=%lld K=%d N=%d must be positive", __func__,
+  RG_REQUIRE(M > 0 && K > 0 && N > 0, "%s: M=%lld K=%d N=%d must be positive", who,
              (long long)M, K, N);
   RG_CHECK_PTR(x);
   RG_CHECK_PTR(w);
   RG_CHECK_OPT_PTR(bias);
   RG_CHECK_PTR(out);
   RG_REQUIRE(out != x && out != w && out != bias, "%s: out must not alias an input",
-             __func__);
+             who);
   rg::MatmulArgs a;
-  if (dtype != RG_DTYPE_BF16 || !gelu_pair_args(x, w, bias, out, M, K, N, &a) ||
-      !rg::matmul_serves(a, rg::kMatmulGeluPair))
-    return fail(RG_ERR_UNSUPPORTED, "%s: M=%lld K=%d N=%d", __func__, (long long)M, K, N);
-  return launch_status(__func__,
+  if (dtype != RG_DTYPE_BF16 || !runs_fit(M, runs, run_count) ||
+      !gelu_pair_args(x, w, bias, out, runs ? 8ll * run_count : M, K, N, &a) ||
+      !with_runs(&a, M, runs) || !rg::matmul_serves(a, rg::kMatmulGeluPair))
+    return fail(RG_ERR_UNSUPPORTED, "%s: M=%lld K=%d N=%d", who, (long long)M, K, N);
+  return launch_status(who,
                        rg::launch_matmul(a, rg::kMatmulGeluPair, (hipStream_t)stream));
+}
+
+#undef RG_WHO
+#define RG_WHO __func__
+
+int rg_linear_gelu_pair(const void* x, const void* w, const void* bias, void* out,
+                        int64_t M, int K, int N, int dtype, void* stream) {
+  return gelu_pair_impl(__func__, x, w, bias, out, M, nullptr, 0, K, N, dtype, stream);
+}
+
+int rg_linear_gelu_pair_runs(const void* x, const void* w, const void* bias, void* out,
+                             int64_t rows, const int32_t* runs, int count, int K, int N,
+                             int dtype, void* stream) {
+  RG_REQUIRE(runs != nullptr, "%s: runs is null", __func__);
+  return gelu_pair_impl(__func__, x, w, bias, out, rows, runs, count, K, N, dtype, stream);
 }
 
 int rg_argmax_rows_split(const void* x, int64_t* out, void* workspace, int rows,
@@ -1510,6 +1561,28 @@ int rg_add_rms_norm(const void* x, const void* addend, const void* scale,
   return launch_status(
       __func__, rg::launch_rms_norm(x, addend, scale, sum_out, out, rows, width,
                                     eps, dtype, (hipStream_t)stream));
+}
+
+int rg_add_rms_norm_runs(const void* x, const void* addend, const void* scale,
+                         void* sum_out, void* out, const int32_t* runs, int count,
+                         int width, float eps, int dtype, void* stream) {
+  RG_CHECK_DTYPE(dtype);
+  RG_REQUIRE(runs != nullptr && count > 0, "%s: no runs", __func__);
+  RG_CHECK_PTR(x);
+  RG_CHECK_PTR(addend);
+  RG_CHECK_PTR(scale);
+  RG_CHECK_PTR(sum_out);
+  RG_CHECK_PTR(out);
+  RG_REQUIRE(out != sum_out && out != x && out != addend && sum_out != x &&
+                 sum_out != addend,
+             "%s: an output aliases an input or the other", __func__);
+  if (dtype != RG_DTYPE_BF16 || width <= 0 || width % 8 || width > 4096 ||
+      !aligned16(x) || !aligned16(addend) || !aligned16(scale) || !aligned16(sum_out) ||
+      !aligned16(out))
+    return fail(RG_ERR_UNSUPPORTED, "%s: width=%d", __func__, width);
+  return launch_status(
+      __func__, rg::launch_add_rms_norm_runs(x, addend, scale, sum_out, out, runs, count,
+                                             width, eps, (hipStream_t)stream));
 }
 
 int rg_rope(const void* x, const void* positions, int positions_is_i64,

@@ -170,16 +170,19 @@ rms_norm_kernel(const T* __restrict__ x, const T* __restrict__ addend,
 // lanes, the row stays in registers between the two passes (one read, one
 // write; the scalar kernel above re-reads through the cache and moved
 // 1.7 TB/s on 131 072 rows of 2560).
-template <bool ADD, bool FROM_PARTIAL>
+// RUNS: of the rows those in runs of eight that start at these.
+template <bool ADD, bool FROM_PARTIAL, bool RUNS = false>
 __global__ void __launch_bounds__(256)
 rms_norm_bf16_rows_kernel(const u32x4* __restrict__ x, PartialRows part,
                           const u32x4* __restrict__ addend,
                           const u32x4* __restrict__ scale,
                           u32x4* __restrict__ sum_out,
                           u32x4* __restrict__ out, int chunks, float inv_width,
-                          float eps) {
+                          float eps, const int* __restrict__ runs = nullptr) {
   __shared__ float partial[4];
-  rms_norm_row<ADD, FROM_PARTIAL, false>(threadIdx.x, blockIdx.x, partial, x, part, addend,
+  const int64_t row =
+      RUNS ? runs[blockIdx.x >> 3] + (int)(blockIdx.x & 7) : (int)blockIdx.x;
+  rms_norm_row<ADD, FROM_PARTIAL, false>(threadIdx.x, row, partial, x, part, addend,
                                          scale, sum_out, out, chunks, inv_width, eps);
 }
 
@@ -440,6 +443,17 @@ hipError_t launch_rms_norm(const void* x, const void* addend, const void* scale,
   };
   if (dtype == 0) run((float*)nullptr);
   else run((uint16_t*)nullptr);
+  return hipGetLastError();
+}
+
+hipError_t launch_add_rms_norm_runs(const void* x, const void* addend, const void* scale,
+                                    void* sum_out, void* out, const int* runs, int count,
+                                    int width, float eps, hipStream_t s) {
+  if (count <= 0 || count > 0x7fffffff / 8 || width % 8 || width > 4096)
+    return hipErrorInvalidValue;
+  rms_norm_bf16_rows_kernel<true, false, true><<<dim3((unsigned)count * 8u), 256, 0, s>>>(
+      (const u32x4*)x, PartialRows{}, (const u32x4*)addend, (const u32x4*)scale,
+      (u32x4*)sum_out, (u32x4*)out, width / 8, 1.0f / (float)width, eps, runs);
   return hipGetLastError();
 }
 

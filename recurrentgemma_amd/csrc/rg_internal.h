@@ -299,6 +299,11 @@ struct MatmulProblem {
 struct MatmulArgs {
   MatmulProblem p[kMaxMatmuls];
   int count;
+  // or null: of the tensors' `rows` rows only those in runs of eight, which start at
+  // these; p[].M is eight times their number (forward and pairs, any order, runs may
+  // overlap)
+  const int* runs;
+  int rows;
 };
 // Whether the launch can be made; and (but for weight gradients) whether it is ahead of
 // the library's products.
@@ -460,6 +465,9 @@ hipError_t launch_linear_rows_normed(const NormedLinearArgs& a, int gelu_pair,
                                      hipStream_t s);
 hipError_t launch_linear_rows_partial(const LinearArgs& a, int slices,
                                       hipStream_t s);
+hipError_t launch_add_rms_norm_runs(const void* x, const void* addend, const void* scale,
+                                    void* sum_out, void* out, const int* runs, int count,
+                                    int width, float eps, hipStream_t s);
 hipError_t launch_rms_norm_partial(const float* sums, int slices,
                                    const void* bias, const void* addend,
                                    const void* scale, void* sum_out, void* out,

@@ -121,14 +121,27 @@ __device__ __forceinline__ f32x4 fragment(bool slow, const uint32_t (&a)[4], uin
 // block of 16 rows, columns 4 quarter .. + 3 of one of 16 columns.  row0: the wave's
 // first row behind m0; column(nb): the first column of block nb (and the next: nb is
 // even).  PAIR: the second half of the blocks are the second weight's.
-template <bool PAIR, int MB, int BLOCKS, class Value, class Column>
-__device__ __forceinline__ void store_tile(const MatmulProblem& p, int m0, int row0, int lane,
-                                           Value&& value, Column&& column) {
+template <bool PAIR, int MB, int BLOCKS, bool RUNS, class Value, class Column>
+__device__ __forceinline__ void store_tile(const MatmulArgs& args, const MatmulProblem& p,
+                                           int m0, int row0, int lane, Value&& value,
+                                           Column&& column) {
   const int n = lane & 15, quarter = lane >> 4;
-  const int64_t skip = 2ll * m0 * p.ldc;
-  const __amdgpu_buffer_rsrc_t rc =
-      make_rsrc((char*)p.c + skip,
-                (uint32_t)(2 * ((int64_t)(p.M - 1) * p.ldc + p.N) - skip));
+  const int64_t skip = RUNS ? 0 : 2ll * m0 * p.ldc;
+  const __amdgpu_buffer_rsrc_t rc = make_rsrc(
+      (char*)p.c + skip,
+      (uint32_t)(2 * ((int64_t)((RUNS ? args.rows : p.M) - 1) * p.ldc + p.N) - skip));
+  // this lane's row of each block of 16
+  uint32_t row_at[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    if (RUNS) {
+      const int run = (m0 + row0) / 8 + 2 * mb + (n >> 3);
+      row_at[mb] = 8 * run < p.M ? (uint32_t)(args.runs[run] + (n & 7)) * 2u * (uint32_t)p.ldc
+                                 : kBufferOutOfRange;
+    } else {
+      row_at[mb] = (uint32_t)(row0 + n + 16 * mb) * 2u * (uint32_t)p.ldc;
+    }
+  }
   const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.bias, p.bias ? 2u * (uint32_t)p.N : 0u);
   const __amdgpu_buffer_rsrc_t rb2 =
       make_rsrc(p.bias2, PAIR && p.bias2 ? 2u * (uint32_t)p.N : 0u);
@@ -172,16 +185,15 @@ __device__ __forceinline__ void store_tile(const MatmulProblem& p, int m0, int r
       const auto s0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
       const auto s1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
       buffer_store_16(u32x4{s0[0], s1[0], s0[1], s1[1]}, rc,
-                      at < p.N ? (uint32_t)(row0 + n + 16 * mb) * 2u * (uint32_t)p.ldc +
-                                     2u * (uint32_t)at
-                               : kBufferOutOfRange,
-                      0);
+                      at < p.N ? row_at[mb] + 2u * (uint32_t)at : kBufferOutOfRange, 0);
     });
   });
 }
 
-// KIND as in rg_internal.h; wave tile 16 MB x 32 NB.
-template <int KIND, int MB, int NB>
+// KIND as in rg_internal.h; wave tile 16 MB x 32 NB.  RUNS: the rows of a tile are runs of
+// eight wherever they lie (a load instruction has eight rows: a scalar offset each, made
+// once), so that padding between sequences is neither read nor multiplied.
+template <int KIND, int MB, int NB, bool RUNS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 matmul_bf16_kernel(MatmulArgs args) {
   constexpr bool kPair = KIND == kMatmulGeluPair;
@@ -210,7 +222,8 @@ matmul_bf16_kernel(MatmulArgs args) {
   const int tm = at.tm, tn = at.tn;
   const int m0 = tm * kTileM, n0 = tn * kTileN;
   const int ldm2 = 2 * p.ldm, ldn2 = 2 * p.ldn;  // bytes
-  u32x4 rm = operand(p, p.m, kSlowM, m0, p.M, p.ldm);
+  static_assert(!RUNS || (!kSlowM && !kTwoStretches), "");
+  u32x4 rm = operand(p, p.m, kSlowM, RUNS ? 0 : m0, RUNS ? args.rows : p.M, p.ldm);
   u32x4 rn = operand(p, p.n, kSlowN, n0, p.N, p.ldn);
   u32x4 rn_up = rn;
   if (kPair) rn_up = operand(p, p.n2, kSlowN, n0, p.N, p.ldn);
@@ -232,6 +245,10 @@ matmul_bf16_kernel(MatmulArgs args) {
     scalar_offset[i] = (is_m ? kSlowM : kSlowN)
                            ? row * (is_m ? ldm2 : ldn2) + 128 * panel
                            : (64 * panel + row) * (is_m ? ldm2 : ldn2);
+    // (behind the last run: the last once more, whose results are dropped)
+    if (RUNS && is_m)
+      scalar_offset[i] =
+          args.runs[min((m0 + 64 * panel + row) / 8, p.M / 8 - 1)] * ldm2;
   }
   auto load = [&](uint32_t stage, auto I) {
     constexpr int i = decltype(I)::value;
@@ -250,6 +267,10 @@ matmul_bf16_kernel(MatmulArgs args) {
     constexpr int kLines = kTileM / 64;  // a row of the contraction is this many lines
     vp0 = kSlowM ? (uint32_t)((16 * (tn & 3) + lane / kLines) * ldm2 + 128 * (lane % kLines))
                  : (uint32_t)((8 * MB * (tn & 3) + lane) * ldm2);
+    if (RUNS) {
+      const int row = m0 + 8 * MB * (tn & 3) + lane;
+      vp0 = (uint32_t)((args.runs[min(row / 8, p.M / 8 - 1)] + (row & 7)) * ldm2);
+    }
   }
   if (wave == 1 && lane < 8 * NB) {
     constexpr int kLines = kTileN / 64;
@@ -387,7 +408,7 @@ matmul_bf16_kernel(MatmulArgs args) {
     if constexpr (b < kAccBlocks) return acc_read<4 * b + r>();
     else return extra[b - kAccBlocks][r];
   };
-  store_tile<kPair, MB, kBlocksN>(p, m0, 16 * MB * wm, lane, value, [&](int nb) {
+  store_tile<kPair, MB, kBlocksN, RUNS>(args, p, m0, 16 * MB * wm, lane, value, [&](int nb) {
     return n0 + (kPair ? 64 * wn + 16 * nb
                  : kSlowN ? 32 * (nb + wn)
                           : 32 * NB * wn + 16 * nb);
@@ -513,7 +534,7 @@ __global__ void __launch_bounds__(256) matmul_small_bf16_kernel(MatmulArgs args)
     constexpr int b = decltype(BLK)::value;
     return acc[b / MB][b % MB][decltype(R)::value];
   };
-  store_tile<kPair, MB, NB>(p, m0, 16 * MB * wm, lane, value, [&](int nb) {
+  store_tile<kPair, MB, NB, false>(args, p, m0, 16 * MB * wm, lane, value, [&](int nb) {
     return n0 + (kPair ? 32 * wn + 16 * nb : 16 * NB * wn + 16 * nb);
   });
 }
@@ -530,15 +551,17 @@ unsigned first_tiles(MatmulArgs& a, int rows, int cols) {
   return (unsigned)tiles;
 }
 
-template <int KIND, int MB, int NB>
+template <int KIND, int MB, int NB, bool RUNS = false>
 hipError_t launch_tiles(MatmulArgs& a, hipStream_t s) {
+  if constexpr (!RUNS && (KIND == kMatmulForward || KIND == kMatmulGeluPair))
+    if (a.runs) return launch_tiles<KIND, MB, NB, true>(a, s);
   constexpr int kTileN = KIND == kMatmulGeluPair ? 32 * NB : 64 * NB;
   constexpr int kLds = 2 * (MB / 2 + NB) * kPanelBytes + 4 * 256;
   static OncePerDevice once;
   hipError_t e = set_max_dynamic_lds(
-      once, (const void*)matmul_bf16_kernel<KIND, MB, NB>, kLds);
+      once, (const void*)matmul_bf16_kernel<KIND, MB, NB, RUNS>, kLds);
   if (e != hipSuccess) return e;
-  matmul_bf16_kernel<KIND, MB, NB><<<dim3(first_tiles(a, 32 * MB, kTileN)), 256, kLds, s>>>(a);
+  matmul_bf16_kernel<KIND, MB, NB, RUNS><<<dim3(first_tiles(a, 32 * MB, kTileN)), 256, kLds, s>>>(a);
   return hipGetLastError();
 }
 
@@ -604,7 +627,7 @@ float best_tile(const MatmulArgs& a, int kind, int* tile) {
   *tile = -1;
   for (int t = 0; t < kTileForms; ++t) {
     const Tile& form = kind == kMatmulGeluPair ? kPairTiles[t] : kTiles[t];
-    if (!form.rows) continue;
+    if (!form.rows || (a.runs && t > 3)) continue;  // (runs: large tiles alone)
     int64_t tiles = 0;
     int steps = 0;
     for (int i = 0; i < a.count; ++i) {
@@ -629,17 +652,20 @@ bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0
 // What the kernel can address: 16-byte loads and stores, offsets below 2^31.
 bool matmul_serves(const MatmulArgs& a, int kind) {
   if (a.count < 1 || a.count > kMaxMatmuls) return false;
+  if (a.runs && (kind == kMatmulBack || kind == kMatmulWeights || a.rows < 8)) return false;
   for (int i = 0; i < a.count; ++i) {
     const MatmulProblem& p = a.p[i];
     if (p.M < 1 || p.N < 8 || p.K < 1 || p.N % 8) return false;
     if (kind == kMatmulWeights ? p.M % 8 : p.K % kStep) return false;
     if ((p.ldm | p.ldn | p.ldc) % 8) return false;
-    const int64_t rows_m = kind == kMatmulWeights ? p.K : p.M;
+    if (a.runs && p.M % 8) return false;
+    const int64_t rows_c = a.runs ? a.rows : p.M;
+    const int64_t rows_m = kind == kMatmulWeights ? p.K : rows_c;
     const int64_t rows_n = kind == kMatmulForward ? p.N : p.K;
     // (a step past the end is asked for, and found out of range)
     if (rows_m >= (1 << 30) || rows_n >= (1 << 30) ||
         (rows_m + 512) * p.ldm >= (1ll << 30) || (rows_n + 512) * p.ldn >= (1ll << 30) ||
-        ((int64_t)p.M + 512) * p.ldc >= (1ll << 30))
+        (rows_c + 512) * p.ldc >= (1ll << 30))
       return false;
     for (const void* t : {p.m, p.n, p.m2, p.n2, p.bias, p.bias2, (const void*)p.c})
       if (!aligned(t)) return false;

@@ -76,6 +76,21 @@ int rg_linear_gelu_pair_pays(int64_t M, int K, int N, int dtype);
 int rg_linear_gelu_pair(const void* x, const void* w, const void* bias, void* out,
                         int64_t M, int K, int N, int dtype, void* stream);
 
+/* rg_linear_many, rg_linear_gelu_pair and rg_add_rms_norm (bf16) of some of the rows of
+ * tensors with `rows` of them: those in `count` runs of eight, which start at the rows in
+ * `runs` (on the GPU, 0 .. rows - 8, any order, overlaps allowed); nothing else is read or
+ * written.  RG_ERR_UNSUPPORTED beyond the sizes of those calls (norm: rows of at most 4096
+ * in eights). */
+int rg_linear_many_runs(const void* x, int64_t rows, const int32_t* runs, int count, int K,
+                        int layers, const void* const* w, const void* const* bias,
+                        void* const* out, const int* N, int dtype, void* stream);
+int rg_linear_gelu_pair_runs(const void* x, const void* w, const void* bias, void* out,
+                             int64_t rows, const int32_t* runs, int count, int K, int N,
+                             int dtype, void* stream);
+int rg_add_rms_norm_runs(const void* x, const void* addend, const void* scale,
+                         void* sum_out, void* out, const int32_t* runs, int count,
+                         int width, float eps, int dtype, void* stream);
+
 /* What such layers give back: dx [M,N] = dy [M,K] . w [K,N] (+ dy2 . w2 of the same
  * sizes: two layers that read the same x; both NULL: none), one rounding; and dw[i]
  * [out_features[i], in_features[i]] = dy[i] [M,out]^T . x[i] [M,in], up to four as one

@@ -31,6 +31,7 @@ from torch import nn
 
 from recurrentgemma_amd import _lib
 from recurrentgemma_amd import compiled
+from recurrentgemma_amd import layers
 from recurrentgemma_amd import modules
 from recurrentgemma_amd import ops
 
@@ -751,6 +752,107 @@ class Griffin(nn.Module):
     if cap:
       logits = ops.soft_cap(logits, cap)
     return logits, (new_cache if return_cache else None)
+
+  def prompt_runs_serve(self) -> bool:
+    """Whether prompt_cache can stand for forward: bf16 on the GPU, sizes that
+    its kernels take, and nothing wrapped, hooked or replaced on the way."""
+    c = self.config
+    lru_width = c.lru_width or c.width
+    plain = modules._as_written
+    if (c.width % 64 or c.width > 4096 or c.mlp_expanded_width % 64 or
+        lru_width % 64 or c.width != 256 * c.num_heads or
+        compiled.tracing() or modules._global_hooks() or
+        not (plain(self, Griffin) and plain(self.embedder, Embedder) and
+             "encode" not in self.embedder.__dict__)):
+      return False
+    table = self.embedder.input_embedding
+    if (not table.is_cuda or table.dtype != torch.bfloat16 or
+        not ops._as_they_lie(table, *self.parameters())):
+      return False
+    for block in self.blocks:
+      if not plain(block, ResidualBlock):
+        return False
+      norms = (block.temporal_pre_norm, block.channel_pre_norm)
+      mlp, own = block.mlp_block, block.temporal_block
+      if not (all(plain(n, RMSNorm) and "add_then_norm" not in n.__dict__
+                  for n in norms) and plain(mlp, MLPBlock) and
+              plain(mlp.ffw_up, _StackedLinear) and plain(mlp.ffw_down, nn.Linear)):
+        return False
+      if plain(own, modules.RecurrentBlock):
+        if not (plain(own.conv_1d, layers.Conv1D) and
+                plain(own.rg_lru, layers.RGLRU) and
+                all(plain(m, nn.Linear) for m in (own.linear_x, own.linear_y,
+                                                  own.linear_out))):
+          return False
+      elif not (plain(own, LocalAttentionBlock) and own.head_dim == 256 and
+                all(plain(m, nn.Linear) for m in (own.proj_q, own.proj_k,
+                                                  own.proj_v, own.proj_final))):
+        return False
+    return True
+
+  @torch.no_grad()
+  def prompt_cache(self, tokens, segment_pos, runs: ops.RowRuns) -> Cache:
+    """The cache that forward(tokens, segment_pos) leaves, for left-padded
+    prompts, with the row-wise layers (norms, products: most of a prompt pass)
+    on the rows in the runs alone.  What they leave out is padding in front of
+    a row's first token, whose position 0 cuts the recurrence and the conv and
+    bounds the attention: nothing behind it depends on what lies there, as long
+    as it is finite -- zeros, in the tensors that the recurrence and the
+    attention read.  Where prompt_runs_serve says so."""
+    b, t = tokens.shape
+    x = self.embedder.encode(tokens)
+
+    def linear(x, *parts, out=None):
+      weights, biases = zip(*(modules._parameters(p, "weight", "bias")
+                              for p in parts))
+      out = out or [x.new_empty(b, t, w.shape[0]) for w in weights]
+      return ops.linear_many_runs(x, weights, biases, runs, out)
+
+    zeroed = {}  # of each width, written by one block after the other
+
+    def zeros(name, width):
+      if (name, width) not in zeroed:
+        zeroed[name, width] = x.new_zeros(b, t, width)
+      return zeroed[name, width]
+
+    new_cache, out = {}, None
+    for i, block in enumerate(self.blocks):
+      norm, own = block.temporal_pre_norm, block.temporal_block
+      if out is None:
+        normed = norm(x)
+      else:
+        x, normed = ops.add_rms_norm_runs(out, x, norm.scale, norm.eps, runs)
+      if block.temporal_block_type is TemporalBlockType.RECURRENT:
+        width = own.lru_width
+        y, xb = linear(normed, own.linear_y, own.linear_x,
+                       out=[x.new_empty(b, t, width), zeros("x", width)])
+        del normed
+        mixed, cache = modules._recurrent_core(
+            own.conv_1d, own.rg_lru, xb, segment_pos, None, True, False, y)
+        del xb, y
+        mixed, = linear(mixed, own.linear_out)
+      else:
+        if own._inv_freq is None or own._inv_freq.device != x.device:
+          own._inv_freq = _inv_frequencies(own.head_dim, x.device)
+        q, k, v = linear(normed, own.proj_q, own.proj_k, own.proj_v,
+                         out=[zeros("x", own.width), zeros("k", own.head_dim),
+                              zeros("v", own.head_dim)])
+        del normed
+        mixed, ring_k, ring_v, count = ops.attention_prompt(
+            q.reshape(b, t, own.num_heads, own.head_dim), k, v, segment_pos,
+            own._inv_freq, _first_visible_key(segment_pos, own.window_size),
+            own.window_size, own.head_dim ** -0.5)
+        cache = AttentionBlockCache(keys=ring_k, values=ring_v, num_tokens=count)
+        mixed, = linear(mixed.reshape(b, t, own.width), own.proj_final)
+      new_cache[f"blocks.{i}"] = cache
+      norm, mlp = block.channel_pre_norm, block.mlp_block
+      x, normed = ops.add_rms_norm_runs(mixed, x, norm.scale, norm.eps, runs)
+      hidden = ops.linear_gelu_pair_runs(
+          normed, *modules._parameters(mlp.ffw_up, "w", "b"), runs)
+      del mixed, normed
+      out, = linear(hidden, mlp.ffw_down)
+      del hidden
+    return new_cache
 
   def init_cache(self, batch_size, dtype, device=None) -> Cache:
     c = self.config

@@ -638,6 +638,72 @@ def linear_gelu_pair(x, w, b):
   return out
 
 
+class RowRuns:
+  """Which rows of a batch of left-padded prompts its row-wise layers compute:
+  runs of eight that hold every real token (and some padding in front of it).
+  Tensors keep their [B, T, ..] layout; rows outside the runs are neither read
+  nor written by the calls that take them."""
+
+  def __init__(self, lengths, tokens, device):
+    """lengths: real tokens of each row, on the host; tokens: T."""
+    first = []
+    for b, n in enumerate(lengths):
+      end = (b + 1) * tokens
+      first += [max(at, 0) for at in range(end - (n + 7) // 8 * 8, end, 8)]
+    self.rows = len(lengths) * tokens
+    self.count = len(first)
+    if self.rows < 8 or not first or not all(
+        0 < n <= tokens for n in lengths):
+      raise ValueError("rows of 1 to T tokens, eight rows in all at least")
+    self.first = torch.tensor(first, dtype=torch.int32).to(device)
+
+
+def _run_rows(t, runs):
+  """Columns of a tensor that has the runs' rows."""
+  assert t.numel() // t.shape[-1] == runs.rows, (t.shape, runs.rows)
+  return t.shape[-1]
+
+
+def linear_many_runs(x, weights, biases, runs, out):
+  """linear_many of the rows in the runs, into the tensors `out` [..., N_i]."""
+  K = _run_rows(x, runs)
+  n = [_run_rows(o, runs) for o in out]
+  assert all(w.shape == (m, K) for w, m in zip(weights, n))
+  assert all(b is None or b.shape == (m,) for b, m in zip(biases, n))
+  pointers = ctypes.c_void_p * len(n)
+  with _on(x.device):
+    _lib.check(_lib.lib().rg_linear_many_runs(
+        _p(x), runs.rows, _p(runs.first), runs.count, K, len(n),
+        pointers(*map(_p, weights)), pointers(*map(_p, biases)),
+        pointers(*map(_p, out)), (ctypes.c_int * len(n))(*n),
+        _dtype_code(x), _stream(x)))
+  return out
+
+
+def linear_gelu_pair_runs(x, w, b, runs):
+  """linear_gelu_pair of the rows in the runs; the others are not written."""
+  K, N = _run_rows(x, runs), w.shape[2]
+  assert w.shape == (2, K, N) and b.numel() == 2 * N
+  out = torch.empty((*x.shape[:-1], N), dtype=x.dtype, device=x.device)
+  with _on(x.device):
+    _lib.check(_lib.lib().rg_linear_gelu_pair_runs(
+        _p(x), _p(w), _p(b), _p(out), runs.rows, _p(runs.first), runs.count, K,
+        N, _dtype_code(x), _stream(x)))
+  return out
+
+
+def add_rms_norm_runs(x, addend, scale, eps, runs):
+  """add_rms_norm of the rows in the runs; the others are not written."""
+  width = _run_rows(x, runs)
+  assert x.shape == addend.shape and scale.shape == (width,)
+  total, out = torch.empty_like(x), torch.empty_like(x)
+  with _on(x.device):
+    _lib.check(_lib.lib().rg_add_rms_norm_runs(
+        _p(x), _p(addend), _p(scale), _p(total), _p(out), _p(runs.first),
+        runs.count, width, eps, _dtype_code(x), _stream(x)))
+  return total, out
+
+
 def rms_norm(x, scale, eps=1e-6):
   """x * rsqrt(mean(x^2, -1) + eps) * (scale + 1), one pass."""
   x = _dev(x, "x")

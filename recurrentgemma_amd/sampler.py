@@ -128,6 +128,25 @@ class Sampler:
       return ops.argmax_last(logits)
     return torch.distributions.Categorical(logits=logits).sample()
 
+  def _prompt_runs(self, batch_size, length, input_lengths):
+    """The rows of the prompts but their last tokens that are worth computing,
+    or None for all of them: where too few are padding to pay for reading the
+    lengths back (a synchronisation) and for the large tiles that rows in runs are
+    multiplied in (3960 rows, 75 % of them real, 3 blocks: 9.75 -> 9.83 ms in
+    all), and where a row has one token or none in front of its last, or is no
+    left-padded row at all.  2B model, 16 prompts of 500 to 1000 tokens, 75 % of
+    the rows, and 32 tokens: 100.4 -> 93.2 ms."""
+    rows = batch_size * (length - 1)
+    if (batch_size < 2 or rows < 8192 or not self.model.prompt_runs_serve() or
+        torch.cuda.is_current_stream_capturing()):
+      return None
+    lengths = [n - 1 for n in input_lengths.tolist()]
+    if not all(1 <= n < length for n in lengths):
+      return None
+    if 8 * sum((n + 7) // 8 for n in lengths) > 0.9 * rows:
+      return None
+    return ops.RowRuns(lengths, length - 1, self.device)
+
   def _step_for(self, batch_size, steps):
     """The captured step of a batch, where this sampler replays one that was
     captured with the parameters as they are."""
@@ -174,9 +193,14 @@ class Sampler:
       # the logits of the first L-1 prompt tokens are never formed unless
       # they are asked for
       before = positions[:, :-1].contiguous()
-      prev_logits, cache = model(padded_tokens[:, :-1], before, None,
-                                 return_logits=return_logits and echo,
-                                 return_cache=True)
+      runs = (None if return_logits and echo else
+              self._prompt_runs(bsz, plen, input_lengths))
+      if runs is not None:
+        cache = model.prompt_cache(padded_tokens[:, :-1], before, runs)
+      else:
+        prev_logits, cache = model(padded_tokens[:, :-1], before, None,
+                                   return_logits=return_logits and echo,
+                                   return_cache=True)
       captured = self._step_for(bsz, total_generation_steps)
       # (2B model, 16 rows: 3.9 -> 1.5 ms.  Not a step captured for this call: the
       # eager one in front of a capture lays the weights out on this stream)

@@ -1,0 +1,109 @@
+"""Prompt passes that leave padding out (ops.RowRuns, Griffin.prompt_cache):
+products and norms of runs of eight rows, and the cache a prompt leaves."""
+
+import pytest
+import torch
+
+from recurrentgemma_amd import _lib
+from recurrentgemma_amd import griffin as G
+from recurrentgemma_amd import ops
+from recurrentgemma_amd import sampler as S
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _runs(lengths, tokens):
+  runs = ops.RowRuns(lengths, tokens, DEV)
+  kept = torch.zeros(runs.rows, dtype=torch.bool)
+  for first in runs.first.tolist():
+    assert 0 <= first <= runs.rows - 8
+    kept[first:first + 8] = True
+  for b, n in enumerate(lengths):
+    assert kept[(b + 1) * tokens - n:(b + 1) * tokens].all()
+  return runs, kept.to(DEV)
+
+
+def _near(got, want, sums):
+  """One bf16 rounding (2^-9 of the value, and as much for a float32 sum next to
+  a boundary) of a float32 sum of terms whose magnitudes add up to `sums`."""
+  assert ((got.double() - want).abs() <= want.abs() * 2**-8 +
+          2**-20 * sums).all()
+
+
+@pytest.mark.parametrize("lengths,T,K,N", [
+    # one run, runs that overlap at the start, a cut tile, every tile size that the
+    # cost model picks from, a few hundred rows to several rounds of the chip
+    ([8], 8, 64, (64,)), ([3, 9, 1], 9, 64, (128, 8)),
+    ([5, 300, 77], 301, 512, (512, 256, 256)),
+    ([999, 500, 640, 801, 555], 999, 256, (2560, 2560)),
+    ([700, 350, 600, 421, 480], 700, 1024, (320,)),
+    ([640] * 9 + [3], 641, 2560, (2560,))])
+def test_products_and_norms_of_runs(lengths, T, K, N):
+  runs, kept = _runs(lengths, T)
+  g = torch.Generator(device=DEV).manual_seed(3)
+  normal = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+  x = normal(runs.rows, K)
+  x[~kept] = float("nan")  # (never read)
+  ws, bs = [normal(n, K) for n in N], [normal(n) for n in N[:-1]] + [None]
+  out = [torch.full((runs.rows, n), 7.0, device=DEV).bfloat16() for n in N]
+  ops.linear_many_runs(x, ws, bs, runs, out)
+  for o, w, b in zip(out, ws, bs):
+    assert (o[~kept] == 7).all()
+    want = x[kept].double() @ w.double().T + (0 if b is None else b.double())
+    _near(o[kept], want, x[kept].double().abs() @ w.double().abs().T)
+  # the pair: what the call for all rows gives for these rows, bit for bit (the same
+  # instructions along K, whatever the tile)
+  w, b = normal(2, K, 256), normal(2, 1, 1, 256)
+  pair = ops.linear_gelu_pair_runs(x, w, b, runs)
+  xk = x[kept]
+  want = torch.empty(len(xk), 256, device=DEV, dtype=torch.bfloat16)
+  _lib.check(_lib.lib().rg_linear_gelu_pair(
+      xk.data_ptr(), w.data_ptr(), b.data_ptr(), want.data_ptr(), len(xk), K, 256,
+      _lib.RG_DTYPE_BF16, torch.cuda.current_stream().cuda_stream))
+  assert torch.equal(pair[kept], want)
+  a = normal(runs.rows, K)
+  scale = normal(K)
+  total, normed = ops.add_rms_norm_runs(x, a, scale, 1e-6, runs)
+  want = ops.add_rms_norm(x[kept], a[kept], scale)
+  assert torch.equal(total[kept], want[0]) and torch.equal(normed[kept], want[1])
+
+
+@pytest.mark.parametrize("lengths,T", [
+    ([301, 2, 100, 299, 17, 8, 150, 64, 33, 200] * 3, 301),
+    ([90, 5, 47] * 30, 97)])
+@torch.no_grad()
+def test_prompts_without_their_padding(lengths, T):
+  torch.manual_seed(11)
+  kinds = (G.TemporalBlockType.RECURRENT, G.TemporalBlockType.ATTENTION,
+           G.TemporalBlockType.RECURRENT)
+  config = G.GriffinConfig(
+      vocab_size=640, width=512, mlp_expanded_width=1536, lru_width=512,
+      num_heads=2, block_types=kinds, embeddings_scale_by_sqrt_dim=True,
+      attention_window_size=64, logits_soft_cap=30.0)
+  model = G.Griffin(config, device=DEV, dtype=torch.bfloat16).eval()
+  B = len(lengths)
+  tokens = torch.randint(1, 640, (B, T), device=DEV)
+  lens = torch.tensor(lengths, device=DEV)
+  plain, runs = S.Sampler(model), S.Sampler(model)
+  plain._prompt_runs = lambda *a: None
+  assert runs._prompt_runs(B, T, lens) is not None
+  want, want_logits = plain.sample_tokens(tokens, lens, 4, return_logits=True)
+  # (whatever a tensor's memory held before: none of it may be looked at)
+  junk = [torch.full((1 << 22,), float("nan"), device=DEV) for _ in range(8)]
+  del junk
+  got, logits = runs.sample_tokens(tokens, lens, 4, return_logits=True)
+  assert torch.isfinite(logits).all()
+  # other sums in front of the roundings of three blocks, about ten tensors each
+  first = (logits[:, 0].float() - want_logits[:, 0].float()).norm()
+  assert first <= 30 ** 0.5 * 2**-8 * want_logits[:, 0].float().norm()
+  same = (got == want).float().mean()
+  assert same > 0.9, same
+  # rows of one token, rows that are full beyond their tokens: all rows as before
+  lens[1] = 1
+  assert runs._prompt_runs(B, T, lens) is None
+  handle = model.blocks[0].mlp_block.ffw_down.register_forward_hook(lambda *a: None)
+  lens[1] = 2
+  assert runs._prompt_runs(B, T, lens) is None
+  handle.remove()
+  assert runs._prompt_runs(B, T, lens) is not None
