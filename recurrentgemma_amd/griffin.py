@@ -684,9 +684,10 @@ class Embedder(nn.Module):
     """Logits.  A few rows: the table streamed by the few-row kernel, from a
     copy of its own in operand order (1.3 GB at 256000 x 2560).  us, library /
     this, replayed from a graph: 1 row 217 / 192, 8 220 / 195, 16 223 / 205, 24
-    228 / 219, but 32 230 / 233, 64 246 / 279."""
+    228 / 219, but 32 230 / 233, 64 246 / 279.  (Small tables, whose product takes
+    little more than a launch, are not worth the copy.)"""
     table = self.input_embedding
-    if (0 < x.numel() <= 24 * self.embed_dim and
+    if (0 < x.numel() <= 24 * self.embed_dim and self.vocab_size >= 32_000 and
         x.shape[-1:] == table.shape[1:] and not compiled.tracing() and
         ops.PackedLinear.usable(x, self.embed_dim, self.vocab_size) and
         ops._as_they_lie(x, table)):

@@ -198,7 +198,7 @@ def test_logits_of_a_few_rows(rows):
   """The token table on the few-row kernel: one rounding of float32 sums, again
   after the table has changed, and not where a gradient is asked for."""
   torch.manual_seed(5)
-  e = G.Embedder(1024, 256, True, device="cuda", dtype=torch.bfloat16)
+  e = G.Embedder(32_000, 256, True, device="cuda", dtype=torch.bfloat16)
   x = torch.randn(rows, 1, 256, device="cuda").bfloat16()
   for _ in range(2):
     with torch.no_grad():
