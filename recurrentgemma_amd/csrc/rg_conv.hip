@@ -131,6 +131,7 @@ conv1d_backward_kernel(const T* __restrict__ dout, const T* __restrict__ x,
 // is used.
 constexpr int kConvRun = 32;    // rows per wave of the forward kernels
 constexpr int kConvBatch = 8;   // rows requested together
+constexpr int kConvFlagRows = 48;  // rows between two looks at 64 rows' flags
 
 template <typename T>
 struct Vec16;
@@ -161,6 +162,26 @@ struct Vec16<uint16_t> {
                  pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
   }
 };
+// four channels of a lane, whatever they are stored as
+template <typename T>
+struct Vec4ch : Vec16<float> {
+  typedef u32x4 Raw;
+};
+template <>
+struct Vec4ch<uint16_t> {
+  static constexpr int N = 4;
+  typedef u32x2 Raw;
+  __device__ static void unpack(u32x2 r, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      v[2 * i] = __uint_as_float(r[i] << 16);
+      v[2 * i + 1] = __uint_as_float(r[i] & 0xffff0000u);
+    }
+  }
+  __device__ static u32x2 pack(const float (&v)[4]) {
+    return u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+  }
+};
 
 // Which of the rows around a run (fewer than `span` of them, from `base` on)
 // is the first token of a sequence row: at most one when the sequences are at
@@ -183,6 +204,17 @@ struct SeqStarts {
 __device__ __forceinline__ bool conv_row_starts(const void* segpos, int seg_kind,
                                                 const SeqStarts& seq, int64_t m) {
   return seq.at(m) || is_doc_start(segpos, seg_kind, m);
+}
+
+// The same for the 64 rows from `base` on, a bit each, rows behind the last one (M - 1)
+// among the starts: a lane a row and one load, where a test of a flag row by row is a
+// branch and a wait for everything the wave has asked for.
+__device__ __forceinline__ uint64_t start_bits(const void* segpos, int seg_kind,
+                                               int64_t base, int T_len, int64_t M) {
+  const int64_t m = base + ((int)threadIdx.x & 63);
+  bool starts = m >= M;
+  if (m >= 0 && m < M) starts = m % T_len == 0 || is_doc_start(segpos, seg_kind, m);
+  return __ballot(starts);
 }
 
 // RUN rows per wave: the longer, the fewer halo rows are read twice (3 per
@@ -363,25 +395,33 @@ conv1d_prefill_k4_kernel(const T* __restrict__ x, const void* __restrict__ segpo
 // dbias go to the chunk's plane of `partial` like the general kernel's.
 //
 // A chunk's rows are shared by the WAVES waves of a workgroup, whose sums meet in LDS.
-// What bounds it: a wave waits for its batch of rows, then works on it, and its
-// registers (200) leave no room for the next batch; so the waves of a CU have to
-// cover each other, of which one a chunk makes five (B4 T2048 W2560 bf16).  Figures
-// beside the launch.
+// What bounds it: memory from some 30 us on, the way of the first rows before that.  A
+// lane has four channels, so that three waves a SIMD have registers (137 of them; with
+// eight channels of bf16 247, two waves and 5 waves for 4 SIMDs at B4 T2048 W2560), and a
+// row's loads are asked for as the row eight (float32: four) in front of it is used up:
+// no branch lies between them, the flags are bits.  bf16 B4 T2048 W2560 with operands in
+// memory: 45 us with a look at the flags row by row, eight channels a lane and a batch of
+// rows waited for at a time; 38 with the bits and loads one by one; 34 with four channels
+// (139 MB: 4.1 TB/s).  Float32 60 either way, 8.5 -> 7.0 at B1 T300.
 template <typename T, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES)
+__global__ void __launch_bounds__(64 * WAVES, 3)
 conv1d_backward_k4_kernel(const T* __restrict__ dout, const T* __restrict__ x,
                           const void* __restrict__ segpos, int seg_kind,
                           const T* __restrict__ w, T* __restrict__ dx,
                           float* __restrict__ partial,
                           float* __restrict__ dx_sums, int T_len, int W,
                           int64_t M, int rows) {
-  using V = Vec16<T>;
+  using V = Vec4ch<T>;
+  using Raw = typename V::Raw;
   constexpr int N = V::N;
+  constexpr int kBatch = sizeof(T) == 4 ? 4 : 8;  // rows on their way
   __shared__ float others[WAVES > 1 ? WAVES - 1 : 1][WAVES > 1 ? 6 * N : 1][64];
   const int lane = (int)threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int c = ((int)blockIdx.y * 64 + lane) * N;
-  if (WAVES == 1 && c >= W) return;
+  // (lanes behind a row's end do the last one's work once more, with its values: every
+  // lane has a row's flag to load)
+  const int own_c = ((int)blockIdx.y * 64 + lane) * N;
+  const int c = own_c < W ? own_c : W - N;
   const int share = rows / WAVES;
   const int64_t m0 = (int64_t)blockIdx.x * rows + wave * share;
   const int64_t m1 = m0 + share < M ? m0 + share : M;
@@ -389,110 +429,107 @@ conv1d_backward_k4_kernel(const T* __restrict__ dout, const T* __restrict__ x,
 #pragma unroll
   for (int e = 0; e < N; ++e)
     d0[e] = d1[e] = d2[e] = d3[e] = db[e] = dxs[e] = 0.0f;
-  if (WAVES == 1 || (c < W && m0 < M)) {
-    const SeqStarts seq(m0 >= 3 ? m0 - 3 : 0, T_len, share + 6);
+  if (WAVES == 1 || m0 < M) {
     auto row = [&](const T* base, int64_t m) {
-      return *reinterpret_cast<const u32x4*>(base + m * W + c);
+      return *reinterpret_cast<const Raw*>(base + m * W + c);
     };
-    // a row behind the last one counts as a start (nothing beyond it is used)
-    auto starts = [&](int64_t m) {
-      return m >= M || conv_row_starts(segpos, seg_kind, seq, m);
+    // (rows outside: any row inside, not used)
+    auto row_in = [&](const T* base, int64_t m) {
+      return row(base, m < 0 ? 0 : m < M ? m : M - 1);
     };
+    Raw taps[4], before[3], after[3], xr[kBatch], gr[kBatch];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      before[k] = row_in(x, m0 - 1 - k);
+      after[k] = row_in(dout, m0 + k);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) taps[k] = row(w, k);
+    // bit 0: row m0 (or the row that begins the present kConvFlagRows)
+    uint64_t bits = start_bits(segpos, seg_kind, m0 - 3, T_len, M);
+    const bool cut1 = (bits >> 2) & 1, cut2 = cut1 || ((bits >> 1) & 1);
+    bits >>= 3;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      xr[u] = row_in(x, m0 + u);
+      gr[u] = row_in(dout, m0 + u + 3);
+    }
     float w0[N], w1[N], w2[N], w3[N];
-    V::unpack(row(w, 0), w0);
-    V::unpack(row(w, 1), w1);
-    V::unpack(row(w, 2), w2);
-    V::unpack(row(w, 3), w3);
-    float h1[N], h2[N], h3[N];
+    V::unpack(taps[0], w0);
+    V::unpack(taps[1], w1);
+    V::unpack(taps[2], w2);
+    V::unpack(taps[3], w3);
+    // the rows before, as far as no start cuts them off; g0 = dout[m], g1 .. g3 the
+    // rows after it
+    float h1[N], h2[N], h3[N], g0[N], g1[N], g2[N], g3[N];
+    auto take = [](bool used, const Raw& r, float (&v)[N]) {
+      V::unpack(used ? r : Raw(0u), v);
+    };
+    // (m0 is 0 or 8 at least)
+    take(m0 > 0, before[0], h1);
+    take(m0 > 0 && !cut1, before[1], h2);
+    take(m0 > 0 && !cut2, before[2], h3);
+    V::unpack(after[0], g0);
+    V::unpack(after[1], g1);
+    V::unpack(after[2], g2);
+    auto one_row = [&](int64_t m, const Raw& xm, const Raw& gm)
+        __attribute__((always_inline)) {
+      float cur[N], o[N];
+      V::unpack(xm, cur);
+      V::unpack(gm, g3);
+      if (bits & 1) {
 #pragma unroll
-    for (int e = 0; e < N; ++e) h1[e] = h2[e] = h3[e] = 0.0f;
-    for (int64_t j = m0 - 3; j < m0; ++j) {
-      if (j < 0) continue;
-      if (conv_row_starts(segpos, seg_kind, seq, j)) {
-#pragma unroll
-        for (int e = 0; e < N; ++e) h1[e] = h2[e] = 0.0f;
+        for (int e = 0; e < N; ++e) h1[e] = h2[e] = h3[e] = 0.0f;
       }
+      // a tap reaches the rows of dout in front of the next start
+      const bool ok1 = !(bits & 2), ok2 = !(bits & 6), ok3 = !(bits & 14);
+      bits >>= 1;
 #pragma unroll
       for (int e = 0; e < N; ++e) {
+        float acc = w3[e] * g0[e];
+        acc = __builtin_fmaf(w2[e], ok1 ? g1[e] : 0.0f, acc);
+        acc = __builtin_fmaf(w1[e], ok2 ? g2[e] : 0.0f, acc);
+        acc = __builtin_fmaf(w0[e], ok3 ? g3[e] : 0.0f, acc);
+        o[e] = acc;
+        d3[e] = __builtin_fmaf(cur[e], g0[e], d3[e]);  // w[3] meets x[t]
+        d2[e] = __builtin_fmaf(h1[e], g0[e], d2[e]);
+        d1[e] = __builtin_fmaf(h2[e], g0[e], d1[e]);
+        d0[e] = __builtin_fmaf(h3[e], g0[e], d0[e]);
+        db[e] += g0[e];
         h3[e] = h2[e];
         h2[e] = h1[e];
+        h1[e] = cur[e];
+        g0[e] = g1[e];
+        g1[e] = g2[e];
+        g2[e] = g3[e];
       }
-      V::unpack(row(x, j), h1);
-    }
-    // g0 = dout[m], g1 .. g3 the rows after it; f1 .. f3: those rows start
-    float g0[N], g1[N], g2[N], g3[N];
-    bool f1, f2, f3;
-    auto dout_row = [&](int64_t m, float (&v)[N]) {
-      if (m < M) {
-        V::unpack(row(dout, m), v);
-      } else {
+      const Raw packed = V::pack(o);
+      *reinterpret_cast<Raw*>(dx + m * W + c) = packed;
+      // (of what is stored: the bias gradient of the layer in front)
+      V::unpack(packed, o);
 #pragma unroll
-        for (int e = 0; e < N; ++e) v[e] = 0.0f;
-      }
+      for (int e = 0; e < N; ++e) dxs[e] += o[e];
     };
-    dout_row(m0, g0);
-    dout_row(m0 + 1, g1);
-    dout_row(m0 + 2, g2);
-    f1 = starts(m0 + 1);
-    f2 = starts(m0 + 2);
-    for (int64_t mb = m0; mb < m1; mb += kConvBatch) {
-      u32x4 xr[kConvBatch], gr[kConvBatch];
-      bool st[kConvBatch], fa[kConvBatch];
+    int64_t mb = m0;
+    // whole batches, without a branch around a load: the row eight on takes the place of
+    // the one that has been used (behind the last one the last once more)
+    for (; mb + kBatch <= m1; mb += kBatch) {
+      if (mb > m0 && (mb - m0) % kConvFlagRows == 0)
+        bits = start_bits(segpos, seg_kind, mb, T_len, M);
 #pragma unroll
-      for (int u = 0; u < kConvBatch; ++u) {
-        const int64_t m = mb + u < m1 ? mb + u : m1 - 1;
-        xr[u] = row(x, m);
-        gr[u] = row(dout, m + 3 < M ? m + 3 : M - 1);
-        st[u] = conv_row_starts(segpos, seg_kind, seq, m);
-        fa[u] = starts(m + 3);
+      for (int u = 0; u < kBatch; ++u) {
+        const int64_t m = mb + u, ahead = m + kBatch < m1 ? m + kBatch : m1 - 1;
+        one_row(m, xr[u], gr[u]);
+        xr[u] = row(x, ahead);
+        gr[u] = row(dout, ahead + 3 < M ? ahead + 3 : M - 1);
       }
+    }
+    if (mb < m1) {
+      if (mb > m0 && (mb - m0) % kConvFlagRows == 0)
+        bits = start_bits(segpos, seg_kind, mb, T_len, M);
 #pragma unroll
-      for (int u = 0; u < kConvBatch; ++u) {
-        const int64_t m = mb + u;
-        if (m < m1) {
-          if (m + 3 < M) {
-            V::unpack(gr[u], g3);
-          } else {
-#pragma unroll
-            for (int e = 0; e < N; ++e) g3[e] = 0.0f;
-          }
-          f3 = fa[u];
-          if (st[u]) {
-#pragma unroll
-            for (int e = 0; e < N; ++e) h1[e] = h2[e] = h3[e] = 0.0f;
-          }
-          float cur[N], o[N];
-          V::unpack(xr[u], cur);
-          const bool ok1 = !f1, ok2 = ok1 && !f2, ok3 = ok2 && !f3;
-#pragma unroll
-          for (int e = 0; e < N; ++e) {
-            float acc = w3[e] * g0[e];
-            acc = __builtin_fmaf(w2[e], ok1 ? g1[e] : 0.0f, acc);
-            acc = __builtin_fmaf(w1[e], ok2 ? g2[e] : 0.0f, acc);
-            acc = __builtin_fmaf(w0[e], ok3 ? g3[e] : 0.0f, acc);
-            o[e] = acc;
-            d3[e] = __builtin_fmaf(cur[e], g0[e], d3[e]);  // w[3] meets x[t]
-            d2[e] = __builtin_fmaf(h1[e], g0[e], d2[e]);
-            d1[e] = __builtin_fmaf(h2[e], g0[e], d1[e]);
-            d0[e] = __builtin_fmaf(h3[e], g0[e], d0[e]);
-            db[e] += g0[e];
-            h3[e] = h2[e];
-            h2[e] = h1[e];
-            h1[e] = cur[e];
-            g0[e] = g1[e];
-            g1[e] = g2[e];
-            g2[e] = g3[e];
-          }
-          f1 = f2;
-          f2 = f3;
-          const u32x4 packed = V::pack(o);
-          *reinterpret_cast<u32x4*>(dx + m * W + c) = packed;
-          // (of what is stored: the bias gradient of the layer in front)
-          V::unpack(packed, o);
-#pragma unroll
-          for (int e = 0; e < N; ++e) dxs[e] += o[e];
-        }
-      }
+      for (int u = 0; u < kBatch; ++u)
+        if (mb + u < m1) one_row(mb + u, xr[u], gr[u]);
     }
   }
   if constexpr (WAVES > 1) {
@@ -517,9 +554,10 @@ conv1d_backward_k4_kernel(const T* __restrict__ dout, const T* __restrict__ x,
     };
     if (wave > 0) meet_all();
     __syncthreads();
-    if (wave > 0 || c >= W) return;
+    if (wave > 0) return;
     meet_all();
   }
+  if (own_c >= W) return;
   if (dx_sums != nullptr) {
 #pragma unroll
     for (int e = 0; e < N; ++e) dx_sums[(int64_t)blockIdx.x * W + c + e] = dxs[e];
@@ -689,20 +727,21 @@ hipError_t launch_conv1d_backward(const ConvBwdArgs& a, int dtype,
   if (dtype == 0 ? conv_k4_fits<float>(a.K, a.W, M)
                  : conv_k4_fits<uint16_t>(a.K, a.W, M)) {
     // waves of a chunk: as many as there is room for on the CUs (us, one / two / four:
-    // bf16 B1 T300 W2560 26 / 17 / 12, B2 T1000 W4096 30 / 23 / 18, B4 T2048 W2560
-    // 40 / 43 / 42, B8 T2048 W4096 108 / 115 / 126; float32 19 / 12 / 8, 23 / 20 / 23,
-    // 49 / 47 / 48)
+    // bf16 B1 T300 W2560 11.2 / 8.7 / 7.1, B1 T1000 13.5 / 10.4 / 9.2, B2 T1000 W4096
+    // 17.3 / 16.6 / 18.5, B4 T2048 W2560 34.1 / 36.0 / 38.7, B8 T2048 W4096 103 / 111 /
+    // 119; float32 12.1 / 8.8 / 7.0, 16.6 / 12.5 / 12.0, 27.3 / 25.4 / 29.8, 60.6 / 60.5 /
+    // 61.0, 189 / 193 / 198)
     auto run = [&](auto* tag, auto waves) {
       typedef std::remove_pointer_t<decltype(tag)> T;
       constexpr int w = decltype(waves)::value;
       conv1d_backward_k4_kernel<T, w>
-          <<<dim3((unsigned)chunks, (unsigned)((a.W / Vec16<T>::N + 63) / 64)), 64 * w,
+          <<<dim3((unsigned)chunks, (unsigned)((a.W / Vec4ch<T>::N + 63) / 64)), 64 * w,
              0, s>>>((const T*)a.dout, (const T*)a.x, a.segpos, a.seg_kind,
                      (const T*)a.w, (T*)a.dx, a.partial, a.dx_sums, a.T, a.W, M, rows);
     };
     auto pick = [&](auto* tag) {
       typedef std::remove_pointer_t<decltype(tag)> T;
-      const int64_t blocks = chunks * ((a.W / Vec16<T>::N + 63) / 64);
+      const int64_t blocks = chunks * ((a.W / Vec4ch<T>::N + 63) / 64);
       if (blocks <= 512) run(tag, std::integral_constant<int, 4>{});
       else if (blocks <= 1024) run(tag, std::integral_constant<int, 2>{});
       else run(tag, std::integral_constant<int, 1>{});

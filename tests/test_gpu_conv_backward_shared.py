@@ -53,3 +53,10 @@ def test_against_float64(dtype, B, T, W):
   want_b = gd.sum((0, 1))
   assert bool(((db.double() - want_b).abs() <= steps * gd.abs().sum((0, 1)) +
                stored * want_b.abs() + 1e-30).all())
+
+
+# chunks of 64 and 256 rows, whose starts are looked up 48 rows at a time
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,W", [(3, 6001, 8), (5, 20003, 8), (70000, 1, 8)])
+def test_chunks_of_more_rows(dtype, B, T, W):
+  test_against_float64(dtype, B, T, W)
