@@ -208,7 +208,8 @@ __device__ __forceinline__ bool conv_row_starts(const void* segpos, int seg_kind
 
 // The same for the 64 rows from `base` on, a bit each, rows behind the last one (M - 1)
 // among the starts: a lane a row and one load, where a test of a flag row by row is a
-// branch and a wait for everything the wave has asked for.
+// branch and a wait for everything the wave has asked for.  Every lane of the wave takes
+// part.
 __device__ __forceinline__ uint64_t start_bits(const void* segpos, int seg_kind,
                                                int64_t base, int T_len, int64_t M) {
   const int64_t m = base + ((int)threadIdx.x & 63);
@@ -230,8 +231,11 @@ conv1d_prefill_k4_kernel(const T* __restrict__ x, const void* __restrict__ segpo
   constexpr int N = V::N;
   // the waves of a workgroup lie side by side along a row (up to 16 of them:
   // 16 KB of a row), so that what they request together is contiguous
-  const int c = ((int)blockIdx.y * (int)blockDim.x + (int)threadIdx.x) * N;
-  if (c >= W) return;  // W % N == 0 (launcher): a lane is inside or outside
+  const int own_c = ((int)blockIdx.y * (int)blockDim.x + (int)threadIdx.x) * N;
+  // (W % N == 0: a lane is inside or outside; those outside do the last one's work once
+  // more, with its values, beside lanes inside: every lane has a row's flag to load)
+  if (own_c - ((int)threadIdx.x & 63) * N >= W) return;
+  const int c = own_c < W ? own_c : W - N;
   const int64_t m0 = (int64_t)blockIdx.x * RUN;
   if (m0 >= M) {
     const int64_t b = (int64_t)blockIdx.x - (M + RUN - 1) / RUN;
@@ -248,14 +252,23 @@ conv1d_prefill_k4_kernel(const T* __restrict__ x, const void* __restrict__ segpo
     return;
   }
   const int64_t m1 = m0 + RUN < M ? m0 + RUN : M;
-  const SeqStarts seq(m0 >= 3 ? m0 - 3 : 0, T_len, RUN + 3);
   auto row = [&](const T* base, int64_t m) {
     return *reinterpret_cast<const u32x4*>(base + m * W + c);
   };
   if constexpr (sizeof(T) == 2) {
     // bf16: the kernels' one width-4 arithmetic (conv4_dot of rg_common.h) on
     // rows that stay packed: per channel the time pairs (x[t-1], x[t]), two
-    // dot products per output
+    // dot products per output.  No branch lies between the loads: the starts are bits, and
+    // the row eight on takes the place of the one that is used up.  us, with a look at the
+    // flags row by row before: B1 T64 W2560 5.5 -> 4.0, B1 T512 6.7 -> 4.6, B4 T2048 22.9
+    // -> 21.3, B16 T4096 138 -> 132.  (Float32 so: 5.3 -> 4.1, 6.3 -> 5.1 and 39.1 -> 38.3,
+    // but B3 T2048 29.0 -> 31.2 and 2 to 3 % at B3 T1001, B2 T2048: left as it was.)
+    u32x4 before[3], raw[kConvBatch];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) before[k] = row(x, m0 ? m0 - 3 + k : 0);
+#pragma unroll
+    for (int u = 0; u < kConvBatch; ++u) raw[u] = row(x, m0 + u < m1 ? m0 + u : m1 - 1);
+    uint64_t bits = start_bits(segpos, seg_kind, m0 - 3, T_len, M);  // bit 0: the next row
     float bb[N];
     V::unpack(*reinterpret_cast<const u32x4*>(bias + c), bb);
     uint32_t w10[N], w32[N];
@@ -291,49 +304,60 @@ conv1d_prefill_k4_kernel(const T* __restrict__ x, const void* __restrict__ segpo
       }
       r1 = cur;
     };
-    for (int64_t j = m0 - 3; j < m0; ++j) {
-      if (j < 0) continue;
-      if (conv_row_starts(segpos, seg_kind, seq, j)) cut();
-      const u32x4 cur = row(x, j);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if (m0) {
+        if (bits & 1) cut();
+        uint32_t pn0[N];
+        push(before[k], pn0);
+        shift(before[k], pn0);
+      }
+      bits >>= 1;
+    }
+    auto one_row = [&](int64_t m, const u32x4& cur) __attribute__((always_inline)) {
+      if (bits & 1) cut();
+      bits >>= 1;
       uint32_t pn0[N];
       push(cur, pn0);
+      float o[N];
+#pragma unroll
+      for (int q = 0; q < N; q += 4) {
+        const uint32_t po[4] = {pn2[q], pn2[q + 1], pn2[q + 2], pn2[q + 3]};
+        const uint32_t pw[4] = {pn0[q], pn0[q + 1], pn0[q + 2], pn0[q + 3]};
+        const uint32_t wa[4] = {w10[q], w10[q + 1], w10[q + 2], w10[q + 3]};
+        const uint32_t wb[4] = {w32[q], w32[q + 1], w32[q + 2], w32[q + 3]};
+        const float bq[4] = {bb[q], bb[q + 1], bb[q + 2], bb[q + 3]};
+        float oq[4];
+        conv4_dot_x4(po, pw, wa, wb, bq, oq);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[q + e] = oq[e];
+      }
       shift(cur, pn0);
+      *reinterpret_cast<u32x4*>(out + m * W + c) = V::pack(o);
+    };
+    auto look = [&](int64_t mb) __attribute__((always_inline)) {
+      if (RUN > kConvFlagRows && mb > m0 && (mb - m0) % kConvFlagRows == 0)
+        bits = start_bits(segpos, seg_kind, mb, T_len, M);
+    };
+    int64_t mb = m0;
+    for (; mb + kConvBatch <= m1; mb += kConvBatch) {
+      look(mb);
+#pragma unroll
+      for (int u = 0; u < kConvBatch; ++u) {
+        one_row(mb + u, raw[u]);
+        const int64_t ahead = mb + u + kConvBatch;
+        if (RUN > kConvBatch) raw[u] = row(x, ahead < m1 ? ahead : m1 - 1);
+      }
     }
-    for (int64_t mb = m0; mb < m1; mb += kConvBatch) {
-      u32x4 raw[kConvBatch];
-      bool st[kConvBatch];
+    if (mb < m1) {
+      look(mb);
 #pragma unroll
-      for (int u = 0; u < kConvBatch; ++u) {
-        const int64_t m = mb + u < m1 ? mb + u : m1 - 1;
-        raw[u] = row(x, m);
-        st[u] = conv_row_starts(segpos, seg_kind, seq, m);
-      }
-#pragma unroll
-      for (int u = 0; u < kConvBatch; ++u) {
-        if (mb + u < m1) {
-          if (st[u]) cut();
-          uint32_t pn0[N];
-          push(raw[u], pn0);
-          float o[N];
-#pragma unroll
-          for (int q = 0; q < N; q += 4) {
-            const uint32_t po[4] = {pn2[q], pn2[q + 1], pn2[q + 2], pn2[q + 3]};
-            const uint32_t pw[4] = {pn0[q], pn0[q + 1], pn0[q + 2], pn0[q + 3]};
-            const uint32_t wa[4] = {w10[q], w10[q + 1], w10[q + 2], w10[q + 3]};
-            const uint32_t wb[4] = {w32[q], w32[q + 1], w32[q + 2], w32[q + 3]};
-            const float bq[4] = {bb[q], bb[q + 1], bb[q + 2], bb[q + 3]};
-            float oq[4];
-            conv4_dot_x4(po, pw, wa, wb, bq, oq);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[q + e] = oq[e];
-          }
-          shift(raw[u], pn0);
-          *reinterpret_cast<u32x4*>(out + (mb + u) * W + c) = V::pack(o);
-        }
-      }
+      for (int u = 0; u < kConvBatch; ++u)
+        if (mb + u < m1) one_row(mb + u, raw[u]);
     }
     return;
   }
+  const SeqStarts seq(m0 >= 3 ? m0 - 3 : 0, T_len, RUN + 3);
   float w0[N], w1[N], w2[N], w3[N], bb[N];
   V::unpack(row(w, 0), w0);
   V::unpack(row(w, 1), w1);
