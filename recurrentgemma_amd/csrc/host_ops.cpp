@@ -569,6 +569,8 @@ PyObject* attention_prompt(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(shape_is(first, {B, T}));
     const int32_t* first_key = (const int32_t*)dense(first, at::kInt, c.device);
     for (const Tensor* t : {&w_q, &w_k, &w_v, &w_o, &b_o}) dense(*t, c.dtype, c.device);
+    // (another thread may replace a parameter while this one is without the interpreter)
+    const Tensor keep[] = {w_q, w_k, w_v, w_o, b_o};
     void* s = c.stream();
 
     const int n_qkv[3] = {(int)W, (int)kHead, (int)kHead}, n_out[1] = {(int)W};
@@ -581,9 +583,9 @@ PyObject* attention_prompt(PyObject*, PyObject* const* v, Py_ssize_t n) {
       val = c.empty({B, T, kHead});
     } else {
       NoGil free;
-      q = at::linear(c.x, w_q);
-      k = at::linear(c.x, w_k);
-      val = at::linear(c.x, w_v);
+      q = at::linear(c.x, keep[0]);
+      k = at::linear(c.x, keep[1]);
+      val = at::linear(c.x, keep[2]);
     }
     if (v[8] == Py_True) {
       ring_k = c.empty({B, window, 1, kHead});
@@ -597,12 +599,10 @@ PyObject* attention_prompt(PyObject*, PyObject* const* v, Py_ssize_t n) {
     void *qp = at_of(q), *kp = at_of(k), *vp = at_of(val), *ap = at_of(attended),
          *op = at_of(out), *rk = at_of(ring_k), *rv = at_of(ring_v), *np = at_of(count),
          *wp = at_of(ws);
-    const void* const w3[3] = {w_q.const_data_ptr(), w_k.const_data_ptr(),
-                               w_v.const_data_ptr()};
-    const void* const w1[1] = {w_o.const_data_ptr()};
-    const void* const b1[1] = {b_o.const_data_ptr()};
-    // (another thread may replace a parameter while this one is without the interpreter)
-    const Tensor keep[] = {w_q, w_k, w_v, w_o, b_o};
+    const void* const w3[3] = {keep[0].const_data_ptr(), keep[1].const_data_ptr(),
+                               keep[2].const_data_ptr()};
+    const void* const w1[1] = {keep[3].const_data_ptr()};
+    const void* const b1[1] = {keep[4].const_data_ptr()};
     launch([&] {
       if (qkv_ours) {
         void* const to[3] = {qp, kp, vp};
