@@ -1317,6 +1317,15 @@ static bool with_runs(rg::MatmulArgs* a, int64_t rows, const int32_t* runs) {
   return true;
 }
 
+// (a run of eight rows stands for all of them: the limits are those of the whole tensors)
+static const int32_t kOneRun = 0;
+int rg_linear_many_runs_serve(int64_t rows, int K, int layers, const int* N, int dtype) {
+  rg::MatmulArgs a;
+  return dtype == RG_DTYPE_BF16 && N && runs_fit(rows, &kOneRun, 1) &&
+         linear_many_args(nullptr, 8, K, layers, nullptr, nullptr, nullptr, N, &a) &&
+         with_runs(&a, rows, &kOneRun) && rg::matmul_serves(a, rg::kMatmulForward);
+}
+
 // (runs: of M rows those in run_count runs of eight)
 #undef RG_WHO
 #define RG_WHO who
@@ -1474,6 +1483,13 @@ int rg_linear_gelu_pair_pays(int64_t M, int K, int N, int dtype) {
   return dtype == RG_DTYPE_BF16 &&
          gelu_pair_args(nullptr, nullptr, nullptr, nullptr, M, K, N, &a) &&
          rg::matmul_pays(a, rg::kMatmulGeluPair);
+}
+
+int rg_linear_gelu_pair_runs_serve(int64_t rows, int K, int N, int dtype) {
+  rg::MatmulArgs a;
+  return dtype == RG_DTYPE_BF16 && runs_fit(rows, &kOneRun, 1) &&
+         gelu_pair_args(nullptr, nullptr, nullptr, nullptr, 8, K, N, &a) &&
+         with_runs(&a, rows, &kOneRun) && rg::matmul_serves(a, rg::kMatmulGeluPair);
 }
 
 #undef RG_WHO

@@ -658,6 +658,21 @@ class RowRuns:
     self.first = torch.tensor(first, dtype=torch.int32).to(device)
 
 
+@functools.lru_cache(maxsize=1024)
+def linear_many_runs_serve(rows, K, *features) -> bool:
+  """Whether linear_many_runs takes tensors of so many rows, whatever the runs."""
+  sizes = (ctypes.c_int * len(features))(*features)
+  return bool(_lib.lib().rg_linear_many_runs_serve(
+      rows, K, len(features), sizes, _lib.RG_DTYPE_BF16))
+
+
+@functools.lru_cache(maxsize=1024)
+def linear_gelu_pair_runs_serve(rows, K, N) -> bool:
+  """As linear_many_runs_serve."""
+  return bool(_lib.lib().rg_linear_gelu_pair_runs_serve(rows, K, N,
+                                                        _lib.RG_DTYPE_BF16))
+
+
 def _run_rows(t, runs):
   """Columns of a tensor that has the runs' rows."""
   assert t.numel() // t.shape[-1] == runs.rows, (t.shape, runs.rows)
@@ -828,10 +843,15 @@ def rope_pair(q, k, positions, inv_freq):
   return q_out, k_out
 
 
+def attention_prompt_row_fits(T, heads, head_dim):
+  """Whether the prompt-pass attention kernel takes rows of T tokens."""
+  return head_dim == 256 and T * heads * 512 < 2**31
+
+
 def attention_prefill_supported(q):
   """Shapes the prompt-pass attention kernel serves (rg_attention_prefill)."""
   return (q.is_cuda and q.dtype == torch.bfloat16 and q.ndim == 4 and
-          q.shape[-1] == 256 and q.shape[1] * q.shape[2] * 512 < 2**31)
+          attention_prompt_row_fits(*q.shape[1:]))
 
 
 def attention_prefill(q, k, v, first_key, scale):

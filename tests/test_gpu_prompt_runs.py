@@ -107,3 +107,26 @@ def test_prompts_without_their_padding(lengths, T):
   assert runs._prompt_runs(B, T, lens) is None
   handle.remove()
   assert runs._prompt_runs(B, T, lens) is not None
+
+
+@torch.no_grad()
+def test_prompts_beyond_what_the_products_address():
+  """Left-padded prompts of more rows than a product of runs takes: all rows, as a
+  sampler that knows of no runs."""
+  torch.manual_seed(12)
+  config = G.GriffinConfig(
+      vocab_size=64, width=256, mlp_expanded_width=16384, lru_width=256,
+      num_heads=1, block_types=(G.TemporalBlockType.RECURRENT,),
+      embeddings_scale_by_sqrt_dim=True, attention_window_size=64,
+      logits_soft_cap=30.0)
+  model = G.Griffin(config, device=DEV, dtype=torch.bfloat16).eval()
+  plain, runs = S.Sampler(model), S.Sampler(model)
+  plain._prompt_runs = lambda *a: None
+  lens = torch.full((32,), 900, device=DEV)
+  for T, fit in ((2032, True), (2033, False)):  # 64 992 rows, 65 024
+    tokens = torch.randint(1, 64, (32, T), device=DEV)
+    assert (runs._prompt_runs(32, T, lens) is not None) == fit
+    got, _ = runs.sample_tokens(tokens, lens, 2)
+    want, _ = plain.sample_tokens(tokens, lens, 2)
+    # (one launch or the library's sums in front of the roundings of one block)
+    assert torch.equal(got, want) if not fit else (got == want).float().mean() > 0.9
