@@ -109,17 +109,38 @@ def test_prompts_without_their_padding(lengths, T):
   assert runs._prompt_runs(B, T, lens) is not None
 
 
+def _small_model(**changes):
+  config = G.GriffinConfig(
+      vocab_size=64, width=256, mlp_expanded_width=256, lru_width=256,
+      num_heads=1, block_types=(G.TemporalBlockType.RECURRENT,),
+      embeddings_scale_by_sqrt_dim=True, attention_window_size=64,
+      logits_soft_cap=30.0)._replace(**changes)
+  return G.Griffin(config, device=DEV, dtype=torch.bfloat16).eval()
+
+
+@pytest.mark.parametrize("lens", [
+    torch.tensor([70]), torch.tensor([70.0]), torch.full((90,), 70.9)])
+@torch.no_grad()
+def test_lengths_as_positions_take_them(lens):
+  """One length for all rows, lengths that are no whole numbers: what the positions
+  are made of (broadcast, cut off) is what the padding is."""
+  torch.manual_seed(13)
+  model = _small_model()
+  tokens = torch.randint(1, 64, (90, 100), device=DEV)
+  plain, runs = S.Sampler(model), S.Sampler(model)
+  plain._prompt_runs = lambda *a: None
+  got, _ = runs.sample_tokens(tokens, lens.to(DEV), 2)
+  want, _ = plain.sample_tokens(tokens, lens.to(DEV), 2)
+  # (other sums in front of the roundings of one block)
+  assert (got == want).float().mean() > 0.9
+
+
 @torch.no_grad()
 def test_prompts_beyond_what_the_products_address():
   """Left-padded prompts of more rows than a product of runs takes: all rows, as a
   sampler that knows of no runs."""
   torch.manual_seed(12)
-  config = G.GriffinConfig(
-      vocab_size=64, width=256, mlp_expanded_width=16384, lru_width=256,
-      num_heads=1, block_types=(G.TemporalBlockType.RECURRENT,),
-      embeddings_scale_by_sqrt_dim=True, attention_window_size=64,
-      logits_soft_cap=30.0)
-  model = G.Griffin(config, device=DEV, dtype=torch.bfloat16).eval()
+  model = _small_model(mlp_expanded_width=16384)
   plain, runs = S.Sampler(model), S.Sampler(model)
   plain._prompt_runs = lambda *a: None
   lens = torch.full((32,), 900, device=DEV)
