@@ -97,15 +97,20 @@ class _CapturedStep:
 class Sampler:
   """Sampler for a Griffin model (greedy, or from the categorical
   distribution of the logits).  use_graph: decode steps replay a captured HIP
-  graph (same kernels, same results as the eager loop)."""
+  graph (same kernels, same results as the eager loop).  drop_padding: batches
+  of left-padded prompts with 8192 rows or more have their lengths read back, for
+  which the caller waits until the GPU has done what was queued before, and leave
+  the padding out where it is a tenth or more; False: sample_tokens reads nothing
+  back (but for an eos_token) and computes all rows."""
 
   def __init__(self, model: griffin_lib.Griffin, vocab=None,
                greedy_sampling: bool = True, is_it_model: bool = False,
-               use_graph: bool = False):
+               use_graph: bool = False, drop_padding: bool = True):
     self.model = model
     self.vocab = vocab
     self.greedy_sampling = greedy_sampling
     self.use_graph = use_graph
+    self.drop_padding = drop_padding
     self._captured = {}
     self._is_it_model = is_it_model
     self._eos_token = (None if vocab is None else torch.tensor(
@@ -135,16 +140,25 @@ class Sampler:
     multiplied in (3960 rows, 75 % of them real, 3 blocks: 9.75 -> 9.83 ms in
     all), and where a row has one token or none in front of its last, or is no
     left-padded row at all.  2B model, 16 prompts of 500 to 1000 tokens, 75 % of
-    the rows, and 32 tokens: 100.4 -> 93.2 ms."""
+    the rows, and 32 tokens: 100.4 -> 93.2 ms.
+
+    Prompts without padding pay for the read: 14 us of host time with the GPU
+    idle; of 2B generations (16 x 1000 + 4 tokens) queued one behind the other each
+    takes 60.7 ms with the read and 60.6 without, but holds its caller for 49 of
+    them instead of 5 (drop_padding).  What the model's layers are asked
+    (prompt_runs_serve, 240 us) comes behind the lengths: in front of them it had
+    every full batch wait, 62.4 ms a generation alone."""
     rows = batch_size * (length - 1)
-    if (batch_size < 2 or rows < 8192 or input_lengths.shape != (batch_size,) or
-        not self.model.prompt_runs_serve(batch_size, length - 1) or
+    if (not self.drop_padding or batch_size < 2 or rows < 8192 or
+        input_lengths.shape != (batch_size,) or self.device.type != "cuda" or
         torch.cuda.is_current_stream_capturing()):
       return None
     lengths = [int(n) - 1 for n in input_lengths.tolist()]
     if not all(1 <= n < length for n in lengths):
       return None
     if 8 * sum((n + 7) // 8 for n in lengths) > 0.9 * rows:
+      return None
+    if not self.model.prompt_runs_serve(batch_size, length - 1):
       return None
     return ops.RowRuns(lengths, length - 1, self.device)
 

@@ -151,3 +151,28 @@ def test_prompts_beyond_what_the_products_address():
     want, _ = plain.sample_tokens(tokens, lens, 2)
     # (one launch or the library's sums in front of the roundings of one block)
     assert torch.equal(got, want) if not fit else (got == want).float().mean() > 0.9
+
+
+@torch.no_grad()
+def test_lengths_are_read_where_they_may_be(monkeypatch):
+  """drop_padding=False reads nothing back; prompts without padding do not have the
+  model's layers looked at."""
+  model = _small_model()
+  tokens = torch.randint(1, 64, (90, 100), device=DEV)
+  full, half = (torch.full((90,), n, device=DEV) for n in (100, 50))
+  declined, runs = S.Sampler(model, drop_padding=False), S.Sampler(model)
+  declined.sample_tokens(tokens, half, 3)
+  torch.cuda.synchronize()
+  torch.cuda.set_sync_debug_mode("error")
+  try:
+    declined.sample_tokens(tokens, half, 3)
+    with pytest.raises(RuntimeError):
+      runs._prompt_runs(90, 100, half)
+  finally:
+    torch.cuda.set_sync_debug_mode("default")
+  asked = []
+  serve = model.prompt_runs_serve
+  monkeypatch.setattr(model, "prompt_runs_serve",
+                      lambda *a: asked.append(a) or serve(*a))
+  assert runs._prompt_runs(90, 100, full) is None and not asked
+  assert runs._prompt_runs(90, 100, half) is not None and asked == [(90, 99)]
