@@ -570,12 +570,24 @@ def _linear_gelu_pair_pays(M, K, N) -> bool:
                                                   _lib.RG_DTYPE_BF16))
 
 
+def _transformed(*tensors) -> bool:
+  """Whether torch.func (vmap, jvp, ..) or forward-mode differentiation stands
+  behind any of the tensors: only torch's operators see what they stand for."""
+  functorch, forward = torch._C._functorch, torch.autograd.forward_ad
+  if functorch.peek_interpreter_stack() is None and forward._current_level < 0:
+    return False
+  return any(functorch.is_functorch_wrapped_tensor(t) or
+             forward.unpack_dual(t).tangent is not None
+             for t in tensors if t is not None)
+
+
 def _as_they_lie(x, *others) -> bool:
   """Whether kernels may read x (bf16) and the others where they lie instead
   of torch's operators: plain dense tensors of one device and dtype, nothing
-  that autograd or autocast would see."""
+  that autograd, autocast or a transform would see."""
   grad = torch.is_grad_enabled()
-  return not torch.is_autocast_enabled("cuda") and all(
+  return not torch.is_autocast_enabled("cuda") and not _transformed(
+      x, *others) and all(
       t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and
                     t.dtype == torch.bfloat16 and t.device == x.device and
                     t.is_contiguous() and not (grad and t.requires_grad) and
