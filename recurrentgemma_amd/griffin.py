@@ -658,13 +658,16 @@ class Embedder(nn.Module):
   """Token table used for both the input embedding and the output logits
   (modules.py:935-1003)."""
 
+  # whether the logits of decode steps may keep a copy of the table (decode)
+  step_copy = True
+  _rows_logits = None  # (a pickle may be of a time when there was none)
+
   def __init__(self, vocab_size, embed_dim, scale_by_sqrt_dim, device=None,
                dtype=None):
     super().__init__()
     self.vocab_size = vocab_size
     self.embed_dim = embed_dim
     self.scale_by_sqrt_dim = scale_by_sqrt_dim
-    self._rows_logits = ops.PackedLinear()
     self.input_embedding = nn.Parameter(
         torch.empty([vocab_size, embed_dim], device=device, dtype=dtype))
     self.reset_parameters()
@@ -680,19 +683,30 @@ class Embedder(nn.Module):
       x = x * torch.tensor(math.sqrt(self.embed_dim)).type(torch.bfloat16)
     return x
 
-  def decode(self, x):
-    """Logits.  A few rows: the table streamed by the few-row kernel, from a
+  def decode(self, x, step=False):
+    """Logits.  step: of a decode step, which many more with the same table
+    follow.  A few rows of those: the table streamed by the few-row kernel, from a
     copy of its own in operand order (1.3 GB at 256000 x 2560).  us, library /
     this, replayed from a graph: 1 row 217 / 192, 8 220 / 195, 16 223 / 205, 24
     228 / 219, but 32 230 / 233, 64 246 / 279.  (Small tables, whose product takes
-    little more than a launch, are not worth the copy.)"""
+    little more than a launch, are not worth the copy.)  The copy is made by the
+    first step behind a write to the table, 600 us, what 25 to 60 steps bring in:
+    not for logits that are asked for once, not for a table whose writes nothing
+    counts (an inference tensor), not with step_copy = False."""
     table = self.input_embedding
-    if (0 < x.numel() <= 24 * self.embed_dim and self.vocab_size >= 32_000 and
+    if (step and self.step_copy and
+        0 < x.numel() <= 24 * self.embed_dim and self.vocab_size >= 32_000 and
         x.shape[-1:] == table.shape[1:] and not compiled.tracing() and
         ops.PackedLinear.usable(x, self.embed_dim, self.vocab_size) and
-        ops._as_they_lie(x, table)):
+        not table.is_inference() and ops._as_they_lie(x, table)):
+      if self._rows_logits is None:
+        self._rows_logits = ops.PackedLinear()
       return self._rows_logits(x, (table,))
     return x @ table.T
+
+
+# (an embedder's own or replaced method may take nothing but x)
+_EMBEDDER_DECODE = Embedder.decode
 
 
 class Griffin(nn.Module):
@@ -748,7 +762,11 @@ class Griffin(nn.Module):
       x = self.final_norm.add_then_norm(x.a, x.b)[1]
     else:
       x = self.final_norm(x)
-    logits = self.embedder.decode(x)
+    decode = self.embedder.decode
+    if (cache is not None and
+        getattr(decode, "__func__", None) is _EMBEDDER_DECODE):
+      decode = functools.partial(decode, step=True)
+    logits = decode(x)
     cap = self.config.logits_soft_cap
     if cap:
       logits = ops.soft_cap(logits, cap)

@@ -2,6 +2,8 @@
 or forward-mode differentiation stands behind to the operators (on the CPU: nothing is
 launched)."""
 
+import functools
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fwd
@@ -22,6 +24,7 @@ def embedder(monkeypatch):
   torch.manual_seed(3)
   e = G.Embedder(32_000, 64, True, dtype=torch.bfloat16)
   e.requires_grad_(False)
+  e.decode = functools.partial(e.decode, step=True)
   return e
 
 
