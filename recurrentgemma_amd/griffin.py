@@ -198,6 +198,10 @@ class MLPBlock(nn.Module):
     torch.nn.init.normal_(self.ffw_down.weight, mean=0.0, std=std)
     torch.nn.init.zeros_(self.ffw_down.bias)
 
+  def _behind_norm(self):
+    """As RecurrentBlock's."""
+    return 2 * self.expanded_width, True
+
   def forward(self, x, residual=None, defer_out=False):
     """residual: added to the result (the block's skip connection,
     modules.py:897-898).  defer_out: the caller normalises the result next and
@@ -342,6 +346,10 @@ class LocalAttentionBlock(nn.Module):
   @property
   def head_dim(self) -> int:
     return self.width // self.num_heads
+
+  def _behind_norm(self):
+    """As RecurrentBlock's."""
+    return self.width + 2 * self.head_dim, False
 
   def reset_parameters(self) -> None:
     for proj in (self.proj_q, self.proj_k, self.proj_v):
@@ -562,13 +570,15 @@ class LocalAttentionBlock(nn.Module):
 
 def _norm_for(reader, norm, x, addend):
   """(x + addend, norm of it) for a block that reads the norm: of partial sums,
-  left to the block's first layers to form in their own launch, as long as
-  nobody but the block's own code gets to see it."""
+  left to the block's first layers to form in their own launch, where that is
+  one for their sizes, and as long as nobody but the block's own code gets to see
+  it."""
   if (isinstance(x, ops.PartialSums) and x.flags is not None and
       type(norm) is RMSNorm and "add_then_norm" not in norm.__dict__ and
       not modules._global_hooks() and
       any(modules._as_written(reader, kind) for kind in
-          (modules.RecurrentBlock, LocalAttentionBlock, MLPBlock))):
+          (modules.RecurrentBlock, LocalAttentionBlock, MLPBlock)) and
+      ops.PendingNorm.served(x, *reader._behind_norm())):
     pending = ops.PendingNorm(x, addend, norm.scale, norm.eps)
     return pending.total, pending
   return norm.add_then_norm(x, addend)

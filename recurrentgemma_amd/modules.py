@@ -220,6 +220,11 @@ class RecurrentBlock(nn.Module):
     std = math.sqrt(self.final_w_init_variance_scale / self.lru_width)
     torch.nn.init.normal_(w, mean=0.0, std=std)
 
+  def _behind_norm(self):
+    """Weight rows of the layers that read a decode step's x in one launch, and
+    whether they are the MLP's pair."""
+    return 2 * self.lru_width, False
+
   def forward(self, x, segment_pos, cache=None, return_cache=True,
               defer_out=False):
     """defer_out: the caller adds the result to a residual and normalises it

@@ -1164,12 +1164,24 @@ class PartialSums:
     return out if self.addend is None else out + self.addend
 
 
+@functools.lru_cache(maxsize=256)
+def _norm_served(M, K, N, gelu_pair) -> bool:
+  return bool(_lib.lib().rg_linear_rows_normed_serve(M, K, N, int(gelu_pair)))
+
+
 class PendingNorm:
   """add_rms_norm of PartialSums, not formed yet: the few-row layers that read
   the norm next do it in their own launch (PackedLinear), `tensor()` in one of
   its own.  total: the sum that was normed, good from then on."""
 
   is_cuda = True
+
+  @staticmethod
+  def served(sums, N, gelu_pair) -> bool:
+    """Whether layers of N weight rows that read the norm of PartialSums have it
+    in their own launch; elsewhere a norm is better formed at once."""
+    _, M, K = sums.sums.shape
+    return _norm_served(M, K, N, gelu_pair)
 
   def __init__(self, sums, addend, scale, eps):
     self.args = _partial_norm_args(sums, addend, scale)
@@ -1361,7 +1373,7 @@ class PackedLinear:
     lib = _lib.lib()
     if (x.shape[-1] != K or x.dtype != weights[0].dtype or
         x.device != weights[0].device or
-        not lib.rg_linear_rows_normed_serve(M, K, N, int(self.gelu_pair))):
+        not _norm_served(M, K, N, self.gelu_pair)):
       return None
     copied, aside = 0, None
     if state is not None:
