@@ -525,12 +525,14 @@ class LocalAttentionBlock(nn.Module):
       raise TypeError("AttentionBlockCache.num_tokens must be int32")
     qkv = self._rows_qkv(
         x, (self.proj_q.weight, self.proj_k.weight, self.proj_v.weight))
-    qkv = qkv.reshape(b, self.width + 2 * self.head_dim)
+    if isinstance(qkv, tuple):  # (one head: three layers of equal size)
+      q, k, v = (t.reshape(b, self.head_dim) for t in qkv)
+    else:
+      q, k, v = qkv.reshape(b, -1).split(
+          (self.width, self.head_dim, self.head_dim), dim=1)
     out = ops.attention_decode_fused(
-        qkv[:, :self.width], qkv[:, self.width:self.width + self.head_dim],
-        qkv[:, self.width + self.head_dim:], segment_pos, self._inv_freq,
-        cache.keys, cache.values, cache.num_tokens, self.head_dim ** -0.5,
-        update_cache=return_cache)
+        q, k, v, segment_pos, self._inv_freq, cache.keys, cache.values,
+        cache.num_tokens, self.head_dim ** -0.5, update_cache=return_cache)
     out = self._project_out(out.reshape(b, 1, self.width), defer_out)
     return out, (cache if return_cache else None)
 

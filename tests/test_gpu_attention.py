@@ -368,3 +368,30 @@ def test_attention_decode_fused_refuses_what_it_cannot_run():
   assert not ops.attention_decode_fused_supported(x, 10, 128, 2048)
   assert not ops.attention_decode_fused_supported(x, 10, 256, 16385)
   assert not ops.attention_decode_fused_supported(x.float(), 10, 256, 2048)
+
+
+@pytest.mark.parametrize("heads", [1, 2])
+@torch.no_grad()
+def test_attention_block_step_of_one_head(heads):
+  """One head: queries, keys and values come from three layers of equal size."""
+  torch.manual_seed(4)
+  block = griffin.LocalAttentionBlock(
+      width=256 * heads, num_heads=heads, window_size=8, device=DEV,
+      dtype=torch.bfloat16)
+  x = torch.randn(3, 1, 256 * heads, device=DEV).bfloat16()
+  pos = torch.tensor([[5], [0], [9]], device=DEV, dtype=torch.int32)
+  g = torch.Generator(device=DEV).manual_seed(5)
+  cache = block.init_cache(3, 8, 256, torch.bfloat16, device=DEV)
+  cache.keys.normal_(generator=g)
+  cache.values.normal_(generator=g)
+  cache.num_tokens.copy_(pos[:, 0])
+  other = type(cache)(*(t.clone() for t in cache))
+  got, cache = block(x, pos, cache)
+  q, k, v = (p(x)[:, 0] for p in (block.proj_q, block.proj_k, block.proj_v))
+  want = block.proj_final(ops.attention_decode_fused(
+      q, k, v, pos, block._inv_freq, other.keys, other.values, other.num_tokens,
+      256 ** -0.5).reshape(3, 1, -1))
+  # (other sums in front of the roundings of two layers and of what is between them)
+  assert helpers.max_rel(got, want) < 4 * 2**-8
+  for a, b in zip(cache, other):
+    assert helpers.max_rel(a, b) < 2 * 2**-8
