@@ -109,6 +109,51 @@ def test_prompts_without_their_padding(lengths, T):
   assert runs._prompt_runs(B, T, lens) is not None
 
 
+@pytest.mark.parametrize("lengths,T,window", [
+    ([301, 2, 100, 299, 17, 8, 150, 64, 33, 200], 301, 64),
+    ([90, 1, 47, 3], 97, 2048), ([5, 40, 33], 40, 32)])
+@torch.no_grad()
+def test_cache_without_the_padding(lengths, T, window):
+  """Every state that prompt_cache leaves against forward's for the same prompts: h,
+  the conv's rows (some of them padding), the rings as far as a step sees them."""
+  torch.manual_seed(14)
+  kinds = (G.TemporalBlockType.RECURRENT, G.TemporalBlockType.ATTENTION,
+           G.TemporalBlockType.RECURRENT)
+  model = _small_model(width=512, mlp_expanded_width=1536, lru_width=512,
+                       num_heads=2, attention_window_size=window,
+                       block_types=kinds)
+  B = len(lengths)
+  tokens = torch.randint(1, 64, (B, T), device=DEV)
+  pos = (torch.arange(T) - T + torch.tensor(lengths)[:, None]).clip(min=-1).to(
+      DEV, torch.int32)
+  assert model.prompt_runs_serve(B, T)
+  _, want = model(tokens, pos, None, return_logits=False)
+  junk = [torch.full((1 << 22,), float("nan"), device=DEV) for _ in range(8)]
+  del junk
+  got = model.prompt_cache(tokens, pos, ops.RowRuns(lengths, T, DEV))
+
+  def near(a, b, tensors):
+    """Other sums in front of the roundings of so many tensors."""
+    a, b = a.double(), b.double()
+    assert torch.isfinite(a).all()
+    assert (a - b).norm() <= tensors ** 0.5 * 2**-8 * b.norm()
+
+  assert got.keys() == want.keys()
+  for i, kind in enumerate(kinds):
+    a, b = got[f"blocks.{i}"], want[f"blocks.{i}"]
+    tensors = 4 + 10 * i
+    assert [t.dtype for t in a] == [t.dtype for t in b]
+    for row, n in enumerate(lengths):
+      if kind is G.TemporalBlockType.RECURRENT:
+        near(a.rg_lru_state[row], b.rg_lru_state[row], tensors)
+        near(a.conv1d_state[row], b.conv1d_state[row], tensors)
+        continue
+      assert a.num_tokens[row] == b.num_tokens[row] == n
+      seen = torch.arange(max(0, n - window), n) % window
+      near(a.keys[row, seen], b.keys[row, seen], tensors)
+      near(a.values[row, seen], b.values[row, seen], tensors)
+
+
 def _small_model(**changes):
   config = G.GriffinConfig(
       vocab_size=64, width=256, mlp_expanded_width=256, lru_width=256,
