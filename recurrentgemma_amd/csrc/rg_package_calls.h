@@ -133,8 +133,7 @@ int rg_recurrent_step_join(const void* x, const void* gate_branch, const void* s
  * normed are written whole) and rg_linear_rows of normed, without a residual, as one
  * launch, with `bytes` copied as in rg_linear_rows_beside (0: none).  The flags serve one
  * such launch.  patience: how often its workgroups look for the rows' norm before they
- * form it themselves, at least a microsecond each.  out has the same bits as the two
- * calls.  RG_ERR_UNSUPPORTED where *_serve says 0. */
+ * form it themselves.  out has the same bits as the two calls.  RG_ERR_UNSUPPORTED where *_serve says 0. */
 #define RG_NORM_FLAGS 64
 int rg_linear_rows_partial_flags(const void* x, const void* w_packed, void* partial,
                                  uint32_t* flags, int M, int K, int N, int slices,

@@ -1450,13 +1450,15 @@ bool prefill_many_serve(int B, int H, int T, int bw, bool joined) {
 bool prefill_narrow_pays(int B, int H, int T, int W) {
   // Against the gate GEMM, the scan and the join as passes of their own: 34 us +
   // 0.0255 us a token of width 5632, as measured at 32 heads of 176.  Checked at 8,
-  // 20 and 32 heads of 136, 152, .. 248 channels, one row of 64 to 64 rows of 128
-  // and 16 of 2048, joined and not (540 pairs of times): whatever it sends here is
-  // faster here (us, apart / here, joined: 8 heads of 136 B8 T64 25 / 11, B16 T2048
-  // 200 / 125; 20 of 200 B32 T512 300 / 248; 32 of 248 B4 T4096 533 / 371, B64 T128
-  // 295 / 207), 30 times it keeps a few long rows apart that would be 1 to 19 %
-  // faster here (8 heads of 248 B4 T4096 199 / 173); one of 4096 tokens in 8 heads
-  // is better apart (184 wide 86 / 171).
+  // 20 and 32 heads of 136, 152, 176, 184, 200 and 248 channels, one row of 64 to 64
+  // rows of 128 and 16 of 2048, joined and not, from a graph (576 pairs of times):
+  // whatever it sends here is faster here, by 6 % or more (us, apart / here, joined: 8
+  // heads of 136 B8 T64 22 / 11, B16 T2048 197 / 112; 20 of 200 B32 T512 310 / 262; 32
+  // of 176 B4 T2048 228 / 118, B64 T27 77 / 46; 32 of 248 B4 T4096 561 / 406, B64 T128
+  // 305 / 223).  48 times it keeps rows of 1000 to 4096 tokens apart that would be 1 to
+  // 28 % faster here, where a pass takes less than `plan` allows for it
+  // (32 of 200 B1 T2048 109 / 87, 8 of 248 B4 T4096 203 / 167); one of 4096 tokens in 8
+  // heads is better apart (184 wide 80 / 164).
   const float apart = 34.0f + 0.0255f / 5632 * (float)B * T * W;
   return plan(B, H, T, W / H, true).split.us < apart;
 }

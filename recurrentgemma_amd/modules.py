@@ -151,11 +151,14 @@ def _recurrent_core(conv_1d, rg_lru, x, segment_pos, cache, return_cache,
     # and 256-wide heads the single-launch kernel, one workgroup per (row,
     # head), per 32 channels of one (few rows of some hundred tokens), per
     # chunk of one (few long ones) or by blocks of 32 tokens (pairs that
-    # do not come out even on the CUs); many rows of a few tokens and every
-    # other dtype or head width: gate GEMM + scan; float32 with 256-wide heads:
-    # one launch for few short rows, else conv, projections and recurrence; and
-    # the join with the gate branch inside those kernels (after the two-kernel
-    # form it is a pass of its own).
+    # do not come out even on the CUs), or several whole rows of up to 16 tokens
+    # to a tile; for bf16 heads of 136 to 248 channels slices of heads, alike;
+    # 256-wide heads beyond 512 pairs of rows that short or 1024 of up to 32
+    # tokens, a few long rows of narrower heads, and every other head width: gate
+    # GEMM + scan; float32 with 256-wide heads: one launch
+    # for few short rows, else conv, projections and recurrence; and the join with
+    # the gate branch inside those kernels (after the two-kernel form it is a pass
+    # of its own).
     if compiled.tracing():
       y, h, conv_state = torch.ops.recurrentgemma_amd.recurrent_core(
           x, segment_pos, *weights, None, gate_branch)

@@ -1135,7 +1135,7 @@ def packed_gate_weights(w_x, w_a):
 
 NORM_FLAGS = 64  # RG_NORM_FLAGS
 # How often a workgroup looks for a norm that others of its launch form, before
-# it forms the norm itself: some 0.3 ms.
+# it forms the norm itself (to be found running late, not to be waited out).
 NORM_PATIENCE = 512
 
 
@@ -1477,9 +1477,9 @@ def recurrent_step(x, segment_pos, conv_cache, h, conv_w, conv_b, w_x, b_x, w_a,
                    conv_aside=None):
   """One decode step of conv -> RG-LRU.  Returns (y, h_new, conv_cache_new).
 
-  bf16 with 256-wide heads runs as one launch on re-laid-out gate weights
-  (packed once per weight version); other shapes as conv step + gate GEMM +
-  scan step.  gate_branch: the block's linear_y output [B,1,W]; y is then
+  256-wide heads run as one launch: bf16 on re-laid-out gate weights (packed once
+  per weight version), float32 where no cache is updated in place (nothing written
+  is read); everything else as conv step + gate GEMM + scan step.  gate_branch: the block's linear_y output [B,1,W]; y is then
   y * gelu(gate_branch) (inside the one launch where that runs).  conv_aside: a
   copy of conv_cache made earlier on the stream (PackedLinear.beside); reading
   it, a step in place may share heads among workgroups."""
