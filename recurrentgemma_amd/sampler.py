@@ -150,6 +150,7 @@ class Sampler:
     every full batch wait, 62.4 ms a generation alone."""
     rows = batch_size * (length - 1)
     if (not self.drop_padding or batch_size < 2 or rows < 8192 or
+        not isinstance(self.model, griffin_lib.Griffin) or
         input_lengths.shape != (batch_size,) or self.device.type != "cuda" or
         torch.cuda.is_current_stream_capturing()):
       return None

@@ -221,3 +221,26 @@ def test_lengths_are_read_where_they_may_be(monkeypatch):
                       lambda *a: asked.append(a) or serve(*a))
   assert runs._prompt_runs(90, 100, full) is None and not asked
   assert runs._prompt_runs(90, 100, half) is not None and asked == [(90, 99)]
+
+
+class _Around(torch.nn.Module):
+  """A caller's own module around the model, with what the sampler asks of one."""
+
+  def __init__(self, model):
+    super().__init__()
+    self.inner, self.calls = model, 0
+    self.config, self.blocks = model.config, model.blocks
+    self.init_cache = model.init_cache
+
+  def forward(self, *args, **kwargs):
+    self.calls += 1
+    return self.inner(*args, **kwargs)
+
+
+@torch.no_grad()
+def test_a_model_of_the_callers_own_is_called():
+  model = _Around(_small_model())
+  tokens = torch.randint(1, 64, (90, 100), device=DEV)
+  lens = torch.full((90,), 50, device=DEV)
+  S.Sampler(model).sample_tokens(tokens, lens, 3)
+  assert model.calls == 4  # the prompt, its last token, two steps
