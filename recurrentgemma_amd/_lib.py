@@ -137,6 +137,8 @@ PACKAGE_SIGNATURES = {
     "rg_linear_gelu_pair": (_i, [_vp] * 4 + [_i64, _i, _i, _i, _vp]),
     "rg_linear_many_runs_serve": (_i, [_i64, _i, _i, _vp, _i]),
     "rg_linear_gelu_pair_runs_serve": (_i, [_i64, _i, _i, _i]),
+    "rg_linear_many_runs_saves_us": (ctypes.c_double, [_i64, _i, _i, _i, _vp, _i]),
+    "rg_linear_gelu_pair_runs_saves_us": (ctypes.c_double, [_i64, _i, _i, _i, _i]),
     "rg_linear_many_runs": (_i, [_vp, _i64, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp]),
     "rg_linear_gelu_pair_runs": (_i, [_vp] * 4 + [_i64, _vp, _i, _i, _i, _i, _vp]),
     "rg_add_rms_norm_runs": (_i, [_vp] * 6 + [_i, _i, ctypes.c_float, _i, _vp]),

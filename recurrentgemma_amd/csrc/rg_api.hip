@@ -1326,6 +1326,20 @@ int rg_linear_many_runs_serve(int64_t rows, int K, int layers, const int* N, int
          with_runs(&a, rows, &kOneRun) && rg::matmul_serves(a, rg::kMatmulForward);
 }
 
+double rg_linear_many_runs_saves_us(int64_t rows, int count, int K, int layers,
+                                    const int* N, int dtype) {
+  rg::MatmulArgs all, some;
+  if (!rg_linear_many_runs_serve(rows, K, layers, N, dtype) ||
+      !runs_fit(rows, &kOneRun, count) ||
+      !linear_many_args(nullptr, rows, K, layers, nullptr, nullptr, nullptr, N, &all) ||
+      !linear_many_args(nullptr, 8ll * count, K, layers, nullptr, nullptr, nullptr, N,
+                        &some))
+    return -1e30;
+  with_runs(&some, rows, &kOneRun);
+  return (double)rg::matmul_us(all, rg::kMatmulForward) -
+         rg::matmul_us(some, rg::kMatmulForward);
+}
+
 // (runs: of M rows those in run_count runs of eight)
 #undef RG_WHO
 #define RG_WHO who
@@ -1490,6 +1504,19 @@ int rg_linear_gelu_pair_runs_serve(int64_t rows, int K, int N, int dtype) {
   return dtype == RG_DTYPE_BF16 && runs_fit(rows, &kOneRun, 1) &&
          gelu_pair_args(nullptr, nullptr, nullptr, nullptr, 8, K, N, &a) &&
          with_runs(&a, rows, &kOneRun) && rg::matmul_serves(a, rg::kMatmulGeluPair);
+}
+
+double rg_linear_gelu_pair_runs_saves_us(int64_t rows, int count, int K, int N,
+                                         int dtype) {
+  rg::MatmulArgs all, some;
+  if (!rg_linear_gelu_pair_runs_serve(rows, K, N, dtype) ||
+      !runs_fit(rows, &kOneRun, count) ||
+      !gelu_pair_args(nullptr, nullptr, nullptr, nullptr, rows, K, N, &all) ||
+      !gelu_pair_args(nullptr, nullptr, nullptr, nullptr, 8ll * count, K, N, &some))
+    return -1e30;
+  with_runs(&some, rows, &kOneRun);
+  return (double)rg::matmul_us(all, rg::kMatmulGeluPair) -
+         rg::matmul_us(some, rg::kMatmulGeluPair);
 }
 
 #undef RG_WHO

@@ -308,6 +308,7 @@ struct MatmulArgs {
 // Whether the launch can be made; and (but for weight gradients) whether it is ahead of
 // the library's products.
 bool matmul_serves(const MatmulArgs& a, int kind);
+float matmul_us(const MatmulArgs& a, int kind);
 bool matmul_pays(const MatmulArgs& a, int kind);
 hipError_t launch_matmul(MatmulArgs a, int kind, hipStream_t s);
 

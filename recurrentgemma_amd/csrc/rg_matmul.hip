@@ -691,10 +691,7 @@ bool matmul_serves(const MatmulArgs& a, int kind) {
 // rows 10.8 / 11.3), 70 to 300 rows 2560 -> 256 7 / 11 and back 8 / 13.5, the pair so 17 /
 // 19; of the other calls of a block 70 rows 2560 -> 2560 twice 17 / 12, thrice 30 / 13, the
 // pair 2560 -> 7680 34 / 20, so that a captured step of more than 64 sequences gains.
-bool matmul_pays(const MatmulArgs& a, int kind) {
-  if (!matmul_serves(a, kind)) return false;
-  int tile;
-  const float own = best_tile(a, kind, &tile);
+static float library_us(const MatmulArgs& a, int kind) {
   constexpr float kCall = 14.0f;
   float library = 0.0f;
   for (int i = 0; i < a.count; ++i) {
@@ -712,7 +709,20 @@ bool matmul_pays(const MatmulArgs& a, int kind) {
       if (kind == kMatmulGeluPair) library += 3.0f + 1.2e-6f * (float)p.M * (float)p.N;
     }
   }
-  return own < library;
+  return library;
+}
+
+bool matmul_pays(const MatmulArgs& a, int kind) {
+  int tile;
+  return matmul_serves(a, kind) && best_tile(a, kind, &tile) < library_us(a, kind);
+}
+
+// What the products take where they are run better: here or by the library, which has
+// no runs.
+float matmul_us(const MatmulArgs& a, int kind) {
+  int tile;
+  const float own = matmul_serves(a, kind) ? best_tile(a, kind, &tile) : 1e30f;
+  return a.runs ? own : fminf(own, library_us(a, kind));
 }
 
 hipError_t launch_matmul(MatmulArgs a, int kind, hipStream_t s) {

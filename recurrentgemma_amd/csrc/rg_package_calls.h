@@ -81,9 +81,14 @@ int rg_linear_gelu_pair(const void* x, const void* w, const void* bias, void* ou
  * `runs` (on the GPU, 0 .. rows - 8, any order, overlaps allowed); nothing else is read or
  * written.  RG_ERR_UNSUPPORTED beyond the sizes of those calls (norm: rows of at most 4096
  * in eights).  *_serve: whether tensors of `rows` rows are within them: (rows + 512) times
- * the widest of K and N below 2^30, however few rows the runs have. */
+ * the widest of K and N below 2^30, however few rows the runs have.  *_saves_us: what
+ * `count` runs take less than all rows as they are run better, here or by the library, by
+ * the times that their rules go by (below zero: they take more). */
 int rg_linear_many_runs_serve(int64_t rows, int K, int layers, const int* N, int dtype);
 int rg_linear_gelu_pair_runs_serve(int64_t rows, int K, int N, int dtype);
+double rg_linear_many_runs_saves_us(int64_t rows, int count, int K, int layers,
+                                    const int* N, int dtype);
+double rg_linear_gelu_pair_runs_saves_us(int64_t rows, int count, int K, int N, int dtype);
 int rg_linear_many_runs(const void* x, int64_t rows, const int32_t* runs, int count, int K,
                         int layers, const void* const* w, const void* const* bias,
                         void* const* out, const int* N, int dtype, void* stream);

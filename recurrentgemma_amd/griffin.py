@@ -842,6 +842,38 @@ class Griffin(nn.Module):
         return False
     return True
 
+  def prompt_runs_pay(self, batch_size, tokens, count) -> bool:
+    """Whether prompt_cache with so many runs is ahead of forward: whether its
+    products and norms save more than what is beside them, 75 us a block (zeroed
+    tensors, large tiles whatever the rows, calls by way of Python).  Prompt passes,
+    all rows / runs, ms, and saved by the estimate, us a block: 6 blocks of width 512,
+    16 x 512 tokens 75 % real 0.93 / 1.22 (-11), 60 x 500 76 % 2.34 / 2.48 (20), 61 %
+    2.35 / 2.22 (48); 6 of 1536, 60 x 500 90 % 10.03 / 10.36 (74), 75 % 9.99 / 8.84;
+    12 of 2560, 16 x 512 90 % 12.76 / 12.49 (72), 83 % 12.78 / 12.05 (77), 75 %
+    12.74 / 10.55 (249); 3 of 4096, 16 x 512 90 % 7.23 / 7.64 (45), 64 x 128 85 %
+    7.32 / 7.39 (69), 16 x 512 75 % 7.27 / 6.30 (409), 16 x 1000 89 % 14.29 / 13.39
+    (307).  Of 210 passes of widths 512 to 4096, 8192 to 30000 rows, 60 to 90 % real,
+    one that goes by runs is slower (2560 x 3, 60 x 500 90 %: 11.66 / 11.75)."""
+    c = self.config
+    rows, lru_width = batch_size * tokens, c.lru_width or c.width
+    many = ops.linear_many_runs_saves_us
+    blocks = len(c.block_types)
+    recurrent = sum(kind is TemporalBlockType.RECURRENT for kind in c.block_types)
+    # (two norms a block: two tensors read, two written, at 4.5 TB/s)
+    saved = blocks * (
+        ops.linear_gelu_pair_runs_saves_us(rows, count, c.width,
+                                           c.mlp_expanded_width) +
+        many(rows, count, c.mlp_expanded_width, c.width) +
+        (rows - 8 * count) * c.width * 16 / 4.5e6)
+    if recurrent:
+      saved += recurrent * (many(rows, count, c.width, lru_width, lru_width) +
+                            many(rows, count, lru_width, c.width))
+    if recurrent < blocks:
+      saved += (blocks - recurrent) * (
+          many(rows, count, c.width, c.width, 256, 256) +
+          many(rows, count, c.width, c.width))
+    return saved > 75 * blocks
+
   @torch.no_grad()
   def prompt_cache(self, tokens, segment_pos, runs: ops.RowRuns) -> Cache:
     """The cache that forward(tokens, segment_pos) leaves, for left-padded

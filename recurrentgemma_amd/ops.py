@@ -685,6 +685,20 @@ def linear_gelu_pair_runs_serve(rows, K, N) -> bool:
                                                         _lib.RG_DTYPE_BF16))
 
 
+def linear_many_runs_saves_us(rows, count, K, *features) -> float:
+  """What linear_many_runs of so many runs takes less, in microseconds, than the
+  layers over all rows (their kernels' or the library's products): an estimate."""
+  sizes = (ctypes.c_int * len(features))(*features)
+  return _lib.lib().rg_linear_many_runs_saves_us(
+      rows, count, K, len(features), sizes, _lib.RG_DTYPE_BF16)
+
+
+def linear_gelu_pair_runs_saves_us(rows, count, K, N) -> float:
+  """As linear_many_runs_saves_us."""
+  return _lib.lib().rg_linear_gelu_pair_runs_saves_us(rows, count, K, N,
+                                                      _lib.RG_DTYPE_BF16)
+
+
 def _run_rows(t, runs):
   """Columns of a tensor that has the runs' rows."""
   assert t.numel() // t.shape[-1] == runs.rows, (t.shape, runs.rows)

@@ -133,14 +133,15 @@ class Sampler:
       return ops.argmax_last(logits)
     return torch.distributions.Categorical(logits=logits).sample()
 
-  def _prompt_runs(self, batch_size, length, input_lengths):
+  def _prompt_runs(self, batch_size, length, input_lengths, pay=None):
     """The rows of the prompts but their last tokens that are worth computing,
     or None for all of them: where too few are padding to pay for reading the
     lengths back (a synchronisation) and for the large tiles that rows in runs are
     multiplied in (3960 rows, 75 % of them real, 3 blocks: 9.75 -> 9.83 ms in
     all), and where a row has one token or none in front of its last, or is no
     left-padded row at all.  2B model, 16 prompts of 500 to 1000 tokens, 75 % of
-    the rows, and 32 tokens: 100.4 -> 93.2 ms.
+    the rows, and 32 tokens: 100.4 -> 93.2 ms.  pay: as Griffin.prompt_runs_pay,
+    asked in front of the lengths, too, about a token or so of each row.
 
     Prompts without padding pay for the read: 14 us of host time with the GPU
     idle; of 2B generations (16 x 1000 + 4 tokens) queued one behind the other each
@@ -154,10 +155,14 @@ class Sampler:
         input_lengths.shape != (batch_size,) or self.device.type != "cuda" or
         torch.cuda.is_current_stream_capturing()):
       return None
+    if pay is not None and not pay(batch_size, length - 1, batch_size):
+      return None
     lengths = [int(n) - 1 for n in input_lengths.tolist()]
     if not all(1 <= n < length for n in lengths):
       return None
-    if 8 * sum((n + 7) // 8 for n in lengths) > 0.9 * rows:
+    count = sum((n + 7) // 8 for n in lengths)
+    if (8 * count > 0.9 * rows or
+        pay is not None and not pay(batch_size, length - 1, count)):
       return None
     if not self.model.prompt_runs_serve(batch_size, length - 1):
       return None
@@ -210,7 +215,8 @@ class Sampler:
       # they are asked for
       before = positions[:, :-1].contiguous()
       runs = (None if return_logits and echo else
-              self._prompt_runs(bsz, plen, input_lengths))
+              self._prompt_runs(bsz, plen, input_lengths,
+                                getattr(model, "prompt_runs_pay", None)))
       if runs is not None:
         cache = model.prompt_cache(padded_tokens[:, :-1], before, runs)
       else:

@@ -160,7 +160,9 @@ def _small_model(**changes):
       num_heads=1, block_types=(G.TemporalBlockType.RECURRENT,),
       embeddings_scale_by_sqrt_dim=True, attention_window_size=64,
       logits_soft_cap=30.0)._replace(**changes)
-  return G.Griffin(config, device=DEV, dtype=torch.bfloat16).eval()
+  model = G.Griffin(config, device=DEV, dtype=torch.bfloat16).eval()
+  model.prompt_runs_pay = lambda *a: True  # (of such a size it never does)
+  return model
 
 
 @pytest.mark.parametrize("lens", [
@@ -244,3 +246,33 @@ def test_a_model_of_the_callers_own_is_called():
   lens = torch.full((90,), 50, device=DEV)
   S.Sampler(model).sample_tokens(tokens, lens, 3)
   assert model.calls == 4  # the prompt, its last token, two steps
+
+
+@torch.no_grad()
+def test_prompts_without_their_padding_where_it_pays(monkeypatch):
+  """As test_prompts_without_their_padding, at a width where the sampler goes by runs
+  of itself; and a narrow model, whose lengths are not even read."""
+  model = _small_model(width=2560, mlp_expanded_width=7680, lru_width=2560,
+                       num_heads=10, block_types=(
+                           G.TemporalBlockType.RECURRENT,
+                           G.TemporalBlockType.ATTENTION))
+  del model.prompt_runs_pay
+  lengths = [301, 2, 100, 299, 17, 8, 150, 64, 33, 200] * 3
+  tokens = torch.randint(1, 64, (30, 301), device=DEV)
+  lens = torch.tensor(lengths, device=DEV)
+  plain, runs = S.Sampler(model, drop_padding=False), S.Sampler(model)
+  want, _ = plain.sample_tokens(tokens, lens, 4)
+  took = []
+  cache = model.prompt_cache
+  monkeypatch.setattr(model, "prompt_cache", lambda *a: took.append(a) or cache(*a))
+  got, _ = runs.sample_tokens(tokens, lens, 4)
+  assert len(took) == 1
+  # (other sums in front of the roundings of two blocks)
+  assert (got == want).float().mean() > 0.9
+  narrow = _small_model()
+  del narrow.prompt_runs_pay
+  torch.cuda.set_sync_debug_mode("error")
+  try:
+    assert S.Sampler(narrow)._prompt_runs(30, 301, lens, narrow.prompt_runs_pay) is None
+  finally:
+    torch.cuda.set_sync_debug_mode("default")

@@ -59,3 +59,25 @@ def test_what_serve_refuses_the_call_refuses(rows, K, N):
       at[0], rows, at[4], 1, K, 1, one(at[1]), one(None), one(at[2]), n,
       _lib.RG_DTYPE_BF16, None) == -2
   assert ops.linear_many_runs_serve(8, 2560, 7680, 7680)
+
+
+@pytest.mark.parametrize("changes,batch,tokens,real,pays", [
+    # (measured passes; 3 blocks each)
+    (dict(width=512, num_heads=2, lru_width=512, mlp_expanded_width=1536), 16, 512,
+     0.5, False),
+    (dict(width=512, num_heads=2, lru_width=512, mlp_expanded_width=1536), 60, 500,
+     0.75, False),
+    (dict(), 16, 1000, 0.75, True), (dict(), 64, 128, 0.85, True),
+    (dict(), 16, 1000, 1.0, False),
+    (dict(width=4096, num_heads=16, lru_width=4096, mlp_expanded_width=12288), 16, 512,
+     0.9, False),
+    (dict(width=4096, num_heads=16, lru_width=4096, mlp_expanded_width=12288), 16, 512,
+     0.75, True)])
+def test_where_leaving_padding_out_pays(changes, batch, tokens, real, pays):
+  R, A = G.TemporalBlockType.RECURRENT, G.TemporalBlockType.ATTENTION
+  for kinds in ((R, R, A), (R,), (A, A)):
+    model = _model(G.Preset.RECURRENT_GEMMA_2B_V1, block_types=kinds, **changes)
+    count = int(batch * tokens * real / 8)
+    assert model.prompt_runs_pay(batch, tokens, count) == pays
+  # beyond what the products address: never
+  assert not model.prompt_runs_pay(batch * 1000, tokens, count)
