@@ -695,19 +695,34 @@ class Embedder(nn.Module):
       x = x * torch.tensor(math.sqrt(self.embed_dim)).type(torch.bfloat16)
     return x
 
+  def _steps_stream(self) -> bool:
+    """Whether up to 24 rows of logits are better formed by the few-row kernel (64
+    rows of the table a workgroup): where a workgroup has a stretch of the table that
+    is long beside what it begins and ends with, and the last workgroups fill the CUs.
+    us, library / this, 16 rows, replayed from a graph over tables that together fill
+    no cache: 32000 x 1024 17 / 14, x 2560 38 / 29, 100000 x 1024 44 / 37, 256000 x
+    1024 98 / 95, x 2048 234 / 173, x 2560 234 / 210 (1 row 226 / 198, 24 238 / 226, 32
+    rows the library's), x 4096 425 / 380; but 50304 (three rounds and a few) x 1024
+    21.8 / 24.2, x 4096 81 / 89, 256000 x 256 33 / 43, x 512 57 / 60.  From 1024
+    features on and with rounds so full, 14 tables of 32000 to 300000 rows are ahead by
+    1 to 130 % (two at 24 rows of 1024 behind by 1 %); 128256 x 4096 is behind by 1 to 5
+    %.  Smaller tables take little more than a launch and are not worth the copy."""
+    rounds = self.vocab_size / (64 * 256)
+    return (self.vocab_size >= 32_000 and self.vocab_size % 64 == 0 and
+            1024 <= self.embed_dim <= 4096 and
+            rounds >= 0.8 * math.ceil(rounds))
+
   def decode(self, x, step=False):
     """Logits.  step: of a decode step, which many more with the same table
     follow.  A few rows of those: the table streamed by the few-row kernel, from a
-    copy of its own in operand order (1.3 GB at 256000 x 2560).  us, library /
-    this, replayed from a graph: 1 row 217 / 192, 8 220 / 195, 16 223 / 205, 24
-    228 / 219, but 32 230 / 233, 64 246 / 279.  (Small tables, whose product takes
-    little more than a launch, are not worth the copy.)  The copy is made by the
-    first step behind a write to the table, 600 us, what 25 to 60 steps bring in:
-    not for logits that are asked for once, not for a table whose writes nothing
-    counts (an inference tensor), not with step_copy = False."""
+    copy of its own in operand order (1.3 GB at 256000 x 2560), where that is ahead
+    (_steps_stream).  The copy is made by the first step behind a write to the table,
+    600 us, what 25 to 60 steps bring in: not for logits that are asked for once, not
+    for a table whose writes nothing counts (an inference tensor), not with step_copy
+    = False."""
     table = self.input_embedding
     if (step and self.step_copy and
-        0 < x.numel() <= 24 * self.embed_dim and self.vocab_size >= 32_000 and
+        0 < x.numel() <= 24 * self.embed_dim and self._steps_stream() and
         x.shape[-1:] == table.shape[1:] and not compiled.tracing() and
         ops.PackedLinear.usable(x, self.embed_dim, self.vocab_size) and
         not table.is_inference() and ops._as_they_lie(x, table)):

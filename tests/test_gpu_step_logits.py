@@ -17,8 +17,8 @@ DEV = "cuda:0"
 def _model():
   torch.manual_seed(6)
   config = G.GriffinConfig(
-      vocab_size=32_000, width=512, mlp_expanded_width=512, lru_width=512,
-      num_heads=2, block_types=(G.TemporalBlockType.RECURRENT,
+      vocab_size=32_000, width=1024, mlp_expanded_width=512, lru_width=512,
+      num_heads=4, block_types=(G.TemporalBlockType.RECURRENT,
                                 G.TemporalBlockType.ATTENTION),
       embeddings_scale_by_sqrt_dim=True, attention_window_size=64,
       logits_soft_cap=30.0)
@@ -33,8 +33,8 @@ def _prompt(rows):
 
 @pytest.mark.parametrize("rows", [1, 3, 24, 25])
 def test_rows_of_a_step(rows):
-  e = G.Embedder(32_000, 256, True, device=DEV, dtype=torch.bfloat16)
-  x = torch.randn(rows, 1, 256, device=DEV).bfloat16()
+  e = G.Embedder(32_000, 1024, True, device=DEV, dtype=torch.bfloat16)
+  x = torch.randn(rows, 1, 1024, device=DEV).bfloat16()
   with torch.no_grad():
     for _ in range(2):
       got = e.decode(x, step=True)
@@ -52,7 +52,7 @@ def test_who_makes_a_copy():
   tokens, pos = _prompt(3)
   last, after = tokens[:, -1:], pos[:, -1:] + 1
   _, cache = model(tokens, pos)  # a prompt of a few rows, asked once
-  model.embedder.decode(torch.randn(2, 512, device=DEV).bfloat16())
+  model.embedder.decode(torch.randn(2, 1024, device=DEV).bfloat16())
   assert model.embedder._rows_logits is None
   model.embedder.step_copy = False
   model(last, after, cache)

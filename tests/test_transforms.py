@@ -22,7 +22,7 @@ def embedder(monkeypatch):
 
   monkeypatch.setattr(ops.PackedLinear, "__call__", refuse)
   torch.manual_seed(3)
-  e = G.Embedder(32_000, 64, True, dtype=torch.bfloat16)
+  e = G.Embedder(32_000, 1024, True, dtype=torch.bfloat16)
   e.requires_grad_(False)
   e.decode = functools.partial(e.decode, step=True)
   return e
@@ -30,7 +30,7 @@ def embedder(monkeypatch):
 
 def test_logits_under_transforms(embedder):
   table = embedder.input_embedding
-  x, dx = torch.randn(2, 3, 64).bfloat16()
+  x, dx = torch.randn(2, 3, 1024).bfloat16()
   with pytest.raises(AssertionError):
     embedder.decode(x)
   # (one rounding of float32 sums each, in whatever order)
@@ -46,3 +46,12 @@ def test_logits_under_transforms(embedder):
     close(got, tangent)
     with pytest.raises(AssertionError):
       embedder.decode(x)  # (no tangent of its own)
+
+
+@pytest.mark.parametrize("vocab,width,streamed", [
+    (256_000, 2560, True), (256_000, 4096, True), (32_000, 1024, True),
+    (128_256, 2560, True), (31_936, 2560, False), (50_304, 2560, False),
+    (256_032, 2560, False), (256_000, 512, False), (256_000, 4160, False)])
+def test_which_tables_are_streamed(vocab, width, streamed):
+  e = G.Embedder(vocab, width, True, device="meta", dtype=torch.bfloat16)
+  assert e._steps_stream() == streamed
