@@ -566,7 +566,16 @@ bool two_tiles(int tiles) { return tiles % 2 == 0 && tiles / 2 >= 200; }
 //   K 2560, N 4096     6.4 /  5.9   7.4 /  6.4   8.8 /  7.8  11.0 / 10.3
 //   K 4096, N 4096     9.6 /  8.5   9.9 /  8.5  11.5 / 10.1  14.6 / 13.6
 //   K 1024, N 2048     4.1 /  3.8   4.2 /  3.9   4.7 /  4.3   5.8 /  5.6
-bool half_tiles(int tiles) { return 2 * tiles <= 256; }
+// Of short rows a workgroup is mostly what it begins and ends with, and more than a few of
+// them are better read once for a whole tile (whole over half; 2.3 to 4 us a layer):
+//   rows                  1     4    16    32
+//   K 128, N 1024      1.06  1.04  0.98  0.97
+//   K 128, N 4096      1.00  1.00  0.92  0.92
+//   K 256, N 2048      1.02  1.04  0.99  0.95
+//   K 512, N 2048      1.09  1.09  1.04  1.03
+bool half_tiles(int tiles, int M, int K) {
+  return 2 * tiles <= 256 && (K >= 512 || M <= 4);
+}
 
 template <int NT, int MODE, int XR, int CPW, bool BESIDE>
 hipError_t launch_normed_of(const NormedLinearArgs& a, int blocks, hipStream_t s) {
@@ -627,7 +636,7 @@ hipError_t launch_linear_rows(const LinearArgs& a, int gelu_pair,
     return hipGetLastError();
   }
   if (two_tiles(tiles)) return launch_rows<2, kStore>(a, dim3(tiles / 2, 1), s);
-  if (half_tiles(tiles))
+  if (half_tiles(tiles, a.M, a.K))
     return launch_rows<1, kStore, false, true>(a, dim3(2 * tiles, 1), s);
   return launch_rows<1, kStore>(a, dim3(tiles, 1), s);
 }

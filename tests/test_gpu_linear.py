@@ -141,6 +141,14 @@ def test_half_tiles_equal_whole_ones(M, K, N):
   _check(alone, x.cpu(), w.cpu(), b.cpu())
 
 
+# short rows: half tiles for up to four of them, whole ones for more
+@pytest.mark.parametrize("M,K,N", [(4, 64, 4096), (5, 64, 4096), (4, 448, 96),
+                                   (5, 448, 96), (5, 512, 96), (33, 448, 4096),
+                                   (33, 512, 4096)])
+def test_half_tiles_of_short_rows(M, K, N):
+  test_half_tiles_equal_whole_ones(M, K, N)
+
+
 @pytest.mark.parametrize("M,K,E", [(64, 2560, 7680), (3, 128, 96)])
 def test_stacked_weight_and_gelu_pairs(M, K, E):
   """The MLP's stacked up-projection [2, K, E] (Einsum "cdD" layout): plain
