@@ -1361,7 +1361,14 @@ Plan plan(int B, int H, int T, int bw, bool joined) {
   const Split wide = best_split(B, H, T, slices, kTiles, 6.2f, 5.2f);
   const int pairs = (bw + kNarrowSlice - 1) / kNarrowSlice;
   const Split roles = best_split(B, H, T, pairs, kNarrowTeams, 7.0f, 3.2f);
-  if (wide.us <= roles.us) return Plan{kSlices11, slices, wide};
+  // (two tiles a workgroup have the two teams one behind the other: while the four-tile
+  // form's workgroups have a CU each that is ahead.  us, two teams / four tiles at once, 33
+  // to 64 tokens, 1 to 32 pairs: 9.7 to 10.1 / 9.6 to 10.0, joined 10.4 to 10.8 / 10.0 to
+  // 10.5; 64 pairs 10.1 to 10.2 / 10.0 to 10.5, joined 10.8 / 10.6; 85 pairs, in two rounds,
+  // 10.0 / 18.0, 128 10.9 / 11.3, joined 11.8 / 12.1)
+  const bool two_tiles = T > kTile && T <= 2 * kTile &&
+                         ((int64_t)B * H + 7) / 8 * 8 * slices <= 256;
+  if (two_tiles || wide.us <= roles.us) return Plan{kSlices11, slices, wide};
   return Plan{kNarrow, pairs, roles};
 }
 

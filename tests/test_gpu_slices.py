@@ -187,3 +187,11 @@ def test_rows_of_a_few_tokens(B, T, bw, H, mean_doc):
                                       (7, 16, 256, 10), (9, 7, 200, 3)])
 def test_rows_of_a_few_tokens_do_not_see_each_other(B, T, bw, H):
   test_rows_do_not_see_each_other(B, T, bw, H, True)
+
+
+# narrow heads, rows of two tiles: four tiles at once for up to 80 pairs, two teams beyond
+@pytest.mark.parametrize("B,T,bw,H", [(1, 33, 136, 1), (1, 64, 176, 32), (5, 50, 176, 8),
+                                      (40, 64, 136, 2), (81, 64, 136, 1)])
+@pytest.mark.parametrize("joined", [False, True])
+def test_rows_of_two_tiles(B, T, bw, H, joined):
+  test_prefill_in_slices(B, T, bw, H, 20, joined)
