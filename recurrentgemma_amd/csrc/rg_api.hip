@@ -845,7 +845,8 @@ int rg_recurrent_core(const void* x, const void* gate_branch,
         __func__, rg::launch_core_f32_small(a, (hipStream_t)stream));
   } else if (p.single || (w_packed != nullptr && dtype == RG_DTYPE_BF16 &&
                           rg::prefill_many_serve(B, H, T, W / H,
-                                                 gate_branch != nullptr))) {
+                                                 gate_branch != nullptr, conv,
+                                                 h0 != nullptr))) {
     // the join is part of the kernel's output stage, for rows in chunks too
     // (the launches that write y apply it)
     const size_t relay_bytes = p.relay_bytes[gate_branch != nullptr];

@@ -406,7 +406,7 @@ bool prefill_short_serves(int B, int H, int T);  // 256-wide heads
 hipError_t launch_block_prefill_short_bf16(const FusedArgs& a, hipStream_t s);
 bool prefill_slices_serve(int B, int H, int T, bool joined);  // 256-wide heads
 // rows of a few tokens, several to a tile (with re-laid-out weights)
-bool prefill_many_serve(int B, int H, int T, int bw, bool joined);
+bool prefill_many_serve(int B, int H, int T, int bw, bool joined, bool conv, bool state);
 bool prefill_narrow_pays(int B, int H, int T, int W);         // narrower ones
 hipError_t launch_block_prefill_slices_bf16(const FusedArgs& a, hipStream_t s);
 // float32, 256-wide heads, few rows: conv, gate projections, gates and

@@ -1007,7 +1007,8 @@ hipError_t launch_block_prefill_bf16(const FusedArgs& a, hipStream_t s) {
   // narrow heads, few pairs, short rows: heads in slices
   if (a.W / a.H != 256 ||
       (a.w_packed &&
-       prefill_many_serve(a.B, a.H, a.T, 256, a.gate_branch != nullptr)) ||
+       prefill_many_serve(a.B, a.H, a.T, 256, a.gate_branch != nullptr,
+                          a.conv_w != nullptr, a.h0 != nullptr)) ||
       (a.chunks <= 1 &&
        prefill_slices_serve(a.B, a.H, a.T, a.gate_branch != nullptr)))
     return launch_block_prefill_slices_bf16(a, s);

@@ -1305,24 +1305,26 @@ block_prefill_narrow_bf16_kernel(FusedArgs p, int slices, int groups) {
 }
 // How many ranges the rows are cut into, and the time that takes: workgroups
 // come in rounds of one per CU, and each costs a fixed part (weights, the
-// first rows) and its passes.
+// first rows) and its passes.  (Pairs are launched in eights: 85 with three slices each are
+// 264 workgroups, and the last eight a round of their own.)
 struct Split {
   int groups;
   float us;
+  int64_t rounds, passes;  // passes: of a workgroup
 };
 Split best_split(int B, int H, int T, int slices, int tiles, float fixed_us,
                  float pass_us) {
   const int64_t tiles_per_row = (T + kTile - 1) / kTile;
-  Split best{1, 1e30f};
+  Split best{1, 1e30f, 1, 1};
   for (int r = 1; r <= 9; ++r) {  // r workgroups per CU, and every row apart
-    int64_t groups = r == 9 ? B : 256 * r / ((int64_t)H * slices);
+    int64_t groups = r == 9 ? B : 256 * r / slices / 8 * 8 / H;
     if (groups < 1) groups = 1;
     if (groups > B) groups = B;
     const int64_t rows = (B + groups - 1) / groups;
     const int64_t passes = (rows * tiles_per_row + tiles - 1) / tiles;
-    const int64_t rounds = (groups * H * slices + 255) / 256;
+    const int64_t rounds = ((groups * H + 7) / 8 * 8 * slices + 255) / 256;
     const float us = rounds * (fixed_us + passes * pass_us);
-    if (us < best.us) best = Split{(int)groups, us};
+    if (us < best.us) best = Split{(int)groups, us, rounds, passes};
   }
   return best;
 }
@@ -1442,12 +1444,26 @@ bool prefill_slices_serve(int B, int H, int T, bool joined) {
 // joined, otherwise / so: W4096 B24 T1 18.7 / 12.3, T9 19.5 / 14.0, W5632 H32 B24 T3 27.1 /
 // 13.0, T9 34.8 / 13.9, B64 T1 26.1 / 13.3, T9 50 / 31; with one pass either way W2560 B24
 // T9 13.2 / 14.2, B2 T1 11.0 / 11.8.
-bool prefill_many_serve(int B, int H, int T, int bw, bool joined) {
+//
+// Beyond 512 pairs rg_recurrent_core's form is gate GEMM + scan.  256-wide heads stay
+// there: its outputs are those of the two calls, bit for bit.  Narrower ones go by what
+// either takes, fitted to 990 calls (heads of 136 to 248, 1 to 32 of them, 64 to 600 rows of
+// 1 to 16 tokens): apart within 20 %, here within 15 % but for single passes (8.2 a pass,
+// 9.3 with a state carried in).  us, here / apart: joined, 176 H10 B64 T16 12.8 / 28.3, B300
+// 46 / 66, 136 H32 B600 T9 175 / 188; without a conv, which costs the two calls a third, 136
+// H10 B300 T16 42.0 / 39.7, H32 B600 T9 166 / 124, 176 H1 B600 T3 11.9 / 16.
+bool prefill_many_serve(int B, int H, int T, int bw, bool joined, bool conv, bool state) {
   if (B < 2 || T > kManyTokens || bw <= 128 || bw > 256 || bw % 8) return false;
-  const float here = many_plan(B, H, T, bw).split.us;
-  // (beyond 512 pairs rg_recurrent_core's form is gate GEMM + scan.  256-wide heads stay
-  // there: its outputs are those of the two calls, bit for bit)
-  if ((int64_t)B * H > 512) return bw < 256;
+  const Split split = many_plan(B, H, T, bw).split;
+  const float here = split.us;
+  if ((int64_t)B * H > 512) {
+    const float rows = 1e-6f * (float)B * (float)(H * bw), elements = rows * (float)T;
+    const float apart = (conv ? 17.2f + 7.5f * rows + 4.6f * elements
+                              : 14.0f + 5.2f * rows + 3.6f * elements) +
+                        (joined ? 1.8f + 0.95f * elements : 0.0f);
+    return bw < 256 &&
+           split.rounds * (5.0f + (state ? 9.3f : 8.4f) * split.passes) < apart;
+  }
   const float apart = plan(B, H, T, bw, joined).split.us;
   return here < (bw < 256 || prefill_slices_serve(B, H, T, joined)
                      ? apart
@@ -1476,7 +1492,8 @@ hipError_t launch_block_prefill_slices_bf16(const FusedArgs& a, hipStream_t s) {
       (int64_t)a.T * a.W * 2 >= (int64_t)0x7fffffff)
     return hipErrorInvalidValue;
   if (a.w_packed &&
-      prefill_many_serve(a.B, a.H, a.T, bw, a.gate_branch != nullptr))
+      prefill_many_serve(a.B, a.H, a.T, bw, a.gate_branch != nullptr,
+                         a.conv_w != nullptr, a.h0 != nullptr))
     return a.gate_branch ? launch_many<true>(a, s) : launch_many<false>(a, s);
   const Plan p = plan(a.B, a.H, a.T, bw, a.gate_branch != nullptr);
   if (a.w_packed)

@@ -195,3 +195,13 @@ def test_rows_of_a_few_tokens_do_not_see_each_other(B, T, bw, H):
 @pytest.mark.parametrize("joined", [False, True])
 def test_rows_of_two_tiles(B, T, bw, H, joined):
   test_prefill_in_slices(B, T, bw, H, 20, joined)
+
+
+# beyond 512 pairs: where the two calls without a conv (a whole row in one call, and its
+# second half with a state) take less than several rows to a tile, and where they do not;
+# five heads of three slices, whose pairs are launched in eights
+@pytest.mark.parametrize("B,T,bw,H", [(600, 3, 136, 1), (600, 9, 136, 2),
+                                      (300, 16, 136, 5), (103, 16, 200, 5)])
+@pytest.mark.parametrize("joined", [False, True])
+def test_many_rows_of_narrow_heads(B, T, bw, H, joined):
+  test_prefill_in_slices(B, T, bw, H, 4, joined)
