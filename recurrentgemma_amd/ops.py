@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import math
 
 import torch
 
@@ -1194,8 +1195,8 @@ class PendingNorm:
   def served(sums, N, gelu_pair) -> bool:
     """Whether layers of N weight rows that read the norm of PartialSums have it
     in their own launch; elsewhere a norm is better formed at once."""
-    _, M, K = sums.sums.shape
-    return _norm_served(M, K, N, gelu_pair)
+    shape = sums.shape
+    return _norm_served(math.prod(shape[:-1]), shape[-1], N, gelu_pair)
 
   def __init__(self, sums, addend, scale, eps):
     self.args = _partial_norm_args(sums, addend, scale)
