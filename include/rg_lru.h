@@ -327,9 +327,9 @@ int rg_recurrent_prefill_gelu_mul(
  * rg_gelu_mul over `out` as a last launch), else the plain RG-LRU output.  `workspace` (16-byte aligned)
  * must hold rg_recurrent_core_workspace_bytes(B, T, W, H, dtype) bytes (0 for
  * whole rows in the single kernel: workspace may then be null).  Same values
- * as the calls it is made of (float32 with 256-wide heads: to rounding; so are bf16
- * rows with 256-wide heads that do not come out even on the CUs where the workspace
- * has B * W * 16 + H * 4 bytes or more, padded to 16: blocks of 32 tokens, whose
+ * as the calls it is made of (float32 with 256-wide heads, and narrower bf16 heads in
+ * the single kernel: to rounding; so are bf16 rows with 256-wide heads that do not come
+ * out even on the CUs where the workspace has B * W * 16 + H * 4 bytes or more, padded to 16: blocks of 32 tokens, whose
  * states go from workgroup to workgroup through it); h0 / h_last / conv_cache_out / w_packed as in
  * rg_recurrent_prefill (w_packed is only read by the single kernel).
  * conv_w == conv_b == NULL (conv_cache_out then NULL too): x is the conv
@@ -367,9 +367,10 @@ int rg_recurrent_step(const void* x, const void* segpos, int segpos_is_i64,
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  The three launches of rg_recurrent_step
  * (conv step, gate projections, scan step) exchange the conv output and the
- * two gate pre-activations through a buffer of RG_STEP_STATIC_SCRATCH_BYTES
- * that is part of the library's code object: every GPU the library runs on
- * holds one copy until the process ends.  Shapes whose
+ * two gate pre-activations (float32 with 256-wide heads, nothing written that is
+ * read, is one launch, which exchanges nothing) through a buffer of
+ * RG_STEP_STATIC_SCRATCH_BYTES that is part of the library's code object: every
+ * GPU the library runs on holds one copy until the process ends.  Shapes whose
  * rg_recurrent_step_workspace_bytes(B, W, dtype) exceeds that size are
  * rejected with RG_ERR_WORKSPACE.  Every call on a GPU uses that GPU's one
  * buffer: calls that overlap on one GPU (two streams, two threads) race;
