@@ -329,8 +329,9 @@ int rg_recurrent_prefill_gelu_mul(
  * whole rows in the single kernel: workspace may then be null).  Same values
  * as the calls it is made of (float32 with 256-wide heads, and narrower bf16 heads in
  * the single kernel: to rounding; so are bf16 rows with 256-wide heads that do not come
- * out even on the CUs where the workspace has B * W * 16 + H * 4 bytes or more, padded to 16: blocks of 32 tokens, whose
- * states go from workgroup to workgroup through it); h0 / h_last / conv_cache_out / w_packed as in
+ * out even on the CUs where the workspace has B * W * 16 + H * 4 bytes or more, padded
+ * to 16: blocks of 32 tokens, whose states go from workgroup to workgroup through it);
+ * h0 / h_last / conv_cache_out / w_packed as in
  * rg_recurrent_prefill (w_packed is only read by the single kernel).
  * conv_w == conv_b == NULL (conv_cache_out then NULL too): x is the conv
  * output already, and the call is RGLRU.forward on its own

@@ -822,10 +822,10 @@ class Griffin(nn.Module):
              many(rows, c.width, c.width) and
              ops.attention_prompt_row_fits(tokens, c.num_heads, head)))
 
-  def prompt_runs_serve(self, batch_size, tokens) -> bool:
+  def prompt_runs_serve(self, batch_size=1, tokens=8) -> bool:
     """Whether prompt_cache can stand for forward for tokens [batch_size,
-    tokens]: bf16 on the GPU, sizes that its kernels take, and nothing wrapped,
-    hooked or replaced on the way."""
+    tokens] (without them: for any at all): bf16 on the GPU, sizes that its
+    kernels take, and nothing wrapped, hooked or replaced on the way."""
     plain = modules._as_written
     if (not self._prompt_runs_sizes_serve(batch_size, tokens) or
         compiled.tracing() or modules._global_hooks() or
